@@ -23,7 +23,7 @@
 // group_m-rastered range of output tiles.
 // Entry point and reference citation: include/evo_mi355x.h.
 #include <stdlib.h>
-#include "common.h"
+#include "gemm_args.h"
 #include "../../include/evo_mi355x.h"
 
 #define GBM 256
@@ -39,18 +39,6 @@ typedef uint32_t g_u32x4 __attribute__((ext_vector_type(4)));
 #define G_VMCNT(N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory")
 #define G_BARRIER() asm volatile("s_barrier" ::: "memory")
 
-struct GemmArgs {
-    const unsigned char* x; const unsigned char* w; const uint16_t* bias; const uint16_t* res; uint16_t* y;
-    int64_t M; int N; int K;
-    int tiles_n; int n_tiles; int tiles_m; int group_m;
-    // RMSNorm folded into the dense layers around it (round 5; persistent kernel only, see gemmr_bf16_kernel's NF parameter)
-    const float* rs = nullptr;               // SCALE: 1 / (rms + eps) per token row, applied to the accumulators in the epilogue
-    float* ss = nullptr;                     // STATS: partial sums of squares of the stored rows, [N / 128 strips][ss_ld] fp32
-    int64_t ss_ld = 0;
-    int act_cols = 0;                        // ACT, mode 0: columns [0, act_cols) of the result go through the activation (a multiple of 256)
-    int64_t w_rows = 0;                      // MODE 3 + SCALE: rows of the token matrix (the kernel's "W" operand): B T
-    int tm_tiles = 0, row_skip = 0;          // MODE 3 + SCALE: a batch row = tm_tiles column tiles; its tokens start row_skip rows further per batch row
-};
 
 template <bool BIAS, bool RES>
 __global__ __launch_bounds__(512, 1) void gemm_bf16_kernel(GemmArgs a) {

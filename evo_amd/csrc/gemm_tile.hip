@@ -1,0 +1,575 @@
+// The dense layer of gemm.hip on smaller output tiles, for the sizes between decoding and full scoring batches: at 65 - 2,000 rows 256 x 256 tiles are
+// 16 - 190 workgroups on 256 CUs (a 4,096-column layer of 161 rows at K = 11,008: 16 workgroups, 187 us where the 90 MB of weights take 15 us).
+//
+// What bounds it: the rate at which a CU takes operands in.  Without products or LDS reads the k-loop runs no faster: 58 - 72 GB/s a CU, whatever the
+// tile and however deep the ring (loads that all hit the L2 reach 105 - 130), because every stage waits for the L2 miss of its newest weight lines
+// and a CU holds about 64 KB in flight.  Hence large tiles (bytes per product fall with the tile's sides), parts of K where large tiles are too few
+// for the chip, and weight lines shared by neighbours on one XCD.  The MFMA order over k is the persistent kernel's, so an unsplit product is bit
+// for bit the same on every tile; parts of K are fp32 sums added in order by a second launch.
+// Inner loop: a ring of NS stages of 64 k, LDS-DMA pieces spread between the products of the first half step (a burst blocks the wave on the
+// vector-memory queue), the next half's fragments requested under the products of the current one, one barrier per stage.
+#include <math.h>
+#include "gemm_args.h"
+#include "../../include/evo_mi355x.h"
+
+#define T_ROW 128                            // bytes per LDS row: one k-step of 64 bf16
+typedef uint32_t t_u32x4 __attribute__((ext_vector_type(4)));
+
+#define T_DSR(DST, ADDR, OFF) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(DST) : "v"(ADDR), "n"(OFF))
+
+// wait until at most N of this wave's LDS reads are out, tied to the fragments that the wait is for
+template <int N, int C>
+__device__ __forceinline__ void t_lgkm(t_u32x4 (&f)[C]) {
+    static_assert(C >= 1 && C <= 8, "fragments of one half step");
+    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
+#pragma unroll
+    for (int i = 0; i < C; ++i) asm volatile("" : "+v"(f[i]));
+}
+
+// SiLU (1), tanh-form GELU (2), square of relu (3): the arithmetic of gemm.hip's epilogue
+__device__ __forceinline__ void t_act(float (&v)[8], int act) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        if (act == 3) { const float t = fmaxf(v[e], 0.f); v[e] = t * t; }
+        else v[e] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(act == 2 ? v[e] * fmaf(v[e] * v[e], -0.1029432395800235f, -2.3022081981443250f)
+                                                                                   : v[e] * -1.4426950408889634f));
+    }
+}
+
+template <int BM, int BN, int WGM, int WGN, int NS, int PER_CU, int MODE, bool XB, bool SPLIT>
+__global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_tile_kernel(GemmArgs a, int act, float* parts, int splits) {
+    constexpr int NW = WGM * WGN, WM = BM / WGM, WN = BN / WGN, MT = WM / 16, NT = WN / 16;
+    constexpr int PX = BM / 8 / NW, PW = BN / 8 / NW, P = PX + PW;      // DMA pieces (8 rows, 1 KiB) of a stage per wave
+    constexpr int SLAB_X = BM * T_ROW, STAGE = (BM + BN) * T_ROW;
+    static_assert(PX >= 1 && PW >= 1 && NS >= 2 && NT % 2 == 0, "whole pieces per wave; column pairs");
+    static_assert(MODE != 1 || SPLIT || WN % 64 == 0, "a wave holds both halves of its gated columns");
+    constexpr bool STATS = MODE == 0 && !SPLIT && BN == 128;     // (a strip of the statistic is 128 columns)
+    __shared__ __attribute__((aligned(16))) unsigned char smem[NS * STAGE];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WGN, wn = wave % WGN;
+    const int l15 = lane & 15, lq = lane >> 4;
+    const int64_t kb = (int64_t)a.K * 2;
+    const int nk_all = a.K / 64;
+
+    // block b runs on XCD b % 8: every XCD gets a contiguous run of tiles, group_m row tiles next to each other before the next column tile
+    int tile;
+    {
+        const int bid = blockIdx.x, q = a.n_tiles >> 3, r = a.n_tiles & 7, xcd = bid & 7, slot = bid >> 3;
+        tile = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + slot;
+    }
+    int k0 = 0, nk = nk_all, sp = 0;
+    if constexpr (SPLIT) {                                       // the parts of a tile's sum are neighbours: they read the same rows, one behind the other
+        sp = tile % splits;
+        tile /= splits;
+        k0 = (int)((int64_t)nk_all * sp / splits);
+        nk = (int)((int64_t)nk_all * (sp + 1) / splits) - k0;
+    }
+    int tm, tn;
+    {
+        const int across = MODE == 3 ? a.tiles_m : a.tiles_n, along = MODE == 3 ? a.tiles_n : a.tiles_m;   // (mode 3: the tokens are the columns)
+        const int per_group = a.group_m * across;
+        const int grp = tile / per_group, in_grp = tile - grp * per_group, first = grp * a.group_m;
+        const int gsz = along - first < a.group_m ? along - first : a.group_m;
+        const int u = in_grp / gsz, v = first + in_grp - u * gsz;
+        tm = MODE == 3 ? u : v;
+        tn = MODE == 3 ? v : u;
+    }
+    const int64_t m0 = (int64_t)tm * BM;
+    const int n0 = tn * BN;
+
+    // ---- operands: LDS row r of a slab = 128 bytes of row r of the tile, granule g of 16 bytes at slot g ^ (r & 7) (a fragment read, 16 rows x 4
+    //      granules, meets no bank twice); the DMA's LDS side is lane-linear, so the lane that fills a slot fetches the granule that belongs there.
+    //      W rows: LDS row 32 b + 16 t + 4 q + r holds W row 32 b + 8 q + 4 t + r, so that a lane's accumulators of a pair of column tiles are
+    //      eight consecutive columns.  Rows behind the matrix read as zero (bounded descriptors).
+    uint32_t xoff[PX], woff[PW];
+    const int swz = ((lane & 7) ^ (lane >> 3)) & 7;
+#pragma unroll
+    for (int i = 0; i < PX; ++i) {
+        const int r = 8 * (wave + NW * i) + (lane >> 3);
+        if constexpr (XB) {                                      // [row block of 128][K / 16][128][16]
+            const int rb = (int)(m0 & 127) + r;
+            xoff[i] = (uint32_t)(rb >> 7) * (uint32_t)(128 * kb) + (rb & 127) * 32u + (swz >> 1) * 4096u + (swz & 1) * 16u;
+        } else xoff[i] = (uint32_t)(r * kb) + swz * 16u;
+    }
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+        const int r = 8 * (wave + NW * i) + (lane >> 3);
+        int wr = (r & ~31) + 8 * ((r >> 2) & 3) + 4 * ((r >> 4) & 1) + (r & 3);
+        if (MODE == 1 && a.w_rows) wr = (wr >> 6) * 32 + (wr & 31) + ((wr >> 5) & 1) * (a.N >> 1);     // [W1; W2] as it is: 32 rows of each in turn
+        woff[i] = (uint32_t)wr * (uint32_t)kb + swz * 16u;
+    }
+    int64_t src = n0, w_rows = a.N;                              // first row of the "W" operand and how many there are
+    if (MODE == 3 && a.rs) {
+        src += (int64_t)((n0 >> 8) / a.tm_tiles) * a.row_skip;
+        w_rows = a.w_rows;
+    }
+    const bool plain_gate = MODE == 1 && a.w_rows;
+    if (plain_gate) src = n0 >> 1;
+    const uint64_t xa = (uint64_t)a.x + (XB ? (m0 & ~(int64_t)127) : m0) * kb, wa = (uint64_t)a.w + src * kb;
+    const int64_t x_left = a.M - (XB ? (m0 & ~(int64_t)127) : m0), x_most = XB ? 256 : BM, x_ok = x_left < x_most ? x_left : x_most;    // (blocked X: whole blocks, M % 128 == 0)
+    const int64_t w_ok = plain_gate || w_rows - src < BN ? w_rows - src : BN;
+    const t_u32x4 rx = {(uint32_t)xa, (uint32_t)(xa >> 32) & 0xffffu, (uint32_t)(x_ok * kb), 0x00020000u};
+    const t_u32x4 rw = {(uint32_t)wa, (uint32_t)(wa >> 32) & 0xffffu, (uint32_t)(w_ok * kb), 0x00020000u};
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+
+    // piece `i` (of P) of stage `s` -> ring slot at byte `slot`; past the last stage the last one again, into a slot nobody reads (constant counts)
+    auto fetch1 = [&](int s, uint32_t slot, int i) {
+        s = (s < nk ? s : nk - 1) + k0;
+        const uint32_t dst = lds0 + slot + wave * 1024;
+        if (i < PX)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                         ::"s"(dst + i * NW * 1024), "v"(xoff[i < PX ? i : 0]), "s"(rx), "s"((uint32_t)s * (XB ? 16384u : 128u)) : "memory", "m0");
+        else
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                         ::"s"(dst + SLAB_X + (i - PX) * NW * 1024), "v"(woff[i < PX ? 0 : i - PX]), "s"(rw), "s"((uint32_t)s * 128u) : "memory", "m0");
+    };
+
+    uint32_t x_rd[2], w_rd[2];
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh) {
+        const int xr = wm * WM + l15, wr = wn * WN + l15;
+        x_rd[kh] = lds0 + (uint32_t)(xr * T_ROW + (((4 * kh + lq) ^ xr) & 7) * 16);
+        w_rd[kh] = lds0 + (uint32_t)(SLAB_X + wr * T_ROW + (((4 * kh + lq) ^ wr) & 7) * 16);
+    }
+    f32x4_t acc[NT][MT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    t_u32x4 wf[2][NT], xf[2][MT];
+    auto read = [&](uint32_t slot, int kh) {
+        const uint32_t wa_ = slot + w_rd[kh], xa_ = slot + x_rd[kh];
+#pragma unroll
+        for (int i = 0; i < NT; ++i) T_DSR(wf[kh][i], wa_, i * 16 * T_ROW);
+#pragma unroll
+        for (int j = 0; j < MT; ++j) T_DSR(xf[kh][j], xa_, j * 16 * T_ROW);
+    };
+    // the products of one half of a k-step; `dma`: with the P pieces of stage `s` between them
+    auto mma = [&](int kh, bool dma, int s, uint32_t fslot) {
+        constexpr int TOTAL = NT * MT;
+#pragma unroll
+        for (int u = 0; u < TOTAL; ++u) {
+            const int i = u / MT, j = u % MT;
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[kh][i]), __builtin_bit_cast(bf16x8_t, xf[kh][j]), acc[i][j], 0, 0, 0);
+            if (dma) {
+#pragma unroll
+                for (int d = u * P / TOTAL; d < (u + 1) * P / TOTAL; ++d) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    fetch1(s, fslot, d);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+    };
+
+    // ---- the pipeline over k-steps; stage k lives in slot k % NS.  Step k:
+    //        half 0   the second half's fragments are requested; products of the first, the DMA of stage k + NS - 1 spread between them (its slot held
+    //                 stage k - 1, which everyone had read before the last barrier)
+    //        wait     own pieces of stage k + 1 have landed, own reads of stage k are done; barrier: everyone's
+    //        half 1   the first fragments of stage k + 1 are requested; products of the second half
+    uint32_t slot = 0, nslot = STAGE, fslot = (NS - 1) * STAGE;
+#pragma unroll
+    for (int s = 0; s < NS - 1; ++s)
+#pragma unroll
+        for (int i = 0; i < P; ++i) fetch1(s, s * STAGE, i);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * P) : "memory");
+    asm volatile("s_barrier" ::: "memory");
+    read(0, 0);
+    for (int k = 0; k < nk; ++k) {
+        read(slot, 1);
+        t_lgkm<NT + MT>(wf[0]);
+        t_lgkm<NT + MT>(xf[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        mma(0, true, k + NS - 1, fslot);
+        __builtin_amdgcn_sched_barrier(0);
+        t_lgkm<0>(wf[1]);
+        t_lgkm<0>(xf[1]);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * P) : "memory");
+        asm volatile("s_barrier" ::: "memory");
+        read(nslot, 0);                                          // (behind the last stage: a slot that is not used any more)
+        __builtin_amdgcn_sched_barrier(0);
+        mma(1, false, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        fslot = slot;
+        slot = nslot;
+        nslot = nslot + STAGE == NS * STAGE ? 0 : nslot + STAGE;
+    }
+    t_lgkm<0>(wf[0]);
+    t_lgkm<0>(xf[0]);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // (the tail's re-fetches land before the LDS is read again or given back)
+
+    if constexpr (SPLIT) {                                       // this part's sums, as they are: [part][row][column]
+        float* out = parts + ((int64_t)sp * a.M) * a.N;
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const int64_t m = m0 + wm * WM + 16 * j + l15;
+            if (m < a.M) {
+#pragma unroll
+                for (int b = 0; b < NT / 2; ++b) {
+                    float* o = out + m * a.N + n0 + wn * WN + 32 * b + 8 * lq;
+                    *(f32x4_t*)o = acc[2 * b][j];
+                    *(f32x4_t*)(o + 4) = acc[2 * b + 1][j];
+                }
+            }
+        }
+        return;
+    }
+
+    // ---- epilogue, straight from registers: a lane's 8 values of (row tile j, column pair b) are columns 32 b + 8 lq .. + 7 of row 16 j + l15
+    if constexpr (MODE == 1) {
+        const int gn = a.N >> 1;
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const int64_t m = m0 + wm * WM + 16 * j + l15;
+            const float f = a.rs && m < a.M ? a.rs[m] : 1.f;
+#pragma unroll
+            for (int p = 0; p < WN / 64; ++p) {
+                float z1[8], z2[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    z1[e] = acc[4 * p + (e >> 2)][j][e & 3];
+                    z2[e] = acc[4 * p + 2 + (e >> 2)][j][e & 3];
+                    if (a.rs) { z1[e] *= f; z2[e] *= f; }
+                }
+                uint32_t o[4];
+#pragma unroll
+                for (int e = 0; e < 8; e += 2) {
+                    const uint32_t u1 = pack_bf2(z1[e], z1[e + 1]), u2 = pack_bf2(z2[e], z2[e + 1]);       // the dense layers' bf16 outputs
+                    const f32x2_t oo = act_gate2(f32x2_t{bf_lo(u1), bf_hi(u1)}, f32x2_t{bf_lo(u2), bf_hi(u2)}, act);
+                    o[e >> 1] = pack_bf2(oo[0], oo[1]);
+                }
+                if (m < a.M) *(uint4*)(a.y + m * gn + (n0 + wn * WN) / 2 + 32 * p + 8 * lq) = make_uint4(o[0], o[1], o[2], o[3]);
+            }
+        }
+        return;
+    }
+    const bool on = n0 < a.act_cols, stats = STATS && a.ss;
+    float ssum[MT];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+        const int64_t m = m0 + wm * WM + 16 * j + l15;
+        const bool ok = m < a.M;
+        const float f = MODE == 0 && a.rs && ok ? a.rs[m] : 1.f;
+        const float rb = MODE == 3 && a.bias ? bf_to_f(a.bias[m]) : 0.f;
+        ssum[j] = 0.f;
+#pragma unroll
+        for (int b = 0; b < NT / 2; ++b) {
+            const int n = n0 + wn * WN + 32 * b + 8 * lq;
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                v[e] = acc[2 * b + (e >> 2)][j][e & 3];
+                if (MODE == 0 && a.rs) v[e] *= f;
+                if (MODE == 3 && a.rs) v[e] *= a.rs[src + (n - n0) + e];
+            }
+            if constexpr (MODE == 3) {
+                if (a.bias) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] += rb;
+                }
+            } else if (a.bias) {
+                const uint4 q = *(const uint4*)(a.bias + n);
+                v[0] += bf_lo(q.x); v[1] += bf_hi(q.x); v[2] += bf_lo(q.y); v[3] += bf_hi(q.y);
+                v[4] += bf_lo(q.z); v[5] += bf_hi(q.z); v[6] += bf_lo(q.w); v[7] += bf_hi(q.w);
+            }
+            if (MODE == 0 && a.res && ok) {
+                const uint4 q = *(const uint4*)(a.res + m * a.N + n);
+                v[0] += bf_lo(q.x); v[1] += bf_hi(q.x); v[2] += bf_lo(q.y); v[3] += bf_hi(q.y);
+                v[4] += bf_lo(q.z); v[5] += bf_hi(q.z); v[6] += bf_lo(q.w); v[7] += bf_hi(q.w);
+            }
+            if (MODE == 0 && act && on) t_act(v, act);
+            const uint4 o = make_uint4(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]), pack_bf2(v[4], v[5]), pack_bf2(v[6], v[7]));    // the one rounding
+            if (ok) {
+                if constexpr (MODE == 3) *(uint4*)(a.y + (((int64_t)(n >> 8) * a.M + m) << 8) + (n & 255)) = o;
+                else *(uint4*)(a.y + m * a.N + n) = o;
+            }
+            if (stats) {
+                const uint32_t d[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { const float lo = bf_lo(d[e]), hi = bf_hi(d[e]); ssum[j] = fmaf(lo, lo, ssum[j]); ssum[j] = fmaf(hi, hi, ssum[j]); }
+            }
+        }
+    }
+    if (stats) {                                                 // a row's 128 columns: four lane groups, then the waves beside each other
+        float* row = (float*)smem;
+        asm volatile("s_barrier" ::: "memory");                  // (every wave is done with the operands)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            float t = ssum[j];
+            t += __shfl_xor(t, 16);
+            t += __shfl_xor(t, 32);
+            if (lq == 0) row[wn * BM + wm * WM + 16 * j + l15] = t;
+        }
+        __syncthreads();
+        for (int r = tid; r < BM; r += 64 * NW) {
+            float t = 0.f;
+#pragma unroll
+            for (int c = 0; c < WGN; ++c) t += row[c * BM + r];
+            if (m0 + r < a.ss_ld) a.ss[(int64_t)(n0 >> 7) * a.ss_ld + m0 + r] = t;
+        }
+    }
+}
+
+// The parts of every sum, added in the order of k, and what the product does behind it.  A thread takes eight columns of a row (mode 1: the eight
+// gated columns of two strips of 32).
+template <int MODE>
+__global__ __launch_bounds__(256) void gemm_parts_kernel(GemmArgs a, int act, const float* __restrict__ part, int splits) {
+    const int n8 = (MODE == 1 ? a.N >> 1 : a.N) >> 3;
+    const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t m = id / n8;
+    const int c8 = (int)(id - m * n8) * 8;
+    const bool ok = m < a.M;                                     // (N % 128 == 0: the 16 threads of a strip are all in or all out)
+    if (!ok) return;
+    const int64_t plane = a.M * a.N;
+    auto sum = [&](int n, float (&v)[8]) {
+        const float* p = part + m * a.N + n;
+        f32x4_t lo = *(const f32x4_t*)p, hi = *(const f32x4_t*)(p + 4);
+        for (int s = 1; s < splits; ++s) {
+            p += plane;
+            lo += *(const f32x4_t*)p;
+            hi += *(const f32x4_t*)(p + 4);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { v[e] = lo[e]; v[4 + e] = hi[e]; }
+    };
+    const float f = a.rs && MODE != 3 ? a.rs[m] : 1.f;
+    if constexpr (MODE == 1) {
+        const int n = (c8 >> 5) * 64 + (c8 & 31);
+        float z1[8], z2[8];
+        sum(n, z1);
+        sum(n + 32, z2);
+        uint32_t o[4];
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) {
+            if (a.rs) { z1[e] *= f; z1[e + 1] *= f; z2[e] *= f; z2[e + 1] *= f; }
+            const uint32_t u1 = pack_bf2(z1[e], z1[e + 1]), u2 = pack_bf2(z2[e], z2[e + 1]);
+            const f32x2_t oo = act_gate2(f32x2_t{bf_lo(u1), bf_hi(u1)}, f32x2_t{bf_lo(u2), bf_hi(u2)}, act);
+            o[e >> 1] = pack_bf2(oo[0], oo[1]);
+        }
+        *(uint4*)(a.y + m * (a.N >> 1) + c8) = make_uint4(o[0], o[1], o[2], o[3]);
+        return;
+    }
+    float v[8];
+    sum(c8, v);
+    if (MODE == 0 && a.rs) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] *= f;
+    }
+    if (MODE == 3 && a.rs) {
+        const int64_t src = c8 + (int64_t)((c8 >> 8) / a.tm_tiles) * a.row_skip;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] *= a.rs[src + e];
+    }
+    if constexpr (MODE == 3) {
+        if (a.bias) {
+            const float rb = bf_to_f(a.bias[m]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] += rb;
+        }
+    } else if (a.bias) {
+        const uint4 q = *(const uint4*)(a.bias + c8);
+        v[0] += bf_lo(q.x); v[1] += bf_hi(q.x); v[2] += bf_lo(q.y); v[3] += bf_hi(q.y);
+        v[4] += bf_lo(q.z); v[5] += bf_hi(q.z); v[6] += bf_lo(q.w); v[7] += bf_hi(q.w);
+    }
+    if (MODE == 0 && a.res) {
+        const uint4 q = *(const uint4*)(a.res + m * a.N + c8);
+        v[0] += bf_lo(q.x); v[1] += bf_hi(q.x); v[2] += bf_lo(q.y); v[3] += bf_hi(q.y);
+        v[4] += bf_lo(q.z); v[5] += bf_hi(q.z); v[6] += bf_lo(q.w); v[7] += bf_hi(q.w);
+    }
+    if (MODE == 0 && act && c8 < a.act_cols) t_act(v, act);
+    const uint4 o = make_uint4(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]), pack_bf2(v[4], v[5]), pack_bf2(v[6], v[7]));
+    if constexpr (MODE == 3) *(uint4*)(a.y + (((int64_t)(c8 >> 8) * a.M + m) << 8) + (c8 & 255)) = o;
+    else *(uint4*)(a.y + m * a.N + c8) = o;
+    if (MODE == 0 && a.ss) {
+        const uint32_t d[4] = {o.x, o.y, o.z, o.w};
+        float t = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { const float lo = bf_lo(d[e]), hi = bf_hi(d[e]); t = fmaf(lo, lo, t); t = fmaf(hi, hi, t); }
+        t += __shfl_xor(t, 1, 16);
+        t += __shfl_xor(t, 2, 16);
+        t += __shfl_xor(t, 4, 16);
+        t += __shfl_xor(t, 8, 16);
+        if ((threadIdx.x & 15) == 0) a.ss[(int64_t)(c8 >> 7) * a.ss_ld + m] = t;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------- which tile
+// Measured times of one k-step (64 deep) of one tile on one CU, in us: 64 x 64 0.267, 128 x 64 0.42, 128 x 128 0.575, 192 x 128 0.70, 256 x 128 0.84,
+// 256 x 256 (the persistent kernel) 1.12 -- all of them the pace at which a CU takes operands in (58 GB/s: 64 KB in flight, about 1 us behind the
+// L2 miss that one of the CUs sharing a row pays), so a product's time is its operand rows per CU, and a larger tile moves fewer.  A launch takes the
+// tile and the number of parts of K whose sum of rounds, partial sums and memory traffic is least.  At K = 4,096 / 11,008 (MI355X, us, persistent
+// kernel -> this choice): 4,096 columns 68 -> 16 / 187 -> 34 at 161 rows, 72 -> 28 / 188 -> 58 at 512, 74 -> 36 / 187 -> 95 at 1,024, 75 -> 57 / 193 ->
+// 147 at 2,048; 12,288 columns 76 -> 36 at 161 rows, 78 -> 58 at 512; 22,016 gated columns 82 -> 53 at 161.
+struct TileKind { int bm, bn; double step_us; };
+static const TileKind kinds[] = {{64, 64, 0.267}, {128, 64, 0.42}, {128, 128, 0.575}, {192, 128, 0.70}, {256, 128, 0.84}, {128, 256, 0.86}};
+#define T_PERSISTENT 99
+
+struct TilePlan { int kind; int splits; double us; int64_t rows; };      // rows: how many of M it takes
+
+static int tile_cus() {
+    static const int n = [] {
+        int dev = 0, c = 256;
+        if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev);
+        return c < 8 ? 8 : c & ~7;
+    }();
+    return n;
+}
+
+// `M` tokens, `N` columns of the weight; mode 3 has them the other way round in the launch
+static TilePlan tile_best(int64_t M, int64_t N, int64_t K, int mode, bool stats, bool splits_ok, bool persistent_ok) {
+    const double cus = tile_cus(), nk = (double)(K / 64), flops = 2.0 * M * N * K;
+    const double memory = (2.0 * (M * K + N * K) + 2.0 * M * N) / 5.3e6, power = flops / 1.56e9;
+    TilePlan best = {-1, 1, 1e30, M};
+    if (persistent_ok) {
+        const double rounds = ceil((double)((M + 255) / 256) * (double)(N / 256) / cus);
+        const double us = rounds * (nk * 1.12 + 6.0);
+        best = {T_PERSISTENT, 1, us > power ? us : power, M};
+        if (memory > best.us) best.us = memory;
+    }
+    for (int c = 0; c < (int)(sizeof(kinds) / sizeof(kinds[0])); ++c) {
+        const int bm = mode == 3 ? kinds[c].bn : kinds[c].bm, bn = mode == 3 ? kinds[c].bm : kinds[c].bn;      // along the tokens, along the weight
+        if ((mode == 1 && c == 0) || (mode != 3 && c == 5)) continue;
+        const double tiles = (double)((M + bm - 1) / bm) * (double)((N + bn - 1) / bn);
+        for (int s = 1; s <= (splits_ok ? 8 : 1); ++s) {
+            if (s == 1 && stats && bn != 128) continue;
+            if (s > 1 && (tiles * s > 2 * cus || nk / s < 8 || (double)s * M * N * 4 > 256e6)) break;
+            double us = ceil(tiles * s / cus) * (ceil(nk / s) * kinds[c].step_us + (mode == 1 && s == 1 ? 6.0 : 3.0));
+            if (us < power * 1.05) us = power * 1.05;
+            if (us < memory) us = memory;
+            if (s > 1) us += 5.0 + (double)s * M * N * 8 / 5.0e6;
+            if (us < best.us) best = {c, s, us, M};
+        }
+    }
+    return best;
+}
+
+// One or two launches: whole rounds of the persistent kernel in front where the last round would leave most of the chip idle.
+static int tile_plan(int64_t M, int64_t N, int64_t K, int mode, bool stats, bool splits_ok, bool persistent_ok, TilePlan (&out)[2]) {
+    out[0] = tile_best(M, N, K, mode, stats, splits_ok, persistent_ok);
+    if (!persistent_ok || mode == 3 || out[0].kind != T_PERSISTENT) return 1;
+    const int64_t tn = N / 256, cus = tile_cus();
+    for (int64_t rounds = (((M + 255) / 256) * tn) / cus; rounds >= 1 && rounds <= 16; --rounds) {
+        const int64_t rows = rounds * cus / tn * 256;            // (as many row tiles as fit the rounds)
+        if (rows < 256 || rows >= M) continue;
+        TilePlan head = tile_best(rows, N, K, mode, stats, false, true), tail = tile_best(M - rows, N, K, mode, stats, splits_ok, true);
+        if (head.kind == T_PERSISTENT && tail.kind != T_PERSISTENT && head.us + tail.us + 4.0 < 0.97 * out[0].us) {
+            out[0] = head;                                       // (`rows` of each are set by tile_best)
+            out[1] = tail;
+            return 2;
+        }
+        break;
+    }
+    return 1;
+}
+
+template <int BM, int BN, int WGM, int WGN, int NS, int PER_CU, bool GATE>
+static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, float* ws, hipStream_t st) {
+    a.tiles_m = (int)((a.M + BM - 1) / BM);
+    a.tiles_n = a.N / BN;
+    a.group_m = 8;
+    a.n_tiles = a.tiles_m * a.tiles_n * splits;
+    const dim3 grid((unsigned)a.n_tiles), block(64 * WGM * WGN);
+#define T_GO(MODE, XB, SPLIT) hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, NS, PER_CU, MODE, XB, SPLIT>), grid, block, 0, st, a, act, ws, splits)
+    if (splits == 1) {
+        if (mode == 3) T_GO(3, false, false);
+        else if (mode == 1) { if constexpr (GATE) T_GO(1, false, false); else return -1; }
+        else if (xblk) T_GO(0, true, false);
+        else T_GO(0, false, false);
+        return evo_launch_status();
+    }
+    if (mode == 3) T_GO(3, false, true);
+    else if (mode == 1) T_GO(1, false, true);
+    else if (xblk) T_GO(0, true, true);
+    else T_GO(0, false, true);
+#undef T_GO
+    const int64_t threads = a.M * ((mode == 1 ? a.N / 2 : a.N) / 8);
+    const dim3 rgrid((unsigned)((threads + 255) / 256)), rblock(256);
+    if (mode == 3) hipLaunchKernelGGL(gemm_parts_kernel<3>, rgrid, rblock, 0, st, a, act, ws, splits);
+    else if (mode == 1) hipLaunchKernelGGL(gemm_parts_kernel<1>, rgrid, rblock, 0, st, a, act, ws, splits);
+    else hipLaunchKernelGGL(gemm_parts_kernel<0>, rgrid, rblock, 0, st, a, act, ws, splits);
+    return evo_launch_status();
+}
+
+static bool dense_shape(int64_t mode, int64_t M, int64_t N, int64_t K) {
+    return mode >= 0 && mode <= 3 && M > 0 && N > 0 && K > 0 && N % 256 == 0 && K % 64 == 0 && N < (1 << 30) && K < (1 << 22) && M < (1ll << 31) - 256
+           && (mode != 3 || M % 256 == 0) && (mode != 2 || N * K * 2 < 0xffffffffll);
+}
+
+static int dense_plan(int64_t mode, bool stats, int64_t M, int64_t N, int64_t K, bool splits_ok, TilePlan (&plan)[2]) {
+    splits_ok = splits_ok && M < 1024;                           // (from 1,024 rows on a row's result is the same bits in every batch: passes may be run in row groups)
+    const bool persistent_ok = mode != 2 && K >= 128 && M * K * 2 < 0xffffffffll && N * K * 2 < 0xffffffffll;
+    return tile_plan(M, N, K, mode == 2 ? 1 : (int)mode, stats, splits_ok, persistent_ok, plan);
+}
+
+extern "C" int evo_dense_ws(int64_t mode, int64_t stats, int64_t M, int64_t N, int64_t K) {
+    if (!dense_shape(mode, M, N, K)) return -1;
+    TilePlan plan[2];
+    const int n = dense_plan(mode, stats != 0, M, N, K, true, plan);
+    int64_t most = 0;
+    for (int i = 0; i < n; ++i)
+        if (plan[i].splits > 1 && plan[i].splits * plan[i].rows * N * 4 > most) most = plan[i].splits * plan[i].rows * N * 4;
+    return (int)most;
+}
+
+extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const void* x, const void* w, const void* bias, const void* residual, void* y,
+                              const float* row_scale, float* sumsq, int64_t ss_ld, int64_t M, int64_t N, int64_t K, int64_t act_cols, int64_t x_rows,
+                              int64_t Tm, int64_t row_skip, void* ws, int64_t ws_bytes, void* stream) {
+    if (!dense_shape(mode, M, N, K) || act < 0 || act > 3 || act_cols < 0 || act_cols > N || act_cols % 256 != 0) return -1;
+    if ((mode == 1 || mode == 2) && (act > 1 || bias || residual || sumsq || xblk)) return -1;
+    if (mode == 3 && (act || residual || sumsq || xblk)) return -1;
+    if ((row_scale && (residual || sumsq)) || (sumsq && (!residual || ss_ld < (M + 255) / 256 * 256))) return -1;
+    if (mode == 0 && act && (residual || row_scale)) return -1;
+    if (xblk && (M % 256 != 0 || row_scale || act)) return -1;
+    if (mode == 3 && row_scale ? (Tm <= 0 || Tm % 256 != 0 || M % Tm != 0 || row_skip < 0 || row_skip > 0x7fff || x_rows < M + (M / Tm - 1) * row_skip)
+                               : (x_rows != 0 || Tm != 0 || row_skip != 0)) return -1;
+    TilePlan plan[2];
+    int n = dense_plan(mode, sumsq != nullptr, M, N, K, true, plan);
+    for (int i = 0; i < n; ++i)
+        if (plan[i].splits > 1 && (!ws || ws_bytes < plan[i].splits * plan[i].rows * N * 4)) {
+            n = dense_plan(mode, sumsq != nullptr, M, N, K, false, plan);
+            break;
+        }
+    int64_t m0 = 0;
+    for (int i = 0; i < n; ++i) {
+        const TilePlan& t = plan[i];
+        const unsigned char* xi = (const unsigned char*)x + m0 * K * 2;
+        const uint16_t* ri = residual ? (const uint16_t*)residual + m0 * N : nullptr;
+        uint16_t* yi = (uint16_t*)y + m0 * (mode == 1 || mode == 2 ? N / 2 : N);
+        const float* si = row_scale ? row_scale + m0 : nullptr;
+        float* qi = sumsq ? sumsq + m0 : nullptr;
+        int rc;
+        if (t.kind == T_PERSISTENT) {
+            if (mode == 1) rc = row_scale ? evo_mlp_gate_mfma_nf_bf16(xi, si, w, yi, t.rows, N / 2, K, stream) : evo_mlp_gate_mfma_bf16(xi, w, yi, t.rows, N / 2, K, act, stream);
+            else if (mode == 3) rc = row_scale ? evo_linear_t_mfma_nf_bf16(x, row_scale, w, bias, y, M, N, K, x_rows, Tm, row_skip, stream)
+                                               : evo_linear_t_mfma_bf16(x, w, bias, y, M, N, K, stream);
+            else if (xblk) rc = evo_linear_xblk_mfma_nf_bf16(xi, w, bias, ri, yi, qi, ss_ld, t.rows, N, K, stream);
+            else if (act) rc = evo_linear_act_mfma_bf16(xi, w, bias, yi, t.rows, N, K, act_cols, act, stream);
+            else rc = evo_linear_mfma_nf_bf16(xi, w, bias, ri, yi, si, qi, ss_ld, t.rows, N, K, stream);
+        } else {
+            GemmArgs a;
+            a.x = xi; a.w = (const unsigned char*)w; a.bias = (const uint16_t*)bias; a.res = ri; a.y = yi;
+            a.M = t.rows; a.N = (int)N; a.K = (int)K;
+            a.rs = si; a.ss = qi; a.ss_ld = ss_ld; a.act_cols = act ? (int)act_cols : 0;
+            if (mode == 2) a.w_rows = N;
+            if (mode == 3) {                                     // the rows of the launch are the weight's, its columns the tokens
+                a.x = (const unsigned char*)w; a.w = (const unsigned char*)x;
+                a.M = N; a.N = (int)M;
+                if (row_scale) { a.w_rows = x_rows; a.tm_tiles = (int)(Tm / 256); a.row_skip = (int)row_skip; }
+            }
+            const int tm = mode == 2 ? 1 : (int)mode;
+            float* f = (float*)ws;
+            hipStream_t st = (hipStream_t)stream;
+            if (t.kind == 0) rc = tile_launch<64, 64, 2, 2, 5, 2, false>(a, tm, (int)act, xblk != 0, t.splits, f, st);
+            else if (t.kind == 1) rc = tile_launch<128, 64, 4, 1, 3, 2, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
+            else if (t.kind == 2) rc = tile_launch<128, 128, 4, 2, 5, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
+            else if (t.kind == 3) rc = tile_launch<192, 128, 4, 2, 4, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
+            else if (t.kind == 4) rc = tile_launch<256, 128, 4, 2, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
+            else rc = tile_launch<128, 256, 2, 4, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
+        }
+        if (rc != 0) return rc;
+        m0 += t.rows;
+    }
+    return 0;
+}

@@ -245,8 +245,8 @@ class MixerOps:
                 and M * K * 2 < 0xffffffff and N * K * 2 < 0xffffffff):
             r = self._tail_rows(x, w)
             y = torch.empty(M, N, dtype=x.dtype, device=x.device)
-            self._call("evo_linear_act_mfma_bf16", x.data_ptr(), w.data_ptr(), None if b is None else b.data_ptr(), y.data_ptr(), M - r, N, K, act_cols,
-                       ACTIVATIONS[act])
+            with self._t("linear_act_mfma_bf16"):
+                self._dense_layer(0, x, w, y, M - r, N, K, act=ACTIVATIONS[act], b=b, act_cols=act_cols)
             if r:
                 self._linear_small_m(x[M - r:], w, b, None, out=y[M - r:])
                 self.act_cols_(y[M - r:], act_cols, act)

@@ -46,6 +46,8 @@ _SIGNATURES = {
     "evo_linear_mfma_nf_bf16": ([_PTR] * 7 + [_I64] * 4 + [_PTR], _c.c_int),
     "evo_linear_xblk_mfma_nf_bf16": ([_PTR] * 6 + [_I64] * 4 + [_PTR], _c.c_int),
     "evo_mlp_gate_mfma_nf_bf16": ([_PTR] * 4 + [_I64] * 3 + [_PTR], _c.c_int),
+    "evo_dense_ws": ([_I64] * 5, _c.c_int),
+    "evo_dense_bf16": ([_I64] * 3 + [_PTR] * 7 + [_I64] * 8 + [_PTR, _I64, _PTR], _c.c_int),
     "evo_linear_t_mfma_nf_bf16": ([_PTR] * 5 + [_I64] * 6 + [_PTR], _c.c_int),
     "evo_rms_finalize_f32": ([_PTR, _I64, _I64, _PTR, _I64, _I64, _I64, _F32, _PTR, _PTR], _c.c_int),
     "evo_probe_copy_f4": ([_PTR, _PTR, _I64, _PTR], _c.c_int),
@@ -84,7 +86,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 12         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 13         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):
@@ -277,6 +279,14 @@ class HipOps(MixerOps):
             return r
         return 0
 
+    def _dense_layer(self, mode, x, w, y, M, N, K, act=0, xblk=0, b=None, res=None, rs=None, ss=None, act_cols=0, x_rows=0, Tm=0, row_skip=0) -> None:
+        """evo_dense_bf16 (include/evo_mi355x.h) with the workspace that its tiles ask for."""
+        n = self.lib.evo_dense_ws(mode, ss is not None, M, N, K)
+        ws = torch.empty(n, dtype=torch.uint8, device=y.device) if n > 0 else None
+        _check(self.lib.evo_dense_bf16(mode, act, xblk, x.data_ptr(), w.data_ptr(), _ptr(b), _ptr(res), y.data_ptr(), _ptr(rs), _ptr(ss),
+                                       0 if ss is None else ss.shape[1], M, N, K, act_cols, x_rows, Tm, row_skip, _ptr(ws), max(n, 0), _stream()),
+               "evo_dense_bf16")
+
     def linear(self, x: torch.Tensor, w: torch.Tensor, b: Optional[torch.Tensor] = None, mfma: bool = False) -> torch.Tensor:
         """x [M,K] @ w[N,K]^T (+ b) -> [M,N] bf16.  M <= 16 (decode) takes the weight-streaming kernels; `mfma=True`
         (the attention block's projections) takes the hand-written MFMA kernel of csrc/gemm.hip when the shape allows
@@ -303,8 +313,7 @@ class HipOps(MixerOps):
     def _linear_into(self, y, x, w, b, mfma):
         if self._take_mfma(mfma) and self.mfma_linear_ok(x, w):
             with self._t("gemm_mfma"):
-                _check(self.lib.evo_linear_mfma_bf16(x.data_ptr(), w.data_ptr(), _ptr(b), None, y.data_ptr(),
-                                                     x.shape[0], w.shape[0], x.shape[1], _stream()), "evo_linear_mfma_bf16")
+                self._dense_layer(0, x, w, y, x.shape[0], w.shape[0], x.shape[1], b=b)
             return
         with self._t("gemm"):
             if b is not None:
@@ -374,8 +383,7 @@ class HipOps(MixerOps):
             self._need(residual, torch.bfloat16, "linear_mfma residual")
         y = residual if residual is not None else torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
         with self._t("gemm_mfma"):
-            _check(self.lib.evo_linear_mfma_bf16(x.data_ptr(), w.data_ptr(), _ptr(b), _ptr(residual), y.data_ptr(),
-                                                 M, N, K, _stream()), "evo_linear_mfma_bf16")
+            self._dense_layer(0, x, w, y, M, N, K, b=b, res=residual)
         return y
 
     # ---- kernels -------------------------------------------------------------------------------------
@@ -499,8 +507,7 @@ class HipOps(MixerOps):
         assert xp.shape[0] >= Mp + B * r
         zt = torch.empty(Mp // 256 + (1 if r and tail else 0), N, 256, dtype=torch.bfloat16, device=xp.device)
         with self._t("gemm_zt"):
-            _check(self.lib.evo_linear_t_mfma_bf16(xp.data_ptr(), w.data_ptr(), _ptr(b), zt.data_ptr(), Mp, N, K, _stream()),
-                   "evo_linear_t_mfma_bf16")
+            self._dense_layer(3, xp, w, zt, Mp, N, K, b=b)
         if r and tail:
             zt[-1].zero_()                                                                # (6 MB: the tail block's unused positions hold zeros, not whatever the allocator left)
             z_tail = self._linear_small_m(xp[Mp:Mp + B * r], w, b, None)                # [B r, N]
@@ -666,8 +673,7 @@ class HipOps(MixerOps):
         if not ok:
             return self.linear_residual_(res, self.yblk_to_rows(y_blk, M).contiguous(), w, bias=bias)
         with self._t("gemm_mfma"):
-            _check(self.lib.evo_linear_xblk_mfma_bf16(y_blk.data_ptr(), w.data_ptr(), _ptr(bias), res.data_ptr(), res.data_ptr(), Mf, N, K,
-                                                      _stream()), "evo_linear_xblk_mfma_bf16")
+            self._dense_layer(0, y_blk, w, res, Mf, N, K, xblk=1, b=bias, res=res)
         if M > Mf:                                           # (<= 255 rows: rows Mf .. M - 1 of the matrix, gathered row-major)
             r = M - Mf
             nb0 = Mf // self.YBLK
@@ -711,8 +717,7 @@ class HipOps(MixerOps):
         Mm = self._nf_main_rows(M)
         ss = torch.empty(N // 128, (Mm + 255) // 256 * 256, dtype=torch.float32, device=res.device)
         with self._t("gemm_mfma"):
-            _check(self.lib.evo_linear_mfma_nf_bf16(x.data_ptr(), w.data_ptr(), _ptr(bias), res.data_ptr(), res.data_ptr(), None, ss.data_ptr(),
-                                                    ss.shape[1], Mm, N, K, _stream()), "evo_linear_mfma_nf_bf16")
+            self._dense_layer(0, x, w, res, Mm, N, K, b=bias, res=res, ss=ss)
         if M > Mm:
             self._linear_small_m(x[Mm:], w, bias, res[Mm:])
         return self.rms_finalize(ss, res, Mm, eps)
@@ -724,8 +729,7 @@ class HipOps(MixerOps):
         Mf = M // 256 * 256
         ss = torch.empty(N // 128, Mf, dtype=torch.float32, device=res.device)
         with self._t("gemm_mfma"):
-            _check(self.lib.evo_linear_xblk_mfma_nf_bf16(y_blk.data_ptr(), w.data_ptr(), _ptr(bias), res.data_ptr(), res.data_ptr(), ss.data_ptr(),
-                                                         Mf, Mf, N, K, _stream()), "evo_linear_xblk_mfma_nf_bf16")
+            self._dense_layer(0, y_blk, w, res, Mf, N, K, xblk=1, b=bias, res=res, ss=ss)
         if M > Mf:
             r = M - Mf
             tail = y_blk[Mf // self.YBLK:].permute(0, 2, 1, 3).reshape(-1, K)[:r].contiguous()
@@ -741,8 +745,7 @@ class HipOps(MixerOps):
         Mm = self._nf_main_rows(M)
         y = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
         with self._t("gemm_mfma"):
-            _check(self.lib.evo_linear_mfma_nf_bf16(x.data_ptr(), w_folded.data_ptr(), _ptr(b), None, y.data_ptr(), rstd.data_ptr(), None, 0,
-                                                    Mm, N, K, _stream()), "evo_linear_mfma_nf_bf16")
+            self._dense_layer(0, x, w_folded, y, Mm, N, K, b=b, rs=rstd)
         if M > Mm:
             y[Mm:] = self.norm_linear(x[Mm:], scale, eps, w, b)
         return y
@@ -756,8 +759,7 @@ class HipOps(MixerOps):
         Mm = self._nf_main_rows(M)
         a = torch.empty(M, I, dtype=torch.bfloat16, device=x.device)
         with self._t("gemm_gate"):
-            _check(self.lib.evo_mlp_gate_mfma_nf_bf16(x.data_ptr(), rstd.data_ptr(), w12g_folded.data_ptr(), a.data_ptr(), Mm, I, K, _stream()),
-                   "evo_mlp_gate_mfma_nf_bf16")
+            self._dense_layer(1, x, w12g_folded, a, Mm, 2 * I, K, rs=rstd)
         if M > Mm:
             a[Mm:] = self.mlp_gate(x[Mm:], w12, scale, eps, w12g=None if w12 is not None else w12g_folded)
         return a
@@ -783,13 +785,11 @@ class HipOps(MixerOps):
         if r == 0:                                    # plain form without a single pad position: z^T position p IS row p of the stream
             zt = torch.empty(Mp // 256, N, 256, dtype=torch.bfloat16, device=x.device)
             with self._t("gemm_zt"):
-                _check(self.lib.evo_linear_t_mfma_nf_bf16(x.data_ptr(), rstd.data_ptr(), w_folded.data_ptr(), _ptr(b), zt.data_ptr(), Mp, N, K,
-                                                          Mp, Mp, 0, _stream()), "evo_linear_t_mfma_nf_bf16")
+                self._dense_layer(3, x, w_folded, zt, Mp, N, K, b=b, rs=rstd, x_rows=Mp, Tm=Mp)
             return zt
         zt = torch.empty(Mp // 256 + (1 if tail else 0), N, 256, dtype=torch.bfloat16, device=x.device)
         with self._t("gemm_zt"):
-            _check(self.lib.evo_linear_t_mfma_nf_bf16(x.data_ptr(), rstd.data_ptr(), w_folded.data_ptr(), _ptr(b), zt.data_ptr(), Mp, N, K,
-                                                      B * T, Tm, r, _stream()), "evo_linear_t_mfma_nf_bf16")
+            self._dense_layer(3, x, w_folded, zt, Mp, N, K, b=b, rs=rstd, x_rows=B * T, Tm=Tm, row_skip=r)
         if not tail:                                  # (the caller runs the tail tokens through the single-token launch: hyena_ct(main_only=True))
             return zt
         zt[-1].zero_()
@@ -1015,8 +1015,7 @@ class HipOps(MixerOps):
             a = torch.empty(M, I, dtype=torch.bfloat16, device=x.device)
             r = self._tail_rows(x, wsrc)                          # the BOS sliver (M % 256 <= 16) goes through the small-M path
             with self._t("gemm_gate"):
-                _check(self.lib.evo_mlp_gate_mfma_bf16(x.data_ptr(), w12g.data_ptr(), a.data_ptr(), M - r, I, K, code, _stream()),
-                       "evo_mlp_gate_mfma_bf16")
+                self._dense_layer(1, x, w12g, a, M - r, 2 * I, K, act=code)
             if r:
                 a[M - r:] = self.mlp_gate(x[M - r:], w12, w12g=w12g if w12 is None else None, act=act)
             return a
@@ -1048,6 +1047,12 @@ class HipOps(MixerOps):
             return a
         if norm_scale is not None:
             x = self.rmsnorm(x, None, norm_scale, eps)
+        if (self.mlp_gate_fused and 64 < M < 1024 and ok_mem and (2 * I) % 256 == 0 and I % 32 == 0 and K % 64 == 0 and 4 * I * K < 0xffffffff):
+            # 65-255 rows, and more where only [W1; W2] is there: the gate in the epilogue of the smaller tiles, which read either order
+            a = torch.empty(M, I, dtype=torch.bfloat16, device=x.device)
+            with self._t("gemm_gate"):
+                self._dense_layer(1 if grouped else 2, x, wsrc, a, M, 2 * I, K, act=code)
+            return a
         g = self.linear(x, wsrc, None)
         if grouped:                                               # columns come out as [32 of z1 | the same 32 of z2] per block: back to [z1 | z2]
             g = g.view(M, I // 32, 2, 32).permute(0, 2, 1, 3).reshape(M, 2 * I).contiguous()

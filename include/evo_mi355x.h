@@ -54,7 +54,7 @@ extern "C" {
  *  12: evo_linear_act_mfma_bf16 (bias, three activations) and evo_act_cols take the places of evo_linear_silu_mfma_bf16 and evo_silu_cols; the
  *      evo_postnorm_* launches gained the norm of the sum (`alpha`, `sum`) and the plain one an activation, as did evo_linear_small_m_bf16; evo_window_attn gained grouped key heads,
  *      kept first tokens and two maps; evo_sum_norm, evo_heads_* and evo_rglru_* added. */
-#define EVO_ABI_VERSION 12
+#define EVO_ABI_VERSION 13
 int evo_abi_version(void);
 
 /* ---- embedding gather ------------------------------------------------------------------------
@@ -301,6 +301,19 @@ int evo_linear_xblk_mfma_nf_bf16(const void* x_blk, const void* w, const void* b
 int evo_mlp_gate_mfma_nf_bf16(const void* x, const float* row_scale, const void* w12g, void* a, int64_t M, int64_t I, int64_t K, void* stream);
 int evo_linear_t_mfma_nf_bf16(const void* x, const float* row_scale, const void* w, const void* bias, void* zt, int64_t Mp, int64_t N,
                               int64_t K, int64_t x_rows, int64_t Tm, int64_t row_skip, void* stream);
+
+/* Any of the dense layers above, on the tiles that its size asks for: the persistent kernel where 256 x 256 tiles fill the chip, otherwise smaller tiles
+ * and, where those are still too few, parts of K whose fp32 sums a second launch adds in the order of k (csrc/gemm_tile.hip has the rule).
+ *   mode 0: y [M, N] = act(x w^T + bias) (+ residual); x row-major, or blocked with xblk != 0 (evo_linear_xblk_mfma_bf16); row_scale, sumsq as in the
+ *           nf entries; act on columns [0, act_cols) as in evo_linear_act_mfma_bf16 (without residual and row_scale)
+ *   mode 1: y [M, N / 2] = gated, w = N rows in evo_mlp_gate_mfma_bf16's order, act 0 gelu, 1 silu; mode 2: the same, w = [W1; W2] as it is
+ *   mode 3: z^T of evo_linear_t_mfma_nf_bf16, M = Mp; x_rows, Tm, row_skip as there with row_scale, 0 without
+ * N % 256 == 0, K % 64 == 0; M % 256 == 0 for mode 3 and xblk; N K 2 < 4 GiB for mode 2.  `ws`: evo_dense_ws(mode, sumsq != NULL, M, N, K) bytes, 16-byte
+ * aligned; NULL or fewer: the same product without parts of K. */
+int evo_dense_ws(int64_t mode, int64_t stats, int64_t M, int64_t N, int64_t K);
+int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const void* x, const void* w, const void* bias, const void* residual, void* y,
+                   const float* row_scale, float* sumsq, int64_t ss_ld, int64_t M, int64_t N, int64_t K, int64_t act_cols, int64_t x_rows,
+                   int64_t Tm, int64_t row_skip, void* ws, int64_t ws_bytes, void* stream);
 int evo_rms_finalize_f32(const float* sumsq, int64_t n_strips, int64_t ss_ld, const void* x, int64_t M_main, int64_t M, int64_t D,
                          float eps, float* rstd, void* stream);
 

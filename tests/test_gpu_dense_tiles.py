@@ -1,0 +1,126 @@
+"""GPU parity of the dense layer's smaller tiles and parts of K (csrc/gemm_tile.hip) through the ops that take them.
+
+Reference: the product of the bf16 operands in fp64, then what follows it, rounded once.  Tolerance: half a bf16 ulp of the result is 2^-9 of it, taken
+twice; the fp32 sums add at most K 2^-24 of the sum of magnitudes, under 1e-3 for operands of unit variance and weights of variance 1 / K.
+"""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# rows on both sides of every tile's edge; columns and depths that lead to each tile, to parts of K, and to two launches one behind the other (6,400 rows)
+SHAPES = [(65, 256, 64), (65, 4096, 4096), (127, 512, 1024), (129, 4096, 4096), (161, 12288, 512), (161, 4096, 11008), (255, 4096, 4096),
+          (385, 4096, 4096), (513, 4096, 11008), (769, 4096, 4096), (770, 4096, 11008), (1023, 4096, 11008), (1024, 4096, 11008), (1537, 4096, 2048), (2048, 4096, 1088), (2049, 4096, 4096),
+          (6400, 4096, 1024)]
+
+
+def _ops():
+    from evo_amd.ops import default_ops
+    return default_ops()
+
+
+def _data(M, N, K, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(M * 13 + N * 3 + K + seed)
+    x = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(N, K, device="cuda", generator=g) / K ** 0.5).bfloat16()
+    return g, x, w
+
+
+def _close(got, want):
+    err = (got.double() - want).abs()
+    assert bool((err <= want.abs() * 2.0 ** -8 + 1e-3).all()), f"max err {err.max().item():.3e}"
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("bias,res", [(False, False), (True, True)])
+def test_plain(M, N, K, bias, res):
+    ops = _ops()
+    g, x, w = _data(M, N, K)
+    b = torch.randn(N, device="cuda", generator=g).bfloat16() if bias else None
+    buf = torch.randn(M + 8, N, device="cuda", generator=g).bfloat16()
+    keep = buf.clone()
+    want = x.double() @ w.double().T
+    want = want if b is None else want + b.double()
+    got = ops.linear_mfma(x, w, b, buf[:M] if res else None)
+    _close(got, want + keep[:M].double() if res else want)
+    assert torch.equal(buf[M:], keep[M:])                       # rows behind the last stay untouched
+    again = ops.linear_mfma(x, w, b, keep[:M].clone() if res else None)
+    assert torch.equal(got, again)                              # the parts are added in a fixed order
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 512, 1024), (161, 4096, 4096), (700, 16384, 512), (1537, 4096, 1024)])
+@pytest.mark.parametrize("act,cols", [("silu", 256), ("gelu_tanh", 512), ("relu2", -1)])
+def test_activation(M, N, K, act, cols):
+    ops = _ops()
+    g, x, w = _data(M, N, K, 1)
+    cols = N if cols < 0 else cols
+    z = x.double() @ w.double().T
+    f = {"silu": torch.nn.functional.silu, "gelu_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh"), "relu2": lambda t: t.relu().square()}[act]
+    want = torch.cat([f(z[:, :cols]), z[:, cols:]], 1)
+    err = (ops.linear_act(x, w, act, cols).double() - want).abs()
+    assert bool((err <= want.abs() * 2.0 ** -8 + 4e-3).all())    # (the square's slope is up to 8 here, and v_rcp / v_exp add 2^-22 each)
+
+
+@pytest.mark.parametrize("M,I,K", [(65, 128, 128), (100, 11008, 4096), (161, 11008, 4096), (255, 384, 1024), (300, 2048, 512), (513, 11008, 256), (1030, 2048, 4096)])
+@pytest.mark.parametrize("order", ["plain", "grouped"])
+@pytest.mark.parametrize("act", ["gelu", "silu"])
+def test_gate(M, I, K, order, act):
+    ops = _ops()
+    g, x, w = _data(M, 2 * I, K, 2)
+    z = (x.double() @ w.double().T).bfloat16().double()
+    z1, z2 = z[:, :I], z[:, I:]
+    want = (torch.nn.functional.gelu(z1) if act == "gelu" else torch.nn.functional.silu(z1)) * z2
+    got = ops.mlp_gate(x, w if order == "plain" else None, w12g=None if order == "plain" else ops.pack_gate_weights(w), act=act)
+    err = (got.double() - want).abs()
+    # a value of z on the edge of two bf16 numbers may round the other way: 2^-8 of it, through a slope of at most 1.13 and the other factor
+    assert bool((err <= want.abs() * 2.0 ** -7 + (z1.abs() + 0.2) * z2.abs() * 2.0 ** -7 + 1e-3).all()), err.max().item()
+
+
+@pytest.mark.parametrize("B,T,N,K", [(1, 256, 768, 256), (1, 500, 12288, 4096), (2, 600, 12288, 1024), (3, 1000, 768, 4096)])
+def test_transposed(B, T, N, K):
+    ops = _ops()
+    g, x, w = _data(B * T, N, K, 3)
+    b = torch.randn(N, device="cuda", generator=g).bfloat16()
+    xp = ops.rmsnorm_rows(x, torch.ones(K, device="cuda").bfloat16(), 1e-6, B, T)
+    zt = ops.linear_t(xp, w, b, B, T)
+    want = xp[: zt.shape[0] * 256].double() @ w.double().T + b.double()
+    got = zt.permute(0, 2, 1).reshape(-1, N)
+    _close(got, want)
+
+
+@pytest.mark.parametrize("M,K", [(1024, 4096), (1536, 1024), (2304, 4096), (6400, 1024)])
+def test_norm_folded(M, K):
+    """Row factors in, sums of squares out, the blocked X: each against the same steps one by one."""
+    ops = _ops()
+    N = 4096
+    g, x, w = _data(M, N, K, 4)
+    res = torch.randn(M, N, device="cuda", generator=g).bfloat16()
+    want = x.double() @ w.double().T + res.double()
+    for blocked in (False, True):
+        r = res.clone()
+        if blocked:
+            xb = x.view(M // 128, 128, K // 16, 16).permute(0, 2, 1, 3).contiguous()
+            rstd = ops.linear_residual_yblk_stats_(r, xb, w, None, 1e-6)
+        else:
+            rstd = ops.linear_residual_stats_(r, x, w, None, 1e-6)
+        _close(r, want)
+        rms = r.double().square().mean(1).sqrt()
+        assert bool(((rstd[:M].double() * (rms + 1e-6) - 1).abs() < 1e-5).all())
+    w2 = (torch.randn(768, N, device="cuda", generator=g) / 64).bfloat16()
+    _close(ops.linear_rs(r, rstd, w2, None, w2, torch.ones(N, device="cuda").bfloat16(), 1e-6), (r.double() / (rms + 1e-6)[:, None]) @ w2.double().T)
+    gate = ops.mlp_gate_rs(r, rstd, ops.pack_gate_weights(w2[:512]), w2[:512], torch.ones(N, device="cuda").bfloat16(), 1e-6)
+    z = ((r.double() / (rms + 1e-6)[:, None]) @ w2[:512].double().T).bfloat16().double()
+    g_want = torch.nn.functional.gelu(z[:, :256]) * z[:, 256:]
+    assert bool(((gate.double() - g_want).abs() <= g_want.abs() * 2.0 ** -7 + (z[:, :256].abs() + 0.2) * z[:, 256:].abs() * 2.0 ** -7 + 1e-3).all())
+
+
+def test_without_a_workspace():
+    """The same product, unsplit, when the caller has no room for the parts."""
+    from evo_amd.ops import _stream
+    ops = _ops()
+    M, N, K = 161, 4096, 11008
+    _, x, w = _data(M, N, K, 5)
+    assert ops.lib.evo_dense_ws(0, 0, M, N, K) > 0
+    y = torch.empty(M, N, device="cuda", dtype=torch.bfloat16)
+    assert ops.lib.evo_dense_bf16(0, 0, 0, x.data_ptr(), w.data_ptr(), None, None, y.data_ptr(), None, None, 0, M, N, K, 0, 0, 0, 0, None, 0, _stream()) == 0
+    _close(y, x.double() @ w.double().T)
