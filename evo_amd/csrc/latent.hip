@@ -331,10 +331,11 @@ __global__ __launch_bounds__(512, 2) void latent_decode_kernel(DecArgs a) {
         }
 }
 
-// Any sizes, both storage types: one wave per (split, head, sequence)
-template <typename T>
+// Any sizes, both storage types: one wave per (split, head, sequence).  V = 4: fp32 rows in 16-byte requests (a lane's key row element by element was one
+// 4-byte request of 64 lines per product: 154 us for 3 sequences x 32 heads behind 500 tokens of 576, 45 now).
+template <typename T, int V>
 __global__ __launch_bounds__(64) void latent_decode_any_kernel(DecArgs a, int dq) {
-    extern __shared__ float qf[];
+    extern __shared__ __attribute__((aligned(16))) float qf[];
     const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z, lane = threadIdx.x;
     const T* q = (const T*)a.q + ((int64_t)b * a.H + h) * a.rs;
     for (int d = lane; d < dq; d += 64) qf[d] = ld1(q + d);
@@ -356,7 +357,16 @@ __global__ __launch_bounds__(64) void latent_decode_any_kernel(DecArgs a, int dq
             float s = -INFINITY;
             if (slot < used && slot_seen(slot, pos, cur, a)) {
                 s = 0.f;
-                for (int d = 0; d < dq; ++d) s = fmaf(qf[d], ld1(base + (int64_t)slot * a.rs + d), s);
+                if constexpr (V == 4) {
+                    const float* row = (const float*)base + (int64_t)slot * a.rs;
+#pragma unroll 8
+                    for (int d = 0; d < dq; d += 4) {
+                        const f32x4_t x = *(const f32x4_t*)(row + d), y = *(const f32x4_t*)(qf + d);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) s = fmaf(y[e], x[e], s);
+                    }
+                } else
+                    for (int d = 0; d < dq; ++d) s = fmaf(qf[d], ld1(base + (int64_t)slot * a.rs + d), s);
                 s *= a.sc2;
             }
             const float top = fmaxf(m, wave_max(s));
@@ -367,18 +377,33 @@ __global__ __launch_bounds__(64) void latent_decode_any_kernel(DecArgs a, int dq
 #pragma unroll
             for (int e = 0; e < 8; ++e) o[e] *= f;
             const int n = used - s0 < 64 ? used - s0 : 64;
-            for (int u = 0; u < n; ++u) {
-                const float pu = __shfl(pr, u, 64);
+            if constexpr (V == 4) {                              // (a lane's eight columns: two runs of four)
+#pragma unroll 4
+                for (int u = 0; u < n; ++u) {
+                    const float pu = __shfl(pr, u, 64);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int r = pass * 512 + lane + 64 * e;
-                    if (r < a.R) o[e] = fmaf(pu, ld1(base + (int64_t)(s0 + u) * a.rs + r), o[e]);
+                    for (int e = 0; e < 8; e += 4) {
+                        const int r = pass * 512 + 4 * lane + 64 * e;
+                        if (r < a.R) {
+                            const f32x4_t x = *(const f32x4_t*)((const float*)base + (int64_t)(s0 + u) * a.rs + r);
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) o[e + i] = fmaf(pu, x[i], o[e + i]);
+                        }
+                    }
                 }
-            }
+            } else
+                for (int u = 0; u < n; ++u) {
+                    const float pu = __shfl(pr, u, 64);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const int r = pass * 512 + lane + 64 * e;
+                        if (r < a.R) o[e] = fmaf(pu, ld1(base + (int64_t)(s0 + u) * a.rs + r), o[e]);
+                    }
+                }
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const int r = pass * 512 + lane + 64 * e;
+            const int r = pass * 512 + (V == 4 ? 4 * lane + 64 * (e & 4) + (e & 3) : lane + 64 * e);
             if (r < a.R) po[r] = o[e];
         }
     }
@@ -423,8 +448,10 @@ extern "C" int evo_latent_decode(const void* q, const void* cache, const int64_t
         return evo_launch_status();
     }
     const dim3 grid((unsigned)n_split, (unsigned)H, (unsigned)B);
-    if (f32) hipLaunchKernelGGL((latent_decode_any_kernel<float>), grid, dim3(64), (size_t)(R + dr) * 4, s, a, (int)(R + dr));
-    else hipLaunchKernelGGL((latent_decode_any_kernel<uint16_t>), grid, dim3(64), (size_t)(R + dr) * 4, s, a, (int)(R + dr));
+    if (f32 && R % 4 == 0 && dr % 4 == 0 && rs % 4 == 0 && ((uintptr_t)cache & 15) == 0)
+        hipLaunchKernelGGL((latent_decode_any_kernel<float, 4>), grid, dim3(64), (size_t)(R + dr) * 4, s, a, (int)(R + dr));
+    else if (f32) hipLaunchKernelGGL((latent_decode_any_kernel<float, 1>), grid, dim3(64), (size_t)(R + dr) * 4, s, a, (int)(R + dr));
+    else hipLaunchKernelGGL((latent_decode_any_kernel<uint16_t, 1>), grid, dim3(64), (size_t)(R + dr) * 4, s, a, (int)(R + dr));
     return evo_launch_status();
 }
 

@@ -456,13 +456,15 @@ extern "C" int evo_rglru_step_bf16(const void* z, int64_t ld, const void* in_b, 
 }
 
 // ------------------------------------------------------------------------------------------------ any sizes, both storage types
-// gates: four tokens of one block per workgroup; -> ab [M][2][W] = (a, sqrt(1 - a^2) i u)
-template <typename T>
+// gates: NT tokens of one block per workgroup; -> ab [M][2][W] = (a, sqrt(1 - a^2) i u).  A thread takes a channel's two rows of weights, V elements a request,
+// for NT tokens at once: 16 of a prompt (1,151 tokens x 16 blocks of 256: 628 us at four tokens and one element a request, 226
+// now), four of a decode step.
+template <typename T, int NT, int V>
 __global__ __launch_bounds__(256) void rglru_gates_any_kernel(RgArgs a, float* __restrict__ ab, int M) {
-    extern __shared__ float us[];                                // [4][bs]
-    const int n = blockIdx.y, m0 = blockIdx.x * 4, bs = a.bs, W = a.W, nt = M - m0 < 4 ? M - m0 : 4;
-    for (int it = threadIdx.x; it < 4 * bs; it += 256) {
-        const int i = it / bs, c = n * bs + it % bs, m = m0 + (i < nt ? i : nt - 1);
+    extern __shared__ __attribute__((aligned(16))) float us[];   // [bs][NT]
+    const int n = blockIdx.y, m0 = blockIdx.x * NT, bs = a.bs, W = a.W, nt = M - m0 < NT ? M - m0 : NT;
+    for (int it = threadIdx.x; it < NT * bs; it += 256) {
+        const int i = it / bs, k = it - i * bs, c = n * bs + k, m = m0 + (i < nt ? i : nt - 1);
         const int b = a.seq ? a.seq[m] : m, t = a.cu ? m - a.cu[b] : 0;      // t: tokens of this portion before this one
         const bool go_on = !a.cu || (a.resume && a.resume[b]);
         const int64_t p = a.pos[m];
@@ -475,26 +477,39 @@ __global__ __launch_bounds__(256) void rglru_gates_any_kernel(RgArgs a, float* _
             else if (go_on && p - back >= 0) x = a.state[((int64_t)b * (1 + a.taps) + 1 + (p - back) % a.taps) * W + c];
             u = fmaf(ld1(cw + a.taps - 1 - back), x, u);
         }
-        us[it] = u;
+        us[k * NT + i] = u;
     }
     __syncthreads();
     for (int c = threadIdx.x; c < bs; c += 256) {
         const int wc = n * bs + c;
         const T *wr = (const T*)a.ra + (int64_t)wc * bs, *wi = (const T*)a.ri + (int64_t)wc * bs;
-        float zr[4], zi[4];
+        float zr[NT], zi[NT];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { zr[i] = ld1((const T*)a.ra_b + wc); zi[i] = ld1((const T*)a.ri_b + wc); }
-        for (int k = 0; k < bs; ++k) {
-            const float p = ld1(wr + k), q = ld1(wi + k);
+        for (int i = 0; i < NT; ++i) { zr[i] = ld1((const T*)a.ra_b + wc); zi[i] = ld1((const T*)a.ri_b + wc); }
+        for (int k0 = 0; k0 < bs; k0 += V) {
+            float p[V], q[V];
+            if constexpr (V == 4) {
+                const f32x4_t x = *(const f32x4_t*)(wr + k0), y = *(const f32x4_t*)(wi + k0);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) { zr[i] = fmaf(p, us[i * bs + k], zr[i]); zi[i] = fmaf(q, us[i * bs + k], zi[i]); }
+                for (int e = 0; e < 4; ++e) { p[e] = x[e]; q[e] = y[e]; }
+            } else { p[0] = ld1(wr + k0); q[0] = ld1(wi + k0); }
+#pragma unroll
+            for (int e = 0; e < V; ++e)
+#pragma unroll
+                for (int i4 = 0; i4 < NT; i4 += 4) {
+                    const f32x4_t u = *(const f32x4_t*)(us + (k0 + e) * NT + i4);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) { zr[i4 + i] = fmaf(p[e], u[i], zr[i4 + i]); zi[i4 + i] = fmaf(q[e], u[i], zi[i4 + i]); }
+                }
         }
-        for (int i = 0; i < nt; ++i) {
-            const float l = a.decay[wc] / (1.0f + expf(-zr[i]));
-            float* d = ab + (int64_t)(m0 + i) * 2 * W + wc;
-            d[0] = expf(l);
-            d[W] = sqrtf(-expm1f(2.0f * l)) / (1.0f + expf(-zi[i])) * us[i * bs + c];
-        }
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+            if (i < nt) {
+                const float l = a.decay[wc] / (1.0f + expf(-zr[i]));
+                float* d = ab + (int64_t)(m0 + i) * 2 * W + wc;
+                d[0] = expf(l);
+                d[W] = sqrtf(-expm1f(2.0f * l)) / (1.0f + expf(-zi[i])) * us[c * NT + i];
+            }
     }
 }
 
@@ -525,11 +540,15 @@ extern "C" int evo_rglru_any(const void* z, int64_t ld, const void* in_b, void* 
     RgArgs a = {z, in_b, o, state, nullptr, conv, conv_b, ra, ra_b, ri, ri_b, decay, pos, seq, cu, resume,
                 ld, (int)W, (int)nb, (int)(W / nb), (int)taps, 1, 0, 1, (int)act, (int)B};
     hipStream_t s = (hipStream_t)stream;
-    const dim3 g1((unsigned)((M + 3) / 4), (unsigned)nb), g2((unsigned)((W + 63) / 64), (unsigned)B), g3((unsigned)((W + 255) / 256), (unsigned)B);
-    const size_t lds = (size_t)(W / nb) * 16;                    // (<= 64 KB)
+    const bool vec = f32 && (W / nb) % 4 == 0 && (((uintptr_t)ra | (uintptr_t)ri) & 15) == 0;
+    const int nt = vec && M >= 64 && W / nb <= 512 ? 16 : 4;
+    const dim3 g1((unsigned)((M + nt - 1) / nt), (unsigned)nb), g2((unsigned)((W + 63) / 64), (unsigned)B), g3((unsigned)((W + 255) / 256), (unsigned)B);
+    const size_t lds = (size_t)(W / nb) * nt * 4;                // (<= 64 KB)
 #define RA(T)                                                                                                              \
     do {                                                                                                                   \
-        hipLaunchKernelGGL((rglru_gates_any_kernel<T>), g1, dim3(256), lds, s, a, ab, (int)M);                             \
+        if (vec && nt == 16) hipLaunchKernelGGL((rglru_gates_any_kernel<float, 16, 4>), g1, dim3(256), lds, s, a, ab, (int)M);    \
+        else if (vec) hipLaunchKernelGGL((rglru_gates_any_kernel<float, 4, 4>), g1, dim3(256), lds, s, a, ab, (int)M);     \
+        else hipLaunchKernelGGL((rglru_gates_any_kernel<T, 4, 1>), g1, dim3(256), lds, s, a, ab, (int)M);                  \
         hipLaunchKernelGGL((rglru_scan_any_kernel<T>), g2, dim3(64), 0, s, a, (const float*)ab);                           \
         if (state) hipLaunchKernelGGL((rglru_tail_kernel<T>), g3, dim3(256), 0, s, a);                                     \
     } while (0)

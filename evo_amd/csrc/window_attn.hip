@@ -297,6 +297,155 @@ __global__ __launch_bounds__(64 * NW, MINW) void window_attn_kernel(WinArgs a, i
     }
 }
 
+// fp32 on the matrix cores (v_mfma_f32_16x16x4_f32: fp32 operands and sums).  A workgroup: 64 queries of one (sequence, head), 16 a wave as MFMA columns;
+// 32 keys at a time in LDS, the rows of K and V 4 floats apart from a multiple of 64 (both read patterns meet every bank once).  Scores come as
+// S^T = K Q^T with the reduced index taken as d = 16 s + 4 g + j (a lane's four d are one 16-byte read), a lane holds keys 4 g + r of its query, which is
+// the operand of O^T = V^T P^T when that product's key index is taken in the same order.  MAPS == 2: the two maps are two column blocks.
+// Bound by the fp32 matrix rate (256 flop a cycle and CU) at length, by its 2 - 16 key tiles at the sizes of a checked trace.  The wave-per-query form
+// below read every key row once per query with one lane a key: 3 prompts of 240 - 500 tokens x 32 heads of 192 x 128 took 5,080 us (139 here),
+// 16 heads of two maps 128 x 256 4,292 us (280 here).
+template <int KS, int DVB, int MAPS>
+__global__ __launch_bounds__(256, 1) void window_attn_f32_kernel(WinArgs a) {
+    constexpr int DQ = 16 * KS, PK = MAPS * DQ + 4, DVP = 16 * DVB, PV = DVP + 4, KT = 32;
+    __shared__ __attribute__((aligned(16))) float ks[KT * PK], vs[KT * PV];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c16 = lane & 15, g = lane >> 4;
+    const int h = blockIdx.y, b = blockIdx.z;
+    const int q0 = a.cu_q[b], nq = a.cu_q[b + 1] - q0, k0 = a.cu_k[b], nk = a.cu_k[b + 1] - k0;
+    const int qb = blockIdx.x * 64;
+    if (qb >= nq) return;
+    const int off = nk - nq, dh = a.dn + a.dr, hk = h / a.grp;
+    const float* kr = (const float*)a.kr + (int64_t)k0 * a.dr;
+    const float* kn = (const float*)a.kn + (int64_t)k0 * a.ldkv + (int64_t)hk * a.dn * MAPS;
+    const float* vg = (const float*)a.v + (int64_t)k0 * a.ldkv + (int64_t)hk * a.dv;
+    const int i = qb + 16 * wave + c16, ki = i + off;            // this lane's query, as a row and as a key
+    f32x4_t qf[MAPS][KS];
+#pragma unroll
+    for (int map = 0; map < MAPS; ++map) {
+        const float* q = (const float*)a.q + (int64_t)(q0 + (i < nq ? i : nq - 1)) * a.ldq + (int64_t)(h * MAPS + map) * dh;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            const int d = 16 * s + 4 * g;
+            qf[map][s] = d < dh ? *(const f32x4_t*)(q + d) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    f32x4_t o[MAPS][DVB];
+    float m[MAPS], l[MAPS];
+#pragma unroll
+    for (int map = 0; map < MAPS; ++map) {
+        m[map] = a.sink ? a.sink[h] : -INFINITY;
+        l[map] = a.sink && g == 0 ? 1.0f : 0.0f;                 // (the lanes of a query hold parts of its sum)
+#pragma unroll
+        for (int e = 0; e < DVB; ++e) o[map][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    const int last = (qb + 63 < nq - 1 ? qb + 63 : nq - 1) + off;
+    const int lo = qb + off - a.window + 1 > 0 ? qb + off - a.window + 1 : 0, kept = a.keep < lo ? a.keep : lo;
+    for (int part = kept > 0 ? 0 : 1; part < 2; ++part)          // the kept keys ahead of every window, then the windows
+        for (int j0 = part ? lo : 0, end = part ? last + 1 : kept; j0 < end; j0 += KT) {
+            __syncthreads();
+            for (int e = tid; e < KT * (MAPS * DQ / 4); e += 256) {
+                const int r = e / (MAPS * DQ / 4), c = (e - r * (MAPS * DQ / 4)) * 4, map = c / DQ, d = c - map * DQ, j = j0 + r;
+                f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+                if (j < end) {
+                    if (d < a.dn) v = *(const f32x4_t*)(kn + j * a.ldkv + map * a.dn + d);
+                    else if (d < dh) v = *(const f32x4_t*)(kr + (int64_t)j * a.dr + (d - a.dn));
+                }
+                *(f32x4_t*)(ks + r * PK + c) = v;
+            }
+            int odd = 0;                                         // an infinite value or none: it may only reach the queries that see its key
+            for (int e = tid; e < KT * (DVP / 4); e += 256) {
+                const int r = e / (DVP / 4), d = (e - r * (DVP / 4)) * 4, j = j0 + r;
+                const f32x4_t v = j < end && d < a.dv ? *(const f32x4_t*)(vg + j * a.ldkv + d) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+                *(f32x4_t*)(vs + r * PV + d) = v;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) odd |= !(fabsf(v[u]) <= 3.402823466e38f);
+            }
+            odd = __syncthreads_or(odd);
+#pragma unroll
+            for (int map = 0; map < MAPS; ++map) {
+                f32x4_t p[2];
+                float top = -INFINITY;
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    p[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                    const float* kp = ks + (16 * t + c16) * PK + map * DQ + 4 * g;
+#pragma unroll
+                    for (int s = 0; s < KS; ++s) {
+                        const f32x4_t kv = *(const f32x4_t*)(kp + 16 * s);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) p[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[j], qf[map][s][j], p[t], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int j = j0 + 16 * t + 4 * g + r;
+                        const bool seen = j < end && j <= ki && (ki - j < a.window || j < a.keep);
+                        p[t][r] = seen ? p[t][r] * a.scale : -INFINITY;
+                        top = fmaxf(top, p[t][r]);
+                    }
+                }
+                top = fmaxf(top, __shfl_xor(top, 16, 64));
+                top = fmaxf(fmaxf(top, __shfl_xor(top, 32, 64)), m[map]);
+                const float base = top == -INFINITY ? 0.f : top, f = expf(m[map] - base);      // (no key seen yet: everything stays zero)
+                m[map] = top;
+                float sum = 0.f;
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) { p[t][r] = expf(p[t][r] - base); sum += p[t][r]; }
+                l[map] = l[map] * f + sum;
+                if (odd) {
+#pragma unroll
+                    for (int e = 0; e < DVB; ++e) o[map][e] *= f;
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            for (int u = 0; u < 4; ++u) {
+                                const int row = 16 * t + 4 * u + r, j = j0 + row;
+                                const float pj = __shfl(p[t][r], 16 * u + c16, 64);
+                                if (j < end && j <= ki && (ki - j < a.window || j < a.keep))
+#pragma unroll
+                                    for (int e = 0; e < DVB; ++e) o[map][e] += pj * *(const f32x4_t*)(vs + row * PV + 16 * e + 4 * g);
+                            }
+                } else
+#pragma unroll
+                for (int e = 0; e < DVB; ++e) {
+                    o[map][e] *= f;
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            o[map][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vs[(16 * t + 4 * g + r) * PV + 16 * e + c16], p[t][r], o[map][e], 0, 0, 0);
+                }
+            }
+        }
+#pragma unroll
+    for (int map = 0; map < MAPS; ++map) {
+        l[map] += __shfl_xor(l[map], 16, 64);
+        l[map] += __shfl_xor(l[map], 32, 64);
+#pragma unroll
+        for (int e = 0; e < DVB; ++e) o[map][e] /= l[map];
+    }
+    float gain = 1.0f;
+    if constexpr (MAPS == 2) {
+        float ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < DVB; ++e) {
+            o[0][e] -= a.lam * o[1][e];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) ss = fmaf(o[0][e][r], o[0][e][r], ss);      // (columns behind dv are zero)
+        }
+        ss += __shfl_xor(ss, 16, 64);
+        ss += __shfl_xor(ss, 32, 64);
+        gain = a.gain / sqrtf(ss / (float)a.dv + a.eps);
+    }
+    if (i < nq) {
+        float* op = (float*)a.o + (int64_t)(q0 + i) * a.H * a.dv + (int64_t)h * a.dv + 4 * g;
+#pragma unroll
+        for (int e = 0; e < DVB; ++e)
+            if (16 * e + 4 * g < a.dv) *(f32x4_t*)(op + 16 * e) = o[0][e] * gain;
+    }
+}
+
 // Any sizes, both storage types: one wave per (query, head); lanes are keys for the scores, value columns for the sum
 template <typename T, int MAPS>
 __global__ __launch_bounds__(64) void window_attn_any_kernel(WinArgs a) {
@@ -407,6 +556,20 @@ extern "C" int evo_window_attn(const void* q, int64_t ldq, const void* kn, const
 #undef WA
 #undef WAN
 #undef WA1
+        return evo_launch_status();
+    }
+    if (f32 && mfma && dq <= (maps == 2 ? 128 : 256) && dv <= 256 && dn % 4 == 0 && dr % 4 == 0 && dv % 4 == 0 && ldq % 4 == 0 && ldkv % 4 == 0 &&
+        (((uintptr_t)q | (uintptr_t)kn | (uintptr_t)v | (uintptr_t)kr | (uintptr_t)o) & 15) == 0) {
+        const dim3 fgrid((unsigned)((max_q + 63) / 64), (unsigned)H, (unsigned)B);
+#define WF(KS, DVB, MAPS) hipLaunchKernelGGL((window_attn_f32_kernel<KS, DVB, MAPS>), fgrid, dim3(256), 0, s, a)
+#define WFV(KS, MAPS) do { if (dv <= 64) WF(KS, 4, MAPS); else if (dv <= 128) WF(KS, 8, MAPS); else WF(KS, 16, MAPS); } while (0)
+        if (maps == 2) { if (dq <= 64) WFV(4, 2); else WFV(8, 2); }
+        else if (dq <= 64) WFV(4, 1);
+        else if (dq <= 128) WFV(8, 1);
+        else if (dq <= 192) WFV(12, 1);
+        else WFV(16, 1);
+#undef WFV
+#undef WF
         return evo_launch_status();
     }
     const dim3 grid((unsigned)max_q, (unsigned)H, (unsigned)B);
