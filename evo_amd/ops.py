@@ -536,7 +536,7 @@ class HipOps(MixerOps):
         return flat.view(C, P // 256, 256).permute(1, 0, 2).contiguous()
 
     def hyena_ct(self, zt, B, T, fir_w, fir_b, table, n_heads, z_halo=None, s0=None, want_state=False, poles=None,
-                 state_only=False, b_first=0, y_blk=None, y_row0=0, b_total=None, main_only=False):
+                 state_only=False, b_first=0, y_blk=None, y_row0=0, b_total=None, main_only=False, at=None, s_out=None):
         """The channel-stationary single-pass operator on CHANNEL-MAJOR z (csrc/hyena_ct.hip: evo_hyena_ct): zt [blocks, 3 D, 256] bf16 =
         linear_t's result (zt_layout of a [b_total, T] batch; b_total defaults to b_first + B); B batch rows of T tokens starting at
         batch row `b_first` of the tensor (a sub-range).  -> y [B,T,D] bf16 | (y, end state [B,D,8] complex64) with `want_state` | the end state alone with `state_only` (stage 1 of a
@@ -546,13 +546,17 @@ class HipOps(MixerOps):
         `main_only` (tail form of zt_layout only): the operator walks the Tm = 512 k main tokens of every row -- whole tiles -- and leaves
         rows b T + Tm .. of y untouched; with `want_state` the state returned is the one after token Tm - 1: the caller finishes the r
         tail tokens with the single-token launch (hyena_decode_fused / hyena_step) from that state (StripedHyena._hyena_block; a ragged
-        tile with one valid step costs the kernel a full tile's issue time: 8 of 136 tile steps at 8 x 8,193)."""
+        tile with one valid step costs the kernel a full tile's issue time: 8 of 136 tile steps at 8 x 8,193).
+        `at`: ONE sequence of T tokens whose first sits at position `at` (a multiple of 8) of z^T, whatever else z^T holds (prompts packed
+        behind each other); its end state goes to `s_out` [1, D, 8] complex64 where that is given."""
         self._need(zt, torch.bfloat16, "hyena z^T")
         assert zt.dim() == 3 and zt.shape[2] == 256
         D3, P = zt.shape[1], zt.shape[0] * 256
         D = D3 // 3
-        Tm, Tp, Mp, r = self.zt_layout(b_first + B if b_total is None else b_total, T)
+        Tm, Tp, Mp, r = self.zt_layout(b_first + B if b_total is None else b_total, T) if at is None else (T, (T + 7) // 8 * 8, P, 0)
         assert D3 == 3 * D and (b_first + B) * Tp <= Mp
+        if at is not None:
+            assert B == 1 and b_first == 0 and not main_only and at % 8 == 0 and 0 <= at and at + Tp <= P
         if main_only:
             assert r > 0 and P in (Mp, Mp + 256) and z_halo is None and s0 is None and not state_only
         else:
@@ -575,7 +579,11 @@ class HipOps(MixerOps):
                 raise RuntimeError("hyena_ct: the end state needs the poles")
             self._need(poles, torch.float32, "hyena poles")
             assert tuple(poles.shape) == (D, 8, 2)
-            s_fin = torch.empty(B, D, 8, 2, dtype=torch.float32, device=zt.device)
+            if s_out is not None:
+                assert s_out.dtype == torch.complex64 and tuple(s_out.shape) == (B, D, 8) and s_out.is_contiguous() and s_out.device == zt.device
+                s_fin = torch.view_as_real(s_out)
+            else:
+                s_fin = torch.empty(B, D, 8, 2, dtype=torch.float32, device=zt.device)
         yb_rows = 0
         if state_only:
             y = None
@@ -589,7 +597,7 @@ class HipOps(MixerOps):
             y = torch.empty(B, T, D, dtype=torch.bfloat16, device=zt.device)
         with self._t("hyena_mfma_state" if state_only else "hyena_mfma"):
             _check(self.lib.evo_hyena_ct(zt.data_ptr(), _ptr(z_halo), fir_w.data_ptr(), fir_b.data_ptr(), table.data_ptr(), _ptr(y),
-                                         _ptr(s0r), _ptr(s_fin), _ptr(poles), B, T_run, D, n_heads, P, Tp, b_first * Tp,
+                                         _ptr(s0r), _ptr(s_fin), _ptr(poles), B, T_run, D, n_heads, P, Tp, b_first * Tp if at is None else at,
                                          Tm if r and not main_only else 0, Mp + 8 * b_first, 1 if state_only else 0, yb_rows, y_row0,
                                          T if main_only else 0, _stream()),
                    "evo_hyena_ct")
@@ -905,7 +913,8 @@ class HipOps(MixerOps):
                                                     float(scaling), B, H, hd, kv.stride(0), kv.stride(1), kv.stride(2),
                                                     kv.stride(3), float(q_scale), _stream()), "evo_rope_append_decode_bf16")
 
-    def attention(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_pos0: int, prescaled: bool = False) -> torch.Tensor:
+    def attention(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_pos0: int, prescaled: bool = False,
+                  out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Causal attention; q [B,Tq,H,128], k/v [B,Tk,H,128] (strided views allowed, last dim dense).  `prescaled`: q already carries
         softmax_scale * log2(e) (rope_'s q_scale = attn_q_scale(hd)): the 64-rows-per-wave kernel then runs without its per-score multiply."""
         for t, nm in ((q, "q"), (k, "k"), (v, "v")):
@@ -915,7 +924,10 @@ class HipOps(MixerOps):
         Tk = k.shape[1]
         if hd != 128:
             raise RuntimeError("attention: head dim must be 128")
-        o = torch.empty(B, Tq, H, hd, dtype=torch.bfloat16, device=q.device)
+        if out is not None:
+            self._need(out, torch.bfloat16, "attention out")
+            assert tuple(out.shape) == (B, Tq, H, hd)
+        o = torch.empty(B, Tq, H, hd, dtype=torch.bfloat16, device=q.device) if out is None else out
         # query ranges longer than one 128-row block: the 64-rows-per-wave kernel, which reads V^T from a workspace its pre-pass fills
         vt = torch.empty(B, H, hd, (Tk + 63) // 64 * 64, dtype=torch.bfloat16, device=q.device) if (Tq > 128 and self.attn_w64) else None
         with self._t("attn_fwd"):

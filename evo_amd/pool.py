@@ -10,9 +10,8 @@ attention all read per-row positions (`evo_attn_decode_bf16` dyn_pos[B]), so str
 and different ages advance together, a finished stream's slot is re-filled while the others keep going, and the
 step has one shape for the whole job -- it is captured once in a hipGraph and replayed.
 
-Prompts are prefilled with the model's ordinary parallel forward (`model.prefill_rows`): one prompt per pass on StripedHyena, whose
-long-convolution kernel ends with the exact modal state; all prompts that find a slot as one packed pass on models that take unequal
-lengths together.  The `n_sample_per_prompt` copies of a prompt share ONE prefill, whose caches are replicated into their slots.  The
+Prompts are prefilled with the model's parallel launches (`model.prefill_rows`), all prompts that find a slot as one packed pass where they
+can share one; StripedHyena's long-convolution kernel ends every prompt with its exact modal state.  The `n_sample_per_prompt` copies of a prompt share ONE prefill, whose caches are replicated into their slots.  The
 pool's own steps -- admit, advance, release -- serve callers that bring their own tokens (evo_amd/trace.py).
 
 Sampling and scoring follow the reference wrapper verbatim (same `sample`, same shifted logits/token pairing

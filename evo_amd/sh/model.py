@@ -884,17 +884,110 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             row = dst["hyena"].state_dict[i][dst_row]
             row.copy_(src["hyena"].state_dict[i][src_row].reshape(row.shape))
 
+    packs_prompts = True         # prefill_rows runs unequal prompts as one pass
+    packed_rows = 64 * 1024      # rows of one such pass
+
+    def _prompt_groups(self, lens: List[int]) -> List[List[int]]:
+        """Prompts that share a pass: those of 32 to 4,096 tokens, as many as fit, when the matrix-core operator takes every Hyena layer.  (Shorter
+        ones take the modal kernels; longer ones fill the dense layers by themselves.)"""
+        if not self._packed:
+            self._pack()
+        ops = self.ops
+        ok = (self.device.type == "cuda" and getattr(ops, "hyena_mfma", False) and getattr(ops, "hyena_ct_flag", False) and hasattr(ops, "hyena_ct")
+              and self.hidden_size == self.num_heads * 128 and ops.zt_shape_ok(1, self.packed_rows, 3 * self.hidden_size, self.hidden_size) and getattr(self, "block_taps", None) is None
+              and all(isinstance(b, _AttentionBlock) or (b.projections.weight.is_contiguous() and b.projections.weight.dtype == torch.bfloat16
+                                                         and self._table_ok(b)) for b in self.blocks))
+        groups, rows = [], 0
+        for n, m in enumerate(lens):
+            need = (m + 63) // 64 * 64
+            share = ok and 32 <= m <= 4096
+            if share and rows and rows + need <= self.packed_rows:
+                groups[-1].append(n)
+                rows += need
+            else:
+                groups.append([n])
+                rows = need if share else 0
+        return groups
+
+    def _prefill_packed(self, prompts: List[torch.Tensor]):
+        """Prompts behind each other as ONE stream of rows, each from a multiple of 64 on (the rows between are token 0 and reach nobody: every
+        launch is row-independent or runs on one prompt's rows): the dense layers see all rows at once, the Hyena operator and the attention walk
+        the prompts one by one.  -> (final-norm rows, first row of every prompt, caches with a row per prompt)."""
+        ops, D, H, hd, K1 = self.ops, self.hidden_size, self.num_heads, self.head_dim, self.short_filter_length - 1
+        dev, lens = self.device, [p.numel() for p in prompts]
+        first, M = [], 0
+        for m in lens:
+            first.append(M)
+            M += (m + 63) // 64 * 64
+        M = (M + 255) // 256 * 256
+        ids = torch.zeros(M, dtype=torch.int64)
+        pos = torch.zeros(M, dtype=torch.int64)
+        ends = torch.tensor([f + m - K1 + j for f, m in zip(first, lens) for j in range(K1)])
+        for f, m in zip(first, lens):
+            pos[f:f + m] = torch.arange(m)
+        ids, pos, ends = ids.to(dev), pos.to(dev), ends.to(dev)
+        for p, f, m in zip(prompts, first, lens):
+            ids[f:f + m] = p.reshape(-1).to(dev)
+        cos, sin = (t[pos] for t in self._rotary(0, max(lens), dev)) if self.attn_layer_idxs else (None, None)
+        pre = bool(getattr(ops, "attn_prescale", False)) and hasattr(ops, "attn_q_scale")
+        ipd = self.initialize_inference_params()
+        ipd["mha"].max_batch_size = ipd["hyena"].max_batch_size = len(lens)
+        ipd["mha"].max_seqlen = max(lens)
+        kvs, hy = ipd["mha"].key_value_memory_dict, ipd["hyena"]
+        x = ops.embed(ids, self.embedding_layer.weight)
+        yb = ops.yblk_empty(M, D, dev).zero_()                     # (the rows between the prompts stay zero)
+        nf, rs = self._nf_ok(M, None), None
+        for i, blk in enumerate(self.blocks):
+            if isinstance(blk, _AttentionBlock):
+                mha = blk.inner_mha_cls
+                if nf and rs is not None:
+                    wqkv_f = self._folded(mha, "_wqkv_f", mha.Wqkv.weight, blk.pre_norm.scale)
+                    qkv = ops.linear_rs(x, rs, wqkv_f, mha.Wqkv.bias, mha.Wqkv.weight, blk.pre_norm.scale, self.eps)
+                else:
+                    qkv = ops.norm_linear(x, blk.pre_norm.scale, self.eps, mha.Wqkv.weight, mha.Wqkv.bias, mfma=True)
+                qkv = qkv.view(1, M, 3, H, hd)
+                ops.rope_(qkv, cos, sin, **({"q_scale": ops.attn_q_scale(hd)} if pre else {}))
+                kv = kvs[i] = torch.zeros(len(lens), max(lens), 2, H, hd, dtype=qkv.dtype, device=dev)
+                y, bias, w = torch.zeros(M, D, dtype=qkv.dtype, device=dev), mha.out_proj.bias, mha.out_proj.weight
+                for n, (f, m) in enumerate(zip(first, lens)):
+                    z = qkv[:, f:f + m]
+                    kv[n, :m].copy_(z[0, :, 1:3])
+                    ops.attention(z[:, :, 0], z[:, :, 1], z[:, :, 2], 0, out=y[f:f + m].view(1, m, H, hd), **({"prescaled": True} if pre else {}))
+            else:
+                f_, pb = blk.filter, None if blk.projections.bias is None else blk.projections.bias.data
+                if nf and rs is not None:
+                    wp_f = self._folded(blk, "_wp_f", blk.projections.weight, blk.pre_norm.scale)
+                    zt = ops.linear_t_rs(x, rs, wp_f, pb, blk.projections.weight.data, blk.pre_norm.scale, self.eps, 1, M)
+                else:
+                    zt = ops.linear_t(ops.rmsnorm(x, None, blk.pre_norm.scale, self.eps), blk.projections.weight.data, pb, 1, M)
+                table = self._mfma_table(blk)
+                state = hy.state_dict[i] = torch.empty(len(lens), D, self.state_size, dtype=torch.complex64, device=dev)
+                for n, (f, m) in enumerate(zip(first, lens)):
+                    ops.hyena_ct(zt, 1, m, f_._fir_w, f_.short_filter_bias, table, H, want_state=True, poles=f_._poles, y_blk=yb, y_row0=f, at=f,
+                                 s_out=state[n:n + 1])
+                hy.fir_state_dict[i] = zt[ends // 256, :, ends % 256].view(len(lens), K1, 3 * D).transpose(1, 2).contiguous()
+                y, bias, w = yb, blk.out_filter_dense.bias, blk.out_filter_dense.weight
+            if nf:
+                rs = self._mlp_residual_rs_(blk, x, self._mixer_out_rs_(blk, x, y, w, bias))
+            else:
+                self._mlp_residual_(blk, x, self._mixer_out_(blk, x, y, w, bias, mfma=True), None)
+        return (x if self.norm is None else ops.rmsnorm(x, None, self.norm.scale, self.eps)), first, ipd
+
     def prefill_rows(self, prompts: List[torch.Tensor], want: Optional[List[List[int]]] = None):
-        """Each prompt ([P] ids) in one parallel pass of its own -> [(logits [wanted, V], caches, row of the caches)]; `want`: the places
-        whose logits are returned (the last token's by default)."""
+        """Prompts ([P] ids) of any lengths -> [(logits [wanted, V], caches, row of the caches)], several in a pass where they can share one
+        (_prompt_groups); `want`: the places whose logits are returned (the last token's by default)."""
         out = []
-        for n, ids in enumerate(prompts):
-            ipd = self.initialize_inference_params()
-            ipd["mha"].max_seqlen = ids.numel()
-            h = self.hidden_states(ids.reshape(1, -1), ipd)
-            at = torch.tensor([ids.numel() - 1] if want is None else want[n], dtype=torch.int64, device=h.device)
-            out.append((self.ops.linear(h[at].contiguous(), self.unembed.weight, None) if at.numel() else
-                        h.new_empty(0, self.vocab_size), ipd, 0))
+        for group in self._prompt_groups([p.numel() for p in prompts]):
+            if len(group) > 1:
+                h, first, ipd = self._prefill_packed([prompts[n] for n in group])
+            else:
+                ipd = self.initialize_inference_params()
+                ipd["mha"].max_seqlen = prompts[group[0]].numel()
+                h, first = self.hidden_states(prompts[group[0]].reshape(1, -1), ipd), [0]
+            at = [[prompts[n].numel() - 1] if want is None else list(want[n]) for n in group]
+            rows = torch.tensor([f + t for f, ts in zip(first, at) for t in ts], dtype=torch.int64, device=h.device)
+            logits = self.ops.linear(h[rows].contiguous(), self.unembed.weight, None) if rows.numel() else h.new_empty(0, self.vocab_size)
+            out += [(lg, ipd, row) for row, lg in enumerate(logits.split([len(ts) for ts in at]))]
         return out
 
     # upstream names, kept for callers that reach for them
