@@ -992,6 +992,121 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_n_kernel(const uint4* __res
     }
 }
 
+// ---- 5 <= M <= 32 on the narrow layers (N < 8192: a workgroup per 16 columns is about one per CU): the k-split form with whole row pieces.  A workgroup =
+// 16 weight rows; its waves take every WAVES-th chunk of CH k and park weight and batch rows of a chunk in a PRIVATE part of LDS (asynchronous loads of
+// 1 KiB = whole row pieces of 2 CH bytes, no registers, no barrier), NB chunks in flight; the WAVES partial tiles meet in LDS at the end.  Granule g of a
+// row sits at slot g ^ (row & 15): a fragment read meets no bank twice.
+// Bound by the weight stream and, at K = 4,096, by a launch's ramp: 4.3 - 4.7 TB/s at 8 rows; the fragment-shaped requests of skinny_mfma_kernel (64 bytes
+// of each of 16 rows) ran at 2.7 - 3.5.
+// XR: batch rows loaded (8, 16 or 32; rows behind M read as zero or are a repeated row, and are never stored).
+#define KW_WAIT(N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory")
+template <int XR, int WAVES, int CH, int NB>
+__global__ __launch_bounds__(64 * WAVES) void skinny_kw_kernel(const unsigned char* __restrict__ x, const unsigned char* __restrict__ w,
+                                                               const uint16_t* __restrict__ bias, const uint16_t* res, uint16_t* y, int M, int N, int K,
+                                                               int act) {   // res may alias y
+    constexpr int MT = XR > 16 ? 2 : 1, ROW = 2 * CH, RPI = 1024 / ROW, GR = ROW / 16;      // bytes of a row piece, rows per request, granules per row piece
+    constexpr int PW = 16 / RPI, PX = XR / RPI, P = PW + PX, BUF = (16 + XR) * ROW;
+    extern __shared__ __attribute__((aligned(16))) unsigned char kw_lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, kb = lane >> 4;
+    const int n0 = blockIdx.x * 16;
+    const uint32_t rowb = (uint32_t)K * 2;
+    const uint64_t wa = (uint64_t)w + (uint64_t)n0 * rowb, xa = (uint64_t)x;
+    const uint32_t wn = (uint32_t)(N - n0 < 16 ? N - n0 : 16);
+    typedef uint32_t kw_u32x4 __attribute__((ext_vector_type(4)));
+    const kw_u32x4 rw = {(uint32_t)wa, (uint32_t)(wa >> 32) & 0xffffu, wn * rowb, 0x00020000u};
+    const kw_u32x4 rx = {(uint32_t)xa, (uint32_t)(xa >> 32) & 0xffffu, (uint32_t)M * rowb, 0x00020000u};
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)kw_lds + wave * (NB * BUF);
+    uint32_t off[PX > PW ? PX : PW];
+#pragma unroll
+    for (int i = 0; i < (PX > PW ? PX : PW); ++i) {
+        const int r = i * RPI + lane / GR;
+        off[i] = (uint32_t)r * rowb + (uint32_t)((lane % GR) ^ (r & 15 & (GR - 1))) * 16u;
+    }
+    const int chunks = K / CH, mine = (chunks - wave + WAVES - 1) / WAVES;
+    auto fetch = [&](int i, uint32_t buf) {
+        const uint32_t so = (uint32_t)(wave + WAVES * i) * ROW;
+#pragma unroll
+        for (int j = 0; j < PW; ++j)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(buf + j * 1024), "v"(off[j]), "s"(rw), "s"(so) : "memory", "m0");
+#pragma unroll
+        for (int j = 0; j < PX; ++j)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(buf + 16 * ROW + j * 1024), "v"(off[j]), "s"(rx), "s"(so) : "memory", "m0");
+    };
+    gv_f32x4 acc[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[t] = gv_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+        if (i < mine) fetch(i, lds0 + i * BUF);
+    uint32_t buf = lds0;
+    const uint32_t wrd = (uint32_t)r16 * ROW;
+    uint32_t xrd[MT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) xrd[t] = 16u * ROW + (uint32_t)((16 * t + r16) & (XR - 1)) * ROW;
+    for (int i = 0; i < mine; ++i) {
+        if (i + NB <= mine) KW_WAIT((NB - 1) * P); else KW_WAIT(0);      // this chunk has landed (the last ones: all of them)
+#pragma unroll
+        for (int h = 0; h < CH / 32; h += 4) {                   // four fragments of 32 k at a time
+            kw_u32x4 wf[4], xf[4][MT];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const uint32_t g = (uint32_t)((4 * (h + u) + kb) ^ (r16 & (GR - 1))) * 16u;
+                asm volatile("ds_read_b128 %0, %1" : "=v"(wf[u]) : "v"(buf + wrd + g));
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    const uint32_t gx = (uint32_t)((4 * (h + u) + kb) ^ (((16 * t + r16) & (XR - 1)) & 15 & (GR - 1))) * 16u;
+                    asm volatile("ds_read_b128 %0, %1" : "=v"(xf[u][t]) : "v"(buf + xrd[t] + gx));
+                }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                asm volatile("" : "+v"(wf[u]));
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    asm volatile("" : "+v"(xf[u][t]));
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[u]), __builtin_bit_cast(bf16x8_t, xf[u][t]), acc[t], 0, 0, 0);
+                }
+            }
+        }
+        if (i + NB < mine) fetch(i + NB, buf);                   // (the chunk has been read: its place takes the next but NB)
+        buf = buf + BUF == lds0 + NB * BUF ? lds0 : buf + BUF;
+    }
+    __syncthreads();                                             // (every wave's loads have landed and been read: the partial tiles go over them)
+    gv_f32x4* part = (gv_f32x4*)kw_lds;
+#pragma unroll
+    for (int t = 0; t < MT; ++t) part[(t * WAVES + wave) * 64 + lane] = acc[t];
+    __syncthreads();
+    if (wave < MT) {
+        gv_f32x4 a_ = part[wave * WAVES * 64 + lane];
+#pragma unroll
+        for (int q = 1; q < WAVES; ++q) a_ += part[(wave * WAVES + q) * 64 + lane];
+        const int m = 16 * wave + r16;
+        if (m < M) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int n = n0 + 4 * kb + r;
+                if (n < N) {
+                    float o = a_[r] + (bias ? bf_to_f(bias[n]) : 0.f);
+                    if (res) o += bf_to_f(res[(int64_t)m * N + n]);
+                    y[(int64_t)m * N + n] = f_to_bf(out_act(o, act));
+                }
+            }
+        }
+    }
+}
+
+template <int XR, int WAVES, int CH, int NB>
+static int kw_launch(const void* x, const void* w, const void* bias, const void* residual, void* y, int64_t M, int64_t N, int64_t K, int act, hipStream_t s) {
+    constexpr size_t lds = (size_t)WAVES * NB * (16 + XR) * 2 * CH;
+    static_assert(lds <= 160 * 1024, "the CU's LDS");
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)skinny_kw_kernel<XR, WAVES, CH, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL((skinny_kw_kernel<XR, WAVES, CH, NB>), dim3((unsigned)((N + 15) / 16)), dim3(64 * WAVES), lds, s, (const unsigned char*)x,
+                       (const unsigned char*)w, (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)K, act);
+    return evo_launch_status();
+}
+
 // ---- the n-split form with CONTIGUOUS weight requests (round 6, second step).  skinny_n_kernel asks for a weight fragment as the MFMA wants it: 64 bytes
 // of each of 16 rows that lie K * 2 bytes apart -- and streams 3.1-3.3 TB/s where the same kernel reading 1 KiB contiguous per request runs 4.3-4.4
 // (profiles/r06_small_m_nsplit_ab.txt).  Here a request covers RPI = 2 (4) whole row pieces of 512 (256) contiguous bytes, the wave parks the chunk in a
@@ -1323,6 +1438,14 @@ extern "C" int evo_linear_small_m_bf16(const void* x, const void* w, const void*
     if ((M > 8 && K % 32 != 0) || (act != 0 && act != 3)) return -1;
     hipStream_t s = (hipStream_t)stream;
     if (M >= 5 && K % 32 == 0) {
+        // narrow layers: whole row pieces through LDS (skinny_kw_kernel).  us before -> now at N = 4,096: K = 4,096 9.7 -> 7.8 at 8 rows, 11.0 -> 9.2 at 16,
+        // 16.1 -> 10.6 at 32; K = 11,008 27.3 -> 19.2, 31.3 -> 20.7, 24.4 -> 24.6 (and one launch less); K = 16,384 39.7 -> 29.8 at 8 -- at 32 rows the split
+        // over K across workgroups below stays ahead there (30.5 against 35.1); N = 6,912, K = 4,096 18.6 -> 13.8, 29.6 -> 17.7; N = 512 8.8 -> 5.7, 14.2 -> 8.1
+        if (N < 8192 && K % 128 == 0 && M <= (K < 12288 ? 32 : 16)) {
+            if (M <= 8) return kw_launch<8, 8, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);
+            if (M <= 16) return kw_launch<16, 8, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);
+            return kw_launch<32, 4, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);
+        }
         // two n tiles per workgroup (every x fragment feeds two weight fragments) where that still leaves a workgroup or more per CU
         static const int nt_env = [] { const char* e = getenv("EVO_SK_NT"); return e ? atoi(e) : 0; }();      // measurement knob: 1 / 2 force, 0 = auto
         const int nt = nt_env ? nt_env : (N >= 8192 && M > 16 ? 2 : 1);
