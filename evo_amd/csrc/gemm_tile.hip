@@ -36,6 +36,31 @@ __device__ __forceinline__ void t_act(float (&v)[8], int act) {
     }
 }
 
+// row factor and bias of eight columns n .. n + 7: one fused step where there are both, as the persistent kernel's epilogue compiles to (the same bits).
+// Mode 3: `rs` the factors of the eight tokens, `rb` the row's bias; else `f` the row's factor.
+template <int MODE>
+__device__ __forceinline__ void t_scale_bias(float (&v)[8], const GemmArgs& a, float f, float rb, const float* rs, int n) {
+    float b[8];
+    if (MODE == 3) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) b[e] = rb;
+    } else if (a.bias) {
+        const uint4 q = *(const uint4*)(a.bias + n);
+        b[0] = bf_lo(q.x); b[1] = bf_hi(q.x); b[2] = bf_lo(q.y); b[3] = bf_hi(q.y);
+        b[4] = bf_lo(q.z); b[5] = bf_hi(q.z); b[6] = bf_lo(q.w); b[7] = bf_hi(q.w);
+    }
+    if (a.rs) {
+        float s[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] = MODE == 3 ? rs[e] : f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = a.bias ? fmaf(v[e], s[e], b[e]) : v[e] * s[e];
+    } else if (a.bias) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] += b[e];
+    }
+}
+
 template <int BM, int BN, int WGM, int WGN, int NS, int PER_CU, int MODE, bool XB, bool SPLIT>
 __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_tile_kernel(GemmArgs a, int act, float* parts, int splits) {
     constexpr int NW = WGM * WGN, WM = BM / WGM, WN = BN / WGN, MT = WM / 16, NT = WN / 16;
@@ -246,14 +271,13 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
         return;
     }
     const bool on = n0 < a.act_cols, stats = STATS && a.ss;
-    float ssum[MT];
+    uint4 kept[STATS ? MT : 1][STATS ? NT / 2 : 1];              // the stored values, for the statistic
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
         const int64_t m = m0 + wm * WM + 16 * j + l15;
         const bool ok = m < a.M;
         const float f = MODE == 0 && a.rs && ok ? a.rs[m] : 1.f;
         const float rb = MODE == 3 && a.bias ? bf_to_f(a.bias[m]) : 0.f;
-        ssum[j] = 0.f;
 #pragma unroll
         for (int b = 0; b < NT / 2; ++b) {
             const int n = n0 + wn * WN + 32 * b + 8 * lq;
@@ -261,19 +285,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 v[e] = acc[2 * b + (e >> 2)][j][e & 3];
-                if (MODE == 0 && a.rs) v[e] *= f;
-                if (MODE == 3 && a.rs) v[e] *= a.rs[src + (n - n0) + e];
             }
-            if constexpr (MODE == 3) {
-                if (a.bias) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) v[e] += rb;
-                }
-            } else if (a.bias) {
-                const uint4 q = *(const uint4*)(a.bias + n);
-                v[0] += bf_lo(q.x); v[1] += bf_hi(q.x); v[2] += bf_lo(q.y); v[3] += bf_hi(q.y);
-                v[4] += bf_lo(q.z); v[5] += bf_hi(q.z); v[6] += bf_lo(q.w); v[7] += bf_hi(q.w);
-            }
+            t_scale_bias<MODE>(v, a, f, rb, MODE == 3 && a.rs ? a.rs + src + (n - n0) : nullptr, n);
             if (MODE == 0 && a.res && ok) {
                 const uint4 q = *(const uint4*)(a.res + m * a.N + n);
                 v[0] += bf_lo(q.x); v[1] += bf_hi(q.x); v[2] += bf_lo(q.y); v[3] += bf_hi(q.y);
@@ -285,29 +298,36 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
                 if constexpr (MODE == 3) *(uint4*)(a.y + (((int64_t)(n >> 8) * a.M + m) << 8) + (n & 255)) = o;
                 else *(uint4*)(a.y + m * a.N + n) = o;
             }
-            if (stats) {
-                const uint32_t d[4] = {o.x, o.y, o.z, o.w};
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { const float lo = bf_lo(d[e]), hi = bf_hi(d[e]); ssum[j] = fmaf(lo, lo, ssum[j]); ssum[j] = fmaf(hi, hi, ssum[j]); }
-            }
+            if constexpr (STATS) kept[j][b] = o;
         }
     }
-    if (stats) {                                                 // a row's 128 columns: four lane groups, then the waves beside each other
-        float* row = (float*)smem;
+    if (stats) {
+        // a row's 128 columns in the order of gemm.hip's epilogue (the same bits): a lane's values of strip after strip, the waves beside each other one
+        // behind the other, then the four lane groups
+        float* part = (float*)smem;                              // [MT rows of tiles][64 lanes] per wave row
         asm volatile("s_barrier" ::: "memory");                  // (every wave is done with the operands)
+        for (int turn = 0; turn < WGN; ++turn) {
+            if (wn == turn) {
 #pragma unroll
-        for (int j = 0; j < MT; ++j) {
-            float t = ssum[j];
-            t += __shfl_xor(t, 16);
-            t += __shfl_xor(t, 32);
-            if (lq == 0) row[wn * BM + wm * WM + 16 * j + l15] = t;
-        }
-        __syncthreads();
-        for (int r = tid; r < BM; r += 64 * NW) {
-            float t = 0.f;
+                for (int j = 0; j < MT; ++j) {
+                    float t = turn ? part[(wm * MT + j) * 64 + lane] : 0.f;
 #pragma unroll
-            for (int c = 0; c < WGN; ++c) t += row[c * BM + r];
-            if (m0 + r < a.ss_ld) a.ss[(int64_t)(n0 >> 7) * a.ss_ld + m0 + r] = t;
+                    for (int b = 0; b < NT / 2; ++b) {
+                        const uint32_t d[4] = {kept[STATS ? j : 0][STATS ? b : 0].x, kept[STATS ? j : 0][STATS ? b : 0].y, kept[STATS ? j : 0][STATS ? b : 0].z,
+                                               kept[STATS ? j : 0][STATS ? b : 0].w};
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) { const float lo = bf_lo(d[e]), hi = bf_hi(d[e]); t = fmaf(lo, lo, t); t = fmaf(hi, hi, t); }
+                    }
+                    if (turn < WGN - 1) part[(wm * MT + j) * 64 + lane] = t;
+                    else {
+                        t += __shfl_xor(t, 16);
+                        t += __shfl_xor(t, 32);
+                        const int64_t m = m0 + wm * WM + 16 * j + l15;
+                        if (lq == 0 && m < a.ss_ld) a.ss[(int64_t)(n0 >> 7) * a.ss_ld + m] = t;
+                    }
+                }
+            }
+            __syncthreads();
         }
     }
 }
@@ -353,26 +373,8 @@ __global__ __launch_bounds__(256) void gemm_parts_kernel(GemmArgs a, int act, co
     }
     float v[8];
     sum(c8, v);
-    if (MODE == 0 && a.rs) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] *= f;
-    }
-    if (MODE == 3 && a.rs) {
-        const int64_t src = c8 + (int64_t)((c8 >> 8) / a.tm_tiles) * a.row_skip;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] *= a.rs[src + e];
-    }
-    if constexpr (MODE == 3) {
-        if (a.bias) {
-            const float rb = bf_to_f(a.bias[m]);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] += rb;
-        }
-    } else if (a.bias) {
-        const uint4 q = *(const uint4*)(a.bias + c8);
-        v[0] += bf_lo(q.x); v[1] += bf_hi(q.x); v[2] += bf_lo(q.y); v[3] += bf_hi(q.y);
-        v[4] += bf_lo(q.z); v[5] += bf_hi(q.z); v[6] += bf_lo(q.w); v[7] += bf_hi(q.w);
-    }
+    t_scale_bias<MODE>(v, a, f, MODE == 3 && a.bias ? bf_to_f(a.bias[m]) : 0.f,
+                       MODE == 3 && a.rs ? a.rs + c8 + (int64_t)((c8 >> 8) / a.tm_tiles) * a.row_skip : nullptr, c8);
     if (MODE == 0 && a.res) {
         const uint4 q = *(const uint4*)(a.res + m * a.N + c8);
         v[0] += bf_lo(q.x); v[1] += bf_hi(q.x); v[2] += bf_lo(q.y); v[3] += bf_hi(q.y);

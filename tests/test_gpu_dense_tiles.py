@@ -124,3 +124,44 @@ def test_without_a_workspace():
     y = torch.empty(M, N, device="cuda", dtype=torch.bfloat16)
     assert ops.lib.evo_dense_bf16(0, 0, 0, x.data_ptr(), w.data_ptr(), None, None, y.data_ptr(), None, None, 0, M, N, K, 0, 0, 0, 0, None, 0, _stream()) == 0
     _close(y, x.double() @ w.double().T)
+
+
+@pytest.mark.parametrize("M", [1024, 1100, 1536, 2304, 3000, 6400])
+def test_same_bits_on_every_tile(M):
+    """From 1,024 rows on a row's result does not depend on the tiles its batch runs on: the persistent kernel's own entries are the yardstick."""
+    from evo_amd.ops import _stream
+    ops, K = _ops(), 1024
+    g, x, w = _data(M, 4096, K, 6)
+    b = torch.randn(4096, device="cuda", generator=g).bfloat16()
+    r = torch.randn(M, 4096, device="cuda", generator=g).bfloat16()
+    rs = torch.rand((M + 255) // 256 * 256, device="cuda", generator=g) + 0.5
+    p = lambda t: None if t is None else t.data_ptr()      # noqa: E731
+    for bias, res, factor, stats in ((b, None, None, False), (b, r, None, False), (b, None, rs, False), (None, None, rs, False), (b, r, None, True)):
+        want, got = (torch.empty(M, 4096, device="cuda", dtype=torch.bfloat16) if res is None else res.clone() for _ in range(2))
+        ss = [torch.zeros(32, rs.numel(), device="cuda") for _ in range(2)] if stats else [None, None]
+        assert ops.lib.evo_linear_mfma_nf_bf16(p(x), p(w), p(bias), None if res is None else p(want), p(want), p(factor), p(ss[0]), rs.numel() if stats else 0,
+                                               M, 4096, K, _stream()) == 0
+        ops._dense_layer(0, x, w, got, M, 4096, K, b=bias, res=None if res is None else got, rs=factor, ss=ss[1])
+        assert torch.equal(got, want)
+        assert not stats or torch.equal(ss[0][:, :M], ss[1][:, :M])
+    for factor in (None, rs):
+        want, got = (torch.empty(M, 2048, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+        if factor is None:
+            assert ops.lib.evo_mlp_gate_mfma_bf16(p(x), p(w), p(want), M, 2048, K, 0, _stream()) == 0
+        else:
+            assert ops.lib.evo_mlp_gate_mfma_nf_bf16(p(x), p(rs), p(w), p(want), M, 2048, K, _stream()) == 0
+        ops._dense_layer(1, x, w, got, M, 4096, K, rs=factor)
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("Mp,Tm", [(1024, 1024), (1536, 512), (2304, 768)])
+def test_same_bits_transposed(Mp, Tm):
+    from evo_amd.ops import _stream
+    ops, N, K = _ops(), 12288, 512
+    skip, rows = 1, Mp + Mp // Tm
+    g, x, w = _data(rows, N, K, 7)
+    b, rs = torch.randn(N, device="cuda", generator=g).bfloat16(), torch.rand(rows, device="cuda", generator=g) + 0.5
+    want, got = (torch.empty(Mp // 256, N, 256, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    assert ops.lib.evo_linear_t_mfma_nf_bf16(x.data_ptr(), rs.data_ptr(), w.data_ptr(), b.data_ptr(), want.data_ptr(), Mp, N, K, rows, Tm, skip, _stream()) == 0
+    ops._dense_layer(3, x, w, got, Mp, N, K, b=b, rs=rs, x_rows=rows, Tm=Tm, row_skip=skip)
+    assert torch.equal(got, want)
