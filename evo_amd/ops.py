@@ -46,6 +46,8 @@ _SIGNATURES = {
     "evo_linear_mfma_nf_bf16": ([_PTR] * 7 + [_I64] * 4 + [_PTR], _c.c_int),
     "evo_linear_xblk_mfma_nf_bf16": ([_PTR] * 6 + [_I64] * 4 + [_PTR], _c.c_int),
     "evo_mlp_gate_mfma_nf_bf16": ([_PTR] * 4 + [_I64] * 3 + [_PTR], _c.c_int),
+    "evo_put_tokens": ([_PTR, _I64, _PTR, _PTR, _I64, _PTR], _c.c_int),
+    "evo_advance_positions": ([_PTR, _I64, _I64, _PTR], _c.c_int),
     "evo_dense_ws": ([_I64] * 5, _c.c_int),
     "evo_dense_bf16": ([_I64] * 3 + [_PTR] * 7 + [_I64] * 8 + [_PTR, _I64, _PTR], _c.c_int),
     "evo_linear_t_mfma_nf_bf16": ([_PTR] * 5 + [_I64] * 6 + [_PTR], _c.c_int),
@@ -407,6 +409,20 @@ class HipOps(MixerOps):
         if flag is not None and int(flag.item()) != 0:
             raise IndexError(f"input_ids contain values outside [0, {V}) (embedding table has {V} rows)")
         return out
+
+    MAX_PUT = 64                 # tokens of one put_tokens launch (csrc/elementwise.hip EVO_PUT_MAX)
+
+    def put_tokens(self, ids: torch.Tensor, slots, tokens) -> None:
+        """ids[slot] = token for up to MAX_PUT pairs of host integers: kernel arguments, no copy from host memory and no wait."""
+        self._need(ids, torch.int64, "put_tokens ids")
+        n = len(slots)
+        arr = _c.c_int64 * n
+        _check(self.lib.evo_put_tokens(ids.data_ptr(), ids.numel(), _c.cast(arr(*slots), _PTR), _c.cast(arr(*tokens), _PTR), n, _stream()), "evo_put_tokens")
+
+    def advance_positions(self, pos: torch.Tensor, last: int) -> None:
+        """pos = min(pos + 1, last), in place."""
+        self._need(pos, torch.int64, "advance_positions pos")
+        _check(self.lib.evo_advance_positions(pos.data_ptr(), pos.numel(), int(last), _stream()), "evo_advance_positions")
 
     def rmsnorm(self, x: torch.Tensor, bias: Optional[torch.Tensor], scale: torch.Tensor, eps: float) -> torch.Tensor:
         """out = scale * x / (rms(x) + eps); with `bias`, x is first updated in place (x += bias)."""

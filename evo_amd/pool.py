@@ -95,8 +95,11 @@ class DecodePool:
 
     def advance(self, tokens: Dict[int, int]) -> torch.Tensor:
         """The next token of each given slot, in one pooled step -> logits [S, V] f32 (rows of the other slots mean nothing)."""
-        slots = list(tokens)
-        self.ids[torch.tensor(slots).to(self.device), 0] = torch.tensor(list(tokens.values()), dtype=torch.int64).to(self.device)
+        slots, put = list(tokens), getattr(self.model.ops, "put_tokens", None)
+        if put is not None and self.ids.is_cuda and 0 < len(slots) <= self.model.ops.MAX_PUT:
+            put(self.ids, slots, list(tokens.values()))
+        else:
+            self.ids[torch.tensor(slots).to(self.device), 0] = torch.tensor(list(tokens.values()), dtype=torch.int64).to(self.device)
         return self._advance(slots)
 
     def _advance(self, slots: Sequence[int]) -> torch.Tensor:
@@ -108,8 +111,6 @@ class DecodePool:
         logits = self._step()
         for s in slots:
             self.length[s] += 1
-        self.pos += 1
-        self.pos.clamp_(max=self.capacity - 1)                        # (free slots drift harmlessly; a full live slot grows the caches first)
         return logits
 
     def release(self, slot: int) -> None:
@@ -127,21 +128,33 @@ class DecodePool:
         finally:
             mha.pos_tensor = None
 
+    def _next_positions(self) -> None:
+        """(free slots drift harmlessly; a full live slot grows the caches first)"""
+        if self.pos.is_cuda and hasattr(self.model.ops, "advance_positions"):
+            self.model.ops.advance_positions(self.pos, self.capacity - 1)
+        else:
+            self.pos += 1
+            self.pos.clamp_(max=self.capacity - 1)
+
     def _step(self) -> torch.Tensor:
-        """self.ids [S,1] at positions self.pos [S] -> logits [S, V] f32 (every slot, active or not)."""
+        """self.ids [S,1] at positions self.pos [S] -> logits [S, V] f32 (every slot, active or not); the positions move on."""
         self.stats["steps"] += 1
         with torch.inference_mode():
             if not self.use_graph or not self.model._graph_shapes_ok(self.n_slots):
-                return self._step_eager().float()
+                out = self._step_eager().float()
+                self._next_positions()
+                return out
             if self._graph is None:
                 # The first step runs eagerly (it also warms the library handles and the M = S GEMM choices) and IS the
                 # step: the caches advance in place, so nothing may run twice.  Capture records without executing.
                 first = self._step_eager().float()
+                self._next_positions()
                 torch.cuda.synchronize(self.device)
                 self.model._graph_prepare(self.n_slots, self.device)
                 g = torch.cuda.CUDAGraph()
                 with torch.cuda.graph(g):
                     out = self._step_eager()
+                    self._next_positions()
                 self._graph = (g, out)
                 return first
             g, out = self._graph

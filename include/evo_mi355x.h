@@ -53,9 +53,15 @@ extern "C" {
  *      fp32-residual-stream kernels, decayed linear attention, latent attention (the last section of this file).
  *  12: evo_linear_act_mfma_bf16 (bias, three activations) and evo_act_cols take the places of evo_linear_silu_mfma_bf16 and evo_silu_cols; the
  *      evo_postnorm_* launches gained the norm of the sum (`alpha`, `sum`) and the plain one an activation, as did evo_linear_small_m_bf16; evo_window_attn gained grouped key heads,
- *      kept first tokens and two maps; evo_sum_norm, evo_heads_* and evo_rglru_* added. */
+ *      kept first tokens and two maps; evo_sum_norm, evo_heads_* and evo_rglru_* added.
+ *  13: evo_dense_bf16 and evo_dense_ws (any dense layer on the tiles its size asks for), evo_put_tokens and evo_advance_positions added. */
 #define EVO_ABI_VERSION 13
 int evo_abi_version(void);
+
+/* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
+ * evo_advance_positions: pos[i] = min(pos[i] + 1, last). */
+int evo_put_tokens(int64_t* ids, int64_t S, const int64_t* slots, const int64_t* tokens, int64_t n, void* stream);
+int evo_advance_positions(int64_t* pos, int64_t n, int64_t last, void* stream);
 
 /* ---- embedding gather ------------------------------------------------------------------------
  * replaces VocabParallelEmbedding.embed (ATen gather)    [REF evo/scoring.py:81; evo/models.py:136]
