@@ -398,14 +398,14 @@ __global__ __launch_bounds__(256) void gemm_parts_kernel(GemmArgs a, int act, co
 }
 
 // ---------------------------------------------------------------------------------------------------------------- which tile
-// Measured times of one k-step (64 deep) of one tile on one CU, in us: 64 x 64 0.267, 128 x 64 0.42, 128 x 128 0.575, 192 x 128 0.70, 256 x 128 0.84,
+// Measured times of one k-step (64 deep) of one tile on one CU, in us: 64 x 64 0.255, 128 x 64 0.435, 128 x 128 0.515, 192 x 128 0.70, 256 x 128 0.84,
 // 256 x 256 (the persistent kernel) 1.12 -- all of them the pace at which a CU takes operands in (58 GB/s: 64 KB in flight, about 1 us behind the
 // L2 miss that one of the CUs sharing a row pays), so a product's time is its operand rows per CU, and a larger tile moves fewer.  A launch takes the
 // tile and the number of parts of K whose sum of rounds, partial sums and memory traffic is least.  At K = 4,096 / 11,008 (MI355X, us, persistent
 // kernel -> this choice): 4,096 columns 68 -> 16 / 187 -> 34 at 161 rows, 72 -> 28 / 188 -> 58 at 512, 74 -> 36 / 187 -> 95 at 1,024, 75 -> 57 / 193 ->
-// 147 at 2,048; 12,288 columns 76 -> 36 at 161 rows, 78 -> 58 at 512; 22,016 gated columns 82 -> 53 at 161.
+// 147 at 2,048; 12,288 columns 76 -> 34 at 161 rows, 78 -> 58 at 512; 22,016 gated columns 82 -> 53 at 161.
 struct TileKind { int bm, bn; double step_us; };
-static const TileKind kinds[] = {{64, 64, 0.267}, {128, 64, 0.42}, {128, 128, 0.575}, {192, 128, 0.70}, {256, 128, 0.84}, {128, 256, 0.86}};
+static const TileKind kinds[] = {{64, 64, 0.255}, {128, 64, 0.435}, {128, 128, 0.515}, {192, 128, 0.70}, {256, 128, 0.84}, {128, 256, 0.86}};
 #define T_PERSISTENT 99
 
 struct TilePlan { int kind; int splits; double us; int64_t rows; };      // rows: how many of M it takes
@@ -422,7 +422,7 @@ static int tile_cus() {
 // `M` tokens, `N` columns of the weight; mode 3 has them the other way round in the launch
 static TilePlan tile_best(int64_t M, int64_t N, int64_t K, int mode, bool stats, bool splits_ok, bool persistent_ok) {
     const double cus = tile_cus(), nk = (double)(K / 64), flops = 2.0 * M * N * K;
-    const double memory = (2.0 * (M * K + N * K) + 2.0 * M * N) / 5.3e6, power = flops / 1.56e9;
+    const double memory = (2.0 * (M * K + N * K) + 2.0 * M * N) / 4.9e6, power = flops / 1.56e9;
     TilePlan best = {-1, 1, 1e30, M};
     if (persistent_ok) {
         const double rounds = ceil((double)((M + 255) / 256) * (double)(N / 256) / cus);
@@ -440,7 +440,7 @@ static TilePlan tile_best(int64_t M, int64_t N, int64_t K, int mode, bool stats,
             double us = ceil(tiles * s / cus) * (ceil(nk / s) * kinds[c].step_us + (mode == 1 && s == 1 ? 6.0 : 3.0));
             if (us < power * 1.05) us = power * 1.05;
             if (us < memory) us = memory;
-            if (s > 1) us += 5.0 + (double)s * M * N * 8 / 5.0e6;
+            if (s > 1) us += 5.6 + (double)s * M * N * 8 / 4.9e6;
             if (us < best.us) best = {c, s, us, M};
         }
     }

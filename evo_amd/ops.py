@@ -166,12 +166,14 @@ def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
-def pick_segment_length(B: int, T: int, H: int, target_waves: int = 4096) -> int:
-    """Time-segment length C of the Hyena kernels: enough (b, head, segment) waves to fill 256 CUs,
-    power of two in [64, 1024]."""
-    c = 1024
-    while c > 64 and B * H * ((T + c - 1) // c) < target_waves:
-        c //= 2
+def pick_segment_length(B: int, T: int, H: int) -> int:
+    """Time-segment length C of the Hyena kernels, a power of two in [4, 1024].  A wave walks its segment one position after the other
+    (about 0.5 us per position over the two passes), and every segment writes and reads a 64-byte state per channel, so the time is a C + b B T / C:
+    least where C^2 is about 2.2 positions at 32 heads.  (Three launches, 4,096 channels, MI355X: 161 positions 46.7 us with C = 64, 24.5 with 16;
+    2,000 57 with 64, 71 with 16; 8,000 150 with 64, 134 with 128; 65,544 970 with 128, 904 with 256 to 512.)"""
+    c = 4
+    while c < 1024 and 40 * c * c <= 11 * B * T * H // 16:         # (2c)^2 <= 2.2 B T H / 32
+        c *= 2
     return c
 
 
@@ -1116,6 +1118,7 @@ class HipOps(MixerOps):
         return lp, en
 
 
+    TAIL_ROWS = 32 * 1024
     def unembed_logprob_ok(self, h: torch.Tensor, emb: torch.Tensor) -> bool:
         return (h.is_cuda and h.dtype == torch.bfloat16 and emb.dtype == torch.bfloat16 and h.is_contiguous()
                 and emb.is_contiguous() and emb.shape[0] == 512 and h.shape[1] % 32 == 0
@@ -1124,7 +1127,9 @@ class HipOps(MixerOps):
     def unembed_logprob(self, h: torch.Tensor, emb: torch.Tensor, target: Optional[torch.Tensor],
                         want_logprob=True, want_entropy=False):
         """Fused scoring tail: h [M,K] bf16 (final-norm output) x emb[512,K]^T -> (logprob [M] f32 | None,
-        entropy [M] f32 | None) without materialising the [M, 512] logits."""
+        entropy [M] f32 | None).  A dense layer and one kernel over its logits, fewer than 64 K rows of them at a time; the one-launch
+        form, whose workgroup holds all 512 logits of its 64 rows, takes the widths that the dense layer does not (us, one launch -> two, K = 4,096,
+        MI355X: 1 row 83 -> 9, 161 rows 101 -> 13, 7,208 100 -> 39, 65,544 463 -> 227, 131,073 853 -> 474)."""
         self._need(h, torch.bfloat16, "unembed_logprob h")
         self._need(emb, torch.bfloat16, "unembed_logprob emb")
         M, K = h.shape
@@ -1134,6 +1139,22 @@ class HipOps(MixerOps):
         if target is not None:
             target = target.reshape(-1).to(torch.int64).contiguous()
             assert target.numel() == M
+        if V == 512 and K % 64 == 0 and 128 <= K <= 32768 and M > 0 and self.all_gemm_mfma:
+            # Whole chunks but for the last, which takes what is left of them: a row's logits are the same bits in any batch of 1,024 rows and more.
+            # (32 K rows are 32 MB of logits, which the second kernel finds in the Infinity Cache.)
+            n = max(1, M // self.TAIL_ROWS)
+            with self._t("unembed_logprob"):
+                for i in range(n):
+                    r0, r1 = i * self.TAIL_ROWS, M if i == n - 1 else (i + 1) * self.TAIL_ROWS
+                    if r1 - r0 <= 64:
+                        logits = self._linear_small_m(h, emb, None, None)
+                    else:
+                        logits = torch.empty(r1 - r0, V, dtype=torch.bfloat16, device=h.device)
+                        self._dense_layer(0, h[r0:r1], emb, logits, r1 - r0, V, K)
+                    _check(self.lib.evo_logprob_entropy(logits.data_ptr(), 0, _ptr(None if target is None else target[r0:r1]),
+                                                        _ptr(None if lp is None else lp[r0:r1]), _ptr(None if en is None else en[r0:r1]),
+                                                        r1 - r0, V, _stream()), "evo_logprob_entropy")
+            return lp, en
         with self._t("unembed_logprob"):
             _check(self.lib.evo_unembed_logprob_bf16(h.data_ptr(), emb.data_ptr(), _ptr(target), _ptr(lp), _ptr(en),
                                                      M, V, K, _stream()), "evo_unembed_logprob_bf16")

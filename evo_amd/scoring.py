@@ -63,7 +63,7 @@ def logits_to_logprobs(logits: torch.Tensor, input_ids: torch.Tensor, trim_bos: 
 
 
 def _fused_tail_ok(model, input_ids) -> bool:
-    """The fused unembed + log-softmax + gather kernel serves the engine's own model class on the GPU."""
+    """The engine's scoring tail (unembed + log-softmax + gather by chunks of rows) serves the engine's own model class on the GPU."""
     ops = getattr(model, "ops", None) if hasattr(model, "hidden_states") else None
     return (ops is not None and getattr(ops, "name", "") == "hip-gfx950" and hasattr(ops, "unembed_logprob")
             and ops.unembed_logprob_ok(model.unembed.weight.new_empty(1, model.hidden_size), model.unembed.weight))
@@ -72,8 +72,8 @@ def _fused_tail_ok(model, input_ids) -> bool:
 def score_logprobs_device(model, input_ids: torch.Tensor, want_entropy: bool = False):
     """What `score_sequences` / `positional_entropies` compute on the device for a BOS-prefixed id matrix [B, T]:
     (log-prob of token t+1 at position t  [B, T-1] f32 | None, entropy of the next-token distribution [B, T-1] f32 |
-    None).  On the MI355X engine the unembedding, the log-softmax and the gather run as ONE kernel
-    (evo_unembed_logprob_bf16) and the [B, T, 512] logits are never materialised; any other model object takes
+    None).  On the MI355X engine the unembedding and then the log-softmax, the gather
+    and the entropy run over chunks of rows and the [B, T, 512] logits are never held as a whole; any other model object takes
     model(ids) -> logits_to_logprobs like the reference [REF evo/scoring.py:80-84,116-121]."""
     B, T = input_ids.shape
     if _fused_tail_ok(model, input_ids):

@@ -557,8 +557,8 @@ class SequenceParallelScorer:
     def score_logprobs(self, ids_full: torch.Tensor) -> torch.Tensor:
         """Log-prob of each next token for this rank's positions: [B, n_local] f32, where global position t
         (t0 <= t < min(t1, T-1)) scores token t+1 -- the rank-local part of evo.scoring.logits_to_logprobs.  On the HIP
-        backend the unembedding, the log-softmax and the gather are ONE kernel (evo_unembed_logprob_bf16): the
-        [B, Tloc, 512] logits are never written."""
+        backend the unembedding and then the log-softmax and the gather run over chunks of rows: the [B, Tloc, 512] logits are
+        never held as a whole."""
         m, ops = self.m, self.m.ops
         B, T = ids_full.shape
         _, t0, t1 = self.shard(T)
