@@ -1,0 +1,279 @@
+// fp32 dense layers on the bf16 matrix cores of gfx950:  y [M, N] = x [M, K] w [N, K]^T (+ bias), all fp32.
+//
+// Every fp32 value is the exact sum of three bf16 ones, x = h + m + l: h its upper 16 bits (cut, so no finite value becomes infinite), m the rest
+// rounded to bf16, l what is left (at most 8 bits, so exact).  A product is h h' + (h m' + m h') + (h l' + l h' + m m') with fp32 accumulation; what
+// is left out, m l' + l m' + l l', is under 2^-22 of a product and mostly 2^-26 with either sign, less than the accumulation rounds.  Six bf16 MFMAs in
+// place of one fp32 MFMA at 1/16 of their rate.
+//
+// Workgroup = BM x BN of y, waves of (BM / WGM) x (BN / WGN) in 32 x 32 x 16 MFMAs, computed transposed (A = rows of w, B = rows of x) so that a lane
+// holds four neighbouring columns of one row of y.  K is walked in steps of 32: a thread loads 8 neighbouring fp32 of a row, splits them in registers
+// and writes the three 16-byte pieces to the planes of an LDS stage; rows of 64 B with the piece index XORed by (row >> 2) & 3: 16 lanes reading one
+// piece of 16 rows touch every bank once.  One stage and two barriers per step: the workgroups that share a CU split and multiply in turn (two
+// stages and one barrier at 256 x 128 were 1.1 to 1.3 times as slow: one workgroup per CU).
+#include "common.h"
+#include "../../include/evo_mi355x.h"
+#define F3_BK 32
+#define F3_ROWB 64
+
+struct F3Args {
+    const float* x; const float* w; const float* bias; float* y; float* parts;
+    int64_t M; int N, K, tiles_m, tiles_n, n_tiles, group_m, splits;
+};
+
+__device__ __forceinline__ void f3_split(const float4 a, const float4 b, uint4& h, uint4& m, uint4& l) {
+    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    uint32_t o[3][4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const uint32_t u0 = __float_as_uint(v[2 * e]), u1 = __float_as_uint(v[2 * e + 1]);
+        o[0][e] = __builtin_amdgcn_perm(u1, u0, 0x07060302);
+        float r0 = v[2 * e] - __uint_as_float(u0 & 0xffff0000u), r1 = v[2 * e + 1] - __uint_as_float(u1 & 0xffff0000u);
+        o[1][e] = pack_bf2(r0, r1);
+        r0 -= bf_lo(o[1][e]);
+        r1 -= bf_hi(o[1][e]);
+        o[2][e] = pack_bf2(r0, r1);
+    }
+    h = make_uint4(o[0][0], o[0][1], o[0][2], o[0][3]);
+    m = make_uint4(o[1][0], o[1][1], o[1][2], o[1][3]);
+    l = make_uint4(o[2][0], o[2][1], o[2][2], o[2][3]);
+}
+
+// Outputs taken again in plain fp32.  An infinite operand has no parts (inf - inf), and a sum that overflows may do so in another order; and where
+// an output is under 2^-90, its operands' last parts may lie under 2^-126, which the matrix cores take as zero.
+__device__ __forceinline__ bool f3_odd(float v) {
+    const uint32_t e = __float_as_uint(v) & 0x7f800000u;
+    return e == 0x7f800000u || (e < (37u << 23) && v != 0.f);
+}
+__device__ __noinline__ float f3_plain(const float* __restrict__ x, const float* __restrict__ w, int K) {
+    float s = 0.f;
+    for (int k = 0; k < K; ++k) s = fmaf(x[k], w[k], s);
+    return s;
+}
+
+template <int BM, int BN, int WGM, int WGN, int PER_CU, bool SPLIT>
+__global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_f32_kernel(F3Args a) {
+    constexpr int NT = 64 * WGM * WGN, TM = BM / WGM / 32, TN = BN / WGN / 32, ROWS = BM + BN, PLANE = ROWS * F3_ROWB, STAGE = 3 * PLANE, NP = ROWS * 4 / NT;
+    static_assert(ROWS * 4 % NT == 0, "whole pieces per thread");
+    __shared__ __attribute__((aligned(16))) unsigned char smem[STAGE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = lane >> 5, l31 = lane & 31;
+    const int wm = wave / WGN, wn = wave % WGN;
+    // block b runs on XCD b % 8: every XCD gets a contiguous run of tiles, group_m row tiles next to each other before the next column tile
+    int tile, part = 0;
+    {
+        const int bid = blockIdx.x, q = a.n_tiles >> 3, r = a.n_tiles & 7, xcd = bid & 7, slot = bid >> 3;
+        tile = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + slot;
+    }
+    if (SPLIT) { part = tile % a.splits; tile /= a.splits; }
+    const int per = a.group_m * a.tiles_n, g = tile / per, gm0 = g * a.group_m, gsz = min(a.tiles_m - gm0, a.group_m);
+    const int tm = gm0 + (tile - g * per) % gsz, tn = (tile - g * per) / gsz;
+    const int64_t m0 = (int64_t)tm * BM;
+    const int n0 = tn * BN;
+    const int nk = a.K / F3_BK, k0 = SPLIT ? (int)((int64_t)nk * part / a.splits) : 0, k1 = SPLIT ? (int)((int64_t)nk * (part + 1) / a.splits) : nk;
+
+    const float* src[NP];
+    int dst[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const int i = p * NT + tid, r = i >> 2, s = i & 3;
+        int64_t m = m0 + r;
+        int n = n0 + r - BM;
+        if (m > a.M - 1) m = a.M - 1;                          // rows past the end: any row that is there (never written)
+        if (n > a.N - 1) n = a.N - 1;
+        src[p] = (r < BM ? a.x + m * a.K : a.w + (int64_t)n * a.K) + (int64_t)k0 * F3_BK + s * 8;
+        dst[p] = r * F3_ROWB + ((s ^ (r >> 2)) & 3) * 16;
+    }
+    float4 st[NP][2];
+    auto fetch = [&]() {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) { st[p][0] = *(const float4*)src[p]; st[p][1] = *(const float4*)(src[p] + 4); src[p] += F3_BK; }
+    };
+    auto put = [&]() {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            uint4 h, m, l;
+            f3_split(st[p][0], st[p][1], h, m, l);
+            *(uint4*)(smem + dst[p]) = h;
+            *(uint4*)(smem + PLANE + dst[p]) = m;
+            *(uint4*)(smem + 2 * PLANE + dst[p]) = l;
+        }
+    };
+    int xo[TM][2], wo[TN][2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) { const int r = wm * (BM / WGM) + i * 32 + l31; xo[i][ks] = r * F3_ROWB + (((2 * ks + half) ^ (r >> 2)) & 3) * 16; }
+#pragma unroll
+        for (int j = 0; j < TN; ++j) { const int r = BM + wn * (BN / WGN) + j * 32 + l31; wo[j][ks] = r * F3_ROWB + (((2 * ks + half) ^ (r >> 2)) & 3) * 16; }
+    }
+    f32x16_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    auto multiply = [&]() {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            bf16x8_t xf[3][TM], wf[3][TN];
+#pragma unroll
+            for (int pl = 0; pl < 3; ++pl) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) xf[pl][i] = *(const bf16x8_t*)(smem + pl * PLANE + xo[i][ks]);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) wf[pl][j] = *(const bf16x8_t*)(smem + pl * PLANE + wo[j][ks]);
+            }
+            constexpr int PX[6] = {0, 2, 1, 0, 1, 0}, PW[6] = {2, 0, 1, 1, 0, 0};        // the smallest products first
+#pragma unroll
+            for (int q = 0; q < 6; ++q)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[PW[q]][j], xf[PX[q]][i], acc[i][j], 0, 0, 0);
+        }
+    };
+    fetch();
+    for (int k = k0; k < k1; ++k) {
+        put();
+        __syncthreads();
+        if (k + 1 < k1) fetch();
+        multiply();
+        __syncthreads();
+    }
+    bool odd = false;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int64_t m = m0 + wm * (BM / WGM) + i * 32 + l31;
+        if (m >= a.M) continue;
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int n = n0 + wn * (BN / WGN) + j * 32 + q * 8 + half * 4;
+                if (n >= a.N) continue;
+                float4 v = make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+                if (SPLIT) { *(float4*)(a.parts + ((int64_t)part * a.M + m) * a.N + n) = v; continue; }
+                if (a.bias) { const float4 b = *(const float4*)(a.bias + n); v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w; }
+                odd |= f3_odd(v.x) | f3_odd(v.y) | f3_odd(v.z) | f3_odd(v.w);
+                *(float4*)(a.y + m * a.N + n) = v;
+            }
+    }
+    if (!SPLIT && odd) {
+        for (int i = 0; i < TM; ++i)
+            for (int c = 0; c < TN * 16; ++c) {
+                const int64_t m = m0 + wm * (BM / WGM) + i * 32 + l31;
+                const int n = n0 + wn * (BN / WGN) + (c >> 4) * 32 + ((c >> 2) & 3) * 8 + half * 4 + (c & 3);
+                if (m >= a.M || n >= a.N || !f3_odd(a.y[m * a.N + n])) continue;
+                const float v = f3_plain(a.x + m * a.K, a.w + (int64_t)n * a.K, a.K);
+                a.y[m * a.N + n] = a.bias ? v + a.bias[n] : v;
+            }
+    }
+}
+
+// the sum of the parts of K
+__global__ __launch_bounds__(256) void gemm_f32_parts_kernel(F3Args a) {
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i >= a.M * a.N) return;
+    const int64_t m = i / a.N;
+    const int n = (int)(i - m * a.N);
+    float4 v = *(const float4*)(a.parts + i);
+    for (int s = 1; s < a.splits; ++s) {
+        const float4 p = *(const float4*)(a.parts + (int64_t)s * a.M * a.N + i);
+        v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
+    }
+    const float4 b = a.bias ? *(const float4*)(a.bias + n) : make_float4(0.f, 0.f, 0.f, 0.f);
+    float o[4] = {v.x, v.y, v.z, v.w};
+    const float c[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (a.bias) o[e] += c[e];
+        if (f3_odd(o[e])) {
+            o[e] = f3_plain(a.x + m * a.K, a.w + (int64_t)(n + e) * a.K, a.K);
+            if (a.bias) o[e] += c[e];
+        }
+    }
+    *(float4*)(a.y + i) = make_float4(o[0], o[1], o[2], o[3]);
+}
+
+// ---------------------------------------------------------------------------------------------------------------- which tile
+// One k-step (32 deep) of the n tiles that share a CU takes `start` + n `each` us (at most `per_cu` share it: LDS and registers), fitted to 33 to 4,000
+// rows of eight layers.  The matrix cores bound the larger tiles: 128 x 128 with two on a CU 222 TF, 256 x 256 235 TF (six bf16 products each: 1.4 PF, what a
+// large bf16 product reaches).  Against the library's fp32 MFMA layers (us, K = 4,096, MI355X,
+// before -> here): 4,096 columns 40 -> 38 at 65 rows, 85 -> 80 at 300, 348 -> 254 at 1,290, 931 -> 623 at 4,000; 22,016 columns 180 -> 141, 442 -> 342,
+// 1,816 -> 1,257, 5,454 -> 3,500; K = 11,008, 4,096 columns 93 -> 86, 230 -> 181, 932 -> 668, 2,421 -> 1,692.  Error against 64 bits (random normal operands,
+// K = 4,096): 1.02e-6 unsplit, less with every split, library 1.15e-6 (its own splits 5.8e-7 at 33 to 200 rows, where this choice splits by 8: 3.6e-7).
+struct F3Kind { int bm, bn, per_cu; double start, each; };
+static const F3Kind f3_kinds[] = {{64, 64, 5, 0.29, 0.33}, {64, 128, 4, 0.30, 0.655}, {128, 128, 2, 0.20, 1.11}, {256, 256, 1, 0.10, 4.36}};
+struct F3Plan { int kind, splits; };
+
+static F3Plan f3_plan(int64_t M, int64_t N, int64_t K) {
+    static const int cus = [] {
+        int dev = 0, c = 256;
+        if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev);
+        return c < 8 ? 8 : c;
+    }();
+    F3Plan best = {0, 1};
+    double least = 1e300;
+    const double memory = 4.0 * ((double)N * K + (double)M * K) / 4.2e6;
+    for (int c = 0; c < 4; ++c) {
+        const F3Kind& k = f3_kinds[c];
+        const double tiles = (double)((M + k.bm - 1) / k.bm) * (double)((N + k.bn - 1) / k.bn);
+        for (int s = 1; s <= 8; ++s) {
+            if (s == 5 || s == 7) continue;
+            if (s > 1 && (K / F3_BK / s < 8 || tiles * s > 12.0 * cus || (double)s * M * N * 4 > 256e6)) break;
+            const double steps = ceil((double)(K / F3_BK) / s), n = ceil(tiles * s / cus), rest = fmod(n, k.per_cu), full = (n - rest) / k.per_cu;
+            const double work = steps * (full * (k.start + k.per_cu * k.each) + (rest > 0 ? k.start + rest * k.each : 0.0)) + 5.0;
+            double us = work > memory ? work + 0.085 * memory : memory + 0.085 * work;
+            if (s > 1) us += 6.0 + (double)s * M * N * 8 / 9.1e6;
+            if (us < least) { least = us; best = {c, s}; }
+        }
+    }
+    return best;
+}
+
+template <int BM, int BN, int WGM, int WGN, int PER_CU>
+static int f3_launch(F3Args a, hipStream_t st) {
+    const int64_t tm = (a.M + BM - 1) / BM, tn = ((int64_t)a.N + BN - 1) / BN;
+    if (tm * tn * a.splits > 0x7fffffff) return -1;
+    a.tiles_m = (int)tm;
+    a.tiles_n = (int)tn;
+    a.n_tiles = (int)(tm * tn * a.splits);
+    a.group_m = 8;
+    const dim3 grid((unsigned)a.n_tiles), block(64 * WGM * WGN);
+    if (a.splits == 1) {
+        hipLaunchKernelGGL((gemm_f32_kernel<BM, BN, WGM, WGN, PER_CU, false>), grid, block, 0, st, a);
+        return evo_launch_status();
+    }
+    hipLaunchKernelGGL((gemm_f32_kernel<BM, BN, WGM, WGN, PER_CU, true>), grid, block, 0, st, a);
+    const int rc = evo_launch_status();
+    if (rc) return rc;
+    hipLaunchKernelGGL(gemm_f32_parts_kernel, dim3((unsigned)((a.M * a.N / 4 + 255) / 256)), dim3(256), 0, st, a);
+    return evo_launch_status();
+}
+
+static bool f3_ok(int64_t M, int64_t N, int64_t K) {
+    return M >= 0 && N > 0 && K >= F3_BK && M <= 0x7fffffff && N <= 0x7fffff00 && K <= 0x7fffff00 && N % 4 == 0 && K % F3_BK == 0 && (double)M * N <= 4e11;
+}
+
+extern "C" int evo_linear_f32_ws(int64_t M, int64_t N, int64_t K) {
+    if (!f3_ok(M, N, K)) return -1;
+    const F3Plan p = f3_plan(M, N, K);
+    return p.splits > 1 ? p.splits : 0;
+}
+
+extern "C" int evo_linear_f32(const float* x, const float* w, const float* bias, float* y, int64_t M, int64_t N, int64_t K, float* ws, int64_t ws_bytes, void* stream) {
+    if (!f3_ok(M, N, K)) return -1;
+    if (M == 0) return 0;
+    if (!x || !w || !y || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)bias | (uintptr_t)y | (uintptr_t)ws) & 15)) return -1;
+    F3Plan p = f3_plan(M, N, K);
+    if (p.splits > 1 && (!ws || ws_bytes < p.splits * M * N * 4)) p.splits = 1;
+    F3Args a = {x, w, bias, y, ws, M, (int)N, (int)K, 0, 0, 0, 0, p.splits};
+    hipStream_t st = (hipStream_t)stream;
+    switch (p.kind) {
+        case 0: return f3_launch<64, 64, 2, 2, 5>(a, st);
+        case 1: return f3_launch<64, 128, 2, 2, 4>(a, st);
+        case 2: return f3_launch<128, 128, 2, 2, 2>(a, st);
+        default: return f3_launch<256, 256, 2, 4, 1>(a, st);
+    }
+}

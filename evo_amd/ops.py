@@ -3,8 +3,8 @@
 `HipOps` is the ONLY compute backend the product ships: it raises if the shared library cannot be
 loaded or a tensor is not on a ROCm device -- there is no CPU / eager fallback.  Every kernel of a scoring or generation
 step -- the dense layers included (csrc/gemm.hip, csrc/gemv.hip) -- is a hand-written gfx950 kernel reached through the C ABI with
-raw device pointers and the caller's current stream; hipBLASLt (through `torch.addmm`) serves only shapes no 7B layer has and the
-in-process A/B knob `all_gemm_mfma = False`.
+raw device pointers and the caller's current stream; hipBLASLt (through `torch.addmm`) serves only shapes no 7B layer has, fp32
+layers of up to 32 rows and the in-process A/B knob `all_gemm_mfma = False`.
 """
 from __future__ import annotations
 
@@ -60,6 +60,8 @@ _SIGNATURES = {
     "evo_hyena_decode_fused_small_m": ([_PTR] * 12 + [_I64] * 3 + [_c.c_float, _PTR], _c.c_int),
     "evo_gelu_gate_bf16": ([_PTR, _PTR, _I64, _I64, _PTR], _c.c_int),
     "evo_logprob_entropy": ([_PTR, _I64, _PTR, _PTR, _PTR, _I64, _I64, _PTR], _c.c_int),
+    "evo_linear_f32_ws": ([_I64] * 3, _c.c_int),
+    "evo_linear_f32": ([_PTR] * 4 + [_I64] * 3 + [_PTR, _I64, _PTR], _c.c_int),
     "evo_unembed_logprob_bf16": ([_PTR] * 5 + [_I64] * 3 + [_PTR], _c.c_int),
     "evo_rope_append_decode_bf16": ([_PTR] * 4 + [_F32] + [_I64] * 7 + [_F32, _PTR], _c.c_int),
     "evo_embed_stream": ([_PTR] * 4 + [_I64] * 3 + [_F32, _PTR, _I64, _PTR], _c.c_int),
@@ -88,7 +90,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 13         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 14         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):
@@ -306,10 +308,34 @@ class HipOps(MixerOps):
             return y
         if self._take_mfma(mfma) and self.mfma_linear_ok(x, w):
             return self.linear_mfma(x, w, b)
+        if self._f32_layer_ok(x, w, b):
+            return self._linear_f32(x, w, b)
         with self._t("gemm"):
             if b is not None:
                 return torch.addmm(b, x, w.t())
             return torch.mm(x, w.t())
+
+    def _f32_layer_ok(self, x, w, b) -> bool:
+        """fp32 layers from 33 rows on take csrc/gemm_f32.hip; below, the weight's own bytes bound the layer and the library reads them at 2.5 to 4.6 TB/s
+        (24 rows: 26 us against 36 at 4,096 x 4,096, 79 against 91 at 22,016 x 4,096; 33 rows: 31 against 28, 117 against 93).  What is traced or
+        differentiated stays with torch."""
+        ts = (x, w) if b is None else (x, w, b)
+        return (self.all_gemm_mfma and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()
+                                           and t.device == x.device and t.data_ptr() % 16 == 0 for t in ts)
+                and x.dim() == 2 and w.dim() == 2 and x.shape[0] > 32 and x.shape[1] == w.shape[1] and x.shape[1] % 32 == 0 and x.shape[1] >= 256
+                and w.shape[0] % 4 == 0 and w.shape[0] >= 256 and (b is None or b.shape == (w.shape[0],))
+                and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
+                and torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None)
+
+    def _linear_f32(self, x, w, b):
+        M, K = x.shape
+        N = w.shape[0]
+        y = torch.empty(M, N, dtype=torch.float32, device=x.device)
+        n = self.lib.evo_linear_f32_ws(M, N, K)
+        ws = torch.empty(n * M * N, dtype=torch.float32, device=x.device) if n > 0 else None
+        with self._t("gemm_f32"):
+            _check(self.lib.evo_linear_f32(x.data_ptr(), w.data_ptr(), _ptr(b), y.data_ptr(), M, N, K, _ptr(ws), max(n, 0) * M * N * 4, _stream()), "evo_linear_f32")
+        return y
 
     def _take_mfma(self, mfma: bool) -> bool:
         return self.all_gemm_mfma or (mfma and self.attn_gemm_mfma)

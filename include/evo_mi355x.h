@@ -54,8 +54,9 @@ extern "C" {
  *  12: evo_linear_act_mfma_bf16 (bias, three activations) and evo_act_cols take the places of evo_linear_silu_mfma_bf16 and evo_silu_cols; the
  *      evo_postnorm_* launches gained the norm of the sum (`alpha`, `sum`) and the plain one an activation, as did evo_linear_small_m_bf16; evo_window_attn gained grouped key heads,
  *      kept first tokens and two maps; evo_sum_norm, evo_heads_* and evo_rglru_* added.
- *  13: evo_dense_bf16 and evo_dense_ws (any dense layer on the tiles its size asks for), evo_put_tokens and evo_advance_positions added. */
-#define EVO_ABI_VERSION 13
+ *  13: evo_dense_bf16 and evo_dense_ws (any dense layer on the tiles its size asks for), evo_put_tokens and evo_advance_positions added.
+ *  14: evo_linear_f32 and evo_linear_f32_ws (fp32 dense layers on the bf16 matrix cores) added. */
+#define EVO_ABI_VERSION 14
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
@@ -382,6 +383,13 @@ int evo_gelu_gate_bf16(const void* g, void* a, int64_t M, int64_t I, void* strea
  * -> logprob [M] f32 (may be NULL), entropy [M] f32 (may be NULL).  fp32 log-softmax. */
 int evo_logprob_entropy(const void* logits, int64_t logits_f32, const int64_t* target, float* logprob,
                         float* entropy, int64_t M, int64_t V, void* stream);
+
+/* ---- fp32 dense layer: y [M, N] = x [M, K] w [N, K]^T (+ bias [N]), all fp32, on the bf16 matrix cores: every operand as the exact sum of three
+ * bf16 values, six products, fp32 accumulation (csrc/gemm_f32.hip).  K % 32 == 0, N % 4 == 0, 16-byte aligned dense operands; infinities and NaN come
+ * out as in a plain fp32 sum.  evo_linear_f32_ws: how many times M N fp32 the workspace holds with which it splits K (0: none; -1: sizes
+ * it does not take); without it, or with a smaller one, it does not. */
+int evo_linear_f32_ws(int64_t M, int64_t N, int64_t K);
+int evo_linear_f32(const float* x, const float* w, const float* bias, float* y, int64_t M, int64_t N, int64_t K, float* ws, int64_t ws_bytes, void* stream);
 
 /* ---- fused scoring tail: unembed + log_softmax + gather (+ entropy) ---------------------------------
  * replaces  logits = x @ E^T ; log_softmax(logits) ; gather(next token) ; -sum p log p

@@ -1,0 +1,95 @@
+"""fp32 dense layers on the bf16 matrix cores (csrc/gemm_f32.hip): operands as three bf16 parts each."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from evo_amd.ops import HipOps
+    return HipOps()
+
+
+def rand(*shape, seed=0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed))
+
+
+# a lone row tile and column tile, remainders of both, one k-step more than the parts of K divide, each tile of the plan, with and without parts
+SHAPES = [(33, 256, 256), (63, 260, 288), (65, 512, 4096), (129, 1028, 1056), (300, 4096, 1024), (513, 260, 256), (1290, 2048, 512), (2049, 2052, 256), (4000, 4096, 256)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("bias", [False, True])
+def test_no_further_from_64_bits_than_fp32(ops, M, N, K, bias):
+    """Against the sum in 64 bits.  Each of the K / 16 x 6 matrix products adds to an fp32 sum: rounding of at most 2^-24 of a partial sum, which random
+    walks to sqrt(K) of a product; the sum over the steps stays under 2^-24 sqrt(6 K / 16) in the mean square, doubled for the parts left out and for
+    adders that cut."""
+    x, w, b = rand(M, K, seed=1).to(DEV), rand(N, K, seed=2).to(DEV), rand(N, seed=3).to(DEV) if bias else None
+    assert ops._f32_layer_ok(x, w, b)
+    y = ops.linear(x, w, b)
+    want = x.double() @ w.double().t() + (b.double() if bias else 0)
+    err = ((y.double() - want).norm() / want.norm()).item()
+    assert err < 2.0 ** -23 * (6 * K / 16) ** 0.5, err
+    plain = torch.addmm(b, x, w.t()) if bias else x @ w.t()
+    assert err < 1.25 * ((plain.double() - want).norm() / want.norm()).item() + 2.0 ** -24
+
+
+def test_parts_are_exact_and_large_values_stay_finite(ops):
+    """One product per output: x (times a power of two) comes back bit for bit, up to the largest fp32 value."""
+    x = torch.cat([rand(40, 256, seed=4), rand(40, 256, seed=5) * 1e30, rand(40, 256, seed=6) * 1e-30]).to(DEV)
+    x[0, 0], x[0, 1] = torch.finfo(torch.float32).max, -torch.finfo(torch.float32).max
+    w = torch.zeros(256, 256, device=DEV)
+    w[torch.arange(256), torch.randperm(256, generator=torch.Generator().manual_seed(7))] = 0.5
+    assert torch.equal(ops.linear(x, w), x[:, w.argmax(1)] * 0.5)
+
+
+@pytest.mark.parametrize("K", [256, 4096])                     # one part of K, several
+def test_infinities_and_nan(ops, K):
+    x, w = rand(70, K, seed=8), rand(512, K, seed=9)
+    x[3, 5] = float("inf")
+    x[9, 0] = float("nan")
+    w[17, 8] = float("-inf")
+    x[20, 8] = 0.0
+    # a sum over the largest value in any order, in one output only: elsewhere in that row no partial sum passes 3e38 (2 x 5e-3 + 4 sqrt(K) / 3e38)
+    x[40, :2] = 3e38
+    w[:, :2] *= 1e-3
+    w[60, :2] = 3.0
+    y, want = ops.linear(x.to(DEV), w.to(DEV)).cpu(), x @ w.t()
+    assert torch.equal(torch.isnan(y), torch.isnan(want))
+    odd = torch.isinf(want)
+    assert torch.equal(y[odd], want[odd]) and torch.isfinite(y[~odd & ~torch.isnan(want)]).all()
+
+
+def test_what_keeps_torch(ops):
+    x, w = rand(40, 256, seed=1).to(DEV), rand(256, 256, seed=2).to(DEV)
+    assert ops._f32_layer_ok(x, w, None)
+    assert not ops._f32_layer_ok(x[:32], w, None)              # few rows
+    assert not ops._f32_layer_ok(x[:, :250].contiguous(), w[:, :250].contiguous(), None)
+    assert not ops._f32_layer_ok(x.t().contiguous().t(), w, None)
+    assert not ops._f32_layer_ok(torch.empty(40 * 256 + 1, device=DEV)[1:].view(40, 256), w, None)
+    g = w.clone().requires_grad_()
+    assert not ops._f32_layer_ok(x, g, None)
+    ops.linear(x, g).sum().backward()
+    assert torch.allclose(g.grad, x.sum(0).expand_as(g), rtol=1e-4, atol=1e-4)
+    with torch.no_grad():
+        assert ops._f32_layer_ok(x, g, None)
+    with torch.autograd.forward_ad.dual_level():
+        assert not ops._f32_layer_ok(x, w, None)
+
+
+def test_under_capture(ops):
+    x, w = rand(300, 1024, seed=1).to(DEV), rand(512, 1024, seed=2).to(DEV)
+    want = ops.linear(x, w).clone()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        y = ops.linear(x, w)
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+        (x * 2).sum().item()
