@@ -331,84 +331,204 @@ extern "C" int evo_lightning_chunk_bf16(const void* z, int64_t ld, void* o, floa
 
 // ------------------------------------------------------------------------------------------------ recurrent form
 // Token by token, any sizes, both storage types: one workgroup per (sequence, head, 8 CW value columns).  Thread (column lane cl, slice):
-// columns cl CW .. + CW - 1, rows slice, slice + 32, ... of the state.  STEP: one token per sequence straight on the state in memory (the
-// decode step: the state is read and written once, 16 bytes per request); otherwise the state's tile stays in LDS across the tokens.
-template <typename T, int CW, bool STEP>
+// columns cl CW .. + CW - 1, rows slice, slice + 32, ... of the state.  The decode step: one token per sequence straight on the state in memory
+// (read and written once, 16 bytes per request).
+template <typename T, int CW>
 __global__ __launch_bounds__(256) void lightning_recur_kernel(LightArgs a, const float* __restrict__ decay) {
     extern __shared__ float sm[];
     const int dk = a.dk, dv = a.dv, h = blockIdx.y, b = blockIdx.z;
-    float* qs = sm;                                              // [dk], [dk], [32], [32 slices][8 CW + 1], state tile [dk][8 CW]
+    float* qs = sm;                                              // [dk], [dk], [32], [32 slices][8 CW + 1]
     float* ks = qs + dk;
     float* vs = ks + dk;
     float* part = vs + 32;
-    float* tile = part + 32 * 33;
+    const int tid = threadIdx.x, cl = tid & 7, sl = tid >> 3;
+    const int c0 = blockIdx.x * 8 * CW, cols = dv - c0 < 8 * CW ? dv - c0 : 8 * CW;
+    const float A = decay[h];
+    float* st = a.state + ((int64_t)b * a.H + h) * dk * dv + c0;
+    const T* z = (const T*)a.z + (int64_t)b * a.ld;
+    for (int k = tid; k < 2 * dk; k += 256) {
+        const float x = ld1(z + (k < dk ? 0 : (int64_t)(a.H - 1) * dk) + (int64_t)h * dk + k);
+        qs[k] = a.act ? silu_t<T>(x) : x;
+    }
+    if (tid < 8 * CW) {
+        const float x = tid < cols ? ld1(z + (int64_t)2 * a.H * dk + (int64_t)h * dv + c0 + tid) : 0.f;
+        vs[tid] = a.act ? silu_t<T>(x) : x;
+    }
+    __syncthreads();
+    float v[CW], o[CW];
+#pragma unroll
+    for (int e = 0; e < CW; ++e) { v[e] = vs[cl * CW + e]; o[e] = 0.f; }
+    if (cl * CW < cols) {
+#pragma unroll 4
+        for (int k = sl; k < dk; k += 32) {
+            float s[CW];
+            float* p = st + (int64_t)k * dv + cl * CW;
+            if constexpr (CW == 4) { const float4 x = *(const float4*)p; s[0] = x.x; s[1] = x.y; s[2] = x.z; s[3] = x.w; }
+            else s[0] = *p;
+#pragma unroll
+            for (int e = 0; e < CW; ++e) {
+                s[e] = fmaf(A, s[e], ks[k] * v[e]);
+                o[e] = fmaf(qs[k], s[e], o[e]);
+            }
+            if constexpr (CW == 4) *(float4*)p = make_float4(s[0], s[1], s[2], s[3]);
+            else *p = s[0];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < CW; ++e) part[sl * 33 + cl * CW + e] = o[e];
+    __syncthreads();
+    if (tid < cols) {
+        float s = 0.f;
+#pragma unroll 8
+        for (int i = 0; i < 32; ++i) s += part[i * 33 + tid];
+        st1((T*)a.o + (int64_t)b * a.H * dv + (int64_t)h * dv + c0 + tid, s);
+    }
+}
+
+// Prompts the same way, LT tokens between barriers: their q, k, v rows are staged together (the next LT's are in flight meanwhile), the slices' shares of
+// LT rows of o meet in LDS at the end of the block, summed in the order of the slices.  R: the state rows of a thread, in registers (dk <= 32 R); 0: in LDS.
+// Bound by issue and latency: 70 instructions a token and wave in sequence.  (3 prompts of up to 500 tokens, 32 heads of 128 x 128, fp32, MI355X: 288 us;
+// one token between barriers, its rows requested when they were needed and the state in LDS, 685 us.)
+template <typename T, int CW, int R, int LT>
+__global__ __launch_bounds__(256) void lightning_tokens_kernel(LightArgs a, const float* __restrict__ decay) {
+    extern __shared__ float sm[];
+    const int dk = a.dk, dv = a.dv, h = blockIdx.y, b = blockIdx.z;
+    float2* kq = (float2*)sm;                                    // [LT][dk] (k, q), [LT][32], [LT][32 slices][33], with R == 0 the state [dk][8 CW]
+    float* vs = sm + 2 * LT * dk;
+    float* part = vs + LT * 32;
+    float* tile = part + LT * 32 * 33;
     const int tid = threadIdx.x, cl = tid & 7, sl = tid >> 3;
     const int c0 = blockIdx.x * 8 * CW, cols = dv - c0 < 8 * CW ? dv - c0 : 8 * CW;
     const bool mine = cl * CW < cols;
     const float A = decay[h];
-    const int row0 = STEP ? b : a.cu[b], n = STEP ? 1 : a.cu[b + 1] - row0;
+    const int row0 = a.cu[b], n = a.cu[b + 1] - row0;
     float* st = a.state ? a.state + ((int64_t)b * a.H + h) * dk * dv + c0 : nullptr;
-    if (!STEP) {
-        const bool keep = st && a.resume && a.resume[b];
+    const bool keep = st && a.resume && a.resume[b];
+    float S[R ? R : 1][CW];
+    if constexpr (R > 0) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int e = 0; e < CW; ++e) S[r][e] = keep && mine && sl + 32 * r < dk ? st[(int64_t)(sl + 32 * r) * dv + cl * CW + e] : 0.f;
+    } else {
         for (int k = sl; k < dk; k += 32)
 #pragma unroll
             for (int e = 0; e < CW; ++e) tile[k * 8 * CW + cl * CW + e] = keep && mine ? st[(int64_t)k * dv + cl * CW + e] : 0.f;
     }
-    for (int t = 0; t < n; ++t) {
-        const T* z = (const T*)a.z + (int64_t)(row0 + t) * a.ld;
-        for (int k = tid; k < 2 * dk; k += 256) {
-            const float x = ld1(z + (k < dk ? 0 : (int64_t)(a.H - 1) * dk) + (int64_t)h * dk + k);
-            qs[k] = a.act ? silu_t<T>(x) : x;
-        }
-        if (tid < 8 * CW) {
-            const float x = tid < cols ? ld1(z + (int64_t)2 * a.H * dk + (int64_t)h * dv + c0 + tid) : 0.f;
-            vs[tid] = a.act ? silu_t<T>(x) : x;
-        }
-        __syncthreads();
-        float v[CW], o[CW];
+    const T* zr = (const T*)a.z + (int64_t)row0 * a.ld;
+    const int64_t hk = (int64_t)h * dk, hv = (int64_t)2 * a.H * dk + (int64_t)h * dv + c0;
+    constexpr int RK = R ? R : 1;                                // staged values of k and of q per thread (R == 0: staged without a request ahead)
+    float zk[RK], zq[RK], zv;
+    // thread (token tid / SW, elements tid % SW + SW j) of a block's k and q; of its v
+    constexpr int SW = 256 / LT;
+    const int tt = tid / SW, te = tid % SW;
+    auto request = [&](int t0) {
+        const T* z = zr + (int64_t)(t0 + tt < n ? t0 + tt : n - 1) * a.ld;
+        if constexpr (R > 0) {
 #pragma unroll
-        for (int e = 0; e < CW; ++e) { v[e] = vs[cl * CW + e]; o[e] = 0.f; }
-        if (mine) {
-#pragma unroll 4
-            for (int k = sl; k < dk; k += 32) {
-                float s[CW];
-                float* p = STEP ? st + (int64_t)k * dv + cl * CW : tile + k * 8 * CW + cl * CW;
-                if constexpr (CW == 4) { const float4 x = *(const float4*)p; s[0] = x.x; s[1] = x.y; s[2] = x.z; s[3] = x.w; }
-                else s[0] = *p;
-#pragma unroll
-                for (int e = 0; e < CW; ++e) {
-                    s[e] = fmaf(A, s[e], ks[k] * v[e]);
-                    o[e] = fmaf(qs[k], s[e], o[e]);
-                }
-                if constexpr (CW == 4) *(float4*)p = make_float4(s[0], s[1], s[2], s[3]);
-                else *p = s[0];
+            for (int j = 0; j < RK; ++j) {
+                const int k = te + SW * j < dk ? te + SW * j : dk - 1;
+                zk[j] = ld1(z + (int64_t)a.H * dk + hk + k);
+                zq[j] = ld1(z + hk + k);
             }
         }
+        zv = te < cols ? ld1(z + hv + te) : 0.f;
+    };
+    auto act = [&](float x) { return a.act ? silu_t<T>(x) : x; };
+    if (n > 0) request(0);
+    for (int t0 = 0; t0 < n; t0 += LT) {
+        const int nb = n - t0 < LT ? n - t0 : LT;
+        if constexpr (R > 0) {
 #pragma unroll
-        for (int e = 0; e < CW; ++e) part[sl * 33 + cl * CW + e] = o[e];
+            for (int j = 0; j < RK; ++j)
+                if (te + SW * j < dk) kq[tt * dk + te + SW * j] = make_float2(act(zk[j]), act(zq[j]));
+        } else if (tt < nb) {
+            const T* z = zr + (int64_t)(t0 + tt) * a.ld;
+            for (int k = te; k < dk; k += SW) kq[tt * dk + k] = make_float2(act(ld1(z + (int64_t)a.H * dk + hk + k)), act(ld1(z + hk + k)));
+        }
+        if (te < 32) vs[tt * 32 + te] = act(zv);
         __syncthreads();
-        if (tid < cols) {
+        if (t0 + LT < n) request(t0 + LT);
+        auto token = [&](int t) __attribute__((always_inline)) {
+            float v[CW], o[CW];
+            if constexpr (CW == 4 && R > 0) { const float4 x = *(const float4*)(vs + t * 32 + cl * 4); v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w; }
+            else {
+#pragma unroll
+                for (int e = 0; e < CW; ++e) v[e] = vs[t * 32 + cl * CW + e];
+            }
+#pragma unroll
+            for (int e = 0; e < CW; ++e) o[e] = 0.f;
+            if constexpr (R > 0) {
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (sl + 32 * r < dk) {
+                        const float2 x = kq[t * dk + sl + 32 * r];
+#pragma unroll
+                        for (int e = 0; e < CW; ++e) {
+                            S[r][e] = fmaf(A, S[r][e], x.x * v[e]);
+                            o[e] = fmaf(x.y, S[r][e], o[e]);
+                        }
+                    }
+            } else if (mine) {
+#pragma unroll 4
+                for (int k = sl; k < dk; k += 32) {
+                    float* p = tile + k * 8 * CW + cl * CW;
+                    const float2 x = kq[t * dk + k];
+#pragma unroll
+                    for (int e = 0; e < CW; ++e) {
+                        p[e] = fmaf(A, p[e], x.x * v[e]);
+                        o[e] = fmaf(x.y, p[e], o[e]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < CW; ++e) part[(t * 32 + sl) * 33 + cl * CW + e] = o[e];
+        };
+        if (nb == LT) {
+#pragma unroll
+            for (int t = 0; t < LT; ++t) token(t);
+        } else {
+            for (int t = 0; t < nb; ++t) token(t);
+        }
+        __syncthreads();
+        if (tt < nb && te < cols) {
             float s = 0.f;
 #pragma unroll 8
-            for (int i = 0; i < 32; ++i) s += part[i * 33 + tid];
-            st1((T*)a.o + (int64_t)(row0 + t) * a.H * dv + (int64_t)h * dv + c0 + tid, s);
+            for (int i = 0; i < 32; ++i) s += part[(tt * 32 + i) * 33 + te];
+            st1((T*)a.o + (int64_t)(row0 + t0 + tt) * a.H * dv + (int64_t)h * dv + c0 + te, s);
         }
-        // (the next token's staging touches qs / ks / vs only, which every thread has finished reading at the barrier above; its `part`
-        //  stores come behind the next barrier, and so behind the sums of this token)
+        // (the next block's staging touches kq / vs only, which every thread has finished reading at the barrier above; its `part`
+        //  stores come behind the next barrier, and so behind the sums of this block)
     }
-    if (!STEP && st && mine)
-        for (int k = sl; k < dk; k += 32)
+    if (st && mine) {
+        if constexpr (R > 0) {
 #pragma unroll
-            for (int e = 0; e < CW; ++e) st[(int64_t)k * dv + cl * CW + e] = tile[k * 8 * CW + cl * CW + e];
+            for (int r = 0; r < R; ++r)
+                if (sl + 32 * r < dk)
+#pragma unroll
+                    for (int e = 0; e < CW; ++e) st[(int64_t)(sl + 32 * r) * dv + cl * CW + e] = S[r][e];
+        } else {
+            for (int k = sl; k < dk; k += 32)
+#pragma unroll
+                for (int e = 0; e < CW; ++e) st[(int64_t)k * dv + cl * CW + e] = tile[k * 8 * CW + cl * CW + e];
+        }
+    }
 }
 
-template <typename T, int CW, bool STEP>
+template <typename T, int CW>
 static int recur_launch(LightArgs a, const float* decay, int64_t B, hipStream_t s) {
-    const size_t lds = (size_t)(2 * a.dk + 32 + 32 * 33 + (STEP ? 0 : a.dk * 8 * CW)) * 4;
+    const size_t lds = (size_t)(2 * a.dk + 32 + 32 * 33) * 4;
+    hipLaunchKernelGGL((lightning_recur_kernel<T, CW>), dim3((unsigned)((a.dv + 8 * CW - 1) / (8 * CW)), (unsigned)a.H, (unsigned)B), dim3(256),
+                       lds, s, a, decay);
+    return evo_launch_status();
+}
+
+template <typename T, int CW, int R, int LT>
+static int tokens_launch(LightArgs a, const float* decay, int64_t B, hipStream_t s) {
+    const size_t lds = ((size_t)LT * (2 * a.dk + 32 + 32 * 33) + (R ? 0 : a.dk * 8 * CW)) * 4;
     if (lds > 160 * 1024) return -1;
-    if (lds > 64 * 1024)
-        (void)hipFuncSetAttribute((const void*)lightning_recur_kernel<T, CW, STEP>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL((lightning_recur_kernel<T, CW, STEP>), dim3((unsigned)((a.dv + 8 * CW - 1) / (8 * CW)), (unsigned)a.H, (unsigned)B), dim3(256),
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)lightning_tokens_kernel<T, CW, R, LT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL((lightning_tokens_kernel<T, CW, R, LT>), dim3((unsigned)((a.dv + 8 * CW - 1) / (8 * CW)), (unsigned)a.H, (unsigned)B), dim3(256),
                        lds, s, a, decay);
     return evo_launch_status();
 }
@@ -420,9 +540,11 @@ extern "C" int evo_lightning_recurrent(const void* z, int64_t ld, void* o, float
     LightArgs a = {z, o, state, nullptr, cu, resume, nullptr, ld, (int)H, (int)dk, (int)dv, 1, 0, act != 0};
     hipStream_t s = (hipStream_t)stream;
     const bool quad = dv % 4 == 0;
-#define LR(T)                                                                                                              \
-    (cu ? (quad && dk <= 1024 ? recur_launch<T, 4, false>(a, decay, B, s) : recur_launch<T, 1, false>(a, decay, B, s))       \
-        : (quad ? recur_launch<T, 4, true>(a, decay, B, s) : recur_launch<T, 1, true>(a, decay, B, s)))
+    // (up to 128 rows the state is in registers and eight tokens share a barrier; wider heads have room for one token's rows beside the state)
+#define LP(T) (dk <= 128 ? (quad ? tokens_launch<T, 4, 4, 8>(a, decay, B, s) : tokens_launch<T, 1, 4, 8>(a, decay, B, s))                                   \
+                         : (quad && dk <= 1024 ? tokens_launch<T, 4, 0, 1>(a, decay, B, s) : tokens_launch<T, 1, 0, 1>(a, decay, B, s)))
+#define LR(T) (cu ? LP(T) : (quad ? recur_launch<T, 4>(a, decay, B, s) : recur_launch<T, 1>(a, decay, B, s)))
     return f32 ? LR(float) : LR(uint16_t);
 #undef LR
+#undef LP
 }
