@@ -456,11 +456,11 @@ extern "C" int evo_rglru_step_bf16(const void* z, int64_t ld, const void* in_b, 
 }
 
 // ------------------------------------------------------------------------------------------------ any sizes, both storage types
-// gates: NT tokens of one block per workgroup; -> ab [M][2][W] = (a, sqrt(1 - a^2) i u).  A thread takes a channel's two rows of weights, V elements a request,
-// for NT tokens at once: 16 of a prompt (1,151 tokens x 16 blocks of 256: 628 us at four tokens and one element a request, 226
-// now), four of a decode step.
-template <typename T, int NT, int V>
+// gates, four tokens of one block per workgroup; -> ab [M][2][W] = (a, sqrt(1 - a^2) i u).  A thread takes a channel's two rows of weights, V elements a
+// request, for four tokens at once.
+template <typename T, int V>
 __global__ __launch_bounds__(256) void rglru_gates_any_kernel(RgArgs a, float* __restrict__ ab, int M) {
+    constexpr int NT = 4;
     extern __shared__ __attribute__((aligned(16))) float us[];   // [bs][NT]
     const int n = blockIdx.y, m0 = blockIdx.x * NT, bs = a.bs, W = a.W, nt = M - m0 < NT ? M - m0 : NT;
     for (int it = threadIdx.x; it < NT * bs; it += 256) {
@@ -513,20 +513,143 @@ __global__ __launch_bounds__(256) void rglru_gates_any_kernel(RgArgs a, float* _
     }
 }
 
+// The same in fp32 on the matrix cores (16 x 16 x 4), 16 tokens of 64 TC channels of a block per workgroup: lane (row l15, lq) requests four neighbouring weights
+// of channel l15 and reads as many inputs of token l15; a lane ends with four neighbouring channels of one token.  Prompts are bound by the fp32 matrix rate and the
+// convolution before it, a decode step by the latency of its loads.  (16 blocks of 256, MI355X, us: 1,151 tokens 137, on the vector units 268 -- every
+// product's input from LDS --; 3 tokens 19, 35 with a workgroup per block.)
+template <int TC>
+__global__ __launch_bounds__(256) void rglru_gates_f32_kernel(RgArgs a, float* __restrict__ ab, int M) {
+    constexpr int NT = 16;
+    extern __shared__ __attribute__((aligned(16))) float us[];   // [NT][pitch]: whole steps of 16 inputs, zeros behind the last
+    __shared__ int from[16 * NT];                                // [back][token]: its input `back` tokens ago is row r >= 0 of z, row -2 - r of the state, nothing (-1)
+    const int n = blockIdx.y, m0 = blockIdx.x * NT, bs = a.bs, W = a.W, nt = M - m0 < NT ? M - m0 : NT;
+    const int steps = (bs + 15) / 16, pitch = 16 * steps + 4;
+    if ((int)threadIdx.x < 16 * a.taps) {                        // (at most 16 taps)
+        const int i = threadIdx.x & 15, back = threadIdx.x >> 4, m = m0 + (i < nt ? i : nt - 1), b = a.seq ? a.seq[m] : m;
+        const int t = a.cu ? m - a.cu[b] : 0;                    // tokens of this portion before this one
+        const int64_t p = a.pos[m] - back;
+        int r = -1;
+        if (back <= t) r = m - back;
+        else if ((!a.cu || (a.resume && a.resume[b])) && p >= 0) r = -2 - (b * (1 + a.taps) + 1 + (int)(p % a.taps));
+        from[threadIdx.x] = r;
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k < 16 * steps; k += 256) {
+        if (k >= bs) {
+#pragma unroll
+            for (int i = 0; i < NT; ++i) us[i * pitch + k] = 0.f;
+            continue;
+        }
+        const int c = n * bs + k;
+        const float *cw = (const float*)a.conv + (int64_t)c * a.taps;
+        const float bias = a.in_b ? ((const float*)a.in_b)[W + c] : 0.f, cb = ((const float*)a.conv_b)[c];
+        float u[NT];
+#pragma unroll
+        for (int i = 0; i < NT; ++i) u[i] = cb;
+        for (int back = 0; back < a.taps; ++back) {              // (no branch between the requests: every token's is out before the first is waited for)
+            const float w = cw[a.taps - 1 - back];
+            float x[NT];
+            int r[NT];
+#pragma unroll
+            for (int i = 0; i < NT; ++i) {
+                r[i] = __builtin_amdgcn_readfirstlane(from[back * NT + i]);
+                const float* p = r[i] < -1 ? a.state + (int64_t)(-2 - r[i]) * W : (const float*)a.z + (int64_t)(r[i] < 0 ? m0 : r[i]) * a.ld + W;
+                x[i] = p[c];
+            }
+#pragma unroll
+            for (int i = 0; i < NT; ++i) u[i] = fmaf(w, r[i] >= 0 ? x[i] + bias : r[i] == -1 ? 0.f : x[i], u[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < NT; ++i) us[i * pitch + k] = u[i];
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l15 = lane & 15, lq = lane >> 4;
+    const int c0 = (blockIdx.z * 4 + wave) * 16 * TC;            // this wave's first channel in the block
+    if (c0 >= bs) return;
+    const float *wr[TC], *wi[TC];
+#pragma unroll
+    for (int t = 0; t < TC; ++t) {
+        const int c = c0 + 16 * t + l15 < bs ? c0 + 16 * t + l15 : bs - 1;
+        wr[t] = (const float*)a.ra + ((int64_t)n * bs + c) * bs + 4 * lq;
+        wi[t] = (const float*)a.ri + ((int64_t)n * bs + c) * bs + 4 * lq;
+    }
+    f32x4_t zr[TC], zi[TC];
+#pragma unroll
+    for (int t = 0; t < TC; ++t) zr[t] = zi[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const float* ur = us + l15 * pitch + 4 * lq;
+    auto step = [&](int k, bool whole) __attribute__((always_inline)) {
+        const f32x4_t u = *(const f32x4_t*)(ur + 16 * k);
+        f32x4_t p[TC], q[TC];
+#pragma unroll
+        for (int t = 0; t < TC; ++t) {
+            const bool in = whole || 16 * k + 4 * lq < bs;       // (bs % 4 == 0)
+            p[t] = in ? *(const f32x4_t*)(wr[t] + 16 * k) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+            q[t] = in ? *(const f32x4_t*)(wi[t] + 16 * k) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int t = 0; t < TC; ++t) {
+                zr[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[t][e], u[e], zr[t], 0, 0, 0);
+                zi[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[t][e], u[e], zi[t], 0, 0, 0);
+            }
+    };
+#pragma unroll 4
+    for (int k = 0; k < bs / 16; ++k) step(k, true);
+    if (bs % 16) step(steps - 1, false);
+    if (l15 >= nt) return;
+#pragma unroll
+    for (int t = 0; t < TC; ++t) {
+        const int c = c0 + 16 * t + 4 * lq, wc = n * bs + c;
+        if (c >= bs) continue;
+        float* d = ab + (int64_t)(m0 + l15) * 2 * W + wc;
+        float f[4], g[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float l = a.decay[wc + e] / (1.0f + expf(-(zr[t][e] + ((const float*)a.ra_b)[wc + e])));
+            f[e] = expf(l);
+            g[e] = sqrtf(-expm1f(2.0f * l)) / (1.0f + expf(-(zi[t][e] + ((const float*)a.ri_b)[wc + e]))) * us[l15 * pitch + c + e];
+        }
+        *(f32x4_t*)d = f32x4_t{f[0], f[1], f[2], f[3]};
+        *(f32x4_t*)(d + W) = f32x4_t{g[0], g[1], g[2], g[3]};
+    }
+}
+
+// (requests of SB tokens ahead of their chain: one token at a time it waits out a load per token, 190 us for 500 tokens; 85 so)
 template <typename T>
 __global__ __launch_bounds__(64) void rglru_scan_any_kernel(RgArgs a, const float* __restrict__ ab) {
+    constexpr int SB = 8;
     const int c = blockIdx.x * 64 + threadIdx.x, b = blockIdx.y, W = a.W;
     if (c >= W) return;
     const int row0 = a.cu ? a.cu[b] : b, len = a.cu ? a.cu[b + 1] - row0 : 1;
     float* st = a.state ? a.state + (int64_t)b * (1 + a.taps) * W + c : nullptr;
     float S = (!a.cu || (a.resume && a.resume[b])) && st ? st[0] : 0.f;
     const float bias = a.in_b ? ld1((const T*)a.in_b + c) : 0.f;
-    for (int t = 0; t < len; ++t) {
-        const int64_t m = row0 + t;
-        S = fmaf(ab[m * 2 * W + c], S, ab[m * 2 * W + W + c]);
-        float y = ld1((const T*)a.z + m * a.ld + c) + bias;
-        if (a.act) y = gelu_tanh_t<T>(y);
-        st1((T*)a.o + m * W + c, S * y);
+    float f[SB], g[SB], z[SB];
+    auto request = [&](int t0) {
+#pragma unroll
+        for (int i = 0; i < SB; ++i) {
+            const int64_t m = row0 + (t0 + i < len ? t0 + i : len - 1);
+            f[i] = ab[m * 2 * W + c];
+            g[i] = ab[m * 2 * W + W + c];
+            z[i] = ld1((const T*)a.z + m * a.ld + c);
+        }
+    };
+    if (len > 0) request(0);
+    for (int t0 = 0; t0 < len; t0 += SB) {
+        float y[SB];
+#pragma unroll
+        for (int i = 0; i < SB; ++i)
+            if (t0 + i < len) {
+                S = fmaf(f[i], S, g[i]);
+                y[i] = z[i] + bias;
+                if (a.act) y[i] = gelu_tanh_t<T>(y[i]);
+                y[i] *= S;
+            }
+        if (t0 + SB < len) request(t0 + SB);
+#pragma unroll
+        for (int i = 0; i < SB; ++i)
+            if (t0 + i < len) st1((T*)a.o + (int64_t)(row0 + t0 + i) * W + c, y[i]);
     }
     if (st && len > 0) st[0] = S;
 }
@@ -541,14 +664,23 @@ extern "C" int evo_rglru_any(const void* z, int64_t ld, const void* in_b, void* 
                 ld, (int)W, (int)nb, (int)(W / nb), (int)taps, 1, 0, 1, (int)act, (int)B};
     hipStream_t s = (hipStream_t)stream;
     const bool vec = f32 && (W / nb) % 4 == 0 && (((uintptr_t)ra | (uintptr_t)ri) & 15) == 0;
-    const int nt = vec && M >= 64 && W / nb <= 512 ? 16 : 4;
-    const dim3 g1((unsigned)((M + nt - 1) / nt), (unsigned)nb), g2((unsigned)((W + 63) / 64), (unsigned)B), g3((unsigned)((W + 255) / 256), (unsigned)B);
-    const size_t lds = (size_t)(W / nb) * nt * 4;                // (<= 64 KB)
+    const int bs = (int)(W / nb);
+    const bool mm = vec && bs <= 1024 && taps <= 16 && ((uintptr_t)ab & 15) == 0;      // (16 tokens' inputs in LDS: 65 KB)
+    const int64_t tiles = (M + 15) / 16 * nb;                    // of 16 tokens; a wave takes four channel tiles where that still fills the chip
+    const bool wide = tiles * ((bs + 255) / 256) >= 256;
+    const dim3 gm((unsigned)((M + 15) / 16), (unsigned)nb, (unsigned)(wide ? (bs + 255) / 256 : (bs + 63) / 64)), g1((unsigned)((M + 3) / 4), (unsigned)nb),
+        g2((unsigned)((W + 63) / 64), (unsigned)B), g3((unsigned)((W + 255) / 256), (unsigned)B);
+    const size_t lds = (size_t)bs * 4 * 4, lds_m = (size_t)16 * ((bs + 15) / 16 * 16 + 4) * 4;      // (<= 64 KB)
+    if (mm && lds_m > 60 * 1024) {
+        (void)hipFuncSetAttribute((const void*)rglru_gates_f32_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_m);
+        (void)hipFuncSetAttribute((const void*)rglru_gates_f32_kernel<1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_m);
+    }
 #define RA(T)                                                                                                              \
     do {                                                                                                                   \
-        if (vec && nt == 16) hipLaunchKernelGGL((rglru_gates_any_kernel<float, 16, 4>), g1, dim3(256), lds, s, a, ab, (int)M);    \
-        else if (vec) hipLaunchKernelGGL((rglru_gates_any_kernel<float, 4, 4>), g1, dim3(256), lds, s, a, ab, (int)M);     \
-        else hipLaunchKernelGGL((rglru_gates_any_kernel<T, 4, 1>), g1, dim3(256), lds, s, a, ab, (int)M);                  \
+        if (mm && wide) hipLaunchKernelGGL((rglru_gates_f32_kernel<4>), gm, dim3(256), lds_m, s, a, ab, (int)M);           \
+        else if (mm) hipLaunchKernelGGL((rglru_gates_f32_kernel<1>), gm, dim3(256), lds_m, s, a, ab, (int)M);              \
+        else if (vec) hipLaunchKernelGGL((rglru_gates_any_kernel<float, 4>), g1, dim3(256), lds, s, a, ab, (int)M);        \
+        else hipLaunchKernelGGL((rglru_gates_any_kernel<T, 1>), g1, dim3(256), lds, s, a, ab, (int)M);                     \
         hipLaunchKernelGGL((rglru_scan_any_kernel<T>), g2, dim3(64), 0, s, a, (const float*)ab);                           \
         if (state) hipLaunchKernelGGL((rglru_tail_kernel<T>), g3, dim3(256), 0, s, a);                                     \
     } while (0)
