@@ -297,6 +297,283 @@ __global__ __launch_bounds__(64 * NW, MINW) void window_attn_kernel(WinArgs a, i
     }
 }
 
+// The same for the head sizes below at length (bf16), with nothing but products and the softmax in the loop: rows of K and V go to LDS by DMA as they lie
+// (granules of 16 bytes XORed by their row on the source side), NS tiles of 64 keys deep, one barrier per tile, and the value fragments are read transposed.
+// A workgroup is eight waves of 32 queries (two column blocks); with two maps, four query groups by two maps -- a wave reads its map's keys only --, which
+// meet in LDS at the end.  A running maximum moves only when a score passes it by 2^WT_STEP (every rounding is relative; sums keep 2^-127 of room).
+// Causal blocks start with the longest.
+// Bound by the chain of a tile -- fragments, scores, maximum, exponentials, values -- of the two waves on a SIMD: about 3.5 us of which the matrix cores take 1.1 to 1.5.
+// MI355X, before (register staging, V transposed by 4-byte stores, one wave for both maps) -> here: two maps, 16 heads of 128 and 256, 8,190 tokens causal
+// 1,872 -> 943 us (874 TF); 32 heads of 192 and 128, window 1,024, six prompts of 700 to 2,500 tokens 526 -> 403; 32 heads of 128, window 1,024 and kept
+// tokens, 8,190 tokens 292 -> 217.  (Waves of a SIMD half a tile apart by two barriers per tile were slower: 465 for the second.)
+#define WT_STEP 8.0f
+typedef short wt_s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) wt_s16x4* wt_tr_ptr;
+// the maximum over the four lanes of a column (lanes 16 apart), one swap each instead of a trip through LDS
+__device__ __forceinline__ float wt_row_max(float v) {
+    const uint32_t u = __float_as_uint(v);
+    const auto p = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    v = fmaxf(__uint_as_float((uint32_t)p[0]), __uint_as_float((uint32_t)p[1]));
+    const uint32_t x = __float_as_uint(v);
+    const auto q = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return fmaxf(__uint_as_float((uint32_t)q[0]), __uint_as_float((uint32_t)q[1]));
+}
+template <int DN, int DR, int DV, int MAPS, bool KEEP>
+__global__ __launch_bounds__(512, 2) void window_tile_kernel(WinArgs a, int B) {
+    static_assert(DN == 128 && (DR == 0 || DR == 64) && (DV == 128 || DV == 256) && (MAPS == 1 || DR == 0), "row widths of the swizzles");
+    constexpr int KN = 64 * DN * 2, KR = 64 * DR * 2, VB = 64 * DV * 2, STAGE = MAPS * KN + KR + VB, NS = STAGE > 48 * 1024 ? 2 : STAGE > 36 * 1024 ? 3 : 4;
+    constexpr int KS = DN / 32, RS = DR / 32, DVB = DV / 16, PK = KN / 8192, PR = KR / 8192, PV = VB / 8192, P = MAPS * PK + PR + PV;   // DMA pieces (1 KiB) per wave
+    constexpr int VRP = 1024 / (2 * DV), VG = DV / 8;            // value rows per piece, granules of a value row
+    constexpr int QB = 256 / MAPS;
+    static_assert(NS * STAGE <= 160 * 1024, "the CU's LDS");
+    __shared__ __attribute__((aligned(16))) unsigned char smem[NS * STAGE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c16 = lane & 15, g = lane >> 4;
+    const int map = MAPS == 2 ? wave >> 2 : 0, grp = MAPS == 2 ? wave & 3 : wave;      // (waves w and w + 4 share a SIMD)
+    // the query blocks of a (sequence, head) share most of their keys: consecutive work items stay on one XCD (block b runs on XCD b % 8)
+    const int per_xcd = gridDim.x >> 3;
+    const int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    const int qb = a.n_qb - 1 - item % a.n_qb, h = item / a.n_qb % a.H, b = item / a.n_qb / a.H;
+    if (b >= B) return;                                          // (the grid is rounded up to a multiple of 8)
+    const int q0 = a.cu_q[b], nq = a.cu_q[b + 1] - q0, k0 = a.cu_k[b], nk = a.cu_k[b + 1] - k0;
+    if (qb * QB >= nq) return;
+    const int off = nk - nq;                                     // key index of query 0
+    const int hk = h / a.grp;
+    constexpr int dh = DN + DR;
+    const uint64_t kr = (uint64_t)((const uint16_t*)a.kr + (int64_t)k0 * DR);
+    const uint64_t kn = (uint64_t)((const uint16_t*)a.kn + (int64_t)k0 * a.ldkv + (int64_t)hk * DN * MAPS);
+    const uint64_t vg = (uint64_t)((const uint16_t*)a.v + (int64_t)k0 * a.ldkv + (int64_t)hk * DV);
+    const uint32_t rowb = (uint32_t)a.ldkv * 2;
+
+    mx_frag qf[2][KS + RS];
+    int qi[2];                                                   // this lane's query of each column block, as a key index
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const int i = qb * QB + grp * 32 + 16 * c + c16;
+        qi[c] = i + off;
+        const uint16_t* p = (const uint16_t*)a.q + (int64_t)(q0 + (i < nq ? i : nq - 1)) * a.ldq + (int64_t)(h * MAPS + map) * dh;
+#pragma unroll
+        for (int ks = 0; ks < KS + RS; ++ks) qf[c][ks] = __builtin_bit_cast(mx_frag, *(const uint4*)(p + 32 * ks + 8 * g));
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int ks = 0; ks < KS + RS; ++ks) asm volatile("" : "+v"(qf[c][ks]));       // (waited for here: a wait in the loop would be one for the DMA)
+
+    // DMA: piece i of this wave is piece wave + 8 i of a slab: key rows 4 to a piece (granule r ^ (row & 15)), shared key rows 8 (r ^ (row / 2 & 7)), value
+    // rows 2 or 4 (r ^ 2 (row & 7)).  Row offsets are in the lanes' part: the descriptor's bound returns zeros behind the last key.
+    typedef uint32_t wt_u32x4 __attribute__((ext_vector_type(4)));
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+    const int kr_ = 4 * wave + (lane >> 4), rr_ = 8 * wave + (lane >> 3), vr_ = VRP * wave + lane / VG;
+    const uint32_t k_off = (uint32_t)kr_ * rowb + (uint32_t)(((lane & 15) ^ (kr_ & 15)) * 16);
+    const uint32_t r_off = (uint32_t)rr_ * (2 * DR) + (uint32_t)(((lane & 7) ^ ((rr_ >> 1) & 7)) * 16);
+    const uint32_t v_off = (uint32_t)vr_ * rowb + (uint32_t)(((lane % VG) ^ (2 * (vr_ & 7))) * 16);
+    auto dma = [&](uint32_t dst, uint32_t voff, wt_u32x4 rsrc) __attribute__((always_inline)) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(dst), "v"(voff), "s"(rsrc) : "memory", "m0");
+    };
+    auto fetch = [&](int j0, bool any, int slot) __attribute__((always_inline)) {      // (none: the same requests with an empty bound)
+        const int left = any ? (nk - j0 < 64 ? nk - j0 : 64) : 0;
+        const uint64_t ka = kn + (any ? (uint64_t)j0 * rowb : 0), va = vg + (any ? (uint64_t)j0 * rowb : 0), ra = kr + (any ? (uint64_t)j0 * (2 * DR) : 0);
+        const uint32_t rows = left > 0 ? (uint32_t)(left - 1) * rowb : 0u;
+        const wt_u32x4 sk = {(uint32_t)ka, (uint32_t)(ka >> 32) & 0xffffu, left > 0 ? rows + MAPS * DN * 2 : 0u, 0x00020000u};
+        const wt_u32x4 sv = {(uint32_t)va, (uint32_t)(va >> 32) & 0xffffu, left > 0 ? rows + DV * 2 : 0u, 0x00020000u};
+        const wt_u32x4 sr = {(uint32_t)ra, (uint32_t)(ra >> 32) & 0xffffu, (uint32_t)left * (2 * DR), 0x00020000u};
+        const uint32_t base = lds0 + (uint32_t)slot * STAGE + wave * 1024;
+#pragma unroll
+        for (int m = 0; m < MAPS; ++m)
+#pragma unroll
+            for (int i = 0; i < PK; ++i) dma(base + m * KN + i * 8192, k_off + (uint32_t)i * 32u * rowb + m * (DN * 2), sk);
+        if constexpr (DR > 0) {
+#pragma unroll
+            for (int i = 0; i < PR; ++i) dma(base + MAPS * KN + i * 8192, r_off + i * (64 * 2 * DR), sr);
+        }
+#pragma unroll
+        for (int i = 0; i < PV; ++i) dma(base + MAPS * KN + KR + i * 8192, v_off + (uint32_t)(i * 8 * VRP) * rowb, sv);
+    };
+
+    const float sc2 = a.scale * LOG2E;
+    f32x4_t o[2][DVB];
+    float mx[2], den[2];                                         // den: this lane's share (its keys); the sink sits in lane group 0's
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        mx[c] = a.sink ? fmaxf(a.sink[h] * LOG2E, FLOOR) : FLOOR;
+        den[c] = a.sink && g == 0 ? 1.0f : 0.0f;
+#pragma unroll
+        for (int db = 0; db < DVB; ++db) o[c][db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    // fragment addresses in a stage: key row c16 (+ 16 jb), granule 4 ks + g; value rows 4 g + c16 / 4 (+ 16 u), columns 16 db + 4 (c16 % 4)
+    uint32_t k_rd[KS], r_rd[RS > 0 ? RS : 1], v_rd[8];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) k_rd[ks] = map * KN + c16 * (DN * 2) + ((4 * ks + g) ^ c16) * 16;
+#pragma unroll
+    for (int ks = 0; ks < RS; ++ks) r_rd[ks] = MAPS * KN + c16 * (DR * 2) + ((4 * ks + g) ^ ((c16 >> 1) & 7)) * 16;
+#pragma unroll
+    for (int db = 0; db < 8; ++db) {
+        const int r = 4 * g + (c16 >> 2);
+        v_rd[db] = MAPS * KN + KR + r * (DV * 2) + ((2 * db + ((c16 & 3) >> 1)) ^ (2 * (r & 7))) * 16 + (c16 & 1) * 8;
+    }
+
+    const int last_q = (qb + 1) * QB < nq ? (qb + 1) * QB - 1 : nq - 1;
+    int j_lo = qb * QB + off - a.window + 1;
+    j_lo = j_lo < 0 ? 0 : j_lo & ~63;
+    const int j_hi = last_q + off;                               // last key any row of this block sees
+    const int w_first = qb * QB + grp * 32 + off, w_last = w_first + 31;        // this wave's queries as key indexes
+    const int keep = !KEEP ? 0 : (a.keep < j_lo ? a.keep : j_lo);   // kept keys ahead of the window's tiles: tiles [0, keep) come first
+    auto after = [&](int j) { return KEEP && j < j_lo && j + 64 >= keep ? j_lo : j + 64; };
+    int j0 = keep > 0 ? 0 : j_lo, jf = j0, slot = 0, fslot = NS - 1;
+#pragma unroll
+    for (int t = 0; t < NS - 1; ++t) {
+        fetch(jf, jf <= j_hi, t);
+        if (jf <= j_hi) jf = after(jf);
+    }
+    for (; j0 <= j_hi; j0 = after(j0)) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * P) : "memory");     // own pieces of this tile; barrier: everyone's, and everyone is done with the last
+        asm volatile("s_barrier" ::: "memory");
+        fetch(jf, jf <= j_hi, fslot);
+        if (jf <= j_hi) jf = after(jf);
+        const unsigned char* st = smem + slot * STAGE;
+        fslot = slot;
+        slot = slot + 1 == NS ? 0 : slot + 1;
+        if (!(j0 <= w_last && (j0 + 63 > w_first - a.window || (KEEP && j0 < a.keep)))) continue;   // no query of this wave sees a key of the tile
+        f32x4_t s[2][4];
+        {
+            constexpr int KF = KS + RS, NF = 4 * KF, D = 4;      // fragments of the tile; read ahead
+            auto frag = [&](int f) __attribute__((always_inline)) {
+                const int jb = f / KF, ks = f % KF;
+                return *(const uint4*)(ks < KS ? st + k_rd[ks < KS ? ks : 0] + jb * (16 * DN * 2) : st + r_rd[ks < KS ? 0 : ks - KS] + jb * (16 * DR * 2));
+            };
+            uint4 kf[D];
+#pragma unroll
+            for (int f = 0; f < D; ++f) kf[f] = frag(f);
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+                const int jb = f / KF, ks = f % KF;
+                if (ks == 0) s[0][jb] = s[1][jb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int c = 0; c < 2; ++c) s[c][jb] = mfma16(__builtin_bit_cast(mx_frag, kf[f % D]), qf[c][ks], s[c][jb]);
+                if (f + D < NF) kf[f % D] = frag(f + D);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (j0 + 63 > w_first || (j0 <= w_last - a.window && (!KEEP || j0 + 63 >= a.keep))) {   // the tile holds an edge of some query's window
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+#pragma unroll
+                for (int jb = 0; jb < 4; ++jb)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int j = j0 + 16 * jb + 4 * g + r, age = qi[c] - j;
+                        s[c][jb][r] = age >= 0 && (age < a.window || (KEEP && j < a.keep)) ? s[c][jb][r] : -INFINITY;
+                    }
+        }
+        mx_frag pf[2][2];
+        // (both column blocks side by side: their chains fill each other's latencies)
+        float top[2];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            float t[4];
+#pragma unroll
+            for (int jb = 0; jb < 4; ++jb) t[jb] = fmaxf(fmaxf(s[c][jb][0], s[c][jb][1]), fmaxf(s[c][jb][2], s[c][jb][3]));
+            top[c] = wt_row_max(fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3]))) * sc2;
+        }
+        if (__builtin_amdgcn_ballot_w64(top[0] > mx[0] + WT_STEP || top[1] > mx[1] + WT_STEP)) {       // a running maximum moves in some column: rescale
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const float m = fmaxf(mx[c], top[c]), f = __builtin_amdgcn_exp2f(mx[c] - m);
+                mx[c] = m;
+                den[c] *= f;
+#pragma unroll
+                for (int db = 0; db < DVB; ++db)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[c][db][r] *= f;
+            }
+        }
+        uint32_t w[2][8];
+#pragma unroll
+        for (int jb = 0; jb < 4; ++jb)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                float e[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) e[r] = __builtin_amdgcn_exp2f(fmaf(s[c][jb][r], sc2, -mx[c]));
+                den[c] += (e[0] + e[1]) + (e[2] + e[3]);
+                w[c][2 * jb] = pack_bf2(e[0], e[1]);
+                w[c][2 * jb + 1] = pack_bf2(e[2], e[3]);
+            }
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int jj = 0; jj < 2; ++jj) pf[c][jj] = frag_of(w[c][4 * jj], w[c][4 * jj + 1], w[c][4 * jj + 2], w[c][4 * jj + 3]);
+        {
+            constexpr int NF = 2 * DVB, D = 4;
+            uint2 va[D], vb[D];
+            auto frag = [&](int f, int i) __attribute__((always_inline)) {
+                const int jj = f / DVB, db = f % DVB;
+                const unsigned char* p = st + v_rd[db & 7] + (db >> 3) * 256 + jj * (32 * DV * 2);
+                va[i] = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((wt_tr_ptr)p));
+                vb[i] = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((wt_tr_ptr)(p + 16 * DV * 2)));
+            };
+#pragma unroll
+            for (int f = 0; f < D; ++f) frag(f, f);
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+                const mx_frag vf = frag_of(va[f % D].x, va[f % D].y, vb[f % D].x, vb[f % D].y);
+#pragma unroll
+                for (int c = 0; c < 2; ++c) o[c][f % DVB] = mfma16(vf, pf[c][f / DVB], o[c][f % DVB]);
+                if (f + D < NF) frag(f + D, f % D);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");             // (the empty requests: nothing may land after the exit, or on what comes below)
+    float inv[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        float l = den[c];
+        l += __shfl_xor(l, 16, 64);
+        l += __shfl_xor(l, 32, 64);
+        inv[c] = 1.0f / l;
+    }
+    if constexpr (MAPS == 2) {                                   // the difference of the maps, its unit norm over the head's values
+        f32x4_t* x = (f32x4_t*)smem + grp * (2 * DVB * 64) + lane;      // [4 query groups][2][DVB][64 lanes]: 128 KB
+        asm volatile("s_barrier" ::: "memory");                  // (everyone is done with the last tile)
+        if (map == 1) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+#pragma unroll
+                for (int db = 0; db < DVB; ++db) x[(c * DVB + db) * 64] = o[c][db] * (inv[c] * a.lam);
+        }
+        __syncthreads();
+        if (map == 1) return;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            float ss = 0.f;
+#pragma unroll
+            for (int db = 0; db < DVB; ++db) {
+                const f32x4_t y = x[(c * DVB + db) * 64];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    o[c][db][r] = fmaf(o[c][db][r], inv[c], -y[r]);
+                    ss = fmaf(o[c][db][r], o[c][db][r], ss);
+                }
+            }
+            ss += __shfl_xor(ss, 16, 64);
+            ss += __shfl_xor(ss, 32, 64);
+            inv[c] = a.gain / sqrtf(ss / (float)DV + a.eps);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        const int i = qi[c] - off;
+        if (i < nq) {
+            uint16_t* op = (uint16_t*)a.o + (int64_t)(q0 + i) * a.H * DV + (int64_t)h * DV + 4 * g;
+#pragma unroll
+            for (int db = 0; db < DVB; ++db)
+                *(uint2*)(op + 16 * db) = make_uint2(pack_bf2(o[c][db][0] * inv[c], o[c][db][1] * inv[c]), pack_bf2(o[c][db][2] * inv[c], o[c][db][3] * inv[c]));
+        }
+    }
+}
+
 // fp32 on the matrix cores (v_mfma_f32_16x16x4_f32: fp32 operands and sums).  A workgroup: 64 queries of one (sequence, head), 16 a wave as MFMA columns;
 // 32 keys at a time in LDS, the rows of K and V 4 floats apart from a multiple of 64 (both read patterns meet every bank once).  Scores come as
 // S^T = K Q^T with the reduced index taken as d = 16 s + 4 g + j (a lane's four d are one 16-byte read), a lane holds keys 4 g + r of its query, which is
@@ -525,6 +802,19 @@ extern "C" int evo_window_attn(const void* q, int64_t ldq, const void* kn, const
     if (!f32 && mfma && dq <= (maps == 2 ? 128 : 256) && dv <= 256) {
         const bool vec = dn % 8 == 0 && dr % 8 == 0 && dv % 8 == 0 && ldq % 8 == 0 && ldkv % 8 == 0 && ldkv <= 0xffffff &&
                          (((uintptr_t)q | (uintptr_t)kn | (uintptr_t)v | (uintptr_t)kr) & 15) == 0;
+        // (more than one block of queries of the workgroups below, head sizes of their swizzles, a positive scale: the maximum is taken before it)
+        if (vec && max_q > 128 && scale > 0.f && dn == 128 && ((dr == 64 && dv == 128 && !kp && maps == 1) || (dr == 0 && (maps == 1 ? dv == 128 : dv == 256 && !kp)))) {
+            a.n_qb = (int)((max_q + 256 / maps - 1) / (256 / maps));
+            const int64_t items = (int64_t)a.n_qb * H * B;
+            if (items <= 0x7ffffff0) {
+                const dim3 wg((unsigned)((items + 7) / 8 * 8)), wb(512);
+                if (maps == 2) hipLaunchKernelGGL((window_tile_kernel<128, 0, 256, 2, false>), wg, wb, 0, s, a, (int)B);
+                else if (dr) hipLaunchKernelGGL((window_tile_kernel<128, 64, 128, 1, false>), wg, wb, 0, s, a, (int)B);
+                else if (kp) hipLaunchKernelGGL((window_tile_kernel<128, 0, 128, 1, true>), wg, wb, 0, s, a, (int)B);
+                else hipLaunchKernelGGL((window_tile_kernel<128, 0, 128, 1, false>), wg, wb, 0, s, a, (int)B);
+                return evo_launch_status();
+            }
+        }
 #define WA1(KS, DVB, QC, VEC, KEEP, MAPS, MINW, NW)                                                                        \
     do {                                                                                                                   \
         a.n_qb = (int)((max_q + 16 * NW * QC / MAPS - 1) / (16 * NW * QC / MAPS));                                         \
