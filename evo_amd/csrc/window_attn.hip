@@ -336,8 +336,11 @@ __global__ __launch_bounds__(512, 2) void window_tile_kernel(WinArgs a, int B) {
     const int qb = a.n_qb - 1 - item % a.n_qb, h = item / a.n_qb % a.H, b = item / a.n_qb / a.H;
     if (b >= B) return;                                          // (the grid is rounded up to a multiple of 8)
     const int q0 = a.cu_q[b], nq = a.cu_q[b + 1] - q0, k0 = a.cu_k[b], nk = a.cu_k[b + 1] - k0;
-    if (qb * QB >= nq) return;
     const int off = nk - nq;                                     // key index of query 0
+    // two maps: blocks of 32 queries start at multiples of 32 keys, so that every tile a wave takes holds a key that all of its queries see (a value that
+    // is not finite goes no further than with blocks of 16); block 0 is the short one
+    const int qs = qb * QB - (MAPS == 2 ? off & 31 : 0);         // this workgroup's first query (may be negative)
+    if (qs >= nq) return;
     const int hk = h / a.grp;
     constexpr int dh = DN + DR;
     const uint64_t kr = (uint64_t)((const uint16_t*)a.kr + (int64_t)k0 * DR);
@@ -349,9 +352,9 @@ __global__ __launch_bounds__(512, 2) void window_tile_kernel(WinArgs a, int B) {
     int qi[2];                                                   // this lane's query of each column block, as a key index
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-        const int i = qb * QB + grp * 32 + 16 * c + c16;
+        const int i = qs + grp * 32 + 16 * c + c16;
         qi[c] = i + off;
-        const uint16_t* p = (const uint16_t*)a.q + (int64_t)(q0 + (i < nq ? i : nq - 1)) * a.ldq + (int64_t)(h * MAPS + map) * dh;
+        const uint16_t* p = (const uint16_t*)a.q + (int64_t)(q0 + (i < 0 ? 0 : i < nq ? i : nq - 1)) * a.ldq + (int64_t)(h * MAPS + map) * dh;
 #pragma unroll
         for (int ks = 0; ks < KS + RS; ++ks) qf[c][ks] = __builtin_bit_cast(mx_frag, *(const uint4*)(p + 32 * ks + 8 * g));
     }
@@ -413,11 +416,11 @@ __global__ __launch_bounds__(512, 2) void window_tile_kernel(WinArgs a, int B) {
         v_rd[db] = MAPS * KN + KR + r * (DV * 2) + ((2 * db + ((c16 & 3) >> 1)) ^ (2 * (r & 7))) * 16 + (c16 & 1) * 8;
     }
 
-    const int last_q = (qb + 1) * QB < nq ? (qb + 1) * QB - 1 : nq - 1;
-    int j_lo = qb * QB + off - a.window + 1;
+    const int last_q = qs + QB < nq ? qs + QB - 1 : nq - 1;
+    int j_lo = qs + off - a.window + 1;
     j_lo = j_lo < 0 ? 0 : j_lo & ~63;
     const int j_hi = last_q + off;                               // last key any row of this block sees
-    const int w_first = qb * QB + grp * 32 + off, w_last = w_first + 31;        // this wave's queries as key indexes
+    const int w_first = qs + grp * 32 + off, w_last = w_first + 31;             // this wave's queries as key indexes
     const int keep = !KEEP ? 0 : (a.keep < j_lo ? a.keep : j_lo);   // kept keys ahead of the window's tiles: tiles [0, keep) come first
     auto after = [&](int j) { return KEEP && j < j_lo && j + 64 >= keep ? j_lo : j + 64; };
     int j0 = keep > 0 ? 0 : j_lo, jf = j0, slot = 0, fslot = NS - 1;
@@ -565,7 +568,7 @@ __global__ __launch_bounds__(512, 2) void window_tile_kernel(WinArgs a, int B) {
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
         const int i = qi[c] - off;
-        if (i < nq) {
+        if (i >= 0 && i < nq) {
             uint16_t* op = (uint16_t*)a.o + (int64_t)(q0 + i) * a.H * DV + (int64_t)h * DV + 4 * g;
 #pragma unroll
             for (int db = 0; db < DVB; ++db)
@@ -802,9 +805,10 @@ extern "C" int evo_window_attn(const void* q, int64_t ldq, const void* kn, const
     if (!f32 && mfma && dq <= (maps == 2 ? 128 : 256) && dv <= 256) {
         const bool vec = dn % 8 == 0 && dr % 8 == 0 && dv % 8 == 0 && ldq % 8 == 0 && ldkv % 8 == 0 && ldkv <= 0xffffff &&
                          (((uintptr_t)q | (uintptr_t)kn | (uintptr_t)v | (uintptr_t)kr) & 15) == 0;
-        // (more than one block of queries of the workgroups below, head sizes of their swizzles, a positive scale: the maximum is taken before it)
-        if (vec && max_q > 128 && scale > 0.f && dn == 128 && ((dr == 64 && dv == 128 && !kp && maps == 1) || (dr == 0 && (maps == 1 ? dv == 128 : dv == 256 && !kp)))) {
-            a.n_qb = (int)((max_q + 256 / maps - 1) / (256 / maps));
+        // (more than one block of queries of the workgroups below, head sizes of their swizzles, a positive scale: the maximum is taken before it;
+        //  two maps without a window: at its lower edge a block of 32 queries reaches 16 keys further than one of 16)
+        if (vec && max_q > 128 && scale > 0.f && dn == 128 && ((dr == 64 && dv == 128 && !kp && maps == 1) || (dr == 0 && (maps == 1 ? dv == 128 : dv == 256 && !kp && w >= 1 << 29)))) {
+            a.n_qb = (int)(maps == 2 ? (max_q + 31 + 127) / 128 : (max_q + 255) / 256);
             const int64_t items = (int64_t)a.n_qb * H * B;
             if (items <= 0x7ffffff0) {
                 const dim3 wg((unsigned)((items + 7) / 8 * 8)), wb(512);

@@ -34,6 +34,20 @@ def test_matches_the_any_size_form(H, G, maps, dr, dv, window, keep, sink, lens,
     assert torch.equal(fast, both(z, kv, kr, *args)[0].float())
 
 
+@pytest.mark.parametrize("H,G,maps,dr,dv", [(2, 2, 1, 64, 128), (2, 1, 1, 0, 128), (2, 2, 2, 0, 256)])
+@pytest.mark.parametrize("past", [0, 5, 16, 40])
+def test_an_infinite_value_stays_near_its_key(H, G, maps, dr, dv, past):
+    """Queries before the tile of 64 keys that holds it, and those whose whole block of 32 (two maps: the whole tile) lies before it, stay finite."""
+    g = torch.Generator(device=DEV).manual_seed(past)
+    n, dn, at = 400, 128, 200
+    z, kv = torch.randn(n, H * maps * (dn + dr), device=DEV, generator=g).bfloat16(), torch.randn(n + past, G * (maps * dn + dv), device=DEV, generator=g).bfloat16()
+    kv[at, G * maps * dn:] = float("inf")
+    kr = torch.randn(n + past, dr, device=DEV, generator=g).bfloat16() if dr else None
+    fast = both(z, kv, kr, None, H, G, maps, dn, dr, dv, 1 << 29, 0, 0.08, [n], [past])[0]
+    clean = at // 64 * 64 - past - (0 if maps == 2 else 31)        # (one map: a block of 32 queries that reaches the tile)
+    assert bool(torch.isfinite(fast[:clean]).all()) and not bool(torch.isfinite(fast[at - past:]).any())
+
+
 def test_negative_scale_and_short_prompts_take_the_other_kernels():
     g = torch.Generator(device=DEV).manual_seed(1)
     z, kv = torch.randn(200, 256, device=DEV, generator=g).bfloat16(), torch.randn(200, 512, device=DEV, generator=g).bfloat16()
