@@ -394,7 +394,7 @@ __global__ __launch_bounds__(256) void heads_decode_kernel(HDecArgs a) {
 }
 
 // Any sizes, both storage types: one wave per (split, head and map, sequence).  V = 4: fp32 rows in 16-byte requests (190 us for 3 sequences x 16 heads
-// of two maps behind 500 tokens element by element, 62 now)
+// of two maps behind 500 tokens element by element, 61 with a lane per key row, 38 with four lanes a row and a wave per 64 slots)
 template <typename T, int V>
 __global__ __launch_bounds__(64) void heads_decode_any_kernel(HDecArgs a, int maps) {
     extern __shared__ __attribute__((aligned(16))) float qs[];
@@ -413,18 +413,12 @@ __global__ __launch_bounds__(64) void heads_decode_any_kernel(HDecArgs a, int ma
     for (int s0 = split * 64; s0 < used; s0 += a.n_split * 64) {
         const int slot = s0 + lane;
         float s = -INFINITY;
-        if (slot < used) {
+        if constexpr (V == 4) {
+            const float dot = dot_rows((const float*)k + (int64_t)s0 * a.rs, a.rs, qs, a.dim, used - s0, lane);
+            if (slot < used) s = dot * a.sc2;
+        } else if (slot < used) {
             s = 0.f;
-            if constexpr (V == 4) {
-                const float* row = (const float*)k + (int64_t)slot * a.rs;
-#pragma unroll 8
-                for (int d = 0; d < a.dim; d += 4) {
-                    const f32x4_t x = *(const f32x4_t*)(row + d), y = *(const f32x4_t*)(qs + d);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) s = fmaf(y[e], x[e], s);
-                }
-            } else
-                for (int d = 0; d < a.dim; ++d) s = fmaf(qs[d], ld1(k + (int64_t)slot * a.rs + d), s);
+            for (int d = 0; d < a.dim; ++d) s = fmaf(qs[d], ld1(k + (int64_t)slot * a.rs + d), s);
             s *= a.sc2;
         }
         const float top = fmaxf(m, wave_max(s)), f = exp2f(m - top), p = exp2f(s - top);

@@ -332,7 +332,7 @@ __global__ __launch_bounds__(512, 2) void latent_decode_kernel(DecArgs a) {
 }
 
 // Any sizes, both storage types: one wave per (split, head, sequence).  V = 4: fp32 rows in 16-byte requests (a lane's key row element by element was one
-// 4-byte request of 64 lines per product: 154 us for 3 sequences x 32 heads behind 500 tokens of 576, 45 now).
+// 4-byte request of 64 lines per product: 154 us for 3 sequences x 32 heads behind 500 tokens of 576, 45 in 16-byte ones, 36 with four lanes a row).
 template <typename T, int V>
 __global__ __launch_bounds__(64) void latent_decode_any_kernel(DecArgs a, int dq) {
     extern __shared__ __attribute__((aligned(16))) float qf[];
@@ -355,18 +355,13 @@ __global__ __launch_bounds__(64) void latent_decode_any_kernel(DecArgs a, int dq
         for (int s0 = split * 64; s0 < used; s0 += a.n_split * 64) {
             const int slot = s0 + lane;
             float s = -INFINITY;
-            if (slot < used && slot_seen(slot, pos, cur, a)) {
+            const bool seen = slot < used && slot_seen(slot, pos, cur, a);
+            if constexpr (V == 4) {
+                const float dot = dot_rows((const float*)base + (int64_t)s0 * a.rs, a.rs, qf, dq, used - s0, lane);
+                if (seen) s = dot * a.sc2;
+            } else if (seen) {
                 s = 0.f;
-                if constexpr (V == 4) {
-                    const float* row = (const float*)base + (int64_t)slot * a.rs;
-#pragma unroll 8
-                    for (int d = 0; d < dq; d += 4) {
-                        const f32x4_t x = *(const f32x4_t*)(row + d), y = *(const f32x4_t*)(qf + d);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) s = fmaf(y[e], x[e], s);
-                    }
-                } else
-                    for (int d = 0; d < dq; ++d) s = fmaf(qf[d], ld1(base + (int64_t)slot * a.rs + d), s);
+                for (int d = 0; d < dq; ++d) s = fmaf(qf[d], ld1(base + (int64_t)slot * a.rs + d), s);
                 s *= a.sc2;
             }
             const float top = fmaxf(m, wave_max(s));

@@ -425,7 +425,8 @@ class MixerOps:
         self._dense(cache, (rows, ring, rs), "key and value cache")
         assert rows >= B and z.shape[1] >= heads * maps * dim and rs >= kv_heads * (maps * dim + dv)
         if n_split is None:
-            n_split = self.heads_split(B * kv_heads * ((heads // kv_heads + 15) // 16), ring)
+            # (fp32: one wave per part, head and sequence, 64 slots a round)
+            n_split = max(1, min((ring + 63) // 64, 4096 // (B * heads * maps), 64)) if f32 else self.heads_split(B * kv_heads * ((heads // kv_heads + 15) // 16), ring)
         part_o = torch.empty(B, heads * maps, n_split, dv, dtype=torch.float32, device=z.device)
         part_ml = torch.empty(B, heads * maps, n_split, 2, dtype=torch.float32, device=z.device)
         self._call("evo_heads_decode", z.data_ptr(), z.stride(0), cache.data_ptr(), self._ix(pos, torch.int64, B, "pos"), part_o.data_ptr(),
