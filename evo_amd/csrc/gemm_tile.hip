@@ -61,6 +61,10 @@ __device__ __forceinline__ void t_scale_bias(float (&v)[8], const GemmArgs& a, f
     }
 }
 
+// Rows of the statistic that a launch stores: its own.  (ss_ld is the pitch of a strip, counted from the first row of the layer: a tail that starts at row m0
+// and stored up to there would reach the next strip's first rows.)
+__host__ __device__ __forceinline__ int64_t t_stat_rows(const GemmArgs& a) { return a.M; }
+
 template <int BM, int BN, int WGM, int WGN, int NS, int PER_CU, int MODE, bool XB, bool SPLIT>
 __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_tile_kernel(GemmArgs a, int act, float* parts, int splits) {
     constexpr int NW = WGM * WGN, WM = BM / WGM, WN = BN / WGN, MT = WM / 16, NT = WN / 16;
@@ -323,7 +327,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
                         t += __shfl_xor(t, 16);
                         t += __shfl_xor(t, 32);
                         const int64_t m = m0 + wm * WM + 16 * j + l15;
-                        if (lq == 0 && m < a.ss_ld) a.ss[(int64_t)(n0 >> 7) * a.ss_ld + m] = t;
+                        if (lq == 0 && m < t_stat_rows(a)) a.ss[(int64_t)(n0 >> 7) * a.ss_ld + m] = t;
                     }
                 }
             }
@@ -513,6 +517,26 @@ extern "C" int evo_dense_ws(int64_t mode, int64_t stats, int64_t M, int64_t N, i
     for (int i = 0; i < n; ++i)
         if (plan[i].splits > 1 && plan[i].splits * plan[i].rows * N * 4 > most) most = plan[i].splits * plan[i].rows * N * 4;
     return (int)most;
+}
+
+extern "C" int evo_dense_plan(int64_t mode, int64_t stats, int64_t M, int64_t N, int64_t K, int64_t* out) {
+    if (!dense_shape(mode, M, N, K) || !out) return -1;
+    TilePlan plan[2];
+    const int n = dense_plan(mode, stats != 0, M, N, K, true, plan);
+    int64_t m0 = 0;
+    for (int i = 0; i < n; ++i) {
+        const TilePlan& t = plan[i];
+        const int bm = t.kind == T_PERSISTENT ? 256 : mode == 3 ? kinds[t.kind].bn : kinds[t.kind].bm, bn = t.kind == T_PERSISTENT ? 256 : mode == 3 ? kinds[t.kind].bm : kinds[t.kind].bn;
+        GemmArgs a;
+        a.M = t.rows;
+        a.ss_ld = (M + 255) / 256 * 256;
+        const int64_t tiles_end = (t.rows + bm - 1) / bm * bm;   // (the persistent kernel stores the statistic of whole tiles)
+        const int64_t stored = !stats ? 0 : t.kind != T_PERSISTENT && t_stat_rows(a) < tiles_end ? t_stat_rows(a) : tiles_end;
+        const int64_t row[7] = {m0, t.rows, bm, bn, t.splits, t.kind == T_PERSISTENT, m0 + stored};
+        for (int k = 0; k < 7; ++k) out[7 * i + k] = row[k];
+        m0 += t.rows;
+    }
+    return n;
 }
 
 extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const void* x, const void* w, const void* bias, const void* residual, void* y,

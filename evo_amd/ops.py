@@ -49,6 +49,7 @@ _SIGNATURES = {
     "evo_put_tokens": ([_PTR, _I64, _PTR, _PTR, _I64, _PTR], _c.c_int),
     "evo_advance_positions": ([_PTR, _I64, _I64, _PTR], _c.c_int),
     "evo_dense_ws": ([_I64] * 5, _c.c_int),
+    "evo_dense_plan": ([_I64] * 5 + [_PTR], _c.c_int),
     "evo_dense_bf16": ([_I64] * 3 + [_PTR] * 7 + [_I64] * 8 + [_PTR, _I64, _PTR], _c.c_int),
     "evo_linear_t_mfma_nf_bf16": ([_PTR] * 5 + [_I64] * 6 + [_PTR], _c.c_int),
     "evo_rms_finalize_f32": ([_PTR, _I64, _I64, _PTR, _I64, _I64, _I64, _F32, _PTR, _PTR], _c.c_int),
@@ -90,7 +91,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 14         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 15         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):

@@ -55,8 +55,9 @@ extern "C" {
  *      evo_postnorm_* launches gained the norm of the sum (`alpha`, `sum`) and the plain one an activation, as did evo_linear_small_m_bf16; evo_window_attn gained grouped key heads,
  *      kept first tokens and two maps; evo_sum_norm, evo_heads_* and evo_rglru_* added.
  *  13: evo_dense_bf16 and evo_dense_ws (any dense layer on the tiles its size asks for), evo_put_tokens and evo_advance_positions added.
- *  14: evo_linear_f32 and evo_linear_f32_ws (fp32 dense layers on the bf16 matrix cores) added. */
-#define EVO_ABI_VERSION 14
+ *  14: evo_linear_f32 and evo_linear_f32_ws (fp32 dense layers on the bf16 matrix cores) added.
+ *  15: evo_dense_plan (the launches of a dense layer) added. */
+#define EVO_ABI_VERSION 15
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
@@ -316,7 +317,11 @@ int evo_linear_t_mfma_nf_bf16(const void* x, const float* row_scale, const void*
  *   mode 1: y [M, N / 2] = gated, w = N rows in evo_mlp_gate_mfma_bf16's order, act 0 gelu, 1 silu; mode 2: the same, w = [W1; W2] as it is
  *   mode 3: z^T of evo_linear_t_mfma_nf_bf16, M = Mp; x_rows, Tm, row_skip as there with row_scale, 0 without
  * N % 256 == 0, K % 64 == 0; M % 256 == 0 for mode 3 and xblk; N K 2 < 4 GiB for mode 2.  `ws`: evo_dense_ws(mode, sumsq != NULL, M, N, K) bytes, 16-byte
- * aligned; NULL or fewer: the same product without parts of K. */
+ * aligned; NULL or fewer: the same product without parts of K.
+ * evo_dense_plan: the one or two launches (the result) that evo_dense_bf16 makes with that workspace, needs no GPU; seven values each in `out` [14], a HOST array:
+ * first row, rows, rows of a tile, columns of a tile (tokens, weight rows for mode 3), parts of K, 1 for the persistent kernel, and the row behind the last whose
+ * sum of squares it stores (at most M rounded up to 256). */
+int evo_dense_plan(int64_t mode, int64_t stats, int64_t M, int64_t N, int64_t K, int64_t* out);
 int evo_dense_ws(int64_t mode, int64_t stats, int64_t M, int64_t N, int64_t K);
 int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const void* x, const void* w, const void* bias, const void* residual, void* y,
                    const float* row_scale, float* sumsq, int64_t ss_ld, int64_t M, int64_t N, int64_t K, int64_t act_cols, int64_t x_rows,

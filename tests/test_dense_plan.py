@@ -1,0 +1,38 @@
+"""The launches of a dense layer (csrc/gemm_tile.hip tile_plan, on the host: 256 CUs where there is no GPU): rows taken once each, statistics inside their strip."""
+import ctypes
+
+import pytest
+
+from evo_amd import ops as evo_ops
+
+KEYS = ("first", "rows", "tile_rows", "tile_cols", "parts", "persistent", "stat_end")
+
+
+def launches(mode, stats, M, N, K):
+    out = (ctypes.c_int64 * 14)()
+    n = evo_ops.load_library().evo_dense_plan(mode, int(stats), M, N, K, ctypes.cast(out, ctypes.c_void_p))
+    assert n in (1, 2), n
+    return [dict(zip(KEYS, out[7 * i:7 * i + 7])) for i in range(n)]
+
+
+# (widths of the dense layers that write the residual stream, and others whose plans end in tiles that overhang the statistic's last rows)
+@pytest.mark.parametrize("N,K", [(4096, 4096), (4096, 11008), (4096, 10944), (2048, 2048), (1024, 1024), (5120, 5120), (768, 768)])
+def test_statistics_stay_in_their_strip(N, K):
+    overhang = 0
+    for M in range(65, 12000):
+        ld, end = (M + 255) // 256 * 256, 0
+        for p in launches(0, True, M, N, K):
+            assert p["first"] == end and p["rows"] > 0
+            end += p["rows"]
+            assert end <= p["stat_end"] <= ld, (M, p)             # every row's, and nothing of the next strip
+            overhang += p["first"] + -(-p["rows"] // p["tile_rows"]) * p["tile_rows"] > ld
+        assert end == M
+    assert overhang > 0 or N == 768
+
+
+def test_null_and_shapes():
+    lib = evo_ops.load_library()
+    out = (ctypes.c_int64 * 14)()
+    assert lib.evo_dense_plan(0, 0, 100, 256, 64, None) == -1
+    assert lib.evo_dense_plan(0, 0, 100, 250, 64, ctypes.cast(out, ctypes.c_void_p)) == -1
+    assert lib.evo_dense_plan(3, 0, 100, 256, 64, ctypes.cast(out, ctypes.c_void_p)) == -1

@@ -165,3 +165,45 @@ def test_same_bits_transposed(Mp, Tm):
     assert ops.lib.evo_linear_t_mfma_nf_bf16(x.data_ptr(), rs.data_ptr(), w.data_ptr(), b.data_ptr(), want.data_ptr(), Mp, N, K, rows, Tm, skip, _stream()) == 0
     ops._dense_layer(3, x, w, got, Mp, N, K, b=b, rs=rs, x_rows=rows, Tm=Tm, row_skip=skip)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("M,K", [(5249, 4096), (5300, 11008), (5376, 4096), (5376, 11008), (5631, 4096)])
+def test_statistics_of_a_tail_launch(M, K):
+    """Whole rounds of the persistent kernel, then a tail on smaller tiles whose last one overhangs the layer: the sums of squares are those of the persistent
+    kernel in every strip, and nothing is written behind the last."""
+    from evo_amd.ops import _stream
+    from test_dense_plan import launches
+    ops, N, ld = _ops(), 4096, (M + 255) // 256 * 256
+    g, x, w = _data(M, N, K, 8)
+    b, r = (torch.randn(*s, device="cuda", generator=g).bfloat16() for s in ((N,), (M, N)))
+    plan = launches(0, True, M, N, K)
+    assert M > 5376 or (len(plan) == 2 and plan[1]["first"] + -(-plan[1]["rows"] // plan[1]["tile_rows"]) * plan[1]["tile_rows"] > ld)
+    want, got = r.clone(), r.clone()
+    ss = [torch.full((N // 128 + 1, ld), -1.0, device="cuda") for _ in range(2)]      # one row more than the strips
+    assert ops.lib.evo_linear_mfma_nf_bf16(x.data_ptr(), w.data_ptr(), b.data_ptr(), want.data_ptr(), want.data_ptr(), None, ss[0].data_ptr(), ld, M, N, K, _stream()) == 0
+    ops._dense_layer(0, x, w, got, M, N, K, b=b, res=got, ss=ss[1][:-1])
+    assert torch.equal(got, want)
+    assert torch.equal(ss[0][:-1, :M], ss[1][:-1, :M]) and bool((ss[1][-1] == -1).all())
+    if M % 128 == 0:
+        blocked = r.clone()
+        ss[1].fill_(-1.0)
+        ops._dense_layer(0, x.view(M // 128, 128, K // 16, 16).permute(0, 2, 1, 3).contiguous(), w, blocked, M, N, K, xblk=1, b=b, res=blocked, ss=ss[1][:-1])
+        assert torch.equal(blocked, want)
+        assert torch.equal(ss[0][:-1, :M], ss[1][:-1, :M]) and bool((ss[1][-1] == -1).all())
+
+
+def test_a_sequence_whose_layers_end_in_a_tail_launch():
+    """One sequence of 5,300 tokens through four layers of width 4,096, norms folded and as passes of their own: two bf16 evaluations of one model."""
+    from test_gpu_model import DEV, acgt, build
+    from test_gpu_packed_prompts import WIDE
+    _, _, m = build(WIDE)
+    ids, was = acgt(1, 5299).to(DEV), m.ops.fuse_norm
+    try:
+        m.ops.fuse_norm = True
+        folded = m(ids)[0].float()
+        m.ops.fuse_norm = False
+        plain = m(ids)[0].float()
+    finally:
+        m.ops.fuse_norm = was
+    for rows in (slice(0, 64), slice(64, 4096), slice(4096, None)):
+        assert ((folded[0, rows] - plain[0, rows]).norm() / plain[0, rows].norm()).item() < 3e-2
