@@ -281,7 +281,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
         const int64_t m = m0 + wm * WM + 16 * j + l15;
         const bool ok = m < a.M;
         const float f = MODE == 0 && a.rs && ok ? a.rs[m] : 1.f;
-        const float rb = MODE == 3 && a.bias ? bf_to_f(a.bias[m]) : 0.f;
+        const float rb = MODE == 3 && a.bias && ok ? bf_to_f(a.bias[m]) : 0.f;
 #pragma unroll
         for (int b = 0; b < NT / 2; ++b) {
             const int n = n0 + wn * WN + 32 * b + 8 * lq;

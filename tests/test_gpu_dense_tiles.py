@@ -207,3 +207,18 @@ def test_a_sequence_whose_layers_end_in_a_tail_launch():
         m.ops.fuse_norm = was
     for rows in (slice(0, 64), slice(64, 4096), slice(4096, None)):
         assert ((folded[0, rows] - plain[0, rows]).norm() / plain[0, rows].norm()).item() < 3e-2
+
+
+@pytest.mark.parametrize("N,Mp", [(1024, 4352), (1280, 3328), (4096, 1280)])
+def test_transposed_last_tile_overhangs_the_weight(N, Mp):
+    """Tiles of 192 weight rows, N no multiple of 192: the last tile's rows behind the weight have no bias."""
+    from evo_amd.ops import _stream
+    from test_dense_plan import launches
+    ops, K = _ops(), 512
+    assert N % 192 and [p["tile_cols"] for p in launches(3, False, Mp, N, K)] == [192]
+    g, x, w = _data(Mp, N, K, 9)
+    b = torch.randn(N, device="cuda", generator=g).bfloat16()
+    want, got = (torch.zeros(Mp // 256, N, 256, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    assert ops.lib.evo_linear_t_mfma_bf16(x.data_ptr(), w.data_ptr(), b.data_ptr(), want.data_ptr(), Mp, N, K, _stream()) == 0
+    ops._dense_layer(3, x, w, got, Mp, N, K, b=b)
+    assert torch.equal(got, want)
