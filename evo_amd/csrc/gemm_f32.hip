@@ -1,9 +1,11 @@
 // fp32 dense layers on the bf16 matrix cores of gfx950:  y [M, N] = x [M, K] w [N, K]^T (+ bias), all fp32.
 //
-// Every fp32 value is the exact sum of three bf16 ones, x = h + m + l: h its upper 16 bits (cut, so no finite value becomes infinite), m the rest
-// rounded to bf16, l what is left (at most 8 bits, so exact).  A product is h h' + (h m' + m h') + (h l' + l h' + m m') with fp32 accumulation; what
-// is left out, m l' + l m' + l l', is under 2^-22 of a product and mostly 2^-26 with either sign, less than the accumulation rounds.  Six bf16 MFMAs in
-// place of one fp32 MFMA at 1/16 of their rate.
+// Every fp32 value is the exact sum of three bf16 ones, x = h + m + l: h the value rounded to bf16, m the rest rounded to bf16, l what is left (at most
+// 8 bits, so exact).  A product is h h' + (h m' + m h') + (h l' + l h' + m m') with fp32 accumulation; what is left out, m l' + l m' + l l', is at most
+// 2^-24 of a product, as much as an fp32 multiplication rounds, and 2^-27 in the mean square (with h cut instead of rounded 2^-22).  A lone product is
+// within 2^-22.7 (the matrix cores' adders cut; 2^-24.8 in the mean square, fp32 2^-25.2), sums of K >= 256 are nearer to 64 bits than the fp32
+// MFMA's: K = 256 2.4e-7 against 2.9e-7, 4,096 3.5e-7 to 4.1e-7 against 5.7e-7 to 1.1e-6, 11,008 6.0e-7 to 7.0e-7 against 0.9e-6 to 1.9e-6.
+// Six bf16 MFMAs in place of one fp32 MFMA at 1/16 of their rate.
 //
 // Workgroup = BM x BN of y, waves of (BM / WGM) x (BN / WGN) in 32 x 32 x 16 MFMAs, computed transposed (A = rows of w, B = rows of x) so that a lane
 // holds four neighbouring columns of one row of y.  K is walked in steps of 32: a thread loads 8 neighbouring fp32 of a row, splits them in registers
@@ -25,9 +27,8 @@ __device__ __forceinline__ void f3_split(const float4 a, const float4 b, uint4& 
     uint32_t o[3][4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        const uint32_t u0 = __float_as_uint(v[2 * e]), u1 = __float_as_uint(v[2 * e + 1]);
-        o[0][e] = __builtin_amdgcn_perm(u1, u0, 0x07060302);
-        float r0 = v[2 * e] - __uint_as_float(u0 & 0xffff0000u), r1 = v[2 * e + 1] - __uint_as_float(u1 & 0xffff0000u);
+        o[0][e] = pack_bf2(v[2 * e], v[2 * e + 1]);
+        float r0 = v[2 * e] - bf_lo(o[0][e]), r1 = v[2 * e + 1] - bf_hi(o[0][e]);
         o[1][e] = pack_bf2(r0, r1);
         r0 -= bf_lo(o[1][e]);
         r1 -= bf_hi(o[1][e]);
@@ -38,7 +39,7 @@ __device__ __forceinline__ void f3_split(const float4 a, const float4 b, uint4& 
     l = make_uint4(o[2][0], o[2][1], o[2][2], o[2][3]);
 }
 
-// Outputs taken again in plain fp32.  An infinite operand has no parts (inf - inf), and a sum that overflows may do so in another order; and where
+// Outputs taken again in plain fp32.  An infinite operand has no parts (inf - inf), one near the largest value rounds to an infinite h, and a sum that overflows may do so in another order; and where
 // an output is under 2^-90, its operands' last parts may lie under 2^-126, which the matrix cores take as zero.
 __device__ __forceinline__ bool f3_odd(float v) {
     const uint32_t e = __float_as_uint(v) & 0x7f800000u;

@@ -45,6 +45,16 @@ def test_parts_are_exact_and_large_values_stay_finite(ops):
     assert torch.equal(ops.linear(x, w), x[:, w.argmax(1)] * 0.5)
 
 
+def test_a_lone_product(ops):
+    """One product per output.  The parts left out are at most 2^-8 2^-17 of a product twice; of the six additions the last one's rounding counts, 2^-23 of
+    the result for adders that cut (the others are of sums 2^-7 as large at most)."""
+    g = torch.Generator().manual_seed(10)
+    x, v = 1 + torch.rand(2048, 256, generator=g), 1 + torch.rand(256, generator=g)
+    want = x.double() * v.double()
+    err = ((ops.linear(x.to(DEV), torch.diag(v).to(DEV)).cpu().double() - want) / want).abs().max().item()
+    assert err <= 2.0 ** -24 + 2.0 ** -23 + 5 * 2.0 ** -30, err
+
+
 @pytest.mark.parametrize("K", [256, 4096])                     # one part of K, several
 def test_infinities_and_nan(ops, K):
     x, w = rand(70, K, seed=8), rand(512, K, seed=9)
