@@ -39,16 +39,21 @@ __device__ __forceinline__ void f3_split(const float4 a, const float4 b, uint4& 
     l = make_uint4(o[2][0], o[2][1], o[2][2], o[2][3]);
 }
 
-// Outputs taken again in plain fp32.  An infinite operand has no parts (inf - inf), one near the largest value rounds to an infinite h, and a sum that overflows may do so in another order; and where
-// an output is under 2^-90, its operands' last parts may lie under 2^-126, which the matrix cores take as zero.
-__device__ __forceinline__ bool f3_odd(float v) {
-    const uint32_t e = __float_as_uint(v) & 0x7f800000u;
-    return e == 0x7f800000u || (e < (37u << 23) && v != 0.f);
+// Outputs taken again with the fp32 matrix instructions, by the wave that holds them.  An infinite operand has no parts (inf - inf), one near the largest value
+// rounds to an infinite h, and the bf16 instructions take parts and sums under 2^-126 as zero: an operand loses at most 2^-124, an output of K products at
+// most K 2^-124 (|x| + |w| + 2), |x| and |w| the largest of its rows.  What is not finite or under 2^26 of that is taken again; a row without a value other
+// than zero is right as it is.  A wave takes a few one after the other, many as a product of its whole part.  (300 x 4,096 x 4,096, 88 us: with a NaN in one
+// row 118, in all rows 224 -- 2,400 and 16,450 output by output --; the maxima and the look at the outputs cost 1 %.)
+__device__ __forceinline__ void f3_row_max(float& m, const float4 a, const float4 b) {
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(a.x), "v"(a.y));
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(a.z), "v"(a.w));
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(b.x), "v"(b.y));
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(b.z), "v"(b.w));
 }
-__device__ __noinline__ float f3_plain(const float* __restrict__ x, const float* __restrict__ w, int K) {
-    float s = 0.f;
-    for (int k = 0; k < K; ++k) s = fmaf(x[k], w[k], s);
-    return s;
+// the least and the largest magnitude so far (the largest is NaN once a value was)
+__device__ __forceinline__ void f3_range(float& lo, float& hi, float a, float b) {
+    asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(lo) : "v"(a), "v"(b));
+    asm("v_maximum3_f32 %0, %0, |%1|, |%2|" : "+v"(hi) : "v"(a), "v"(b));
 }
 
 template <int BM, int BN, int WGM, int WGN, int PER_CU, bool SPLIT>
@@ -84,6 +89,9 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_f
         dst[p] = r * F3_ROWB + ((s ^ (r >> 2)) & 3) * 16;
     }
     float4 st[NP][2];
+    float top[NP];                                             // the largest of this thread's values of each row
+#pragma unroll
+    for (int p = 0; p < NP; ++p) top[p] = 0.f;
     auto fetch = [&]() {
 #pragma unroll
         for (int p = 0; p < NP; ++p) { st[p][0] = *(const float4*)src[p]; st[p][1] = *(const float4*)(src[p] + 4); src[p] += F3_BK; }
@@ -93,6 +101,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_f
         for (int p = 0; p < NP; ++p) {
             uint4 h, m, l;
             f3_split(st[p][0], st[p][1], h, m, l);
+            f3_row_max(top[p], st[p][0], st[p][1]);
             *(uint4*)(smem + dst[p]) = h;
             *(uint4*)(smem + PLANE + dst[p]) = m;
             *(uint4*)(smem + 2 * PLANE + dst[p]) = l;
@@ -142,34 +151,145 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_f
         multiply();
         __syncthreads();
     }
-    bool odd = false;
+    float* row_max = (float*)smem;                             // (a row of zeros: -inf, which no output is under)
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        top[p] = fmaxf(top[p], dpp_fetch<EVO_DPP_XOR1>(top[p]));
+        top[p] = fmaxf(top[p], dpp_fetch<EVO_DPP_XOR2>(top[p]));
+        if ((tid & 3) == 0) row_max[(p * NT + tid) >> 2] = top[p] > 0.f ? top[p] : -INFINITY;
+    }
+    __syncthreads();
+    const float least = (float)(k1 - k0) * (F3_BK * 0x1p-98f);
+    float wide = 0.f;                                          // the largest of this lane's columns
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4 w = *(const float4*)(row_max + BM + wn * (BN / WGN) + j * 32 + q * 8 + half * 4);
+            wide = fmaxf(fmaxf(fmaxf(wide, w.x), fmaxf(w.y, w.z)), w.w);
+        }
+    auto at = [&](int64_t m, int n) { return SPLIT ? a.parts + ((int64_t)part * a.M + m) * a.N + n : a.y + m * a.N + n; };
+    bool look = false;                                         // an output may have to be taken again
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-        const int64_t m = m0 + wm * (BM / WGM) + i * 32 + l31;
+        const int r = wm * (BM / WGM) + i * 32 + l31;
+        const int64_t m = m0 + r;
         if (m >= a.M) continue;
+        float lo = INFINITY, hi = 0.f;
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
+                float4 v = make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+                f3_range(lo, hi, v.x, v.y);
+                f3_range(lo, hi, v.z, v.w);
                 const int n = n0 + wn * (BN / WGN) + j * 32 + q * 8 + half * 4;
                 if (n >= a.N) continue;
-                float4 v = make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
-                if (SPLIT) { *(float4*)(a.parts + ((int64_t)part * a.M + m) * a.N + n) = v; continue; }
-                if (a.bias) { const float4 b = *(const float4*)(a.bias + n); v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w; }
-                odd |= f3_odd(v.x) | f3_odd(v.y) | f3_odd(v.z) | f3_odd(v.w);
-                *(float4*)(a.y + m * a.N + n) = v;
+                if (!SPLIT && a.bias) { const float4 b = *(const float4*)(a.bias + n); v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w; }
+                *(float4*)at(m, n) = v;
+            }
+        look |= !(lo >= fmaf(least, wide, fmaf(least, fmaxf(row_max[r], 0.f), least)) && hi <= 3.402823466e38f);
+    }
+    if (__builtin_amdgcn_ballot_w64(look) == 0) return;
+    uint32_t odd[(TM * TN + 1) / 2] = {};                      // which ones: 16 outputs of each of two products
+    int n_odd = 0;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int r = wm * (BM / WGM) + i * 32 + l31;
+        if (m0 + r >= a.M) continue;
+        const float bound = fmaf(least, row_max[r], least);
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int c = wn * (BN / WGN) + j * 32 + q * 8 + half * 4;
+                if (n0 + c >= a.N) continue;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float u = fabsf(acc[i][j][4 * q + e]);
+                    odd[(i * TN + j) >> 1] |= (u >= fmaf(least, row_max[BM + c + e], bound) && u <= 3.402823466e38f ? 0u : 1u) << (((i * TN + j) & 1) * 16 + 4 * q + e);
+                }
             }
     }
-    if (!SPLIT && odd) {
-        for (int i = 0; i < TM; ++i)
-            for (int c = 0; c < TN * 16; ++c) {
-                const int64_t m = m0 + wm * (BM / WGM) + i * 32 + l31;
-                const int n = n0 + wn * (BN / WGN) + (c >> 4) * 32 + ((c >> 2) & 3) * 8 + half * 4 + (c & 3);
-                if (m >= a.M || n >= a.N || !f3_odd(a.y[m * a.N + n])) continue;
-                const float v = f3_plain(a.x + m * a.K, a.w + (int64_t)n * a.K, a.K);
-                a.y[m * a.N + n] = a.bias ? v + a.bias[n] : v;
+#pragma unroll
+    for (uint32_t w : odd) n_odd += __popc(w);
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) n_odd += __shfl_xor(n_odd, d, 64);
+    if (n_odd == 0) return;
+    if (n_odd <= 8 * TM * TN) {                                // a few (sums that cancel to zero): one after the other, the wave along k
+#pragma unroll
+        for (int s = 0; s < (TM * TN + 1) / 2; ++s)
+            for (uint64_t lanes = __builtin_amdgcn_ballot_w64(odd[s] != 0); lanes; lanes &= lanes - 1) {
+                const int owner = __builtin_ctzll(lanes);
+                for (uint32_t bits = (uint32_t)__builtin_amdgcn_readlane((int)odd[s], owner); bits; bits &= bits - 1) {
+                    const int t = __builtin_ctz(bits), ij = 2 * s + (t >> 4), i = ij / TN, j = ij - i * TN;
+                    const int64_t m = m0 + wm * (BM / WGM) + i * 32 + (owner & 31);
+                    const int n = n0 + wn * (BN / WGN) + j * 32 + ((t >> 2) & 3) * 8 + (owner >> 5) * 4 + (t & 3);
+                    const float *x = a.x + m * a.K, *w = a.w + (int64_t)n * a.K;
+                    float sum = 0.f;
+#pragma unroll 4
+                    for (int k = k0 * F3_BK + 4 * lane; k < k1 * F3_BK; k += 256) {
+                        const f32x4_t u = *(const f32x4_t*)(x + k), v = *(const f32x4_t*)(w + k);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) sum = fmaf(u[e], v[e], sum);
+                    }
+                    sum = wave_sum(sum);
+                    if (lane == owner) *at(m, n) = !SPLIT && a.bias ? sum + a.bias[n] : sum;
+                }
             }
+        return;
     }
+    // lane (l31, half): four neighbouring k of its rows per request, a product of two k per component, as both operands take them
+    const float *xr[TM], *wr[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int64_t m = m0 + wm * (BM / WGM) + i * 32 + l31;
+        xr[i] = a.x + (m < a.M ? m : a.M - 1) * a.K + (int64_t)k0 * F3_BK + half * 4;
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const int n = n0 + wn * (BN / WGN) + j * 32 + l31;
+        wr[j] = a.w + (int64_t)(n < a.N ? n : a.N - 1) * a.K + (int64_t)k0 * F3_BK + half * 4;
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+#pragma unroll 1
+    for (int k = k0; k < k1; ++k) {
+        f32x4_t xf[TM][4], wf[TN][4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) xf[i][t] = *(const f32x4_t*)(xr[i] + 8 * t);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) wf[j][t] = *(const f32x4_t*)(wr[j] + 8 * t);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[j][t][e], xf[i][t][e], acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) xr[i] += F3_BK;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) wr[j] += F3_BK;
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int t = 0; t < 16; ++t)
+                if (odd[(i * TN + j) >> 1] >> (((i * TN + j) & 1) * 16 + t) & 1) {     // (set only for outputs that are there)
+                    const int n = n0 + wn * (BN / WGN) + j * 32 + (t >> 2) * 8 + half * 4 + (t & 3);
+                    *at(m0 + wm * (BM / WGM) + i * 32 + l31, n) = !SPLIT && a.bias ? acc[i][j][t] + a.bias[n] : acc[i][j][t];
+                }
 }
 
 // the sum of the parts of K
@@ -183,18 +303,8 @@ __global__ __launch_bounds__(256) void gemm_f32_parts_kernel(F3Args a) {
         const float4 p = *(const float4*)(a.parts + (int64_t)s * a.M * a.N + i);
         v.x += p.x; v.y += p.y; v.z += p.z; v.w += p.w;
     }
-    const float4 b = a.bias ? *(const float4*)(a.bias + n) : make_float4(0.f, 0.f, 0.f, 0.f);
-    float o[4] = {v.x, v.y, v.z, v.w};
-    const float c[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        if (a.bias) o[e] += c[e];
-        if (f3_odd(o[e])) {
-            o[e] = f3_plain(a.x + m * a.K, a.w + (int64_t)(n + e) * a.K, a.K);
-            if (a.bias) o[e] += c[e];
-        }
-    }
-    *(float4*)(a.y + i) = make_float4(o[0], o[1], o[2], o[3]);
+    if (a.bias) { const float4 b = *(const float4*)(a.bias + n); v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w; }
+    *(float4*)(a.y + i) = v;
 }
 
 // ---------------------------------------------------------------------------------------------------------------- which tile

@@ -55,6 +55,45 @@ def test_a_lone_product(ops):
     assert err <= 2.0 ** -24 + 2.0 ** -23 + 5 * 2.0 ** -30, err
 
 
+@pytest.mark.parametrize("M,N", [(70, 256), (300, 256), (2100, 4096)])       # small tiles with parts of K, larger ones, the largest
+@pytest.mark.parametrize("a,b", [(-70, -70), (-74, -75), (-110, 40), (-120, 100), (-130, 0), (-130, 40), (-145, 60), (60, -145), (-100, -30), (0, 0)])
+def test_operands_and_results_near_the_smallest(ops, M, N, a, b):
+    """One product per output, operands of 2^a and 2^b, beside columns of ordinary size in the other rows: what an fp32 multiplication gives, 2^-24 of the result
+    and half the smallest value (or the lone product's 2^-22.4 where no part is near 2^-126)."""
+    g = torch.Generator().manual_seed(11)
+    K = 256
+    x, w = (1 + torch.rand(M, K, generator=g)).double(), torch.zeros(N, K, dtype=torch.float64)
+    at = torch.arange(N) % K
+    w[torch.arange(N), at] = (1 + torch.rand(N, generator=g)).double()
+    x[::3] *= 2.0 ** a
+    w[::2] *= 2.0 ** b
+    x[1::3, at[1]] = 0.0                                       # (an exact zero beside them)
+    x, w = x.float(), w.float()
+    want = x.double()[:, at] * w.double()[torch.arange(N), at]
+    y = ops.linear(x.to(DEV), w.to(DEV)).cpu().double()
+    assert bool(((y - want).abs() <= want.abs() * (2.0 ** -24 + 2.0 ** -23 + 5 * 2.0 ** -30) + 2.0 ** -150).all())
+
+
+def test_rows_of_zeros(ops):
+    x, w = rand(300, 512, seed=12).to(DEV), rand(516, 512, seed=13).to(DEV)
+    x[7], x[100:200], w[3], w[260:300] = 0.0, 0.0, 0.0, 0.0
+    y = ops.linear(x, w)
+    want = x.double() @ w.double().t()
+    assert torch.equal(y == 0, want == 0) and ((y.double() - want).norm() / want.norm()).item() < 1e-6
+    assert not ops.linear(torch.zeros_like(x), w).any()
+
+
+def test_a_value_that_is_not_finite_leaves_the_other_rows_alone(ops):
+    """Every tile of the plan, with and without parts: the rows without it bit for bit as without it."""
+    for M, N, K in SHAPES:
+        x, w = rand(M, K, seed=14).to(DEV), rand(N, K, seed=15).to(DEV)
+        y = ops.linear(x, w)
+        x[M // 2, K // 2] = float("nan")
+        z = ops.linear(x, w)
+        assert bool(torch.isnan(z[M // 2]).all())
+        assert torch.equal(y[: M // 2], z[: M // 2]) and torch.equal(y[M // 2 + 1:], z[M // 2 + 1:])
+
+
 @pytest.mark.parametrize("K", [256, 4096])                     # one part of K, several
 def test_infinities_and_nan(ops, K):
     x, w = rand(70, K, seed=8), rand(512, K, seed=9)
