@@ -912,7 +912,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
     def _prefill_packed(self, prompts: List[torch.Tensor]):
         """Prompts behind each other as ONE stream of rows, each from a multiple of 64 on (the rows between are token 0 and reach nobody: every
         launch is row-independent or runs on one prompt's rows): the dense layers see all rows at once, the Hyena operator and the attention walk
-        the prompts one by one.  -> (final-norm rows, first row of every prompt, caches with a row per prompt)."""
+        the prompts one by one.  -> (final-norm rows, first row of every prompt, caches of every prompt, each of its own length)."""
         ops, D, H, hd, K1 = self.ops, self.hidden_size, self.num_heads, self.head_dim, self.short_filter_length - 1
         dev, lens = self.device, [p.numel() for p in prompts]
         first, M = [], 0
@@ -930,10 +930,9 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             ids[f:f + m] = p.reshape(-1).to(dev)
         cos, sin = (t[pos] for t in self._rotary(0, max(lens), dev)) if self.attn_layer_idxs else (None, None)
         pre = bool(getattr(ops, "attn_prescale", False)) and hasattr(ops, "attn_q_scale")
-        ipd = self.initialize_inference_params()
-        ipd["mha"].max_batch_size = ipd["hyena"].max_batch_size = len(lens)
-        ipd["mha"].max_seqlen = max(lens)
-        kvs, hy = ipd["mha"].key_value_memory_dict, ipd["hyena"]
+        caches = [self.initialize_inference_params() for _ in lens]
+        for ipd, m in zip(caches, lens):
+            ipd["mha"].max_seqlen = m
         x = ops.embed(ids, self.embedding_layer.weight)
         yb = ops.yblk_empty(M, D, dev).zero_()                     # (the rows between the prompts stay zero)
         nf, rs = self._nf_ok(M, None), None
@@ -947,11 +946,10 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
                     qkv = ops.norm_linear(x, blk.pre_norm.scale, self.eps, mha.Wqkv.weight, mha.Wqkv.bias, mfma=True)
                 qkv = qkv.view(1, M, 3, H, hd)
                 ops.rope_(qkv, cos, sin, **({"q_scale": ops.attn_q_scale(hd)} if pre else {}))
-                kv = kvs[i] = torch.zeros(len(lens), max(lens), 2, H, hd, dtype=qkv.dtype, device=dev)
                 y, bias, w = torch.zeros(M, D, dtype=qkv.dtype, device=dev), mha.out_proj.bias, mha.out_proj.weight
                 for n, (f, m) in enumerate(zip(first, lens)):
                     z = qkv[:, f:f + m]
-                    kv[n, :m].copy_(z[0, :, 1:3])
+                    caches[n]["mha"].key_value_memory_dict[i] = z[:, :, 1:3].contiguous()
                     ops.attention(z[:, :, 0], z[:, :, 1], z[:, :, 2], 0, out=y[f:f + m].view(1, m, H, hd), **({"prescaled": True} if pre else {}))
             else:
                 f_, pb = blk.filter, None if blk.projections.bias is None else blk.projections.bias.data
@@ -961,17 +959,19 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
                 else:
                     zt = ops.linear_t(ops.rmsnorm(x, None, blk.pre_norm.scale, self.eps), blk.projections.weight.data, pb, 1, M)
                 table = self._mfma_table(blk)
-                state = hy.state_dict[i] = torch.empty(len(lens), D, self.state_size, dtype=torch.complex64, device=dev)
+                state = torch.empty(len(lens), D, self.state_size, dtype=torch.complex64, device=dev)
                 for n, (f, m) in enumerate(zip(first, lens)):
                     ops.hyena_ct(zt, 1, m, f_._fir_w, f_.short_filter_bias, table, H, want_state=True, poles=f_._poles, y_blk=yb, y_row0=f, at=f,
                                  s_out=state[n:n + 1])
-                hy.fir_state_dict[i] = zt[ends // 256, :, ends % 256].view(len(lens), K1, 3 * D).transpose(1, 2).contiguous()
+                fir = zt[ends // 256, :, ends % 256].view(len(lens), K1, 3 * D).transpose(1, 2).contiguous()
+                for n, ipd in enumerate(caches):
+                    ipd["hyena"].state_dict[i], ipd["hyena"].fir_state_dict[i] = state[n:n + 1], fir[n:n + 1]
                 y, bias, w = yb, blk.out_filter_dense.bias, blk.out_filter_dense.weight
             if nf:
                 rs = self._mlp_residual_rs_(blk, x, self._mixer_out_rs_(blk, x, y, w, bias))
             else:
                 self._mlp_residual_(blk, x, self._mixer_out_(blk, x, y, w, bias, mfma=True), None)
-        return (x if self.norm is None else ops.rmsnorm(x, None, self.norm.scale, self.eps)), first, ipd
+        return (x if self.norm is None else ops.rmsnorm(x, None, self.norm.scale, self.eps)), first, caches
 
     def prefill_rows(self, prompts: List[torch.Tensor], want: Optional[List[List[int]]] = None):
         """Prompts ([P] ids) of any lengths -> [(logits [wanted, V], caches, row of the caches)], several in a pass where they can share one
@@ -979,15 +979,15 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         out = []
         for group in self._prompt_groups([p.numel() for p in prompts]):
             if len(group) > 1:
-                h, first, ipd = self._prefill_packed([prompts[n] for n in group])
+                h, first, caches = self._prefill_packed([prompts[n] for n in group])
             else:
-                ipd = self.initialize_inference_params()
-                ipd["mha"].max_seqlen = prompts[group[0]].numel()
-                h, first = self.hidden_states(prompts[group[0]].reshape(1, -1), ipd), [0]
+                caches = [self.initialize_inference_params()]
+                caches[0]["mha"].max_seqlen = prompts[group[0]].numel()
+                h, first = self.hidden_states(prompts[group[0]].reshape(1, -1), caches[0]), [0]
             at = [[prompts[n].numel() - 1] if want is None else list(want[n]) for n in group]
             rows = torch.tensor([f + t for f, ts in zip(first, at) for t in ts], dtype=torch.int64, device=h.device)
             logits = self.ops.linear(h[rows].contiguous(), self.unembed.weight, None) if rows.numel() else h.new_empty(0, self.vocab_size)
-            out += [(lg, ipd, row) for row, lg in enumerate(logits.split([len(ts) for ts in at]))]
+            out += [(lg, ipd, 0) for lg, ipd in zip(logits.split([len(ts) for ts in at]), caches)]
         return out
 
     # upstream names, kept for callers that reach for them

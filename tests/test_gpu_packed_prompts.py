@@ -49,3 +49,18 @@ def test_packed_prompts_are_the_prompts_alone(dims, lens):
         b = alone.advance({s: int(t[k]) for s, t in zip(first, nxt)})
         for i, (s, f) in enumerate(zip(slots, first)):
             close(a[s], b[f], ("step", k, lens[i]))
+
+
+def test_caches_take_the_prompts_own_lengths():
+    """Short prompts beside a long one: the keys and values that a pass keeps are those of its tokens."""
+    from evo_amd.pool import DecodePool
+    _, _, m = build(dict(SMALL4))
+    lens = [33, 2000] + [40] * 30
+    assert len(m._prompt_groups(lens)) == 1
+    got = DecodePool(m, None, n_slots=2).prefill(prompts_of(lens))
+    kept = {}
+    for (_, ipd, row), n in zip(got, lens):
+        kv = ipd["mha"].key_value_memory_dict[1]
+        assert kv.shape[1] >= n and row < kv.shape[0]
+        kept[kv.untyped_storage().data_ptr()] = kv.untyped_storage().nbytes()
+    assert sum(kept.values()) == sum(lens) * 2 * m.hidden_size * 2
