@@ -973,6 +973,13 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
                 self._mlp_residual_(blk, x, self._mixer_out_(blk, x, y, w, bias, mfma=True), None)
         return (x if self.norm is None else ops.rmsnorm(x, None, self.norm.scale, self.eps)), first, caches
 
+    @staticmethod
+    def _place(t, n: int) -> int:
+        """Place `t` of a prompt of n tokens, from the end where it is negative; one that is not there is another prompt's row or none."""
+        if not -n <= t < n:
+            raise IndexError(f"place {int(t)} of a prompt of {n} tokens")
+        return int(t) % n
+
     def prefill_rows(self, prompts: List[torch.Tensor], want: Optional[List[List[int]]] = None):
         """Prompts ([P] ids) of any lengths -> [(logits [wanted, V], caches, row of the caches)], several in a pass where they can share one
         (_prompt_groups); `want`: the places whose logits are returned (the last token's by default)."""
@@ -984,7 +991,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
                 caches = [self.initialize_inference_params()]
                 caches[0]["mha"].max_seqlen = prompts[group[0]].numel()
                 h, first = self.hidden_states(prompts[group[0]].reshape(1, -1), caches[0]), [0]
-            at = [[prompts[n].numel() - 1] if want is None else list(want[n]) for n in group]
+            at = [[prompts[n].numel() - 1] if want is None else [self._place(t, prompts[n].numel()) for t in want[n]] for n in group]
             rows = torch.tensor([f + t for f, ts in zip(first, at) for t in ts], dtype=torch.int64, device=h.device)
             logits = self.ops.linear(h[rows].contiguous(), self.unembed.weight, None) if rows.numel() else h.new_empty(0, self.vocab_size)
             out += [(lg, ipd, 0) for lg, ipd in zip(logits.split([len(ts) for ts in at]), caches)]

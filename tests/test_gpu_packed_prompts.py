@@ -64,3 +64,18 @@ def test_caches_take_the_prompts_own_lengths():
         assert kv.shape[1] >= n and row < kv.shape[0]
         kept[kv.untyped_storage().data_ptr()] = kv.untyped_storage().nbytes()
     assert sum(kept.values()) == sum(lens) * 2 * m.hidden_size * 2
+
+
+def test_places_from_the_end_and_places_that_are_not_there():
+    _, _, m = build(dict(SMALL4))
+    lens = [40, 65, 33]
+    prompts = prompts_of(lens)
+    with torch.inference_mode():
+        for group in (prompts, prompts[:1]):                     # packed, alone
+            a = m.prefill_rows(group, [[-1, -len(p), 5] for p in group])
+            b = m.prefill_rows(group, [[len(p) - 1, 0, 5] for p in group])
+            for x, y in zip(a, b):
+                assert torch.equal(x[0], y[0])
+            for bad in (len(group[0]), -len(group[0]) - 1):
+                with pytest.raises(IndexError):
+                    m.prefill_rows(group, [[bad]] + [[0]] * (len(group) - 1))
