@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+import operator
 import os
 import threading
 from typing import Optional, Tuple
@@ -448,9 +449,14 @@ class HipOps(MixerOps):
     MAX_PUT = 64                 # tokens of one put_tokens launch (csrc/elementwise.hip EVO_PUT_MAX)
 
     def put_tokens(self, ids: torch.Tensor, slots, tokens) -> None:
-        """ids[slot] = token for up to MAX_PUT pairs of host integers: kernel arguments, no copy from host memory and no wait."""
+        """ids[slot] = token for up to MAX_PUT pairs of host integers: kernel arguments, no copy from host memory and no wait.  Tokens of other kinds are what
+        torch.tensor(tokens, dtype=torch.int64) makes of them."""
         self._need(ids, torch.int64, "put_tokens ids")
-        n = len(slots)
+        n, slots = len(slots), [operator.index(s) for s in slots]
+        if not all(0 <= s < ids.numel() for s in slots):
+            raise RuntimeError(f"put_tokens: slots {slots} of {ids.numel()}")
+        if not all(type(t) is int and -(1 << 63) <= t < 1 << 63 for t in tokens):
+            tokens = torch.tensor(tokens, dtype=torch.int64).tolist()
         arr = _c.c_int64 * n
         _check(self.lib.evo_put_tokens(ids.data_ptr(), ids.numel(), _c.cast(arr(*slots), _PTR), _c.cast(arr(*tokens), _PTR), n, _stream()), "evo_put_tokens")
 

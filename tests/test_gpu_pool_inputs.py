@@ -28,6 +28,22 @@ def test_put_tokens_refuses_slots_outside():
     assert not ids.any()
 
 
+def test_tokens_of_other_kinds():
+    """What an int64 tensor takes: floats, numpy and tensor scalars, truth values; and what it refuses."""
+    import numpy as np
+    from evo_amd.ops import default_ops
+    ops = default_ops()
+    for tokens in ([3.0, 65], [np.int64(7), np.int32(-1)], [torch.tensor(9), torch.tensor(84, device="cuda")], [True, 67], [(1 << 63) - 1, -(1 << 63)]):
+        ids = torch.zeros(5, 1, dtype=torch.int64, device="cuda")
+        ops.put_tokens(ids, [4, np.int64(1)], tokens)
+        assert ids[[4, 1], 0].tolist() == torch.tensor(tokens, dtype=torch.int64).tolist() and ids.count_nonzero().item() == 2
+    ids = torch.zeros(5, 1, dtype=torch.int64, device="cuda")
+    for slots, tokens in (([0], [1 << 63]), ([0], ["A"]), ([1.0], [5]), ([1 << 64], [5])):
+        with pytest.raises((RuntimeError, TypeError, ValueError, OverflowError)):
+            ops.put_tokens(ids, slots, tokens)
+    assert not ids.any()
+
+
 @pytest.mark.parametrize("n", [1, 256, 257])
 def test_advance_positions(n):
     from evo_amd.ops import default_ops
