@@ -399,7 +399,7 @@ __global__ __launch_bounds__(512, 2) void window_tile_kernel(WinArgs a, int B) {
     float mx[2], den[2];                                         // den: this lane's share (its keys); the sink sits in lane group 0's
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-        mx[c] = a.sink ? fmaxf(a.sink[h] * LOG2E, FLOOR) : FLOOR;
+        mx[c] = a.sink && !(a.sink[h] * LOG2E <= FLOOR) ? a.sink[h] * LOG2E : FLOOR;     // (a NaN stays one)
         den[c] = a.sink && g == 0 ? 1.0f : 0.0f;
 #pragma unroll
         for (int db = 0; db < DVB; ++db) o[c][db] = f32x4_t{0.f, 0.f, 0.f, 0.f};

@@ -55,3 +55,17 @@ def test_negative_scale_and_short_prompts_take_the_other_kernels():
     assert ((fast.float() - slow.float()).norm() / slow.float().norm()).item() < 8e-3
     fast, slow = both(z[:100], kv[:100], None, None, 2, 2, 1, 128, 0, 128, 1 << 29, 0, 0.1, [100], [0])
     assert ((fast.float() - slow.float()).norm() / slow.float().norm()).item() < 8e-3
+
+
+@pytest.mark.parametrize("dr,keep", [(64, 0), (0, 0), (0, 5)])
+def test_a_sink_that_is_not_finite(dr, keep):
+    """NaN: that head's outputs are; -inf: no sink; +inf: all weight is the sink's."""
+    H, dn, dv, n = 4, 128, 128, 200
+    g = torch.Generator(device=DEV).manual_seed(dr + keep)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g).bfloat16()      # noqa: E731
+    z, kv, kr = rnd(n, H * (dn + dr)), rnd(n, H * (dn + dv)), (rnd(n, dr) if dr else None)
+    run = lambda s: both(z, kv, kr, s, H, H, 1, dn, dr, dv, 150, keep, 0.08, [n], [0])[0].view(n, H, dv)      # noqa: E731
+    plain = run(None)
+    got = run(torch.tensor([float("nan"), -math.inf, math.inf, -math.inf], device=DEV))
+    assert bool(torch.isnan(got[:, 0]).all()) and not got[:, 2].any()
+    assert torch.equal(got[:, 1], plain[:, 1]) and torch.equal(got[:, 3], plain[:, 3])
