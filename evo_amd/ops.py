@@ -16,6 +16,7 @@ import threading
 from typing import Optional, Tuple
 
 import torch
+from torch.utils._device import DeviceContext
 
 from . import _build
 from .mixer_ops import MixerOps
@@ -323,6 +324,15 @@ class HipOps(MixerOps):
                 return torch.addmm(b, x, w.t())
             return torch.mm(x, w.t())
 
+    @staticmethod
+    def _watched() -> bool:
+        """Whether torch would do more than compute: a dispatch or function mode (traces, counters; not that of a default device), jit tracing, a compiler's
+        frame, autocast."""
+        return (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 or torch._C._get_tracing_state() is not None
+                or torch.is_autocast_enabled("cuda")
+                or (torch._C._len_torch_function_stack() > 0
+                    and any(type(m) is not DeviceContext for m in torch.overrides._get_current_function_mode_stack())))
+
     def _f32_layer_ok(self, x, w, b) -> bool:
         """fp32 layers from 33 rows on take csrc/gemm_f32.hip; below, the weight's own bytes bound the layer and the library reads them at 2.5 to 4.6 TB/s
         (24 rows: 26 us against 36 at 4,096 x 4,096, 79 against 91 at 22,016 x 4,096; 33 rows: 31 against 28, 117 against 93).  What is traced or
@@ -333,7 +343,7 @@ class HipOps(MixerOps):
                 and x.dim() == 2 and w.dim() == 2 and x.shape[0] > 32 and x.shape[1] == w.shape[1] and x.shape[1] % 32 == 0 and x.shape[1] >= 256
                 and w.shape[0] % 4 == 0 and w.shape[0] >= 256 and (b is None or b.shape == (w.shape[0],))
                 and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
-                and torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None)
+                and torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None and not self._watched())
 
     def _linear_f32(self, x, w, b):
         M, K = x.shape

@@ -128,6 +128,37 @@ def test_what_keeps_torch(ops):
         assert not ops._f32_layer_ok(x, w, None)
 
 
+@pytest.mark.filterwarnings("ignore")
+def test_traces_counters_and_autocast_see_the_product(ops):
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.overrides import TorchFunctionMode
+    from torch.utils.flop_counter import FlopCounterMode
+    x, w = rand(40, 256, seed=1).to(DEV), rand(256, 256, seed=2).to(DEV)
+    assert ops._f32_layer_ok(x, w, None)
+    graph = make_fx(lambda a: ops.linear(a, w))(x)
+    assert any("mm" in str(n.target) for n in graph.graph.nodes)
+    assert torch.allclose(graph(2 * x), 2 * (x @ w.t()), rtol=1e-4, atol=1e-4)
+    traced = torch.jit.trace(lambda a: ops.linear(a, w), x)
+    assert torch.allclose(traced(2 * x), 2 * (x @ w.t()), rtol=1e-4, atol=1e-4)
+    counter = FlopCounterMode(display=False)
+    with counter:
+        ops.linear(x, w)
+    assert counter.get_total_flops() == 2 * 40 * 256 * 256
+    with torch.autocast("cuda", torch.bfloat16):
+        assert ops.linear(x, w).dtype == torch.bfloat16
+    seen = []
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+    with Mode():
+        ops.linear(x, w)
+    assert torch.mm in seen
+    with torch.device(DEV):                                      # a default device watches nothing
+        assert ops._f32_layer_ok(x, w, None)
+
+
 def test_under_capture(ops):
     x, w = rand(300, 1024, seed=1).to(DEV), rand(512, 1024, seed=2).to(DEV)
     want = ops.linear(x, w).clone()
