@@ -8,7 +8,8 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# rows on both sides of every tile's edge; columns and depths that lead to each tile, to parts of K, and to two launches one behind the other (6,400 rows)
+# rows on both sides of every tile's edge; columns and depths that lead to each tile, to parts of K, and to the persistent kernel
+# (two launches one behind the other: test_two_launches)
 SHAPES = [(65, 256, 64), (65, 4096, 4096), (127, 512, 1024), (129, 4096, 4096), (161, 12288, 512), (161, 4096, 11008), (255, 4096, 4096),
           (385, 4096, 4096), (513, 4096, 11008), (769, 4096, 4096), (770, 4096, 11008), (1023, 4096, 11008), (1024, 4096, 11008), (1537, 4096, 2048), (2048, 4096, 1088), (2049, 4096, 4096),
           (6400, 4096, 1024)]
@@ -152,6 +153,24 @@ def test_same_bits_on_every_tile(M):
             assert ops.lib.evo_mlp_gate_mfma_nf_bf16(p(x), p(rs), p(w), p(want), M, 2048, K, _stream()) == 0
         ops._dense_layer(1, x, w, got, M, 4096, K, rs=factor)
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("M,tail", [(4700, (128, 128)), (5300, (192, 128)), (5700, (256, 128)), (8200, (64, 64)), (8500, (128, 64))])
+def test_two_launches(M, tail):
+    """Whole rounds of the persistent kernel, then the rest on each smaller tile: every form of the layer as above, the activation, the gate."""
+    from evo_amd.ops import _stream
+    from test_dense_plan import launches
+    plan = launches(0, False, M, 4096, 1024)
+    assert len(plan) == 2 and plan[0]["persistent"] and (plan[1]["tile_rows"], plan[1]["tile_cols"]) == tail
+    assert M > 8000 or len(launches(0, True, M, 4096, 1024)) == 2
+    assert M == 5700 or len(launches(1, False, M, 4096, 1024)) == 2
+    test_same_bits_on_every_tile(M)
+    ops = _ops()
+    g, x, w = _data(M, 4096, 1024, 10)
+    want, got = (torch.empty(M, 4096, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    assert ops.lib.evo_linear_act_mfma_bf16(x.data_ptr(), w.data_ptr(), None, want.data_ptr(), M, 4096, 1024, 2048, 1, _stream()) == 0
+    ops._dense_layer(0, x, w, got, M, 4096, 1024, act=1, act_cols=2048)
+    assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("Mp,Tm", [(1024, 1024), (1536, 512), (2304, 768)])
