@@ -373,6 +373,15 @@ extern "C" int evo_linear_f32_ws(int64_t M, int64_t N, int64_t K) {
     return p.splits > 1 ? p.splits : 0;
 }
 
+extern "C" int evo_linear_f32_plan(int64_t M, int64_t N, int64_t K, int64_t* out) {
+    if (!f3_ok(M, N, K) || !out) return -1;
+    const F3Plan p = f3_plan(M, N, K);
+    out[0] = f3_kinds[p.kind].bm;
+    out[1] = f3_kinds[p.kind].bn;
+    out[2] = p.splits;
+    return 0;
+}
+
 extern "C" int evo_linear_f32(const float* x, const float* w, const float* bias, float* y, int64_t M, int64_t N, int64_t K, float* ws, int64_t ws_bytes, void* stream) {
     if (!f3_ok(M, N, K)) return -1;
     if (M == 0) return 0;

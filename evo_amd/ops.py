@@ -64,6 +64,7 @@ _SIGNATURES = {
     "evo_gelu_gate_bf16": ([_PTR, _PTR, _I64, _I64, _PTR], _c.c_int),
     "evo_logprob_entropy": ([_PTR, _I64, _PTR, _PTR, _PTR, _I64, _I64, _PTR], _c.c_int),
     "evo_linear_f32_ws": ([_I64] * 3, _c.c_int),
+    "evo_linear_f32_plan": ([_I64] * 3 + [_PTR], _c.c_int),
     "evo_linear_f32": ([_PTR] * 4 + [_I64] * 3 + [_PTR, _I64, _PTR], _c.c_int),
     "evo_unembed_logprob_bf16": ([_PTR] * 5 + [_I64] * 3 + [_PTR], _c.c_int),
     "evo_rope_append_decode_bf16": ([_PTR] * 4 + [_F32] + [_I64] * 7 + [_F32, _PTR], _c.c_int),

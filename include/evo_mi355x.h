@@ -56,7 +56,7 @@ extern "C" {
  *      kept first tokens and two maps; evo_sum_norm, evo_heads_* and evo_rglru_* added.
  *  13: evo_dense_bf16 and evo_dense_ws (any dense layer on the tiles its size asks for), evo_put_tokens and evo_advance_positions added.
  *  14: evo_linear_f32 and evo_linear_f32_ws (fp32 dense layers on the bf16 matrix cores) added.
- *  15: evo_dense_plan (the launches of a dense layer) added. */
+ *  15: evo_dense_plan and evo_linear_f32_plan (the launches of a dense layer) added. */
 #define EVO_ABI_VERSION 15
 int evo_abi_version(void);
 
@@ -392,8 +392,10 @@ int evo_logprob_entropy(const void* logits, int64_t logits_f32, const int64_t* t
 /* ---- fp32 dense layer: y [M, N] = x [M, K] w [N, K]^T (+ bias [N]), all fp32, on the bf16 matrix cores: every operand as the exact sum of three
  * bf16 values, six products, fp32 accumulation (csrc/gemm_f32.hip).  K % 32 == 0, N % 4 == 0, 16-byte aligned dense operands; infinities and NaN come
  * out as in a plain fp32 sum.  evo_linear_f32_ws: how many times M N fp32 the workspace holds with which it splits K (0: none; -1: sizes
- * it does not take); without it, or with a smaller one, it does not. */
+ * it does not take); without it, or with a smaller one, it does not.  evo_linear_f32_plan: rows and columns of a tile and the parts of K with that workspace,
+ * in `out` [3], a HOST array; needs no GPU. */
 int evo_linear_f32_ws(int64_t M, int64_t N, int64_t K);
+int evo_linear_f32_plan(int64_t M, int64_t N, int64_t K, int64_t* out);
 int evo_linear_f32(const float* x, const float* w, const float* bias, float* y, int64_t M, int64_t N, int64_t K, float* ws, int64_t ws_bytes, void* stream);
 
 /* ---- fused scoring tail: unembed + log_softmax + gather (+ entropy) ---------------------------------

@@ -1,4 +1,6 @@
 """fp32 dense layers on the bf16 matrix cores (csrc/gemm_f32.hip): operands as three bf16 parts each."""
+import ctypes
+
 import pytest
 import torch
 
@@ -16,7 +18,7 @@ def rand(*shape, seed=0):
     return torch.randn(*shape, generator=torch.Generator().manual_seed(seed))
 
 
-# a lone row tile and column tile, remainders of both, one k-step more than the parts of K divide, each tile of the plan, with and without parts
+# a lone row tile and column tile, remainders of both, one k-step more than the parts of K divide (each tile and number of parts: PLANS below)
 SHAPES = [(33, 256, 256), (63, 260, 288), (65, 512, 4096), (129, 1028, 1056), (300, 4096, 1024), (513, 260, 256), (1290, 2048, 512), (2049, 2052, 256), (4000, 4096, 256)]
 
 
@@ -45,6 +47,27 @@ def test_parts_are_exact_and_large_values_stay_finite(ops):
     assert torch.equal(ops.linear(x, w), x[:, w.argmax(1)] * 0.5)
 
 
+# tile, parts of K: a size that takes them, remainders of rows and columns where that is one
+PLANS = [((64, 64), 2, (657, 2044, 1024)), ((64, 64), 3, (257, 2048, 1056)), ((64, 128), 1, (642, 8196, 256)), ((64, 128), 4, (642, 2044, 1024)), ((64, 128), 8, (131, 4092, 4096)),
+         ((128, 128), 1, (390, 8188, 256)), ((128, 128), 2, (775, 2044, 1024)), ((128, 128), 3, (517, 2044, 1024)), ((128, 128), 8, (69, 4092, 4096)),
+         ((256, 256), 1, (1539, 8188, 256)), ((256, 256), 2, (1671, 4092, 4096)), ((256, 256), 8, (391, 4092, 4096))]
+
+
+@pytest.mark.parametrize("tile,parts,shape", PLANS)
+def test_every_tile_and_number_of_parts(ops, tile, parts, shape):
+    """The bound above; a row that is not finite leaves the others bit for bit as they were."""
+    M, N, K = shape
+    out = (ctypes.c_int64 * 3)()
+    assert ops.lib.evo_linear_f32_plan(M, N, K, ctypes.cast(out, ctypes.c_void_p)) == 0 and list(out) == [*tile, parts]
+    test_no_further_from_64_bits_than_fp32(ops, M, N, K, True)
+    x, w = rand(M, K, seed=14).to(DEV), rand(N, K, seed=15).to(DEV)
+    y = ops.linear(x, w)
+    x[M // 2, K // 2] = float("nan")
+    z = ops.linear(x, w)
+    assert bool(torch.isnan(z[M // 2]).all())
+    assert torch.equal(y[: M // 2], z[: M // 2]) and torch.equal(y[M // 2 + 1:], z[M // 2 + 1:])
+
+
 def test_a_lone_product(ops):
     """One product per output.  The parts left out are at most 2^-8 2^-17 of a product twice; of the six additions the last one's rounding counts, 2^-23 of
     the result for adders that cut (the others are of sums 2^-7 as large at most)."""
@@ -55,7 +78,7 @@ def test_a_lone_product(ops):
     assert err <= 2.0 ** -24 + 2.0 ** -23 + 5 * 2.0 ** -30, err
 
 
-@pytest.mark.parametrize("M,N", [(70, 256), (300, 256), (2100, 4096)])       # small tiles with parts of K, larger ones, the largest
+@pytest.mark.parametrize("M,N", [(70, 256), (390, 8192), (1540, 8192)])      # 64 x 64, 128 x 128, 256 x 256 tiles
 @pytest.mark.parametrize("a,b", [(-70, -70), (-74, -75), (-110, 40), (-120, 100), (-130, 0), (-130, 40), (-145, 60), (60, -145), (-100, -30), (0, 0)])
 def test_operands_and_results_near_the_smallest(ops, M, N, a, b):
     """One product per output, operands of 2^a and 2^b, beside columns of ordinary size in the other rows: what an fp32 multiplication gives, 2^-24 of the result
@@ -81,17 +104,6 @@ def test_rows_of_zeros(ops):
     want = x.double() @ w.double().t()
     assert torch.equal(y == 0, want == 0) and ((y.double() - want).norm() / want.norm()).item() < 1e-6
     assert not ops.linear(torch.zeros_like(x), w).any()
-
-
-def test_a_value_that_is_not_finite_leaves_the_other_rows_alone(ops):
-    """Every tile of the plan, with and without parts: the rows without it bit for bit as without it."""
-    for M, N, K in SHAPES:
-        x, w = rand(M, K, seed=14).to(DEV), rand(N, K, seed=15).to(DEV)
-        y = ops.linear(x, w)
-        x[M // 2, K // 2] = float("nan")
-        z = ops.linear(x, w)
-        assert bool(torch.isnan(z[M // 2]).all())
-        assert torch.equal(y[: M // 2], z[: M // 2]) and torch.equal(y[M // 2 + 1:], z[M // 2 + 1:])
 
 
 @pytest.mark.parametrize("K", [256, 4096])                     # one part of K, several
