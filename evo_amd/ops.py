@@ -172,15 +172,15 @@ def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
-def pick_segment_length(B: int, T: int, H: int) -> int:
+def pick_segment_length(B: int, T: int, H: int, target_waves: int = 4096) -> int:
     """Time-segment length C of the Hyena kernels, a power of two in [4, 1024].  A wave walks its segment one position after the other
     (about 0.5 us per position over the two passes), and every segment writes and reads a 64-byte state per channel, so the time is a C + b B T / C:
     least where C^2 is about 2.2 positions at 32 heads.  (Three launches, 4,096 channels, MI355X: 161 positions 46.7 us with C = 64, 24.5 with 16;
-    500 49 with 64, 36 with 32; 2,000 57 with 64.)  From 1,024 positions on the largest C that leaves 4,096 (batch, head, segment) waves, 64 at
+    500 49 with 64, 36 with 32; 2,000 57 with 64.)  From 1,024 positions on the largest C that leaves `target_waves` (batch, head, segment) waves, 64 at
     least: a row's bits are the same in any such batch that this gives the same C (8,000 positions 150 us with it, 134 with 128)."""
     if B * T * H >= 32 * 1024:
         c = 1024
-        while c > 64 and B * H * ((T + c - 1) // c) < 4096:
+        while c > 64 and B * H * ((T + c - 1) // c) < target_waves:
             c //= 2
         return c
     c = 4

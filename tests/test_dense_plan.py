@@ -36,3 +36,14 @@ def test_null_and_shapes():
     assert lib.evo_dense_plan(0, 0, 100, 256, 64, None) == -1
     assert lib.evo_dense_plan(0, 0, 100, 250, 64, ctypes.cast(out, ctypes.c_void_p)) == -1
     assert lib.evo_dense_plan(3, 0, 100, 256, 64, ctypes.cast(out, ctypes.c_void_p)) == -1
+
+
+def test_segments_for_a_number_of_waves():
+    """From 1,024 positions (32 heads) on: the largest segment that leaves the waves asked for, 4,096 of them by default."""
+    for B, T, H in ((1, 1024, 32), (8, 8193, 32), (1, 131072, 32), (3, 5000, 16)):
+        for waves in (256, 4096, 65536):
+            c = evo_ops.pick_segment_length(B, T, H, target_waves=waves)
+            assert c in (64, 128, 256, 512, 1024)
+            assert c == 64 or B * H * -(-T // c) >= waves
+            assert c == 1024 or B * H * -(-T // (2 * c)) < waves
+        assert evo_ops.pick_segment_length(B, T, H) == evo_ops.pick_segment_length(B, T, H, 4096)
