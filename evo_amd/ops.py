@@ -337,11 +337,11 @@ class HipOps(MixerOps):
     def _f32_layer_ok(self, x, w, b) -> bool:
         """fp32 layers from 33 rows on take csrc/gemm_f32.hip; below, the weight's own bytes bound the layer and the library reads them at 2.5 to 4.6 TB/s
         (24 rows: 26 us against 36 at 4,096 x 4,096, 79 against 91 at 22,016 x 4,096; 33 rows: 31 against 28, 117 against 93).  What is traced or
-        differentiated stays with torch."""
+        differentiated stays with torch, and so does what lies on another device than the current one, whose stream the launch goes to."""
         ts = (x, w) if b is None else (x, w, b)
         return (self.all_gemm_mfma and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()
                                            and t.device == x.device and t.data_ptr() % 16 == 0 for t in ts)
-                and x.dim() == 2 and w.dim() == 2 and x.shape[0] > 32 and x.shape[1] == w.shape[1] and x.shape[1] % 32 == 0 and x.shape[1] >= 256
+                and x.device.index == torch.cuda.current_device() and x.dim() == 2 and w.dim() == 2 and x.shape[0] > 32 and x.shape[1] == w.shape[1] and x.shape[1] % 32 == 0 and x.shape[1] >= 256
                 and w.shape[0] % 4 == 0 and w.shape[0] >= 256 and (b is None or b.shape == (w.shape[0],))
                 and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
                 and torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None and not self._watched())

@@ -140,6 +140,13 @@ def test_what_keeps_torch(ops):
         assert not ops._f32_layer_ok(x, w, None)
 
 
+def test_tensors_of_another_device_keep_torch(ops, monkeypatch):
+    x, w = rand(40, 256, seed=1).to(DEV), rand(256, 256, seed=2).to(DEV)
+    assert ops._f32_layer_ok(x, w, None)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    assert not ops._f32_layer_ok(x, w, None)
+
+
 @pytest.mark.filterwarnings("ignore")
 def test_traces_counters_and_autocast_see_the_product(ops):
     from torch.fx.experimental.proxy_tensor import make_fx
