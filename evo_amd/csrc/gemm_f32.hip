@@ -4,7 +4,8 @@
 // 8 bits, so exact).  A product is h h' + (h m' + m h') + (h l' + l h' + m m') with fp32 accumulation; what is left out, m l' + l m' + l l', is at most
 // 2^-24 of a product, as much as an fp32 multiplication rounds, and 2^-27 in the mean square (with h cut instead of rounded 2^-22).  A lone product is
 // within 2^-22.7 (the matrix cores' adders cut; 2^-24.8 in the mean square, fp32 2^-25.2), sums of K >= 256 are nearer to 64 bits than the fp32
-// MFMA's: K = 256 2.4e-7 against 2.9e-7, 4,096 3.5e-7 to 4.1e-7 against 5.7e-7 to 1.1e-6, 11,008 6.0e-7 to 7.0e-7 against 0.9e-6 to 1.9e-6.
+// MFMA's (1,024 columns, 40 to 1,290 rows: K = 256 2.4e-7 against 2.9e-7, 4,096 3.5e-7 to 4.1e-7 against 5.7e-7 to 1.1e-6, 11,008 6.0e-7 to 7.0e-7
+// against 0.9e-6 to 1.9e-6; unsplit 4,096 1.00e-6 against 1.15e-6).
 // Six bf16 MFMAs in place of one fp32 MFMA at 1/16 of their rate.
 //
 // Workgroup = BM x BN of y, waves of (BM / WGM) x (BN / WGN) in 32 x 32 x 16 MFMAs, computed transposed (A = rows of w, B = rows of x) so that a lane
@@ -313,7 +314,7 @@ __global__ __launch_bounds__(256) void gemm_f32_parts_kernel(F3Args a) {
 // large bf16 product reaches).  Against the library's fp32 MFMA layers (us, K = 4,096, MI355X,
 // before -> here): 4,096 columns 40 -> 38 at 65 rows, 85 -> 80 at 300, 348 -> 254 at 1,290, 931 -> 623 at 4,000; 22,016 columns 180 -> 141, 442 -> 342,
 // 1,816 -> 1,257, 5,454 -> 3,500; K = 11,008, 4,096 columns 93 -> 86, 230 -> 181, 932 -> 668, 2,421 -> 1,692.  Error against 64 bits (random normal operands,
-// K = 4,096): 1.02e-6 unsplit, less with every split, library 1.15e-6 (its own splits 5.8e-7 at 33 to 200 rows, where this choice splits by 8: 3.6e-7).
+// 4,096 x 4,096): 1.00e-6 unsplit, 7.1e-7 in two parts, 5.0e-7 in four, 3.5e-7 in eight; library 1.14e-6.
 struct F3Kind { int bm, bn, per_cu; double start, each; };
 static const F3Kind f3_kinds[] = {{64, 64, 5, 0.29, 0.33}, {64, 128, 4, 0.30, 0.655}, {128, 128, 2, 0.20, 1.11}, {256, 256, 1, 0.10, 4.36}};
 struct F3Plan { int kind, splits; };
