@@ -389,12 +389,13 @@ __global__ __launch_bounds__(256) void lightning_recur_kernel(LightArgs a, const
 // LT rows of o meet in LDS at the end of the block, summed in the order of the slices.  R: the state rows of a thread, in registers (dk <= 32 R); 0: in LDS.
 // Bound by issue and latency: 70 instructions a token and wave in sequence.  (3 prompts of up to 500 tokens, 32 heads of 128 x 128, fp32, MI355X: 288 us;
 // one token between barriers, its rows requested when they were needed and the state in LDS, 685 us.)
+// The state in LDS is read and written in 16-byte requests (200 tokens, 4 heads of 512 x 64, fp32: 367 us; element by element 573, the form before 471).
 template <typename T, int CW, int R, int LT>
 __global__ __launch_bounds__(256) void lightning_tokens_kernel(LightArgs a, const float* __restrict__ decay) {
     extern __shared__ float sm[];
     const int dk = a.dk, dv = a.dv, h = blockIdx.y, b = blockIdx.z;
     float2* kq = (float2*)sm;                                    // [LT][dk] (k, q), [LT][32], [LT][32 slices][33], with R == 0 the state [dk][8 CW]
-    float* vs = sm + 2 * LT * dk;
+    float* vs = sm + (CW == 4 ? (2 * LT * dk + 3) & ~3 : 2 * LT * dk);         // (rows of the state below are 16-byte requests then)
     float* part = vs + LT * 32;
     float* tile = part + LT * 32 * 33;
     const int tid = threadIdx.x, cl = tid & 7, sl = tid >> 3;
@@ -474,11 +475,16 @@ __global__ __launch_bounds__(256) void lightning_tokens_kernel(LightArgs a, cons
                 for (int k = sl; k < dk; k += 32) {
                     float* p = tile + k * 8 * CW + cl * CW;
                     const float2 x = kq[t * dk + k];
+                    float s[CW];
+                    if constexpr (CW == 4) { const float4 y = *(const float4*)p; s[0] = y.x; s[1] = y.y; s[2] = y.z; s[3] = y.w; }
+                    else s[0] = *p;
 #pragma unroll
                     for (int e = 0; e < CW; ++e) {
-                        p[e] = fmaf(A, p[e], x.x * v[e]);
-                        o[e] = fmaf(x.y, p[e], o[e]);
+                        s[e] = fmaf(A, s[e], x.x * v[e]);
+                        o[e] = fmaf(x.y, s[e], o[e]);
                     }
+                    if constexpr (CW == 4) *(float4*)p = make_float4(s[0], s[1], s[2], s[3]);
+                    else *p = s[0];
                 }
             }
 #pragma unroll
@@ -525,7 +531,7 @@ static int recur_launch(LightArgs a, const float* decay, int64_t B, hipStream_t 
 
 template <typename T, int CW, int R, int LT>
 static int tokens_launch(LightArgs a, const float* decay, int64_t B, hipStream_t s) {
-    const size_t lds = ((size_t)LT * (2 * a.dk + 32 + 32 * 33) + (R ? 0 : a.dk * 8 * CW)) * 4;
+    const size_t lds = ((size_t)LT * (2 * a.dk + 32 + 32 * 33) + (CW == 4 ? (4 - 2 * LT * a.dk % 4) % 4 : 0) + (R ? 0 : a.dk * 8 * CW)) * 4;
     if (lds > 160 * 1024) return -1;
     if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)lightning_tokens_kernel<T, CW, R, LT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     hipLaunchKernelGGL((lightning_tokens_kernel<T, CW, R, LT>), dim3((unsigned)((a.dv + 8 * CW - 1) / (8 * CW)), (unsigned)a.H, (unsigned)B), dim3(256),
