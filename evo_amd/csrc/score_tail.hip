@@ -2,8 +2,9 @@
 // i.e. unembed + log_softmax + gather(next token) (+ entropy) in ONE kernel: the [M, 512] logits never reach HBM
 // (67 MB per 8 x 8,193 batch, 1.07 GB at 8 x 131,073).   [REF evo/scoring.py:47-57,81-84,119-121]
 //
-// The two-launch form (dense layer, evo_logprob_entropy) is 2 to 10 times as fast wherever the dense layer takes the width (K % 64 == 0): this kernel
-// reads all of E per 64 rows, 1 us per 36 KiB step whatever M (101 us at 161 rows against 13, 463 at 65,544 against 227).  It takes the other widths.
+// The two-launch form (dense layer, evo_logprob_entropy) is 2 to 10 times as fast where the dense layer takes the width (K % 64 == 0): this kernel
+// reads all of E per 64 rows, 1 us per 36 KiB step whatever M (K = 4,096: 101 us at 161 rows against 13, 463 at 65,544 against 227).  It takes the other
+// widths, and from 4,096 rows on (98,304 at K = 512) K < 768, where the logits' way through memory is longer than the product (131,073 rows of 256: 74 against 113).
 //
 // Numerics are those of the two-kernel path (unembed -> bf16 logits -> evo_logprob_entropy):
 // fp32 MFMA accumulation, ONE rounding of every logit to bf16 (the reference's logits are a bf16 tensor), then

@@ -1167,8 +1167,15 @@ class HipOps(MixerOps):
                "evo_logprob_entropy")
         return lp, en
 
-
     TAIL_ROWS = 32 * 1024
+
+    @staticmethod
+    def _tail_in_two(M: int, K: int) -> bool:
+        """Whether the scoring tail is a dense layer and a kernel over its logits.  The one-launch form has no logits to write and read, about as long as 512 to
+        768 k of the product at many rows (us on the GPU, one launch -> two: K = 128 9 -> 6 at 1,024 rows, 9 -> 11 at 5,000, 52 -> 107 at 131,073; 256 11 -> 7,
+        11 -> 11, 74 -> 113; 512 16 -> 7, 16 -> 13, 60 -> 55 at 65,000, 120 -> 136 at 131,073; 768 20 -> 8, 21 -> 14, 172 -> 161)."""
+        return K % 64 == 0 and 128 <= K <= 32768 and 0 < M < (4096 if K < 512 else 98304 if K < 768 else 1 << 62)
+
     def unembed_logprob_ok(self, h: torch.Tensor, emb: torch.Tensor) -> bool:
         return (h.is_cuda and h.dtype == torch.bfloat16 and emb.dtype == torch.bfloat16 and h.is_contiguous()
                 and emb.is_contiguous() and emb.shape[0] == 512 and h.shape[1] % 32 == 0
@@ -1178,8 +1185,8 @@ class HipOps(MixerOps):
                         want_logprob=True, want_entropy=False):
         """Fused scoring tail: h [M,K] bf16 (final-norm output) x emb[512,K]^T -> (logprob [M] f32 | None,
         entropy [M] f32 | None).  A dense layer and one kernel over its logits, fewer than 64 K rows of them at a time; the one-launch
-        form, whose workgroup holds all 512 logits of its 64 rows, takes the widths that the dense layer does not (us, one launch -> two, K = 4,096,
-        MI355X: 1 row 83 -> 9, 161 rows 101 -> 13, 7,208 100 -> 39, 65,544 463 -> 227, 131,073 853 -> 474)."""
+        form, whose workgroup holds all 512 logits of its 64 rows, takes the widths that the dense layer does not and many rows of narrow ones
+        (us, one launch -> two, K = 4,096, MI355X: 1 row 83 -> 9, 161 rows 101 -> 13, 7,208 100 -> 39, 65,544 463 -> 227, 131,073 853 -> 474)."""
         self._need(h, torch.bfloat16, "unembed_logprob h")
         self._need(emb, torch.bfloat16, "unembed_logprob emb")
         M, K = h.shape
@@ -1189,7 +1196,7 @@ class HipOps(MixerOps):
         if target is not None:
             target = target.reshape(-1).to(torch.int64).contiguous()
             assert target.numel() == M
-        if V == 512 and K % 64 == 0 and 128 <= K <= 32768 and M > 0 and self.all_gemm_mfma:
+        if V == 512 and self.all_gemm_mfma and self._tail_in_two(M, K):
             # Whole chunks but for the last, which takes what is left of them: a row's logits are the same bits in any batch of 1,024 rows and more.
             # (32 K rows are 32 MB of logits, which the second kernel finds in the Infinity Cache.)
             n = max(1, M // self.TAIL_ROWS)

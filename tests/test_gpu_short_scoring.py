@@ -33,6 +33,22 @@ def test_tail_matches_the_oracle(ops, M, K):
     assert only is None and torch.equal(none, en)
 
 
+@pytest.mark.parametrize("M,K,two", [(4095, 448, True), (4096, 448, False), (4096, 512, True), (98303, 512, True), (98304, 512, False), (98304, 768, True)])
+def test_tail_on_both_sides_of_its_rule(ops, M, K, two):
+    """The two forms round the same logits once: equal but where an fp32 sum in the other order crosses a rounding boundary (one bf16 step of a logit)."""
+    assert ops._tail_in_two(M, K) == two
+    hid, emb = bf(torch.randn(M, K, generator=gen(46))).to(DEV), bf(torch.randn(512, K, generator=gen(47)) * (4.0 / math.sqrt(K))).to(DEV)
+    tgt = torch.randint(0, 512, (M,), generator=gen(48)).to(DEV)
+    lp, en = ops.unembed_logprob(hid, emb, tgt, want_entropy=True)
+    ops._tail_in_two = lambda M, K: not two
+    try:
+        lp2, en2 = ops.unembed_logprob(hid, emb, tgt, want_entropy=True)
+    finally:
+        del ops._tail_in_two
+    ulp = 32 * 2.0 ** -7                                         # (logits of up to 5 sigma = 20)
+    assert (lp - lp2).abs().max() <= 2.5 * ulp and (lp - lp2).abs().mean() <= 0.02 * ulp and (en - en2).abs().max() <= 2.5 * ulp
+
+
 def test_tail_in_chunks_is_bitwise_the_whole(ops):
     hid, emb = bf(torch.randn(5000, 512, generator=gen(43))).to(DEV), bf(torch.randn(512, 512, generator=gen(44)) * 0.2).to(DEV)
     tgt = torch.randint(0, 512, (5000,), generator=gen(45)).to(DEV)
