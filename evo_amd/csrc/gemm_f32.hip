@@ -312,8 +312,9 @@ __global__ __launch_bounds__(256) void gemm_f32_parts_kernel(F3Args a) {
 // One k-step (32 deep) of the n tiles that share a CU takes `start` + n `each` us (at most `per_cu` share it: LDS and registers), fitted to 33 to 4,000
 // rows of eight layers.  The matrix cores bound the larger tiles: 128 x 128 with two on a CU 222 TF, 256 x 256 235 TF (six bf16 products each: 1.4 PF, what a
 // large bf16 product reaches).  Against the library's fp32 MFMA layers (us, K = 4,096, MI355X,
-// before -> here): 4,096 columns 40 -> 38 at 65 rows, 85 -> 80 at 300, 348 -> 254 at 1,290, 931 -> 623 at 4,000; 22,016 columns 180 -> 141, 442 -> 342,
-// 1,816 -> 1,257, 5,454 -> 3,500; K = 11,008, 4,096 columns 93 -> 86, 230 -> 181, 932 -> 668, 2,421 -> 1,692.  Error against 64 bits (random normal operands,
+// back to back on the GPU, before -> here): 4,096 columns 38 -> 41 at 65 rows, 56 -> 49 at 161, 90 -> 82 at 300, 1,002 -> 627 at 4,000; 22,016 columns
+// 160 -> 135, 290 -> 232, 456 -> 359, at 1,500 2,212 -> 1,424; K = 11,008, 4,096 columns 89 -> 92, 140 -> 117, 222 -> 190, at 1,500 1,039 -> 703.  Small layers are left
+// to the library (HipOps._f32_layer_pays).  Error against 64 bits (random normal operands,
 // 4,096 x 4,096): 1.00e-6 unsplit, 7.1e-7 in two parts, 5.0e-7 in four, 3.5e-7 in eight; library 1.14e-6.
 struct F3Kind { int bm, bn, per_cu; double start, each; };
 static const F3Kind f3_kinds[] = {{64, 64, 5, 0.29, 0.33}, {64, 128, 4, 0.30, 0.655}, {128, 128, 2, 0.20, 1.11}, {256, 256, 1, 0.10, 4.36}};

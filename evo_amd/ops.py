@@ -4,7 +4,7 @@
 loaded or a tensor is not on a ROCm device -- there is no CPU / eager fallback.  Every kernel of a scoring or generation
 step -- the dense layers included (csrc/gemm.hip, csrc/gemv.hip) -- is a hand-written gfx950 kernel reached through the C ABI with
 raw device pointers and the caller's current stream; hipBLASLt (through `torch.addmm`) serves only shapes no 7B layer has, fp32
-layers of up to 32 rows and the in-process A/B knob `all_gemm_mfma = False`.
+layers of up to 32 rows, small ones and the in-process A/B knob `all_gemm_mfma = False`.
 """
 from __future__ import annotations
 
@@ -318,7 +318,7 @@ class HipOps(MixerOps):
             return y
         if self._take_mfma(mfma) and self.mfma_linear_ok(x, w):
             return self.linear_mfma(x, w, b)
-        if self._f32_layer_ok(x, w, b):
+        if x.dtype == torch.float32 and x.dim() == w.dim() == 2 and self._f32_layer_pays(x.shape[0], *w.shape) and self._f32_layer_ok(x, w, b):
             return self._linear_f32(x, w, b)
         with self._t("gemm"):
             if b is not None:
@@ -334,10 +334,17 @@ class HipOps(MixerOps):
                 or (torch._C._len_torch_function_stack() > 0
                     and any(type(m) is not DeviceContext for m in torch.overrides._get_current_function_mode_stack())))
 
+    @staticmethod
+    def _f32_layer_pays(M: int, N: int, K: int) -> bool:
+        """Whether the layer is large enough for csrc/gemm_f32.hip: a step of 32 k takes its tiles 0.9 us however few they are, and below this the library's tiles
+        are done sooner (back to back on the GPU, us, library -> here.  4,096 x 4,096: 33 rows 24 -> 27, 100 39 -> 42, 161 56 -> 49, 1,000 256 -> 183; 512 x 4,096:
+        300 22 -> 25, 1,500 56 -> 50; 4,096 x 512: 300 16 -> 20, 513 29 -> 26; 2,048 x 1,024: 513 26 -> 33, 700 44 -> 33; 256 x 16,384: 300 45 -> 56, 1,500
+        127 -> 99).  Above it 0.9 to 2 times as fast, 1.1 and more but for single sizes."""
+        return M * N >= 1350000 or M * N * K >= 2200000000
+
     def _f32_layer_ok(self, x, w, b) -> bool:
-        """fp32 layers from 33 rows on take csrc/gemm_f32.hip; below, the weight's own bytes bound the layer and the library reads them at 2.5 to 4.6 TB/s
-        (24 rows: 26 us against 36 at 4,096 x 4,096, 79 against 91 at 22,016 x 4,096; 33 rows: 31 against 28, 117 against 93).  What is traced or
-        differentiated stays with torch, and so does what lies on another device than the current one, whose stream the launch goes to."""
+        """What csrc/gemm_f32.hip takes, from 33 rows on; below, the weight's own bytes bound the layer and the library reads them at 2.5 to 4.6 TB/s.  What is
+        traced or differentiated stays with torch, and so does what lies on another device than the current one, whose stream the launch goes to."""
         ts = (x, w) if b is None else (x, w, b)
         return (self.all_gemm_mfma and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()
                                            and t.device == x.device and t.data_ptr() % 16 == 0 for t in ts)

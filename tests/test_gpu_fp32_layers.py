@@ -11,7 +11,9 @@ DEV = "cuda:0"
 @pytest.fixture(scope="module")
 def ops():
     from evo_amd.ops import HipOps
-    return HipOps()
+    o = HipOps()
+    o._f32_layer_pays = lambda M, N, K: True                     # (the kernel itself, at sizes that the library would take too)
+    return o
 
 
 def rand(*shape, seed=0):
@@ -138,6 +140,16 @@ def test_what_keeps_torch(ops):
         assert ops._f32_layer_ok(x, g, None)
     with torch.autograd.forward_ad.dual_level():
         assert not ops._f32_layer_ok(x, w, None)
+
+
+@pytest.mark.parametrize("M,N,K,own", [(33, 4096, 4096, False), (131, 4096, 4096, False), (132, 4096, 4096, True), (33, 22016, 4096, True), (329, 4096, 256, False), (330, 4096, 256, True),
+                                       (32, 22016, 11008, False)])
+def test_small_layers_are_the_librarys(M, N, K, own, monkeypatch):
+    from evo_amd.ops import HipOps
+    o, took = HipOps(), []
+    monkeypatch.setattr(o, "_linear_f32", lambda x, w, b: took.append(x.shape) or torch.mm(x, w.t()))
+    x, w = torch.zeros(M, K, device=DEV), torch.zeros(N, K, device=DEV)
+    assert o.linear(x, w).shape == (M, N) and bool(took) == own
 
 
 def test_tensors_of_another_device_keep_torch(ops, monkeypatch):
