@@ -297,7 +297,7 @@ class HipOps(MixerOps):
 
     def _dense_layer(self, mode, x, w, y, M, N, K, act=0, xblk=0, b=None, res=None, rs=None, ss=None, act_cols=0, x_rows=0, Tm=0, row_skip=0) -> None:
         """evo_dense_bf16 (include/evo_mi355x.h) with the workspace that its tiles ask for."""
-        n = self.lib.evo_dense_ws(mode, ss is not None, M, N, K)
+        n = self.lib.evo_dense_ws(mode, ss is not None, M, N, K) if M < 1024 else 0          # (parts of K only below)
         ws = torch.empty(n, dtype=torch.uint8, device=y.device) if n > 0 else None
         _check(self.lib.evo_dense_bf16(mode, act, xblk, x.data_ptr(), w.data_ptr(), _ptr(b), _ptr(res), y.data_ptr(), _ptr(rs), _ptr(ss),
                                        0 if ss is None else ss.shape[1], M, N, K, act_cols, x_rows, Tm, row_skip, _ptr(ws), max(n, 0), _stream()),
@@ -318,7 +318,7 @@ class HipOps(MixerOps):
             return y
         if self._take_mfma(mfma) and self.mfma_linear_ok(x, w):
             return self.linear_mfma(x, w, b)
-        if x.dtype == torch.float32 and x.dim() == w.dim() == 2 and self._f32_layer_pays(x.shape[0], *w.shape) and self._f32_layer_ok(x, w, b):
+        if x.dtype == torch.float32 and x.shape[0] > 32 and x.dim() == w.dim() == 2 and self._f32_layer_pays(x.shape[0], *w.shape) and self._f32_layer_ok(x, w, b):
             return self._linear_f32(x, w, b)
         with self._t("gemm"):
             if b is not None:
