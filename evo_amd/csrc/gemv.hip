@@ -897,107 +897,13 @@ __global__ __launch_bounds__(512) void skinny_mfma_kernel(const uint4* __restric
     }
 }
 
-// ---- 5 <= M <= 64, N >= 8192: n-split form (round 6).  The k-split form above is bound by L2, not by HBM: every weight fragment (1 KiB per
-// wave) pulls MT x fragments of the same size through L2 -- weights + x add up to 6-7 TB/s at every M (4.0 TB/s of weights at 8 rows, 3.4 at
-// 16, 2.2 at 32, 1.5 at 64; tools/bench_gemv.py) where hipBLASLt streams 4.2 TB/s at 32-64 rows.  Here a workgroup is WAVES waves, each owning a
-// 16-row n tile for the WHOLE K (no partial sums, no reduction), and the x rows of a 256-k chunk are staged in LDS once per workgroup and
-// read by all its waves as B fragments (ds_read_b128, conflict-free at a row pitch of 528 B): x costs L2 MT / WAVES of the weight bytes
-// instead of MT.  Weight fragments of chunk c + 1 and the x rows of chunk c + 1 are requested before chunk c is multiplied.  K % 256 == 0.
-template <int MT, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void skinny_n_kernel(const uint4* __restrict__ x, const uint4* __restrict__ w,
-                                                              const uint16_t* __restrict__ bias, const uint16_t* res,
-                                                              uint16_t* y, int M, int N, int nvec, int act) {   // res may alias y
-    constexpr int KC = 8, ROWB = KC * 64 + 16;                   // steps per chunk; LDS bytes per x row (512 + 16 pad)
-    constexpr int XL = (MT * 16 * KC * 4 + 64 * WAVES - 1) / (64 * WAVES);   // 16-byte pieces of an x chunk per thread
-    __shared__ __attribute__((aligned(16))) unsigned char xs[2][MT * 16 * ROWB];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r16 = lane & 15, kb = lane >> 4;
-    const int n0 = (blockIdx.x * WAVES + wave) * 16;
-    const int nrow = n0 + r16 < N ? n0 + r16 : N - 1;
-    const uint4* wp = w + (int64_t)nrow * nvec + kb;
-    const int n_chunk = nvec / (KC * 4);
-    gv_f32x4 acc[MT];
-#pragma unroll
-    for (int t = 0; t < MT; ++t) acc[t] = gv_f32x4{0.f, 0.f, 0.f, 0.f};
-    // x chunk pieces of this thread: piece p = tid + i * threads -> row p / 32 (32 pieces of 16 B per 512-byte row), column p % 32
-    // (native vectors, not HIP's uint4 struct: as a loop-carried, conditionally written array of uint4 the pieces stayed in scratch memory)
-    typedef unsigned int sn_u32x4 __attribute__((ext_vector_type(4)));
-    sn_u32x4 xr[XL];
-#define SN_X_LOAD(C)                                                                                          \
-    _Pragma("unroll") for (int i_ = 0; i_ < XL; ++i_) {                                                       \
-        const int pidx_ = tid + i_ * 64 * WAVES;                                                              \
-        int row_ = pidx_ >> 5;                                                                                \
-        row_ = row_ < M ? row_ : M - 1;              /* rows past M (and pieces past the chunk) re-read a valid row: never stored */ \
-        xr[i_] = *(const sn_u32x4*)(x + (int64_t)row_ * nvec + (C) * (KC * 4) + (pidx_ & 31));               \
-    }
-#define SN_X_STORE(BUF)                                                                                       \
-    _Pragma("unroll") for (int i_ = 0; i_ < XL; ++i_) {                                                       \
-        const int pidx_ = tid + i_ * 64 * WAVES;                                                              \
-        if (pidx_ < MT * 16 * 32) *(sn_u32x4*)(xs[BUF] + (pidx_ >> 5) * ROWB + (pidx_ & 31) * 16) = xr[i_];   \
-    }
-#ifndef SN_PROBE_CONTIG
-#define SN_PROBE_CONTIG 0                    // measurement only (WRONG results): weight fragments read as if stored fragment-major, 1 KiB contiguous per request
-#endif
-    auto w_load = [&](int c, uint4 (&wf)[KC]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < KC; ++u)
-            wf[u] = SN_PROBE_CONTIG ? ld_stream(w + ((int64_t)(n0 >> 4) * (nvec >> 2) + c * KC + u) * 64 + lane) : ld_stream(wp + 4 * (c * KC + u));
-    };
-    auto mul = [&](int buf, const uint4 (&wf)[KC]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < KC; ++u)
-#pragma unroll
-            for (int t = 0; t < MT; ++t) {
-                const uint4 xv = *(const uint4*)(xs[buf] + (16 * t + r16) * ROWB + u * 64 + kb * 16);
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[u]), __builtin_bit_cast(bf16x8_t, xv), acc[t], 0, 0, 0);
-            }
-    };
-    // weight fragments: chunk c multiplies while c + 1 is in flight (a ring of three -- 16 KiB per wave in flight -- measured 5-8 % SLOWER: the form is
-    // not latency-bound; what caps it is the access pattern, 64-byte pieces of 16 rows per request: read as if the weight were stored fragment-major
-    // (1 KiB contiguous per request, SN_PROBE_CONTIG) the same kernel streams 4.3-4.4 TB/s at 17-32 rows, hipBLASLt's rate, instead of 3.1-3.3)
-    uint4 wA[KC], wB[KC];
-    SN_X_LOAD(0);
-    w_load(0, wA);
-    SN_X_STORE(0);
-    __syncthreads();
-#define SN_STAGE(C, WCUR, WNEXT, BUF)                                                                         \
-    if ((C) < n_chunk) {                                                                                      \
-        if ((C) + 1 < n_chunk) { SN_X_LOAD((C) + 1); w_load((C) + 1, WNEXT); }                                \
-        mul(BUF, WCUR);                                                                                       \
-        if ((C) + 1 < n_chunk) { SN_X_STORE((BUF) ^ 1); }                                                     \
-        __syncthreads();                                                                                      \
-    }
-    for (int c = 0; c < n_chunk; c += 2) {                       // two chunks per trip: the fragment sets alternate without register copies
-        SN_STAGE(c, wA, wB, 0) SN_STAGE(c + 1, wB, wA, 1)
-    }
-#undef SN_STAGE
-#undef SN_X_LOAD
-#undef SN_X_STORE
-    // D[n][m]: lane holds n = n0 + 4 kb + r, m = 16 t + r16 -- four consecutive output columns of its row
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        const int m = 16 * t + r16;
-        if (m < M) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int n = n0 + 4 * kb + r;
-                if (n < N) {
-                    float o = acc[t][r] + (bias ? bf_to_f(bias[n]) : 0.f);
-                    if (res) o += bf_to_f(res[(int64_t)m * N + n]);
-                    y[(int64_t)m * N + n] = f_to_bf(out_act(o, act));
-                }
-            }
-        }
-    }
-}
-
-// ---- 5 <= M <= 32 on the narrow layers (N < 8192: a workgroup per 16 columns is about one per CU): the k-split form with whole row pieces.  A workgroup =
+// ---- 3 to 32 rows on the narrow layers (N <= 4096: a workgroup per 16 columns is about one per CU): the k-split form with whole row pieces.  A workgroup =
 // 16 weight rows; its waves take every WAVES-th chunk of CH k and park weight and batch rows of a chunk in a PRIVATE part of LDS (asynchronous loads of
 // 1 KiB = whole row pieces of 2 CH bytes, no registers, no barrier), NB chunks in flight; the WAVES partial tiles meet in LDS at the end.  Granule g of a
 // row sits at slot g ^ (row & 15): a fragment read meets no bank twice.
-// Bound by the weight stream and, at K = 4,096, by a launch's ramp: 4.3 - 4.7 TB/s at 8 rows; the fragment-shaped requests of skinny_mfma_kernel (64 bytes
-// of each of 16 rows) ran at 2.7 - 3.5.
+// Bound by the weight stream and, at K = 4,096, by a launch's ramp (us at 8 / 16 / 32 rows, a plain read of the matrix in brackets; all workgroups from K = 0 on ->
+// three chunks apart by turns, four waves): 4,096 x 4,096 [6.5] 8.0 / 8.9 / 10.6 -> 7.6 / 8.2 / 9.8; K = 11,008 [14.1] 18.6 / 20.1 / 23.3 -> 16.1 / 17.6 / 21.8;
+// K = 16,384 [22.0] 28.5 / 29.9 / 33.3 -> 22.8 / 22.3 / 29.3.
 // XR: batch rows loaded (8, 16 or 32; rows behind M read as zero or are a repeated row, and are never stored).
 #define KW_WAIT(N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory")
 template <int XR, int WAVES, int CH, int NB>
@@ -1024,7 +930,9 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kw_kernel(const unsigned ch
         off[i] = (uint32_t)r * rowb + (uint32_t)((lane % GR) ^ (r & 15 & (GR - 1))) * 16u;
     }
     const int chunks = K / CH, mine = (chunks - wave + WAVES - 1) / WAVES;
+    const int start = mine > 0 && gridDim.x >= 128 ? (int)(blockIdx.x >> 3) * 3 % mine : 0;       // (workgroups of an XCD don't walk K in step: skinny_ring_kernel)
     auto fetch = [&](int i, uint32_t buf) {
+        i = start + i >= mine ? start + i - mine : start + i;
         const uint32_t so = (uint32_t)(wave + WAVES * i) * ROW;
 #pragma unroll
         for (int j = 0; j < PW; ++j)
@@ -1107,150 +1015,171 @@ static int kw_launch(const void* x, const void* w, const void* bias, const void*
     return evo_launch_status();
 }
 
-// ---- the n-split form with CONTIGUOUS weight requests (round 6, second step).  skinny_n_kernel asks for a weight fragment as the MFMA wants it: 64 bytes
-// of each of 16 rows that lie K * 2 bytes apart -- and streams 3.1-3.3 TB/s where the same kernel reading 1 KiB contiguous per request runs 4.3-4.4
-// (profiles/r06_small_m_nsplit_ab.txt).  Here a request covers RPI = 2 (4) whole row pieces of 512 (256) contiguous bytes, the wave parks the chunk in a
-// PRIVATE LDS region in row order and reads its fragments back from there (ds_write_b128 / ds_read_b128, both conflict-free at the padded row pitch);
-// the requests of chunk c + 1 are in flight while chunk c multiplies.  Everything else as skinny_n_kernel.
-// SPLITK (N < 8192, the two N = 4,096 layers of a block): blockIdx.y is a slice of the 256-k chunks; the slice's fp32 partial sums go to
-// ws [slices][M][N] and skinny_reduce_kernel adds them in slice order (+ bias, + residual, one rounding) -- 64 n groups x 4 slices = a workgroup
-// per CU with x still shared four ways, where the k-split form is L2-bound on x (2.1 TB/s at 32 rows).
-// GATE (WAVES = 4): the gated MLP's first half [REF stripedhyena/layers.py ParallelGatedMLP: gelu(l1 x) * l2 x] in one launch -- a workgroup's 64 weight rows are
-// 32 rows of W1 (waves 0, 1) and the MATCHING 32 rows of W2 (waves 2, 3): one block of the grouped layout (`gate_layout` 1: HipOps.pack_gate_weights), or rows
-// c .. c + 31 and I + c .. of the plain [W1; W2] (2).  Waves 2, 3 hand their z2 tiles over through LDS; z1, z2 are rounded to bf16 (the dense layer's outputs),
-// the gate is evaluated in fp32 and rounded once: bit for bit the dense layer + evo_gelu_gate_bf16.  N = 2 I, y = a [M, I].
-template <int MT, int WAVES, bool SPLITK = false, bool GATE = false>
-__global__ __launch_bounds__(64 * WAVES) void skinny_nw_kernel(const uint4* __restrict__ x, const uint4* __restrict__ w,
-                                                               const uint16_t* __restrict__ bias, const uint16_t* res,
-                                                               uint16_t* y, int M, int N, int nvec, float* __restrict__ ws = nullptr,
-                                                               int gate_layout = 0, int act = 0) {   // res may alias y
-    static_assert(!GATE || (WAVES == 4 && !SPLITK), "a gated workgroup is one 32 + 32 row block");
-    constexpr int KC = MT <= 2 ? 8 : 4;                          // MFMA steps (32 k) per chunk
-    constexpr int ROWB = KC * 64 + 16;                           // LDS bytes per row of a chunk (+ 16 pad: b128 accesses at this pitch touch all banks)
-    constexpr int PPR = KC * 4;                                  // 16-byte pieces per row of a chunk
-    constexpr int RPI = 64 / PPR;                                // weight rows per request
-    constexpr int XL = (MT * 16 * PPR + 64 * WAVES - 1) / (64 * WAVES);   // x pieces per thread and chunk
-    __shared__ __attribute__((aligned(16))) unsigned char xs[2][MT * 16 * ROWB];
-    __shared__ __attribute__((aligned(16))) unsigned char wsm[WAVES][16 * ROWB];
-    typedef unsigned int sn_u32x4 __attribute__((ext_vector_type(4)));   // (native vectors: loop-carried uint4 arrays end up in scratch memory)
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+// ---- 3 to 64 rows on the wide layers (and, with parts of K, on the narrow ones from 17 rows on): a workgroup owns N / gridDim.x weight rows (any number up to
+// 16 T, a wave per 16 of them) and walks K in chunks of 128; weight and batch rows of a chunk arrive in LDS by asynchronous loads (no registers) into a ring
+// of NB stages, NB - 1 of them under way, one barrier per chunk.  LDS rows of 256 B, granule g of row r at slot g ^ (r & 15): a fragment read meets no bank twice.
+// What bounds it is the weight stream, under three conditions that decide the layout (us, MI355X, launches back to back; a plain read of the matrix in brackets):
+//  * every CU has the same number of rows: 22,016 x 4,096 [26.3] at 16 rows takes 28.6 in 256 x 86 rows, 36.2 in 344 x 64;
+//  * workgroups of one XCD don't walk K in step: rows lie a power of two apart, so equal places of K are the same L2 channels.  Starts one chunk apart by turns
+//    took 16,384 x 4,096 [22.0] at 16 rows from 34.8 to 21.4 (32 rows a workgroup), 8,192 x 28,672 [69] from 107 to 69;
+//  * the batch rows, read once per workgroup, are few against its weight rows.
+// At 8 / 16 / 32 / 64 rows: 22,016 x 4,096 32.6 / 33.4 / 36.6 / 46.4 (register-staged chunks, 64 rows a workgroup, all from K = 0 on) -> 28.4 / 28.6 / 29.4 / 32.5;
+// 16,384 x 4,096 26.1 / 26.3 / 29.2 / 36.3 -> 22.1 / 22.3 / 23.2 / 26.0; 12,288 x 4,096 [16.0] 20.8 / 21.4 / 22.4 / 34.0 -> 17.1 / 17.1 / 17.6 / 21.8;
+// 8,192 x 4,096 [11.4] 20.4 / 20.4 / 21.1 / 30.6 -> 12.1 / 12.3 / 13.8 / 17.5.
+// MODE 0: y = x w^T (+ bias, + residual, activation).  MODE 1: the gated MLP's first half [REF stripedhyena/layers.py ParallelGatedMLP: gelu(l1 x) * l2 x]: a wave's 16
+// rows are 8 of W1 and the same 8 of W2 (`layout` 1: HipOps.pack_gate_weights' blocks of 32 + 32 rows, 2: plain [W1; W2]), z2 crosses by one lane exchange, both are
+// rounded to bf16 (the dense layer's outputs), the gate is evaluated in fp32 and rounded once; N = 2 I, y = a [M, I].  A column's first chunk follows its place:
+// where N >= 16,384 is no multiple of 4,096 workgroup b of MODE 1 starts where b / 2 and b / 2 + half of MODE 0 do, which hold its columns of plain [W1; W2]: both
+// give the same bits there.
+// MODE 2: blockIdx.y is a part of K, fp32 partial sums to ws [parts][M][N] (skinny_reduce_kernel adds them in order).
+typedef uint32_t rg_u32x4 __attribute__((ext_vector_type(4)));
+#define RG_WAIT(N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory")
+#define RG_ROWB 256                          // bytes of a row's piece of a chunk
+#define RG_NONE 0xf0000000u                  // behind every buffer: nothing is read, zero arrives
+template <int XR, int T, int NB, int MODE>
+__global__ __launch_bounds__(64 * T) void skinny_ring_kernel(const unsigned char* __restrict__ x, const unsigned char* __restrict__ w, const uint16_t* __restrict__ bias,
+                                                             const uint16_t* res, uint16_t* y, int M, int N, int K, int act, int layout, float* __restrict__ ws) {   // res may alias y
+    constexpr int MT = XR / 16, PX = (XR / 4 + T - 1) / T, PW = 4, P = PX + PW;      // requests of 1 KiB (4 rows) per wave and chunk
+    constexpr int XOFF = T * 16 * RG_ROWB, BUF = XOFF + T * PX * 1024;
+    static_assert(XR % 16 == 0 && NB >= 2 && (NB - 2) * P < 64, "the wait counter has six bits");
+    extern __shared__ __attribute__((aligned(16))) unsigned char rg_lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, kb = lane >> 4;
-    const int n0 = GATE && gate_layout == 2 ? (wave < 2 ? blockIdx.x * 32 + wave * 16 : (N >> 1) + blockIdx.x * 32 + (wave - 2) * 16)
-                                            : (blockIdx.x * WAVES + wave) * 16;
-    const int n_chunk_all = nvec / PPR;
-    const int c_first = SPLITK ? (int)((int64_t)n_chunk_all * blockIdx.y / gridDim.y) : 0;
-    const int n_chunk = SPLITK ? (int)((int64_t)n_chunk_all * (blockIdx.y + 1) / gridDim.y) : n_chunk_all;   // chunks [c_first, n_chunk) are this workgroup's
-    // request i of a chunk: weight row n0 + RPI i + lane / PPR, piece lane % PPR
-    const int q_row = lane / PPR, q_piece = lane % PPR;
-    const sn_u32x4* wq[KC];
+    const uint32_t rowb = (uint32_t)K * 2;
+    const int cols = MODE == 1 ? N >> 1 : N;                     // result columns; this workgroup's: lo .. hi - 1
+    const uint32_t each = (uint32_t)cols / gridDim.x, more = (uint32_t)cols % gridDim.x;
+    const int lo = (int)(blockIdx.x * each + blockIdx.x * more / gridDim.x), hi = (int)((blockIdx.x + 1) * each + (blockIdx.x + 1) * more / gridDim.x);
+    // weight rows: four requests of four rows; of MODE 1 the first two from W1, the others from W2
+    rg_u32x4 rw[2];
+    uint32_t ow[PW];
 #pragma unroll
-    for (int i = 0; i < KC; ++i) {
-        const int row = n0 + RPI * i + q_row < N ? n0 + RPI * i + q_row : N - 1;
-        wq[i] = (const sn_u32x4*)(w + (int64_t)row * nvec + q_piece);
+    for (int h = 0; h < 2; ++h) {
+        const bool grouped = MODE == 1 && layout == 1;
+        const int64_t first = MODE != 1 ? lo : (grouped ? 64 * (int64_t)(lo >> 5) + 32 * h : (int64_t)h * cols + lo);
+        const uint64_t a = (uint64_t)w + (uint64_t)first * rowb;
+        const uint32_t rows = grouped ? 64 * (((hi - 1) >> 5) - (lo >> 5)) + 32 : hi - lo;
+        rw[h] = rg_u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, rows * rowb, 0x00020000u};
     }
-    unsigned char* wmine = wsm[wave];
-    const int w_st = q_row * ROWB + q_piece * 16;               // + RPI * i * ROWB
-    const int f_rd = r16 * ROWB + kb * 16;                       // + u * 64
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+        const int q = i * 4 + (lane >> 4), c = MODE == 1 ? lo + 8 * wave + (q & 7) : lo + 16 * wave + q;     // row of the tile, its column
+        const int r = MODE == 1 && layout == 1 ? 64 * ((c >> 5) - (lo >> 5)) + (c & 31) : c - lo;
+        ow[i] = c < hi ? (uint32_t)r * rowb + (uint32_t)((lane & 15) ^ q) * 16u : RG_NONE;
+    }
+    const uint64_t xa = (uint64_t)x;
+    const rg_u32x4 rx = {(uint32_t)xa, (uint32_t)(xa >> 32) & 0xffffu, (uint32_t)M * rowb, 0x00020000u};
+    uint32_t ox[PX];
+#pragma unroll
+    for (int i = 0; i < PX; ++i) {
+        const int r = (wave * PX + i) * 4 + (lane >> 4);
+        ox[i] = r < M ? (uint32_t)r * rowb + (uint32_t)((lane & 15) ^ (r & 15)) * 16u : RG_NONE;
+    }
+    // bias and residual values of this lane's results, requested ahead of everything (from places that are there, and looked at behind the last product: no wait here)
+    uint32_t pb[4], pr[MODE == 0 ? MT : 1][4];
+    const int n0 = lo + 16 * wave + 4 * kb;
+    if (MODE == 0 && bias) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) pb[r] = bias[n0 + r < N ? n0 + r : N - 1];
+    }
+    if (MODE == 0 && res) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const uint16_t* from = res + (int64_t)(16 * t + r16 < M ? 16 * t + r16 : M - 1) * N;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) pr[t][r] = from[n0 + r < N ? n0 + r : N - 1];
+        }
+    }
+    const int all = K / 128, c0 = MODE == 2 ? (int)((int64_t)all * blockIdx.y / gridDim.y) : 0;
+    const int chunks = (MODE == 2 ? (int)((int64_t)all * (blockIdx.y + 1) / gridDim.y) : all) - c0;
+    // (block b runs on XCD b % 8; where halves start alike they meet in the L2 channels if they lie a power of two apart: 8,192 x 4,096 at 8 rows 16.2 us, 12.1 without)
+    const bool halves = N >= 16384 && (N & 4095) != 0;
+    int at = (int)(halves ? (MODE == 1 ? blockIdx.x >> 1 : blockIdx.x) >> 3 & 15 : blockIdx.x >> 3) % chunks;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)rg_lds;
+    auto fetch = [&](uint32_t buf) {
+        const uint32_t so = (uint32_t)(c0 + at) * RG_ROWB;
+#pragma unroll
+        for (int j = 0; j < PX; ++j)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(buf + XOFF + (wave * PX + j) * 1024), "v"(ox[j]), "s"(rx), "s"(so) : "memory", "m0");
+#pragma unroll
+        for (int j = 0; j < PW; ++j)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(buf + (wave * PW + j) * 1024), "v"(ow[j]), "s"(rw[j >> 1]), "s"(so) : "memory", "m0");
+        at = at + 1 == chunks ? 0 : at + 1;
+    };
     gv_f32x4 acc[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = gv_f32x4{0.f, 0.f, 0.f, 0.f};
-    sn_u32x4 xr[XL], wr[KC];
-#define SW_X_LOAD(C)                                                                                          \
-    _Pragma("unroll") for (int i_ = 0; i_ < XL; ++i_) {                                                       \
-        const int pidx_ = tid + i_ * 64 * WAVES;                                                              \
-        int row_ = pidx_ / PPR;                                                                               \
-        row_ = row_ < M ? row_ : M - 1;              /* rows past M (and pieces past the chunk) re-read a valid row: never stored */ \
-        xr[i_] = *(const sn_u32x4*)(x + (int64_t)row_ * nvec + (C) * PPR + (pidx_ % PPR));                    \
-    }
-#define SW_X_STORE(BUF)                                                                                       \
-    _Pragma("unroll") for (int i_ = 0; i_ < XL; ++i_) {                                                       \
-        const int pidx_ = tid + i_ * 64 * WAVES;                                                              \
-        if (pidx_ < MT * 16 * PPR) *(sn_u32x4*)(xs[BUF] + (pidx_ / PPR) * ROWB + (pidx_ % PPR) * 16) = xr[i_]; \
-    }
-#define SW_W_LOAD(C) _Pragma("unroll") for (int i_ = 0; i_ < KC; ++i_) wr[i_] = __builtin_nontemporal_load(wq[i_] + (C) * PPR);
-#define SW_W_STORE() _Pragma("unroll") for (int i_ = 0; i_ < KC; ++i_) *(sn_u32x4*)(wmine + w_st + RPI * i_ * ROWB) = wr[i_];
-    auto mul = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < KC; ++u) {
-            const uint4 wv = *(const uint4*)(wmine + f_rd + u * 64);
+    for (int i = 0; i < NB - 1; ++i)
+        if (i < chunks) fetch(lds0 + i * BUF);
+    uint32_t buf = lds0, nxt = lds0 + (NB - 1) * BUF, g[4];
 #pragma unroll
-            for (int t = 0; t < MT; ++t) {
-                const uint4 xv = *(const uint4*)(xs[buf] + (16 * t + r16) * ROWB + u * 64 + kb * 16);
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wv), __builtin_bit_cast(bf16x8_t, xv), acc[t], 0, 0, 0);
+    for (int u = 0; u < 4; ++u) g[u] = (uint32_t)r16 * RG_ROWB + (uint32_t)((4 * u + kb) ^ r16) * 16u;
+    for (int i = 0; i < chunks; ++i) {
+        if (i + NB - 1 <= chunks) RG_WAIT((NB - 2) * P); else RG_WAIT(0);      // this wave's part of chunk i has landed,
+        asm volatile("s_barrier" ::: "memory");                                // every wave's; and every wave has read chunk i - 1, whose place is free
+        if (i + NB - 1 < chunks) fetch(nxt);
+        nxt = nxt + BUF == lds0 + NB * BUF ? lds0 : nxt + BUF;
+#pragma unroll
+        for (int h = 0; h < 4; h += 2) {
+            rg_u32x4 wf[2], xf[2][MT];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                asm volatile("ds_read_b128 %0, %1" : "=v"(wf[u]) : "v"(buf + wave * (16 * RG_ROWB) + g[h + u]));
+#pragma unroll
+                for (int t = 0; t < MT; ++t) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(xf[u][t]) : "v"(buf + XOFF + g[h + u]), "n"(t * 16 * RG_ROWB));
             }
-        }
-    };
-    SW_X_LOAD(c_first);
-    SW_W_LOAD(c_first);
-    SW_X_STORE(c_first & 1);
-    SW_W_STORE();
-    __syncthreads();
-    for (int c = c_first; c < n_chunk; ++c) {
-        const int buf = c & 1;
-        if (c + 1 < n_chunk) { SW_X_LOAD(c + 1); SW_W_LOAD(c + 1); }
-        mul(buf);
-        // no barrier here: x buffer buf ^ 1 has been free since the last barrier, and the weight region is the wave's own -- its stores follow its reads
-        // in program order (same LDS array: the compiler keeps the order, the LDS unit executes a wave's accesses in order)
-#ifdef SW_TWO_BARRIERS
-        __syncthreads();
-#endif
-        if (c + 1 < n_chunk) { SW_X_STORE(buf ^ 1); SW_W_STORE(); }
-        __syncthreads();
-    }
-#undef SW_X_LOAD
-#undef SW_X_STORE
-#undef SW_W_LOAD
-#undef SW_W_STORE
-    if constexpr (GATE) {
-        // (the last barrier of the chunk loop is behind every wave's last fragment read: xs is free)
-        float* ex = (float*)&xs[0][0];                           // [2 waves][MT][64 lanes] x 16 B <= 4 KiB
-        if (wave >= 2) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-            for (int t = 0; t < MT; ++t) *(gv_f32x4*)(ex + (((wave - 2) * MT + t) * 64 + lane) * 4) = acc[t];
-        }
-        __syncthreads();
-        if (wave < 2) {
-            const int I_ = N >> 1;
-            const int col0 = blockIdx.x * 32 + wave * 16 + 4 * kb;           // this lane's four gated columns
+            for (int u = 0; u < 2; ++u) {
+                asm volatile("" : "+v"(wf[u]));
 #pragma unroll
-            for (int t = 0; t < MT; ++t) {
-                const gv_f32x4 z2 = *(const gv_f32x4*)(ex + ((wave * MT + t) * 64 + lane) * 4);
-                const int m = 16 * t + r16;
-                if (m < M && col0 < I_) {
-                    const f32x2_t ua = {round_bf(acc[t][0]), round_bf(acc[t][1])}, ga = {round_bf(z2[0]), round_bf(z2[1])};
-                    const f32x2_t ub = {round_bf(acc[t][2]), round_bf(acc[t][3])}, gb = {round_bf(z2[2]), round_bf(z2[3])};
-                    const f32x2_t oa = act_gate2(ua, ga, act), ob = act_gate2(ub, gb, act);
-                    uint2 o;
-                    o.x = pack_bf2(oa[0], oa[1]);
-                    o.y = pack_bf2(ob[0], ob[1]);
-                    *(uint2*)(y + (int64_t)m * I_ + col0) = o;               // (I % 32 == 0: whole groups of four)
+                for (int t = 0; t < MT; ++t) {
+                    asm volatile("" : "+v"(xf[u][t]));
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[u]), __builtin_bit_cast(bf16x8_t, xf[u][t]), acc[t], 0, 0, 0);
                 }
             }
         }
-        return;
+        buf = buf + BUF == lds0 + NB * BUF ? lds0 : buf + BUF;
     }
-    if constexpr (SPLITK) {
-        float* wsl = ws + (int64_t)blockIdx.y * M * N;
+    // D[n][m]: lane holds rows 4 kb + r of its wave's tile, m = 16 t + r16
+    if constexpr (MODE == 1) {
+        const int c = lo + 8 * wave + 4 * (kb & 1);              // kb 0, 1: columns c .. c + 3 of W1; kb 2, 3: the same of W2
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
-            const int m = 16 * t + r16;
-            if (m < M && n0 + 4 * kb < N) *(gv_f32x4*)(wsl + (int64_t)m * N + n0 + 4 * kb) = acc[t];     // (N % 4 == 0 on this path)
-        }
-        return;
-    }
+            float z[4];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        const int m = 16 * t + r16;
-        if (m < M) {
+            for (int r = 0; r < 4; ++r) z[r] = __shfl_xor(acc[t][r], 32, 64);
+            const int m = 16 * t + r16;
+            if (kb < 2 && m < M) {
+                const f32x2_t ua = {round_bf(acc[t][0]), round_bf(acc[t][1])}, ub = {round_bf(acc[t][2]), round_bf(acc[t][3])};
+                const f32x2_t oa = act_gate2(ua, f32x2_t{round_bf(z[0]), round_bf(z[1])}, act), ob = act_gate2(ub, f32x2_t{round_bf(z[2]), round_bf(z[3])}, act);
+                uint16_t* to = y + (int64_t)m * cols + c;
+                const float o[4] = {oa[0], oa[1], ob[0], ob[1]};
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (c + r < hi) to[r] = f_to_bf(o[r]);
+            }
+        }
+    } else if constexpr (MODE == 2) {                            // (N / gridDim.x a multiple of 4: the host checks)
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+            if (16 * t + r16 < M && n0 < hi) *(gv_f32x4*)(ws + ((int64_t)blockIdx.y * M + 16 * t + r16) * N + n0) = acc[t];
+    } else {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            float o[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int n = n0 + 4 * kb + r;
-                if (n < N) {
-                    float o = acc[t][r] + (bias ? bf_to_f(bias[n]) : 0.f);
-                    if (res) o += bf_to_f(res[(int64_t)m * N + n]);
-                    y[(int64_t)m * N + n] = f_to_bf(out_act(o, act));
-                }
+                o[r] = acc[t][r];
+                if (bias) o[r] += bf_to_f((uint16_t)pb[r]);
+                if (res) o[r] += bf_to_f((uint16_t)pr[t][r]);
+                o[r] = out_act(o[r], act);
+            }
+            if (16 * t + r16 < M) {
+                uint16_t* to = y + (int64_t)(16 * t + r16) * N + n0;
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (n0 + r < hi) to[r] = f_to_bf(o[r]);
             }
         }
     }
@@ -1272,6 +1201,34 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
     out.x = pack_bf2(out_act(o[0], act), out_act(o[1], act));
     out.y = pack_bf2(out_act(o[2], act), out_act(o[3], act));
     *(uint2*)(y + e) = out;
+}
+
+// Ring launches.  Rows per workgroup: what 256 CUs get each, in as few rounds as 96 rows (T = 6) allow, at least 32; T: waves for them.  Stages: four (42 KB
+// each at T = 6 and 64 batch rows: three).
+template <int XR, int T, int MODE>
+static int ring_go(dim3 grid, const void* x, const void* w, const void* bias, const void* res, void* y, int64_t M, int64_t N, int64_t K, int act, int layout, float* ws,
+                   hipStream_t s) {
+    constexpr int NB = T == 6 && XR == 64 ? 3 : 4;
+    constexpr size_t lds = (size_t)NB * T * (16 * RG_ROWB + (XR / 4 + T - 1) / T * 1024);
+    static_assert(lds <= 160 * 1024, "the CU's LDS");
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)skinny_ring_kernel<XR, T, NB, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL((skinny_ring_kernel<XR, T, NB, MODE>), grid, dim3(64 * T), lds, s, (const unsigned char*)x, (const unsigned char*)w, (const uint16_t*)bias,
+                       (const uint16_t*)res, (uint16_t*)y, (int)M, (int)N, (int)K, act, layout, ws);
+    return evo_launch_status();
+}
+// parts > 0: MODE 2, 64 rows a workgroup (N a multiple of 64)
+template <int MODE>
+static int ring_launch(const void* x, const void* w, const void* bias, const void* res, void* y, int64_t M, int64_t N, int64_t K, int act, int layout, float* ws, int parts,
+                       hipStream_t s) {
+    const int64_t rounds = (N + 256 * 96 - 1) / (256 * 96), share = (N + 31) / 32;
+    const int64_t groups = parts ? N / 64 : (share < 256 ? share : 256 * rounds), rows = (N + groups - 1) / groups;
+    const dim3 grid((unsigned)groups, (unsigned)(parts ? parts : 1));
+#define EVO_RG(XR, T) ring_go<XR, T, MODE>(grid, x, w, bias, res, y, M, N, K, act, layout, ws, s)
+#define EVO_RG1(T) (M <= 16 ? EVO_RG(16, T) : M <= 32 ? EVO_RG(32, T) : EVO_RG(64, T))
+    if (MODE == 2) return EVO_RG1(4);
+    return rows <= 32 ? EVO_RG1(2) : rows <= 48 ? EVO_RG1(3) : rows <= 64 ? EVO_RG1(4) : EVO_RG1(6);
+#undef EVO_RG1
+#undef EVO_RG
 }
 
 template <int M>
@@ -1412,16 +1369,12 @@ static int mlp_gate_launch(const void* x, const void* scale, const void* w12, vo
 extern "C" int evo_mlp_gate_small_m_bf16(const void* x, const void* w12, void* a, int64_t M, int64_t I, int64_t K,
                                          int64_t grouped, int64_t act, void* stream) {
     if (act != 0 && act != 1) return -1;
-    if (M >= 5 && M <= 64) {
-        // 5-64 rows: the MFMA weight-streaming form with the gate in its epilogue (skinny_nw_kernel GATE), both weight layouts
-        if (I <= 0 || I % 32 != 0 || K <= 0 || K % 256 != 0 || I > 0x1fffffff) return -1;
-        hipStream_t s = (hipStream_t)stream;
-#define EVO_SNG(MT) hipLaunchKernelGGL((skinny_nw_kernel<MT, 4, false, true>), dim3((unsigned)(I / 32)), dim3(256), 0, s, (const uint4*)x, (const uint4*)w12,   \
-                                       (const uint16_t*)nullptr, (const uint16_t*)nullptr, (uint16_t*)a, (int)M, (int)(2 * I), (int)(K / 8), (float*)nullptr,     \
-                                       grouped ? 1 : 2, (int)act)
-        if (M <= 16) EVO_SNG(1); else if (M <= 32) EVO_SNG(2); else if (M <= 48) EVO_SNG(3); else EVO_SNG(4);
-#undef EVO_SNG
-        return evo_launch_status();
+    // (three and four rows: 34.4 -> 28.6 us at I = 11,008, K = 4,096; small layers, or where the asynchronous loads can't go, keep the dot2 form)
+    const bool ring = I > 0 && I % 32 == 0 && K > 0 && K % 128 == 0 && I <= 0x1fffffff && K <= 0x9fffff && (((uintptr_t)x | (uintptr_t)w12) & 15) == 0;
+    if (M >= 5 ? M <= 64 : (M >= 3 && ring && I * K >= 1 << 24)) {
+        // the MFMA weight-streaming form with the gate in its epilogue, both weight layouts
+        if (!ring) return -1;
+        return ring_launch<1>(x, w12, nullptr, nullptr, a, M, 2 * I, K, (int)act, grouped ? 1 : 2, nullptr, 0, (hipStream_t)stream);
     }
     return mlp_gate_launch(x, nullptr, w12, a, M, I, K, 0.f, grouped, (int)act, (hipStream_t)stream);
 }
@@ -1437,70 +1390,43 @@ extern "C" int evo_linear_small_m_bf16(const void* x, const void* w, const void*
     if (M < 1 || M > 64 || N <= 0 || K <= 0 || K % 8 != 0 || N > 0x7fffffff - 16) return -1;
     if ((M > 8 && K % 32 != 0) || (act != 0 && act != 3)) return -1;
     hipStream_t s = (hipStream_t)stream;
-    if (M >= 5 && K % 32 == 0) {
-        // narrow layers: whole row pieces through LDS (skinny_kw_kernel).  us before -> now at N = 4,096: K = 4,096 9.7 -> 7.8 at 8 rows, 11.0 -> 9.2 at 16,
-        // 16.1 -> 10.6 at 32; K = 11,008 27.3 -> 19.2, 31.3 -> 20.7, 24.4 -> 24.6 (and one launch less); K = 16,384 39.7 -> 29.8 at 8 -- at 32 rows the split
-        // over K across workgroups below stays ahead there (30.5 against 35.1); N = 6,912, K = 4,096 18.6 -> 13.8, 29.6 -> 17.7; N = 512 8.8 -> 5.7, 14.2 -> 8.1
-        if (N < 8192 && K % 128 == 0 && M <= (K < 12288 ? 32 : 16)) {
-            if (M <= 8) return kw_launch<8, 8, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);
-            if (M <= 16) return kw_launch<16, 8, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);
-            return kw_launch<32, 4, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);
-        }
-        // two n tiles per workgroup (every x fragment feeds two weight fragments) where that still leaves a workgroup or more per CU
-        static const int nt_env = [] { const char* e = getenv("EVO_SK_NT"); return e ? atoi(e) : 0; }();      // measurement knob: 1 / 2 force, 0 = auto
-        const int nt = nt_env ? nt_env : (N >= 8192 && M > 16 ? 2 : 1);
-        const dim3 block(512);
-        // n-split form: wide layers (a workgroup or more per CU with WAVES n tiles per workgroup), K in whole 256-k chunks
-        static const int ns_env = [] { const char* e = getenv("EVO_SK_NSPLIT"); return e ? atoi(e) : -1; }();  // measurement knob: 0 off, 2 / 4 force WAVES
-        // (measured, tools/bench_gemv.py: ahead of the k-split form from 17 rows up on the wide layers -- 2.2 -> 3.3+ TB/s at 32 rows, 1.4 -> 2.9 at 64;
-        //  behind it at <= 16 rows, where x is a small share of the L2 traffic and the k-split form's 11,000 short waves hide latency better)
-        const int waves_n = ns_env >= 0 ? ns_env : (K % 256 == 0 && N >= 8192 && M > 16 ? 4 : 0);
-        static const int nw_env = [] { const char* e = getenv("EVO_SK_WLDS"); return e ? atoi(e) : 1; }();    // measurement knob: 0 = fragment-shaped weight requests (skinny_n_kernel)
-        static const int nwm_env = [] { const char* e = getenv("EVO_SK_WLDS_MINM"); return e ? atoi(e) : 5; }();    // measurement knob: first row count on the contiguous form (measured ahead of the k-split form from 5 rows up on the wide layers)
-        static const int nww_env = [] { const char* e = getenv("EVO_SK_WLDS_WAVES"); return e ? atoi(e) : 0; }();   // measurement knob: 2 / 4 waves per workgroup (0 = auto)
-        // narrow layers (N < 8192: out_filter_dense / out_proj / l3 of a 7B block) with a workspace from the caller: four waves per workgroup AND a split
-        // over K across workgroups, partial sums through ws (see skinny_nw_kernel SPLITK)
-        static const int sk_env = [] { const char* e = getenv("EVO_SK_SPLITK"); return e ? atoi(e) : 1; }();      // measurement knob: 0 off
-        static const int skm_env = [] { const char* e = getenv("EVO_SK_SPLITK_MINM"); return e ? atoi(e) : 17; }();
-        // (K = 4,096 at <= 32 rows: four chunks per slice are too short a run -- 2.0 against 2.45 TB/s at 17 rows -- the k-split form keeps those)
-        if (ws && sk_env && nw_env && ns_env < 0 && K % 256 == 0 && K >= 1024 && N < 8192 && N >= 1024 && N % 64 == 0 && M >= skm_env && (K >= 8192 || M > 32)) {
-            int64_t slices = (256 + N / 64 - 1) / (N / 64);              // a workgroup per CU
-            if (slices > K / 256) slices = K / 256;
-            if (slices > 8) slices = 8;
-            if (slices >= 2 && ws_bytes >= slices * M * N * 4 && ((uintptr_t)ws & 15) == 0) {
-                const dim3 grid((unsigned)(N / 64), (unsigned)slices);
-#define EVO_SNK(MT) hipLaunchKernelGGL((skinny_nw_kernel<MT, 4, true>), grid, dim3(256), 0, s, (const uint4*)x, (const uint4*)w, (const uint16_t*)nullptr,       \
-                                       (const uint16_t*)nullptr, (uint16_t*)nullptr, (int)M, (int)N, (int)(K / 8), (float*)ws)
-                if (M <= 16) EVO_SNK(1); else if (M <= 32) EVO_SNK(2); else if (M <= 48) EVO_SNK(3); else EVO_SNK(4);
-#undef EVO_SNK
-                hipLaunchKernelGGL(skinny_reduce_kernel, dim3((unsigned)((M * N / 4 + 255) / 256)), dim3(256), 0, s, (const float*)ws, (const uint16_t*)bias,
-                                   (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)slices, (int)act);
-                return evo_launch_status();
+    // Three and four rows take the matrix cores' forms too where those are ahead of the dot2 form below (us at 4 rows: 4,096 x 4,096 9.5 -> 7.9, K = 11,008 19.7 -> 16.1,
+    // 16,384 x 4,096 26.2 -> 22.1; at 2 rows 8.0, 17.2 and 24.3 against the same).  Layers of 4,097 to 16,383 columns stay: the fused Hyena step of up to four rows sums its
+    // 12,288 columns in the dot2 form's order, and agrees with the unfused one bit for bit.
+    if ((M >= 5 || (M >= 3 && K % 128 == 0 && (N <= 4096 ? N >= 2048 && K >= 2048 : N >= 16384))) && K % 32 == 0) {
+        // (asynchronous loads of 16 bytes; an offset of 96 rows, 64 batch rows or 16 weight rows in 32 bits)
+        if (K % 128 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && K <= 0x9fffff) {
+            // wide layers
+            if (N > 4096) return ring_launch<0>(x, w, bias, residual, y, M, N, K, (int)act, 0, nullptr, 0, s);
+            // narrow layers, 16 rows a CU: parts of K where the batch rows would be read more often than the weights
+            if (ws && M >= 17 && (K >= 8192 || M > 32) && N % 64 == 0 && N >= 1024 && K >= 1024) {
+                int64_t parts = (256 + N / 64 - 1) / (N / 64);       // a workgroup per CU
+                if (parts > K / 256) parts = K / 256;
+                if (parts > 8) parts = 8;
+                if (parts >= 2 && ws_bytes >= parts * M * N * 4 && ((uintptr_t)ws & 15) == 0) {
+                    const int rc = ring_launch<2>(x, w, nullptr, nullptr, nullptr, M, N, K, 0, 0, (float*)ws, (int)parts, s);
+                    if (rc) return rc;
+                    hipLaunchKernelGGL(skinny_reduce_kernel, dim3((unsigned)((M * N / 4 + 255) / 256)), dim3(256), 0, s, (const float*)ws, (const uint16_t*)bias,
+                                       (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)parts, (int)act);
+                    return evo_launch_status();
+                }
             }
+            // (few workgroups, the unembedding's 512 columns: more waves in each -- us at 8 / 16 / 32 rows, K = 4,096: 6.0 / 6.8 / 8.4, with four 6.1 / 6.9 / 8.8)
+            if (N < 2048) {
+                if (M <= 8) return kw_launch<8, 8, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);
+                if (M <= 16) return kw_launch<16, 8, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);
+                if (M <= 32) return kw_launch<32, 4, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);
+            }
+            if (M <= 8) return kw_launch<8, 4, 128, 3>(x, w, bias, residual, y, M, N, K, (int)act, s);
+            if (M <= 16) return kw_launch<16, 4, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);
+            if (M <= 32) return kw_launch<32, 3, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);
         }
-        if (K % 256 == 0 && N >= 8192 && nw_env && M >= nwm_env && ns_env < 0) {
-            const int wv = nww_env ? nww_env : (N >= 256 * 64 ? 4 : (N >= 256 * 48 ? 3 : (N >= 256 * 32 ? 2 : 4)));   // a workgroup or more per CU where N allows
-#define EVO_SNW(MT, WV) hipLaunchKernelGGL((skinny_nw_kernel<MT, WV>), dim3((unsigned)((N + 16 * WV - 1) / (16 * WV))), dim3(64 * WV), 0, s, (const uint4*)x, \
-                                           (const uint4*)w, (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)(K / 8), (float*)nullptr, 0, (int)act)
-            if (wv == 4) { if (M <= 16) EVO_SNW(1, 4); else if (M <= 32) EVO_SNW(2, 4); else if (M <= 48) EVO_SNW(3, 4); else EVO_SNW(4, 4); }
-            else if (wv == 3) { if (M <= 16) EVO_SNW(1, 3); else if (M <= 32) EVO_SNW(2, 3); else if (M <= 48) EVO_SNW(3, 3); else EVO_SNW(4, 3); }
-            else { if (M <= 16) EVO_SNW(1, 2); else if (M <= 32) EVO_SNW(2, 2); else if (M <= 48) EVO_SNW(3, 2); else EVO_SNW(4, 2); }
-#undef EVO_SNW
-            return evo_launch_status();
-        }
-        if (waves_n && K % 256 == 0) {
-#define EVO_SN(MT, WV)                                                                                                     \
-            hipLaunchKernelGGL((skinny_n_kernel<MT, WV>), dim3((unsigned)((N + 16 * WV - 1) / (16 * WV))), dim3(64 * WV), 0, s, (const uint4*)x,  \
-                               (const uint4*)w, (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)(K / 8), (int)act)
-            if (waves_n == 4) { if (M <= 16) EVO_SN(1, 4); else if (M <= 32) EVO_SN(2, 4); else if (M <= 48) EVO_SN(3, 4); else EVO_SN(4, 4); }
-            else { if (M <= 16) EVO_SN(1, 2); else if (M <= 32) EVO_SN(2, 2); else if (M <= 48) EVO_SN(3, 2); else EVO_SN(4, 2); }
-#undef EVO_SN
-            return evo_launch_status();
-        }
+        // what is left (K not in whole chunks): two n tiles per workgroup (every x fragment feeds two weight fragments) where that still leaves a workgroup or more per CU
+        const dim3 block(512);
 #define EVO_SK(MT, NT)                                                                                                     \
         hipLaunchKernelGGL((skinny_mfma_kernel<MT, NT>), dim3((unsigned)((N + 16 * NT - 1) / (16 * NT))), block, 0, s, (const uint4*)x, (const uint4*)w, \
                            (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)(K / 8), (int)act)
-        if (nt == 2) { if (M <= 16) EVO_SK(1, 2); else if (M <= 32) EVO_SK(2, 2); else if (M <= 48) EVO_SK(3, 2); else EVO_SK(4, 2); }
+        if (N >= 8192 && M > 16) { if (M <= 32) EVO_SK(2, 2); else if (M <= 48) EVO_SK(3, 2); else EVO_SK(4, 2); }
         else { if (M <= 16) EVO_SK(1, 1); else if (M <= 32) EVO_SK(2, 1); else if (M <= 48) EVO_SK(3, 1); else EVO_SK(4, 1); }
 #undef EVO_SK
         return evo_launch_status();

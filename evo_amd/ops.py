@@ -416,9 +416,9 @@ class HipOps(MixerOps):
         M, K = x.shape
         N = w.shape[0]
         y = res if res is not None else (out if out is not None else torch.empty(M, N, dtype=torch.bfloat16, device=x.device))
-        # 17-64 rows on a narrow layer (N < 8192): a workspace for the partial sums of the split over K (csrc/gemv.hip skinny_nw_kernel SPLITK); up to
-        # 32 rows only where K is long
-        ws = torch.empty(8 * M * N, dtype=torch.float32, device=x.device) if (M > (16 if K >= 12288 else 32) and N < 8192 and K % 256 == 0 and N % 64 == 0) else None
+        # 17-64 rows on a narrow layer: a workspace for the partial sums of the split over K (csrc/gemv.hip skinny_ring_kernel, MODE 2); up to 32 rows only
+        # where K is long
+        ws = torch.empty(8 * M * N, dtype=torch.float32, device=x.device) if (M > (16 if K >= 8192 else 32) and 1024 <= N <= 4096 and K % 128 == 0 and N % 64 == 0) else None
         with self._t("gemv"):
             _check(self.lib.evo_linear_small_m_bf16(x.data_ptr(), w.data_ptr(), _ptr(b), _ptr(res), y.data_ptr(),
                                                     M, N, K, _ptr(ws), 0 if ws is None else ws.numel() * 4, act, _stream()), "evo_linear_small_m_bf16")
@@ -937,10 +937,10 @@ class HipOps(MixerOps):
 
     def hyena_decode_fused(self, x, norm_scale, eps, proj_w, proj_b, fir_state, iir_state, fir_w, fir_b, poles,
                            residues, dskip, n_heads: int) -> torch.Tensor:
-        """One decode token through pre-norm + projections + FIR/modal step + gate in ONE launch (M = batch <= 4, or <= 8 at D = 4096);
-        states are updated in place.  Falls back to the two kernels otherwise."""
+        """One decode token through pre-norm + projections + FIR/modal step + gate in ONE launch (M = batch <= 4, or <= 6 at D = 4096: 23.5 us
+        against 23 in three launches, 26.8 against 23 at 8); states are updated in place.  Falls back to the separate kernels otherwise."""
         M, D = x.shape
-        ok = ((1 <= M <= 4 or (M <= 8 and D == 4096)) and x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and proj_w.is_contiguous()
+        ok = ((1 <= M <= 4 or (M <= 6 and D == 4096)) and x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and proj_w.is_contiguous()
               and proj_w.dtype == torch.bfloat16 and norm_scale.dtype == torch.bfloat16 and proj_b is not None
               and fir_state.dtype == torch.bfloat16 and fir_state.is_contiguous() and fir_state.shape[0] == M
               and iir_state.dtype == torch.complex64 and iir_state.is_contiguous() and iir_state.shape[0] == M
@@ -1051,7 +1051,8 @@ class HipOps(MixerOps):
         """linear(rmsnorm(x) * scale, w, b).  Decode-sized batches (M <= 4) with a wide layer take ONE weight-streaming
         launch that rebuilds the normalised row on the fly; everything else is the two kernels."""
         M, K = x.shape
-        if ((1 <= M <= 4 or (M <= 8 and K == 4096)) and w.shape[0] > 4096 and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+        # (five rows and more: the norm's own launch and the matrix cores' form are ahead -- 20.5 -> 19.3 us at 5 rows and 12,288 x 4,096, 26.5 -> 19.3 at 8)
+        if (1 <= M <= 4 and w.shape[0] > 4096 and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
                 and scale.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous() and scale.is_contiguous()
                 and K % 8 == 0):
             y = torch.empty(M, w.shape[0], dtype=torch.bfloat16, device=x.device)
@@ -1109,10 +1110,10 @@ class HipOps(MixerOps):
             return a
         ok_mem = (x.is_cuda and x.dtype == torch.bfloat16 and wsrc.dtype == torch.bfloat16 and x.is_contiguous() and wsrc.is_contiguous()
                   and (norm_scale is None or (norm_scale.dtype == torch.bfloat16 and norm_scale.is_contiguous())))
-        # (5-8 rows WITH a norm keep the dot2 launch that norms for itself: one launch -- the BOS sliver of a scoring batch -- against norm pass + 44 us)
-        if self.gate_small_m_mfma and 5 <= M <= 64 and (M > 8 or norm_scale is None) and K % 256 == 0 and I % 32 == 0 and ok_mem:
-            # round 6: 5-64 rows on the MFMA weight-streaming form with the gate in its epilogue (csrc/gemv.hip skinny_nw_kernel GATE; 512-byte weight
-            # requests, x shared by the workgroup: 5.4 TB/s of weights at 8 rows where the dot2 launch runs 3.6); the norm as its own small pass in front
+        if (self.gate_small_m_mfma and (5 <= M <= 64 or (3 <= M <= 4 and I * K >= 1 << 24)) and K % 128 == 0 and I % 32 == 0 and ok_mem
+                and (x.data_ptr() | wsrc.data_ptr()) % 16 == 0):
+            # 3-64 rows on the MFMA weight-streaming form with the gate in its epilogue (csrc/gemv.hip skinny_ring_kernel); the norm as its own small pass in
+            # front (us at I = 11,008, K = 4,096, against the dot2 launch that norms for itself: 30.7 : 31.2 at 3 rows, 30.7 : 32.1 at 4, 30.7 : 45.0 at 8)
             if norm_scale is not None:
                 x = self.rmsnorm(x, None, norm_scale, eps)
             a = torch.empty(M, I, dtype=torch.bfloat16, device=x.device)
@@ -1141,6 +1142,8 @@ class HipOps(MixerOps):
             with self._t("gemm_gate"):
                 self._dense_layer(1 if grouped else 2, x, wsrc, a, M, 2 * I, K, act=code)
             return a
+        if grouped and 5 <= M <= 64 and K % 128 == 0:             # (a column's sums follow its place there: the rows back in their order)
+            wsrc, grouped = wsrc.view(I // 32, 2, 32, K).transpose(0, 1).reshape(2 * I, K), 0
         g = self.linear(x, wsrc, None)
         if grouped:                                               # columns come out as [32 of z1 | the same 32 of z2] per block: back to [z1 | z2]
             g = g.view(M, I // 32, 2, 32).permute(0, 2, 1, 3).reshape(M, 2 * I).contiguous()

@@ -251,10 +251,10 @@ int evo_attn_decode_bf16(const void* q, const void* k, const void* v, void* o,
  * replaces cuBLAS GEMV-shaped nn.Linear calls of the single-token forward   [REF evo/generation.py:151-155]
  * y [M, N] = x [M, K] . w [N, K]^T (+ bias [N]) (+ residual [M, N]);  1 <= M <= 64 (ABI 10; 16 before), K % 8 == 0 (K % 32 == 0
  * for M > 8), all bf16, fp32 accumulate, one rounding.  Weight-streaming (HBM-bound) forms: dot2 on the VALU up to
- * M = 4, v_mfma_f32_16x16x32_bf16 with the batch rows on the MFMA's N side from M = 5 -- one to four tiles of 16 rows per weight pass
- * (17-64 rows: the pooled decode step of 17-64 live streams); `residual` may alias `y`.  From 5 rows on layers with N >= 8192 and K % 256 == 0 the
- * weight is requested in whole 512-byte row pieces and the x rows of a 256-k chunk are shared by the workgroup's waves through LDS (csrc/gemv.hip
- * skinny_nw_kernel).  `ws` (ABI 10; may be NULL): a 16-byte aligned fp32 workspace of `ws_bytes` >= 8 M N 4 bytes lets the narrow layers (N < 8192) at
+ * M = 4 (M = 2 on layers that the other form is ahead on), v_mfma_f32_16x16x32_bf16 with the batch rows on the MFMA's N side from there -- one to four tiles
+ * of 16 rows per weight pass (17-64 rows: the pooled decode step of 17-64 live streams); `residual` may alias `y`.  With K % 128 == 0 and x, w 16-byte aligned
+ * weight and batch rows reach LDS by asynchronous loads of whole row pieces (csrc/gemv.hip skinny_ring_kernel, skinny_kw_kernel).
+ * `ws` (ABI 10; may be NULL): a 16-byte aligned fp32 workspace of `ws_bytes` >= 8 M N 4 bytes lets the narrow layers (N <= 4096) at
  * 17-64 rows split K over workgroups -- partial sums through ws, added in a fixed order by a second small launch; without it they run the k-split form.
  * act 3: the square of relu before the rounding (0: none). */
 int evo_linear_small_m_bf16(const void* x, const void* w, const void* bias, const void* residual, void* y,
@@ -355,9 +355,9 @@ int evo_norm_linear_small_m_bf16(const void* x, const void* scale, const void* w
  * I % 2 == 0, K % 8 == 0.  Both products are rounded to bf16 before the gate, as the unfused layers store them.
  * `grouped` != 0 (ABI 10): w12 is given in the row order of evo_mlp_gate_mfma_bf16's w12g -- blocks of 64 rows = 32 rows of W1 followed
  * by the same 32 rows of W2 (I % 32 == 0) -- so that ONE copy of l1 | l2 serves the prefill launch and the decode launches.
- * 5 <= M <= 64 (ABI 10; I % 32 == 0, K % 256 == 0, either layout): the MFMA weight-streaming form with the gate in its epilogue (csrc/gemv.hip
- * skinny_nw_kernel GATE) -- the pooled decode step of 5-64 live streams and the BOS sliver rows of a scoring batch; bit for bit
- * evo_linear_small_m_bf16 on w12 followed by evo_gelu_gate_bf16. */
+ * 5 <= M <= 64 (ABI 10; I % 32 == 0, K % 128 == 0, x and w12 16-byte aligned, either layout; large layers from M = 3): the MFMA weight-streaming form with the
+ * gate in its epilogue (csrc/gemv.hip skinny_ring_kernel, MODE 1) -- the pooled decode step of 5-64 live streams and the BOS sliver rows of a scoring batch; bit
+ * for bit evo_linear_small_m_bf16 on [W1; W2] followed by evo_gelu_gate_bf16 where 2 I >= 16,384 is no multiple of 4,096. */
 int evo_mlp_gate_small_m_bf16(const void* x, const void* w12, void* a, int64_t M, int64_t I, int64_t K, int64_t grouped, int64_t act,
                               void* stream);
 /* same with the post-mixer RMSNorm folded in: x is the residual row, `scale` [K] the norm weight (bit-identical to

@@ -1,0 +1,73 @@
+"""GPU parity of the weight-streaming layers whose operands reach LDS by asynchronous loads (csrc/gemv.hip skinny_ring_kernel).  Reference: the product of the bf16
+operands in fp64, bias, residual and activation, one rounding.  Tolerance: twice half a bf16 ulp (2^-8 of the result) and 1e-3 for the fp32 sums of up to
+12,288 products of variance 1 / K.  Rows behind the operands' ends hold NaN: nothing of them may reach a result."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _framed(rows, cols, g, scale=1.0):
+    """[rows, cols] bf16, 64 rows of NaN behind it in the same buffer."""
+    t = torch.full((rows + 64, cols), float("nan"), device=DEV, dtype=torch.bfloat16)
+    t[:rows] = (torch.randn(rows, cols, device=DEV, generator=g) * scale).bfloat16()
+    return t[:rows]
+
+
+# rows at the edges of 16, 32 and 64; columns that leave unequal and odd shares on 256 workgroups, every number of waves, two rounds; one chunk of 128 k, fewer
+# than stages, more than starts.  The last three: parts of K
+@pytest.mark.parametrize("M", [3, 5, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(4097, 128), (8191, 384), (8192, 4096), (12289, 256), (16386, 640), (22016, 4224), (24577, 384), (4096, 8192), (1024, 12288), (2048, 1152)])
+@pytest.mark.parametrize("extra", [False, True])
+def test_linear(M, N, K, extra):
+    from evo_amd.ops import default_ops
+    ops = default_ops()
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x, w = _framed(M, K, g), _framed(N, K, g, K ** -0.5)
+    want = x.double() @ w.double().T
+    if extra:
+        b, r = torch.randn(N, device=DEV, generator=g).bfloat16(), torch.randn(M + 1, N, device=DEV, generator=g).bfloat16()
+        keep, want = r.clone(), want + b.double()
+        got, want = ops._linear_small_m(x, w, b, r[:M]), want + keep[:M].double()
+        assert got.data_ptr() == r.data_ptr() and torch.equal(r[M], keep[M])
+    else:
+        got, want = ops._linear_small_m(x, w, None, None, act=3), want.relu().square()
+    assert bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + (1e-3 if extra else 4e-3)).all())        # (the square's slope is up to 8)
+
+
+@pytest.mark.parametrize("M", [3, 5, 16, 17, 33, 64])
+@pytest.mark.parametrize("I,K", [(32, 128), (96, 384), (2080, 256), (5504, 1152), (8224, 2176), (12320, 1408)])
+@pytest.mark.parametrize("grouped", [False, True])
+def test_gate(M, I, K, grouped):
+    from evo_amd.ops import default_ops
+    ops = default_ops()
+    g = torch.Generator(device=DEV).manual_seed(M + I + K)
+    x, w = _framed(M, K, g), _framed(2 * I, K, g, 1.5 * K ** -0.5)
+    packed = None
+    if grouped:
+        packed = _framed(2 * I, K, g)
+        packed.copy_(ops.pack_gate_weights(w.contiguous()))
+    for act in ("gelu", "silu"):
+        got = ops.mlp_gate(x, None if grouped else w, w12g=packed, act=act)
+        z = (x.double() @ w.double().T).float().bfloat16().double()
+        u, v = z[:, :I], z[:, I:]
+        want = (torch.nn.functional.gelu(u) if act == "gelu" else torch.nn.functional.silu(u)) * v
+        # (a product whose sum lies between two bf16 values may round to the other one: 2^-8 of it, and the gate's slope is at most 1.13)
+        assert got.shape == (M, I) and bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -6 + 2e-3 * want.abs().max()).all())
+        assert ((got.double() - want).norm() / want.norm()).item() < 4e-3
+
+
+def test_rows_off_16_bytes():
+    """Operands that the asynchronous loads can't take keep the other forms."""
+    from evo_amd.ops import default_ops
+    ops = default_ops()
+    g = torch.Generator(device=DEV).manual_seed(1)
+    M, N, K = 8, 8192, 512
+    x = torch.randn(M * K + 4, device=DEV, generator=g).bfloat16()[4:].view(M, K)
+    w = (torch.randn(N, K, device=DEV, generator=g) * K ** -0.5).bfloat16()
+    want = x.double() @ w.double().T
+    assert bool(((ops.linear(x, w).double() - want).abs() <= want.abs() * 2.0 ** -8 + 1e-3).all())
+    u, v = want.float().bfloat16().double().split(N // 2, 1)
+    gate = torch.nn.functional.gelu(u) * v
+    assert ((ops.mlp_gate(x, w).double() - gate).norm() / gate.norm()).item() < 4e-3
