@@ -6,6 +6,10 @@
 // and a CU holds about 64 KB in flight.  Hence large tiles (bytes per product fall with the tile's sides), parts of K where large tiles are too few
 // for the chip, and weight lines shared by neighbours on one XCD.  The MFMA order over k is the persistent kernel's, so an unsplit product is bit
 // for bit the same on every tile; parts of K are fp32 sums added in order by a second launch.
+// Below 256 rows the tiles of neighbouring weight rows start one k-step apart (`turn`) and go round: rows lie a power of two apart, so tiles that walk k in step
+// meet in the same L2 channels.  us at 65 / 161 rows, K = 4,096: 22,016 gated columns 47.1 / 56.8 -> 39.3 / 51.5, 12,288 columns 31.6 / 35.8 -> 26.7 / 33.3;
+// K = 11,008, 4,096 columns 30.8 / 34.6 -> 27.4 / 32.9.  (From 256 rows on, where it gives 3 to 6 %, the gated, the ungated and the blocked forms of a layer agree bit
+// for bit, whichever tiles they take.)
 // Inner loop: a ring of NS stages of 64 k, LDS-DMA pieces spread between the products of the first half step (a burst blocks the wave on the
 // vector-memory queue), the next half's fragments requested under the products of the current one, one barrier per stage.
 #include <math.h>
@@ -66,7 +70,7 @@ __device__ __forceinline__ void t_scale_bias(float (&v)[8], const GemmArgs& a, f
 __host__ __device__ __forceinline__ int64_t t_stat_rows(const GemmArgs& a) { return a.M; }
 
 template <int BM, int BN, int WGM, int WGN, int NS, int PER_CU, int MODE, bool XB, bool SPLIT>
-__global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_tile_kernel(GemmArgs a, int act, float* parts, int splits) {
+__global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_tile_kernel(GemmArgs a, int act, float* parts, int splits, int turn) {
     constexpr int NW = WGM * WGN, WM = BM / WGM, WN = BN / WGN, MT = WM / 16, NT = WN / 16;
     constexpr int PX = BM / 8 / NW, PW = BN / 8 / NW, P = PX + PW;      // DMA pieces (8 rows, 1 KiB) of a stage per wave
     constexpr int SLAB_X = BM * T_ROW, STAGE = (BM + BN) * T_ROW;
@@ -143,8 +147,10 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
 
     // piece `i` (of P) of stage `s` -> ring slot at byte `slot`; past the last stage the last one again, into a slot nobody reads (constant counts)
+    const int start = turn * (MODE == 3 ? tm : tn) % nk;
     auto fetch1 = [&](int s, uint32_t slot, int i) {
-        s = (s < nk ? s : nk - 1) + k0;
+        s = start + (s < nk ? s : nk - 1);
+        s = k0 + (s < nk ? s : s - nk);
         const uint32_t dst = lds0 + slot + wave * 1024;
         if (i < PX)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
@@ -471,13 +477,13 @@ static int tile_plan(int64_t M, int64_t N, int64_t K, int mode, bool stats, bool
 }
 
 template <int BM, int BN, int WGM, int WGN, int NS, int PER_CU, bool GATE>
-static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, float* ws, hipStream_t st) {
+static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, int turn, float* ws, hipStream_t st) {
     a.tiles_m = (int)((a.M + BM - 1) / BM);
     a.tiles_n = a.N / BN;
     a.group_m = 8;
     a.n_tiles = a.tiles_m * a.tiles_n * splits;
     const dim3 grid((unsigned)a.n_tiles), block(64 * WGM * WGN);
-#define T_GO(MODE, XB, SPLIT) hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, NS, PER_CU, MODE, XB, SPLIT>), grid, block, 0, st, a, act, ws, splits)
+#define T_GO(MODE, XB, SPLIT) hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, NS, PER_CU, MODE, XB, SPLIT>), grid, block, 0, st, a, act, ws, splits, turn)
     if (splits == 1) {
         if (mode == 3) T_GO(3, false, false);
         else if (mode == 1) { if constexpr (GATE) T_GO(1, false, false); else return -1; }
@@ -557,6 +563,7 @@ extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const voi
             n = dense_plan(mode, sumsq != nullptr, M, N, K, false, plan);
             break;
         }
+    const int turn = M < 256 ? 1 : 0;                            // (from 256 rows on the order of k is the persistent kernel's)
     int64_t m0 = 0;
     for (int i = 0; i < n; ++i) {
         const TilePlan& t = plan[i];
@@ -587,12 +594,12 @@ extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const voi
             const int tm = mode == 2 ? 1 : (int)mode;
             float* f = (float*)ws;
             hipStream_t st = (hipStream_t)stream;
-            if (t.kind == 0) rc = tile_launch<64, 64, 2, 2, 5, 2, false>(a, tm, (int)act, xblk != 0, t.splits, f, st);
-            else if (t.kind == 1) rc = tile_launch<128, 64, 4, 1, 3, 2, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
-            else if (t.kind == 2) rc = tile_launch<128, 128, 4, 2, 5, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
-            else if (t.kind == 3) rc = tile_launch<192, 128, 4, 2, 4, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
-            else if (t.kind == 4) rc = tile_launch<256, 128, 4, 2, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
-            else rc = tile_launch<128, 256, 2, 4, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
+            if (t.kind == 0) rc = tile_launch<64, 64, 2, 2, 5, 2, false>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
+            else if (t.kind == 1) rc = tile_launch<128, 64, 4, 1, 3, 2, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
+            else if (t.kind == 2) rc = tile_launch<128, 128, 4, 2, 5, 1, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
+            else if (t.kind == 3) rc = tile_launch<192, 128, 4, 2, 4, 1, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
+            else if (t.kind == 4) rc = tile_launch<256, 128, 4, 2, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
+            else rc = tile_launch<128, 256, 2, 4, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
         }
         if (rc != 0) return rc;
         m0 += t.rows;
