@@ -888,6 +888,29 @@ extern "C" int evo_attn_fwd_causal_bf16(const void* q, const void* k, const void
     return evo_launch_status();
 }
 
+extern "C" int evo_attn_fwd_packed_bf16(const void* q, const void* k, const void* v, void* o, int64_t H, int64_t rows, int64_t q_st, int64_t q_sh, int64_t k_st,
+                                        int64_t k_sh, int64_t v_st, int64_t v_sh, const int32_t* blocks, const int32_t* blocks_host, int64_t n_blocks,
+                                        const int32_t* valid, float softmax_scale, void* vt_ws, void* stream) {
+    if (!q || !k || !v || !o || !blocks || !blocks_host || !valid || !vt_ws || H <= 0 || H > 65535 || rows <= 0 || rows > 0x7fffff00 || n_blocks <= 0 || n_blocks > 0x7fffffff)
+        return -1;
+    if (attn_check_strides(0, q_st, q_sh, 0, k_st, k_sh, 0, v_st, v_sh) || ((uintptr_t)blocks & 15)) return -1;
+    for (int64_t i = 0; i < n_blocks; ++i) {
+        const int64_t first = blocks_host[4 * i], len = blocks_host[4 * i + 1], q0 = blocks_host[4 * i + 2];
+        if (first < 0 || first % 64 != 0 || len <= 0 || first + len > rows || q0 <= -256 || q0 + 256 > len) return -1;
+    }
+    AttnArgs a;
+    a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v; a.o = (uint16_t*)o;
+    a.Tq = rows; a.Tk = rows; a.q_pos0 = 0;
+    a.q_sb = 0; a.q_st = q_st; a.q_sh = q_sh; a.k_sb = 0; a.k_st = k_st; a.k_sh = k_sh; a.v_sb = 0; a.v_st = v_st; a.v_sh = v_sh;
+    a.H = (int)H;
+    a.prescaled = softmax_scale <= 0.f ? 1 : 0;
+    a.scale_log2 = a.prescaled ? 1.0f : softmax_scale * 1.4426950408889634f;
+    a.dyn_pos = nullptr; a.part_o = nullptr; a.part_ml = nullptr; a.n_splits = 1;
+    a.n_qblocks = (int)n_blocks;
+    a.blocks = (const int4*)blocks;
+    return evo_attn_w64_packed_launch(a, valid, vt_ws, stream);
+}
+
 extern "C" int evo_attn_decode_bf16(const void* q, const void* k, const void* v, void* o, int64_t B, int64_t H,
                                     int64_t Tk, int64_t q_sb, int64_t q_sh, int64_t k_sb, int64_t k_st,
                                     int64_t k_sh, int64_t v_sb, int64_t v_st, int64_t v_sh, const int64_t* dyn_pos,

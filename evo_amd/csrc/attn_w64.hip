@@ -196,7 +196,7 @@ __device__ __forceinline__ void w_static_for(F&& f) { w_static_for_impl(f, std::
 // tile may also move it down): P = 2^s up to 2^64, l <= 2^81, |O| <= 2^91 at T = 131,073 -- fp32 / bf16 carry the exponent, every rounding is
 // relative.  While no row of the wave has moved nothing is subtracted at all; once one has (wave-uniform `any_nm`) the tile's scores get
 // their row's offset in a burst between the two phases, like the masking of a diagonal tile.
-template <bool PRE>
+template <bool PRE, bool PACKED = false>
 __global__ __launch_bounds__(256, 1) void attn_fwd_w64_kernel(AttnArgs a) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[W_LDS];
 
@@ -207,12 +207,21 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_w64_kernel(AttnArgs a) {
     const int l31 = lane & 31;
     const int np = wave == 0 ? 9 : 8;                                   // DMA pieces of this wave per trip (17 K + 16 V over 4 waves)
 
-    const int64_t Tk_ = a.Tk, q_pos0_ = a.q_pos0;
+    int64_t Tk_ = a.Tk, q_pos0_ = a.q_pos0, q0, vt_col = 0;
     int qblk, head, bat;
     attn_block_map(a, qblk, head, bat);
-    const int64_t q0 = (int64_t)qblk * W_QB - a.q_pad;                  // block 0 starts q_pad rows before the range (those rows: clamped, not stored)
     const uint16_t* qp = a.q + bat * a.q_sb + head * a.q_sh;
     const unsigned char* kp = (const unsigned char*)(a.k + bat * a.k_sb + head * a.k_sh);
+    int64_t out_row0 = (int64_t)bat * a.Tq;
+    if constexpr (PACKED) {                                             // (the host lists the longest blocks last: the map walks from the end)
+        const int4 e = a.blocks[qblk];
+        qp += e.x * a.q_st;
+        kp += e.x * a.k_st * 2;
+        Tk_ = e.y;
+        q_pos0_ = 0;
+        q0 = e.z;
+        vt_col = out_row0 = e.x;
+    } else q0 = (int64_t)qblk * W_QB - a.q_pad;                         // block 0 starts q_pad rows before the range (those rows: clamped, not stored)
     const int64_t kst_b = a.k_st * 2;
 
     // ---- this lane's two query rows (column l31 of the wave's two 32-row blocks) ---------------------------------------------------
@@ -257,7 +266,7 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_w64_kernel(AttnArgs a) {
         dv_off = (uint32_t)r * (uint32_t)vt_row_b + (uint32_t)(((lane & 7) ^ f) << 4);
     }
     const uint32_t dv_soff = (uint32_t)(8 * vt_row_b);                 // per V^T piece: 8 rows
-    const unsigned char* vtp = (const unsigned char*)(a.vt + ((int64_t)bat * a.H + head) * DH * a.vt_row);
+    const unsigned char* vtp = (const unsigned char*)(a.vt + ((int64_t)bat * a.H + head) * DH * a.vt_row + vt_col);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
     // Buffer descriptors of one tile: base = its first row, num_records = bytes up to the end of the last VALID key (0 past the end):
     // the hardware bounds check returns zeros beyond -- no clamping, every trip issues the same instructions.  Branch-free scalar code:
@@ -275,7 +284,7 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_w64_kernel(AttnArgs a) {
         return d;
     };
     // V^T tile: base = column 64 tile of the head's plane, rows vt_row_b apart; the plane is padded to whole tiles
-    const int n_vt = (int)(a.vt_row / KB);
+    const int n_vt = PACKED ? (int)((Tk_ + KB - 1) / KB) : (int)(a.vt_row / KB);
     auto vt_srd = [&](int tile) __attribute__((always_inline)) {
         const uint64_t a64 = (uint64_t)vtp + (uint64_t)(uint32_t)tile * (uint64_t)(KB * 2);
         w_srd_t d;
@@ -765,7 +774,7 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_w64_kernel(AttnArgs a) {
 #endif
         const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
         const bool ok = x == 0 ? row_ok0 : row_ok1;
-        uint16_t* orow = a.o + ((int64_t)(bat * a.Tq + (x == 0 ? orow_first : orow_second)) * a.H + head) * DH;
+        uint16_t* orow = a.o + ((out_row0 + (x == 0 ? orow_first : orow_second)) * a.H + head) * DH;
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt) {
             const f32x16_t ov = oacc[x][dt];
@@ -799,11 +808,12 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_w64_kernel(AttnArgs a) {
 // (64-key tile, head, batch row).  Whole 256-byte rows in (16 lanes each), whole 128-byte row pieces out (8 lanes each); the tile
 // turns in LDS ([64 keys][130] halves: both sides conflict-free).  2 bytes moved per byte of V.
 __global__ __launch_bounds__(256) void attn_vt_kernel(const uint16_t* __restrict__ v, uint16_t* __restrict__ vt, int64_t Tk, int64_t v_sb,
-                                                      int64_t v_st, int64_t v_sh, int64_t vt_row, int H) {
+                                                      int64_t v_st, int64_t v_sh, int64_t vt_row, int H, const int32_t* __restrict__ valid) {
     __shared__ uint16_t tile[KB][DH + 2];
     const int tid = threadIdx.x, head = blockIdx.y, bat = blockIdx.z;
     const int64_t k0 = (int64_t)blockIdx.x * KB;
     const uint16_t* vp = v + bat * v_sb + head * v_sh;
+    if (valid) Tk = k0 + valid[blockIdx.x];                      // (unequal sequences behind each other, each from a multiple of 64 on: the rows between read as zero)
 #pragma unroll
     for (int ps = 0; ps < 4; ++ps) {
         const int key = (tid >> 4) + 16 * ps, ch = tid & 15;
@@ -835,8 +845,25 @@ int evo_attn_w64_launch(AttnArgs a, int64_t B, void* vt_ws, void* stream) {
     const int64_t n_wg = (int64_t)a.n_qblocks * a.nbh;
     if (n_wg > 0x7fffffff || a.vt_row / KB > 0x7fffffff || DH * a.vt_row * 2 > 0xffffffffll) return -1;
     hipLaunchKernelGGL(attn_vt_kernel, dim3((unsigned)(a.vt_row / KB), (unsigned)a.H, (unsigned)B), dim3(256), 0, (hipStream_t)stream,
-                       a.v, (uint16_t*)vt_ws, a.Tk, a.v_sb, a.v_st, a.v_sh, a.vt_row, a.H);
+                       a.v, (uint16_t*)vt_ws, a.Tk, a.v_sb, a.v_st, a.v_sh, a.vt_row, a.H, (const int32_t*)nullptr);
     if (a.prescaled) hipLaunchKernelGGL(attn_fwd_w64_kernel<true>, dim3((unsigned)n_wg), dim3(256), 0, (hipStream_t)stream, a);
     else hipLaunchKernelGGL(attn_fwd_w64_kernel<false>, dim3((unsigned)n_wg), dim3(256), 0, (hipStream_t)stream, a);
+    return evo_launch_status();
+}
+
+// Unequal sequences behind each other, all their query blocks in one launch (evo_attn_fwd_packed_bf16 in csrc/attn.hip has checked the blocks): a launch per
+// sequence of a few hundred rows has 32 heads x 1 to 5 blocks for 256 CUs and lasts as long as its longest block.  16 sequences of 220 to 1,100 rows, 32 heads:
+// 16 x (40 + 6.5) us -> 245 + 37 us (the longest blocks, 1,100 keys, are a third of it).
+int evo_attn_w64_packed_launch(AttnArgs a, const int32_t* valid, void* vt_ws, void* stream) {
+    a.nbh = a.H;
+    a.q_pad = 0;
+    a.vt = (const uint16_t*)vt_ws;
+    a.vt_row = (a.Tk + KB - 1) / KB * KB;
+    const int64_t n_wg = (int64_t)a.n_qblocks * a.H;
+    if (n_wg > 0x7fffffff || DH * a.vt_row * 2 > 0xffffffffll) return -1;
+    hipLaunchKernelGGL(attn_vt_kernel, dim3((unsigned)(a.vt_row / KB), (unsigned)a.H, 1), dim3(256), 0, (hipStream_t)stream, a.v, (uint16_t*)vt_ws, a.Tk, a.v_sb, a.v_st,
+                       a.v_sh, a.vt_row, a.H, valid);
+    if (a.prescaled) hipLaunchKernelGGL((attn_fwd_w64_kernel<true, true>), dim3((unsigned)n_wg), dim3(256), 0, (hipStream_t)stream, a);
+    else hipLaunchKernelGGL((attn_fwd_w64_kernel<false, true>), dim3((unsigned)n_wg), dim3(256), 0, (hipStream_t)stream, a);
     return evo_launch_status();
 }

@@ -172,13 +172,18 @@ class LayeredDecoder(DecodeGraphMixin, nn.Module):
             layer.mix.store(ipd)[i] = t
         return ipd
 
-    def copy_row(self, dst: dict, dst_row: int, src: dict, src_row: int, n_tokens: int) -> None:
-        """One sequence's state after `n_tokens` tokens from one set of rows to another."""
+    def row_pieces(self, dst: dict, dst_row: int, src: dict, src_row: int, n_tokens: int):
+        """(to, from) for each layer's state of one sequence after `n_tokens` tokens in two sets of rows."""
+        out = []
         for i, layer in enumerate(self.layers):
             d, s = layer.mix.store(dst)[i][dst_row], layer.mix.store(src)[i][src_row]
-            if layer.mix.grows:
-                d, s = d[:n_tokens], s[:n_tokens]
-            d.copy_(s)
+            out.append((d[:n_tokens], s[:n_tokens]) if layer.mix.grows else (d, s))
+        return out
+
+    def copy_row(self, dst: dict, dst_row: int, src: dict, src_row: int, n_tokens: int) -> None:
+        """One sequence's state after `n_tokens` tokens from one set of rows to another."""
+        for to, fro in self.row_pieces(dst, dst_row, src, src_row, n_tokens):
+            to.copy_(fro)
 
     def _room(self, ipd) -> int:
         """Positions the records hold."""

@@ -50,6 +50,9 @@ _SIGNATURES = {
     "evo_mlp_gate_mfma_nf_bf16": ([_PTR] * 4 + [_I64] * 3 + [_PTR], _c.c_int),
     "evo_put_tokens": ([_PTR, _I64, _PTR, _PTR, _I64, _PTR], _c.c_int),
     "evo_advance_positions": ([_PTR, _I64, _I64, _PTR], _c.c_int),
+    "evo_copy_rows": ([_PTR, _I64, _PTR], _c.c_int),
+    "evo_hyena_ct_packed": ([_PTR] * 9 + [_I64] * 5 + [_PTR], _c.c_int),
+    "evo_attn_fwd_packed_bf16": ([_PTR] * 4 + [_I64] * 8 + [_PTR] * 2 + [_I64, _PTR, _F32, _PTR, _PTR], _c.c_int),
     "evo_dense_ws": ([_I64] * 5, _c.c_int),
     "evo_dense_plan": ([_I64] * 5 + [_PTR], _c.c_int),
     "evo_dense_bf16": ([_I64] * 3 + [_PTR] * 7 + [_I64] * 8 + [_PTR, _I64, _PTR], _c.c_int),
@@ -94,7 +97,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 15         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 16         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):
@@ -483,6 +486,32 @@ class HipOps(MixerOps):
         self._need(pos, torch.int64, "advance_positions pos")
         _check(self.lib.evo_advance_positions(pos.data_ptr(), pos.numel(), int(last), _stream()), "evo_advance_positions")
 
+    def copy_rows(self, pairs) -> None:
+        """dst.copy_(src) for each pair of tensors of one shape and type, many to a launch.  Pieces that are not whole rows of 16 bytes are copied by torch."""
+        pieces = []
+        for dst, src in pairs:
+            if dst.shape != src.shape:
+                raise RuntimeError(f"copy_rows: {tuple(src.shape)} into {tuple(dst.shape)}")
+            if dst.numel() == 0:
+                continue
+            q = None
+            if (dst.is_cuda and src.is_cuda and dst.device == src.device and dst.device.index == torch.cuda.current_device() and dst.dtype == src.dtype
+                    and not dst.is_conj() and not src.is_conj() and not dst.is_neg() and not src.is_neg()):
+                n, e = dst.numel() * dst.element_size(), dst.element_size()
+                if dst.is_contiguous() and src.is_contiguous():
+                    q = [dst.data_ptr(), src.data_ptr(), 1, n, 0, 0]
+                elif dst.dim() > 1 and dst[0].is_contiguous() and src[0].is_contiguous():
+                    q = [dst.data_ptr(), src.data_ptr(), dst.shape[0], n // dst.shape[0], dst.stride(0) * e, src.stride(0) * e]
+                    if dst.shape[0] > 1 and min(q[4:]) < q[3]:
+                        q = None
+            if q is None or any(v % 16 for v in q[:2] + q[3:]):
+                dst.copy_(src)
+            else:
+                pieces += q
+        if pieces:
+            arr = (_c.c_int64 * len(pieces))(*pieces)
+            _check(self.lib.evo_copy_rows(_c.cast(arr, _PTR), len(pieces) // 6, _stream()), "evo_copy_rows")
+
     def rmsnorm(self, x: torch.Tensor, bias: Optional[torch.Tensor], scale: torch.Tensor, eps: float) -> torch.Tensor:
         """out = scale * x / (rms(x) + eps); with `bias`, x is first updated in place (x += bias)."""
         self._need(x, torch.bfloat16, "rmsnorm x")
@@ -681,6 +710,25 @@ class HipOps(MixerOps):
             return torch.view_as_complex(s_fin)
         self.last_hyena_io = {"mfma": B * T_run * 3 * D * 2 + B * T_run * D * 2}
         return (y, torch.view_as_complex(s_fin)) if want_state else y
+
+    def hyena_ct_packed(self, zt, fir_w, fir_b, table, n_heads, seqs, seqs_host, poles, y_blk, s_out) -> None:
+        """The operator on unequal sequences behind each other in z^T (hyena_ct's `at`, all of them in one launch): seqs [n, 2] int32 = (position of the first
+        token = its row in y_blk, tokens), on the device and on the host; their end states to s_out [n, D, 8] complex64."""
+        self._need(zt, torch.bfloat16, "hyena z^T")
+        self._need(y_blk, torch.bfloat16, "hyena y (blocked)")
+        self._need(poles, torch.float32, "hyena poles")
+        for t, nm in ((fir_w, "fir_w"), (fir_b, "fir_b")):
+            self._need(t, torch.bfloat16, "hyena " + nm)
+        D, n = zt.shape[1] // 3, seqs.shape[0]
+        assert zt.dim() == 3 and zt.shape[1:] == (3 * D, 256) and tuple(y_blk.shape[1:]) == (D // 16, self.YBLK, 16) and tuple(poles.shape) == (D, 8, 2)
+        assert table.dtype == torch.int32 and tuple(table.shape) == (D, 52, 64) and table.is_contiguous() and table.is_cuda
+        assert s_out.dtype == torch.complex64 and tuple(s_out.shape) == (n, D, 8) and s_out.is_contiguous() and s_out.device == zt.device
+        for t, dev in ((seqs, zt.device), (seqs_host, torch.device("cpu"))):
+            assert t.dtype == torch.int32 and tuple(t.shape) == (n, 2) and t.is_contiguous() and t.device == dev
+        with self._t("hyena_mfma"):
+            _check(self.lib.evo_hyena_ct_packed(zt.data_ptr(), fir_w.data_ptr(), fir_b.data_ptr(), table.data_ptr(), y_blk.data_ptr(), torch.view_as_real(s_out).data_ptr(),
+                                                poles.data_ptr(), seqs.data_ptr(), seqs_host.data_ptr(), n, D, n_heads, zt.shape[0] * 256, y_blk.shape[0] * self.YBLK,
+                                                _stream()), "evo_hyena_ct_packed")
 
     def hyena_prefill(self, z: torch.Tensor, fir_w: torch.Tensor, fir_b: torch.Tensor, poles: torch.Tensor,
                       residues: torch.Tensor, dskip: torch.Tensor, n_heads: int,
@@ -1012,6 +1060,38 @@ class HipOps(MixerOps):
                 q.stride(0), q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2),
                 v.stride(0), v.stride(1), v.stride(2), 0.0 if prescaled else 1.0 / math.sqrt(hd), _ptr(vt), _stream()), "evo_attn_fwd_causal_bf16")
         return o
+
+    ATTN_QB = 256                # queries of a block of attention_packed (csrc/attn_w64.hip W_QB)
+
+    @staticmethod
+    def packed_blocks(first, lens, rows: int):
+        """What attention_packed wants of sequences of `lens` tokens from row `first` (multiples of 64) of `rows` rows on -> (query blocks [n, 4] int32: first row,
+        length, first query, 0, in the order of their work; [ceil(rows / 64)] int32: the rows of every 64 that belong to a sequence), on the host."""
+        QB = HipOps.ATTN_QB
+        blocks = sorted((q0, f, m) for f, m in zip(first, lens) for q0 in range(m - (m + QB - 1) // QB * QB, m, QB))
+        valid = [0] * ((rows + 63) // 64)
+        for f, m in zip(first, lens):
+            for i in range((m + 63) // 64):
+                valid[f // 64 + i] = min(64, m - 64 * i)
+        return torch.tensor([[f, m, q0, 0] for q0, f, m in blocks], dtype=torch.int32), torch.tensor(valid, dtype=torch.int32)
+
+    def attention_packed(self, q, k, v, blocks, blocks_host, valid, out: torch.Tensor, prescaled: bool = False) -> None:
+        """Causal attention of unequal sequences behind each other, every one among its own rows; q, k, v [rows, H, 128] (strided views), out [rows, H * 128]; blocks, valid:
+        packed_blocks, on the device (and the blocks on the host).  Rows between the sequences stay as they are in `out`."""
+        for t, nm in ((q, "q"), (k, "k"), (v, "v")):
+            if not t.is_cuda or t.dtype != torch.bfloat16 or t.stride(-1) != 1:
+                raise RuntimeError(f"attention {nm}: need a ROCm bf16 tensor with a dense last dim")
+        M, H, hd = q.shape
+        self._need(out, torch.bfloat16, "attention out")
+        assert hd == 128 and k.shape == q.shape == v.shape and tuple(out.shape) == (M, H * hd)
+        for t, dev in ((blocks, q.device), (blocks_host, torch.device("cpu"))):
+            assert t.dtype == torch.int32 and t.dim() == 2 and t.shape[1] == 4 and t.is_contiguous() and t.device == dev and t.shape == blocks.shape
+        assert valid.dtype == torch.int32 and valid.is_contiguous() and valid.device == q.device and valid.numel() == (M + 63) // 64
+        vt = torch.empty(H, hd, (M + 63) // 64 * 64, dtype=torch.bfloat16, device=q.device)
+        with self._t("attn_fwd"):
+            _check(self.lib.evo_attn_fwd_packed_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), H, M, q.stride(0), q.stride(1), k.stride(0), k.stride(1),
+                                                     v.stride(0), v.stride(1), blocks.data_ptr(), blocks_host.data_ptr(), blocks.shape[0], valid.data_ptr(),
+                                                     0.0 if prescaled else 1.0 / math.sqrt(hd), vt.data_ptr(), _stream()), "evo_attn_fwd_packed_bf16")
 
     def attention_decode(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                          pos: Optional[torch.Tensor] = None, n_splits: Optional[int] = None, prescaled: bool = False) -> torch.Tensor:

@@ -76,14 +76,34 @@ class DecodePool:
 
     def install(self, prefilled, n_tokens: int, reserve: int = 1) -> int:
         """Takes a free slot for a prefilled sequence of `n_tokens` tokens (one more slot if none is free) and returns it."""
-        need = n_tokens + reserve
-        self._allocate(max(need, self.capacity), len(self.length) + 1)
-        slot = self.free.pop(0)
-        _, ipd, row = prefilled
+        return self._install([prefilled], [n_tokens], reserve)[0]
+
+    def _install(self, prefilled, n_tokens: Sequence[int], reserve: int) -> List[int]:
+        """Slots for several prefilled sequences; their states move in one launch where the ops have one for it."""
+        slots, pieces, ops = [], [], self.model.ops
+        for n in n_tokens:
+            self._allocate(max(n + reserve, self.capacity), len(self.length) + 1)
+            slots.append(self.free.pop(0))
+            self.length[slots[-1]] = n
         with torch.inference_mode():
-            self.model.copy_row(self.ipd, slot, ipd, row, n_tokens)
-        self.pos[slot] = self.length[slot] = n_tokens                 # where the slot's next token sits
-        return slot
+            for (_, ipd, row), slot, n in zip(prefilled, slots, n_tokens):
+                if hasattr(ops, "copy_rows") and hasattr(self.model, "row_pieces"):
+                    pieces += self.model.row_pieces(self.ipd, slot, ipd, row, n)
+                else:
+                    self.model.copy_row(self.ipd, slot, ipd, row, n)
+            if pieces:
+                ops.copy_rows(pieces)
+        if slots:
+            self._put(self.pos, slots, n_tokens)                      # where the slots' next tokens sit
+        return slots
+
+    def _put(self, where: torch.Tensor, slots: Sequence[int], values) -> None:
+        """where[slot] = value for host integers: a launch without a copy from host memory where the ops have one."""
+        put = getattr(self.model.ops, "put_tokens", None)
+        if put is not None and where.is_cuda and 0 < len(slots) <= self.model.ops.MAX_PUT:
+            put(where, slots, list(values))
+        else:
+            where.view(-1)[torch.tensor(slots).to(self.device)] = torch.tensor(list(values), dtype=torch.int64).to(self.device)
 
     def admit(self, prompts: Sequence[torch.Tensor], want: Optional[List[List[int]]] = None, reserve: int = 1):
         """Starts sequences: one batch of prompts -> (slots, wanted logits f32 per prompt)."""
@@ -91,15 +111,12 @@ class DecodePool:
         if self.ipd is None or len(self.free) < len(prompts):
             self._allocate(max(max(p.numel() for p in prompts) + reserve, self.capacity), len(self.length) + len(prompts))
         got = self.prefill(prompts, want)
-        return [self.install(g, p.numel(), reserve) for g, p in zip(got, prompts)], [g[0] for g in got]
+        return self._install(got, [p.numel() for p in prompts], reserve), [g[0] for g in got]
 
     def advance(self, tokens: Dict[int, int]) -> torch.Tensor:
         """The next token of each given slot, in one pooled step -> logits [S, V] f32 (rows of the other slots mean nothing)."""
-        slots, put = list(tokens), getattr(self.model.ops, "put_tokens", None)
-        if put is not None and self.ids.is_cuda and 0 < len(slots) <= self.model.ops.MAX_PUT:
-            put(self.ids, slots, list(tokens.values()))
-        else:
-            self.ids[torch.tensor(slots).to(self.device), 0] = torch.tensor(list(tokens.values()), dtype=torch.int64).to(self.device)
+        slots = list(tokens)
+        self._put(self.ids, slots, tokens.values())
         return self._advance(slots)
 
     def _advance(self, slots: Sequence[int]) -> torch.Tensor:

@@ -875,14 +875,19 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
                 hy.state_dict[i][: prev.state_dict[i].shape[0]] = prev.state_dict[i]
         return ipd
 
+    def row_pieces(self, dst: dict, dst_row: int, src: dict, src_row: int, n_tokens: int):
+        """(to, from) for each of one sequence's caches (its first `n_tokens` positions) in two sets of rows."""
+        out = [(dst["mha"].key_value_memory_dict[i][dst_row, :n_tokens], src["mha"].key_value_memory_dict[i][src_row, :n_tokens]) for i in self.attn_layer_idxs]
+        for i in self.hyena_layer_idxs:
+            out.append((dst["hyena"].fir_state_dict[i][dst_row], src["hyena"].fir_state_dict[i][src_row]))
+            row = dst["hyena"].state_dict[i][dst_row]
+            out.append((row, src["hyena"].state_dict[i][src_row].reshape(row.shape)))
+        return out
+
     def copy_row(self, dst: dict, dst_row: int, src: dict, src_row: int, n_tokens: int) -> None:
         """One sequence's caches (its first `n_tokens` positions) from one set of rows to another."""
-        for i in self.attn_layer_idxs:
-            dst["mha"].key_value_memory_dict[i][dst_row, :n_tokens] = src["mha"].key_value_memory_dict[i][src_row, :n_tokens]
-        for i in self.hyena_layer_idxs:
-            dst["hyena"].fir_state_dict[i][dst_row] = src["hyena"].fir_state_dict[i][src_row]
-            row = dst["hyena"].state_dict[i][dst_row]
-            row.copy_(src["hyena"].state_dict[i][src_row].reshape(row.shape))
+        for to, fro in self.row_pieces(dst, dst_row, src, src_row, n_tokens):
+            to.copy_(fro)
 
     packs_prompts = True         # prefill_rows runs unequal prompts as one pass
     packed_rows = 64 * 1024      # rows of one such pass
@@ -893,7 +898,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         if not self._packed:
             self._pack()
         ops = self.ops
-        ok = (self.device.type == "cuda" and getattr(ops, "hyena_mfma", False) and getattr(ops, "hyena_ct_flag", False) and hasattr(ops, "hyena_ct")
+        ok = (self.device.type == "cuda" and getattr(ops, "hyena_mfma", False) and getattr(ops, "hyena_ct_flag", False) and hasattr(ops, "hyena_ct_packed") and getattr(ops, "attn_w64", True)
               and self.hidden_size == self.num_heads * 128 and ops.zt_shape_ok(1, self.packed_rows, 3 * self.hidden_size, self.hidden_size) and getattr(self, "block_taps", None) is None
               and all(isinstance(b, _AttentionBlock) or (b.projections.weight.is_contiguous() and b.projections.weight.dtype == torch.bfloat16
                                                          and self._table_ok(b)) for b in self.blocks))
@@ -911,8 +916,8 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
 
     def _prefill_packed(self, prompts: List[torch.Tensor]):
         """Prompts behind each other as ONE stream of rows, each from a multiple of 64 on (the rows between are token 0 and reach nobody: every
-        launch is row-independent or runs on one prompt's rows): the dense layers see all rows at once, the Hyena operator and the attention walk
-        the prompts one by one.  -> (final-norm rows, first row of every prompt, caches of every prompt, each of its own length)."""
+        launch is row-independent or keeps to one prompt's rows): the dense layers see all rows at once, the Hyena operator and the attention take
+        all prompts in one launch.  -> (final-norm rows, first row of every prompt, caches of every prompt, each of its own length)."""
         ops, D, H, hd, K1 = self.ops, self.hidden_size, self.num_heads, self.head_dim, self.short_filter_length - 1
         dev, lens = self.device, [p.numel() for p in prompts]
         first, M = [], 0
@@ -920,14 +925,19 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             first.append(M)
             M += (m + 63) // 64 * 64
         M = (M + 255) // 256 * 256
-        ids = torch.zeros(M, dtype=torch.int64)
-        pos = torch.zeros(M, dtype=torch.int64)
-        ends = torch.tensor([f + m - K1 + j for f, m in zip(first, lens) for j in range(K1)])
-        for f, m in zip(first, lens):
-            pos[f:f + m] = torch.arange(m)
-        ids, pos, ends = ids.to(dev), pos.to(dev), ends.to(dev)
-        for p, f, m in zip(prompts, first, lens):
-            ids[f:f + m] = p.reshape(-1).to(dev)
+        places = torch.zeros(M + K1 * len(lens), dtype=torch.int64)       # every row's position, the rows of every prompt's last K1 tokens
+        for n, (f, m) in enumerate(zip(first, lens)):
+            places[f:f + m] = torch.arange(m)
+            places[M + K1 * n:M + K1 * (n + 1)] = torch.arange(f + m - K1, f + m)
+        pos, ends = places.to(dev).split([M, K1 * len(lens)])
+        seqs_h = torch.tensor(list(zip(first, lens)), dtype=torch.int32)
+        blocks_h, valid = ops.packed_blocks(first, lens, M)
+        blocks, seqs, valid = torch.cat([blocks_h.view(-1), seqs_h.view(-1), valid]).to(dev).split([blocks_h.numel(), seqs_h.numel(), valid.numel()])
+        blocks, seqs = blocks.view(-1, 4), seqs.view(-1, 2)
+        none, parts = torch.zeros(512, dtype=torch.int64, device=dev), []
+        for p, f, end in zip(prompts, first, first[1:] + [M]):
+            parts += [p.reshape(-1).to(dev, torch.int64), none[:end - f - p.numel()]]
+        ids = torch.cat(parts)
         cos, sin = (t[pos] for t in self._rotary(0, max(lens), dev)) if self.attn_layer_idxs else (None, None)
         pre = bool(getattr(ops, "attn_prescale", False)) and hasattr(ops, "attn_q_scale")
         caches = [self.initialize_inference_params() for _ in lens]
@@ -947,10 +957,10 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
                 qkv = qkv.view(1, M, 3, H, hd)
                 ops.rope_(qkv, cos, sin, **({"q_scale": ops.attn_q_scale(hd)} if pre else {}))
                 y, bias, w = torch.zeros(M, D, dtype=qkv.dtype, device=dev), mha.out_proj.bias, mha.out_proj.weight
-                for n, (f, m) in enumerate(zip(first, lens)):
-                    z = qkv[:, f:f + m]
-                    caches[n]["mha"].key_value_memory_dict[i] = z[:, :, 1:3].contiguous()
-                    ops.attention(z[:, :, 0], z[:, :, 1], z[:, :, 2], 0, out=y[f:f + m].view(1, m, H, hd), **({"prescaled": True} if pre else {}))
+                for ipd, m in zip(caches, lens):
+                    ipd["mha"].key_value_memory_dict[i] = torch.empty(1, m, 2, H, hd, dtype=qkv.dtype, device=dev)
+                ops.copy_rows([(ipd["mha"].key_value_memory_dict[i][0], qkv[0, f:f + m, 1:3]) for ipd, f, m in zip(caches, first, lens)])
+                ops.attention_packed(qkv[0, :, 0], qkv[0, :, 1], qkv[0, :, 2], blocks, blocks_h, valid, y, **({"prescaled": True} if pre else {}))
             else:
                 f_, pb = blk.filter, None if blk.projections.bias is None else blk.projections.bias.data
                 if nf and rs is not None:
@@ -960,9 +970,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
                     zt = ops.linear_t(ops.rmsnorm(x, None, blk.pre_norm.scale, self.eps), blk.projections.weight.data, pb, 1, M)
                 table = self._mfma_table(blk)
                 state = torch.empty(len(lens), D, self.state_size, dtype=torch.complex64, device=dev)
-                for n, (f, m) in enumerate(zip(first, lens)):
-                    ops.hyena_ct(zt, 1, m, f_._fir_w, f_.short_filter_bias, table, H, want_state=True, poles=f_._poles, y_blk=yb, y_row0=f, at=f,
-                                 s_out=state[n:n + 1])
+                ops.hyena_ct_packed(zt, f_._fir_w, f_.short_filter_bias, table, H, seqs, seqs_h, f_._poles, yb, state)
                 fir = zt[ends // 256, :, ends % 256].view(len(lens), K1, 3 * D).transpose(1, 2).contiguous()
                 for n, ipd in enumerate(caches):
                     ipd["hyena"].state_dict[i], ipd["hyena"].fir_state_dict[i] = state[n:n + 1], fir[n:n + 1]

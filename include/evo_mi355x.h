@@ -56,14 +56,18 @@ extern "C" {
  *      kept first tokens and two maps; evo_sum_norm, evo_heads_* and evo_rglru_* added.
  *  13: evo_dense_bf16 and evo_dense_ws (any dense layer on the tiles its size asks for), evo_put_tokens and evo_advance_positions added.
  *  14: evo_linear_f32 and evo_linear_f32_ws (fp32 dense layers on the bf16 matrix cores) added.
- *  15: evo_dense_plan and evo_linear_f32_plan (the launches of a dense layer) added. */
-#define EVO_ABI_VERSION 15
+ *  15: evo_dense_plan and evo_linear_f32_plan (the launches of a dense layer) added.
+ *  16: evo_hyena_ct_packed and evo_attn_fwd_packed_bf16 (unequal sequences in one launch), evo_copy_rows added. */
+#define EVO_ABI_VERSION 16
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
  * evo_advance_positions: pos[i] = min(pos[i] + 1, last). */
 int evo_put_tokens(int64_t* ids, int64_t S, const int64_t* slots, const int64_t* tokens, int64_t n, void* stream);
 int evo_advance_positions(int64_t* pos, int64_t n, int64_t last, void* stream);
+/* n copies between device buffers that don't overlap, 64 to a launch: `pieces` (HOST) holds six values of each -- destination, source, rows, bytes per row (a multiple of
+ * 16), the destination's and the source's pitch in bytes (looked at with more rows than one); everything 16-byte aligned. */
+int evo_copy_rows(const int64_t* pieces, int64_t n, void* stream);
 
 /* ---- embedding gather ------------------------------------------------------------------------
  * replaces VocabParallelEmbedding.embed (ATen gather)    [REF evo/scoring.py:81; evo/models.py:136]
@@ -161,6 +165,11 @@ int evo_hyena_ct(const void* zt, const void* z_halo, const void* fir_w, const vo
                  const float* s0, float* s_out, const float* poles, int64_t B, int64_t T, int64_t D, int64_t n_heads,
                  int64_t zt_pitch, int64_t row_pitch, int64_t zt_row0, int64_t tail_T, int64_t tail_pos0, int64_t state_only,
                  int64_t y_blocked_rows, int64_t y_row0, int64_t y_row_pitch, void* stream);
+/* the same operator (outputs blocked, end states, no halo and no carry-in) on n unequal sequences behind each other in z^T, one launch: sequence i has
+ * seqs[2 i + 1] steps from position seqs[2 i] (a multiple of 8) on, its outputs are the same rows of y, its end state is s_out[i].  seqs [n][2] int32 on the
+ * device, seqs_host the same on the host (checked against zt_pitch and y_blocked_rows before the launch). */
+int evo_hyena_ct_packed(const void* zt, const void* fir_w, const void* fir_b, const void* table, void* y, float* s_out, const float* poles, const int32_t* seqs,
+                        const int32_t* seqs_host, int64_t n, int64_t D, int64_t n_heads, int64_t zt_pitch, int64_t y_blocked_rows, void* stream);
 
 /* The Hyena block's output projection on the blocked y of evo_hyena_ct               [REF stripedhyena/model.py ParallelGatedConvBlock:
  * out_filter_dense]:  y [M, N] = x . w^T (+ bias [N]) (+ residual [M, N], may alias y), x = [M / 128][K / 16][128][16] bf16.  The persistent dense
@@ -228,6 +237,14 @@ int evo_attn_fwd_causal_bf16(const void* q, const void* k, const void* v, void* 
                              int64_t k_sb, int64_t k_st, int64_t k_sh,
                              int64_t v_sb, int64_t v_st, int64_t v_sh,
                              float softmax_scale, void* vt_ws, void* stream);
+/* the same on unequal sequences behind each other in `rows` rows (strides as above without a batch), each from a multiple of 64 on, in one launch: blocks
+ * [n_blocks][4] int32 (16-byte aligned) are the query blocks of 256 rows -- first row and length of their sequence, their first query in it (the last block of a sequence
+ * ends with it, the first may begin before it: q0 > -256), one value unused --, the longest LAST (they run first); blocks_host the same on the host, checked before the launch;
+ * valid [ceil(rows / 64)] int32 on the device: how many of the 64 rows from a multiple on belong to a sequence.  Rows between the sequences are not written.
+ * vt_ws: H 128 (rows rounded up to 64) bf16. */
+int evo_attn_fwd_packed_bf16(const void* q, const void* k, const void* v, void* o, int64_t H, int64_t rows, int64_t q_st, int64_t q_sh, int64_t k_st, int64_t k_sh,
+                             int64_t v_st, int64_t v_sh, const int32_t* blocks, const int32_t* blocks_host, int64_t n_blocks, const int32_t* valid, float softmax_scale,
+                             void* vt_ws, void* stream);
 
 /* decode form (one query per sequence, Tq = 1): split-K over the key range ("flash-decoding") + combine.
  * replaces flash_attn_with_kvcache                           [REF evo/generation.py:109-110,138-155]
