@@ -74,8 +74,11 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
     constexpr int NW = WGM * WGN, WM = BM / WGM, WN = BN / WGN, MT = WM / 16, NT = WN / 16;
     constexpr int PX = BM / 8 / NW, PW = BN / 8 / NW, P = PX + PW;      // DMA pieces (8 rows, 1 KiB) of a stage per wave
     constexpr int SLAB_X = BM * T_ROW, STAGE = (BM + BN) * T_ROW;
-    static_assert(PX >= 1 && PW >= 1 && NS >= 2 && NT % 2 == 0, "whole pieces per wave; column pairs");
-    static_assert(MODE != 1 || SPLIT || WN % 64 == 0, "a wave holds both halves of its gated columns");
+    constexpr bool ODD = BN % 64 != 0;                           // 96 or 48 columns: column tiles as they are, the last tile of a launch may be ragged
+    static_assert(PX >= 1 && PW >= 1 && NS >= 2 && PX * NW * 8 == BM && PW * NW * 8 == BN, "whole pieces per wave");
+    static_assert(ODD || NT % 2 == 0, "column pairs");
+    static_assert(MODE != 1 || SPLIT || WN % 64 == 0 || (ODD && WN % 32 == 0), "a wave holds both halves of its gated columns");
+    static_assert(!ODD || (MODE <= 1 && !SPLIT && !XB), "the launches that take such tiles");
     constexpr bool STATS = MODE == 0 && !SPLIT && BN == 128;     // (a strip of the statistic is 128 columns)
     __shared__ __attribute__((aligned(16))) unsigned char smem[NS * STAGE];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -115,6 +118,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
     //      granules, meets no bank twice); the DMA's LDS side is lane-linear, so the lane that fills a slot fetches the granule that belongs there.
     //      W rows: LDS row 32 b + 16 t + 4 q + r holds W row 32 b + 8 q + 4 t + r, so that a lane's accumulators of a pair of column tiles are
     //      eight consecutive columns.  Rows behind the matrix read as zero (bounded descriptors).
+    //      ODD: LDS row 16 t + c holds column c of column tile t; gated, tiles 2 p and 2 p + 1 are the two halves of the gated columns 16 p .. 16 p + 15.
     uint32_t xoff[PX], woff[PW];
     const int swz = ((lane & 7) ^ (lane >> 3)) & 7;
 #pragma unroll
@@ -129,7 +133,13 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
     for (int i = 0; i < PW; ++i) {
         const int r = 8 * (wave + NW * i) + (lane >> 3);
         int wr = (r & ~31) + 8 * ((r >> 2) & 3) + 4 * ((r >> 4) & 1) + (r & 3);
-        if (MODE == 1 && a.w_rows) wr = (wr >> 6) * 32 + (wr & 31) + ((wr >> 5) & 1) * (a.N >> 1);     // [W1; W2] as it is: 32 rows of each in turn
+        if constexpr (ODD) {
+            wr = r;
+            if (MODE == 1) {
+                const int c = (r >> 5) * 16 + (r & 15), half = (r >> 4) & 1, g = ((n0 >> 1) & 31) + c;
+                wr = a.w_rows ? half * (a.N >> 1) + c : (g >> 5) * 64 + half * 32 + (g & 31);
+            }
+        } else if (MODE == 1 && a.w_rows) wr = (wr >> 6) * 32 + (wr & 31) + ((wr >> 5) & 1) * (a.N >> 1);     // [W1; W2] as it is: 32 rows of each in turn
         woff[i] = (uint32_t)wr * (uint32_t)kb + swz * 16u;
     }
     int64_t src = n0, w_rows = a.N;                              // first row of the "W" operand and how many there are
@@ -139,9 +149,10 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
     }
     const bool plain_gate = MODE == 1 && a.w_rows;
     if (plain_gate) src = n0 >> 1;
+    else if (ODD && MODE == 1) src = n0 >> 6 << 6;               // (whole groups of 32 rows of each half)
     const uint64_t xa = (uint64_t)a.x + (XB ? (m0 & ~(int64_t)127) : m0) * kb, wa = (uint64_t)a.w + src * kb;
     const int64_t x_left = a.M - (XB ? (m0 & ~(int64_t)127) : m0), x_most = XB ? 256 : BM, x_ok = x_left < x_most ? x_left : x_most;    // (blocked X: whole blocks, M % 128 == 0)
-    const int64_t w_ok = plain_gate || w_rows - src < BN ? w_rows - src : BN;
+    const int64_t w_ok = plain_gate || w_rows - src < BN || (ODD && MODE == 1) ? w_rows - src : BN;
     const t_u32x4 rx = {(uint32_t)xa, (uint32_t)(xa >> 32) & 0xffffu, (uint32_t)(x_ok * kb), 0x00020000u};
     const t_u32x4 rw = {(uint32_t)wa, (uint32_t)(wa >> 32) & 0xffffu, (uint32_t)(w_ok * kb), 0x00020000u};
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
@@ -252,6 +263,52 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
         return;
     }
 
+    if constexpr (ODD) {                                         // a lane's 4 values of a column tile t are its columns 4 lq .. + 3
+        const int gn = a.N >> 1;
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            const int64_t m = m0 + wm * WM + 16 * j + l15;
+            const bool ok = m < a.M;
+            const float f = a.rs && ok ? a.rs[m] : 1.f;
+            if constexpr (MODE == 1) {
+#pragma unroll
+                for (int p = 0; p < NT / 2; ++p) {
+                    const int c = (n0 + wn * WN) / 2 + 16 * p + 4 * lq;
+                    uint32_t o[2];
+#pragma unroll
+                    for (int e = 0; e < 4; e += 2) {
+                        float z1[2] = {acc[2 * p][j][e], acc[2 * p][j][e + 1]}, z2[2] = {acc[2 * p + 1][j][e], acc[2 * p + 1][j][e + 1]};
+                        if (a.rs) { z1[0] *= f; z1[1] *= f; z2[0] *= f; z2[1] *= f; }
+                        const uint32_t u1 = pack_bf2(z1[0], z1[1]), u2 = pack_bf2(z2[0], z2[1]);                // the dense layers' bf16 outputs
+                        const f32x2_t oo = act_gate2(f32x2_t{bf_lo(u1), bf_hi(u1)}, f32x2_t{bf_lo(u2), bf_hi(u2)}, act);
+                        o[e >> 1] = pack_bf2(oo[0], oo[1]);
+                    }
+                    if (ok && c < gn) *(uint2*)(a.y + m * gn + c) = make_uint2(o[0], o[1]);
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const int n = n0 + wn * WN + 16 * t + 4 * lq;
+                    if (!ok || n >= a.N) continue;
+                    float v[8] = {acc[t][j][0], acc[t][j][1], acc[t][j][2], acc[t][j][3], 0.f, 0.f, 0.f, 0.f};
+                    float b[4] = {0.f, 0.f, 0.f, 0.f};
+                    if (a.bias) {
+                        const uint2 q = *(const uint2*)(a.bias + n);
+                        b[0] = bf_lo(q.x); b[1] = bf_hi(q.x); b[2] = bf_lo(q.y); b[3] = bf_hi(q.y);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = a.rs ? fmaf(v[e], f, b[e]) : v[e] + b[e];
+                    if (a.res) {
+                        const uint2 q = *(const uint2*)(a.res + m * a.N + n);
+                        v[0] += bf_lo(q.x); v[1] += bf_hi(q.x); v[2] += bf_lo(q.y); v[3] += bf_hi(q.y);
+                    }
+                    if (act && n < a.act_cols) t_act(v, act);
+                    *(uint2*)(a.y + m * a.N + n) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));      // the one rounding
+                }
+            }
+        }
+        return;
+    }
     // ---- epilogue, straight from registers: a lane's 8 values of (row tile j, column pair b) are columns 32 b + 8 lq .. + 7 of row 16 j + l15
     if constexpr (MODE == 1) {
         const int gn = a.N >> 1;
@@ -415,7 +472,14 @@ __global__ __launch_bounds__(256) void gemm_parts_kernel(GemmArgs a, int act, co
 // kernel -> this choice): 4,096 columns 68 -> 16 / 187 -> 34 at 161 rows, 72 -> 28 / 188 -> 58 at 512, 74 -> 36 / 187 -> 95 at 1,024, 75 -> 57 / 193 ->
 // 147 at 2,048; 12,288 columns 76 -> 34 at 161 rows, 78 -> 58 at 512; 22,016 gated columns 82 -> 53 at 161.
 struct TileKind { int bm, bn; double step_us; };
-static const TileKind kinds[] = {{64, 64, 0.255}, {128, 64, 0.435}, {128, 128, 0.515}, {192, 128, 0.70}, {256, 128, 0.84}, {128, 256, 0.86}};
+static const TileKind kinds[] = {{64, 64, 0.255}, {128, 64, 0.435}, {128, 128, 0.515}, {192, 128, 0.70}, {256, 128, 0.84}, {128, 256, 0.86},
+                                 {96, 96, 0.50}, {192, 96, 0.667}, {96, 48, 0.35}};
+// The last three, below 256 rows and without parts, statistics or a transposed result: narrow enough that a layer of 12,288 to 24,576 columns is one round of
+// nearly all CUs.  us, before -> with them: 22,016 gated columns, K = 4,096 (172 tiles of 128 -> 230 of 96) 39.6 -> 37.7 at 65 rows, 42.2 -> 40.8 at 96, 48.0 -> 44.8
+// at 129, 51.7 -> 48.7 at 161, 53.6 -> 51.4 at 192; 12,288 columns (192 tiles of 64 -> 256 of 48) 27.2 -> 24.4 at 65, 29.8 -> 27.8 at 96; 11,264 columns 30.5 -> 23.5 and 33.1 -> 26.7.  Twelve waves for
+// 192 x 96 (six 49.8, four 56.7: a wave alone on its SIMD waits for its own fragments).  Not taken: 128 x 96 (43.4 - 45.1 at 97 - 128 rows, 42.4 - 46.6 with 128 x 128),
+// 256 x 96 (66.5 against 56.5 at 193) and 192 x 48 (35.7 against 34.2).
+#define T_ODD 6                              // first of them
 #define T_PERSISTENT 99
 
 struct TilePlan { int kind; int splits; double us; int64_t rows; };      // rows: how many of M it takes
@@ -443,8 +507,10 @@ static TilePlan tile_best(int64_t M, int64_t N, int64_t K, int mode, bool stats,
     for (int c = 0; c < (int)(sizeof(kinds) / sizeof(kinds[0])); ++c) {
         const int bm = mode == 3 ? kinds[c].bn : kinds[c].bm, bn = mode == 3 ? kinds[c].bm : kinds[c].bn;      // along the tokens, along the weight
         if ((mode == 1 && c == 0) || (mode != 3 && c == 5)) continue;
+        if (c >= T_ODD && (M >= 256 || mode == 3 || stats || (mode == 1) != (c < T_ODD + 2))) continue;
+        if (c == T_ODD + 2 && N / 48 < 0.9 * cus) continue;      // (10,240 columns, 214 tiles: 26.3 us at 96 rows, 25.9 without)
         const double tiles = (double)((M + bm - 1) / bm) * (double)((N + bn - 1) / bn);
-        for (int s = 1; s <= (splits_ok ? 8 : 1); ++s) {
+        for (int s = 1; s <= (splits_ok && c < T_ODD ? 8 : 1); ++s) {
             if (s == 1 && stats && bn != 128) continue;
             if (s > 1 && (tiles * s > 2 * cus || nk / s < 8 || (double)s * M * N * 4 > 256e6)) break;
             double us = ceil(tiles * s / cus) * (ceil(nk / s) * kinds[c].step_us + (mode == 1 && s == 1 ? 6.0 : 3.0));
@@ -479,7 +545,7 @@ static int tile_plan(int64_t M, int64_t N, int64_t K, int mode, bool stats, bool
 template <int BM, int BN, int WGM, int WGN, int NS, int PER_CU, bool GATE>
 static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, int turn, float* ws, hipStream_t st) {
     a.tiles_m = (int)((a.M + BM - 1) / BM);
-    a.tiles_n = a.N / BN;
+    a.tiles_n = (a.N + BN - 1) / BN;
     a.group_m = 8;
     a.n_tiles = a.tiles_m * a.tiles_n * splits;
     const dim3 grid((unsigned)a.n_tiles), block(64 * WGM * WGN);
@@ -501,6 +567,16 @@ static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, int
     if (mode == 3) hipLaunchKernelGGL(gemm_parts_kernel<3>, rgrid, rblock, 0, st, a, act, ws, splits);
     else if (mode == 1) hipLaunchKernelGGL(gemm_parts_kernel<1>, rgrid, rblock, 0, st, a, act, ws, splits);
     else hipLaunchKernelGGL(gemm_parts_kernel<0>, rgrid, rblock, 0, st, a, act, ws, splits);
+    return evo_launch_status();
+}
+
+template <int BM, int BN, int WGM, int WGN, int NS, int MODE>
+static int tile_launch_odd(GemmArgs a, int act, int turn, hipStream_t st) {
+    a.tiles_m = (int)((a.M + BM - 1) / BM);
+    a.tiles_n = (a.N + BN - 1) / BN;
+    a.group_m = 8;
+    a.n_tiles = a.tiles_m * a.tiles_n;
+    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, NS, 1, MODE, false, false>), dim3((unsigned)a.n_tiles), dim3(64 * WGM * WGN), 0, st, a, act, nullptr, 1, turn);
     return evo_launch_status();
 }
 
@@ -599,7 +675,11 @@ extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const voi
             else if (t.kind == 2) rc = tile_launch<128, 128, 4, 2, 5, 1, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
             else if (t.kind == 3) rc = tile_launch<192, 128, 4, 2, 4, 1, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
             else if (t.kind == 4) rc = tile_launch<256, 128, 4, 2, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
-            else rc = tile_launch<128, 256, 2, 4, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
+            else if (t.kind == 5) rc = tile_launch<128, 256, 2, 4, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
+            else if (xblk || tm > 1 || (tm == 1) != (t.kind < T_ODD + 2)) rc = -1;
+            else if (t.kind == T_ODD) rc = tile_launch_odd<96, 96, 2, 3, 6, 1>(a, (int)act, turn, st);
+            else if (t.kind == T_ODD + 1) rc = tile_launch_odd<192, 96, 4, 3, 4, 1>(a, (int)act, turn, st);
+            else rc = tile_launch_odd<96, 48, 3, 1, 8, 0>(a, (int)act, turn, st);
         }
         if (rc != 0) return rc;
         m0 += t.rows;

@@ -241,3 +241,45 @@ def test_transposed_last_tile_overhangs_the_weight(N, Mp):
     assert ops.lib.evo_linear_t_mfma_bf16(x.data_ptr(), w.data_ptr(), b.data_ptr(), want.data_ptr(), Mp, N, K, _stream()) == 0
     ops._dense_layer(3, x, w, got, Mp, N, K, b=b)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("M,N,K,tile", [(65, 12288, 4096, (96, 48)), (96, 12288, 256, (96, 48)), (67, 11264, 1088, (96, 48)), (65, 22016, 4096, (96, 96)),
+                                        (96, 20992, 512, (96, 96)), (129, 22016, 4096, (192, 96)), (161, 21760, 1088, (192, 96)), (192, 24576, 256, (192, 96))])
+def test_tiles_of_odd_widths(M, N, K, tile):
+    """Tiles of 96 and 48 columns: every epilogue, the last tile of a width that they do not divide, rows and columns behind the result untouched."""
+    from evo_amd.ops import _stream
+    import ctypes
+    ops = _ops()
+    gated = tile[1] == 96
+    out = (ctypes.c_int64 * 14)()
+    assert ops.lib.evo_dense_plan(int(gated), 0, M, N, K, ctypes.cast(out, ctypes.c_void_p)) == 1 and tuple(out[2:4]) == tile
+    g, x, w = _data(M, N, K, 7)
+    z = x.double() @ w.double().T
+    rs = torch.rand(M, device="cuda", generator=g) + 0.5
+    if gated:
+        for order in (1, 2):
+            wk = ops.pack_gate_weights(w) if order == 1 else w
+            for act, f in ((0, torch.nn.functional.gelu), (1, torch.nn.functional.silu)):
+                for scale in (None, rs) if act == 0 else (None,):
+                    y = torch.full((M + 3, N // 2), 7.0, device="cuda", dtype=torch.bfloat16)
+                    assert ops.lib.evo_dense_bf16(order, act, 0, x.data_ptr(), wk.data_ptr(), None, None, y.data_ptr(), None if scale is None else scale.data_ptr(), None, 0,
+                                                  M, N, K, 0, 0, 0, 0, None, 0, _stream()) == 0
+                    zz = (z if scale is None else z * scale.double()[:, None]).bfloat16().double()
+                    z1, z2 = zz[:, :N // 2], zz[:, N // 2:]
+                    want = f(z1) * z2
+                    err = (y[:M].double() - want).abs()
+                    assert bool((err <= want.abs() * 2.0 ** -7 + (z1.abs() + 0.2) * z2.abs() * 2.0 ** -7 + 1e-3).all()), err.max().item()      # (as test_gate)
+                    assert bool((y[M:] == 7).all())
+        return
+    b = torch.randn(N, device="cuda", generator=g).bfloat16()
+    r = torch.randn(M, N, device="cuda", generator=g).bfloat16()
+    for bias, res, scale, act in ((0, 0, 0, 0), (1, 1, 0, 0), (1, 0, 1, 0), (0, 0, 1, 0), (1, 0, 0, 3)):
+        y = torch.full((M + 3, N), 7.0, device="cuda", dtype=torch.bfloat16)
+        assert ops.lib.evo_dense_bf16(0, act, 0, x.data_ptr(), w.data_ptr(), b.data_ptr() if bias else None, r.data_ptr() if res else None, y.data_ptr(),
+                                      rs.data_ptr() if scale else None, None, 0, M, N, K, 256 if act else 0, 0, 0, 0, None, 0, _stream()) == 0
+        want = (z * rs.double()[:, None] if scale else z) + (b.double() if bias else 0) + (r.double() if res else 0)
+        if act:
+            want = torch.cat([want[:, :256].relu().square(), want[:, 256:]], 1)
+        err = (y[:M].double() - want).abs()
+        assert bool((err <= want.abs() * 2.0 ** -8 + (4e-3 if act else 1e-3)).all()), err.max().item()                          # (as test_plain, test_activation)
+        assert bool((y[M:] == 7).all())
