@@ -76,46 +76,45 @@ extern "C" int evo_latent_prep(void* q, int64_t ldq, void* c, void* kr, void* ca
 
 // ------------------------------------------------------------------------------------------------ decode: query side of the key map
 // out[b][h] = [W_uk,h^T q_n (R) | rotated q (dr) | zeros up to rs].  Workgroup: 64 V latent columns of one head, NB sequences; eight waves
-// share the dn rows of the map, a lane owns V adjacent columns.
+// share the dn rows of the map, a lane owns V adjacent columns.  Latency bounds it (4 MB of map at 32 heads of 128 x 512): a wave asks for its first 16 rows
+// before anything else, and columns are halved where that leaves fewer than 128 workgroups.
 template <typename T, int NB, int V>
 __global__ __launch_bounds__(512) void latent_absorb_kernel(const void* __restrict__ q_, int64_t ldq, const void* __restrict__ w_, void* __restrict__ out_,
                                                             int B, int H, int dn, int dr, int R, int rs) {
     extern __shared__ float sm[];                                // q parts [NB][dn], partial sums [8][NB][64 V]
+    constexpr int U = 16;                                        // rows of a wave in flight
     float* part = sm + NB * dn;
     const int h = blockIdx.y, b0 = blockIdx.z * NB, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nb = B - b0 < NB ? B - b0 : NB, dh = dn + dr;
+    const int r0 = blockIdx.x * 64 * V, r = r0 + lane * V;
+    const T* w = (const T*)w_ + (int64_t)h * dn * R + (r < R ? r : 0);       // (lanes behind the last column read the first ones and store nothing)
+    float f[U][V];
+    auto fetch = [&](int n) __attribute__((always_inline)) {     // rows n + 8 u; past the last one the last again, not used
+#pragma unroll
+        for (int u = 0; u < U; ++u) vec_io<T, V>::load(w + (int64_t)(n + 8 * u < dn ? n + 8 * u : dn - 1) * R, f[u]);
+    };
+    fetch(wave);                                                 // (no need of the queries: on their way behind each other)
 #pragma unroll
     for (int i = 0; i < NB; ++i)
         for (int n = tid; n < dn; n += 512) sm[i * dn + n] = i < nb ? ld1((const T*)q_ + (int64_t)(b0 + i) * ldq + (int64_t)h * dh + n) : 0.f;
     __syncthreads();
-    const int r0 = blockIdx.x * 64 * V, r = r0 + lane * V;
-    const T* w = (const T*)w_ + (int64_t)h * dn * R + r;
     float acc[NB][V];
 #pragma unroll
     for (int i = 0; i < NB; ++i)
 #pragma unroll
         for (int e = 0; e < V; ++e) acc[i][e] = 0.f;
-    if (r < R) {
-        int n = wave;
-        for (; n + 24 < dn; n += 32) {
-            float f[4][V];
+    for (int n = wave; n < dn; n += 8 * U) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) vec_io<T, V>::load(w + (int64_t)(n + 8 * u) * R, f[u]);
+        for (int u = 0; u < U; ++u) {
+            if (n + 8 * u >= dn) break;
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+            for (int i = 0; i < NB; ++i) {
+                const float q = sm[i * dn + n + 8 * u];
 #pragma unroll
-                for (int i = 0; i < NB; ++i)
-#pragma unroll
-                    for (int e = 0; e < V; ++e) acc[i][e] = fmaf(f[u][e], sm[i * dn + n + 8 * u], acc[i][e]);
+                for (int e = 0; e < V; ++e) acc[i][e] = fmaf(f[u][e], q, acc[i][e]);
+            }
         }
-        for (; n < dn; n += 8) {
-            float f[V];
-            vec_io<T, V>::load(w + (int64_t)n * R, f);
-#pragma unroll
-            for (int i = 0; i < NB; ++i)
-#pragma unroll
-                for (int e = 0; e < V; ++e) acc[i][e] = fmaf(f[e], sm[i * dn + n], acc[i][e]);
-        }
+        if (n + 8 * U < dn) fetch(n + 8 * U);
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) vec_io<float, V>::store(part + ((wave * NB + i) * 64 + lane) * V, acc[i]);
@@ -139,7 +138,9 @@ __global__ __launch_bounds__(512) void latent_absorb_kernel(const void* __restri
 extern "C" int evo_latent_absorb(const void* q, int64_t ldq, const void* wuk, void* out, int64_t B, int64_t H, int64_t dn, int64_t dr, int64_t R,
                                  int64_t rs, int64_t f32, void* stream) {
     if (!q || !wuk || !out || B <= 0 || H <= 0 || H > 65535 || dn <= 0 || dn > 4096 || dr < 0 || R <= 0 || rs < R + dr || ldq < H * (dn + dr)) return -1;
-    const int nb = B > 2 ? 4 : (int)B, v = R % 8 == 0 && ((uintptr_t)wuk & 15) == 0 ? 8 : 1;
+    const int nb = B > 2 ? 4 : (int)B;
+    int v = R % 8 == 0 && ((uintptr_t)wuk & 15) == 0 ? 8 : 1;
+    if (v == 8 && ((R + 511) / 512) * H * ((B + nb - 1) / nb) < 128) v = 4;
     const dim3 grid((unsigned)((R + 64 * v - 1) / (64 * v)), (unsigned)H, (unsigned)((B + nb - 1) / nb)), block(512);
     const size_t lds = (size_t)nb * (dn + 512 * v) * 4;          // (<= 128 KB)
     hipStream_t s = (hipStream_t)stream;
@@ -149,8 +150,8 @@ extern "C" int evo_latent_absorb(const void* q, int64_t ldq, const void* wuk, vo
         hipLaunchKernelGGL((latent_absorb_kernel<T, NB, V>), grid, block, lds, s, q, ldq, wuk, out, (int)B, (int)H, (int)dn, (int)dr, (int)R, (int)rs); \
     } while (0)
 #define ABV(T, V) do { if (nb == 1) AB(T, 1, V); else if (nb == 2) AB(T, 2, V); else AB(T, 4, V); } while (0)
-    if (f32) { if (v == 8) ABV(float, 8); else ABV(float, 1); }
-    else { if (v == 8) ABV(uint16_t, 8); else ABV(uint16_t, 1); }
+    if (f32) { if (v == 8) ABV(float, 8); else if (v == 4) ABV(float, 4); else ABV(float, 1); }
+    else { if (v == 8) ABV(uint16_t, 8); else if (v == 4) ABV(uint16_t, 4); else ABV(uint16_t, 1); }
 #undef ABV
 #undef AB
     return evo_launch_status();
@@ -531,7 +532,10 @@ __global__ __launch_bounds__(512) void latent_up_kernel(const float* __restrict_
     }
 }
 
-// The same for 16 sequences at a time on the matrix cores (bf16, R % 32 == 0): 128 value rows of one head, a wave owns 16 of them
+// The same on the matrix cores (bf16, R % 32 == 0): 128 value rows of one head and NS sequences, a wave owns 16 of the rows.  Latency and the pace of one CU bound
+// it: at 8 sequences of 16 parts a head's merge reads 262 KB, its rows 131 KB.  So sequences are spread over up to 256 workgroups (a head's rows are read by
+// several), and the first 512 columns of the rows are asked for before the parts.
+// latent_absorb to here, 32 heads, R = 512, 900 slots, in a graph: 3 / 8 / 16 / 32 sequences 28.0 / 34.9 / 39.4 / 48.0 -> 25.7 / 30.6 / 32.3 / 37.2 us.
 template <int NS>
 __global__ __launch_bounds__(512) void latent_up_mfma_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, const float* __restrict__ sink,
                                                              const uint16_t* __restrict__ w, uint16_t* __restrict__ o, int B, int H, int R, int dv, int n_split) {
@@ -540,6 +544,10 @@ __global__ __launch_bounds__(512) void latent_up_mfma_kernel(const float* __rest
     const int pr = R + 8, c16 = lane & 15, g = lane >> 4;
     float* wt = (float*)(lat + NS * pr);
     const int v0 = blockIdx.x * 128 + 16 * wave;
+    const uint16_t* wr = w + ((int64_t)h * dv + (v0 + c16 < dv ? v0 + c16 : dv - 1)) * R + 8 * g;
+    uint4 first[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) first[k] = *(const uint4*)(wr + (32 * k < R ? 32 * k : 0));
     for (int i = wave; i < NS; i += 8) {
         const int b = b0 + i < B ? b0 + i : B - 1;
         const float* ml = part_ml + ((int64_t)b * H + h) * n_split * 2;
@@ -563,11 +571,13 @@ __global__ __launch_bounds__(512) void latent_up_mfma_kernel(const float* __rest
     }
     __syncthreads();
     if (v0 >= dv) return;
-    const uint16_t* wr = w + ((int64_t)h * dv + (v0 + c16 < dv ? v0 + c16 : dv - 1)) * R + 8 * g;
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
     const int cl = c16 < NS ? c16 : 0;                           // (columns beyond NS repeat the first and are not stored)
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+        if (32 * k < R) acc = mfma16(__builtin_bit_cast(mx_frag, first[k]), __builtin_bit_cast(mx_frag, *(const uint4*)(lat + cl * pr + 32 * k + 8 * g)), acc);
 #pragma unroll 8
-    for (int k = 0; k < R; k += 32)
+    for (int k = 512; k < R; k += 32)
         acc = mfma16(__builtin_bit_cast(mx_frag, *(const uint4*)(wr + k)), __builtin_bit_cast(mx_frag, *(const uint4*)(lat + cl * pr + k + 8 * g)), acc);
     if (c16 < NS && b0 + c16 < B) {
         uint16_t* op = o + (int64_t)(b0 + c16) * H * dv + (int64_t)h * dv + v0 + 4 * g;
@@ -581,13 +591,18 @@ extern "C" int evo_latent_up(const float* part_o, const float* part_ml, const fl
                              int64_t dv, int64_t n_split, int64_t f32, int64_t mfma, void* stream) {
     if (!part_o || !part_ml || !sink || !wuv || !o || B <= 0 || H <= 0 || H > 65535 || R <= 0 || R > 8192 || dv <= 0 || n_split <= 0 || n_split > 64) return -1;
     if (!f32 && mfma && B > 2 && R % 32 == 0 && R <= 1024 && (((uintptr_t)wuv | (uintptr_t)part_o) & 15) == 0) {
-        const int ns = B <= 8 ? 8 : 16;
+        int ns = 2;                                              // as many workgroups as there are CUs, if there are that many heads and sequences
+        const int64_t per = H * ((dv + 127) / 128);
+        while (ns < 16 && per * ((B + ns - 1) / ns) > 256) ns *= 2;
         const dim3 grid((unsigned)((dv + 127) / 128), (unsigned)H, (unsigned)((B + ns - 1) / ns));
         const size_t lds = (size_t)ns * ((R + 8) * 2 + n_split * 4);
-        if (ns == 8) hipLaunchKernelGGL((latent_up_mfma_kernel<8>), grid, dim3(512), lds, (hipStream_t)stream, part_o, part_ml, sink, (const uint16_t*)wuv,
-                                        (uint16_t*)o, (int)B, (int)H, (int)R, (int)dv, (int)n_split);
-        else hipLaunchKernelGGL((latent_up_mfma_kernel<16>), grid, dim3(512), lds, (hipStream_t)stream, part_o, part_ml, sink, (const uint16_t*)wuv,
-                                (uint16_t*)o, (int)B, (int)H, (int)R, (int)dv, (int)n_split);
+#define UPM(NS) hipLaunchKernelGGL((latent_up_mfma_kernel<NS>), grid, dim3(512), lds, (hipStream_t)stream, part_o, part_ml, sink, (const uint16_t*)wuv, \
+                                   (uint16_t*)o, (int)B, (int)H, (int)R, (int)dv, (int)n_split)
+        if (ns == 2) UPM(2);
+        else if (ns == 4) UPM(4);
+        else if (ns == 8) UPM(8);
+        else UPM(16);
+#undef UPM
         return evo_launch_status();
     }
     const int nb = B > 2 ? 4 : (int)B;

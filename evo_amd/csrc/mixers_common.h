@@ -35,6 +35,19 @@ template <> struct vec_io<float, 8> {
         ((float4*)p)[1] = make_float4(f[4], f[5], f[6], f[7]);
     }
 };
+template <> struct vec_io<uint16_t, 4> {
+    static __device__ __forceinline__ void load(const uint16_t* p, float* f) {
+        const uint2 v = *(const uint2*)p;
+        f[0] = bf_lo(v.x); f[1] = bf_hi(v.x); f[2] = bf_lo(v.y); f[3] = bf_hi(v.y);
+    }
+};
+template <> struct vec_io<float, 4> {
+    static __device__ __forceinline__ void load(const float* p, float* f) {
+        const float4 a = *(const float4*)p;
+        f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w;
+    }
+    static __device__ __forceinline__ void store(float* p, const float* f) { *(float4*)p = make_float4(f[0], f[1], f[2], f[3]); }
+};
 template <typename T> struct vec_io<T, 1> {
     static __device__ __forceinline__ void load(const T* p, float* f) { f[0] = ld1(p); }
     static __device__ __forceinline__ void store(T* p, const float* f) { st1(p, f[0]); }

@@ -323,3 +323,10 @@ def test_latent_decode(ops, mfma, dt, H, dn, dr, dv, R, window, ring):
             want = V.windowed_sink_attention(q[b:b + 1, :H * (dn + dr)].double().view(1, H, dn + dr), k, v, scale, window, sink, torch.tensor([p]),
                                              torch.tensor(list(js)))
             assert rel_err(got[b:b + 1], want.reshape(1, -1)) < tol(dt, 2e-2, 1e-5), (b, p, n_split)
+
+
+@TYPES
+@pytest.mark.parametrize("H,dn,dr,dv,R", [(70, 40, 16, 72, 64), (2, 136, 24, 130, 640), (1, 7, 8, 17, 1024), (100, 16, 8, 16, 64), (200, 16, 8, 24, 32), (300, 8, 8, 16, 32)])
+def test_latent_decode_maps(ops, mfma, dt, H, dn, dr, dv, R):
+    """The maps around the decode kernel: whole and halved columns, more than one run of rows in flight, rows over 512 wide, 2 to 16 sequences a workgroup."""
+    test_latent_decode(ops, mfma, dt, H, dn, dr, dv, R, 20, 20)
