@@ -202,7 +202,10 @@ struct HDecArgs {
 //   softmax  a lane holds four slots of each of two 16-slot blocks for one query head
 //   sum      O^T = V^T P^T: the probabilities are an operand as they stand (split key order); V goes through a wave-private LDS tile and
 //            is read as dwords, two adjacent dimensions of a slot: the even and the odd dimensions are two operands
-// The waves' sums meet in LDS at the end.  The loads carry no branch: rows past the slots in use repeat a valid one and are masked.
+// The waves' sums meet in LDS at the end, side by side where there is room, else one wave after the other.  The loads carry no branch: rows past the slots in
+// use repeat the last of them, one line for the whole wave, and are masked.  (They were clamped to the ring only: a wave's request behind its last slots
+// read 32 KB of unused cache.  16 heads of two maps, 640 slots, in a graph with the merge: 16 / 24 sequences of up to 600 tokens 38.2 / 55.2 -> 32.9 / 45.8 us;
+// 8 key heads with 4 query heads each, 1,028 slots: 8 / 24 sequences of up to 600 12.4 / 21.2 -> 11.0 / 16.5.)
 // KS: 32-wide steps of a key, NG: 32-wide groups of a value, MAPS: maps per head ([map 1 | map 2] in keys and queries).
 template <int KS, int NG, int MAPS>
 __global__ __launch_bounds__(256) void heads_decode_kernel(HDecArgs a) {
@@ -233,12 +236,14 @@ __global__ __launch_bounds__(256) void heads_decode_kernel(HDecArgs a) {
                 qf[m][ks] = __builtin_bit_cast(mx_frag, v);
             }
     }
+    const int64_t pos = a.pos[b];
+    const int used = pos + 1 < a.ring ? (int)pos + 1 : a.ring, last = used > 0 ? used - 1 : 0;
     mx_u32x4 kf[2][MAPS][KS], rv[2 * NG];
     auto load_k = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll
         for (int jb = 0; jb < 2; ++jb) {
             const int r = s0 + 16 * jb + c16;
-            const uint16_t* p = base + (int64_t)(r < a.ring ? r : a.ring - 1) * a.rs;
+            const uint16_t* p = base + (int64_t)(r < used ? r : last) * a.rs;
 #pragma unroll
             for (int m = 0; m < MAPS; ++m)
 #pragma unroll
@@ -252,15 +257,13 @@ __global__ __launch_bounds__(256) void heads_decode_kernel(HDecArgs a) {
 #pragma unroll
         for (int i = 0; i < 2 * NG; ++i) {
             const int it = lane + 64 * i, r = s0 + it / (4 * NG), d = 8 * (it % (4 * NG));
-            rv[i] = *(const mx_u32x4*)(vbase + (int64_t)(r < a.ring ? r : a.ring - 1) * a.rs + (d < dv ? d : dv - 8));
+            rv[i] = *(const mx_u32x4*)(vbase + (int64_t)(r < used ? r : last) * a.rs + (d < dv ? d : dv - 8));
         }
     };
     const int step = a.n_split * 128;
     int s0 = (split * 4 + wave) * 32;
     load_k(s0);
     load_v(s0);
-    const int64_t pos = a.pos[b];
-    const int used = pos + 1 < a.ring ? (int)pos + 1 : a.ring;
     f32x4_t o[MAPS][NG][2];
     float mx[MAPS], den[MAPS];                                   // den: this lane's slots
 #pragma unroll
@@ -371,6 +374,28 @@ __global__ __launch_bounds__(256) void heads_decode_kernel(HDecArgs a) {
             dst[1] = l;
         }
     }
+    if (MAPS * nq <= 16) {                                       // room for all four waves' sums side by side
+        if (c16 < nq)
+#pragma unroll
+            for (int m = 0; m < MAPS; ++m)
+#pragma unroll
+                for (int n = 0; n < NG; ++n)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        *(float2*)(acc + ((wave * MAPS + m) * nq + c16) * AP + 32 * n + 8 * g + 2 * r) = make_float2(o[m][n][0][r] * f[m], o[m][n][1][r] * f[m]);
+        __syncthreads();
+        for (int it = tid; it < MAPS * nq * (dv / 4); it += 256) {
+            const int m = it / (nq * (dv / 4)), c = it / (dv / 4) % nq, d = it % (dv / 4) * 4;
+            float4 v = *(const float4*)(acc + (m * nq + c) * AP + d);
+#pragma unroll
+            for (int w = 1; w < 4; ++w) {
+                const float4 x = *(const float4*)(acc + ((w * MAPS + m) * nq + c) * AP + d);
+                v.x += x.x; v.y += x.y; v.z += x.z; v.w += x.w;
+            }
+            *(float4*)(a.part_o + ((((int64_t)b * a.H + h0 + c) * MAPS + m) * a.n_split + split) * dv + d) = v;
+        }
+        return;
+    }
     for (int w = 0; w < 4; ++w) {
         if (wave == w) {
 #pragma unroll
@@ -470,7 +495,7 @@ extern "C" int evo_heads_decode(const void* z, int64_t ld, const void* cache, co
         const dim3 grid((unsigned)n_split, (unsigned)(kv_heads * a.n_qb), (unsigned)B);
 #define HD(KS, NG, MAPS)                                                                                                   \
     do {                                                                                                                   \
-        constexpr int tiles = 4 * 32 * (32 * NG + 8) * 2, meet = MAPS * 16 * (32 * NG + 4) * 4, bytes = tiles > meet ? tiles : meet;   \
+        constexpr int tiles = 4 * 32 * (32 * NG + 8) * 2, meet = (MAPS == 1 ? 4 : MAPS) * 16 * (32 * NG + 4) * 4, bytes = tiles > meet ? tiles : meet;   \
         if (bytes > 60 * 1024) (void)hipFuncSetAttribute((const void*)heads_decode_kernel<KS, NG, MAPS>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes); \
         hipLaunchKernelGGL((heads_decode_kernel<KS, NG, MAPS>), grid, dim3(256), (size_t)bytes, s, a);                     \
     } while (0)
