@@ -39,7 +39,7 @@ COMPONENTS = {
         "evo_postnorm_mlp_gate_small_m_bf16", "evo_probe_copy_f4", "evo_probe_mfma_bf16",
     ]),
     "stripedhyena": ("_stripedhyena", ["attn", "attn_w64", "hyena", "hyena_ct"], ["attn_common.h"], [
-        "evo_hyena_seg_state", "evo_hyena_carry_scan", "evo_hyena_carry_add", "evo_hyena_apply", "evo_hyena_step", "evo_hyena_ct", "evo_hyena_ct_packed",
+        "evo_hyena_seg_state", "evo_hyena_short", "evo_hyena_carry_scan", "evo_hyena_carry_add", "evo_hyena_apply", "evo_hyena_step", "evo_hyena_ct", "evo_hyena_ct_packed",
         "evo_attn_fwd_causal_bf16", "evo_attn_fwd_packed_bf16", "evo_attn_decode_bf16",
     ]),
     "mixers": ("_mixers", ["stream", "window_attn"], ["mixers_common.h"], [

@@ -490,6 +490,140 @@ HY_PRAGMA_UNROLL(HY_UNROLL_A)
     }
 }
 
+// ------------------------------------------------------------------------------------------------ the whole operator, short rows
+// Up to SH_T positions: one launch.  A workgroup owns 16 channels of one batch row and all of its positions, cut into 32 segments of C steps (C odd); a lane is a
+// (channel, segment).  z rows come once into LDS (pitch 100 bytes, so that 32 segments of an odd number of rows meet 32 banks); then the same three steps as
+// above: end states from zero, their scan in fp64 by a thread per (channel, mode), the recurrence from the entering states.  y replaces x2 in LDS and leaves in
+// 16-byte pieces.
+// What bounds it: the recurrence itself, 48 multiply-adds a position, channel and pass on every SIMD of the chip (12 ns a position at 4,096 channels), behind about 6 us
+// of loads and barriers.  The three launches leave most of the chip idle here (352 waves at 161 positions).  us, 4,096 channels, three
+// launches -> one: 41 positions 17.6 -> 6.0, 161 24.5 -> 10.0, 500 35.7 -> 20.3, 1,024 52 -> 35; 6 x 161 45.6 -> 34.5, 2 x 600 51.7 -> 42.5.
+#define SH_T 1024
+#define SH_PITCH 100
+#define SH_E 129                             // states of a segment: 16 channels x 8 modes, one more for the banks
+
+__global__ __launch_bounds__(512, 4) void hyena_short_kernel(const unsigned char* __restrict__ z, const unsigned char* __restrict__ z_halo, const uint16_t* __restrict__ fir_w,
+                                                             const uint16_t* __restrict__ fir_b, const float2* __restrict__ poles, const float2* __restrict__ residues,
+                                                             const uint16_t* __restrict__ dskip, const float2* __restrict__ s0, float2* __restrict__ s_final,
+                                                             unsigned char* __restrict__ y, int T, int D, int C) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char sh[];
+    float2* E = (float2*)sh;                                     // [32][SH_E] end states, then entering states
+    unsigned char* zt = sh + 32 * SH_E * 8;                      // [T + 2][SH_PITCH]: x2 | x1 | v of the 16 channels, two rows of history in front
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int d0 = blockIdx.x * 16, b = blockIdx.y;
+    const int64_t rowb = 6 * (int64_t)D;
+    const int col = ((d0 / HD) * 3 * HD + d0 % HD) * 2;
+    const unsigned char* zb = z + (int64_t)b * T * rowb + col;
+    const unsigned char* hb = z_halo ? z_halo + (int64_t)b * 2 * rowb + col : nullptr;
+#pragma unroll 4
+    for (int it = tid; it < (T + 2) * 6; it += 512) {
+        const int r = it / 6, part = it - 6 * r, o = (part >> 1) * (2 * HD) + (part & 1) * 16;
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (r >= 2) v = *(const uint4*)(zb + (int64_t)(r - 2) * rowb + o);
+        else if (hb) v = *(const uint4*)(hb + r * rowb + o);
+        uint32_t* q = (uint32_t*)(zt + r * SH_PITCH + part * 16);
+        q[0] = v.x; q[1] = v.y; q[2] = v.z; q[3] = v.w;
+    }
+    const int seg = lane & 31, ch = 2 * wave + (lane >> 5), d = d0 + ch;
+    const int fc = (d / HD) * 3 * HD + d % HD;                   // x2's column of this channel; x1's and v's HD and 2 HD behind
+    float w[3][3], wb[3], pr[NS], pi[NS];
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) w[g][k] = bf_to_f(fir_w[(fc + g * HD) * 3 + k]);
+        wb[g] = bf_to_f(fir_b[fc + g * HD]);
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s) { const float2 p = poles[(int64_t)d * NS + s]; pr[s] = p.x; pi[s] = p.y; }
+    const int t0 = seg * C, n = T - t0 < C ? T - t0 : C;         // (n <= 0: nothing)
+    const unsigned char* q = zt + (t0 < T ? t0 : 0) * SH_PITCH + ch * 2;          // row t0 - 2
+    auto at = [&](int k, int g) __attribute__((always_inline)) { return bf_to_f(*(const uint16_t*)(q + k * SH_PITCH + g * 32)); };
+    auto fir = [&](int g, float a, float b1, float c) __attribute__((always_inline)) { return fmaf(w[g][2], c, fmaf(w[g][1], b1, fmaf(w[g][0], a, wb[g]))); };
+    __syncthreads();
+
+    float sr[NS], si[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) sr[s] = si[s] = 0.f;
+    float m2[3], m1[3];
+#pragma unroll
+    for (int g = 0; g < 3; ++g) { m2[g] = at(0, g); m1[g] = at(1, g); }
+    {
+        float a1 = m2[1], av = m2[2], b1 = m1[1], bv = m1[2];
+        for (int k = 0; k < n; ++k) {
+            const float c1 = at(k + 2, 1), cv = at(k + 2, 2);
+            const float x = fir(1, a1, b1, c1) * fir(2, av, bv, cv);
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                const float t = fmaf(-pi[s], si[s], x), u = pi[s] * sr[s];
+                sr[s] = fmaf(pr[s], sr[s], t);
+                si[s] = fmaf(pr[s], si[s], u);
+            }
+            a1 = b1; b1 = c1; av = bv; bv = cv;
+        }
+    }
+    if (n > 0) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) E[seg * SH_E + ch * NS + s] = make_float2(sr[s], si[s]);
+    }
+    __syncthreads();                                             // (everyone has the history that its own rows begin with)
+    if (tid < 16 * NS) {                                         // the carry scan of a (channel, mode)
+        const int64_t ds = (int64_t)d0 * NS + tid;
+        const float2 p = poles[ds];
+        double pcr, pci, rr = 0.0, ri = 0.0;
+        cpow_int((double)p.x, (double)p.y, C, pcr, pci);
+        if (s0) { const float2 v = s0[(int64_t)b * D * NS + ds]; rr = v.x; ri = v.y; }
+        const int lead = (T + C - 1) / C - 1;                    // segments of C steps
+        float2* e = E + tid;
+#pragma unroll 4
+        for (int k = 0; k < lead; ++k) {
+            const float2 v = e[k * SH_E];
+            e[k * SH_E] = make_float2((float)rr, (float)ri);
+            const double nr = pcr * rr - pci * ri + (double)v.x;
+            ri = pcr * ri + pci * rr + (double)v.y;
+            rr = nr;
+        }
+        const float2 v = e[lead * SH_E];
+        e[lead * SH_E] = make_float2((float)rr, (float)ri);
+        if (s_final) {
+            double qr, qi;
+            cpow_int((double)p.x, (double)p.y, T - lead * C, qr, qi);
+            const double nr = qr * rr - qi * ri + (double)v.x;
+            ri = qr * ri + qi * rr + (double)v.y;
+            s_final[(int64_t)b * D * NS + ds] = make_float2((float)nr, (float)ri);
+        }
+    }
+    float rr[NS], ri[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) { const float2 r = residues[(int64_t)d * NS + s]; rr[s] = r.x; ri[s] = r.y; }
+    const float dk = bf_to_f(dskip[d]);
+    __syncthreads();
+    if (n > 0) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) { const float2 e = E[seg * SH_E + ch * NS + s]; sr[s] = e.x; si[s] = e.y; }
+        for (int k = 0; k < n; ++k) {
+            float c[3], f[3];
+#pragma unroll
+            for (int g = 0; g < 3; ++g) { c[g] = at(k + 2, g); f[g] = fir(g, m2[g], m1[g], c[g]); m2[g] = m1[g]; m1[g] = c[g]; }
+            const float x = f[1] * f[2];
+            float acc[2] = {0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                const float t = fmaf(-pi[s], si[s], x), u = pi[s] * sr[s];
+                sr[s] = fmaf(pr[s], sr[s], t);
+                si[s] = fmaf(pr[s], si[s], u);
+                acc[s & 1] = fmaf(rr[s], sr[s], fmaf(-ri[s], si[s], acc[s & 1]));
+            }
+            *(uint16_t*)(zt + (t0 + k + 2) * SH_PITCH + ch * 2) = f_to_bf(fmaf(x, dk, acc[0] + acc[1]) * f[0]);   // (y + x1v * D) * x2
+        }
+    }
+    __syncthreads();
+    unsigned char* yb = y + (int64_t)b * T * D * 2 + d0 * 2;
+    for (int it = tid; it < 2 * T; it += 512) {
+        const uint32_t* o = (const uint32_t*)(zt + ((it >> 1) + 2) * SH_PITCH + (it & 1) * 16);
+        *(uint4*)(yb + (int64_t)(it >> 1) * D * 2 + (it & 1) * 16) = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+}
+
 // ------------------------------------------------------------------------------------------------ decode step
 // one thread per (b, channel pair): FIR step with the 2-sample history, roll, modal update, gate.
 __global__ __launch_bounds__(256) void hyena_step_kernel(
@@ -576,6 +710,19 @@ extern "C" int evo_hyena_carry_scan(float* agg, const float* poles, const float*
     hipLaunchKernelGGL(hyena_carry_scan_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
                        (float2*)agg, (const float2*)poles, (const float2*)s0, (float2*)s_final, (int)B, T, (int)D,
                        (int)seg_len, n_seg);
+    return evo_launch_status();
+}
+
+extern "C" int evo_hyena_short(const void* z, const void* z_halo, const void* fir_w, const void* fir_b, const float* poles, const float* residues, const void* dskip,
+                               const float* s0, float* s_final, void* y, int64_t B, int64_t T, int64_t D, int64_t n_heads, void* stream) {
+    if (hyena_check(B, T, D, n_heads, CH) || T > SH_T || B > 65535 || D > 0xfffff) return -1;
+    if (((uintptr_t)z | (uintptr_t)z_halo | (uintptr_t)y) & 15) return -1;
+    const int C = (int)((T + 31) / 32) | 1;                      // (odd: the banks)
+    const size_t lds = 32 * SH_E * 8 + (size_t)(T + 2) * SH_PITCH;                // (<= 133 KB)
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)hyena_short_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 32 * SH_E * 8 + (SH_T + 2) * SH_PITCH);
+    hipLaunchKernelGGL(hyena_short_kernel, dim3((unsigned)(D / 16), (unsigned)B), dim3(512), lds, (hipStream_t)stream, (const unsigned char*)z,
+                       (const unsigned char*)z_halo, (const uint16_t*)fir_w, (const uint16_t*)fir_b, (const float2*)poles, (const float2*)residues, (const uint16_t*)dskip,
+                       (const float2*)s0, (float2*)s_final, (unsigned char*)y, (int)T, (int)D, C);
     return evo_launch_status();
 }
 

@@ -30,6 +30,7 @@ _SIGNATURES = {
     "evo_abi_version": ([], _c.c_int),
     "evo_embed_bf16": ([_PTR, _PTR, _PTR, _I64, _I64, _I64, _PTR, _PTR], _c.c_int),
     "evo_rmsnorm_bf16": ([_PTR, _PTR, _PTR, _PTR, _I64, _I64, _F32, _PTR], _c.c_int),
+    "evo_hyena_short": ([_PTR] * 10 + [_I64] * 4 + [_PTR], _c.c_int),
     "evo_hyena_seg_state": ([_PTR, _PTR, _PTR, _PTR, _PTR, _PTR, _PTR, _I64, _I64, _I64, _I64, _I64, _PTR], _c.c_int),
     "evo_hyena_carry_scan": ([_PTR, _PTR, _PTR, _PTR, _I64, _I64, _I64, _I64, _PTR], _c.c_int),
     "evo_hyena_carry_add": ([_PTR, _PTR, _PTR, _I64, _I64, _I64, _I64, _PTR], _c.c_int),
@@ -97,7 +98,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 16         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 17         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):
@@ -730,6 +731,13 @@ class HipOps(MixerOps):
                                                 poles.data_ptr(), seqs.data_ptr(), seqs_host.data_ptr(), n, D, n_heads, zt.shape[0] * 256, y_blk.shape[0] * self.YBLK,
                                                 _stream()), "evo_hyena_ct_packed")
 
+    @staticmethod
+    def _hyena_short_ok(B, T, z, z_halo, poles, residues) -> bool:
+        """One launch (csrc/hyena.hip hyena_short_kernel) for the rows and alignments that it takes, while its 3.5 + B (0.9 + 0.033 T) us at 4,096 channels, every
+        batch row a round of workgroups, are less than the 21 + 0.021 B T us of the three launches (12 x 41 positions: 33 against 36 us; 32 x 41: 78 against 45; 18 x 5: 28 against 21)."""
+        return (T <= 1024 and B * (T + 75) <= 1450 and (B <= 8 or T >= 41) and z.data_ptr() % 16 == 0 and (z_halo is None or z_halo.data_ptr() % 16 == 0) and poles.data_ptr() % 8 == 0
+                and residues.data_ptr() % 8 == 0)
+
     def hyena_prefill(self, z: torch.Tensor, fir_w: torch.Tensor, fir_b: torch.Tensor, poles: torch.Tensor,
                       residues: torch.Tensor, dskip: torch.Tensor, n_heads: int,
                       z_halo: Optional[torch.Tensor] = None, s0: Optional[torch.Tensor] = None,
@@ -756,6 +764,14 @@ class HipOps(MixerOps):
         if s0 is not None:
             s0r = torch.view_as_real(s0.to(torch.complex64).contiguous())
             assert s0r.shape == (B, D, 8, 2)
+        if mask is None and not seg_len and not self.seg_len_override and self._hyena_short_ok(B, T, z, z_halo, poles, residues):
+            y = torch.empty(B, T, D, dtype=torch.bfloat16, device=z.device)
+            s_final = torch.empty(B, D, 8, 2, dtype=torch.float32, device=z.device) if want_state else None
+            with self._t("hyena_short"):
+                _check(self.lib.evo_hyena_short(z.data_ptr(), _ptr(z_halo), fir_w.data_ptr(), fir_b.data_ptr(), poles.data_ptr(), residues.data_ptr(), dskip.data_ptr(),
+                                                _ptr(s0r), _ptr(s_final), y.data_ptr(), B, T, D, n_heads, _stream()), "evo_hyena_short")
+            self.last_hyena_io = {"short": (z.numel() + y.numel()) * 2}
+            return y, torch.view_as_complex(s_final) if want_state else None
         C = seg_len or self.seg_len_override or pick_segment_length(B, T, n_heads)
         n_seg = (T + C - 1) // C
         agg = torch.empty(B, n_seg, D, 8, 2, dtype=torch.float32, device=z.device)

@@ -57,8 +57,9 @@ extern "C" {
  *  13: evo_dense_bf16 and evo_dense_ws (any dense layer on the tiles its size asks for), evo_put_tokens and evo_advance_positions added.
  *  14: evo_linear_f32 and evo_linear_f32_ws (fp32 dense layers on the bf16 matrix cores) added.
  *  15: evo_dense_plan and evo_linear_f32_plan (the launches of a dense layer) added.
- *  16: evo_hyena_ct_packed and evo_attn_fwd_packed_bf16 (unequal sequences in one launch), evo_copy_rows added. */
-#define EVO_ABI_VERSION 16
+ *  16: evo_hyena_ct_packed and evo_attn_fwd_packed_bf16 (unequal sequences in one launch), evo_copy_rows added.
+ *  17: evo_hyena_short added. */
+#define EVO_ABI_VERSION 17
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
@@ -117,6 +118,9 @@ int evo_hyena_seg_state(const void* z, const void* z_halo, const void* fir_w, co
                         int64_t B, int64_t T, int64_t D, int64_t n_heads, int64_t seg_len, void* stream);
 int evo_hyena_carry_scan(float* agg, const float* poles, const float* s0, float* s_final,
                          int64_t B, int64_t T, int64_t D, int64_t seg_len, void* stream);
+/* the three launches in one, for rows of up to 1,024 positions; z, z_halo and y 16-byte aligned, poles, residues, s0 and s_final 8-byte */
+int evo_hyena_short(const void* z, const void* z_halo, const void* fir_w, const void* fir_b, const float* poles, const float* residues, const void* dskip,
+                    const float* s0, float* s_final, void* y, int64_t B, int64_t T, int64_t D, int64_t n_heads, void* stream);
 /* sequence-parallel fix-up (new; the reference has no multi-GPU path): `agg` already scanned with a zero
  * carry-in gets p^(k*seg_len) * s0 added to segment k once the state s0 entering this shard is known. */
 int evo_hyena_carry_add(float* agg, const float* poles, const float* s0,
