@@ -35,7 +35,7 @@ COMPONENTS = {
         "evo_hyena_decode_fused_small_m", "evo_linear_mfma_bf16", "evo_linear_mfma_nf_bf16", "evo_mlp_gate_mfma_bf16",
         "evo_mlp_gate_mfma_nf_bf16", "evo_linear_xblk_mfma_bf16", "evo_linear_xblk_mfma_nf_bf16", "evo_linear_t_mfma_bf16",
         "evo_linear_t_mfma_nf_bf16", "evo_linear_act_mfma_bf16", "evo_dense_ws", "evo_dense_plan", "evo_dense_bf16", "evo_linear_f32_ws", "evo_linear_f32_plan", "evo_linear_f32", "evo_put_tokens",
-        "evo_advance_positions", "evo_copy_rows", "evo_postnorm_linear_small_m_bf16",
+        "evo_advance_positions", "evo_copy_rows", "evo_linear_parts", "evo_linear_parts_bf16", "evo_postnorm_linear_small_m_bf16",
         "evo_postnorm_mlp_gate_small_m_bf16", "evo_probe_copy_f4", "evo_probe_mfma_bf16",
     ]),
     "stripedhyena": ("_stripedhyena", ["attn", "attn_w64", "hyena", "hyena_ct"], ["attn_common.h"], [
@@ -43,12 +43,12 @@ COMPONENTS = {
         "evo_attn_fwd_causal_bf16", "evo_attn_fwd_packed_bf16", "evo_attn_decode_bf16",
     ]),
     "mixers": ("_mixers", ["stream", "window_attn"], ["mixers_common.h"], [
-        "evo_embed_stream", "evo_postnorm_residual", "evo_sum_norm", "evo_rmsnorm_stream", "evo_gated_norm", "evo_silu_gate", "evo_act_cols",
+        "evo_embed_stream", "evo_postnorm_residual", "evo_sum_norm", "evo_closing_parts", "evo_rmsnorm_stream", "evo_gated_norm", "evo_silu_gate", "evo_act_cols",
         "evo_window_attn",
     ]),
     "lightning": ("_lightning", ["lightning"], ["mixers_common.h"], ["evo_lightning_chunk_bf16", "evo_lightning_recurrent"]),
     "latent": ("_latent", ["latent"], ["mixers_common.h"], ["evo_latent_prep", "evo_latent_absorb", "evo_latent_decode", "evo_latent_up"]),
-    "heads": ("_heads", ["heads"], ["mixers_common.h"], ["evo_heads_prep", "evo_heads_decode", "evo_heads_merge"]),
+    "heads": ("_heads", ["heads"], ["mixers_common.h"], ["evo_heads_prep", "evo_heads_decode", "evo_heads_decode_whole", "evo_heads_merge"]),
     "rglru": ("_rglru", ["rglru"], ["mixers_common.h"], ["evo_rglru_chunk_bf16", "evo_rglru_step_bf16", "evo_rglru_any"]),
 }
 

@@ -1385,6 +1385,20 @@ extern "C" int evo_norm_mlp_gate_small_m_bf16(const void* x, const void* scale, 
     return mlp_gate_launch(x, scale, w12, a, M, I, K, eps, grouped, 0, (hipStream_t)stream);
 }
 
+// narrow layers, 16 rows a CU: parts of K where the batch rows would be read more often than the weights; a workgroup per CU.  0: one sum
+static int small_m_parts(int64_t M, int64_t N, int64_t K) {
+    if (M < 17 || M > 64 || N > 4096 || N < 1024 || N % 64 != 0 || K < 1024 || K % 128 != 0 || K > 0x9fffff || (K < 8192 && M <= 32)) return 0;
+    int64_t parts = (256 + N / 64 - 1) / (N / 64);
+    if (parts > K / 256) parts = K / 256;
+    if (parts > 8) parts = 8;
+    return parts >= 2 ? (int)parts : 0;
+}
+extern "C" int evo_linear_parts(int64_t M, int64_t N, int64_t K) { return small_m_parts(M, N, K); }
+extern "C" int evo_linear_parts_bf16(const void* x, const void* w, float* ws, int64_t M, int64_t N, int64_t K, int64_t parts, void* stream) {
+    if (!x || !w || !ws || parts < 2 || parts != small_m_parts(M, N, K) || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)ws) & 15)) return -1;
+    return ring_launch<2>(x, w, nullptr, nullptr, nullptr, M, N, K, 0, 0, ws, (int)parts, (hipStream_t)stream);
+}
+
 extern "C" int evo_linear_small_m_bf16(const void* x, const void* w, const void* bias, const void* residual, void* y,
                                        int64_t M, int64_t N, int64_t K, void* ws, int64_t ws_bytes, int64_t act, void* stream) {
     if (M < 1 || M > 64 || N <= 0 || K <= 0 || K % 8 != 0 || N > 0x7fffffff - 16) return -1;
@@ -1398,18 +1412,13 @@ extern "C" int evo_linear_small_m_bf16(const void* x, const void* w, const void*
         if (K % 128 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && K <= 0x9fffff) {
             // wide layers
             if (N > 4096) return ring_launch<0>(x, w, bias, residual, y, M, N, K, (int)act, 0, nullptr, 0, s);
-            // narrow layers, 16 rows a CU: parts of K where the batch rows would be read more often than the weights
-            if (ws && M >= 17 && (K >= 8192 || M > 32) && N % 64 == 0 && N >= 1024 && K >= 1024) {
-                int64_t parts = (256 + N / 64 - 1) / (N / 64);       // a workgroup per CU
-                if (parts > K / 256) parts = K / 256;
-                if (parts > 8) parts = 8;
-                if (parts >= 2 && ws_bytes >= parts * M * N * 4 && ((uintptr_t)ws & 15) == 0) {
-                    const int rc = ring_launch<2>(x, w, nullptr, nullptr, nullptr, M, N, K, 0, 0, (float*)ws, (int)parts, s);
-                    if (rc) return rc;
-                    hipLaunchKernelGGL(skinny_reduce_kernel, dim3((unsigned)((M * N / 4 + 255) / 256)), dim3(256), 0, s, (const float*)ws, (const uint16_t*)bias,
-                                       (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)parts, (int)act);
-                    return evo_launch_status();
-                }
+            const int64_t parts = ws && ((uintptr_t)ws & 15) == 0 ? small_m_parts(M, N, K) : 0;
+            if (parts && ws_bytes >= parts * M * N * 4) {
+                const int rc = ring_launch<2>(x, w, nullptr, nullptr, nullptr, M, N, K, 0, 0, (float*)ws, (int)parts, s);
+                if (rc) return rc;
+                hipLaunchKernelGGL(skinny_reduce_kernel, dim3((unsigned)((M * N / 4 + 255) / 256)), dim3(256), 0, s, (const float*)ws, (const uint16_t*)bias,
+                                   (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)parts, (int)act);
+                return evo_launch_status();
             }
             // (few workgroups, the unembedding's 512 columns: more waves in each -- us at 8 / 16 / 32 rows, K = 4,096: 6.0 / 6.8 / 8.4, with four 6.1 / 6.9 / 8.8)
             if (N < 2048) {

@@ -194,6 +194,8 @@ struct HDecArgs {
     const void* z; int64_t ld; const void* cache; const int64_t* pos; float* part_o; float* part_ml;
     int H, G, dim, dv, rs, ring, n_split, n_qb;                  // n_qb: blocks of 16 query heads per key head
     float sc2;                                                   // scale * log2(e)
+    uint16_t* o = nullptr;                                       // n_split 1, maps x query heads of a workgroup <= 16: the result itself, no parts
+    float lam = 0.f, gain = 1.f, eps = 0.f;                      // (heads_merge_kernel's; what it measured: MixerOps.heads_whole_ok)
 };
 
 // Matrix cores (bf16).  A workgroup: one (sequence, key head, up to 16 of its query heads) and its share of the slots, 32 at a time per wave
@@ -365,7 +367,7 @@ __global__ __launch_bounds__(256) void heads_decode_kernel(HDecArgs a) {
     for (int m = 0; m < MAPS; ++m) {
         const float top = fmaxf(fmaxf(ml[0][m][c16][0], ml[1][m][c16][0]), fmaxf(ml[2][m][c16][0], ml[3][m][c16][0]));
         f[m] = __builtin_amdgcn_exp2f(mx[m] - top);
-        if (wave == 0 && g == 0 && c16 < nq) {
+        if (!a.o && wave == 0 && g == 0 && c16 < nq) {
             float l = 0.f;
 #pragma unroll
             for (int w = 0; w < 4; ++w) l = fmaf(ml[w][m][c16][1], __builtin_amdgcn_exp2f(ml[w][m][c16][0] - top), l);
@@ -384,6 +386,38 @@ __global__ __launch_bounds__(256) void heads_decode_kernel(HDecArgs a) {
                     for (int r = 0; r < 4; ++r)
                         *(float2*)(acc + ((wave * MAPS + m) * nq + c16) * AP + 32 * n + 8 * g + 2 * r) = make_float2(o[m][n][0][r] * f[m], o[m][n][1][r] * f[m]);
         __syncthreads();
+        if (a.o) {                                               // heads_merge_kernel's steps on one part: a wave per query head, four values a lane
+            for (int c = wave; c < nq; c += 4) {
+                float x[4] = {0.f, 0.f, 0.f, 0.f}, ss = 0.f;
+                const int d = 4 * lane;
+#pragma unroll
+                for (int m = 0; m < MAPS; ++m) {
+                    const float top = fmaxf(fmaxf(ml[0][m][c][0], ml[1][m][c][0]), fmaxf(ml[2][m][c][0], ml[3][m][c][0]));
+                    float l = 0.f;
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) l = fmaf(ml[w][m][c][1], __builtin_amdgcn_exp2f(ml[w][m][c][0] - top), l);
+                    const float wt = 1.0f / l;
+                    if (d < dv) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            float v = acc[(m * nq + c) * AP + d + e];
+#pragma unroll
+                            for (int w = 1; w < 4; ++w) v += acc[((w * MAPS + m) * nq + c) * AP + d + e];
+                            v *= wt;
+                            x[e] = m == 0 ? v : x[e] - a.lam * v;
+                        }
+                    }
+                }
+                float f = 1.0f;
+                if constexpr (MAPS == 2) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) ss = fmaf(x[e], x[e], ss);
+                    f = a.gain / sqrtf(wave_sum(ss) / (float)dv + a.eps);
+                }
+                if (d < dv) *(uint2*)(a.o + ((int64_t)b * a.H + h0 + c) * dv + d) = make_uint2(pack_bf2(x[0] * f, x[1] * f), pack_bf2(x[2] * f, x[3] * f));
+            }
+            return;
+        }
         for (int it = tid; it < MAPS * nq * (dv / 4); it += 256) {
             const int m = it / (nq * (dv / 4)), c = it / (dv / 4) % nq, d = it % (dv / 4) * 4;
             float4 v = *(const float4*)(acc + (m * nq + c) * AP + d);
@@ -481,17 +515,18 @@ __global__ __launch_bounds__(64) void heads_decode_any_kernel(HDecArgs a, int ma
     if (lane == 0) { a.part_ml[2 * p] = m; a.part_ml[2 * p + 1] = l; }
 }
 
-extern "C" int evo_heads_decode(const void* z, int64_t ld, const void* cache, const int64_t* pos, float* part_o, float* part_ml, int64_t B, int64_t H,
+static int heads_decode(void* o, float lam, float gain, float eps, const void* z, int64_t ld, const void* cache, const int64_t* pos, float* part_o, float* part_ml, int64_t B, int64_t H,
                                 int64_t kv_heads, int64_t maps, int64_t dim, int64_t dv, int64_t ring, int64_t rs, int64_t n_split, float scale,
                                 int64_t f32, int64_t mfma, void* stream) {
-    if (!z || !cache || !pos || !part_o || !part_ml || B <= 0 || B > 65535 || H <= 0 || H > 16384 || kv_heads <= 0 || H % kv_heads) return -1;
+    if (!z || !cache || !pos || (o ? n_split != 1 : !part_o || !part_ml) || B <= 0 || B > 65535 || H <= 0 || H > 16384 || kv_heads <= 0 || H % kv_heads) return -1;
     if ((maps != 1 && maps != 2) || dim <= 0 || dim > 8192 || dv <= 0 || dv > 512 || ring <= 0 || ring > 0x3fffffff || n_split <= 0 || n_split > 1024) return -1;
     if (ld < H * maps * dim || rs < kv_heads * (maps * dim + dv) || rs > 0x3fffffff) return -1;
     const int64_t Q = H / kv_heads;
     HDecArgs a = {z, ld, cache, pos, part_o, part_ml, (int)H, (int)kv_heads, (int)dim, (int)dv, (int)rs, (int)ring, (int)n_split, (int)((Q + 15) / 16), scale * LOG2E};
+    a.o = (uint16_t*)o; a.lam = lam; a.gain = gain; a.eps = eps;
     hipStream_t s = (hipStream_t)stream;
     if (!f32 && mfma && dim % 8 == 0 && dv % 8 == 0 && ld % 8 == 0 && rs % 8 == 0 && dim <= (maps == 2 ? 128 : 256) && dv <= 256 &&
-        (((uintptr_t)z | (uintptr_t)cache | (uintptr_t)part_o) & 15) == 0) {
+        (((uintptr_t)z | (uintptr_t)cache | (uintptr_t)part_o | (uintptr_t)o) & 15) == 0 && (!o || maps * (Q < 16 ? Q : 16) <= 16)) {
         const dim3 grid((unsigned)n_split, (unsigned)(kv_heads * a.n_qb), (unsigned)B);
 #define HD(KS, NG, MAPS)                                                                                                   \
     do {                                                                                                                   \
@@ -506,12 +541,25 @@ extern "C" int evo_heads_decode(const void* z, int64_t ld, const void* cache, co
 #undef HD
         return evo_launch_status();
     }
+    if (o) return -1;
     const dim3 grid((unsigned)n_split, (unsigned)(H * maps), (unsigned)B);
     if (f32 && dim % 4 == 0 && dv % 4 == 0 && rs % 4 == 0 && ((uintptr_t)cache & 15) == 0)
         hipLaunchKernelGGL((heads_decode_any_kernel<float, 4>), grid, dim3(64), (size_t)dim * 4, s, a, (int)maps);
     else if (f32) hipLaunchKernelGGL((heads_decode_any_kernel<float, 1>), grid, dim3(64), (size_t)dim * 4, s, a, (int)maps);
     else hipLaunchKernelGGL((heads_decode_any_kernel<uint16_t, 1>), grid, dim3(64), (size_t)dim * 4, s, a, (int)maps);
     return evo_launch_status();
+}
+
+extern "C" int evo_heads_decode(const void* z, int64_t ld, const void* cache, const int64_t* pos, float* part_o, float* part_ml, int64_t B, int64_t H,
+                                int64_t kv_heads, int64_t maps, int64_t dim, int64_t dv, int64_t ring, int64_t rs, int64_t n_split, float scale,
+                                int64_t f32, int64_t mfma, void* stream) {
+    return heads_decode(nullptr, 0.f, 1.f, 0.f, z, ld, cache, pos, part_o, part_ml, B, H, kv_heads, maps, dim, dv, ring, rs, n_split, scale, f32, mfma, stream);
+}
+
+extern "C" int evo_heads_decode_whole(const void* z, int64_t ld, const void* cache, const int64_t* pos, void* o, int64_t B, int64_t H, int64_t kv_heads, int64_t maps,
+                                      int64_t dim, int64_t dv, int64_t ring, int64_t rs, float scale, float lam, float gain, float eps, void* stream) {
+    if (!o) return -1;
+    return heads_decode(o, lam, gain, eps, z, ld, cache, pos, nullptr, nullptr, B, H, kv_heads, maps, dim, dv, ring, rs, 1, scale, 0, 1, stream);
 }
 
 // o = the merged parts of a head; two maps: gain * unit_rms(o1 - lam o2) over its dv values

@@ -49,9 +49,10 @@ extern "C" int evo_embed_stream(const int64_t* ids, const void* w, float* x, voi
 // SUM: x = norm(alpha x + y) * (off + w); `y` below is then the sum.
 // y stays in registers between the two passes (rows up to 4,096 elements); x is written in fp32 and, for the next sublayer's matrix
 // product, once more in bf16.
-template <typename T, int V, bool SUM>
+// PARTS: y is the sum of `parts` fp32 planes [gridDim.x, D] one behind the other, added in their order and rounded to bf16 (what evo_linear_small_m_bf16 stores).
+template <typename T, int V, bool SUM, bool PARTS = false>
 __device__ __forceinline__ void closing_norm(const void* __restrict__ y_, const void* __restrict__ w_, float* __restrict__ x,
-                                             uint16_t* __restrict__ xb, int D, float alpha, float eps, float off) {
+                                             uint16_t* __restrict__ xb, int D, float alpha, float eps, float off, int parts = 0) {
     constexpr int KEEP = V == 8 ? 2 : 4;                         // runs of V elements a thread keeps in registers (D <= 256 V KEEP)
     __shared__ float red[4];
     const T* w = (const T*)w_;
@@ -60,7 +61,18 @@ __device__ __forceinline__ void closing_norm(const void* __restrict__ y_, const 
     float keep[KEEP][V];
     float ss = 0.f;
     auto load = [&](int c, float* f) {
-        vec_io<T, V>::load(y + c, f);
+        if constexpr (PARTS) {
+            const float* p = (const float*)y_ + row * D + c;
+            vec_io<float, V>::load(p, f);
+            for (int s = 1; s < parts; ++s) {
+                float q[V];
+                vec_io<float, V>::load(p + s * ((int64_t)gridDim.x * D), q);
+#pragma unroll
+                for (int e = 0; e < V; ++e) f[e] += q[e];
+            }
+#pragma unroll
+            for (int e = 0; e < V; ++e) f[e] = bf_to_f(f_to_bf(f[e]));
+        } else vec_io<T, V>::load(y + c, f);
         if constexpr (SUM) {
             float r[V];
             vec_io<float, V>::load(x + row * D + c, r);
@@ -128,6 +140,23 @@ extern "C" int evo_sum_norm(const void* y, const void* w, float* x, void* xb, in
     if (!y || !w || !x || M < 0 || M > 0x7fffffff || D <= 0 || D > 0x3fffffff) return -1;
     if (M == 0) return 0;
     STREAM_DISPATCH(sum_norm_kernel, D % 8 == 0, (unsigned)M, y, w, x, (uint16_t*)xb, (int)D, alpha, eps, w_offset);
+}
+
+// Both on the parts of a dense layer's sum (evo_linear_parts_bf16): the launch that added and rounded them was 4.7 us of its own, a decode layer of 17 to 64 rows.
+template <bool SUM>
+__global__ __launch_bounds__(256) void closing_parts_kernel(const float* __restrict__ y, const void* __restrict__ w, float* __restrict__ x, uint16_t* __restrict__ xb, int D,
+                                                            float alpha, float eps, float off, int parts) {
+    closing_norm<uint16_t, 8, SUM, true>(y, w, x, xb, D, alpha, eps, off, parts);
+}
+
+extern "C" int evo_closing_parts(const float* y, int64_t parts, const void* w, float* x, void* xb, int64_t M, int64_t D, int64_t sum, float alpha, float eps, float w_offset,
+                                 void* stream) {
+    if (!y || !w || !x || !xb || parts < 1 || parts > 64 || M < 0 || M > 0x7fffffff || D <= 0 || D > 0x3fffffff || D % 8 != 0) return -1;
+    if (((uintptr_t)y | (uintptr_t)w | (uintptr_t)x | (uintptr_t)xb) & 15) return -1;
+    if (M == 0) return 0;
+    if (sum) hipLaunchKernelGGL(closing_parts_kernel<true>, dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream, y, w, x, (uint16_t*)xb, (int)D, alpha, eps, w_offset, (int)parts);
+    else hipLaunchKernelGGL(closing_parts_kernel<false>, dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream, y, w, x, (uint16_t*)xb, (int)D, 1.f, eps, w_offset, (int)parts);
+    return evo_launch_status();
 }
 
 // ---------------------------------------------------------------------------------------------- out = norm(x) * (off + w), x the stream

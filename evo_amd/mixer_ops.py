@@ -56,8 +56,17 @@ class Stream:
         self.spare = None                                        # the buffer the next such launch writes x to
         self.behind = False                                      # xb does not hold the current x
 
+    def product(self, a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+        """a @ w^T of a sublayer, for `add` -- or its parts over K [parts, M, N], where a few rows' layer is summed in parts: the closing norm adds them."""
+        parts = self.ops.linear_parts(a, w) if self.xb.dtype == torch.bfloat16 and hasattr(self.ops, "linear_parts") else None
+        return self.ops.linear(a, w) if parts is None else parts
+
     def add(self, y: torch.Tensor, w: torch.Tensor) -> None:
         self.flush()
+        if y.dim() == 3:                                         # (parts)
+            self.ops.closing_parts_(self.x, self.xb, y, w, self.alpha, self.eps, self.w_offset)
+            self.behind = False
+            return
         self.open = (y, w)
         if not self.ops.fuse_postnorm_ok(y):
             self.flush()
@@ -172,6 +181,20 @@ class MixerOps:
     def sum_norm_(self, x: torch.Tensor, xb: torch.Tensor, y: torch.Tensor, w: torch.Tensor, alpha: float, eps: float, w_offset: float) -> None:
         """x = rms_norm(alpha x + y) * (w_offset + w) in place; xb follows."""
         self._call("evo_sum_norm", *self._closing_args(x, xb, y, w), float(alpha), float(eps), float(w_offset), int(y.dtype == torch.float32))
+
+    def closing_parts_(self, x: torch.Tensor, xb: torch.Tensor, y: torch.Tensor, w: torch.Tensor, alpha: Optional[float], eps: float, w_offset: float) -> None:
+        """sum_norm_ (`alpha` given) or postnorm_residual_ on the parts y [parts, M, D] of a dense layer (HipOps.linear_parts)."""
+        n, M, D = y.shape
+        assert y.dtype == torch.float32 and y.is_contiguous() and x.dtype == torch.float32 and self._store(xb, w) == 0
+        self._dense(x, (M, D), "x"), self._dense(xb, (M, D), "xb"), self._dense(w, (D,), "w")
+        if (x.data_ptr() | xb.data_ptr() | w.data_ptr()) % 16:   # (a norm weight cut out of a larger tensor)
+            total = y[0]
+            for part in y[1:]:
+                total = total + part
+            total = total.to(xb.dtype)
+            return self.postnorm_residual_(x, xb, total, w, eps, w_offset) if alpha is None else self.sum_norm_(x, xb, total, w, alpha, eps, w_offset)
+        self._call("evo_closing_parts", y.data_ptr(), n, w.data_ptr(), x.data_ptr(), xb.data_ptr(), M, D, int(alpha is not None), float(alpha or 0.0), float(eps),
+                   float(w_offset))
 
     fuse_postnorm = True       # False: every closing norm as its own launch (tests, measurements)
 
@@ -418,6 +441,15 @@ class MixerOps:
         """Parts of the cache in the decode kernel: a workgroup per CU, at least 128 slots (one round of a workgroup's waves) each."""
         return max(1, min((ring + 127) // 128, (cus + groups - 1) // groups, 64))
 
+    def heads_whole_ok(self, groups: int, ring: int, Q: int, maps: int, dim: int, dv: int, z, cache) -> bool:
+        """One workgroup per (sequence, key head) walks its whole cache and writes the result itself: no parts, no merge launch.  From 160 of them on, and from 80 on
+        where a whole cache is short.  us in a graph, parts and merge -> whole: 16 heads of two maps, 640 slots, 10 / 24 / 32 sequences of up to 600 tokens 32.2 / 45.9 /
+        52.0 -> 25.1 / 42.1 / 46.9 (2,048 slots, 10 of up to 1,500 48.4 -> 49.4); 8 key heads of 4 queries each, 1,028 slots, 10 / 24 sequences of up to 600
+        13.2 / 16.6 -> 10.3 / 12.6, of up to 1,500 16.5 / 25.6 -> 14.8 / 22.5 (8 sequences 13.4 -> 14.8: not taken)."""
+        return (self.mixer_mfma and z.dtype == torch.bfloat16 and dim % 8 == 0 and dv % 8 == 0 and z.stride(0) % 8 == 0 and cache.shape[2] % 8 == 0
+                and dim <= (128 if maps == 2 else 256) and dv <= 256 and maps * min(Q, 16) <= 16 and (z.data_ptr() | cache.data_ptr()) % 16 == 0
+                and (groups >= 160 or (groups >= 80 and ring * (maps * dim + dv) <= 300000)))
+
     def heads_decode(self, z: torch.Tensor, cache: torch.Tensor, pos: torch.Tensor, heads: int, kv_heads: int, maps: int, dim: int, dv: int, scale: float,
                      lam: float, gain: float, eps: float, n_split: Optional[int] = None) -> torch.Tensor:
         """One token per cache row (already appended by heads_prep) -> [B, heads dv]."""
@@ -426,9 +458,15 @@ class MixerOps:
         rows, ring, rs = cache.shape
         self._dense(cache, (rows, ring, rs), "key and value cache")
         assert rows >= B and z.shape[1] >= heads * maps * dim and rs >= kv_heads * (maps * dim + dv)
+        groups = B * kv_heads * ((heads // kv_heads + 15) // 16)
+        if n_split is None and self.heads_whole_ok(groups, ring, heads // kv_heads, maps, dim, dv, z, cache):
+            o = torch.empty(B, heads * dv, dtype=z.dtype, device=z.device)
+            self._call("evo_heads_decode_whole", z.data_ptr(), z.stride(0), cache.data_ptr(), self._ix(pos, torch.int64, B, "pos"), o.data_ptr(), B, heads, kv_heads,
+                       maps, dim, dv, ring, rs, float(scale), float(lam), float(gain), float(eps))
+            return o
         if n_split is None:
             # (fp32: one wave per part, head and sequence, 64 slots a round)
-            n_split = max(1, min((ring + 63) // 64, 4096 // (B * heads * maps), 64)) if f32 else self.heads_split(B * kv_heads * ((heads // kv_heads + 15) // 16), ring)
+            n_split = max(1, min((ring + 63) // 64, 4096 // (B * heads * maps), 64)) if f32 else self.heads_split(groups, ring)
         part_o = torch.empty(B, heads * maps, n_split, dv, dtype=torch.float32, device=z.device)
         part_ml = torch.empty(B, heads * maps, n_split, 2, dtype=torch.float32, device=z.device)
         self._call("evo_heads_decode", z.data_ptr(), z.stride(0), cache.data_ptr(), self._ix(pos, torch.int64, B, "pos"), part_o.data_ptr(),

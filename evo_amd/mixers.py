@@ -97,7 +97,7 @@ class LightningMixer(Sublayer):
         # [q | k | v | g]; a prompt's q, k, v come activated, a decode step activates its own
         z = stream.linear(self.w_in) if batch.decode else ops.linear_act(stream.input(), self.w_in, "silu", g0)
         o = ops.lightning(z, H, dk, dv, self.decay, self.log2_decay, batch, cache)
-        return ops.linear(ops.gated_norm(o, z[:, g0:g0 + H * dv], self.w_norm, self.eps), self.w_o)
+        return stream.product(ops.gated_norm(o, z[:, g0:g0 + H * dv], self.w_norm, self.eps), self.w_o)
 
 
 class LatentAttention(Sublayer):
@@ -156,7 +156,7 @@ class LatentAttention(Sublayer):
         if batch.decode:
             ops.latent_prep(qd, H, dn, dr, R, self.w_norm, self.inv_freq, self.eps, batch, cache, want_kv=False)
             a = ops.latent_decode(qd, cache, batch.pos, self.w_kv[:H * dn], self.w_kv[H * dn:], self.sink, H, dn, dr, dv, R, self.window, self.scale)
-            return ops.linear(a, self.w_o)
+            return stream.product(a, self.w_o)
         old, seen = (None, None) if batch.resume is None else self._earlier(batch, cache)   # (read before the ring moves on)
         c, kr = ops.latent_prep(qd, H, dn, dr, R, self.w_norm, self.inv_freq, self.eps, batch, cache, want_kv=True)
         cu_k = batch.cu
@@ -168,7 +168,7 @@ class LatentAttention(Sublayer):
             cu_k = total.to(torch.int32).to(c.device)
         kv = ops.linear(c, self.w_kv)                             # every head's keys, then every head's values
         a = ops.window_attention(qd, kv, kr, H, dn, dr, dv, self.window, self.scale, self.sink, batch.cu, cu_k, max(batch.lens))
-        return ops.linear(a, self.w_o)
+        return stream.product(a, self.w_o)
 
 
 def rotation(rot: dict, where: str):
@@ -282,13 +282,13 @@ class HeadAttention(Sublayer):
                        batch, cache, self.keep)
         tail = (self.scale, self.lam, 1.0 - self.diff, self.eps)
         if batch.decode:
-            return ops.linear(ops.heads_decode(z, cache, batch.pos, H, G, self.maps, n, dv, *tail), self.w_o)
+            return stream.product(ops.heads_decode(z, cache, batch.pos, H, G, self.maps, n, dv, *tail), self.w_o)
         kv, cu_k = z[:, self.nq * n: (self.nq + self.nk) * n + self.nv], batch.cu
         if old is not None:
             kv = torch.cat([t for o, new in zip(old, kv.split(batch.lens)) for t in (o[:, : kv.shape[1]], new)])
             cu_k = torch.tensor([0] + [o.shape[0] + m for o, m in zip(old, batch.lens)]).cumsum(0).to(torch.int32).to(z.device)
         a = ops.heads_attention(z, kv, H, G, self.maps, n, dv, self.window, self.keep, *tail, batch.cu, cu_k, max(batch.lens))
-        return ops.linear(a, self.w_o)
+        return stream.product(a, self.w_o)
 
 
 class GatedRecurrence(Sublayer):
@@ -336,7 +336,7 @@ class GatedRecurrence(Sublayer):
         z = stream.linear(self.w_in) if batch.decode else ops.linear_act(stream.input(), self.w_in, "gelu_tanh", self.W, self.b_in)
         o = ops.rglru(z, self.b_in if batch.decode else None, batch.decode, self.W, self.conv, self.conv_b, self.ra, self.ra_b, self.ri, self.ri_b, self.decay,
                       batch, cache)
-        return ops.linear(o, self.w_o)
+        return stream.product(o, self.w_o)
 
 
 class PlainFF(Sublayer):
@@ -360,7 +360,7 @@ class PlainFF(Sublayer):
         return [tuple(self.w_up.shape), tuple(self.w_down.shape)]
 
     def forward_ff(self, ops, stream: Stream) -> torch.Tensor:
-        return ops.linear(stream.linear(self.w_up, act=self.act), self.w_down)
+        return stream.product(stream.linear(self.w_up, act=self.act), self.w_down)
 
 
 class GatedFF(Sublayer):
@@ -389,7 +389,7 @@ class GatedFF(Sublayer):
         return [tuple(self.w12.shape), tuple(self.w3.shape)]
 
     def forward_ff(self, ops, stream: Stream) -> torch.Tensor:
-        return ops.linear(stream.gate(self.w12, self.grouped, "silu"), self.w3)
+        return stream.product(stream.gate(self.w12, self.grouped, "silu"), self.w3)
 
 
 def build_mixer(kinds: dict, layer: dict, width: int, eps: float, dtype: torch.dtype, where: str) -> Sublayer:

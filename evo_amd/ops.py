@@ -80,6 +80,9 @@ _SIGNATURES = {
     "evo_lightning_chunk_bf16": ([_PTR, _I64] + [_PTR] * 6 + [_I64] * 6 + [_PTR], _c.c_int),
     "evo_postnorm_linear_small_m_bf16": ([_PTR] * 6 + [_I64] * 3 + [_F32, _I64] + [_F32] * 2 + [_I64, _PTR], _c.c_int),
     "evo_postnorm_mlp_gate_small_m_bf16": ([_PTR] * 6 + [_I64] * 3 + [_F32, _I64] + [_F32] * 2 + [_I64] * 2 + [_PTR], _c.c_int),
+    "evo_linear_parts": ([_I64] * 3, _c.c_int),
+    "evo_linear_parts_bf16": ([_PTR] * 3 + [_I64] * 4 + [_PTR], _c.c_int),
+    "evo_closing_parts": ([_PTR, _I64] + [_PTR] * 3 + [_I64] * 3 + [_F32] * 3 + [_PTR], _c.c_int),
     "evo_sum_norm": ([_PTR] * 4 + [_I64] * 2 + [_F32] * 3 + [_I64, _PTR], _c.c_int),
     "evo_act_cols": ([_PTR] + [_I64] * 5 + [_PTR], _c.c_int),
     "evo_linear_act_mfma_bf16": ([_PTR] * 4 + [_I64] * 5 + [_PTR], _c.c_int),
@@ -88,6 +91,7 @@ _SIGNATURES = {
     "evo_window_attn": ([_PTR, _I64, _PTR, _PTR, _I64] + [_PTR] * 5 + [_I64] * 10 + [_F32] * 4 + [_I64] * 2 + [_PTR], _c.c_int),
     "evo_heads_prep": ([_PTR, _I64] + [_PTR] * 7 + [_I64] * 9 + [_F32] * 2 + [_I64] * 2 + [_PTR], _c.c_int),
     "evo_heads_decode": ([_PTR, _I64] + [_PTR] * 4 + [_I64] * 9 + [_F32] + [_I64] * 2 + [_PTR], _c.c_int),
+    "evo_heads_decode_whole": ([_PTR, _I64] + [_PTR] * 3 + [_I64] * 8 + [_F32] * 4 + [_PTR], _c.c_int),
     "evo_heads_merge": ([_PTR] * 3 + [_I64] * 5 + [_F32] * 3 + [_I64, _PTR], _c.c_int),
     "evo_rglru_chunk_bf16": ([_PTR, _I64] + [_PTR] * 13 + [_I64] * 6 + [_PTR], _c.c_int),
     "evo_rglru_step_bf16": ([_PTR, _I64] + [_PTR] * 11 + [_I64] * 5 + [_PTR], _c.c_int),
@@ -98,7 +102,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 17         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 18         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):
@@ -427,6 +431,20 @@ class HipOps(MixerOps):
             _check(self.lib.evo_linear_small_m_bf16(x.data_ptr(), w.data_ptr(), _ptr(b), _ptr(res), y.data_ptr(),
                                                     M, N, K, _ptr(ws), 0 if ws is None else ws.numel() * 4, act, _stream()), "evo_linear_small_m_bf16")
         return y
+
+    def linear_parts(self, x, w) -> Optional[torch.Tensor]:
+        """The fp32 parts [parts, M, N] of x @ w^T that `linear` would add and round in a launch of their own (MixerOps.closing_parts_ does both for a closing norm),
+        or None where it takes one sum."""
+        M, K = x.shape
+        if M > 64 or not self._use_small_m(x, w) or (x.data_ptr() | w.data_ptr()) % 16:
+            return None
+        n = self.lib.evo_linear_parts(M, w.shape[0], K)
+        if n <= 0:
+            return None
+        ws = torch.empty(n, M, w.shape[0], dtype=torch.float32, device=x.device)
+        with self._t("gemv"):
+            _check(self.lib.evo_linear_parts_bf16(x.data_ptr(), w.data_ptr(), ws.data_ptr(), M, w.shape[0], K, n, _stream()), "evo_linear_parts_bf16")
+        return ws
 
     @staticmethod
     def mfma_linear_ok(x, w):

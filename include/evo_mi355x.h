@@ -58,8 +58,9 @@ extern "C" {
  *  14: evo_linear_f32 and evo_linear_f32_ws (fp32 dense layers on the bf16 matrix cores) added.
  *  15: evo_dense_plan and evo_linear_f32_plan (the launches of a dense layer) added.
  *  16: evo_hyena_ct_packed and evo_attn_fwd_packed_bf16 (unequal sequences in one launch), evo_copy_rows added.
- *  17: evo_hyena_short added. */
-#define EVO_ABI_VERSION 17
+ *  17: evo_hyena_short added.
+ *  18: evo_linear_parts, evo_linear_parts_bf16, evo_closing_parts and evo_heads_decode_whole added. */
+#define EVO_ABI_VERSION 18
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
@@ -281,6 +282,10 @@ int evo_attn_decode_bf16(const void* q, const void* k, const void* v, void* o,
 int evo_linear_small_m_bf16(const void* x, const void* w, const void* bias, const void* residual, void* y,
                             int64_t M, int64_t N, int64_t K, void* ws, int64_t ws_bytes, int64_t act, void* stream);
 
+/* Parts of K that evo_linear_small_m_bf16 takes for a narrow layer with such a workspace (0: one sum), and the launch that leaves them in ws [parts][M][N]. */
+int evo_linear_parts(int64_t M, int64_t N, int64_t K);
+int evo_linear_parts_bf16(const void* x, const void* w, float* ws, int64_t M, int64_t N, int64_t K, int64_t parts, void* stream);
+
 /* ---- dense layer on the MFMA pipe (prefill) --------------------------------------------------------------
  * replaces the cuBLAS nn.Linear GEMMs of the attention block: Wqkv (with bias) and out_proj (+ residual)
  *                                                     [REF stripedhyena/model.py:52-59 (MHA projections), :84-92]
@@ -454,6 +459,10 @@ int evo_postnorm_residual(const void* y, const void* w, float* x, void* xb, int6
 /* x <- t / sqrt(mean(t^2) + eps) * (w_offset + w) with t = alpha * x + y, in place, and the bf16 copy xb of the new x (NULL: not wanted). */
 int evo_sum_norm(const void* y, const void* w, float* x, void* xb, int64_t M, int64_t D, float alpha, float eps, float w_offset, int64_t f32,
                  void* stream);
+/* evo_sum_norm (`sum`) or evo_postnorm_residual on y = the `parts` planes of evo_linear_parts_bf16, added in their order and rounded to bf16: the same bits as
+ * evo_linear_small_m_bf16 in front of them.  bf16 weights and xb, D % 8 == 0, everything 16-byte aligned. */
+int evo_closing_parts(const float* y, int64_t parts, const void* w, float* x, void* xb, int64_t M, int64_t D, int64_t sum, float alpha, float eps, float w_offset,
+                      void* stream);
 /* out = x / sqrt(mean(x^2) + eps) * (w_offset + w) */
 int evo_rmsnorm_stream(const float* x, const void* w, void* out, int64_t M, int64_t D, float eps, float w_offset, int64_t f32, void* stream);
 /* out = o / sqrt(mean(o^2) + eps) * w * sigmoid(g); g rows have pitch ldg. */
@@ -504,6 +513,9 @@ int evo_heads_prep(void* z, int64_t ld, void* cache, const void* qw, const void*
 int evo_heads_decode(const void* z, int64_t ld, const void* cache, const int64_t* pos, float* part_o, float* part_ml, int64_t B, int64_t H,
                      int64_t kv_heads, int64_t maps, int64_t dim, int64_t dv, int64_t ring, int64_t rs, int64_t n_split, float scale, int64_t f32,
                      int64_t mfma, void* stream);
+/* both in one launch (n_split 1, bf16, dim and dv as the matrix-core kernel takes them, maps x query heads per key head, at most 16 of them, at most 16): -1 for others */
+int evo_heads_decode_whole(const void* z, int64_t ld, const void* cache, const int64_t* pos, void* o, int64_t B, int64_t H, int64_t kv_heads, int64_t maps,
+                           int64_t dim, int64_t dv, int64_t ring, int64_t rs, float scale, float lam, float gain, float eps, void* stream);
 int evo_heads_merge(const float* part_o, const float* part_ml, void* o, int64_t B, int64_t H, int64_t maps, int64_t dv, int64_t n_split, float lam,
                     float gain, float eps, int64_t f32, void* stream);
 

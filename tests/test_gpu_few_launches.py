@@ -1,0 +1,73 @@
+"""Launches that took over what stood behind them in a decode step: closing norms on the parts of a dense layer, decode attention that writes its own result."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV, BF = "cuda", torch.bfloat16
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from evo_amd.ops import default_ops
+    return default_ops()
+
+
+def rnd(*shape, seed, scale=1.0):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randn(*shape, generator=g) * scale)
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 4096, 8192), (24, 1024, 11008), (32, 4096, 16384), (33, 4096, 4096), (64, 1088, 1024), (64, 3072, 8320)])
+@pytest.mark.parametrize("alpha", [None, 2.0])
+def test_closing_norm_of_parts(ops, M, N, K, alpha):
+    """The same bits as the layer with its sum rounded by itself and the closing norm behind it; a norm weight at an odd place takes those."""
+    a, w = rnd(M, K, seed=1).to(DEV, BF), rnd(N, K, seed=2, scale=K ** -0.5).to(DEV, BF)
+    for g in (rnd(N, seed=3).to(DEV, BF), rnd(N + 1, seed=4).to(DEV, BF)[1:]):
+        x, xb = rnd(M, N, seed=5).to(DEV), torch.zeros(M, N, device=DEV, dtype=BF)
+        x2, xb2 = x.clone(), xb.clone()
+        parts = ops.linear_parts(a, w)
+        assert parts is not None and parts.dim() == 3
+        ops.closing_parts_(x, xb, parts, g, alpha, 1e-6, 1.0)
+        y = ops.linear(a, w)
+        if alpha is None:
+            ops.postnorm_residual_(x2, xb2, y, g, 1e-6, 1.0)
+        else:
+            ops.sum_norm_(x2, xb2, y, g, alpha, 1e-6, 1.0)
+        assert torch.equal(x, x2) and torch.equal(xb, xb2)
+
+
+def test_one_sum_stays_one_sum(ops):
+    for M, N, K in ((16, 4096, 16384), (24, 4096, 4096), (65, 4096, 16384), (24, 4160, 16384), (24, 4096, 16416), (24, 512, 16384)):
+        assert ops.linear_parts(torch.zeros(M, K, device=DEV, dtype=BF), torch.zeros(N, K, device=DEV, dtype=BF)) is None
+    assert ops.linear_parts(torch.zeros(24, 8192, device=DEV), torch.zeros(4096, 8192, device=DEV)) is None
+
+
+@pytest.mark.parametrize("H,G,maps,n,dv,ring", [(4, 4, 1, 128, 128, 40), (6, 2, 1, 56, 40, 129), (16, 1, 1, 64, 64, 300), (40, 2, 1, 64, 128, 64), (2, 1, 1, 256, 256, 33),
+                                                (8, 1, 2, 64, 64, 200), (3, 3, 2, 56, 112, 500), (2, 2, 2, 128, 256, 130)])
+def test_decode_attention_in_one_launch(ops, H, G, maps, n, dv, ring, monkeypatch):
+    """Against one part and its merge: the same sums, divided and combined in another order, rounded once (bf16: half an ulp is 2^-9 of the value, two roundings of
+    nearly the same number differ by at most one ulp, 2^-7 of the smaller one)."""
+    B = 5
+    z = rnd(B, (H + G) * maps * n + G * dv, seed=1, scale=2.0).to(DEV, BF)
+    z = torch.nn.functional.pad(z, (0, -z.shape[1] % 8))
+    cache = rnd(B, ring, (G * (maps * n + dv) + 7) // 8 * 8, seed=2).to(DEV, BF)
+    pos = torch.tensor([0, 31, 32, ring - 1, 3 * ring], device=DEV)
+    args = (z, cache, pos, H, G, maps, n, dv, n ** -0.5, 0.45, 0.7, 1e-4)
+    want = ops.heads_decode(*args, n_split=1).float()
+    whole = ops.heads_whole_ok
+    assert whole(160, ring, H // G, maps, n, dv, z, cache) and not whole(79, ring, H // G, maps, n, dv, z, cache)
+    names = []
+    real = ops._t
+    monkeypatch.setattr(ops, "heads_whole_ok", lambda *a: True, raising=False)
+    monkeypatch.setattr(ops, "_t", lambda name: (names.append(name), real(name))[1], raising=False)
+    got = ops.heads_decode(*args).float()
+    assert names == ["heads_decode_whole"]
+    assert bool(((got - want).abs() <= want.abs() * 2.0 ** -7 + 1e-5).all()), (got - want).abs().max().item()
+    assert (got != want).float().mean() < 0.02
+
+
+def test_what_one_launch_refuses(ops):
+    z, cache, pos = torch.zeros(2, 17 * 2 * 64, device=DEV, dtype=BF), torch.zeros(2, 16, 192, device=DEV, dtype=BF), torch.zeros(2, dtype=torch.int64, device=DEV)
+    o = torch.zeros(2, 17 * 64, device=DEV, dtype=BF)
+    assert not ops.heads_whole_ok(1000, 16, 17, 2, 64, 64, z, cache)
+    assert ops.lib.evo_heads_decode_whole(z.data_ptr(), z.stride(0), cache.data_ptr(), pos.data_ptr(), o.data_ptr(), 2, 17, 1, 2, 64, 64, 16, 192, 0.1, 0.5, 0.5, 1e-5, None) == -1
