@@ -534,6 +534,30 @@ extern "C" int evo_advance_positions(int64_t* pos, int64_t n, int64_t last, void
     return evo_launch_status();
 }
 
+// The end of a pooled step in one launch: the logits of every slot in fp32, and the positions one further (two launches of 4 to 5 us were a hundredth of a step).
+template <bool VEC>
+__global__ __launch_bounds__(256) void step_out_kernel(const uint16_t* __restrict__ logits, float* __restrict__ out, int64_t n, int64_t* __restrict__ pos, int64_t S, int64_t last) {
+    if (blockIdx.x == 0)
+        for (int64_t i = threadIdx.x; i < S; i += 256) pos[i] = pos[i] + 1 < last ? pos[i] + 1 : last;
+    const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
+    if (VEC) {
+        if (e >= n) return;
+        const uint4 q = *(const uint4*)(logits + e);
+        *(float4*)(out + e) = make_float4(bf_lo(q.x), bf_hi(q.x), bf_lo(q.y), bf_hi(q.y));
+        *(float4*)(out + e + 4) = make_float4(bf_lo(q.z), bf_hi(q.z), bf_lo(q.w), bf_hi(q.w));
+    } else
+        for (int64_t k = e; k < n && k < e + 8; ++k) out[k] = bf_to_f(logits[k]);
+}
+
+extern "C" int evo_step_out(const void* logits, float* out, int64_t n, int64_t* pos, int64_t S, int64_t last, void* stream) {
+    if (!logits || !out || !pos || n <= 0 || S <= 0 || last < 0 || n > (1ll << 40)) return -1;
+    const dim3 grid((unsigned)((n + 2047) / 2048)), block(256);
+    if (n % 8 == 0 && (((uintptr_t)logits | (uintptr_t)out) & 15) == 0)
+        hipLaunchKernelGGL(step_out_kernel<true>, grid, block, 0, (hipStream_t)stream, (const uint16_t*)logits, out, n, pos, S, last);
+    else hipLaunchKernelGGL(step_out_kernel<false>, grid, block, 0, (hipStream_t)stream, (const uint16_t*)logits, out, n, pos, S, last);
+    return evo_launch_status();
+}
+
 extern "C" int evo_abi_version(void) { return EVO_ABI_VERSION; }
 
 // ---- many small copies in one launch: piece i is `rows` rows of `bytes` (a multiple of 16) at their pitches.  Bound by the bytes; a launch of its own per piece costs

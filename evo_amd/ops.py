@@ -51,6 +51,7 @@ _SIGNATURES = {
     "evo_mlp_gate_mfma_nf_bf16": ([_PTR] * 4 + [_I64] * 3 + [_PTR], _c.c_int),
     "evo_put_tokens": ([_PTR, _I64, _PTR, _PTR, _I64, _PTR], _c.c_int),
     "evo_advance_positions": ([_PTR, _I64, _I64, _PTR], _c.c_int),
+    "evo_step_out": ([_PTR] * 2 + [_I64, _PTR] + [_I64] * 2 + [_PTR], _c.c_int),
     "evo_copy_rows": ([_PTR, _I64, _PTR], _c.c_int),
     "evo_hyena_ct_packed": ([_PTR] * 9 + [_I64] * 5 + [_PTR], _c.c_int),
     "evo_attn_fwd_packed_bf16": ([_PTR] * 4 + [_I64] * 8 + [_PTR] * 2 + [_I64, _PTR, _F32, _PTR, _PTR], _c.c_int),
@@ -102,7 +103,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 18         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 19         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):
@@ -504,6 +505,14 @@ class HipOps(MixerOps):
         """pos = min(pos + 1, last), in place."""
         self._need(pos, torch.int64, "advance_positions pos")
         _check(self.lib.evo_advance_positions(pos.data_ptr(), pos.numel(), int(last), _stream()), "evo_advance_positions")
+
+    def step_out(self, logits: torch.Tensor, pos: torch.Tensor, last: int) -> torch.Tensor:
+        """logits.float(), and advance_positions, in one launch."""
+        self._need(logits, torch.bfloat16, "step_out logits")
+        self._need(pos, torch.int64, "step_out pos")
+        out = torch.empty(logits.shape, dtype=torch.float32, device=logits.device)
+        _check(self.lib.evo_step_out(logits.data_ptr(), out.data_ptr(), logits.numel(), pos.data_ptr(), pos.numel(), int(last), _stream()), "evo_step_out")
+        return out
 
     def copy_rows(self, pairs) -> None:
         """dst.copy_(src) for each pair of tensors of one shape and type, many to a launch.  Pieces that are not whole rows of 16 bytes are copied by torch."""

@@ -145,6 +145,15 @@ class DecodePool:
         finally:
             mha.pos_tensor = None
 
+    def _finish(self, logits: torch.Tensor) -> torch.Tensor:
+        """The step's logits in fp32, a tensor of their own; the positions move on."""
+        ops = self.model.ops
+        if hasattr(ops, "step_out") and logits.is_cuda and logits.dtype == torch.bfloat16 and logits.is_contiguous() and self.pos.is_contiguous():
+            return ops.step_out(logits, self.pos, self.capacity - 1)
+        out = logits.float()
+        self._next_positions()
+        return out
+
     def _next_positions(self) -> None:
         """(free slots drift harmlessly; a full live slot grows the caches first)"""
         if self.pos.is_cuda and hasattr(self.model.ops, "advance_positions"):
@@ -158,25 +167,21 @@ class DecodePool:
         self.stats["steps"] += 1
         with torch.inference_mode():
             if not self.use_graph or not self.model._graph_shapes_ok(self.n_slots):
-                out = self._step_eager().float()
-                self._next_positions()
-                return out
+                return self._finish(self._step_eager())
             if self._graph is None:
                 # The first step runs eagerly (it also warms the library handles and the M = S GEMM choices) and IS the
                 # step: the caches advance in place, so nothing may run twice.  Capture records without executing.
-                first = self._step_eager().float()
-                self._next_positions()
+                first = self._finish(self._step_eager())
                 torch.cuda.synchronize(self.device)
                 self.model._graph_prepare(self.n_slots, self.device)
                 g = torch.cuda.CUDAGraph()
                 with torch.cuda.graph(g):
                     out = self._step_eager()
-                    self._next_positions()
                 self._graph = (g, out)
                 return first
             g, out = self._graph
             g.replay()
-            return out.float()
+            return self._finish(out)
 
     # ------------------------------------------------------------------ the job
     def generate(self, prompts: Sequence[str], n_tokens: int = 1000, n_sample_per_prompt: int = 1,

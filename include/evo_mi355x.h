@@ -59,12 +59,14 @@ extern "C" {
  *  15: evo_dense_plan and evo_linear_f32_plan (the launches of a dense layer) added.
  *  16: evo_hyena_ct_packed and evo_attn_fwd_packed_bf16 (unequal sequences in one launch), evo_copy_rows added.
  *  17: evo_hyena_short added.
- *  18: evo_linear_parts, evo_linear_parts_bf16, evo_closing_parts and evo_heads_decode_whole added. */
-#define EVO_ABI_VERSION 18
+ *  18: evo_linear_parts, evo_linear_parts_bf16, evo_closing_parts and evo_heads_decode_whole added.
+ *  19: evo_step_out added. */
+#define EVO_ABI_VERSION 19
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
- * evo_advance_positions: pos[i] = min(pos[i] + 1, last). */
+ * evo_advance_positions: pos[i] = min(pos[i] + 1, last).  evo_step_out: that, and out [n] fp32 = the n bf16 logits. */
+int evo_step_out(const void* logits, float* out, int64_t n, int64_t* pos, int64_t S, int64_t last, void* stream);
 int evo_put_tokens(int64_t* ids, int64_t S, const int64_t* slots, const int64_t* tokens, int64_t n, void* stream);
 int evo_advance_positions(int64_t* pos, int64_t n, int64_t last, void* stream);
 /* n copies between device buffers that don't overlap, 64 to a launch: `pieces` (HOST) holds six values of each -- destination, source, rows, bytes per row (a multiple of

@@ -71,3 +71,13 @@ def test_what_one_launch_refuses(ops):
     o = torch.zeros(2, 17 * 64, device=DEV, dtype=BF)
     assert not ops.heads_whole_ok(1000, 16, 17, 2, 64, 64, z, cache)
     assert ops.lib.evo_heads_decode_whole(z.data_ptr(), z.stride(0), cache.data_ptr(), pos.data_ptr(), o.data_ptr(), 2, 17, 1, 2, 64, 64, 16, 192, 0.1, 0.5, 0.5, 1e-5, None) == -1
+
+
+@pytest.mark.parametrize("S,V", [(1, 512), (3, 37), (300, 512), (16, 1001)])
+def test_end_of_a_step(ops, S, V):
+    logits = rnd(S, V, seed=1).to(DEV, BF)
+    pos = torch.arange(S, device=DEV) + 95
+    out = ops.step_out(logits, pos, 99)
+    assert torch.equal(out, logits.float()) and torch.equal(pos.cpu(), (torch.arange(S) + 96).clamp(max=99))
+    odd = logits.reshape(-1)[1:]                                  # (not 16-byte aligned)
+    assert torch.equal(ops.step_out(odd, pos, 99), odd.float())
