@@ -34,7 +34,9 @@ __global__ __launch_bounds__(4 * DV, 2) void lightning_chunk_kernel(LightArgs a)
     uint16_t* const p_lo = k_rows + LC * PT;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c16 = lane & 15, g = lane >> 4;
-    const int seg = blockIdx.x % a.n_seg, vt = blockIdx.x / a.n_seg, h = blockIdx.y, b = blockIdx.z;
+    // (heads first: workgroup i runs on XCD i % 8, and a short sequence's later segments are empty -- segments first, five sequences of 3,000 and 300 tokens in
+    //  segments of 384 had all of their short ones on one XCD: 204 -> 102 us)
+    const int h = blockIdx.x % a.H, seg = blockIdx.x / a.H % a.n_seg, vt = blockIdx.x / a.H / a.n_seg, b = blockIdx.z;
     const int dk = a.dk, dv = a.dv, v0 = vt * DV;
     const int row0 = a.cu[b] + seg * a.seg_len;
     int len = a.cu[b + 1] - row0;
@@ -304,7 +306,7 @@ __global__ __launch_bounds__(256) void lightning_scan_kernel(LightArgs a) {
 
 template <int DK, int DV, bool VEC>
 static void chunk_launch(LightArgs a, int64_t B, hipStream_t s) {
-    const dim3 grid((unsigned)(a.n_seg * ((a.dv + DV - 1) / DV)), (unsigned)a.H, (unsigned)B), block(4 * DV);
+    const dim3 grid((unsigned)(a.H * a.n_seg * ((a.dv + DV - 1) / DV)), 1, (unsigned)B), block(4 * DV);
     if (a.n_seg > 1) {
         hipLaunchKernelGGL((lightning_chunk_kernel<DK, DV, false, VEC>), grid, block, 0, s, a);
         hipLaunchKernelGGL(lightning_scan_kernel, dim3((unsigned)((a.dk * a.dv + 255) / 256), (unsigned)a.H, (unsigned)B), dim3(256), 0, s, a);
@@ -319,6 +321,7 @@ extern "C" int evo_lightning_chunk_bf16(const void* z, int64_t ld, void* o, floa
     if (max_len <= 0 || max_len > 0x7fffffff || seg_len <= 0 || seg_len % LC != 0 || ld < H * (2 * dk + dv) || (resume && !state)) return -1;
     LightArgs a = {z, o, state, log2_decay, cu, resume, seg, ld, (int)H, (int)dk, (int)dv, (int)((max_len + seg_len - 1) / seg_len), (int)seg_len, 0};
     if (a.n_seg > 1 && !seg) return -1;
+    if (H * a.n_seg * ((dv + 63) / 64) > 0x7fffffff) return -1;
     if (a.n_seg == 1) a.seg = nullptr;
     hipStream_t s = (hipStream_t)stream;
     const bool vec = dk % 8 == 0 && dv % 8 == 0 && ld % 8 == 0 && ((uintptr_t)z & 15) == 0;

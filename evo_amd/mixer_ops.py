@@ -3,6 +3,7 @@ attention, decayed linear attention, latent attention, gated linear recurrence. 
 arithmetic is fp32."""
 from __future__ import annotations
 
+import functools
 from dataclasses import dataclass
 from typing import List, Optional, Sequence, Tuple
 
@@ -310,7 +311,7 @@ class MixerOps:
             self._call("evo_lightning_recurrent", z.data_ptr(), z.stride(0), o.data_ptr(), sp, dp, cu, resume, B, heads, dk, dv, 0, f32)
             return o
         L = max(batch.lens)
-        seg_len = seg_len or self.lightning_segment(L, B * heads * ((dv + 127) // 128))
+        seg_len = seg_len or self.lightning_segment(tuple(sorted(batch.lens)), heads * ((dv + 127) // 128), dk * dv)
         n_seg = (L + seg_len - 1) // seg_len
         seg = torch.empty(B, n_seg, heads, dk, dv, dtype=torch.float32, device=z.device) if n_seg > 1 else None
         self._call("evo_lightning_chunk_bf16", z.data_ptr(), z.stride(0), o.data_ptr(), sp, None if seg is None else seg.data_ptr(),
@@ -318,11 +319,25 @@ class MixerOps:
         return o
 
     @staticmethod
-    def lightning_segment(L: int, columns: int, target: int = 256) -> int:
-        """Tokens per segment: one segment when (sequence, head) pairs alone fill the chip, else enough segments for a workgroup per CU,
-        of at least four chunks each (a segment's state costs as much traffic as ~dk + dv tokens)."""
-        want = max(1, (target + columns - 1) // columns)
-        return max(4 * LC, (L + want * LC - 1) // (want * LC) * LC)
+    @functools.lru_cache(maxsize=64)
+    def lightning_segment(lens: Tuple[int, ...], columns: int, state: int, cus: int = 256) -> int:
+        """Tokens per segment (whole chunks): the least of what the launches cost, for `columns` (head, value tile) pairs a sequence and `state` elements of one.
+        A workgroup a CU takes 5.4 us a chunk; cut sequences need another pass for their segments' states (2.2 us a chunk) and every segment's state crosses memory four
+        times.  (us at 32 heads of 128 x 128, the rule before, segments for a workgroup per CU -> this one.  6 sequences of 1,459 to 2,500 tokens: 295 in
+        segments of 1,280, 214 uncut; 5,000 and 300: 148 -> 101 in segments of 768; 3,000 and four times 300: 177 -> 102; 1,500 and three times 100: 98 -> 57;
+        4,000 twice 133 as before, 311 uncut.)"""
+        longest = max(lens)
+        chunks = sum((n + LC - 1) // LC for n in lens) * columns / cus
+        best = None
+        for seg in sorted({max(4 * LC, (longest + n * LC - 1) // (n * LC) * LC) for n in range(1, 33)}, reverse=True):
+            n_wg = sum((n + seg - 1) // seg for n in lens) * columns
+            top = min(seg, (longest + LC - 1) // LC * LC) / LC
+            us = 6.0 + 5.3 * (top if n_wg <= cus else max(top, chunks + top / 2))
+            if seg < longest:
+                us += 3.0 + 2.2 * max(top, chunks) + n_wg * state * 16 / 4.5e6
+            if best is None or us < best[0]:
+                best = (us, seg)
+        return best[1]
 
     # ---- latent attention -----------------------------------------------------------------------------------------------
     @staticmethod
