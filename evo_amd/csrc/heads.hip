@@ -208,6 +208,8 @@ struct HDecArgs {
 // use repeat the last of them, one line for the whole wave, and are masked.  (They were clamped to the ring only: a wave's request behind its last slots
 // read 32 KB of unused cache.  16 heads of two maps, 640 slots, in a graph with the merge: 16 / 24 sequences of up to 600 tokens 38.2 / 55.2 -> 32.9 / 45.8 us;
 // 8 key heads with 4 query heads each, 1,028 slots: 8 / 24 sequences of up to 600 12.4 / 21.2 -> 11.0 / 16.5.)
+// Heads are the grid's fastest index: workgroup i runs on XCD i % 8, and behind a short sequence's tokens whole parts have nothing to do (parts first, 16 heads of
+// two maps in 5 to 8 parts: 1 / 3 sequences of up to 300 16.6 / 17.7 -> 14.1 / 15.0; key heads of four queries alike).
 // KS: 32-wide steps of a key, NG: 32-wide groups of a value, MAPS: maps per head ([map 1 | map 2] in keys and queries).
 template <int KS, int NG, int MAPS>
 __global__ __launch_bounds__(256) void heads_decode_kernel(HDecArgs a) {
@@ -216,7 +218,7 @@ __global__ __launch_bounds__(256) void heads_decode_kernel(HDecArgs a) {
     __shared__ float ml[4][MAPS][16][2];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c16 = lane & 15, g = lane >> 4;
-    const int split = blockIdx.x, hk = blockIdx.y / a.n_qb, qb = blockIdx.y % a.n_qb, b = blockIdx.z;
+    const int split = blockIdx.y, hk = blockIdx.x / a.n_qb, qb = blockIdx.x % a.n_qb, b = blockIdx.z;
     const int Q = a.H / a.G, nq = Q - 16 * qb < 16 ? Q - 16 * qb : 16;    // query heads of this workgroup
     const int h0 = hk * Q + 16 * qb;
     const int dim = a.dim, dv = a.dv;
@@ -527,7 +529,7 @@ static int heads_decode(void* o, float lam, float gain, float eps, const void* z
     hipStream_t s = (hipStream_t)stream;
     if (!f32 && mfma && dim % 8 == 0 && dv % 8 == 0 && ld % 8 == 0 && rs % 8 == 0 && dim <= (maps == 2 ? 128 : 256) && dv <= 256 &&
         (((uintptr_t)z | (uintptr_t)cache | (uintptr_t)part_o | (uintptr_t)o) & 15) == 0 && (!o || maps * (Q < 16 ? Q : 16) <= 16)) {
-        const dim3 grid((unsigned)n_split, (unsigned)(kv_heads * a.n_qb), (unsigned)B);
+        const dim3 grid((unsigned)(kv_heads * a.n_qb), (unsigned)n_split, (unsigned)B);
 #define HD(KS, NG, MAPS)                                                                                                   \
     do {                                                                                                                   \
         constexpr int tiles = 4 * 32 * (32 * NG + 8) * 2, meet = (MAPS == 1 ? 4 : MAPS) * 16 * (32 * NG + 4) * 4, bytes = tiles > meet ? tiles : meet;   \
