@@ -22,6 +22,18 @@ struct WinArgs {
 // as S^T = K Q^T (a lane holds one query's scores of four keys per 16-key block), so the softmax needs two cross-lane steps, the
 // probabilities are the next product's operand as they stand (split key order), and O^T = V^T P^T is rescaled by one factor per lane.
 // VEC: every row piece of eight elements is 16-byte aligned.
+// Work item of this workgroup, (sequence, head, query block) in one number.  The query blocks of a (sequence, head) share most of their keys, as do the heads of a
+// key head: they stay on one XCD (block b runs on XCD b % 8).  Where the key heads are a multiple of eight, every XCD gets as many of every sequence; a contiguous run
+// of items per XCD, as for other numbers, gives one XCD the longest sequence.  us, runs -> key heads over the XCDs, latent attention of 32 heads / 8 key heads of four
+// queries in a window of 1,024 / 16 heads of two maps: 6 sequences of 1,459 to 2,500 tokens 355 / 317 / 509 -> 304 / 268 / 369; 24 of 180 to 600 202 / 185 / 196
+// -> 122 / 107 / 126; 3,000 and three times 300 265 / 265 / 442 -> 96 / 94 / 139; one of 8,190 214 / 196 / 705 -> 205 / 191 / 704.
+__device__ __forceinline__ int work_item(const WinArgs& a) {
+    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3, G = a.H / a.grp;
+    if (G & 7) return xcd * (int)(gridDim.x >> 3) + j;
+    const int each = a.grp * a.n_qb;                             // items of a key head: they stay together
+    return (j / each * 8 + xcd) * each + j % each;
+}
+
 // MAPS == 2: the two column blocks of a wave are the two maps of the same 16 queries -- rows of q and k hold [map 1 | map 2] per head --, the
 // values are shared, and the maps meet in the epilogue.  KEEP: a.keep is not zero.  NW: waves
 // (8: wide heads, whose sums leave a SIMD room for two waves of one workgroup only).  NH: a tile's keys are gone through in NH parts (2: half
@@ -36,10 +48,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void window_attn_kernel(WinArgs a, i
     __shared__ __attribute__((aligned(16))) uint16_t k_rows[64 * PR], v_cols[DVP * PT];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c16 = lane & 15, g = lane >> 4;
-    // the query blocks of a (sequence, head) share most of their keys: consecutive work items stay on one XCD (block b runs on XCD b % 8)
-    const int per_xcd = gridDim.x >> 3;
-    const int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    const int qb = item % a.n_qb, h = item / a.n_qb % a.H, b = item / a.n_qb / a.H;
+    const int item = work_item(a), qb = item % a.n_qb, h = item / a.n_qb % a.H, b = item / a.n_qb / a.H;
     if (b >= B) return;                                          // (the grid is rounded up to a multiple of 8)
     const int q0 = a.cu_q[b], nq = a.cu_q[b + 1] - q0, k0 = a.cu_k[b], nk = a.cu_k[b + 1] - k0;
     if (qb * QB >= nq) return;
@@ -330,10 +339,7 @@ __global__ __launch_bounds__(512, 2) void window_tile_kernel(WinArgs a, int B) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c16 = lane & 15, g = lane >> 4;
     const int map = MAPS == 2 ? wave >> 2 : 0, grp = MAPS == 2 ? wave & 3 : wave;      // (waves w and w + 4 share a SIMD)
-    // the query blocks of a (sequence, head) share most of their keys: consecutive work items stay on one XCD (block b runs on XCD b % 8)
-    const int per_xcd = gridDim.x >> 3;
-    const int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    const int qb = a.n_qb - 1 - item % a.n_qb, h = item / a.n_qb % a.H, b = item / a.n_qb / a.H;
+    const int item = work_item(a), qb = a.n_qb - 1 - item % a.n_qb, h = item / a.n_qb % a.H, b = item / a.n_qb / a.H;
     if (b >= B) return;                                          // (the grid is rounded up to a multiple of 8)
     const int q0 = a.cu_q[b], nq = a.cu_q[b + 1] - q0, k0 = a.cu_k[b], nk = a.cu_k[b + 1] - k0;
     const int off = nk - nq;                                     // key index of query 0
