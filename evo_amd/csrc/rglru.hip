@@ -58,7 +58,8 @@ __global__ __launch_bounds__(64 * NW) void rglru_chunk_kernel(RgArgs a) {
     uint16_t* const yo = (uint16_t*)(cb + KP);                   // [2][RT][YP] y, replaced by the outputs where they are made
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c16 = lane & 15, g = lane >> 4;
-    const int cg = blockIdx.x % a.n_cg, seg = blockIdx.x / a.n_cg, n = blockIdx.y, b = blockIdx.z;
+    // (blocks first: workgroup i runs on XCD i % 8, and a short sequence's later segments are empty)
+    const int n = blockIdx.x % a.nb, cg = blockIdx.x / a.nb % a.n_cg, seg = blockIdx.x / a.nb / a.n_cg, b = blockIdx.z;
     const int bs = a.bs, W = a.W, row0 = a.cu[b];
     const int len_all = a.cu[b + 1] - row0, s_lo = seg * a.seg_len;
     int s_hi = s_lo + a.seg_len;
@@ -303,11 +304,11 @@ extern "C" int evo_rglru_chunk_bf16(const void* z, int64_t ld, void* o, float* s
     if (n_seg > 1 && !seg) return -1;
     const int nw = bs <= 64 ? 4 : 8;
     const int64_t n_cg = (bs + 16 * nw - 1) / (16 * nw);
-    if (n_seg * n_cg > 0x7fffffff) return -1;
+    if (n_seg * n_cg * nb > 0x7fffffff) return -1;
     RgArgs a = {z, nullptr, o, state, n_seg > 1 ? seg : nullptr, conv, conv_b, ra, ra_b, ri, ri_b, decay, pos, nullptr, cu, resume,
                 ld, (int)W, (int)nb, (int)bs, (int)taps, (int)n_seg, (int)seg_len, (int)n_cg, 0, (int)B};
     hipStream_t s = (hipStream_t)stream;
-    const dim3 grid((unsigned)(n_seg * n_cg), (unsigned)nb, (unsigned)B);
+    const dim3 grid((unsigned)(n_seg * n_cg * nb), 1, (unsigned)B);
 #define RC(KS, NW)                                                                                                         \
     do {                                                                                                                   \
         constexpr int bytes = 2 * RT * (32 * KS + 8) * 2 + 3 * 32 * KS * 4 + 2 * RT * (16 * NW + 8) * 2;                                       \

@@ -326,17 +326,23 @@ class MixerOps:
         times.  (us at 32 heads of 128 x 128, the rule before, segments for a workgroup per CU -> this one.  6 sequences of 1,459 to 2,500 tokens: 295 in
         segments of 1,280, 214 uncut; 5,000 and 300: 148 -> 101 in segments of 768; 3,000 and four times 300: 177 -> 102; 1,500 and three times 100: 98 -> 57;
         4,000 twice 133 as before, 311 uncut.)"""
+        def us(seg, span, busy, n_wg):
+            return 6.0 + 5.3 * span + (3.0 + 2.2 * busy + n_wg * state * 16 / 4.5e6 if seg < max(lens) else 0.0)
+        return MixerOps.cheapest_segment(lens, columns, us, cus)
+
+    @staticmethod
+    def cheapest_segment(lens: Tuple[int, ...], columns: int, us, cus: int) -> int:
+        """The segment length, whole chunks of a share of the longest sequence, of least us(segment, chunks of the launch's end, chunks at the most of a CU where two
+        workgroups share one, workgroups).  Several rounds of workgroups end half a workgroup late."""
         longest = max(lens)
         chunks = sum((n + LC - 1) // LC for n in lens) * columns / cus
         best = None
         for seg in sorted({max(4 * LC, (longest + n * LC - 1) // (n * LC) * LC) for n in range(1, 33)}, reverse=True):
             n_wg = sum((n + seg - 1) // seg for n in lens) * columns
             top = min(seg, (longest + LC - 1) // LC * LC) / LC
-            us = 6.0 + 5.3 * (top if n_wg <= cus else max(top, chunks + top / 2))
-            if seg < longest:
-                us += 3.0 + 2.2 * max(top, chunks) + n_wg * state * 16 / 4.5e6
-            if best is None or us < best[0]:
-                best = (us, seg)
+            t = us(seg, top if n_wg <= cus else max(top, chunks + top / 2), max(top, chunks), n_wg)
+            if best is None or t < best[0]:
+                best = (t, seg)
         return best[1]
 
     # ---- latent attention -----------------------------------------------------------------------------------------------
@@ -498,11 +504,15 @@ class MixerOps:
         return dtype == torch.bfloat16 and bs % 8 == 0 and bs <= 384 and taps <= 4
 
     @staticmethod
-    def rglru_segment(L: int, walkers: int, target: int = 256) -> int:
-        """Tokens per segment: one segment while the walking workgroups fill most of the chip, else as many as give every CU one (a segment's
-        state costs another pass over its gates)."""
-        want = max(1, target // walkers) if walkers <= target * 5 // 8 else 1
-        return max(256, (L + want * 64 - 1) // (want * 64) * 64) if want > 1 else (L + 63) // 64 * 64
+    @functools.lru_cache(maxsize=64)
+    def rglru_segment(lens: Tuple[int, ...], columns: int, cus: int = 256) -> int:
+        """Tokens per segment, as lightning_segment: 4.4 us a chunk, and 3.9 for its gates once more where sequences are cut; the carries walk the segments one by one.
+        (us at 4,096 channels in 16 blocks, the rule before, from the longest sequence alone -> this one.  4,000, 1,000 and 2,000 tokens 262 -> 144 in segments of
+        1,024; 3,000 and three times 300 202 -> 113; 2,000 and three times 500 144 -> 89; 5,000 and 300 173 -> 116; 500 52 -> 44 uncut; one of 8,190 152 -> 145 and
+        six of 1,459 to 2,500, uncut, 187 -> 186 are cut as they were.)"""
+        def us(seg, span, busy, n_wg):
+            return 8.0 + 4.4 * span + (3.0 + 3.9 * span + 2.5 * ((max(lens) + seg - 1) // seg) if seg < max(lens) else 0.0)
+        return MixerOps.cheapest_segment(lens, columns, us, cus)
 
     def rglru(self, z: torch.Tensor, in_b: Optional[torch.Tensor], act: bool, W: int, conv: torch.Tensor, conv_b: torch.Tensor, ra, ra_b, ri, ri_b,
               decay: torch.Tensor, batch: TokenBatch, state: Optional[torch.Tensor] = None, seg_len: Optional[int] = None) -> torch.Tensor:
@@ -532,7 +542,7 @@ class MixerOps:
         if fast and in_b is None and not act:
             assert sum(batch.lens) == M
             L = max(batch.lens)
-            seg_len = seg_len or self.rglru_segment(L, B * nb * ((bs + 127) // 128))
+            seg_len = seg_len or self.rglru_segment(tuple(sorted(batch.lens)), nb * ((bs + 127) // 128))
             n_seg = (L + seg_len - 1) // seg_len
             seg = torch.empty(B, n_seg, 2, W, dtype=torch.float32, device=z.device) if n_seg > 1 else None
             self._call("evo_rglru_chunk_bf16", *head, o.data_ptr(), sp, None if seg is None else seg.data_ptr(), *w, cu, resume, B, W, nb, taps, L, seg_len)

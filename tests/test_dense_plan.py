@@ -49,14 +49,16 @@ def test_segments_for_a_number_of_waves():
         assert evo_ops.pick_segment_length(B, T, H) == evo_ops.pick_segment_length(B, T, H, 4096)
 
 
-def test_segments_of_decayed_linear_attention():
+def test_segments_of_recurrent_mixers():
     """Whole chunks, at least four; uncut where sequences and heads fill the chip; one long sequence in as many segments as there are CUs for it."""
     from evo_amd.mixer_ops import MixerOps
     plan = MixerOps.lightning_segment
     for lens in ((1,), (64,), (257,), (500,), (8190,), (131072,), (300, 5000), (1000, 2000, 3000), (4000, 4000), (1,) * 100, (1459, 1667, 1875, 2084, 2292, 2500)):
         for columns in (1, 8, 32, 64):
-            seg = plan(lens, columns, 128 * 128)
-            assert seg % 64 == 0 and seg >= 256 and (seg == 256 or seg < max(lens) + 64)
+            for seg in (plan(lens, columns, 128 * 128), MixerOps.rglru_segment(lens, columns)):
+                assert seg % 64 == 0 and seg >= 256 and (seg == 256 or seg < max(lens) + 64)
     assert plan((1459, 1667, 1875, 2084, 2292, 2500), 32, 16384) >= 2500
     assert plan((1000,) * 8, 32, 16384) >= 1000
     assert plan((4000, 4000), 32, 16384) == 1024 and plan((8190,), 32, 16384) == 1024
+    plan = MixerOps.rglru_segment
+    assert plan((1459, 1667, 1875, 2084, 2292, 2500), 32) >= 2500 and plan((500,), 32) == 512 and plan((8190,), 32) == 1024 and plan((1000, 2000, 4000), 32) == 1024
