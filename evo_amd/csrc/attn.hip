@@ -629,11 +629,11 @@ __device__ __forceinline__ float attn_dot8(const uint4& a, const uint4& b) {
     return acc;
 }
 
-__global__ __launch_bounds__(256) void attn_decode_stream_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256) void attn_decode_stream_kernel(AttnArgs a, int heads_first) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int head = blockIdx.y, bat = blockIdx.z;
-    const int split = blockIdx.x * 4 + wave;                 // one split of the key range per wave
+    const int head = heads_first ? blockIdx.x : blockIdx.y, bat = blockIdx.z;
+    const int split = (heads_first ? blockIdx.y : blockIdx.x) * 4 + wave;        // one split of the key range per wave
     int64_t n_keys = a.Tk;
     if (a.dyn_pos) n_keys = a.dyn_pos[bat] + 1;              // the query at position p sees keys [0, p]
     const int nblk = (int)((n_keys + 63) >> 6);              // split s takes blocks s, s + n_splits, ...: the waves resident at one
@@ -933,7 +933,15 @@ extern "C" int evo_attn_decode_bf16(const void* q, const void* k, const void* v,
     // EVO_ATTN_DECODE_FORM=0 keeps the MFMA split kernel (measurement builds); default: the streaming kernel, one split per wave
     static const int form = [] { const char* e = getenv("EVO_ATTN_DECODE_FORM"); return e ? atoi(e) : 1; }();
     if (form != 0 && Tk * k_st * 2 < 0xffffffffll && Tk * v_st * 2 < 0xffffffffll)
-        hipLaunchKernelGGL(attn_decode_stream_kernel, dim3((unsigned)((n_splits + 3) / 4), (unsigned)H, (unsigned)B), dim3(256), 0, s, a);
+    {
+        // Workgroup i runs on XCD i % 8: with an even number of them per head, parts first ties a part to some XCDs, and the parts differ by a block of keys (us,
+        // parts -> heads first: 8 of them, 1 x 3,020 / 8,000 / 30,000 keys 16.1 / 30.1 / 95.5 -> 15.7 / 28.9 / 90; 16 rows of 340 to 1,100 keys in a cache of
+        // 2,048 66.8 -> 47.3; 6 of them, 4 x 1,200 19.2 -> 18.3).  An odd number spreads by itself, and parts of a head next to each other read
+        // neighbouring rows (5, 16 rows of up to 1,100: 44.1 against 46.4).
+        const unsigned parts = (unsigned)((n_splits + 3) / 4);
+        const int heads_first = parts % 2 == 0;
+        hipLaunchKernelGGL(attn_decode_stream_kernel, heads_first ? dim3((unsigned)H, parts, (unsigned)B) : dim3(parts, (unsigned)H, (unsigned)B), dim3(256), 0, s, a, heads_first);
+    }
     else
         hipLaunchKernelGGL(attn_fwd_kernel<true>, dim3((unsigned)n_splits, (unsigned)H, (unsigned)B), dim3(256), 0, s, a);
     hipLaunchKernelGGL(attn_decode_combine_kernel, dim3((unsigned)H, (unsigned)B), dim3(512), 0, s, part_o, part_ml,
