@@ -252,6 +252,10 @@ class HipOps(MixerOps):
         self.attn_gemm_mfma = True
         # prefill attention on the 64-rows-per-wave kernel of round 5 (csrc/attn_w64.hip); False: the 8-wave kernel of rounds 2-4 (bench A/B leg)
         self.attn_w64 = True
+        # ... from this many keys on.  Its blocks of 256 rows and its pass over V cost more than its inner loop saves below: us, 64 rows a wave : 8 waves, 32 heads,
+        # 1 x 161 20.3 : 12.6, 1 x 1,000 45.9 : 37.1, 8 x 900 199 : 149, 32 x 500 306 : 214, 8 x 3,000 934 : 809, 1 x 3,000 131 : 127, 1 x 4,000 200 : 206, 8 x 6,000
+        # 2,699 : 2,701, 1 x 8,000 547 : 571.  (Off fp64 by 2.3e-3 and 1.8e-3 to 2.0e-3, the rounding of the result included.)
+        self.attn_w64_from = 3500
         # round 5: the RMSNorm passes of prefill-sized batches ride in the epilogues of the dense layers around them (csrc/gemm.hip, NF;
         # False = the separate rmsnorm launches: bench.py's A/B leg, the routing test)
         self.fuse_norm = True
@@ -1095,8 +1099,8 @@ class HipOps(MixerOps):
             self._need(out, torch.bfloat16, "attention out")
             assert tuple(out.shape) == (B, Tq, H, hd)
         o = torch.empty(B, Tq, H, hd, dtype=torch.bfloat16, device=q.device) if out is None else out
-        # query ranges longer than one 128-row block: the 64-rows-per-wave kernel, which reads V^T from a workspace its pre-pass fills
-        vt = torch.empty(B, H, hd, (Tk + 63) // 64 * 64, dtype=torch.bfloat16, device=q.device) if (Tq > 128 and self.attn_w64) else None
+        # query ranges longer than one 128-row block on many keys: the 64-rows-per-wave kernel, which reads V^T from a workspace its pre-pass fills
+        vt = torch.empty(B, H, hd, (Tk + 63) // 64 * 64, dtype=torch.bfloat16, device=q.device) if (Tq > 128 and Tk >= self.attn_w64_from and self.attn_w64) else None
         with self._t("attn_fwd"):
             _check(self.lib.evo_attn_fwd_causal_bf16(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), B, H, Tq, Tk, int(q_pos0),

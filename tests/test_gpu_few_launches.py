@@ -81,3 +81,18 @@ def test_end_of_a_step(ops, S, V):
     assert torch.equal(out, logits.float()) and torch.equal(pos.cpu(), (torch.arange(S) + 96).clamp(max=99))
     odd = logits.reshape(-1)[1:]                                  # (not 16-byte aligned)
     assert torch.equal(ops.step_out(odd, pos, 99), odd.float())
+
+
+@pytest.mark.parametrize("first", [0, 1 << 30])
+@pytest.mark.parametrize("B,Tq,past", [(1, 129, 0), (2, 255, 0), (1, 256, 0), (3, 257, 0), (1, 513, 0), (2, 140, 300), (1, 300, 1)])
+def test_both_prompt_attention_kernels(ops, B, Tq, past, first, monkeypatch):
+    """The kernel of many keys and that of few, either side of `attn_w64_from`, against fp64.  Both round the probabilities and the result to bf16: 2^-9 of it each, and
+    the largest error by an outlier's share of a row (measured 2.3e-3 of the norm)."""
+    monkeypatch.setattr(ops, "attn_w64_from", first, raising=False)
+    H, Tk = 4, Tq + past
+    q, k, v = (rnd(B, n, H, 128, seed=i, scale=s).to(DEV, BF) for i, (n, s) in enumerate(((Tq, 0.2), (Tk, 1.0), (Tk, 1.0))))
+    seen = torch.arange(Tk, device=DEV)[None] <= torch.arange(Tq, device=DEV)[:, None] + past
+    s = (q.double().transpose(1, 2) @ k.double().permute(0, 2, 3, 1).contiguous()) * 0.6931471805599453                    # (scores are exponents of two)
+    want = (s.masked_fill(~seen, float("-inf")).softmax(-1) @ v.double().transpose(1, 2).contiguous()).transpose(1, 2)
+    got = ops.attention(q, k, v, past, prescaled=True).double()
+    assert (got - want).norm() / want.norm() < 4e-3
