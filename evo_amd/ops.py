@@ -926,7 +926,7 @@ class HipOps(MixerOps):
         with self._t("gemm_mfma"):
             self._dense_layer(0, x, w_folded, y, Mm, N, K, b=b, rs=rstd)
         if M > Mm:
-            y[Mm:] = self.norm_linear(x[Mm:], scale, eps, w, b)
+            y[Mm:] = self.norm_linear(x[Mm:], scale, eps, w, b, one_launch=True)
         return y
 
     def mlp_gate_rs(self, x: torch.Tensor, rstd: torch.Tensor, w12g_folded: torch.Tensor, w12: torch.Tensor, scale: torch.Tensor,
@@ -940,7 +940,7 @@ class HipOps(MixerOps):
         with self._t("gemm_gate"):
             self._dense_layer(1, x, w12g_folded, a, Mm, 2 * I, K, rs=rstd)
         if M > Mm:
-            a[Mm:] = self.mlp_gate(x[Mm:], w12, scale, eps, w12g=None if w12 is not None else w12g_folded)
+            a[Mm:] = self.mlp_gate(x[Mm:], w12, scale, eps, w12g=None if w12 is not None else w12g_folded, one_launch=True)
         return a
 
     def zt_stream_rows_ok(self, B: int, T: int) -> bool:
@@ -973,7 +973,7 @@ class HipOps(MixerOps):
             return zt
         zt[-1].zero_()
         x_tail = x.view(B, T, K)[:, Tm:].reshape(B * r, K).contiguous()                           # (a copy of B r <= 16 rows)
-        z_tail = self.norm_linear(x_tail, scale, eps, w, b)                             # [B r, N]
+        z_tail = self.norm_linear(x_tail, scale, eps, w, b, one_launch=True)                             # [B r, N]
         zt[-1].view(N, 32, 8)[:, :B, :r] = z_tail.view(B, r, N).permute(2, 0, 1)        # position Mp + 8 b + j
         return zt
 
@@ -1031,11 +1031,12 @@ class HipOps(MixerOps):
         return y
 
     def hyena_decode_fused(self, x, norm_scale, eps, proj_w, proj_b, fir_state, iir_state, fir_w, fir_b, poles,
-                           residues, dskip, n_heads: int) -> torch.Tensor:
+                           residues, dskip, n_heads: int, one_launch: bool = False) -> torch.Tensor:
         """One decode token through pre-norm + projections + FIR/modal step + gate in ONE launch (M = batch <= 4, or <= 6 at D = 4096: 23.5 us
-        against 23 in three launches, 26.8 against 23 at 8); states are updated in place.  Falls back to the separate kernels otherwise."""
+        against 23 in three launches, 26.8 against 23 at 8); states are updated in place.  Falls back to the separate kernels otherwise.  `one_launch`: up to 8 rows
+        (the last tokens of a scoring batch, whose launches are few beside the batch's own)."""
         M, D = x.shape
-        ok = ((1 <= M <= 4 or (M <= 6 and D == 4096)) and x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and proj_w.is_contiguous()
+        ok = ((1 <= M <= 4 or (M <= (8 if one_launch else 6) and D == 4096)) and x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and proj_w.is_contiguous()
               and proj_w.dtype == torch.bfloat16 and norm_scale.dtype == torch.bfloat16 and proj_b is not None
               and fir_state.dtype == torch.bfloat16 and fir_state.is_contiguous() and fir_state.shape[0] == M
               and iir_state.dtype == torch.complex64 and iir_state.is_contiguous() and iir_state.shape[0] == M
@@ -1174,12 +1175,12 @@ class HipOps(MixerOps):
         return o
 
     def norm_linear(self, x: torch.Tensor, scale: torch.Tensor, eps: float, w: torch.Tensor,
-                    b: Optional[torch.Tensor] = None, mfma: bool = False) -> torch.Tensor:
-        """linear(rmsnorm(x) * scale, w, b).  Decode-sized batches (M <= 4) with a wide layer take ONE weight-streaming
-        launch that rebuilds the normalised row on the fly; everything else is the two kernels."""
+                    b: Optional[torch.Tensor] = None, mfma: bool = False, one_launch: bool = False) -> torch.Tensor:
+        """linear(rmsnorm(x) * scale, w, b).  Decode-sized batches (M <= 4; `one_launch`, the rows that a scoring batch leaves over: <= 8 at K = 4,096) with a wide
+        layer take ONE weight-streaming launch that rebuilds the normalised row on the fly; everything else is the two kernels."""
         M, K = x.shape
         # (five rows and more: the norm's own launch and the matrix cores' form are ahead -- 20.5 -> 19.3 us at 5 rows and 12,288 x 4,096, 26.5 -> 19.3 at 8)
-        if (1 <= M <= 4 and w.shape[0] > 4096 and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+        if ((1 <= M <= 4 or (one_launch and M <= 8 and K == 4096)) and w.shape[0] > 4096 and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
                 and scale.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous() and scale.is_contiguous()
                 and K % 8 == 0):
             y = torch.empty(M, w.shape[0], dtype=torch.bfloat16, device=x.device)
@@ -1210,14 +1211,14 @@ class HipOps(MixerOps):
                 and M * K * 2 < 0xffffffff and w12g.shape[0] * K * 2 < 0xffffffff)
 
     def mlp_gate(self, x: torch.Tensor, w12: Optional[torch.Tensor], norm_scale: Optional[torch.Tensor] = None,
-                 eps: float = 0.0, w12g: Optional[torch.Tensor] = None, act: str = "gelu") -> torch.Tensor:
+                 eps: float = 0.0, w12g: Optional[torch.Tensor] = None, act: str = "gelu", one_launch: bool = False) -> torch.Tensor:
         """a [M, I] = gelu(x' @ W1^T) * (x' @ W2^T), w12 = [W1; W2] ([2I, K]); x' = x, or rmsnorm(x) * norm_scale when
         `norm_scale` is given.  Decode-sized batches (M <= 4) take ONE weight-streaming launch; prefill-sized ones the
         matrix-core dense layer with the gate in its epilogue when `w12g` (pack_gate_weights(w12)) is given -- the
         [M, 2 I] intermediate is never written; everything else is (norm,) dense layer and gate kernel.
         `w12 = None` (round 6, one weight set: StripedHyena.fold_norms_): only the regrouped copy w12g exists -- the weight-streaming
         launches read it in that row order (`grouped`), the unfused fallback un-groups the dense layer's columns.
-        `act="silu"`: SiLU in the place of the GELU (without a folded norm)."""
+        `act="silu"`: SiLU in the place of the GELU (without a folded norm).  `one_launch`: up to 8 rows norm for themselves, as in norm_linear."""
         M, K = x.shape
         code = {"gelu": 0, "silu": 1}[act]
         if code and norm_scale is not None:
@@ -1237,7 +1238,7 @@ class HipOps(MixerOps):
             return a
         ok_mem = (x.is_cuda and x.dtype == torch.bfloat16 and wsrc.dtype == torch.bfloat16 and x.is_contiguous() and wsrc.is_contiguous()
                   and (norm_scale is None or (norm_scale.dtype == torch.bfloat16 and norm_scale.is_contiguous())))
-        if (self.gate_small_m_mfma and (5 <= M <= 64 or (3 <= M <= 4 and I * K >= 1 << 24)) and K % 128 == 0 and I % 32 == 0 and ok_mem
+        if (self.gate_small_m_mfma and not (one_launch and M <= 8 and K == 4096 and norm_scale is not None) and (5 <= M <= 64 or (3 <= M <= 4 and I * K >= 1 << 24)) and K % 128 == 0 and I % 32 == 0 and ok_mem
                 and (x.data_ptr() | wsrc.data_ptr()) % 16 == 0):
             # 3-64 rows on the MFMA weight-streaming form with the gate in its epilogue (csrc/gemv.hip skinny_ring_kernel); the norm as its own small pass in
             # front (us at I = 11,008, K = 4,096, against the dot2 launch that norms for itself: 30.7 : 31.2 at 3 rows, 30.7 : 32.1 at 4, 30.7 : 45.0 at 8)

@@ -594,7 +594,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
                 fir = zt[ix["zblk"], :, 256 - K1:].contiguous()                         # [B, 3 D, 2]: steps Tm - 2, Tm - 1 of every row, oldest first
                 x_tail = x2d.view(B, T, D)[:, Tm].contiguous()                          # the raw stream's rows (the launch norms them itself)
                 y_tail = ops.hyena_decode_fused(x_tail, blk.pre_norm.scale, self.eps, blk.projections.weight, blk.projections.bias, fir, state,
-                                                f._fir_w, f.short_filter_bias, f._poles, f._residues, f.D, H)
+                                                f._fir_w, f.short_filter_bias, f._poles, f._residues, f.D, H, one_launch=True)
                 yb[ix["yblk"], :, ix["yrow"], :] = y_tail.view(B, D // 16, 16)          # rows b T + Tm of the blocked y
             elif cache is None:
                 y = ops.hyena_ct(zt, B, T, f._fir_w, f.short_filter_bias, table, H, y_blk=yb)
