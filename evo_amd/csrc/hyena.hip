@@ -502,10 +502,11 @@ HY_PRAGMA_UNROLL(HY_UNROLL_A)
 #define SH_PITCH 100
 #define SH_E 129                             // states of a segment: 16 channels x 8 modes, one more for the banks
 
+template <bool MASK>
 __global__ __launch_bounds__(512, 4) void hyena_short_kernel(const unsigned char* __restrict__ z, const unsigned char* __restrict__ z_halo, const uint16_t* __restrict__ fir_w,
                                                              const uint16_t* __restrict__ fir_b, const float2* __restrict__ poles, const float2* __restrict__ residues,
                                                              const uint16_t* __restrict__ dskip, const float2* __restrict__ s0, float2* __restrict__ s_final,
-                                                             unsigned char* __restrict__ y, int T, int D, int C) {
+                                                             unsigned char* __restrict__ y, const uint8_t* __restrict__ mask, int T, int D, int C) {
     extern __shared__ __attribute__((aligned(16))) unsigned char sh[];
     float2* E = (float2*)sh;                                     // [32][SH_E] end states, then entering states
     unsigned char* zt = sh + 32 * SH_E * 8;                      // [T + 2][SH_PITCH]: x2 | x1 | v of the 16 channels, two rows of history in front
@@ -536,6 +537,7 @@ __global__ __launch_bounds__(512, 4) void hyena_short_kernel(const unsigned char
 #pragma unroll
     for (int s = 0; s < NS; ++s) { const float2 p = poles[(int64_t)d * NS + s]; pr[s] = p.x; pi[s] = p.y; }
     const int t0 = seg * C, n = T - t0 < C ? T - t0 : C;         // (n <= 0: nothing)
+    const uint8_t* mrow = MASK ? mask + (int64_t)b * T : nullptr;
     const unsigned char* q = zt + (t0 < T ? t0 : 0) * SH_PITCH + ch * 2;          // row t0 - 2
     auto at = [&](int k, int g) __attribute__((always_inline)) { return bf_to_f(*(const uint16_t*)(q + k * SH_PITCH + g * 32)); };
     auto fir = [&](int g, float a, float b1, float c) __attribute__((always_inline)) { return fmaf(w[g][2], c, fmaf(w[g][1], b1, fmaf(w[g][0], a, wb[g]))); };
@@ -551,7 +553,9 @@ __global__ __launch_bounds__(512, 4) void hyena_short_kernel(const unsigned char
         float a1 = m2[1], av = m2[2], b1 = m1[1], bv = m1[2];
         for (int k = 0; k < n; ++k) {
             const float c1 = at(k + 2, 1), cv = at(k + 2, 2);
-            const float x = fir(1, a1, b1, c1) * fir(2, av, bv, cv);
+            float f1 = fir(1, a1, b1, c1);
+            if (MASK && !mrow[t0 + k]) f1 = 0.f;                 // (a padded position injects nothing, and its y is zero)
+            const float x = f1 * fir(2, av, bv, cv);
 #pragma unroll
             for (int s = 0; s < NS; ++s) {
                 const float t = fmaf(-pi[s], si[s], x), u = pi[s] * sr[s];
@@ -604,6 +608,7 @@ __global__ __launch_bounds__(512, 4) void hyena_short_kernel(const unsigned char
             float c[3], f[3];
 #pragma unroll
             for (int g = 0; g < 3; ++g) { c[g] = at(k + 2, g); f[g] = fir(g, m2[g], m1[g], c[g]); m2[g] = m1[g]; m1[g] = c[g]; }
+            if (MASK && !mrow[t0 + k]) f[0] = f[1] = 0.f;
             const float x = f[1] * f[2];
             float acc[2] = {0.f, 0.f};
 #pragma unroll
@@ -714,15 +719,21 @@ extern "C" int evo_hyena_carry_scan(float* agg, const float* poles, const float*
 }
 
 extern "C" int evo_hyena_short(const void* z, const void* z_halo, const void* fir_w, const void* fir_b, const float* poles, const float* residues, const void* dskip,
-                               const float* s0, float* s_final, void* y, int64_t B, int64_t T, int64_t D, int64_t n_heads, void* stream) {
+                               const float* s0, float* s_final, void* y, const uint8_t* mask, int64_t B, int64_t T, int64_t D, int64_t n_heads, void* stream) {
     if (hyena_check(B, T, D, n_heads, CH) || T > SH_T || B > 65535 || D > 0xfffff) return -1;
     if (((uintptr_t)z | (uintptr_t)z_halo | (uintptr_t)y) & 15) return -1;
     const int C = (int)((T + 31) / 32) | 1;                      // (odd: the banks)
     const size_t lds = 32 * SH_E * 8 + (size_t)(T + 2) * SH_PITCH;                // (<= 133 KB)
-    if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)hyena_short_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 32 * SH_E * 8 + (SH_T + 2) * SH_PITCH);
-    hipLaunchKernelGGL(hyena_short_kernel, dim3((unsigned)(D / 16), (unsigned)B), dim3(512), lds, (hipStream_t)stream, (const unsigned char*)z,
-                       (const unsigned char*)z_halo, (const uint16_t*)fir_w, (const uint16_t*)fir_b, (const float2*)poles, (const float2*)residues, (const uint16_t*)dskip,
-                       (const float2*)s0, (float2*)s_final, (unsigned char*)y, (int)T, (int)D, C);
+#define EVO_HS(MASK)                                                                                                       \
+    do {                                                                                                                   \
+        if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)hyena_short_kernel<MASK>, hipFuncAttributeMaxDynamicSharedMemorySize, 32 * SH_E * 8 + (SH_T + 2) * SH_PITCH); \
+        hipLaunchKernelGGL(hyena_short_kernel<MASK>, dim3((unsigned)(D / 16), (unsigned)B), dim3(512), lds, (hipStream_t)stream, (const unsigned char*)z, \
+                           (const unsigned char*)z_halo, (const uint16_t*)fir_w, (const uint16_t*)fir_b, (const float2*)poles, (const float2*)residues, \
+                           (const uint16_t*)dskip, (const float2*)s0, (float2*)s_final, (unsigned char*)y, mask, (int)T, (int)D, C); \
+    } while (0)
+    if (mask) EVO_HS(true);
+    else EVO_HS(false);
+#undef EVO_HS
     return evo_launch_status();
 }
 

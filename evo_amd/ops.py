@@ -30,7 +30,7 @@ _SIGNATURES = {
     "evo_abi_version": ([], _c.c_int),
     "evo_embed_bf16": ([_PTR, _PTR, _PTR, _I64, _I64, _I64, _PTR, _PTR], _c.c_int),
     "evo_rmsnorm_bf16": ([_PTR, _PTR, _PTR, _PTR, _I64, _I64, _F32, _PTR], _c.c_int),
-    "evo_hyena_short": ([_PTR] * 10 + [_I64] * 4 + [_PTR], _c.c_int),
+    "evo_hyena_short": ([_PTR] * 11 + [_I64] * 4 + [_PTR], _c.c_int),
     "evo_hyena_seg_state": ([_PTR, _PTR, _PTR, _PTR, _PTR, _PTR, _PTR, _I64, _I64, _I64, _I64, _I64, _PTR], _c.c_int),
     "evo_hyena_carry_scan": ([_PTR, _PTR, _PTR, _PTR, _I64, _I64, _I64, _I64, _PTR], _c.c_int),
     "evo_hyena_carry_add": ([_PTR, _PTR, _PTR, _I64, _I64, _I64, _I64, _PTR], _c.c_int),
@@ -103,7 +103,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 19         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 20         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):
@@ -765,8 +765,9 @@ class HipOps(MixerOps):
     @staticmethod
     def _hyena_short_ok(B, T, z, z_halo, poles, residues) -> bool:
         """One launch (csrc/hyena.hip hyena_short_kernel) for the rows and alignments that it takes, while its 3.5 + B (0.9 + 0.033 T) us at 4,096 channels, every
-        batch row a round of workgroups, are less than the 21 + 0.021 B T us of the three launches (12 x 41 positions: 33 against 36 us; 32 x 41: 78 against 45; 18 x 5: 28 against 21)."""
-        return (T <= 1024 and B * (T + 75) <= 1450 and (B <= 8 or T >= 41) and z.data_ptr() % 16 == 0 and (z_halo is None or z_halo.data_ptr() % 16 == 0) and poles.data_ptr() % 8 == 0
+        batch row a round of workgroups, are less than the 21 + 0.021 B T us of the three launches (12 x 41 positions: 33 against 36 us; 32 x 41: 78 against 45; 18 x 5: 28 against 21).
+        From 1,024 positions on a row's bits are the same in every batch (row groups of a pass): those stay with the three launches."""
+        return (B * T < 1024 and B * (T + 75) <= 1450 and (B <= 8 or T >= 41) and z.data_ptr() % 16 == 0 and (z_halo is None or z_halo.data_ptr() % 16 == 0) and poles.data_ptr() % 8 == 0
                 and residues.data_ptr() % 8 == 0)
 
     def hyena_prefill(self, z: torch.Tensor, fir_w: torch.Tensor, fir_b: torch.Tensor, poles: torch.Tensor,
@@ -795,12 +796,12 @@ class HipOps(MixerOps):
         if s0 is not None:
             s0r = torch.view_as_real(s0.to(torch.complex64).contiguous())
             assert s0r.shape == (B, D, 8, 2)
-        if mask is None and not seg_len and not self.seg_len_override and self._hyena_short_ok(B, T, z, z_halo, poles, residues):
+        if not seg_len and not self.seg_len_override and self._hyena_short_ok(B, T, z, z_halo, poles, residues):
             y = torch.empty(B, T, D, dtype=torch.bfloat16, device=z.device)
             s_final = torch.empty(B, D, 8, 2, dtype=torch.float32, device=z.device) if want_state else None
             with self._t("hyena_short"):
                 _check(self.lib.evo_hyena_short(z.data_ptr(), _ptr(z_halo), fir_w.data_ptr(), fir_b.data_ptr(), poles.data_ptr(), residues.data_ptr(), dskip.data_ptr(),
-                                                _ptr(s0r), _ptr(s_final), y.data_ptr(), B, T, D, n_heads, _stream()), "evo_hyena_short")
+                                                _ptr(s0r), _ptr(s_final), y.data_ptr(), _ptr(mask), B, T, D, n_heads, _stream()), "evo_hyena_short")
             self.last_hyena_io = {"short": (z.numel() + y.numel()) * 2}
             return y, torch.view_as_complex(s_final) if want_state else None
         C = seg_len or self.seg_len_override or pick_segment_length(B, T, n_heads)

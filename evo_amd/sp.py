@@ -347,7 +347,7 @@ class SequenceParallelScorer:
                 if ztm:
                     # (norm + projection of the 2 B halo rows: ONE weight-streaming launch up to 8 rows at D = 4096, else norm + launch)
                     xh = x2d.view(B, Tloc, D)[:, -2:, :].reshape(B * 2, D).contiguous()
-                    parts = [ops.norm_linear(xh[i:i + 8], blk.pre_norm.scale, m.eps, w_p, b_p) for i in range(0, 2 * B, 8)]   # (8 rows per fused launch)
+                    parts = [ops.norm_linear(xh[i:i + 8], blk.pre_norm.scale, m.eps, w_p, b_p, one_launch=True) for i in range(0, 2 * B, 8)]   # (8 rows per fused launch)
                     tail = (parts[0] if len(parts) == 1 else torch.cat(parts, 0)).view(B, 2, 3 * D)
                 else:
                     tail = ops.linear(n1.view(B, Tloc, D)[:, -2:, :].reshape(B * 2, D), w_p, b_p).view(B, 2, 3 * D)

@@ -60,8 +60,9 @@ extern "C" {
  *  16: evo_hyena_ct_packed and evo_attn_fwd_packed_bf16 (unequal sequences in one launch), evo_copy_rows added.
  *  17: evo_hyena_short added.
  *  18: evo_linear_parts, evo_linear_parts_bf16, evo_closing_parts and evo_heads_decode_whole added.
- *  19: evo_step_out added. */
-#define EVO_ABI_VERSION 19
+ *  19: evo_step_out added.
+ *  20: evo_hyena_short gained `mask`. */
+#define EVO_ABI_VERSION 20
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
@@ -123,7 +124,7 @@ int evo_hyena_carry_scan(float* agg, const float* poles, const float* s0, float*
                          int64_t B, int64_t T, int64_t D, int64_t seg_len, void* stream);
 /* the three launches in one, for rows of up to 1,024 positions; z, z_halo and y 16-byte aligned, poles, residues, s0 and s_final 8-byte */
 int evo_hyena_short(const void* z, const void* z_halo, const void* fir_w, const void* fir_b, const float* poles, const float* residues, const void* dskip,
-                    const float* s0, float* s_final, void* y, int64_t B, int64_t T, int64_t D, int64_t n_heads, void* stream);
+                    const float* s0, float* s_final, void* y, const uint8_t* mask, int64_t B, int64_t T, int64_t D, int64_t n_heads, void* stream);
 /* sequence-parallel fix-up (new; the reference has no multi-GPU path): `agg` already scanned with a zero
  * carry-in gets p^(k*seg_len) * s0 added to segment k once the state s0 entering this shard is known. */
 int evo_hyena_carry_add(float* agg, const float* poles, const float* s0,
