@@ -275,7 +275,7 @@ class HipOps(MixerOps):
         self.timer: Optional[KernelTimer] = None
         self.validate_ids = os.environ.get("EVO_AMD_VALIDATE_IDS", "1") != "0"   # one 4-byte D2H read per forward
         # the single-pass matrix-core Hyena operator on CHANNEL-MAJOR z^T (csrc/hyena_ct.hip: the projection launched with swapped
-        # operands, no input window in LDS); False: the modal three-launch kernels (the tests' yardstick, padding masks, tiny inputs)
+        # operands, no input window in LDS); False: the modal kernels (the tests' yardstick, padding masks, tiny inputs: one launch below 1,024 positions, else three)
         self.hyena_mfma = True
         self.hyena_ct_flag = True
         self._xpad = threading.local()  # per thread: the zero-initialised padded input of the swapped-operand projection (_xpad_buffer)
@@ -776,8 +776,8 @@ class HipOps(MixerOps):
                       want_state: bool = False, seg_len: Optional[int] = None,
                       mask: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
         """z [B,T,3D] bf16 -> y [B,T,D] bf16 (+ complex64 state [B,D,8] after the last token).  `mask` [B,T] (bool /
-        uint8, 1 = token) is upstream's padding_mask: padded positions get a zero FIR output.  The three-launch MODAL form
-        (csrc/hyena.hip: segment states, carry scan, apply) on token-major z: padding masks, inputs the single-pass kernel's
+        uint8, 1 = token) is upstream's padding_mask: padded positions get a zero FIR output.  The MODAL form
+        (csrc/hyena.hip: segment states, carry scan, apply; one launch for short rows, _hyena_short_ok) on token-major z: padding masks, inputs the single-pass kernel's
         contract excludes, and the yardstick the tests hold hyena_ct against."""
         if mask is not None:
             mask = mask.to(device=z.device, dtype=torch.uint8).contiguous()
