@@ -1036,6 +1036,11 @@ typedef uint32_t rg_u32x4 __attribute__((ext_vector_type(4)));
 #define RG_WAIT(N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory")
 #define RG_ROWB 256                          // bytes of a row's piece of a chunk
 #define RG_NONE 0xf0000000u                  // behind every buffer: nothing is read, zero arrives
+// first of the columns of workgroup `b` (b = groups: behind the last): floor(b cols / groups).  b * more has 32 bits up to 65,536 workgroups only (6.3 M columns).
+static __host__ __device__ __forceinline__ uint32_t ring_edge(uint32_t cols, uint32_t groups, uint32_t b) {
+    const uint32_t each = cols / groups, more = cols % groups;
+    return b * each + (groups <= 0x10000 ? b * more / groups : (uint32_t)((uint64_t)b * more / groups));
+}
 template <int XR, int T, int NB, int MODE>
 __global__ __launch_bounds__(64 * T) void skinny_ring_kernel(const unsigned char* __restrict__ x, const unsigned char* __restrict__ w, const uint16_t* __restrict__ bias,
                                                              const uint16_t* res, uint16_t* y, int M, int N, int K, int act, int layout, float* __restrict__ ws) {   // res may alias y
@@ -1047,8 +1052,7 @@ __global__ __launch_bounds__(64 * T) void skinny_ring_kernel(const unsigned char
     const int r16 = lane & 15, kb = lane >> 4;
     const uint32_t rowb = (uint32_t)K * 2;
     const int cols = MODE == 1 ? N >> 1 : N;                     // result columns; this workgroup's: lo .. hi - 1
-    const uint32_t each = (uint32_t)cols / gridDim.x, more = (uint32_t)cols % gridDim.x;
-    const int lo = (int)(blockIdx.x * each + blockIdx.x * more / gridDim.x), hi = (int)((blockIdx.x + 1) * each + (blockIdx.x + 1) * more / gridDim.x);
+    const int lo = (int)ring_edge(cols, gridDim.x, blockIdx.x), hi = (int)ring_edge(cols, gridDim.x, blockIdx.x + 1);
     // weight rows: four requests of four rows; of MODE 1 the first two from W1, the others from W2
     rg_u32x4 rw[2];
     uint32_t ow[PW];
@@ -1076,7 +1080,7 @@ __global__ __launch_bounds__(64 * T) void skinny_ring_kernel(const unsigned char
     }
     // bias and residual values of this lane's results, requested ahead of everything (from places that are there, and looked at behind the last product: no wait here)
     uint32_t pb[4], pr[MODE == 0 ? MT : 1][4];
-    const int n0 = lo + 16 * wave + 4 * kb;
+    const uint32_t n0 = (uint32_t)lo + 16 * wave + 4 * kb;       // (may be behind 2^31)
     if (MODE == 0 && bias) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) pb[r] = bias[n0 + r < N ? n0 + r : N - 1];
@@ -1216,17 +1220,35 @@ static int ring_go(dim3 grid, const void* x, const void* w, const void* bias, co
                        (const uint16_t*)res, (uint16_t*)y, (int)M, (int)N, (int)K, act, layout, ws);
     return evo_launch_status();
 }
+static int64_t ring_groups(int64_t N) {
+    const int64_t rounds = (N + 256 * 96 - 1) / (256 * 96), share = (N + 31) / 32;
+    return share < 256 ? share : 256 * rounds;
+}
+static int ring_waves(int64_t N) {
+    const int64_t groups = ring_groups(N), rows = (N + groups - 1) / groups;
+    return rows <= 32 ? 2 : rows <= 48 ? 3 : rows <= 64 ? 4 : 6;
+}
+// What workgroup `block` of N weight rows (gated: N / 2 result columns) takes: out = workgroups, its first column, the next one's, columns that it has room for
+extern "C" int evo_linear_ring_share(int64_t N, int64_t gated, int64_t block, int64_t* out) {
+    if (!out || N <= 0 || N > 0x7fffffff - 16 || (gated && N % 2)) return -1;
+    const int64_t groups = ring_groups(N), cols = gated ? N / 2 : N;
+    if (block < 0 || block >= groups) return -1;
+    out[0] = groups;
+    out[1] = ring_edge((uint32_t)cols, (uint32_t)groups, (uint32_t)block);
+    out[2] = ring_edge((uint32_t)cols, (uint32_t)groups, (uint32_t)block + 1);
+    out[3] = (gated ? 8 : 16) * ring_waves(N);
+    return 0;
+}
 // parts > 0: MODE 2, 64 rows a workgroup (N a multiple of 64)
 template <int MODE>
 static int ring_launch(const void* x, const void* w, const void* bias, const void* res, void* y, int64_t M, int64_t N, int64_t K, int act, int layout, float* ws, int parts,
                        hipStream_t s) {
-    const int64_t rounds = (N + 256 * 96 - 1) / (256 * 96), share = (N + 31) / 32;
-    const int64_t groups = parts ? N / 64 : (share < 256 ? share : 256 * rounds), rows = (N + groups - 1) / groups;
-    const dim3 grid((unsigned)groups, (unsigned)(parts ? parts : 1));
+    const int waves = ring_waves(N);
+    const dim3 grid((unsigned)(parts ? N / 64 : ring_groups(N)), (unsigned)(parts ? parts : 1));
 #define EVO_RG(XR, T) ring_go<XR, T, MODE>(grid, x, w, bias, res, y, M, N, K, act, layout, ws, s)
 #define EVO_RG1(T) (M <= 16 ? EVO_RG(16, T) : M <= 32 ? EVO_RG(32, T) : EVO_RG(64, T))
     if (MODE == 2) return EVO_RG1(4);
-    return rows <= 32 ? EVO_RG1(2) : rows <= 48 ? EVO_RG1(3) : rows <= 64 ? EVO_RG1(4) : EVO_RG1(6);
+    return waves == 2 ? EVO_RG1(2) : waves == 3 ? EVO_RG1(3) : waves == 4 ? EVO_RG1(4) : EVO_RG1(6);
 #undef EVO_RG1
 #undef EVO_RG
 }

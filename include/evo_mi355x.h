@@ -61,8 +61,9 @@ extern "C" {
  *  17: evo_hyena_short added.
  *  18: evo_linear_parts, evo_linear_parts_bf16, evo_closing_parts and evo_heads_decode_whole added.
  *  19: evo_step_out added.
- *  20: evo_hyena_short gained `mask`. */
-#define EVO_ABI_VERSION 20
+ *  20: evo_hyena_short gained `mask`.
+ *  21: evo_linear_ring_share added. */
+#define EVO_ABI_VERSION 21
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
@@ -284,6 +285,10 @@ int evo_attn_decode_bf16(const void* q, const void* k, const void* v, void* o,
  * act 3: the square of relu before the rounding (0: none). */
 int evo_linear_small_m_bf16(const void* x, const void* w, const void* bias, const void* residual, void* y,
                             int64_t M, int64_t N, int64_t K, void* ws, int64_t ws_bytes, int64_t act, void* stream);
+
+/* Columns per workgroup of that launch on a wide layer (N > 4096, K % 128 == 0) and of the gated one (`gated`: N = 2 I, I columns): out [4] = workgroups, first column of workgroup
+ * `block`, first behind it, columns that a workgroup has room for.  On the host, no launch; -1: no such workgroup. */
+int evo_linear_ring_share(int64_t N, int64_t gated, int64_t block, int64_t* out);
 
 /* Parts of K that evo_linear_small_m_bf16 takes for a narrow layer with such a workspace (0: one sum), and the launch that leaves them in ws [parts][M][N]. */
 int evo_linear_parts(int64_t M, int64_t N, int64_t K);
