@@ -152,7 +152,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
     else if (ODD && MODE == 1) src = n0 >> 6 << 6;               // (whole groups of 32 rows of each half)
     const uint64_t xa = (uint64_t)a.x + (XB ? (m0 & ~(int64_t)127) : m0) * kb, wa = (uint64_t)a.w + src * kb;
     const int64_t x_left = a.M - (XB ? (m0 & ~(int64_t)127) : m0), x_most = XB ? 256 : BM, x_ok = x_left < x_most ? x_left : x_most;    // (blocked X: whole blocks, M % 128 == 0)
-    const int64_t w_ok = plain_gate || w_rows - src < BN || (ODD && MODE == 1) ? w_rows - src : BN;
+    // (ODD, gated: 48 columns from the first or the middle one of a group of 32 on lie in two groups; [W1; W2] as it is: both halves, below 4 GiB)
+    const int64_t w_left = w_rows - src, w_most = ODD && MODE == 1 ? 128 : BN, w_ok = plain_gate || w_left < w_most ? w_left : w_most;
     const t_u32x4 rx = {(uint32_t)xa, (uint32_t)(xa >> 32) & 0xffffu, (uint32_t)(x_ok * kb), 0x00020000u};
     const t_u32x4 rw = {(uint32_t)wa, (uint32_t)(wa >> 32) & 0xffffu, (uint32_t)(w_ok * kb), 0x00020000u};
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;

@@ -283,3 +283,27 @@ def test_tiles_of_odd_widths(M, N, K, tile):
         err = (y[:M].double() - want).abs()
         assert bool((err <= want.abs() * 2.0 ** -8 + (4e-3 if act else 1e-3)).all()), err.max().item()                          # (as test_plain, test_activation)
         assert bool((y[M:] == 7).all())
+
+
+def test_gate_on_a_weight_of_more_than_4_gib():
+    """Tiles of 96 gated columns, the grouped weight's bytes more than 32 bits hold: every tile finds its rows (22,016 x 98,304; the tiles see 128 rows of it at a time)."""
+    from evo_amd.ops import _stream
+    import ctypes
+    ops = _ops()
+    M, N, K = 161, 22016, 98304
+    out = (ctypes.c_int64 * 14)()
+    assert ops.lib.evo_dense_plan(1, 0, M, N, K, ctypes.cast(out, ctypes.c_void_p)) == 1 and tuple(out[2:4]) == (192, 96)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    w = torch.empty(N // 64, 64, K, device="cuda", dtype=torch.bfloat16)          # (blocks of 32 rows of each half)
+    for part in w.split(16):
+        part.copy_(torch.randn(part.shape, device="cuda", generator=g) * K ** -0.5)
+    y = torch.full((M, N // 2), 7.0, device="cuda", dtype=torch.bfloat16)
+    assert ops.lib.evo_dense_bf16(1, 0, 0, x.data_ptr(), w.data_ptr(), None, None, y.data_ptr(), None, None, 0, M, N, K, 0, 0, 0, 0, None, 0, _stream()) == 0
+    xd = x.double()
+    for i, part in enumerate(w.split(8)):
+        z = (xd @ part.reshape(-1, K).double().T).bfloat16().double().view(M, -1, 2, 32)
+        z1, z2 = z[:, :, 0].reshape(M, -1), z[:, :, 1].reshape(M, -1)
+        want, got = torch.nn.functional.gelu(z1) * z2, y[:, 256 * i:256 * i + z1.shape[1]].double()
+        err = (got - want).abs()
+        assert bool((err <= want.abs() * 2.0 ** -7 + (z1.abs() + 0.2) * z2.abs() * 2.0 ** -7 + 1e-3).all()), (i, err.max().item())             # (as test_gate)
