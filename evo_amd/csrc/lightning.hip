@@ -9,7 +9,8 @@
 // 16 of the columns, so the state lives in the accumulators: S is accumulated as [k rows, v columns], which IS the layout of the S^T operand
 // of the next product under the split k order of frag_split -- it never passes through LDS.  The decayed scores are shared: every wave
 // computes a block or two of them, their hi and lo halves go through the LDS rows of k (done with by then).
-// Long sequences are cut into segments that run in parallel: (1) every segment's end state from zero, (2) a scan over segments, (3) outputs.
+// Long sequences are cut into segments that run in parallel: (1) every segment's end state from zero, (2) a scan over segments, (3) outputs.  Sequences of one segment
+// in the same launch take (3) alone, straight on their state, and no workspace.
 #include "mixers_common.h"
 #include "../../include/evo_mi355x.h"
 
@@ -17,7 +18,7 @@
 
 struct LightArgs {
     const void* z; void* o; float* state; const float* log2_decay; const int* cu; const int* resume;
-    float* seg;                                                  // [B][n_seg][H][dk][dv] or null: states per segment
+    float* seg;                                                  // [slot][H][dk][dv] or null: states per segment, at segment_slot
     int64_t ld;
     int H, dk, dv, n_seg, seg_len, act;                          // act: z still needs its SiLU (recurrent form)
 };
@@ -42,6 +43,8 @@ __global__ __launch_bounds__(4 * DV, 2) void lightning_chunk_kernel(LightArgs a)
     int len = a.cu[b + 1] - row0;
     len = len < a.seg_len ? len : a.seg_len;
     if (len <= 0 && (seg > 0 || len < 0)) return;
+    const bool cut = a.seg && a.cu[b + 1] - a.cu[b] > a.seg_len;
+    if (!OUT && !cut) return;
     const float l2 = a.log2_decay[h];
     const uint16_t* zq = (const uint16_t*)a.z + row0 * a.ld + (int64_t)h * dk;
     const uint16_t* zk = zq + (int64_t)a.H * dk;
@@ -63,7 +66,7 @@ __global__ __launch_bounds__(4 * DV, 2) void lightning_chunk_kernel(LightArgs a)
     const int64_t st_off = ((int64_t)b * a.H + h) * dk * dv;
     {
         const float* src = nullptr;
-        if (OUT && a.seg && (seg > 0 || a.resume)) src = a.seg + (((int64_t)b * a.n_seg + seg) * a.H + h) * dk * dv;
+        if (OUT && cut && (seg > 0 || a.resume)) src = a.seg + (segment_slot(a.cu, b, seg, a.seg_len) * a.H + h) * dk * dv;
         else if (OUT && a.resume && a.resume[b]) src = a.state + st_off;
 #pragma unroll
         for (int kb = 0; kb < NKB; ++kb)
@@ -270,8 +273,8 @@ __global__ __launch_bounds__(4 * DV, 2) void lightning_chunk_kernel(LightArgs a)
         __syncthreads();
     }
     float* dst = nullptr;                                        // end state: of the segment (state-only walk), or of the sequence
-    if (!OUT) dst = a.seg + (((int64_t)b * a.n_seg + seg) * a.H + h) * dk * dv;
-    else if (a.state && !a.seg) dst = a.state + st_off;
+    if (!OUT) dst = a.seg + (segment_slot(a.cu, b, seg, a.seg_len) * a.H + h) * dk * dv;
+    else if (a.state && !cut) dst = a.state + st_off;
     if (dst) {
 #pragma unroll
         for (int kb = 0; kb < NKB; ++kb)
@@ -283,20 +286,21 @@ __global__ __launch_bounds__(4 * DV, 2) void lightning_chunk_kernel(LightArgs a)
     }
 }
 
-// seg[b][s] <- the state BEFORE segment s (it held the segment's own end state from zero); state[b] <- the state after the last token
+// a sequence's slots: segment s <- the state BEFORE it (it held the segment's own end state from zero); state[b] <- the state after the last token
 __global__ __launch_bounds__(256) void lightning_scan_kernel(LightArgs a) {
     const int h = blockIdx.y, b = blockIdx.z;
     const int64_t per = (int64_t)a.dk * a.dv, e = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (e >= per) return;
     const float l2 = a.log2_decay[h];
     const int len = a.cu[b + 1] - a.cu[b];
+    if (len <= a.seg_len) return;
     const int64_t so = ((int64_t)b * a.H + h) * per + e;
     float s = a.resume && a.resume[b] ? a.state[so] : 0.f;
     for (int i = 0; i < a.n_seg; ++i) {
         int n = len - i * a.seg_len;
         if (n <= 0) break;
         n = n < a.seg_len ? n : a.seg_len;
-        float* p = a.seg + (((int64_t)b * a.n_seg + i) * a.H + h) * per + e;
+        float* p = a.seg + (segment_slot(a.cu, b, i, a.seg_len) * a.H + h) * per + e;
         const float own = *p;
         *p = s;
         s = s * pow_log2(l2, n) + own;

@@ -13,6 +13,13 @@ template <typename T> __device__ __forceinline__ void st1(T* p, float v);
 template <> __device__ __forceinline__ void st1<uint16_t>(uint16_t* p, float v) { *p = f_to_bf(v); }
 template <> __device__ __forceinline__ void st1<float>(float* p, float v) { *p = v; }
 
+// Workspace slot of segment `seg` of sequence `b` where sequences of more than `len` tokens are cut into segments of `len`: behind the cut ones before it.  Those have at most
+// cu / len whole segments, and a ragged one each, of which there are no more than sequences and no more than whole segments.  Slots there are: segment_slots.
+__device__ __forceinline__ int64_t segment_slot(const int* cu, int b, int seg, int len) {
+    const int whole = cu[b] / len;
+    return (int64_t)whole + (b < whole ? b : whole) + seg;
+}
+
 // V consecutive elements (V = 8: 16-byte aligned bf16 / 32-byte fp32 runs; V = 1: any alignment)
 template <typename T, int V> struct vec_io;
 template <> struct vec_io<uint16_t, 8> {

@@ -17,7 +17,7 @@
 #define TAPS 4                                                   // convolution taps the matrix-core kernels hold (fewer: zeros in front)
 
 struct RgArgs {
-    const void* z; const void* in_b; void* o; float* state; float* seg;   // seg [B][n_seg][2][W]
+    const void* z; const void* in_b; void* o; float* state; float* seg;   // seg [slot][2][W], at segment_slot
     const void *conv, *conv_b, *ra, *ra_b, *ri, *ri_b;
     const float* decay; const int64_t* pos; const int* seq; const int* cu; const int* resume;
     int64_t ld;
@@ -64,7 +64,8 @@ __global__ __launch_bounds__(64 * NW) void rglru_chunk_kernel(RgArgs a) {
     const int len_all = a.cu[b + 1] - row0, s_lo = seg * a.seg_len;
     int s_hi = s_lo + a.seg_len;
     s_hi = s_hi < len_all ? s_hi : len_all;
-    if (s_lo >= s_hi) return;
+    const bool cut = a.seg && len_all > a.seg_len;               // (sequences of one segment: the second pass alone, straight on their state)
+    if (s_lo >= s_hi || (!OUT && !cut)) return;
     const bool go_on = a.resume && a.resume[b];
     const int ch = cg * 16 * NW + 16 * wave + c16, cc = ch < bs ? ch : bs - 1;   // this lane's channel of the block (clamped for loads)
     const int wch = n * bs + cc;                                 // ... of the whole width
@@ -154,7 +155,7 @@ __global__ __launch_bounds__(64 * NW) void rglru_chunk_kernel(RgArgs a) {
 
     float S = 0.f, A = 1.f;                                      // the carried state (the same in the four lane groups); OUT = false: the product of a
     if (OUT) {
-        if (a.seg && (seg > 0 || go_on)) S = a.seg[(((int64_t)b * a.n_seg + seg) * 2 + 1) * W + wch];
+        if (cut && (seg > 0 || go_on)) S = a.seg[(segment_slot(a.cu, b, seg, a.seg_len) * 2 + 1) * W + wch];
         else if (go_on) S = st[cc];
     }
     // y and the outputs move 16 bytes at a time: thread (row, run of eight channels) of two runs, the same ones in both directions
@@ -255,7 +256,7 @@ __global__ __launch_bounds__(64 * NW) void rglru_chunk_kernel(RgArgs a) {
     }
     if (g == 0 && ch < bs) {
         if (!OUT) {
-            float* p = a.seg + ((int64_t)b * a.n_seg + seg) * 2 * W + wch;
+            float* p = a.seg + segment_slot(a.cu, b, seg, a.seg_len) * 2 * W + wch;
             p[0] = A;
             p[W] = S;
         } else if (st && s_hi == len_all) st[cc] = S;
@@ -267,9 +268,10 @@ __global__ __launch_bounds__(256) void rglru_carry_kernel(RgArgs a) {
     const int c = blockIdx.x * 256 + threadIdx.x, b = blockIdx.y;
     if (c >= a.W) return;
     const int len = a.cu[b + 1] - a.cu[b], n = (len + a.seg_len - 1) / a.seg_len;
+    if (n < 2) return;
     float S = a.resume && a.resume[b] ? a.state[(int64_t)b * (1 + a.taps) * a.W + c] : 0.f;
     for (int s = 0; s < n; ++s) {
-        float* p = a.seg + ((int64_t)b * a.n_seg + s) * 2 * a.W + c;
+        float* p = a.seg + segment_slot(a.cu, b, s, a.seg_len) * 2 * a.W + c;
         const float in = S;
         S = fmaf(p[0], S, p[a.W]);
         p[a.W] = in;

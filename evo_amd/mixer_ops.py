@@ -312,8 +312,7 @@ class MixerOps:
             return o
         L = max(batch.lens)
         seg_len = seg_len or self.lightning_segment(tuple(sorted(batch.lens)), heads * ((dv + 127) // 128), dk * dv)
-        n_seg = (L + seg_len - 1) // seg_len
-        seg = torch.empty(B, n_seg, heads, dk, dv, dtype=torch.float32, device=z.device) if n_seg > 1 else None
+        seg = torch.empty(self.segment_slots(B, M, seg_len), heads, dk, dv, dtype=torch.float32, device=z.device) if L > seg_len else None
         self._call("evo_lightning_chunk_bf16", z.data_ptr(), z.stride(0), o.data_ptr(), sp, None if seg is None else seg.data_ptr(),
                    self._ix(log2_decay, torch.float32, heads, "log2_decay"), cu, resume, B, heads, dk, dv, L, seg_len)
         return o
@@ -322,25 +321,33 @@ class MixerOps:
     @functools.lru_cache(maxsize=64)
     def lightning_segment(lens: Tuple[int, ...], columns: int, state: int, cus: int = 256) -> int:
         """Tokens per segment (whole chunks): the least of what the launches cost, for `columns` (head, value tile) pairs a sequence and `state` elements of one.
-        A workgroup a CU takes 5.4 us a chunk; cut sequences need another pass for their segments' states (2.2 us a chunk) and every segment's state crosses memory four
+        A workgroup a CU takes 5.4 us a chunk; cut sequences need another pass for their segments' states (2.2 us a chunk) and each of those crosses memory four
         times.  (us at 32 heads of 128 x 128, the rule before, segments for a workgroup per CU -> this one.  6 sequences of 1,459 to 2,500 tokens: 295 in
         segments of 1,280, 214 uncut; 5,000 and 300: 148 -> 101 in segments of 768; 3,000 and four times 300: 177 -> 102; 1,500 and three times 100: 98 -> 57;
         4,000 twice 133 as before, 311 uncut.)"""
-        def us(seg, span, busy, n_wg):
-            return 6.0 + 5.3 * span + (3.0 + 2.2 * busy + n_wg * state * 16 / 4.5e6 if seg < max(lens) else 0.0)
+        def us(seg, span, busy, n_cut):
+            return 6.0 + 5.3 * span + (3.0 + 2.2 * busy + n_cut * state * 16 / 4.5e6 if n_cut else 0.0)
         return MixerOps.cheapest_segment(lens, columns, us, cus)
 
     @staticmethod
+    def segment_slots(B: int, rows: int, seg_len: int) -> int:
+        """Workspace slots of the segments of cut sequences (csrc/mixers_common.h segment_slot): by the rows, however many sequences share the pass."""
+        whole = rows // seg_len
+        return whole + min(B, whole)
+
+    @staticmethod
     def cheapest_segment(lens: Tuple[int, ...], columns: int, us, cus: int) -> int:
-        """The segment length, whole chunks of a share of the longest sequence, of least us(segment, chunks of the launch's end, chunks at the most of a CU where two
-        workgroups share one, workgroups).  Several rounds of workgroups end half a workgroup late."""
+        """The segment length, whole chunks of a share of the longest sequence, of least us(segment, chunks of the launch's end, chunks of cut sequences at the most of a
+        CU where two workgroups share one, workgroups of cut sequences).  Several rounds of workgroups end half a workgroup late."""
         longest = max(lens)
         chunks = sum((n + LC - 1) // LC for n in lens) * columns / cus
         best = None
         for seg in sorted({max(4 * LC, (longest + n * LC - 1) // (n * LC) * LC) for n in range(1, 33)}, reverse=True):
             n_wg = sum((n + seg - 1) // seg for n in lens) * columns
+            cut = [n for n in lens if n > seg]
             top = min(seg, (longest + LC - 1) // LC * LC) / LC
-            t = us(seg, top if n_wg <= cus else max(top, chunks + top / 2), max(top, chunks), n_wg)
+            t = us(seg, top if n_wg <= cus else max(top, chunks + top / 2), max(top, sum((n + LC - 1) // LC for n in cut) * columns / cus),
+                   sum((n + seg - 1) // seg for n in cut) * columns)
             if best is None or t < best[0]:
                 best = (t, seg)
         return best[1]
@@ -543,8 +550,7 @@ class MixerOps:
             assert sum(batch.lens) == M
             L = max(batch.lens)
             seg_len = seg_len or self.rglru_segment(tuple(sorted(batch.lens)), nb * ((bs + 127) // 128))
-            n_seg = (L + seg_len - 1) // seg_len
-            seg = torch.empty(B, n_seg, 2, W, dtype=torch.float32, device=z.device) if n_seg > 1 else None
+            seg = torch.empty(self.segment_slots(B, M, seg_len), 2, W, dtype=torch.float32, device=z.device) if L > seg_len else None
             self._call("evo_rglru_chunk_bf16", *head, o.data_ptr(), sp, None if seg is None else seg.data_ptr(), *w, cu, resume, B, W, nb, taps, L, seg_len)
             return o
         ab = torch.empty(M, 2, W, dtype=torch.float32, device=z.device)

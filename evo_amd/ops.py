@@ -104,7 +104,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 21         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 22         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):

@@ -62,8 +62,9 @@ extern "C" {
  *  18: evo_linear_parts, evo_linear_parts_bf16, evo_closing_parts and evo_heads_decode_whole added.
  *  19: evo_step_out added.
  *  20: evo_hyena_short gained `mask`.
- *  21: evo_linear_ring_share added. */
-#define EVO_ABI_VERSION 21
+ *  21: evo_linear_ring_share added.
+ *  22: evo_lightning_chunk_bf16 and evo_rglru_chunk_bf16 keep the states of cut sequences only: `seg` by the rows, not by the sequences. */
+#define EVO_ABI_VERSION 22
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
@@ -484,8 +485,8 @@ int evo_act_cols(void* z, int64_t ld, int64_t M, int64_t n, int64_t act, int64_t
 /* ---- linear attention with a constant decay per head: S_t = a_h S_{t-1} + k_t v_t^T, o_t = S_t^T q_t ------------------------------
  * z rows (pitch ld) start with [q (H dk) | k (H dk) | v (H dv)] after their SiLU; o [M, H dv]; state [B, H, dk, dv] fp32 (may be NULL:
  * nothing is kept), read where resume[b] != 0 (resume NULL: every sequence starts from zero) and left after the last token.
- * evo_lightning_chunk_bf16: the prompt form on the matrix cores; dk <= 128; seg_len % 64 == 0; seg [B, ceil(max_len / seg_len), H, dk, dv]
- * fp32 workspace, needed when there is more than one segment.  log2_decay [H].
+ * evo_lightning_chunk_bf16: the prompt form on the matrix cores; dk <= 128; seg_len % 64 == 0; seg [slots, H, dk, dv] fp32
+ * workspace, needed when max_len > seg_len: sequences of more than seg_len tokens are cut, slots = n + min(B, n) with n = rows / seg_len rounded down.  log2_decay [H].
  * evo_lightning_recurrent: token by token; cu NULL = one token per sequence (row b), updating state[b] in place: the decode step.
  * act != 0: z is still before its SiLU. */
 int evo_lightning_chunk_bf16(const void* z, int64_t ld, void* o, float* state, float* seg, const float* log2_decay, const int* cu,
@@ -535,7 +536,7 @@ int evo_heads_merge(const float* part_o, const float* part_ml, void* o, int64_t 
  * state [rows, 1 + taps, W] fp32 (may be NULL: nothing is kept): row 0 is S, row 1 + p % taps the x of position p; read where resume[b] != 0
  * (resume NULL: every sequence starts from zero), left after the last token.  pos [M]: position of every row's token.
  * evo_rglru_chunk_bf16: prompts on the matrix cores; bs % 8 == 0, bs <= 384, taps <= 4, in_b NULL and y activated by the caller; seg_len % 64 == 0;
- *   seg [B, ceil(max_len / seg_len), 2, W] fp32 workspace, needed when there is more than one segment.
+ *   seg [slots, 2, W] fp32 workspace, needed when max_len > seg_len: slots as for evo_lightning_chunk_bf16.
  * evo_rglru_step_bf16: one token per sequence (row b), same sizes, updates state[b] in place.
  * evo_rglru_any: any sizes, both storage types; ab [M, 2, W] fp32 workspace; cu NULL: one token per sequence. */
 int evo_rglru_chunk_bf16(const void* z, int64_t ld, void* o, float* state, float* seg, const void* conv, const void* conv_b, const void* ra,

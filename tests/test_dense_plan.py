@@ -84,3 +84,29 @@ def test_columns_of_weight_streaming_workgroups(N, gated):
             assert lib.evo_linear_ring_share(N, 0, b // 2, ctypes.cast(half, ctypes.c_void_p)) == 0 and half[1] == out[1]
     assert out[2] == cols
     assert lib.evo_linear_ring_share(N, gated, groups, ctypes.cast(out, ctypes.c_void_p)) == -1
+
+
+def test_workspace_of_segments():
+    """Slots of cut sequences don't meet and stay inside the workspace, whose size follows the rows: one long prompt among many short ones asks for its own segments only."""
+    import random
+    from evo_amd.mixer_ops import MixerOps
+    rng = random.Random(1)
+    cases = [([100] * 200 + [32000], 1280), ([32000] + [50] * 400, 1280), ([0, 64, 0, 65, 128, 129], 64), ([64] * 9, 64), ([65] * 9, 64)]
+    for _ in range(300):
+        seg = 64 * rng.randint(1, 30)
+        cases.append(([rng.choice((0, 1, seg - 1, seg, seg + 1, 3 * seg, rng.randint(0, 5 * seg))) for _ in range(rng.randint(1, 40))], seg))
+    for lens, seg in cases:
+        slots, at, end = MixerOps.segment_slots(len(lens), sum(lens), seg), 0, 0
+        for b, n in enumerate(lens):
+            if n > seg:                                           # csrc/mixers_common.h segment_slot
+                first = at // seg + min(b, at // seg)
+                assert first >= end
+                end = first + -(-n // seg)
+            at += n
+        assert end <= slots <= 2 * (sum(lens) // seg)
+    for many in ([100] * 200, [50] * 400):
+        for lens in (many + [32000], [32000] + many):
+            seg = MixerOps.lightning_segment(tuple(sorted(lens)), 32, 128 * 128)
+            assert MixerOps.segment_slots(len(lens), sum(lens), seg) * 32 * 128 * 128 * 4 < 256 << 20
+            seg = MixerOps.rglru_segment(tuple(sorted(lens)), 32)
+            assert MixerOps.segment_slots(len(lens), sum(lens), seg) * 2 * 4096 * 4 < 16 << 20

@@ -164,6 +164,31 @@ def test_lightning_segments_and_carried_states(ops, H, dk, dv):
     lightning_case(ops, F32, lens, H, dk, dv, decay, states=states)
 
 
+@pytest.mark.parametrize("H,dk,dv", [(2, 64, 64), (1, 128, 200)])
+@pytest.mark.parametrize("lens", [[64] * 5 + [1500] + [1, 128, 129] * 3, [700, 128, 129, 64, 257, 1], [129] * 4])
+def test_lightning_segments_of_unequal_sequences(ops, H, dk, dv, lens):
+    """Cut sequences beside others: the bits of each sequence alone, whichever slots its segments have; sequences of one segment ask for no workspace."""
+    from evo_amd.mixer_ops import TokenBatch
+    decay = torch.tensor([0.999, 0.9][:H])
+    z, states = rnd(sum(lens), H * (2 * dk + dv), seed=1, dt=BF).to(DEV), rnd(len(lens), H, dk, dv, seed=2).to(DEV)
+    past = [5 * (b % 2) for b in range(len(lens))]
+
+    def run(rows, of, st):
+        return ops.lightning(rows, H, dk, dv, decay.to(DEV), decay.double().log2().float().to(DEV), TokenBatch.of_prompts([lens[b] for b in of], [past[b] for b in of], DEV),
+                             st, seg_len=128)
+    st = states.clone()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    o = run(z, list(range(len(lens))), st)
+    slots = sum(lens) // 128 + min(len(lens), sum(lens) // 128)
+    assert torch.cuda.max_memory_allocated() - before <= o.numel() * 2 + slots * H * dk * dv * 4 + (1 << 16)
+    at = 0
+    for b, n in enumerate(lens):
+        alone = states[b:b + 1].clone()
+        assert torch.equal(run(z[at:at + n], [b], alone), o[at:at + n]) and torch.equal(alone[0], st[b])
+        at += n
+
+
 def test_lightning_decays_of_zero_and_one(ops):
     for dt in (BF, F32):
         lightning_case(ops, dt, [140, 66], 3, 32, 32, [0.0, 1.0, 0.5])

@@ -116,6 +116,22 @@ def test_recurrence_in_segments(ops, W, nb, taps, seg):
     prompt_case(ops, BF, [700, 130, 64, 1, 321], W, nb, taps, past=[9, 0, 2, 40, 0], seg_len=seg, seed=9)
 
 
+@pytest.mark.parametrize("W,nb", [(96, 4), (512, 2), (800, 2)])
+@pytest.mark.parametrize("lens", [[64] * 5 + [1500] + [1, 128, 129] * 3, [700, 128, 129, 64, 257, 1], [129] * 4])
+def test_segments_of_unequal_sequences(ops, W, nb, lens):
+    """Cut sequences beside others: the bits of each sequence alone, whichever slots its segments have."""
+    from evo_amd.mixer_ops import TokenBatch
+    w, z = layer(W, nb, 4, BF, 3), rnd(sum(lens), 2 * W + 8, seed=4, dt=BF)
+    states, past = rnd(len(lens), 5, W, seed=5).to(BF).float().to(DEV), [7 * (b % 2) for b in range(len(lens))]
+    st = states.clone()
+    o, at = run_kernel(ops, z, None, False, W, w, TokenBatch.of_prompts(lens, past, DEV), st, seg_len=128), 0
+    for b, n in enumerate(lens):
+        alone = states[b:b + 1].clone()
+        got = run_kernel(ops, z[at:at + n].contiguous(), None, False, W, w, TokenBatch.of_prompts([n], [past[b]], DEV), alone, seg_len=128)
+        assert torch.equal(got, o[at:at + n]) and torch.equal(alone[0], st[b])
+        at += n
+
+
 def test_slow_decays_carry_far(ops):
     """A decay close to one: what the first tokens leave behind is still there 1,500 tokens later."""
     from evo_amd.mixer_ops import TokenBatch
