@@ -311,7 +311,7 @@ class MixerOps:
             self._call("evo_lightning_recurrent", z.data_ptr(), z.stride(0), o.data_ptr(), sp, dp, cu, resume, B, heads, dk, dv, 0, f32)
             return o
         L = max(batch.lens)
-        seg_len = seg_len or self.lightning_segment(tuple(sorted(batch.lens)), heads * ((dv + 127) // 128), dk * dv)
+        seg_len = seg_len or self.lightning_segment(tuple(sorted(batch.lens)), heads * ((dv + 127) // 128), dk * min(dv, 128))
         seg = torch.empty(self.segment_slots(B, M, seg_len), heads, dk, dv, dtype=torch.float32, device=z.device) if L > seg_len else None
         self._call("evo_lightning_chunk_bf16", z.data_ptr(), z.stride(0), o.data_ptr(), sp, None if seg is None else seg.data_ptr(),
                    self._ix(log2_decay, torch.float32, heads, "log2_decay"), cu, resume, B, heads, dk, dv, L, seg_len)
@@ -320,14 +320,14 @@ class MixerOps:
     @staticmethod
     @functools.lru_cache(maxsize=64)
     def lightning_segment(lens: Tuple[int, ...], columns: int, state: int, cus: int = 256) -> int:
-        """Tokens per segment (whole chunks): the least of what the launches cost, for `columns` (head, value tile) pairs a sequence and `state` elements of one.
+        """Tokens per segment (whole chunks): the least of what the launches cost, for `columns` (head, value tile) pairs a sequence and `state` elements of one such tile.
         A workgroup a CU takes 5.4 us a chunk; cut sequences need another pass for their segments' states (2.2 us a chunk) and each of those crosses memory four
         times.  (us at 32 heads of 128 x 128, the rule before, segments for a workgroup per CU -> this one.  6 sequences of 1,459 to 2,500 tokens: 295 in
         segments of 1,280, 214 uncut; 5,000 and 300: 148 -> 101 in segments of 768; 3,000 and four times 300: 177 -> 102; 1,500 and three times 100: 98 -> 57;
         4,000 twice 133 as before, 311 uncut.)"""
         def us(seg, span, busy, n_cut):
             return 6.0 + 5.3 * span + (3.0 + 2.2 * busy + n_cut * state * 16 / 4.5e6 if n_cut else 0.0)
-        return MixerOps.cheapest_segment(lens, columns, us, cus)
+        return MixerOps.cheapest_segment(lens, columns, us, cus, 0.7 if state <= 4096 else 1.0)
 
     @staticmethod
     def segment_slots(B: int, rows: int, seg_len: int) -> int:
@@ -336,17 +336,20 @@ class MixerOps:
         return whole + min(B, whole)
 
     @staticmethod
-    def cheapest_segment(lens: Tuple[int, ...], columns: int, us, cus: int) -> int:
+    def cheapest_segment(lens: Tuple[int, ...], columns: int, us, cus: int, share: float = 1.0) -> int:
         """The segment length, whole chunks of a share of the longest sequence, of least us(segment, chunks of the launch's end, chunks of cut sequences at the most of a
-        CU where two workgroups share one, workgroups of cut sequences).  Several rounds of workgroups end half a workgroup late."""
+        CU where two workgroups share one, workgroups of cut sequences).  Several rounds of workgroups end half a workgroup late, and each costs 1.3 chunks before its
+        first; `share`: what a chunk costs where small workgroups share a CU (6 sequences of 1,459 to 2,500 tokens: 32 heads of 64 x 64 uncut 129, 1,280 115, 768 96; 16 blocks
+        of 64 channels 896 104, 1,280 101, 256 to 512 71).  Few columns: shares down to a workgroup per CU (us, 32 shares at the most -> as many as CUs.  Decayed linear attention, 131,072 tokens at two heads
+        of 128 x 128 431 -> 164, one of 64 x 64 277 -> 113; 32,000 at four heads 130 -> 94; gated recurrence, 131,072 tokens in two blocks of 256 526 -> 310)."""
         longest = max(lens)
         chunks = sum((n + LC - 1) // LC for n in lens) * columns / cus
         best = None
-        for seg in sorted({max(4 * LC, (longest + n * LC - 1) // (n * LC) * LC) for n in range(1, 33)}, reverse=True):
+        for seg in sorted({max(4 * LC, (longest + n * LC - 1) // (n * LC) * LC) for n in range(1, 33 + cus // (columns * len(lens)))}, reverse=True):
             n_wg = sum((n + seg - 1) // seg for n in lens) * columns
             cut = [n for n in lens if n > seg]
             top = min(seg, (longest + LC - 1) // LC * LC) / LC
-            t = us(seg, top if n_wg <= cus else max(top, chunks + top / 2), max(top, sum((n + LC - 1) // LC for n in cut) * columns / cus),
+            t = us(seg, top if n_wg <= cus else max(top, share * (chunks + 1.3 * n_wg / cus + 0.55 * top)), max(top, sum((n + LC - 1) // LC for n in cut) * columns / cus),
                    sum((n + seg - 1) // seg for n in cut) * columns)
             if best is None or t < best[0]:
                 best = (t, seg)
@@ -512,14 +515,14 @@ class MixerOps:
 
     @staticmethod
     @functools.lru_cache(maxsize=64)
-    def rglru_segment(lens: Tuple[int, ...], columns: int, cus: int = 256) -> int:
+    def rglru_segment(lens: Tuple[int, ...], columns: int, cus: int = 256, small: bool = False) -> int:
         """Tokens per segment, as lightning_segment: 4.4 us a chunk, and 3.9 for its gates once more where sequences are cut; the carries walk the segments one by one.
         (us at 4,096 channels in 16 blocks, the rule before, from the longest sequence alone -> this one.  4,000, 1,000 and 2,000 tokens 262 -> 144 in segments of
         1,024; 3,000 and three times 300 202 -> 113; 2,000 and three times 500 144 -> 89; 5,000 and 300 173 -> 116; 500 52 -> 44 uncut; one of 8,190 152 -> 145 and
         six of 1,459 to 2,500, uncut, 187 -> 186 are cut as they were.)"""
         def us(seg, span, busy, n_wg):
-            return 8.0 + 4.4 * span + (3.0 + 3.9 * span + 2.5 * ((max(lens) + seg - 1) // seg) if seg < max(lens) else 0.0)
-        return MixerOps.cheapest_segment(lens, columns, us, cus)
+            return 8.0 + 4.4 * span + (3.0 + 3.9 * span + 0.3 * ((max(lens) + seg - 1) // seg) if seg < max(lens) else 0.0)
+        return MixerOps.cheapest_segment(lens, columns, us, cus, 0.65 if small else 1.0)
 
     def rglru(self, z: torch.Tensor, in_b: Optional[torch.Tensor], act: bool, W: int, conv: torch.Tensor, conv_b: torch.Tensor, ra, ra_b, ri, ri_b,
               decay: torch.Tensor, batch: TokenBatch, state: Optional[torch.Tensor] = None, seg_len: Optional[int] = None) -> torch.Tensor:
@@ -549,7 +552,7 @@ class MixerOps:
         if fast and in_b is None and not act:
             assert sum(batch.lens) == M
             L = max(batch.lens)
-            seg_len = seg_len or self.rglru_segment(tuple(sorted(batch.lens)), nb * ((bs + 127) // 128))
+            seg_len = seg_len or self.rglru_segment(tuple(sorted(batch.lens)), nb * ((bs + 127) // 128), small=bs <= 64)
             seg = torch.empty(self.segment_slots(B, M, seg_len), 2, W, dtype=torch.float32, device=z.device) if L > seg_len else None
             self._call("evo_rglru_chunk_bf16", *head, o.data_ptr(), sp, None if seg is None else seg.data_ptr(), *w, cu, resume, B, W, nb, taps, L, seg_len)
             return o

@@ -110,3 +110,15 @@ def test_workspace_of_segments():
             assert MixerOps.segment_slots(len(lens), sum(lens), seg) * 32 * 128 * 128 * 4 < 256 << 20
             seg = MixerOps.rglru_segment(tuple(sorted(lens)), 32)
             assert MixerOps.segment_slots(len(lens), sum(lens), seg) * 2 * 4096 * 4 < 16 << 20
+
+
+def test_long_prompts_of_few_heads_fill_the_chip():
+    """As many segments as CUs where the heads are few, and none too many where they pay nothing: several rounds of wide blocks against one."""
+    from evo_amd.mixer_ops import MixerOps
+    for columns in (1, 2, 4, 8, 32):
+        for n in (32000, 131072):
+            for seg in (MixerOps.lightning_segment((n,), columns, 128 * 128), MixerOps.rglru_segment((n,), columns)):
+                assert 100 <= -(-n // seg) * columns <= 256
+    six = (1459, 1667, 1875, 2084, 2292, 2500)
+    assert MixerOps.rglru_segment(six, 20) == 1280 and MixerOps.rglru_segment(six, 16, small=True) <= 512
+    assert MixerOps.lightning_segment(six, 32, 64 * 64) <= 768 and MixerOps.lightning_segment(six, 64, 64 * 128) >= 2500
