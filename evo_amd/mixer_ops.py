@@ -473,13 +473,15 @@ class MixerOps:
         return max(1, min((ring + 127) // 128, (cus + groups - 1) // groups, 64))
 
     def heads_whole_ok(self, groups: int, ring: int, Q: int, maps: int, dim: int, dv: int, z, cache) -> bool:
-        """One workgroup per (sequence, key head) walks its whole cache and writes the result itself: no parts, no merge launch.  From 160 of them on, and from 80 on
-        where a whole cache is short.  us in a graph, parts and merge -> whole: 16 heads of two maps, 640 slots, 10 / 24 / 32 sequences of up to 600 tokens 32.2 / 45.9 /
-        52.0 -> 25.1 / 42.1 / 46.9 (2,048 slots, 10 of up to 1,500 48.4 -> 49.4); 8 key heads of 4 queries each, 1,028 slots, 10 / 24 sequences of up to 600
-        13.2 / 16.6 -> 10.3 / 12.6, of up to 1,500 16.5 / 25.6 -> 14.8 / 22.5 (8 sequences 13.4 -> 14.8: not taken)."""
+        """One workgroup per (sequence, key head) walks its whole cache and writes the result itself: no parts, no merge launch.  From 256 of them on the cache had one
+        part anyway; with fewer only where a whole cache is short, as parts share a long sequence among short ones (us in a graph, parts and merge : whole.  Full caches /
+        lengths from all of it down to a third / one full, the others 100 tokens.  10 sequences, 16 heads of two maps of 128, values of 256: 640 slots 43 : 29, 33 : 27, 21 : 23;
+        1,028 slots 56 : 43, 40 : 40, 27 : 33; 2,048 88 : 73, 58 : 65, 37 : 50.  8 key heads of four queries, 128: 20 sequences, 1,536 slots 36 : 31, 28 : 27, 17 : 19,
+        2,048 46 : 41, 36 : 37, 20 : 24; 10 sequences, 1,028 slots 18 : 16, 15 : 15, 13 : 15, 1,536 23 : 27, 18 : 21, 14 : 18.  16 heads of 64: 8 sequences, 2,048 slots
+        21 : 25, 16 : 19, 13 : 15, 10 of them 30 : 26, 22 : 23, 13 : 15.  200 tokens each 12 : 7 to 25 : 15)."""
         return (self.mixer_mfma and z.dtype == torch.bfloat16 and dim % 8 == 0 and dv % 8 == 0 and z.stride(0) % 8 == 0 and cache.shape[2] % 8 == 0
                 and dim <= (128 if maps == 2 else 256) and dv <= 256 and maps * min(Q, 16) <= 16 and (z.data_ptr() | cache.data_ptr()) % 16 == 0
-                and (groups >= 160 or (groups >= 80 and ring * (maps * dim + dv) <= 300000)))
+                and groups >= 80 and (groups >= 256 or ring * (maps * dim + dv + 64) <= (500000 if groups >= 160 else 330000)))
 
     def heads_decode(self, z: torch.Tensor, cache: torch.Tensor, pos: torch.Tensor, heads: int, kv_heads: int, maps: int, dim: int, dv: int, scale: float,
                      lam: float, gain: float, eps: float, n_split: Optional[int] = None) -> torch.Tensor:

@@ -122,3 +122,18 @@ def test_long_prompts_of_few_heads_fill_the_chip():
     six = (1459, 1667, 1875, 2084, 2292, 2500)
     assert MixerOps.rglru_segment(six, 20) == 1280 and MixerOps.rglru_segment(six, 16, small=True) <= 512
     assert MixerOps.lightning_segment(six, 32, 64 * 64) <= 768 and MixerOps.lightning_segment(six, 64, 64 * 128) >= 2500
+
+
+def test_decode_attention_in_one_launch_where_caches_are_short():
+    """A workgroup per key head walks its whole cache from 256 of them on, below that on short caches only: parts share a long sequence among short ones."""
+    import types
+    import torch
+    from evo_amd.mixer_ops import MixerOps
+    ops, t = types.SimpleNamespace(mixer_mfma=True), torch.zeros(1, 1, 64, dtype=torch.bfloat16)
+
+    def whole(groups, ring, maps, dim, dv):
+        return MixerOps.heads_whole_ok(ops, groups, ring, 1, maps, dim, dv, t[0], t)
+    for maps, dim, dv, few, more in ((2, 128, 256, 512, 800), (1, 128, 128, 1028, 1536), (1, 64, 64, 1536, 2048)):
+        assert whole(256, 1 << 20, maps, dim, dv) and not whole(79, 64, maps, dim, dv)
+        for groups, ring in ((80, few), (159, few), (160, more), (255, more)):
+            assert whole(groups, ring, maps, dim, dv) and not whole(groups, 2 * ring, maps, dim, dv)
