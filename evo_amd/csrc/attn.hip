@@ -27,7 +27,8 @@
 // every split streams its share of the KV cache and leaves an unnormalised partial (O, m, l) that
 // attn_decode_combine_kernel merges.  The key count may come from device memory (dyn_pos), so the launch is
 // position-independent and can sit inside a captured hipGraph.
-template <bool DECODE>
+// PACKED (here and below): the query blocks of unequal sequences behind each other, a.blocks.
+template <bool DECODE, bool PACKED = false>
 __global__ __launch_bounds__(256, DECODE ? 1 : 2) void attn_fwd_kernel(AttnArgs a) {
     // two stages of {Ks 16 KiB, Vt 16 KiB}: tile t+1 is written while tile t is consumed -> one barrier per tile
     __shared__ __attribute__((aligned(16))) unsigned char smem[2 * 2 * KB * DH * 2];
@@ -43,15 +44,23 @@ __global__ __launch_bounds__(256, DECODE ? 1 : 2) void attn_fwd_kernel(AttnArgs 
     if (DECODE && a.dyn_pos) { q_pos0_ = a.dyn_pos[blockIdx.z]; Tk_ = q_pos0_ + a.Tq; }
     int qb = 0, head = blockIdx.y, bat = blockIdx.z;
     if (!DECODE) attn_block_map(a, qb, head, bat);
-    const int64_t q0 = (int64_t)qb * QB;
+    int64_t q0 = (int64_t)qb * QB, Tq_ = a.Tq, out_row0 = bat * a.Tq;
 
     const uint16_t* qp = a.q + bat * a.q_sb + head * a.q_sh;
     const uint16_t* kp = a.k + bat * a.k_sb + head * a.k_sh;
     const uint16_t* vp = a.v + bat * a.v_sb + head * a.v_sh;
+    if constexpr (PACKED) {
+        const int4 e = a.blocks[qb];
+        qp += e.x * a.q_st; kp += e.x * a.k_st; vp += e.x * a.v_st;
+        Tq_ = Tk_ = e.y;
+        q_pos0_ = 0;
+        q0 = e.z;
+        out_row0 = e.x;
+    }
 
     // ---- Q fragment: this lane's query row, 8 k-steps x 16 bytes -------------------------------------
     const int64_t qrow = q0 + wave * 32 + l31;
-    const int64_t qrow_c = qrow < a.Tq ? qrow : a.Tq - 1;
+    const int64_t qrow_c = qrow < Tq_ ? qrow : Tq_ - 1;
     uint4 qf[8];
     {
         const uint4* qr = (const uint4*)(qp + qrow_c * a.q_st);
@@ -61,7 +70,7 @@ __global__ __launch_bounds__(256, DECODE ? 1 : 2) void attn_fwd_kernel(AttnArgs 
 
     // ---- key range of this workgroup / wave -------------------------------------------------------------
     int64_t q_last = q0 + QB - 1;
-    if (q_last > a.Tq - 1) q_last = a.Tq - 1;
+    if (q_last > Tq_ - 1) q_last = Tq_ - 1;
     int64_t max_key = q_last + q_pos0_;
     if (max_key > Tk_ - 1) max_key = Tk_ - 1;
     const int n_tiles = (int)(max_key / KB) + 1;
@@ -270,8 +279,8 @@ __global__ __launch_bounds__(256, DECODE ? 1 : 2) void attn_fwd_kernel(AttnArgs 
         return;
     }
     const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
-    if (qrow < a.Tq) {
-        uint16_t* orow = a.o + ((int64_t)(bat * a.Tq + qrow) * a.H + head) * DH;
+    if (qrow < Tq_) {
+        uint16_t* orow = a.o + ((out_row0 + qrow) * a.H + head) * DH;
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
@@ -338,6 +347,7 @@ __device__ __forceinline__ float max3_raw(float a, float b, float c) {
     } while (0)
 #define P_BARRIER() asm volatile("s_barrier" ::: "memory")
 
+template <bool PACKED>
 __global__ __launch_bounds__(512, 1) void attn_fwd_pipe_kernel(AttnArgs a) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[P_NSTG * P_STAGE];
 
@@ -348,17 +358,25 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pipe_kernel(AttnArgs a) {
     const int l31 = lane & 31;
     const int np = wave + 32 < P_NDMA ? 5 : 4;                          // DMA pieces of this wave per tile
 
-    const int64_t Tk_ = a.Tk, q_pos0_ = a.q_pos0;
+    int64_t Tk_ = a.Tk, q_pos0_ = a.q_pos0;
     int qb, head, bat;
     attn_block_map(a, qb, head, bat);
-    const int64_t q0 = (int64_t)qb * PQB;
+    int64_t q0 = (int64_t)qb * PQB, Tq_ = a.Tq, out_row0 = bat * a.Tq;
     const uint16_t* qp = a.q + bat * a.q_sb + head * a.q_sh;
     const unsigned char* kp = (const unsigned char*)(a.k + bat * a.k_sb + head * a.k_sh);
     const unsigned char* vp = (const unsigned char*)(a.v + bat * a.v_sb + head * a.v_sh);
     const int64_t kst_b = a.k_st * 2, vst_b = a.v_st * 2;
+    if constexpr (PACKED) {
+        const int4 e = a.blocks[qb];
+        qp += e.x * a.q_st; kp += e.x * kst_b; vp += e.x * vst_b;
+        Tq_ = Tk_ = e.y;
+        q_pos0_ = 0;
+        q0 = e.z;
+        out_row0 = e.x;
+    }
 
     const int64_t qrow = q0 + wave * 32 + l31;
-    const int64_t qrow_c = qrow < a.Tq ? qrow : a.Tq - 1;
+    const int64_t qrow_c = qrow < Tq_ ? qrow : Tq_ - 1;
     uint4 qf[8];
     {
         const uint4* qr = (const uint4*)(qp + qrow_c * a.q_st);
@@ -366,7 +384,7 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pipe_kernel(AttnArgs a) {
         for (int ks = 0; ks < 8; ++ks) qf[ks] = qr[2 * ks + half];
     }
     int64_t q_last = q0 + PQB - 1;
-    if (q_last > a.Tq - 1) q_last = a.Tq - 1;
+    if (q_last > Tq_ - 1) q_last = Tq_ - 1;
     int64_t max_key = q_last + q_pos0_;
     if (max_key > Tk_ - 1) max_key = Tk_ - 1;
     const int n_tiles = (int)(max_key / KB) + 1;
@@ -597,8 +615,8 @@ __global__ __launch_bounds__(512, 1) void attn_fwd_pipe_kernel(AttnArgs a) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // the trailing (empty) DMA pieces: nothing may land after exit
     const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
     const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
-    if (qrow < a.Tq) {
-        uint16_t* orow = a.o + ((int64_t)(bat * a.Tq + qrow) * a.H + head) * DH;
+    if (qrow < Tq_) {
+        uint16_t* orow = a.o + ((out_row0 + qrow) * a.H + head) * DH;
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
@@ -882,21 +900,26 @@ extern "C" int evo_attn_fwd_causal_bf16(const void* q, const void* k, const void
     const int64_t n_wg = (int64_t)a.n_qblocks * a.nbh;
     if (n_wg > 0x7fffffff) return -1;
     if (use_pipe)
-        hipLaunchKernelGGL(attn_fwd_pipe_kernel, dim3((unsigned)n_wg), dim3(512), 0, (hipStream_t)stream, a);
+        hipLaunchKernelGGL(attn_fwd_pipe_kernel<false>, dim3((unsigned)n_wg), dim3(512), 0, (hipStream_t)stream, a);
     else
         hipLaunchKernelGGL(attn_fwd_kernel<false>, dim3((unsigned)n_wg), dim3(256), 0, (hipStream_t)stream, a);
     return evo_launch_status();
 }
 
+// A launch for each kernel that the sequences would take alone, so that they keep their bits.  us, 32 heads, all on 64 rows a wave -> this: 16 sequences of 220 to 1,100 rows
+// 245 -> 193, 16 of 100 44 -> 19, 2,000 / 3,000 / 2,500 233 -> 208, 3,000 beside three of up to 700 150 -> 152; two launches with an end each: 4,000 beside 1,000 and
+// 300 213 -> 250.
 extern "C" int evo_attn_fwd_packed_bf16(const void* q, const void* k, const void* v, void* o, int64_t H, int64_t rows, int64_t q_st, int64_t q_sh, int64_t k_st,
-                                        int64_t k_sh, int64_t v_st, int64_t v_sh, const int32_t* blocks, const int32_t* blocks_host, int64_t n_blocks,
+                                        int64_t k_sh, int64_t v_st, int64_t v_sh, int64_t form, const int32_t* blocks, const int32_t* blocks_host, int64_t n_blocks,
                                         const int32_t* valid, float softmax_scale, void* vt_ws, void* stream) {
-    if (!q || !k || !v || !o || !blocks || !blocks_host || !valid || !vt_ws || H <= 0 || H > 65535 || rows <= 0 || rows > 0x7fffff00 || n_blocks <= 0 || n_blocks > 0x7fffffff)
+    if (!q || !k || !v || !o || !blocks || !blocks_host || H <= 0 || H > 65535 || rows <= 0 || rows > 0x7fffff00 || n_blocks <= 0 || n_blocks > 0x7fffffff)
         return -1;
+    if (form < 0 || form > 2 || (form == 2 && (!valid || !vt_ws)) || n_blocks * H > 0x7fffffff) return -1;
     if (attn_check_strides(0, q_st, q_sh, 0, k_st, k_sh, 0, v_st, v_sh) || ((uintptr_t)blocks & 15)) return -1;
     for (int64_t i = 0; i < n_blocks; ++i) {
         const int64_t first = blocks_host[4 * i], len = blocks_host[4 * i + 1], q0 = blocks_host[4 * i + 2];
-        if (first < 0 || first % 64 != 0 || len <= 0 || first + len > rows || q0 <= -256 || q0 + 256 > len) return -1;
+        if (first < 0 || first % 64 != 0 || len <= 0 || first + len > rows) return -1;
+        if (form == 2 ? q0 <= -256 || q0 + 256 > len : q0 < 0 || q0 >= len || q0 % PQB != 0 || (form == 0) != (len <= QB)) return -1;
     }
     AttnArgs a;
     a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v; a.o = (uint16_t*)o;
@@ -908,7 +931,12 @@ extern "C" int evo_attn_fwd_packed_bf16(const void* q, const void* k, const void
     a.dyn_pos = nullptr; a.part_o = nullptr; a.part_ml = nullptr; a.n_splits = 1;
     a.n_qblocks = (int)n_blocks;
     a.blocks = (const int4*)blocks;
-    return evo_attn_w64_packed_launch(a, valid, vt_ws, stream);
+    if (form == 2) return evo_attn_w64_packed_launch(a, valid, vt_ws, stream);
+    a.nbh = (int)H; a.q_pad = 0; a.vt = nullptr; a.vt_row = 0;
+    const dim3 grid((unsigned)(n_blocks * H));
+    if (form == 1) hipLaunchKernelGGL(attn_fwd_pipe_kernel<true>, grid, dim3(512), 0, (hipStream_t)stream, a);
+    else hipLaunchKernelGGL((attn_fwd_kernel<false, true>), grid, dim3(256), 0, (hipStream_t)stream, a);
+    return evo_launch_status();
 }
 
 extern "C" int evo_attn_decode_bf16(const void* q, const void* k, const void* v, void* o, int64_t B, int64_t H,

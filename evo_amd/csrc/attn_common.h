@@ -28,7 +28,7 @@ struct AttnArgs {
     int q_pad;                // attn_fwd_w64_kernel: query blocks are aligned to the END of the query range; block 0 starts at row -q_pad
     const uint16_t* vt;       // attn_fwd_w64_kernel: V^T [B][H][128][vt_row] (keys contiguous; written by attn_vt_kernel from v)
     int64_t vt_row;           // keys per row of vt (Tk rounded up to 64)
-    const int4* blocks;       // attn_fwd_w64_kernel<.., true>: the n_qblocks query blocks of unequal sequences behind each other: first row, length, first query (may be < 0)
+    const int4* blocks;       // PACKED kernels: the n_qblocks query blocks of unequal sequences behind each other: first row, length, first query (attn_fwd_w64_kernel: may be < 0)
 };
 
 // Workgroup -> (query block, head, batch) for the prefill kernel, 1-D grid.  Blocks are dispatched round-robin

@@ -852,8 +852,7 @@ int evo_attn_w64_launch(AttnArgs a, int64_t B, void* vt_ws, void* stream) {
 }
 
 // Unequal sequences behind each other, all their query blocks in one launch (evo_attn_fwd_packed_bf16 in csrc/attn.hip has checked the blocks): a launch per
-// sequence of a few hundred rows has 32 heads x 1 to 5 blocks for 256 CUs and lasts as long as its longest block.  16 sequences of 220 to 1,100 rows, 32 heads:
-// 16 x (40 + 6.5) us -> 245 + 37 us (the longest blocks, 1,100 keys, are a third of it).
+// sequence lasts as long as its longest block and leaves most CUs idle behind it.
 int evo_attn_w64_packed_launch(AttnArgs a, const int32_t* valid, void* vt_ws, void* stream) {
     a.nbh = a.H;
     a.q_pad = 0;

@@ -54,7 +54,7 @@ _SIGNATURES = {
     "evo_step_out": ([_PTR] * 2 + [_I64, _PTR] + [_I64] * 2 + [_PTR], _c.c_int),
     "evo_copy_rows": ([_PTR, _I64, _PTR], _c.c_int),
     "evo_hyena_ct_packed": ([_PTR] * 9 + [_I64] * 5 + [_PTR], _c.c_int),
-    "evo_attn_fwd_packed_bf16": ([_PTR] * 4 + [_I64] * 8 + [_PTR] * 2 + [_I64, _PTR, _F32, _PTR, _PTR], _c.c_int),
+    "evo_attn_fwd_packed_bf16": ([_PTR] * 4 + [_I64] * 9 + [_PTR] * 2 + [_I64, _PTR, _F32, _PTR, _PTR], _c.c_int),
     "evo_dense_ws": ([_I64] * 5, _c.c_int),
     "evo_dense_plan": ([_I64] * 5 + [_PTR], _c.c_int),
     "evo_dense_bf16": ([_I64] * 3 + [_PTR] * 7 + [_I64] * 8 + [_PTR, _I64, _PTR], _c.c_int),
@@ -104,7 +104,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 22         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 23         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):
@@ -1102,8 +1102,7 @@ class HipOps(MixerOps):
             self._need(out, torch.bfloat16, "attention out")
             assert tuple(out.shape) == (B, Tq, H, hd)
         o = torch.empty(B, Tq, H, hd, dtype=torch.bfloat16, device=q.device) if out is None else out
-        # query ranges longer than one 128-row block on many keys: the 64-rows-per-wave kernel, which reads V^T from a workspace its pre-pass fills
-        vt = torch.empty(B, H, hd, (Tk + 63) // 64 * 64, dtype=torch.bfloat16, device=q.device) if (Tq > 128 and Tk >= self.attn_w64_from and self.attn_w64) else None
+        vt = torch.empty(B, H, hd, (Tk + 63) // 64 * 64, dtype=torch.bfloat16, device=q.device) if self._attn_w64_takes(Tq, Tk) else None
         with self._t("attn_fwd"):
             _check(self.lib.evo_attn_fwd_causal_bf16(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), B, H, Tq, Tk, int(q_pos0),
@@ -1111,23 +1110,30 @@ class HipOps(MixerOps):
                 v.stride(0), v.stride(1), v.stride(2), 0.0 if prescaled else 1.0 / math.sqrt(hd), _ptr(vt), _stream()), "evo_attn_fwd_causal_bf16")
         return o
 
-    ATTN_QB = 256                # queries of a block of attention_packed (csrc/attn_w64.hip W_QB)
+    ATTN_QB = 256                # queries of a block of attention_packed (csrc/attn.hip PQB, csrc/attn_w64.hip W_QB); 128 where a sequence has no more
 
-    @staticmethod
-    def packed_blocks(first, lens, rows: int):
+    def _attn_w64_takes(self, Tq: int, Tk: int) -> bool:
+        """Query ranges longer than one 128-row block on many keys: the 64-rows-per-wave kernel, which reads V^T from a workspace that its pre-pass fills."""
+        return Tq > 128 and Tk >= self.attn_w64_from and self.attn_w64
+
+    def packed_blocks(self, first, lens, rows: int):
         """What attention_packed wants of sequences of `lens` tokens from row `first` (multiples of 64) of `rows` rows on -> (query blocks [n, 4] int32: first row,
-        length, first query, 0, in the order of their work; [ceil(rows / 64)] int32: the rows of every 64 that belong to a sequence), on the host."""
-        QB = HipOps.ATTN_QB
-        blocks = sorted((q0, f, m) for f, m in zip(first, lens) for q0 in range(m - (m + QB - 1) // QB * QB, m, QB))
+        length, first query, form, those of a form together and in the order of their work; [ceil(rows / 64)] int32: the rows of every 64 that belong to a sequence), on
+        the host.  A sequence takes the kernel (form) that it takes alone: its bits are the same in every batch."""
+        QB, blocks = self.ATTN_QB, []
+        for f, m in zip(first, lens):
+            form = 2 if self._attn_w64_takes(m, m) else int(m > 128)
+            blocks += [(form, q0, f, m) for q0 in range(m - (m + QB - 1) // QB * QB if form == 2 else 0, m, QB)]
         valid = [0] * ((rows + 63) // 64)
         for f, m in zip(first, lens):
             for i in range((m + 63) // 64):
                 valid[f // 64 + i] = min(64, m - 64 * i)
-        return torch.tensor([[f, m, q0, 0] for q0, f, m in blocks], dtype=torch.int32), torch.tensor(valid, dtype=torch.int32)
+        return torch.tensor([[f, m, q0, form] for form, q0, f, m in sorted(blocks)], dtype=torch.int32), torch.tensor(valid, dtype=torch.int32)
 
     def attention_packed(self, q, k, v, blocks, blocks_host, valid, out: torch.Tensor, prescaled: bool = False) -> None:
-        """Causal attention of unequal sequences behind each other, every one among its own rows; q, k, v [rows, H, 128] (strided views), out [rows, H * 128]; blocks, valid:
-        packed_blocks, on the device (and the blocks on the host).  Rows between the sequences stay as they are in `out`."""
+        """Causal attention of unequal sequences behind each other, every one among its own rows, a launch per kernel that they would take alone; q, k, v [rows, H, 128]
+        (strided views), out [rows, H * 128]; blocks, valid: packed_blocks, on the device (and the blocks on the host).  Rows between the sequences stay as they
+        are in `out`."""
         for t, nm in ((q, "q"), (k, "k"), (v, "v")):
             if not t.is_cuda or t.dtype != torch.bfloat16 or t.stride(-1) != 1:
                 raise RuntimeError(f"attention {nm}: need a ROCm bf16 tensor with a dense last dim")
@@ -1137,11 +1143,15 @@ class HipOps(MixerOps):
         for t, dev in ((blocks, q.device), (blocks_host, torch.device("cpu"))):
             assert t.dtype == torch.int32 and t.dim() == 2 and t.shape[1] == 4 and t.is_contiguous() and t.device == dev and t.shape == blocks.shape
         assert valid.dtype == torch.int32 and valid.is_contiguous() and valid.device == q.device and valid.numel() == (M + 63) // 64
-        vt = torch.empty(H, hd, (M + 63) // 64 * 64, dtype=torch.bfloat16, device=q.device)
-        with self._t("attn_fwd"):
-            _check(self.lib.evo_attn_fwd_packed_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), H, M, q.stride(0), q.stride(1), k.stride(0), k.stride(1),
-                                                     v.stride(0), v.stride(1), blocks.data_ptr(), blocks_host.data_ptr(), blocks.shape[0], valid.data_ptr(),
-                                                     0.0 if prescaled else 1.0 / math.sqrt(hd), vt.data_ptr(), _stream()), "evo_attn_fwd_packed_bf16")
+        forms = blocks_host[:, 3].tolist()
+        assert forms == sorted(forms)
+        for form in sorted(set(forms)):
+            at, n = forms.index(form), forms.count(form)
+            vt = torch.empty(H, hd, (M + 63) // 64 * 64, dtype=torch.bfloat16, device=q.device) if form == 2 else None
+            with self._t("attn_fwd"):
+                _check(self.lib.evo_attn_fwd_packed_bf16(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), H, M, q.stride(0), q.stride(1), k.stride(0), k.stride(1),
+                                                         v.stride(0), v.stride(1), form, blocks.data_ptr() + 16 * at, blocks_host.data_ptr() + 16 * at, n,
+                                                         valid.data_ptr(), 0.0 if prescaled else 1.0 / math.sqrt(hd), _ptr(vt), _stream()), "evo_attn_fwd_packed_bf16")
 
     def attention_decode(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                          pos: Optional[torch.Tensor] = None, n_splits: Optional[int] = None, prescaled: bool = False) -> torch.Tensor:

@@ -898,7 +898,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         if not self._packed:
             self._pack()
         ops = self.ops
-        ok = (self.device.type == "cuda" and getattr(ops, "hyena_mfma", False) and getattr(ops, "hyena_ct_flag", False) and hasattr(ops, "hyena_ct_packed") and getattr(ops, "attn_w64", True)
+        ok = (self.device.type == "cuda" and getattr(ops, "hyena_mfma", False) and getattr(ops, "hyena_ct_flag", False) and hasattr(ops, "hyena_ct_packed")
               and self.hidden_size == self.num_heads * 128 and ops.zt_shape_ok(1, self.packed_rows, 3 * self.hidden_size, self.hidden_size) and getattr(self, "block_taps", None) is None
               and all(isinstance(b, _AttentionBlock) or (b.projections.weight.is_contiguous() and b.projections.weight.dtype == torch.bfloat16
                                                          and self._table_ok(b)) for b in self.blocks))
@@ -917,7 +917,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
     def _prefill_packed(self, prompts: List[torch.Tensor]):
         """Prompts behind each other as ONE stream of rows, each from a multiple of 64 on (the rows between are token 0 and reach nobody: every
         launch is row-independent or keeps to one prompt's rows): the dense layers see all rows at once, the Hyena operator and the attention take
-        all prompts in one launch.  -> (final-norm rows, first row of every prompt, caches of every prompt, each of its own length)."""
+        all prompts in one launch, or one for each kernel that they would take alone.  -> (final-norm rows, first row of every prompt, caches of every prompt, each of its own length)."""
         ops, D, H, hd, K1 = self.ops, self.hidden_size, self.num_heads, self.head_dim, self.short_filter_length - 1
         dev, lens = self.device, [p.numel() for p in prompts]
         first, M = [], 0

@@ -63,8 +63,9 @@ extern "C" {
  *  19: evo_step_out added.
  *  20: evo_hyena_short gained `mask`.
  *  21: evo_linear_ring_share added.
- *  22: evo_lightning_chunk_bf16 and evo_rglru_chunk_bf16 keep the states of cut sequences only: `seg` by the rows, not by the sequences. */
-#define EVO_ABI_VERSION 22
+ *  22: evo_lightning_chunk_bf16 and evo_rglru_chunk_bf16 keep the states of cut sequences only: `seg` by the rows, not by the sequences.
+ *  23: evo_attn_fwd_packed_bf16 gained `form`. */
+#define EVO_ABI_VERSION 23
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
@@ -247,14 +248,15 @@ int evo_attn_fwd_causal_bf16(const void* q, const void* k, const void* v, void* 
                              int64_t k_sb, int64_t k_st, int64_t k_sh,
                              int64_t v_sb, int64_t v_st, int64_t v_sh,
                              float softmax_scale, void* vt_ws, void* stream);
-/* the same on unequal sequences behind each other in `rows` rows (strides as above without a batch), each from a multiple of 64 on, in one launch: blocks
- * [n_blocks][4] int32 (16-byte aligned) are the query blocks of 256 rows -- first row and length of their sequence, their first query in it (the last block of a sequence
- * ends with it, the first may begin before it: q0 > -256), one value unused --, the longest LAST (they run first); blocks_host the same on the host, checked before the launch;
- * valid [ceil(rows / 64)] int32 on the device: how many of the 64 rows from a multiple on belong to a sequence.  Rows between the sequences are not written.
- * vt_ws: H 128 (rows rounded up to 64) bf16. */
+/* the same on unequal sequences behind each other in `rows` rows (strides as above without a batch), each from a multiple of 64 on, in one launch of the kernel that a
+ * sequence alone takes: `form` 0: up to 128 queries, 1: more, without vt_ws, 2: more, with it.  A sequence's bits are those of evo_attn_fwd_causal_bf16.  blocks
+ * [n_blocks][4] int32 (16-byte aligned) are the query blocks of 128 (form 0) or 256 rows -- first row and length of their sequence, their first query in it (form 2:
+ * the last block of a sequence ends with it, the first may begin before it, q0 > -256; others: 0, 256, ..), one value unused --, the longest LAST (they run
+ * first); blocks_host the same on the host, checked before the launch.  Form 2 (NULL for others): valid [ceil(rows / 64)] int32 on the device: how many of the 64 rows from
+ * a multiple on belong to a sequence; vt_ws: H 128 (rows rounded up to 64) bf16.  Rows between the sequences are not written. */
 int evo_attn_fwd_packed_bf16(const void* q, const void* k, const void* v, void* o, int64_t H, int64_t rows, int64_t q_st, int64_t q_sh, int64_t k_st, int64_t k_sh,
-                             int64_t v_st, int64_t v_sh, const int32_t* blocks, const int32_t* blocks_host, int64_t n_blocks, const int32_t* valid, float softmax_scale,
-                             void* vt_ws, void* stream);
+                             int64_t v_st, int64_t v_sh, int64_t form, const int32_t* blocks, const int32_t* blocks_host, int64_t n_blocks, const int32_t* valid,
+                             float softmax_scale, void* vt_ws, void* stream);
 
 /* decode form (one query per sequence, Tq = 1): split-K over the key range ("flash-decoding") + combine.
  * replaces flash_attn_with_kvcache                           [REF evo/generation.py:109-110,138-155]

@@ -84,6 +84,35 @@ def test_attention(H, lens, prescaled, monkeypatch):
             ops.attention_packed(qkv[:, 0], qkv[:, 1], qkv[:, 2], t.to(DEV), t, valid.to(DEV), out)
 
 
+# a sequence on each kernel, at the edges between them (the line between 8 waves and 64 rows a wave lowered to 640 keys, and where it is)
+@pytest.mark.parametrize("H,lens,first", [(4, [1, 128, 129, 255, 256, 257, 639, 640, 641, 64, 1100], 640), (5, [128, 40], None), (32, [1030, 129, 513], None),
+                                          (4, [3499, 100, 3500, 3501, 1300], None)])
+@pytest.mark.parametrize("prescaled", [False, True])
+def test_attention_has_the_bits_of_each_sequence_alone(H, lens, first, prescaled, monkeypatch):
+    ops = _ops()
+    if first is not None:
+        monkeypatch.setattr(ops, "attn_w64_from", first, raising=False)
+    g = torch.Generator(device=DEV).manual_seed(sum(lens))
+    at, M = _places(lens)
+    qkv = torch.full((M, 3, H, 128), float("nan"), device=DEV, dtype=torch.bfloat16)
+    for f, m in zip(at, lens):
+        qkv[f:f + m] = torch.randn(m, 3, H, 128, device=DEV, generator=g).bfloat16()
+    blocks, valid = ops.packed_blocks(at, lens, M)
+    assert sorted(set(blocks[:, 3].tolist())) == sorted({0 if m <= 128 else 1 if m < (first or 3500) else 2 for m in lens})
+    out = torch.full((M, H * 128), 7.0, device=DEV, dtype=torch.bfloat16)
+    ops.attention_packed(qkv[:, 0], qkv[:, 1], qkv[:, 2], blocks.to(DEV), blocks, valid.to(DEV), out, prescaled=prescaled)
+    inside = torch.zeros(M, dtype=torch.bool, device=DEV)
+    for f, m in zip(at, lens):
+        inside[f:f + m] = True
+        q, k, v = (qkv[f:f + m, i][None] for i in range(3))
+        assert torch.equal(out[f:f + m], ops.attention(q, k, v, 0, prescaled=prescaled)[0].reshape(m, H * 128)), m
+    assert bool((out[~inside] == 7.0).all())
+    for bad in ([0, 100, 1, 0], [0, 300, 0, 0], [0, 300, 128, 1], [0, 300, 512, 1], [0, 100, 0, 1], [0, 300, 100, 2], [0, M + 64, 0, 1], [32, 300, 0, 1], [0, 300, 0, 3]):
+        t = torch.tensor([bad], dtype=torch.int32)
+        with pytest.raises(Exception):
+            ops.attention_packed(qkv[:, 0], qkv[:, 1], qkv[:, 2], t.to(DEV), t, valid.to(DEV), out)
+
+
 def test_copies():
     """Dense pieces, rows at a pitch, one element, nothing, sizes off 16 bytes, more pieces than one launch takes; what lies beside them stays."""
     ops = _ops()

@@ -79,3 +79,20 @@ def test_places_from_the_end_and_places_that_are_not_there():
             for bad in (len(group[0]), -len(group[0]) - 1):
                 with pytest.raises(IndexError):
                     m.prefill_rows(group, [[bad]] + [[0]] * (len(group) - 1))
+
+
+@pytest.mark.parametrize("dims", ["toy", "wide"])
+@pytest.mark.parametrize("n", [1024, 2304, 3584])
+def test_whole_row_tiles_have_the_same_bits_alone_and_packed(dims, n):
+    """A prompt of 1,024 tokens and more, a multiple of 256: its keys, values and states are the same bits alone and beside others, either side of 3,500 keys."""
+    _, _, m = build(dict(SMALL4 if dims == "toy" else WIDE))
+    p = prompts_of([n, 300, 700, 1200])
+    with torch.inference_mode():
+        _, alone, row = m.prefill_rows([p[0]])[0]
+        for at, group in ((0, [p[0], p[1]]), (1, [p[2], p[0], p[3]])):
+            assert len(m._prompt_groups([q.numel() for q in group])) == 1
+            _, ipd, r = m.prefill_rows(group)[at]
+            assert torch.equal(ipd["mha"].key_value_memory_dict[1][r, :n], alone["mha"].key_value_memory_dict[1][row, :n])
+            for i in m.hyena_layer_idxs:
+                a, b = (torch.view_as_real(d["hyena"].state_dict[i][k]) for d, k in ((ipd, r), (alone, row)))
+                assert torch.equal(a.reshape(b.shape), b)
