@@ -1251,11 +1251,13 @@ class HipOps(MixerOps):
         ok_mem = (x.is_cuda and x.dtype == torch.bfloat16 and wsrc.dtype == torch.bfloat16 and x.is_contiguous() and wsrc.is_contiguous()
                   and (norm_scale is None or (norm_scale.dtype == torch.bfloat16 and norm_scale.is_contiguous())))
         if (self.gate_small_m_mfma and not (one_launch and M <= 8 and K == 4096 and norm_scale is not None) and (5 <= M <= 64 or (3 <= M <= 4 and I * K >= 1 << 24)) and K % 128 == 0 and I % 32 == 0 and ok_mem
-                and (x.data_ptr() | wsrc.data_ptr()) % 16 == 0):
+                and wsrc.data_ptr() % 16 == 0):
             # 3-64 rows on the MFMA weight-streaming form with the gate in its epilogue (csrc/gemv.hip skinny_ring_kernel); the norm as its own small pass in
             # front (us at I = 11,008, K = 4,096, against the dot2 launch that norms for itself: 30.7 : 31.2 at 3 rows, 30.7 : 32.1 at 4, 30.7 : 45.0 at 8)
             if norm_scale is not None:
                 x = self.rmsnorm(x, None, norm_scale, eps)
+            elif x.data_ptr() % 16:
+                x = x.clone()                                     # (a few rows, for loads of 16 bytes)
             a = torch.empty(M, I, dtype=torch.bfloat16, device=x.device)
             with self._t("gemv_gate"):
                 _check(self.lib.evo_mlp_gate_small_m_bf16(x.data_ptr(), wsrc.data_ptr(), a.data_ptr(), M, I, K, grouped, code, _stream()),

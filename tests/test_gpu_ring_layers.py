@@ -71,3 +71,4 @@ def test_rows_off_16_bytes():
     u, v = want.float().bfloat16().double().split(N // 2, 1)
     gate = torch.nn.functional.gelu(u) * v
     assert ((ops.mlp_gate(x, w).double() - gate).norm() / gate.norm()).item() < 4e-3
+    assert torch.equal(ops.mlp_gate(x, None, w12g=ops.pack_gate_weights(w)), ops.mlp_gate(x.clone(), w))     # (copied to a place that they can)
