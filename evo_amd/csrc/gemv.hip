@@ -638,13 +638,14 @@ __global__ __launch_bounds__(256) void gemv_gate_kernel(const uint4* __restrict_
 //   x' = x + y / sqrt(mean(y^2) + eps) * (off + g)       (rows of the stream; workgroup 0 also stores them)
 //   SUM: x' = t / sqrt(mean(t^2) + eps) * (off + g), t = alpha x + y
 //   plain: z = bf16(x') . W^T (act 3: through the square of relu)         gated: a = act(bf16(x') . W1^T) * (bf16(x') . W2^T), w = [W1; W2] or its grouped order
-// Every workgroup rebuilds the M rows -- 8 bytes per element from L2 -- into LDS while its first weight requests are under way.
-template <int M, bool GATE, bool SUM>
+// Every workgroup rebuilds the row -- 8 bytes per element from L2 -- into LDS while its first weight requests are under way.  One row: with more the norm's own launch is
+// ahead (what both take: MixerOps.fuse_postnorm_ok).
+template <bool GATE, bool SUM>
 __global__ __launch_bounds__(256) void postnorm_gemv_kernel(const uint4* __restrict__ y, const uint4* __restrict__ g, const float4* __restrict__ x,
                                                             float4* __restrict__ x_out, const uint4* __restrict__ w, uint16_t* __restrict__ out, int N,
                                                             int nvec, float alpha, float eps, float off, int grouped, int act) {
-    extern __shared__ uint4 pn_x[];                              // [M][nvec]
-    __shared__ float red[M][4];
+    extern __shared__ uint4 pn_x[];                              // [nvec]
+    __shared__ float red[4];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t n0 = ((int64_t)blockIdx.x * 4 + wave) * (GATE ? 2 : 4);     // first output column of this wave
@@ -663,54 +664,44 @@ __global__ __launch_bounds__(256) void postnorm_gemv_kernel(const uint4* __restr
         wa[r] = ld_stream(wrow[r] + (lane < nvec ? lane : nvec - 1));
         wa[4 + r] = ld_stream(wrow[r] + (lane + 64 < nvec ? lane + 64 : nvec - 1));
     }
+    float ss = 0.f;
+    for (int v = tid; v < nvec; v += 256) {
+        const uint4 yv = y[v];
+        if (SUM) {
+            const float4 a = x[v * 2], b = x[v * 2 + 1];
+            const float t[8] = {fmaf(alpha, a.x, bf_lo(yv.x)), fmaf(alpha, a.y, bf_hi(yv.x)), fmaf(alpha, a.z, bf_lo(yv.y)), fmaf(alpha, a.w, bf_hi(yv.y)),
+                                fmaf(alpha, b.x, bf_lo(yv.z)), fmaf(alpha, b.y, bf_hi(yv.z)), fmaf(alpha, b.z, bf_lo(yv.w)), fmaf(alpha, b.w, bf_hi(yv.w))};
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-        float ss = 0.f;
-        for (int v = tid; v < nvec; v += 256) {
-            const uint4 yv = y[(int64_t)m * nvec + v];
-            if (SUM) {
-                const float4 a = x[((int64_t)m * nvec + v) * 2], b = x[((int64_t)m * nvec + v) * 2 + 1];
-                const float t[8] = {fmaf(alpha, a.x, bf_lo(yv.x)), fmaf(alpha, a.y, bf_hi(yv.x)), fmaf(alpha, a.z, bf_lo(yv.y)), fmaf(alpha, a.w, bf_hi(yv.y)),
-                                    fmaf(alpha, b.x, bf_lo(yv.z)), fmaf(alpha, b.y, bf_hi(yv.z)), fmaf(alpha, b.z, bf_lo(yv.w)), fmaf(alpha, b.w, bf_hi(yv.w))};
-#pragma unroll
-                for (int e = 0; e < 8; ++e) ss = fmaf(t[e], t[e], ss);
-            } else ss = gv_sumsq8(yv, ss);
-        }
-        ss = wave_sum(ss);
-        if (lane == 0) red[m][wave] = ss;
+            for (int e = 0; e < 8; ++e) ss = fmaf(t[e], t[e], ss);
+        } else ss = gv_sumsq8(yv, ss);
     }
+    ss = wave_sum(ss);
+    if (lane == 0) red[wave] = ss;
     __syncthreads();
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-        const float inv = 1.0f / sqrtf((red[m][0] + red[m][1] + red[m][2] + red[m][3]) / (float)(nvec * 8) + eps);
-        for (int v = tid; v < nvec; v += 256) {
-            const uint4 yv = y[(int64_t)m * nvec + v], gv = g[v];
-            float4 a = x[((int64_t)m * nvec + v) * 2], b = x[((int64_t)m * nvec + v) * 2 + 1];
-            if (SUM) {
-                a.x = fmaf(alpha, a.x, bf_lo(yv.x)) * inv * (off + bf_lo(gv.x)); a.y = fmaf(alpha, a.y, bf_hi(yv.x)) * inv * (off + bf_hi(gv.x));
-                a.z = fmaf(alpha, a.z, bf_lo(yv.y)) * inv * (off + bf_lo(gv.y)); a.w = fmaf(alpha, a.w, bf_hi(yv.y)) * inv * (off + bf_hi(gv.y));
-                b.x = fmaf(alpha, b.x, bf_lo(yv.z)) * inv * (off + bf_lo(gv.z)); b.y = fmaf(alpha, b.y, bf_hi(yv.z)) * inv * (off + bf_hi(gv.z));
-                b.z = fmaf(alpha, b.z, bf_lo(yv.w)) * inv * (off + bf_lo(gv.w)); b.w = fmaf(alpha, b.w, bf_hi(yv.w)) * inv * (off + bf_hi(gv.w));
-            } else {
+    const float inv = 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)(nvec * 8) + eps);
+    for (int v = tid; v < nvec; v += 256) {
+        const uint4 yv = y[v], gv = g[v];
+        float4 a = x[v * 2], b = x[v * 2 + 1];
+        if (SUM) {
+            a.x = fmaf(alpha, a.x, bf_lo(yv.x)) * inv * (off + bf_lo(gv.x)); a.y = fmaf(alpha, a.y, bf_hi(yv.x)) * inv * (off + bf_hi(gv.x));
+            a.z = fmaf(alpha, a.z, bf_lo(yv.y)) * inv * (off + bf_lo(gv.y)); a.w = fmaf(alpha, a.w, bf_hi(yv.y)) * inv * (off + bf_hi(gv.y));
+            b.x = fmaf(alpha, b.x, bf_lo(yv.z)) * inv * (off + bf_lo(gv.z)); b.y = fmaf(alpha, b.y, bf_hi(yv.z)) * inv * (off + bf_hi(gv.z));
+            b.z = fmaf(alpha, b.z, bf_lo(yv.w)) * inv * (off + bf_lo(gv.w)); b.w = fmaf(alpha, b.w, bf_hi(yv.w)) * inv * (off + bf_hi(gv.w));
+        } else {
             a.x += bf_lo(yv.x) * inv * (off + bf_lo(gv.x)); a.y += bf_hi(yv.x) * inv * (off + bf_hi(gv.x));
             a.z += bf_lo(yv.y) * inv * (off + bf_lo(gv.y)); a.w += bf_hi(yv.y) * inv * (off + bf_hi(gv.y));
             b.x += bf_lo(yv.z) * inv * (off + bf_lo(gv.z)); b.y += bf_hi(yv.z) * inv * (off + bf_hi(gv.z));
             b.z += bf_lo(yv.w) * inv * (off + bf_lo(gv.w)); b.w += bf_hi(yv.w) * inv * (off + bf_hi(gv.w));
-            }
-            pn_x[m * nvec + v] = make_uint4(pack_bf2(a.x, a.y), pack_bf2(a.z, a.w), pack_bf2(b.x, b.y), pack_bf2(b.z, b.w));
-            if (blockIdx.x == 0) {
-                x_out[((int64_t)m * nvec + v) * 2] = a;
-                x_out[((int64_t)m * nvec + v) * 2 + 1] = b;
-            }
+        }
+        pn_x[v] = make_uint4(pack_bf2(a.x, a.y), pack_bf2(a.z, a.w), pack_bf2(b.x, b.y), pack_bf2(b.z, b.w));
+        if (blockIdx.x == 0) {
+            x_out[v * 2] = a;
+            x_out[v * 2 + 1] = b;
         }
     }
     __syncthreads();
     if (n0 >= N) return;
-    float acc[4][M];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int m = 0; m < M; ++m) acc[r][m] = 0.f;
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
     int v = lane;
     for (; v + 64 < nvec; v += 128) {
         uint4 wb[8];
@@ -722,45 +713,34 @@ __global__ __launch_bounds__(256) void postnorm_gemv_kernel(const uint4* __restr
                 wb[4 + r] = ld_stream(wrow[r] + (v + 192 < nvec ? v + 192 : nvec - 1));
             }
         }
+        const uint4 x0 = pn_x[v], x1 = pn_x[v + 64];
 #pragma unroll
-        for (int m = 0; m < M; ++m) {
-            const uint4 x0 = pn_x[m * nvec + v], x1 = pn_x[m * nvec + v + 64];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[r][m] = dot8(wa[4 + r], x1, dot8(wa[r], x0, acc[r][m]));
-        }
+        for (int r = 0; r < 4; ++r) acc[r] = dot8(wa[4 + r], x1, dot8(wa[r], x0, acc[r]));
         if (more) {
 #pragma unroll
             for (int r = 0; r < 8; ++r) wa[r] = wb[r];
         }
     }
     if (v < nvec) {                                              // one vector left for this lane: its request is in wa already
+        const uint4 x0 = pn_x[v];
 #pragma unroll
-        for (int m = 0; m < M; ++m) {
-            const uint4 x0 = pn_x[m * nvec + v];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[r][m] = dot8(wa[r], x0, acc[r][m]);
-        }
+        for (int r = 0; r < 4; ++r) acc[r] = dot8(wa[r], x0, acc[r]);
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int m = 0; m < M; ++m) acc[r][m] = wave_sum(acc[r][m]);
+    for (int r = 0; r < 4; ++r) acc[r] = wave_sum(acc[r]);
     if (lane == 0) {
+        if (GATE) {
+            const f32x2_t u = {round_bf(acc[0]), round_bf(acc[1])}, z = {round_bf(acc[2]), round_bf(acc[3])};
+            const f32x2_t o = act_gate2(u, z, act);
+            out[n0] = f_to_bf(o[0]);
+            if (n0 + 1 < N) out[n0 + 1] = f_to_bf(o[1]);
+        } else {
 #pragma unroll
-        for (int m = 0; m < M; ++m) {
-            if (GATE) {
-                const f32x2_t u = {round_bf(acc[0][m]), round_bf(acc[1][m])}, z = {round_bf(acc[2][m]), round_bf(acc[3][m])};
-                const f32x2_t o = act_gate2(u, z, act);
-                out[(int64_t)m * N + n0] = f_to_bf(o[0]);
-                if (n0 + 1 < N) out[(int64_t)m * N + n0 + 1] = f_to_bf(o[1]);
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (n0 + r < N) {
-                        const float z = act ? fmaxf(acc[r][m], 0.f) : acc[r][m];
-                        out[(int64_t)m * N + n0 + r] = f_to_bf(act ? z * z : z);
-                    }
-            }
+            for (int r = 0; r < 4; ++r)
+                if (n0 + r < N) {
+                    const float z = act ? fmaxf(acc[r], 0.f) : acc[r];
+                    out[n0 + r] = f_to_bf(act ? z * z : z);
+                }
         }
     }
 }
@@ -770,19 +750,14 @@ static int postnorm_gemv_launch(const void* y, const void* g, const float* x, fl
     if (M < 1 || M > 4 || N <= 0 || N > 0x3fffffff || K <= 0 || K % 8 != 0 || K > 8192 || !y || !g || !x || !x_out || !w || !out || x == x_out) return -1;
     if (gate ? ((act != 0 && act != 1) || (grouped && N % 32 != 0)) : (act != 0 && act != 3)) return -1;
     const dim3 grid((unsigned)((N + (gate ? 7 : 15)) / (gate ? 8 : 16))), block(256);
-    const size_t lds = (size_t)M * K * 2;                        // (<= 64 KB)
-#define EVO_PN(MM, G, S) hipLaunchKernelGGL((postnorm_gemv_kernel<MM, G, S>), grid, block, lds, (hipStream_t)stream, (const uint4*)y, (const uint4*)g,    \
-                                            (const float4*)x, (float4*)x_out, (const uint4*)w, (uint16_t*)out, (int)N, (int)(K / 8), alpha, eps, off, \
-                                            grouped ? 1 : 0, (int)act)
-#define EVO_PN1(MM) do { if (gate) { if (sum) EVO_PN(MM, true, true); else EVO_PN(MM, true, false); }                       \
-                         else { if (sum) EVO_PN(MM, false, true); else EVO_PN(MM, false, false); } } while (0)
-    switch (M) {
-        case 1: EVO_PN1(1); break;
-        case 2: EVO_PN1(2); break;
-        case 3: EVO_PN1(3); break;
-        default: EVO_PN1(4); break;
+    const size_t lds = (size_t)K * 2;                            // (<= 16 KB)
+#define EVO_PN(G, S) hipLaunchKernelGGL((postnorm_gemv_kernel<G, S>), grid, block, lds, (hipStream_t)stream, (const uint4*)y + m * (K / 8), (const uint4*)g,    \
+                                        (const float4*)x + m * (K / 4), (float4*)x_out + m * (K / 4), (const uint4*)w, (uint16_t*)out + m * N, (int)N, (int)(K / 8), \
+                                        alpha, eps, off, grouped ? 1 : 0, (int)act)
+    for (int64_t m = 0; m < M; ++m) {
+        if (gate) { if (sum) EVO_PN(true, true); else EVO_PN(true, false); }
+        else { if (sum) EVO_PN(false, true); else EVO_PN(false, false); }
     }
-#undef EVO_PN1
 #undef EVO_PN
     return evo_launch_status();
 }

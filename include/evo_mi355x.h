@@ -407,7 +407,7 @@ int evo_norm_mlp_gate_small_m_bf16(const void* x, const void* scale, const void*
  * x_out = t / sqrt(mean(t^2) + eps) * (w_offset + g), t = alpha x + y                              (sum 1),
  * fp32 [M, K] (x_out is another buffer than x), and on its bf16 rounding
  *   z [M, N] = x_out . w^T, through the square of relu with act 3 (0: none), or        a [M, I] = act(x_out . W1^T) * (x_out . W2^T)   (w12, grouped, act as in evo_mlp_gate_small_m_bf16)
- * y [M, K], g [K] bf16; 1 <= M <= 4, K % 8 == 0, K <= 8192. */
+ * y [M, K], g [K] bf16; 1 <= M <= 4 (a launch per row: with more than one, evo_postnorm_residual or evo_sum_norm and the layer are ahead), K % 8 == 0, K <= 8192. */
 int evo_postnorm_linear_small_m_bf16(const void* y, const void* g, const float* x, float* x_out, const void* w, void* z, int64_t M, int64_t N,
                                      int64_t K, float alpha, int64_t sum, float eps, float w_offset, int64_t act, void* stream);
 int evo_postnorm_mlp_gate_small_m_bf16(const void* y, const void* g, const float* x, float* x_out, const void* w12, void* a, int64_t M, int64_t I,
