@@ -766,9 +766,10 @@ class HipOps(MixerOps):
     @staticmethod
     def _hyena_short_ok(B, T, z, z_halo, poles, residues) -> bool:
         """One launch (csrc/hyena.hip hyena_short_kernel) for the rows and alignments that it takes, while its 3.5 + B (0.9 + 0.033 T) us at 4,096 channels, every
-        batch row a round of workgroups, are less than the 21 + 0.021 B T us of the three launches (12 x 41 positions: 33 against 36 us; 32 x 41: 78 against 45; 18 x 5: 28 against 21).
+        batch row a round of workgroups, are less than the 21 + 0.021 B T us of the three launches (12 x 41 positions: 33 against 36 us; 32 x 41: 78 against 45; 18 x 5: 28 against 21).  Wider layers take as
+        many rounds more (8,192 channels: 1 x 500 40 against 40, 1 x 1,000 67 against 57, 12 x 41 62 against 51), narrower ones are ahead by more (1,024: 12 x 41 11 against 23).
         From 1,024 positions on a row's bits are the same in every batch (row groups of a pass): those stay with the three launches."""
-        return (B * T < 1024 and B * (T + 75) <= 1450 and (B <= 8 or T >= 41) and z.data_ptr() % 16 == 0 and (z_halo is None or z_halo.data_ptr() % 16 == 0) and poles.data_ptr() % 8 == 0
+        return (B * T < 1024 and B * (T + 75) * max(z.shape[-1], 3 * 4096) <= 1450 * 3 * 4096 and (B <= 8 or T >= 41) and z.data_ptr() % 16 == 0 and (z_halo is None or z_halo.data_ptr() % 16 == 0) and poles.data_ptr() % 8 == 0
                 and residues.data_ptr() % 8 == 0)
 
     def hyena_prefill(self, z: torch.Tensor, fir_w: torch.Tensor, fir_b: torch.Tensor, poles: torch.Tensor,

@@ -137,3 +137,16 @@ def test_decode_attention_in_one_launch_where_caches_are_short():
         assert whole(256, 1 << 20, maps, dim, dv) and not whole(79, 64, maps, dim, dv)
         for groups, ring in ((80, few), (159, few), (160, more), (255, more)):
             assert whole(groups, ring, maps, dim, dv) and not whole(groups, 2 * ring, maps, dim, dv)
+
+
+def test_short_rows_by_their_width():
+    """The Hyena operator in one launch: up to 4,096 channels as measured there, less of wider layers, whose rows take more rounds of workgroups; never from 1,024 positions on."""
+    import torch
+    p = torch.zeros(8)
+
+    def short(B, T, D):
+        return evo_ops.HipOps._hyena_short_ok(B, T, torch.empty(B, T, 3 * D, dtype=torch.bfloat16, device="meta"), None, p, p)
+    for D in (128, 1024, 4096):
+        assert short(1, 5, D) and short(1, 1023, D) and short(12, 41, D) and short(6, 161, D) and short(8, 90, D)
+        assert not short(1, 1024, D) and not short(2, 512, D) and not short(32, 41, D) and not short(18, 5, D)
+    assert short(1, 500, 8192) and short(2, 161, 8192) and not short(1, 1000, 8192) and not short(12, 41, 8192) and not short(2, 500, 8192)
