@@ -178,10 +178,10 @@ def test_lightning_segments_of_unequal_sequences(ops, H, dk, dv, lens):
                              st, seg_len=128)
     st = states.clone()
     torch.cuda.reset_peak_memory_stats()
-    before = torch.cuda.memory_allocated()
+    before = torch.cuda.memory_stats()["requested_bytes.all.current"]
     o = run(z, list(range(len(lens))), st)
     slots = sum(lens) // 128 + min(len(lens), sum(lens) // 128)
-    assert torch.cuda.max_memory_allocated() - before <= o.numel() * 2 + slots * H * dk * dv * 4 + (1 << 16)
+    assert torch.cuda.memory_stats()["requested_bytes.all.peak"] - before <= o.numel() * 2 + slots * H * dk * dv * 4 + (1 << 16)
     at = 0
     for b, n in enumerate(lens):
         alone = states[b:b + 1].clone()
