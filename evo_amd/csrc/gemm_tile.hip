@@ -6,7 +6,7 @@
 // and a CU holds about 64 KB in flight.  Hence large tiles (bytes per product fall with the tile's sides), parts of K where large tiles are too few
 // for the chip, and weight lines shared by neighbours on one XCD.  The MFMA order over k is the persistent kernel's, so an unsplit product is bit
 // for bit the same on every tile; parts of K are fp32 sums added in order by a second launch.
-// Below 256 rows the tiles of neighbouring weight rows start one k-step apart (`turn`) and go round: rows lie a power of two apart, so tiles that walk k in step
+// Below 256 rows and above 2,048 k the tiles of neighbouring weight rows start one k-step apart (`turn`) and go round: rows lie a power of two apart, so tiles that walk k in step
 // meet in the same L2 channels.  us at 65 / 161 rows, K = 4,096: 22,016 gated columns 47.1 / 56.8 -> 39.3 / 51.5, 12,288 columns 31.6 / 35.8 -> 26.7 / 33.3;
 // K = 11,008, 4,096 columns 30.8 / 34.6 -> 27.4 / 32.9.  (From 256 rows on, where it gives 3 to 6 %, the gated, the ungated and the blocked forms of a layer agree bit
 // for bit, whichever tiles they take.)
@@ -70,7 +70,7 @@ __device__ __forceinline__ void t_scale_bias(float (&v)[8], const GemmArgs& a, f
 __host__ __device__ __forceinline__ int64_t t_stat_rows(const GemmArgs& a) { return a.M; }
 
 template <int BM, int BN, int WGM, int WGN, int NS, int PER_CU, int MODE, bool XB, bool SPLIT>
-__global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_tile_kernel(GemmArgs a, int act, float* parts, int splits, int turn) {
+__global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_tile_kernel(GemmArgs a, int act, float* parts, int splits) {
     constexpr int NW = WGM * WGN, WM = BM / WGM, WN = BN / WGN, MT = WM / 16, NT = WN / 16;
     constexpr int PX = BM / 8 / NW, PW = BN / 8 / NW, P = PX + PW;      // DMA pieces (8 rows, 1 KiB) of a stage per wave
     constexpr int SLAB_X = BM * T_ROW, STAGE = (BM + BN) * T_ROW;
@@ -158,11 +158,14 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
     const t_u32x4 rw = {(uint32_t)wa, (uint32_t)(wa >> 32) & 0xffffu, (uint32_t)(w_ok * kb), 0x00020000u};
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
 
-    // piece `i` (of P) of stage `s` -> ring slot at byte `slot`; past the last stage the last one again, into a slot nobody reads (constant counts)
-    const int start = turn * (MODE == 3 ? tm : tn) % nk;
+    // piece `i` (of P) of k-step `s` -> ring slot at byte `slot`; past the last stage the last one again, into a slot nobody reads (constant counts)
+    int at = k0, past = 1;                                       // k-step of the next stage to fetch, stages fetched after it
+    if (a.turn) at += (MODE == 3 ? tm : tn) % nk;
+    auto next = [&] {
+        if (past < nk) at = at + 1 == k0 + nk ? k0 : at + 1;
+        ++past;
+    };
     auto fetch1 = [&](int s, uint32_t slot, int i) {
-        s = start + (s < nk ? s : nk - 1);
-        s = k0 + (s < nk ? s : s - nk);
         const uint32_t dst = lds0 + slot + wave * 1024;
         if (i < PX)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
@@ -193,7 +196,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
 #pragma unroll
         for (int j = 0; j < MT; ++j) T_DSR(xf[kh][j], xa_, j * 16 * T_ROW);
     };
-    // the products of one half of a k-step; `dma`: with the P pieces of stage `s` between them
+    // the products of one half of a k-step; `dma`: with the P pieces of k-step `s` between them
     auto mma = [&](int kh, bool dma, int s, uint32_t fslot) {
         constexpr int TOTAL = NT * MT;
 #pragma unroll
@@ -218,9 +221,11 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
     //        half 1   the first fragments of stage k + 1 are requested; products of the second half
     uint32_t slot = 0, nslot = STAGE, fslot = (NS - 1) * STAGE;
 #pragma unroll
-    for (int s = 0; s < NS - 1; ++s)
+    for (int s = 0; s < NS - 1; ++s) {
 #pragma unroll
-        for (int i = 0; i < P; ++i) fetch1(s, s * STAGE, i);
+        for (int i = 0; i < P; ++i) fetch1(at, s * STAGE, i);
+        next();
+    }
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * P) : "memory");
     asm volatile("s_barrier" ::: "memory");
     read(0, 0);
@@ -229,8 +234,9 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
         t_lgkm<NT + MT>(wf[0]);
         t_lgkm<NT + MT>(xf[0]);
         __builtin_amdgcn_sched_barrier(0);
-        mma(0, true, k + NS - 1, fslot);
+        mma(0, true, at, fslot);
         __builtin_amdgcn_sched_barrier(0);
+        next();
         t_lgkm<0>(wf[1]);
         t_lgkm<0>(xf[1]);
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * P) : "memory");
@@ -544,13 +550,13 @@ static int tile_plan(int64_t M, int64_t N, int64_t K, int mode, bool stats, bool
 }
 
 template <int BM, int BN, int WGM, int WGN, int NS, int PER_CU, bool GATE>
-static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, int turn, float* ws, hipStream_t st) {
+static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, float* ws, hipStream_t st) {
     a.tiles_m = (int)((a.M + BM - 1) / BM);
     a.tiles_n = (a.N + BN - 1) / BN;
     a.group_m = 8;
     a.n_tiles = a.tiles_m * a.tiles_n * splits;
     const dim3 grid((unsigned)a.n_tiles), block(64 * WGM * WGN);
-#define T_GO(MODE, XB, SPLIT) hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, NS, PER_CU, MODE, XB, SPLIT>), grid, block, 0, st, a, act, ws, splits, turn)
+#define T_GO(MODE, XB, SPLIT) hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, NS, PER_CU, MODE, XB, SPLIT>), grid, block, 0, st, a, act, ws, splits)
     if (splits == 1) {
         if (mode == 3) T_GO(3, false, false);
         else if (mode == 1) { if constexpr (GATE) T_GO(1, false, false); else return -1; }
@@ -572,12 +578,12 @@ static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, int
 }
 
 template <int BM, int BN, int WGM, int WGN, int NS, int MODE>
-static int tile_launch_odd(GemmArgs a, int act, int turn, hipStream_t st) {
+static int tile_launch_odd(GemmArgs a, int act, hipStream_t st) {
     a.tiles_m = (int)((a.M + BM - 1) / BM);
     a.tiles_n = (a.N + BN - 1) / BN;
     a.group_m = 8;
     a.n_tiles = a.tiles_m * a.tiles_n;
-    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, NS, 1, MODE, false, false>), dim3((unsigned)a.n_tiles), dim3(64 * WGM * WGN), 0, st, a, act, nullptr, 1, turn);
+    hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, NS, 1, MODE, false, false>), dim3((unsigned)a.n_tiles), dim3(64 * WGM * WGN), 0, st, a, act, nullptr, 1);
     return evo_launch_status();
 }
 
@@ -640,7 +646,9 @@ extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const voi
             n = dense_plan(mode, sumsq != nullptr, M, N, K, false, plan);
             break;
         }
-    const int turn = M < 256 ? 1 : 0;                            // (from 256 rows on the order of k is the persistent kernel's)
+    // (from 256 rows on the order of k is the persistent kernel's.  us, in step -> in turn: K = 2,048, 4,096 columns 8.5 -> 9.1 at 65 rows, 22,016 24.8 -> 23.4; [W1; W2] as it is
+    //  with halves a power of two apart, 8,192 gated columns 37.3 -> 42.7)
+    const int turn = M < 256 && K > 2048 && !(mode == 2 && (N & (N - 1)) == 0) ? 1 : 0;
     int64_t m0 = 0;
     for (int i = 0; i < n; ++i) {
         const TilePlan& t = plan[i];
@@ -661,7 +669,7 @@ extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const voi
             GemmArgs a;
             a.x = xi; a.w = (const unsigned char*)w; a.bias = (const uint16_t*)bias; a.res = ri; a.y = yi;
             a.M = t.rows; a.N = (int)N; a.K = (int)K;
-            a.rs = si; a.ss = qi; a.ss_ld = ss_ld; a.act_cols = act ? (int)act_cols : 0;
+            a.rs = si; a.ss = qi; a.ss_ld = ss_ld; a.act_cols = act ? (int)act_cols : 0; a.turn = turn;
             if (mode == 2) a.w_rows = N;
             if (mode == 3) {                                     // the rows of the launch are the weight's, its columns the tokens
                 a.x = (const unsigned char*)w; a.w = (const unsigned char*)x;
@@ -671,16 +679,16 @@ extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const voi
             const int tm = mode == 2 ? 1 : (int)mode;
             float* f = (float*)ws;
             hipStream_t st = (hipStream_t)stream;
-            if (t.kind == 0) rc = tile_launch<64, 64, 2, 2, 5, 2, false>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
-            else if (t.kind == 1) rc = tile_launch<128, 64, 4, 1, 3, 2, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
-            else if (t.kind == 2) rc = tile_launch<128, 128, 4, 2, 5, 1, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
-            else if (t.kind == 3) rc = tile_launch<192, 128, 4, 2, 4, 1, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
-            else if (t.kind == 4) rc = tile_launch<256, 128, 4, 2, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
-            else if (t.kind == 5) rc = tile_launch<128, 256, 2, 4, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, turn, f, st);
+            if (t.kind == 0) rc = tile_launch<64, 64, 2, 2, 5, 2, false>(a, tm, (int)act, xblk != 0, t.splits, f, st);
+            else if (t.kind == 1) rc = tile_launch<128, 64, 4, 1, 3, 2, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
+            else if (t.kind == 2) rc = tile_launch<128, 128, 4, 2, 5, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
+            else if (t.kind == 3) rc = tile_launch<192, 128, 4, 2, 4, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
+            else if (t.kind == 4) rc = tile_launch<256, 128, 4, 2, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
+            else if (t.kind == 5) rc = tile_launch<128, 256, 2, 4, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
             else if (xblk || tm > 1 || (tm == 1) != (t.kind < T_ODD + 2)) rc = -1;
-            else if (t.kind == T_ODD) rc = tile_launch_odd<96, 96, 2, 3, 6, 1>(a, (int)act, turn, st);
-            else if (t.kind == T_ODD + 1) rc = tile_launch_odd<192, 96, 4, 3, 4, 1>(a, (int)act, turn, st);
-            else rc = tile_launch_odd<96, 48, 3, 1, 8, 0>(a, (int)act, turn, st);
+            else if (t.kind == T_ODD) rc = tile_launch_odd<96, 96, 2, 3, 6, 1>(a, (int)act, st);
+            else if (t.kind == T_ODD + 1) rc = tile_launch_odd<192, 96, 4, 3, 4, 1>(a, (int)act, st);
+            else rc = tile_launch_odd<96, 48, 3, 1, 8, 0>(a, (int)act, st);
         }
         if (rc != 0) return rc;
         m0 += t.rows;

@@ -307,3 +307,22 @@ def test_gate_on_a_weight_of_more_than_4_gib():
         want, got = torch.nn.functional.gelu(z1) * z2, y[:, 256 * i:256 * i + z1.shape[1]].double()
         err = (got - want).abs()
         assert bool((err <= want.abs() * 2.0 ** -7 + (z1.abs() + 0.2) * z2.abs() * 2.0 ** -7 + 1e-3).all()), (i, err.max().item())             # (as test_gate)
+
+
+@pytest.mark.parametrize("K", [2048, 2112])
+@pytest.mark.parametrize("N", [16384, 12288])
+def test_gate_either_side_of_the_staggered_starts(N, K):
+    """Tiles in step up to 2,048 k and where halves of [W1; W2] lie a power of two apart, otherwise a k-step apart."""
+    from evo_amd.ops import _stream
+    ops = _ops()
+    M = 65
+    g, x, w = _data(M, N, K, 11)
+    z = (x.double() @ w.double().T).bfloat16().double()
+    z1, z2 = z[:, :N // 2], z[:, N // 2:]
+    want = torch.nn.functional.gelu(z1) * z2
+    for order in (1, 2):
+        wk, y = ops.pack_gate_weights(w) if order == 1 else w, torch.full((M + 3, N // 2), 7.0, device="cuda", dtype=torch.bfloat16)
+        assert ops.lib.evo_dense_bf16(order, 0, 0, x.data_ptr(), wk.data_ptr(), None, None, y.data_ptr(), None, None, 0, M, N, K, 0, 0, 0, 0, None, 0, _stream()) == 0
+        err = (y[:M].double() - want).abs()
+        assert bool((err <= want.abs() * 2.0 ** -7 + (z1.abs() + 0.2) * z2.abs() * 2.0 ** -7 + 1e-3).all()), err.max().item()              # (as test_gate)
+        assert bool((y[M:] == 7).all())
