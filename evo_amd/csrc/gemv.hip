@@ -905,7 +905,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kw_kernel(const unsigned ch
         off[i] = (uint32_t)r * rowb + (uint32_t)((lane % GR) ^ (r & 15 & (GR - 1))) * 16u;
     }
     const int chunks = K / CH, mine = (chunks - wave + WAVES - 1) / WAVES;
-    const int start = mine > 0 && gridDim.x >= 128 ? (int)(blockIdx.x >> 3) * 3 % mine : 0;       // (workgroups of an XCD don't walk K in step: skinny_ring_kernel)
+    const int start = mine > 4 && gridDim.x >= 128 ? (int)(blockIdx.x >> 3) * 3 % mine : 0;       // (workgroups of an XCD don't walk K in step: skinny_ring_kernel)
     auto fetch = [&](int i, uint32_t buf) {
         i = start + i >= mine ? start + i - mine : start + i;
         const uint32_t so = (uint32_t)(wave + WAVES * i) * ROW;
@@ -990,7 +990,7 @@ static int kw_launch(const void* x, const void* w, const void* bias, const void*
     return evo_launch_status();
 }
 
-// ---- 3 to 64 rows on the wide layers (and, with parts of K, on the narrow ones from 17 rows on): a workgroup owns N / gridDim.x weight rows (any number up to
+// ---- 3 to 64 rows on the wide layers (and, with parts of K, on those of up to 8,192 columns from 17 rows on): a workgroup owns N / gridDim.x weight rows (any number up to
 // 16 T, a wave per 16 of them) and walks K in chunks of 128; weight and batch rows of a chunk arrive in LDS by asynchronous loads (no registers) into a ring
 // of NB stages, NB - 1 of them under way, one barrier per chunk.  LDS rows of 256 B, granule g of row r at slot g ^ (r & 15): a fragment read meets no bank twice.
 // What bounds it is the weight stream, under three conditions that decide the layout (us, MI355X, launches back to back; a plain read of the matrix in brackets):
@@ -1182,12 +1182,14 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
     *(uint2*)(y + e) = out;
 }
 
-// Ring launches.  Rows per workgroup: what 256 CUs get each, in as few rounds as 96 rows (T = 6) allow, at least 32; T: waves for them.  Stages: four (42 KB
-// each at T = 6 and 64 batch rows: three).
-template <int XR, int T, int MODE>
+// Ring launches.  Rows per workgroup: up to 24,576 columns what 256 CUs get each, at least 32; more columns are rounds of up to 64 rows; T: waves for them.  Stages: four
+// (42 KB each at T = 6 and 64 batch rows: three); of several rounds three, two at 64 batch rows, so that a CU starts its next workgroup while one ends.  us at 5 / 16 / 32 / 64
+// rows, rounds of up to 96 rows and four stages -> this: 28,672 x 1,024 11.6 / 12.3 / 15.4 / 20.0 -> 11.4 / 12.2 / 13.7 / 16.7, 50,304 x 1,024 22.4 / 24.1 / 27.1 / 33.0 ->
+// 18.4 / 19.7 / 23.4 / 31.4, 65,536 x 4,096 78 / 80 / 86 / 102 -> 79 / 78 / 80 / 95, 151,936 x 512 34 / 40 / 47 / 59 -> 28 / 32 / 38 / 55 (x 4,096 179 / 192 / 214 / 251 ->
+// 182 / 191 / 216 / 263).
+template <int XR, int T, int MODE, int NB>
 static int ring_go(dim3 grid, const void* x, const void* w, const void* bias, const void* res, void* y, int64_t M, int64_t N, int64_t K, int act, int layout, float* ws,
                    hipStream_t s) {
-    constexpr int NB = T == 6 && XR == 64 ? 3 : 4;
     constexpr size_t lds = (size_t)NB * T * (16 * RG_ROWB + (XR / 4 + T - 1) / T * 1024);
     static_assert(lds <= 160 * 1024, "the CU's LDS");
     if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)skinny_ring_kernel<XR, T, NB, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -1196,8 +1198,8 @@ static int ring_go(dim3 grid, const void* x, const void* w, const void* bias, co
     return evo_launch_status();
 }
 static int64_t ring_groups(int64_t N) {
-    const int64_t rounds = (N + 256 * 96 - 1) / (256 * 96), share = (N + 31) / 32;
-    return share < 256 ? share : 256 * rounds;
+    const int64_t share = (N + 31) / 32;
+    return share < 256 ? share : N <= 256 * 96 ? 256 : 256 * ((N + 256 * 64 - 1) / (256 * 64));
 }
 static int ring_waves(int64_t N) {
     const int64_t groups = ring_groups(N), rows = (N + groups - 1) / groups;
@@ -1220,10 +1222,15 @@ static int ring_launch(const void* x, const void* w, const void* bias, const voi
                        hipStream_t s) {
     const int waves = ring_waves(N);
     const dim3 grid((unsigned)(parts ? N / 64 : ring_groups(N)), (unsigned)(parts ? parts : 1));
-#define EVO_RG(XR, T) ring_go<XR, T, MODE>(grid, x, w, bias, res, y, M, N, K, act, layout, ws, s)
-#define EVO_RG1(T) (M <= 16 ? EVO_RG(16, T) : M <= 32 ? EVO_RG(32, T) : EVO_RG(64, T))
-    if (MODE == 2) return EVO_RG1(4);
-    return waves == 2 ? EVO_RG1(2) : waves == 3 ? EVO_RG1(3) : waves == 4 ? EVO_RG1(4) : EVO_RG1(6);
+#define EVO_RG(XR, T, NB) ring_go<XR, T, MODE, NB>(grid, x, w, bias, res, y, M, N, K, act, layout, ws, s)
+#define EVO_RG1(T) (M <= 16 ? EVO_RG(16, T, 4) : M <= 32 ? EVO_RG(32, T, 4) : EVO_RG(64, T, (T == 6 ? 3 : 4)))
+#define EVO_RGN(T) (M <= 16 ? EVO_RG(16, T, 3) : M <= 32 ? EVO_RG(32, T, 3) : EVO_RG(64, T, 2))
+    if constexpr (MODE == 2) return EVO_RG1(4);
+    else {
+        if (grid.x > 256) return waves == 3 ? EVO_RGN(3) : EVO_RGN(4);         // (33 to 64 rows)
+        return waves == 2 ? EVO_RG1(2) : waves == 3 ? EVO_RG1(3) : waves == 4 ? EVO_RG1(4) : EVO_RG1(6);
+    }
+#undef EVO_RGN
 #undef EVO_RG1
 #undef EVO_RG
 }
@@ -1382,10 +1389,15 @@ extern "C" int evo_norm_mlp_gate_small_m_bf16(const void* x, const void* scale, 
     return mlp_gate_launch(x, scale, w12, a, M, I, K, eps, grouped, 0, (hipStream_t)stream);
 }
 
-// narrow layers, 16 rows a CU: parts of K where the batch rows would be read more often than the weights; a workgroup per CU.  0: one sum
+// Parts of K where the batch rows would be read more often than the weights, 64 weight rows a workgroup and no more workgroups than CUs (each takes a CU's LDS: a second
+// round of a few costs as much as the first).  0: one sum.  us at 33 / 64 rows, one sum (up to 8,192 columns) or one part more (3,072) -> this: 3,072 x 4,096 14.6 / 17.0 ->
+// 10.9 / 12.7, 4,160 x 8,192 28.7 / 29.9 -> 17.7 / 20.9, 5,120 x 11,008 37.1 / 39.9 -> 24.7 / 27.7, 6,912 x 4,096 16.6 / 17.6 -> 14.8 / 17.7, x 8,192 29.2 / 31.1 -> 23.3 / 28.0,
+// 8,192 x 8,192 29.6 / 31.5 -> 25.6 / 29.3, but x 2,048 10.3 / 11.4 -> 11.2 / 13.4.  At 17 / 32 rows two parts are not ahead: 5,120 x 11,008 27.6 / 29.6 -> 23.6 / 24.4 in
+// three, 6,912 x 11,008 29.2 / 31.6 -> 32.3 / 33.4 in two.
 static int small_m_parts(int64_t M, int64_t N, int64_t K) {
-    if (M < 17 || M > 64 || N > 4096 || N < 1024 || N % 64 != 0 || K < 1024 || K % 128 != 0 || K > 0x9fffff || (K < 8192 && M <= 32)) return 0;
-    int64_t parts = (256 + N / 64 - 1) / (N / 64);
+    if (M < 17 || M > 64 || N > 8192 || N < 1024 || N % 64 != 0 || K < 1024 || K % 128 != 0 || K > 0x9fffff || (K < 8192 && M <= 32) || (N > 4096 && K < 4096)) return 0;
+    int64_t parts = 256 / (N / 64);
+    if (N > 4096 && M <= 32 && parts < 3) return 0;
     if (parts > K / 256) parts = K / 256;
     if (parts > 8) parts = 8;
     return parts >= 2 ? (int)parts : 0;
@@ -1407,8 +1419,6 @@ extern "C" int evo_linear_small_m_bf16(const void* x, const void* w, const void*
     if ((M >= 5 || (M >= 3 && K % 128 == 0 && (N <= 4096 ? N >= 2048 && K >= 2048 : N >= 16384))) && K % 32 == 0) {
         // (asynchronous loads of 16 bytes; an offset of 96 rows, 64 batch rows or 16 weight rows in 32 bits)
         if (K % 128 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0 && K <= 0x9fffff) {
-            // wide layers
-            if (N > 4096) return ring_launch<0>(x, w, bias, residual, y, M, N, K, (int)act, 0, nullptr, 0, s);
             const int64_t parts = ws && ((uintptr_t)ws & 15) == 0 ? small_m_parts(M, N, K) : 0;
             if (parts && ws_bytes >= parts * M * N * 4) {
                 const int rc = ring_launch<2>(x, w, nullptr, nullptr, nullptr, M, N, K, 0, 0, (float*)ws, (int)parts, s);
@@ -1417,6 +1427,8 @@ extern "C" int evo_linear_small_m_bf16(const void* x, const void* w, const void*
                                    (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)parts, (int)act);
                 return evo_launch_status();
             }
+            // wide layers
+            if (N > 4096) return ring_launch<0>(x, w, bias, residual, y, M, N, K, (int)act, 0, nullptr, 0, s);
             // (few workgroups, the unembedding's 512 columns: more waves in each -- us at 8 / 16 / 32 rows, K = 4,096: 6.0 / 6.8 / 8.4, with four 6.1 / 6.9 / 8.8)
             if (N < 2048) {
                 if (M <= 8) return kw_launch<8, 8, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);
@@ -1425,6 +1437,7 @@ extern "C" int evo_linear_small_m_bf16(const void* x, const void* w, const void*
             }
             if (M <= 8) return kw_launch<8, 4, 128, 3>(x, w, bias, residual, y, M, N, K, (int)act, s);
             if (M <= 16) return kw_launch<16, 4, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);
+            if (M <= 32 && K <= 1024) return kw_launch<32, 4, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);     // (a chunk or two a wave: 3.6 -> 3.3 us at 512)
             if (M <= 32) return kw_launch<32, 3, 128, 2>(x, w, bias, residual, y, M, N, K, (int)act, s);
         }
         // what is left (K not in whole chunks): two n tiles per workgroup (every x fragment feeds two weight fragments) where that still leaves a workgroup or more per CU

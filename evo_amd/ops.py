@@ -430,9 +430,9 @@ class HipOps(MixerOps):
         M, K = x.shape
         N = w.shape[0]
         y = res if res is not None else (out if out is not None else torch.empty(M, N, dtype=torch.bfloat16, device=x.device))
-        # 17-64 rows on a narrow layer: a workspace for the partial sums of the split over K (csrc/gemv.hip skinny_ring_kernel, MODE 2); up to 32 rows only
-        # where K is long
-        ws = torch.empty(8 * M * N, dtype=torch.float32, device=x.device) if (M > (16 if K >= 8192 else 32) and 1024 <= N <= 4096 and K % 128 == 0 and N % 64 == 0) else None
+        # 17-64 rows on a layer of up to 8,192 columns: a workspace for the partial sums of the split over K (csrc/gemv.hip skinny_ring_kernel, MODE 2)
+        parts = self.lib.evo_linear_parts(M, N, K) if M > 16 else 0
+        ws = torch.empty(parts * M * N, dtype=torch.float32, device=x.device) if parts > 0 else None
         with self._t("gemv"):
             _check(self.lib.evo_linear_small_m_bf16(x.data_ptr(), w.data_ptr(), _ptr(b), _ptr(res), y.data_ptr(),
                                                     M, N, K, _ptr(ws), 0 if ws is None else ws.numel() * 4, act, _stream()), "evo_linear_small_m_bf16")
@@ -442,8 +442,8 @@ class HipOps(MixerOps):
         """The fp32 parts [parts, M, N] of x @ w^T that `linear` would add and round in a launch of their own (MixerOps.closing_parts_ does both for a closing norm),
         or None where it takes one sum."""
         M, K = x.shape
-        if M > 64 or not self._use_small_m(x, w) or (x.data_ptr() | w.data_ptr()) % 16:
-            return None
+        if M > 64 or w.shape[0] > 4096 or not self._use_small_m(x, w) or (x.data_ptr() | w.data_ptr()) % 16:
+            return None                                           # (wider rows: the parts are more for a norm's one workgroup a row to add than for a launch of their own)
         n = self.lib.evo_linear_parts(M, w.shape[0], K)
         if n <= 0:
             return None

@@ -283,7 +283,7 @@ int evo_attn_decode_bf16(const void* q, const void* k, const void* v, void* o,
  * M = 4 (M = 2 on layers that the other form is ahead on), v_mfma_f32_16x16x32_bf16 with the batch rows on the MFMA's N side from there -- one to four tiles
  * of 16 rows per weight pass (17-64 rows: the pooled decode step of 17-64 live streams); `residual` may alias `y`.  With K % 128 == 0 and x, w 16-byte aligned
  * weight and batch rows reach LDS by asynchronous loads of whole row pieces (csrc/gemv.hip skinny_ring_kernel, skinny_kw_kernel).
- * `ws` (ABI 10; may be NULL): a 16-byte aligned fp32 workspace of `ws_bytes` >= 8 M N 4 bytes lets the narrow layers (N <= 4096) at
+ * `ws` (ABI 10; may be NULL): a 16-byte aligned fp32 workspace of `ws_bytes` >= 8 M N 4 bytes lets layers of up to 8,192 columns at
  * 17-64 rows split K over workgroups -- partial sums through ws, added in a fixed order by a second small launch; without it they run the k-split form.
  * act 3: the square of relu before the rounding (0: none). */
 int evo_linear_small_m_bf16(const void* x, const void* w, const void* bias, const void* residual, void* y,

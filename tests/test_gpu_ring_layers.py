@@ -36,8 +36,24 @@ def test_linear(M, N, K, extra):
     assert bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + (1e-3 if extra else 4e-3)).all())        # (the square's slope is up to 8)
 
 
+# several rounds of workgroups, of three and of four waves; parts of K on 4,097 to 8,192 columns, and the sizes around them that take one sum
+@pytest.mark.parametrize("M", [5, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K,few,many", [(24578, 256, 0, 0), (33024, 640, 0, 0), (50304, 384, 0, 0), (4160, 8192, 3, 3), (5120, 4096, 0, 3), (5504, 8192, 0, 2), (8192, 4224, 0, 2),
+                                          (8192, 3968, 0, 0), (3072, 8320, 5, 5), (8256, 8192, 0, 0)])
+def test_linear_in_rounds_and_parts(M, N, K, few, many):
+    from evo_amd.ops import default_ops
+    ops = default_ops()
+    assert ops.lib.evo_linear_parts(M, N, K) == (0 if M < 17 else few if M <= 32 else many)
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x, w = _framed(M, K, g), _framed(N, K, g, K ** -0.5)
+    b, r = torch.randn(N, device=DEV, generator=g).bfloat16(), torch.randn(M + 1, N, device=DEV, generator=g).bfloat16()
+    keep = r.clone()
+    got, want = ops._linear_small_m(x, w, b, r[:M]), x.double() @ w.double().T + b.double() + keep[:M].double()
+    assert torch.equal(r[M], keep[M]) and bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + 1e-3).all())
+
+
 @pytest.mark.parametrize("M", [3, 5, 16, 17, 33, 64])
-@pytest.mark.parametrize("I,K", [(32, 128), (96, 384), (2080, 256), (5504, 1152), (8224, 2176), (12320, 1408)])
+@pytest.mark.parametrize("I,K", [(32, 128), (96, 384), (2080, 256), (5504, 1152), (8224, 2176), (12320, 1408), (16416, 256)])
 @pytest.mark.parametrize("grouped", [False, True])
 def test_gate(M, I, K, grouped):
     from evo_amd.ops import default_ops
