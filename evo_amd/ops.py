@@ -1189,11 +1189,12 @@ class HipOps(MixerOps):
 
     def norm_linear(self, x: torch.Tensor, scale: torch.Tensor, eps: float, w: torch.Tensor,
                     b: Optional[torch.Tensor] = None, mfma: bool = False, one_launch: bool = False) -> torch.Tensor:
-        """linear(rmsnorm(x) * scale, w, b).  Decode-sized batches (M <= 4; `one_launch`, the rows that a scoring batch leaves over: <= 8 at K = 4,096) with a wide
-        layer take ONE weight-streaming launch that rebuilds the normalised row on the fly; everything else is the two kernels."""
+        """linear(rmsnorm(x) * scale, w, b).  Decode-sized batches (M <= 4, 6 at K = 4,096 and up to 8,192 columns; `one_launch`, the rows that a scoring batch leaves over: <= 8 at
+        K = 4,096) with a wide layer take ONE weight-streaming launch that rebuilds the normalised row on the fly; everything else is the two kernels."""
         M, K = x.shape
-        # (five rows and more: the norm's own launch and the matrix cores' form are ahead -- 20.5 -> 19.3 us at 5 rows and 12,288 x 4,096, 26.5 -> 19.3 at 8)
-        if ((1 <= M <= 4 or (one_launch and M <= 8 and K == 4096)) and w.shape[0] > 4096 and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
+        # (five rows and more: the norm's own launch and the matrix cores' form are ahead -- 20.0 -> 19.8 us at 5 rows and 12,288 x 4,096, 25.0 -> 19.8 at 8 --, up to
+        # 8,192 columns from seven on: 15.7 : 16.8 at 5, 16.2 : 16.9 at 6, 17.3 : 16.9 at 8)
+        if ((1 <= M <= 4 or (M <= (8 if one_launch else 6 if w.shape[0] <= 8192 else 4) and K == 4096)) and w.shape[0] > 4096 and x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
                 and scale.dtype == torch.bfloat16 and x.is_contiguous() and w.is_contiguous() and scale.is_contiguous()
                 and K % 8 == 0):
             y = torch.empty(M, w.shape[0], dtype=torch.bfloat16, device=x.device)
@@ -1251,10 +1252,11 @@ class HipOps(MixerOps):
             return a
         ok_mem = (x.is_cuda and x.dtype == torch.bfloat16 and wsrc.dtype == torch.bfloat16 and x.is_contiguous() and wsrc.is_contiguous()
                   and (norm_scale is None or (norm_scale.dtype == torch.bfloat16 and norm_scale.is_contiguous())))
-        if (self.gate_small_m_mfma and not (one_launch and M <= 8 and K == 4096 and norm_scale is not None) and (5 <= M <= 64 or (3 <= M <= 4 and I * K >= 1 << 24)) and K % 128 == 0 and I % 32 == 0 and ok_mem
+        if (self.gate_small_m_mfma and not (one_launch and M <= 8 and K == 4096 and norm_scale is not None) and (5 <= M <= 64 or (3 <= M <= 4 and I * K >= (1 << 24 if norm_scale is None else 40000000))) and K % 128 == 0 and I % 32 == 0 and ok_mem
                 and wsrc.data_ptr() % 16 == 0):
             # 3-64 rows on the MFMA weight-streaming form with the gate in its epilogue (csrc/gemv.hip skinny_ring_kernel); the norm as its own small pass in
-            # front (us at I = 11,008, K = 4,096, against the dot2 launch that norms for itself: 30.7 : 31.2 at 3 rows, 30.7 : 32.1 at 4, 30.7 : 45.0 at 8)
+            # front (us at I = 11,008, K = 4,096, against the dot2 launch that norms for itself: 30.7 : 31.2 at 3 rows, 30.7 : 32.1 at 4, 30.7 : 45.0 at 8; 8,192
+            # 29.0 : 26.1 and 29.1 : 27.3, 4,096 15.4 : 14.1 and 15.4 : 14.9)
             if norm_scale is not None:
                 x = self.rmsnorm(x, None, norm_scale, eps)
             elif x.data_ptr() % 16:
