@@ -535,7 +535,8 @@ __global__ __launch_bounds__(512) void latent_up_kernel(const float* __restrict_
 // The same on the matrix cores (bf16, R % 32 == 0): 128 value rows of one head and NS sequences, a wave owns 16 of the rows.  Latency and the pace of one CU bound
 // it: at 8 sequences of 16 parts a head's merge reads 262 KB, its rows 131 KB.  So sequences are spread over up to 256 workgroups (a head's rows are read by
 // several), and the first 512 columns of the rows are asked for before the parts.
-// latent_absorb to here, 32 heads, R = 512, 900 slots, in a graph: 3 / 8 / 16 / 32 sequences 28.0 / 34.9 / 39.4 / 48.0 -> 25.7 / 30.6 / 32.3 / 37.2 us.
+// latent_absorb to here, 32 heads, R = 512, 900 slots, in a graph: 3 / 8 / 16 / 32 sequences 28.0 / 34.9 / 39.4 / 48.0 -> 23.8 / 27.9 / 29.9 / 36.7 us; of 64 x 128
+// 14.4 / 16.4 / 19.2 / 22.3 -> 14.4 / 15.9 / 17.4 / 20.3.
 template <int NS>
 __global__ __launch_bounds__(512) void latent_up_mfma_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, const float* __restrict__ sink,
                                                              const uint16_t* __restrict__ w, uint16_t* __restrict__ o, int B, int H, int R, int dv, int n_split) {
@@ -545,9 +546,10 @@ __global__ __launch_bounds__(512) void latent_up_mfma_kernel(const float* __rest
     float* wt = (float*)(lat + NS * pr);
     const int v0 = blockIdx.x * 128 + 16 * wave;
     const uint16_t* wr = w + ((int64_t)h * dv + (v0 + c16 < dv ? v0 + c16 : dv - 1)) * R + 8 * g;
-    uint4 first[16];
+    mx_u32x4 first[16];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) first[k] = *(const uint4*)(wr + (32 * k < R ? 32 * k : 0));
+    for (int k = 0; k < 16; ++k)
+        if (32 * k < R) first[k] = *(const mx_u32x4*)(wr + 32 * k);
     for (int i = wave; i < NS; i += 8) {
         const int b = b0 + i < B ? b0 + i : B - 1;
         const float* ml = part_ml + ((int64_t)b * H + h) * n_split * 2;
@@ -560,14 +562,22 @@ __global__ __launch_bounds__(512) void latent_up_mfma_kernel(const float* __rest
     for (int it = tid; it < NS * (R / 4); it += 512) {
         const int i = it / (R / 4), r = it % (R / 4) * 4, b = b0 + i < B ? b0 + i : B - 1;
         const float* po = part_o + ((int64_t)b * H + h) * n_split * R + r;
-        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll 8
-        for (int s = 0; s < n_split; ++s) {
-            const float4 x = *(const float4*)(po + (int64_t)s * R);
-            const float f = wt[i * n_split + s];
-            acc.x = fmaf(x.x, f, acc.x); acc.y = fmaf(x.y, f, acc.y); acc.z = fmaf(x.z, f, acc.z); acc.w = fmaf(x.w, f, acc.w);
+        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < n_split; s += 8) {                   // (eight requests on their way together: left to itself the compiler waits for each)
+            f32x4_t x[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) x[u] = *(const f32x4_t*)(po + (int64_t)(s + u < n_split ? s + u : n_split - 1) * R);
+#pragma unroll
+            for (int u = 0; u < 8; ++u) asm volatile("" : "+v"(x[u]));
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                if (s + u >= n_split) break;
+                const float f = wt[i * n_split + s + u];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] = fmaf(x[u][e], f, acc[e]);
+            }
         }
-        *(uint2*)(lat + i * pr + r) = make_uint2(pack_bf2(acc.x, acc.y), pack_bf2(acc.z, acc.w));
+        *(uint2*)(lat + i * pr + r) = make_uint2(pack_bf2(acc[0], acc[1]), pack_bf2(acc[2], acc[3]));
     }
     __syncthreads();
     if (v0 >= dv) return;
