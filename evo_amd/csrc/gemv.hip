@@ -1392,10 +1392,10 @@ extern "C" int evo_norm_mlp_gate_small_m_bf16(const void* x, const void* scale, 
 // Parts of K where the batch rows would be read more often than the weights, 64 weight rows a workgroup and no more workgroups than CUs (each takes a CU's LDS: a second
 // round of a few costs as much as the first).  0: one sum.  us at 33 / 64 rows, one sum (up to 8,192 columns) or one part more (3,072) -> this: 3,072 x 4,096 14.6 / 17.0 ->
 // 10.9 / 12.7, 4,160 x 8,192 28.7 / 29.9 -> 17.7 / 20.9, 5,120 x 11,008 37.1 / 39.9 -> 24.7 / 27.7, 6,912 x 4,096 16.6 / 17.6 -> 14.8 / 17.7, x 8,192 29.2 / 31.1 -> 23.3 / 28.0,
-// 8,192 x 8,192 29.6 / 31.5 -> 25.6 / 29.3, but x 2,048 10.3 / 11.4 -> 11.2 / 13.4.  At 17 / 32 rows two parts are not ahead: 5,120 x 11,008 27.6 / 29.6 -> 23.6 / 24.4 in
+// 8,192 x 8,192 29.6 / 31.5 -> 25.6 / 29.3, but x 4,096 16.4 / 17.7 -> 15.9 / 18.4, x 2,048 10.3 / 11.4 -> 11.2 / 13.4.  At 17 / 32 rows two parts are not ahead: 5,120 x 11,008 27.6 / 29.6 -> 23.6 / 24.4 in
 // three, 6,912 x 11,008 29.2 / 31.6 -> 32.3 / 33.4 in two.
 static int small_m_parts(int64_t M, int64_t N, int64_t K) {
-    if (M < 17 || M > 64 || N > 8192 || N < 1024 || N % 64 != 0 || K < 1024 || K % 128 != 0 || K > 0x9fffff || (K < 8192 && M <= 32) || (N > 4096 && K < 4096)) return 0;
+    if (M < 17 || M > 64 || N > 8192 || N < 1024 || N % 64 != 0 || K < 1024 || K % 128 != 0 || K > 0x9fffff || (K < 8192 && M <= 32) || (N > 4096 && K < (N <= 7168 ? 4096 : 8192))) return 0;
     int64_t parts = 256 / (N / 64);
     if (N > 4096 && M <= 32 && parts < 3) return 0;
     if (parts > K / 256) parts = K / 256;

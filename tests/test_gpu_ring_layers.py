@@ -38,8 +38,8 @@ def test_linear(M, N, K, extra):
 
 # several rounds of workgroups, of three and of four waves; parts of K on 4,097 to 8,192 columns, and the sizes around them that take one sum
 @pytest.mark.parametrize("M", [5, 17, 32, 33, 64])
-@pytest.mark.parametrize("N,K,few,many", [(24578, 256, 0, 0), (33024, 640, 0, 0), (50304, 384, 0, 0), (4160, 8192, 3, 3), (5120, 4096, 0, 3), (5504, 8192, 0, 2), (8192, 4224, 0, 2),
-                                          (8192, 3968, 0, 0), (3072, 8320, 5, 5), (8256, 8192, 0, 0)])
+@pytest.mark.parametrize("N,K,few,many", [(24578, 256, 0, 0), (33024, 640, 0, 0), (50304, 384, 0, 0), (4160, 8192, 3, 3), (5120, 4096, 0, 3), (5504, 8192, 0, 2), (6912, 4224, 0, 2),
+                                          (8192, 8320, 0, 2), (8192, 4224, 0, 0), (6912, 3968, 0, 0), (3072, 8320, 5, 5), (8256, 8192, 0, 0)])
 def test_linear_in_rounds_and_parts(M, N, K, few, many):
     from evo_amd.ops import default_ops
     ops = default_ops()
