@@ -1252,7 +1252,13 @@ class HipOps(MixerOps):
             return a
         ok_mem = (x.is_cuda and x.dtype == torch.bfloat16 and wsrc.dtype == torch.bfloat16 and x.is_contiguous() and wsrc.is_contiguous()
                   and (norm_scale is None or (norm_scale.dtype == torch.bfloat16 and norm_scale.is_contiguous())))
-        if (self.gate_small_m_mfma and not (one_launch and M <= 8 and K == 4096 and norm_scale is not None) and (5 <= M <= 64 or (3 <= M <= 4 and I * K >= (1 << 24 if norm_scale is None else 40000000))) and K % 128 == 0 and I % 32 == 0 and ok_mem
+        # narrow layers of long rows: 16 columns a workgroup or parts of K, and the gate behind them, fill more of the chip than one launch's N / 32 workgroups (us, one
+        # launch : two, and with the columns of regrouped weights put back, at 8 / 32 / 64 rows: 1,024 x 4,096 11.3 : 8.7 : 11.7, 12.9 : 11.3 : 14.4, 17.6 : 14.2 : 18.2;
+        # x 8,192 19.0 : 11.8 : 15.0, 21.9 : 14.9 : 18.5, 29.8 : 16.9 : 20.5; 2,048 x 3,072 9.9 : 8.8, 11.2 : 10.6, 15.2 : 14.8; x 2,176 8.1 : 7.7, 9.3 : 9.1, 12.3 : 14.0;
+        # x 1,536 6.9 : 7.0, 7.7 : 7.7, 10.2 : 12.6; 2,816 x 8,192 20.3 : 23.3, 23.3 : 25.5, 30.9 : 29.5; 256 x 4,096 11.0 : 8.1, 12.8 : 10.5, 17.4 : 24.5)
+        narrow = 2 * I <= 4096
+        apart = 5 <= M <= 64 and narrow and (K >= 8192 if grouped else K > 2048 if M <= 32 else K >= 3072) and (2 * I >= 1024 or M <= 32)
+        if (self.gate_small_m_mfma and not apart and not (one_launch and M <= 8 and K == 4096 and norm_scale is not None) and (5 <= M <= 64 or (3 <= M <= 4 and I * K >= (1 << 24 if norm_scale is None else 40000000))) and K % 128 == 0 and I % 32 == 0 and ok_mem
                 and wsrc.data_ptr() % 16 == 0):
             # 3-64 rows on the MFMA weight-streaming form with the gate in its epilogue (csrc/gemv.hip skinny_ring_kernel); the norm as its own small pass in
             # front (us at I = 11,008, K = 4,096, against the dot2 launch that norms for itself: 30.7 : 31.2 at 3 rows, 30.7 : 32.1 at 4, 30.7 : 45.0 at 8; 8,192
@@ -1266,7 +1272,7 @@ class HipOps(MixerOps):
                 _check(self.lib.evo_mlp_gate_small_m_bf16(x.data_ptr(), wsrc.data_ptr(), a.data_ptr(), M, I, K, grouped, code, _stream()),
                        "evo_mlp_gate_small_m_bf16")
             return a
-        if ((1 <= M <= 4 or (M <= 8 and K == 4096 and norm_scale is not None)) and x.is_cuda and x.dtype == torch.bfloat16 and wsrc.dtype == torch.bfloat16 and x.is_contiguous()
+        if ((1 <= M <= 4 or (M <= 8 and K == 4096 and norm_scale is not None and (one_launch or not apart))) and x.is_cuda and x.dtype == torch.bfloat16 and wsrc.dtype == torch.bfloat16 and x.is_contiguous()
                 and wsrc.is_contiguous() and K % 8 == 0 and I % 2 == 0 and (not grouped or I % 32 == 0)
                 and (norm_scale is None or (norm_scale.dtype == torch.bfloat16 and norm_scale.is_contiguous()))):
             a = torch.empty(M, I, dtype=torch.bfloat16, device=x.device)
@@ -1287,7 +1293,7 @@ class HipOps(MixerOps):
             with self._t("gemm_gate"):
                 self._dense_layer(1 if grouped else 2, x, wsrc, a, M, 2 * I, K, act=code)
             return a
-        if grouped and 5 <= M <= 64 and K % 128 == 0:             # (a column's sums follow its place there: the rows back in their order)
+        if grouped and 5 <= M <= 64 and K % 128 == 0 and not narrow:             # (a column's sums follow its place there: the rows back in their order)
             wsrc, grouped = wsrc.view(I // 32, 2, 32, K).transpose(0, 1).reshape(2 * I, K), 0
         g = self.linear(x, wsrc, None)
         if grouped:                                               # columns come out as [32 of z1 | the same 32 of z2] per block: back to [z1 | z2]

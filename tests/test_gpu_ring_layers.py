@@ -74,6 +74,32 @@ def test_gate(M, I, K, grouped):
         assert ((got.double() - want).norm() / want.norm()).item() < 4e-3
 
 
+@pytest.mark.parametrize("I,K,M,names", [(1024, 2176, 8, 2), (2048, 3072, 64, 2), (256, 8192, 32, 2), (1376, 8320, 17, 2), (256, 4096, 33, 1), (1024, 2048, 8, 1),
+                                         (1024, 2944, 33, 1), (2080, 4096, 8, 1), (1024, 4096, 4, 1)])
+@pytest.mark.parametrize("grouped", [False, True])
+def test_gate_of_narrow_layers(I, K, M, names, grouped):
+    """Up to 2,048 gated columns of long rows: the layer and the gate in a launch each; regrouped weights from K = 8,192 on."""
+    from evo_amd.ops import default_ops
+    ops = default_ops()
+    g = torch.Generator(device=DEV).manual_seed(M + I + K)
+    x, w = _framed(M, K, g), _framed(2 * I, K, g, 1.5 * K ** -0.5).contiguous()
+    ran, real = [], ops._t
+    ops._t = lambda name: (ran.append(name), real(name))[1]
+    try:
+        wg = ops.pack_gate_weights(w) if grouped else None
+        got, plain = ops.mlp_gate(x, None if grouped else w, w12g=wg), ran[:]
+        scale = torch.rand(K, generator=g, device=DEV).bfloat16() + 0.5
+        normed, want_n = ops.mlp_gate(x, None if grouped else w, scale, 1e-6, w12g=wg), ops.mlp_gate(ops.rmsnorm(x, None, scale, 1e-6), None if grouped else w, w12g=wg)
+    finally:
+        del ops._t
+    assert M < 5 or torch.equal(normed, want_n)
+    assert plain == (["gemv", "gelu_gate"] if names == 2 and (not grouped or K >= 8192) else ["gemv_gate"])
+    z = (x.double() @ w.double().T).float().bfloat16().double()
+    want = torch.nn.functional.gelu(z[:, :I]) * z[:, I:]
+    assert bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -6 + 2e-3 * want.abs().max()).all())            # (as test_gate)
+    assert ((got.double() - want).norm() / want.norm()).item() < 4e-3
+
+
 def test_rows_off_16_bytes():
     """Operands that the asynchronous loads can't take keep the other forms."""
     from evo_amd.ops import default_ops
