@@ -13,49 +13,14 @@
 // and writes the three 16-byte pieces to the planes of an LDS stage; rows of 64 B with the piece index XORed by (row >> 2) & 3: 16 lanes reading one
 // piece of 16 rows touch every bank once.  One stage and two barriers per step: the workgroups that share a CU split and multiply in turn (two
 // stages and one barrier at 256 x 128 were 1.1 to 1.3 times as slow: one workgroup per CU).
-#include "common.h"
+#include "gemm_f32.h"
 #include "../../include/evo_mi355x.h"
-#define F3_BK 32
 #define F3_ROWB 64
 
 struct F3Args {
     const float* x; const float* w; const float* bias; float* y; float* parts;
     int64_t M; int N, K, tiles_m, tiles_n, n_tiles, group_m, splits;
 };
-
-__device__ __forceinline__ void f3_split(const float4 a, const float4 b, uint4& h, uint4& m, uint4& l) {
-    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    uint32_t o[3][4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        o[0][e] = pack_bf2(v[2 * e], v[2 * e + 1]);
-        float r0 = v[2 * e] - bf_lo(o[0][e]), r1 = v[2 * e + 1] - bf_hi(o[0][e]);
-        o[1][e] = pack_bf2(r0, r1);
-        r0 -= bf_lo(o[1][e]);
-        r1 -= bf_hi(o[1][e]);
-        o[2][e] = pack_bf2(r0, r1);
-    }
-    h = make_uint4(o[0][0], o[0][1], o[0][2], o[0][3]);
-    m = make_uint4(o[1][0], o[1][1], o[1][2], o[1][3]);
-    l = make_uint4(o[2][0], o[2][1], o[2][2], o[2][3]);
-}
-
-// Outputs taken again with the fp32 matrix instructions, by the wave that holds them.  An infinite operand has no parts (inf - inf), one near the largest value
-// rounds to an infinite h, and the bf16 instructions take parts and sums under 2^-126 as zero: an operand loses at most 2^-124, an output of K products at
-// most K 2^-124 (|x| + |w| + 2), |x| and |w| the largest of its rows.  What is not finite or under 2^26 of that is taken again; a row without a value other
-// than zero is right as it is.  A wave takes a few one after the other, many as a product of its whole part.  (300 x 4,096 x 4,096, 88 us: with a NaN in one
-// row 118, in all rows 224 -- 2,400 and 16,450 output by output --; the maxima and the look at the outputs cost 1 %.)
-__device__ __forceinline__ void f3_row_max(float& m, const float4 a, const float4 b) {
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(a.x), "v"(a.y));
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(a.z), "v"(a.w));
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(b.x), "v"(b.y));
-    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(b.z), "v"(b.w));
-}
-// the least and the largest magnitude so far (the largest is NaN once a value was)
-__device__ __forceinline__ void f3_range(float& lo, float& hi, float a, float b) {
-    asm("v_min3_f32 %0, %0, |%1|, |%2|" : "+v"(lo) : "v"(a), "v"(b));
-    asm("v_maximum3_f32 %0, %0, |%1|, |%2|" : "+v"(hi) : "v"(a), "v"(b));
-}
 
 template <int BM, int BN, int WGM, int WGN, int PER_CU, bool SPLIT>
 __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_f32_kernel(F3Args a) {
@@ -191,106 +156,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_f
             }
         look |= !(lo >= fmaf(least, wide, fmaf(least, fmaxf(row_max[r], 0.f), least)) && hi <= 3.402823466e38f);
     }
-    if (__builtin_amdgcn_ballot_w64(look) == 0) return;
-    uint32_t odd[(TM * TN + 1) / 2] = {};                      // which ones: 16 outputs of each of two products
-    int n_odd = 0;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-        const int r = wm * (BM / WGM) + i * 32 + l31;
-        if (m0 + r >= a.M) continue;
-        const float bound = fmaf(least, row_max[r], least);
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int c = wn * (BN / WGN) + j * 32 + q * 8 + half * 4;
-                if (n0 + c >= a.N) continue;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float u = fabsf(acc[i][j][4 * q + e]);
-                    odd[(i * TN + j) >> 1] |= (u >= fmaf(least, row_max[BM + c + e], bound) && u <= 3.402823466e38f ? 0u : 1u) << (((i * TN + j) & 1) * 16 + 4 * q + e);
-                }
-            }
-    }
-#pragma unroll
-    for (uint32_t w : odd) n_odd += __popc(w);
-#pragma unroll
-    for (int d = 1; d < 64; d *= 2) n_odd += __shfl_xor(n_odd, d, 64);
-    if (n_odd == 0) return;
-    if (n_odd <= 8 * TM * TN) {                                // a few (sums that cancel to zero): one after the other, the wave along k
-#pragma unroll
-        for (int s = 0; s < (TM * TN + 1) / 2; ++s)
-            for (uint64_t lanes = __builtin_amdgcn_ballot_w64(odd[s] != 0); lanes; lanes &= lanes - 1) {
-                const int owner = __builtin_ctzll(lanes);
-                for (uint32_t bits = (uint32_t)__builtin_amdgcn_readlane((int)odd[s], owner); bits; bits &= bits - 1) {
-                    const int t = __builtin_ctz(bits), ij = 2 * s + (t >> 4), i = ij / TN, j = ij - i * TN;
-                    const int64_t m = m0 + wm * (BM / WGM) + i * 32 + (owner & 31);
-                    const int n = n0 + wn * (BN / WGN) + j * 32 + ((t >> 2) & 3) * 8 + (owner >> 5) * 4 + (t & 3);
-                    const float *x = a.x + m * a.K, *w = a.w + (int64_t)n * a.K;
-                    float sum = 0.f;
-#pragma unroll 4
-                    for (int k = k0 * F3_BK + 4 * lane; k < k1 * F3_BK; k += 256) {
-                        const f32x4_t u = *(const f32x4_t*)(x + k), v = *(const f32x4_t*)(w + k);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) sum = fmaf(u[e], v[e], sum);
-                    }
-                    sum = wave_sum(sum);
-                    if (lane == owner) *at(m, n) = !SPLIT && a.bias ? sum + a.bias[n] : sum;
-                }
-            }
-        return;
-    }
-    // lane (l31, half): four neighbouring k of its rows per request, a product of two k per component, as both operands take them
-    const float *xr[TM], *wr[TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-        const int64_t m = m0 + wm * (BM / WGM) + i * 32 + l31;
-        xr[i] = a.x + (m < a.M ? m : a.M - 1) * a.K + (int64_t)k0 * F3_BK + half * 4;
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        const int n = n0 + wn * (BN / WGN) + j * 32 + l31;
-        wr[j] = a.w + (int64_t)(n < a.N ? n : a.N - 1) * a.K + (int64_t)k0 * F3_BK + half * 4;
-    }
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-#pragma unroll 1
-    for (int k = k0; k < k1; ++k) {
-        f32x4_t xf[TM][4], wf[TN][4];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i) xf[i][t] = *(const f32x4_t*)(xr[i] + 8 * t);
-#pragma unroll
-            for (int j = 0; j < TN; ++j) wf[j][t] = *(const f32x4_t*)(wr[j] + 8 * t);
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[j][t][e], xf[i][t][e], acc[i][j], 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < TM; ++i) xr[i] += F3_BK;
-#pragma unroll
-        for (int j = 0; j < TN; ++j) wr[j] += F3_BK;
-    }
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int t = 0; t < 16; ++t)
-                if (odd[(i * TN + j) >> 1] >> (((i * TN + j) & 1) * 16 + t) & 1) {     // (set only for outputs that are there)
-                    const int n = n0 + wn * (BN / WGN) + j * 32 + (t >> 2) * 8 + half * 4 + (t & 3);
-                    *at(m0 + wm * (BM / WGM) + i * 32 + l31, n) = !SPLIT && a.bias ? acc[i][j][t] + a.bias[n] : acc[i][j][t];
-                }
+    f3_again<TM, TN>(acc, look, a.x, a.w, SPLIT ? nullptr : a.bias, m0 + wm * (BM / WGM), a.M, n0 + wn * (BN / WGN), a.N, a.K, k0, k1, row_max + wm * (BM / WGM),
+                     row_max + BM + wn * (BN / WGN), at);
 }
 
 // the sum of the parts of K
@@ -318,7 +185,7 @@ __global__ __launch_bounds__(256) void gemm_f32_parts_kernel(F3Args a) {
 // 4,096 x 4,096): 1.00e-6 unsplit, 7.1e-7 in two parts, 5.0e-7 in four, 3.5e-7 in eight; library 1.14e-6.
 struct F3Kind { int bm, bn, per_cu; double start, each; };
 static const F3Kind f3_kinds[] = {{64, 64, 5, 0.29, 0.33}, {64, 128, 4, 0.30, 0.655}, {128, 128, 2, 0.20, 1.11}, {256, 256, 1, 0.10, 4.36}};
-struct F3Plan { int kind, splits; };
+struct F3Plan { int kind, splits; double us; };
 
 static F3Plan f3_plan(int64_t M, int64_t N, int64_t K) {
     static const int cus = [] {
@@ -326,8 +193,7 @@ static F3Plan f3_plan(int64_t M, int64_t N, int64_t K) {
         if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev);
         return c < 8 ? 8 : c;
     }();
-    F3Plan best = {0, 1};
-    double least = 1e300;
+    F3Plan best = {0, 1, 1e300};
     const double memory = 4.0 * ((double)N * K + (double)M * K) / 4.2e6;
     for (int c = 0; c < 4; ++c) {
         const F3Kind& k = f3_kinds[c];
@@ -339,11 +205,13 @@ static F3Plan f3_plan(int64_t M, int64_t N, int64_t K) {
             const double work = steps * (full * (k.start + k.per_cu * k.each) + (rest > 0 ? k.start + rest * k.each : 0.0)) + 5.0;
             double us = work > memory ? work + 0.085 * memory : memory + 0.085 * work;
             if (s > 1) us += 6.0 + (double)s * M * N * 8 / 9.1e6;
-            if (us < least) { least = us; best = {c, s}; }
+            if (us < best.us) best = {c, s, us};
         }
     }
     return best;
 }
+
+double f3_tiles_us(int64_t M, int64_t N, int64_t K) { return f3_plan(M, N, K).us; }
 
 template <int BM, int BN, int WGM, int WGN, int PER_CU>
 static int f3_launch(F3Args a, hipStream_t st) {

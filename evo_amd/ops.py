@@ -70,6 +70,8 @@ _SIGNATURES = {
     "evo_logprob_entropy": ([_PTR, _I64, _PTR, _PTR, _PTR, _I64, _I64, _PTR], _c.c_int),
     "evo_linear_f32_ws": ([_I64] * 3, _c.c_int),
     "evo_linear_f32_plan": ([_I64] * 3 + [_PTR], _c.c_int),
+    "evo_linear_f32_ahead_plan": ([_I64] * 3 + [_PTR], _c.c_int),
+    "evo_linear_f32_ahead": ([_PTR] * 4 + [_I64] * 3 + [_PTR, _I64, _PTR], _c.c_int),
     "evo_linear_f32": ([_PTR] * 4 + [_I64] * 3 + [_PTR, _I64, _PTR], _c.c_int),
     "evo_unembed_logprob_bf16": ([_PTR] * 5 + [_I64] * 3 + [_PTR], _c.c_int),
     "evo_rope_append_decode_bf16": ([_PTR] * 4 + [_F32] + [_I64] * 7 + [_F32, _PTR], _c.c_int),
@@ -104,7 +106,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 23         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 24         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):
@@ -371,6 +373,12 @@ class HipOps(MixerOps):
         M, K = x.shape
         N = w.shape[0]
         y = torch.empty(M, N, dtype=torch.float32, device=x.device)
+        plan = (_c.c_int64 * 6)()
+        if self.lib.evo_linear_f32_ahead_plan(M, N, K, _c.cast(plan, _PTR)) == 1:
+            ws = torch.empty(plan[5], dtype=torch.uint8, device=x.device)
+            with self._t("gemm_f32"):
+                _check(self.lib.evo_linear_f32_ahead(x.data_ptr(), w.data_ptr(), _ptr(b), y.data_ptr(), M, N, K, ws.data_ptr(), plan[5], _stream()), "evo_linear_f32_ahead")
+            return y
         n = self.lib.evo_linear_f32_ws(M, N, K)
         ws = torch.empty(n * M * N, dtype=torch.float32, device=x.device) if n > 0 else None
         with self._t("gemm_f32"):

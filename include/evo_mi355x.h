@@ -64,8 +64,9 @@ extern "C" {
  *  20: evo_hyena_short gained `mask`.
  *  21: evo_linear_ring_share added.
  *  22: evo_lightning_chunk_bf16 and evo_rglru_chunk_bf16 keep the states of cut sequences only: `seg` by the rows, not by the sequences.
- *  23: evo_attn_fwd_packed_bf16 gained `form`. */
-#define EVO_ABI_VERSION 23
+ *  23: evo_attn_fwd_packed_bf16 gained `form`.
+ *  24: evo_linear_f32_ahead and evo_linear_f32_ahead_plan added. */
+#define EVO_ABI_VERSION 24
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
@@ -434,6 +435,11 @@ int evo_logprob_entropy(const void* logits, int64_t logits_f32, const int64_t* t
 int evo_linear_f32_ws(int64_t M, int64_t N, int64_t K);
 int evo_linear_f32_plan(int64_t M, int64_t N, int64_t K, int64_t* out);
 int evo_linear_f32(const float* x, const float* w, const float* bias, float* y, int64_t M, int64_t N, int64_t K, float* ws, int64_t ws_bytes, void* stream);
+/* The same with the rows of x split ahead into the workspace (csrc/gemm_f32_ahead.hip).  N % 32 == 0, K % 32 == 0, 16-byte aligned dense operands.
+ * evo_linear_f32_ahead_plan: 1 if it is the faster form of this layer, 0 if not, -1: sizes it does not take; out: rows and columns of a tile, tiles taken by a
+ * workgroup each, tiles shared out, the workgroups they are shared by (0: none), bytes of the workspace. */
+int evo_linear_f32_ahead_plan(int64_t M, int64_t N, int64_t K, int64_t* out);
+int evo_linear_f32_ahead(const float* x, const float* w, const float* bias, float* y, int64_t M, int64_t N, int64_t K, void* ws, int64_t ws_bytes, void* stream);
 
 /* ---- fused scoring tail: unembed + log_softmax + gather (+ entropy) ---------------------------------
  * replaces  logits = x @ E^T ; log_softmax(logits) ; gather(next token) ; -sum p log p
