@@ -72,6 +72,7 @@ _SIGNATURES = {
     "evo_linear_f32_plan": ([_I64] * 3 + [_PTR], _c.c_int),
     "evo_linear_f32_ahead_plan": ([_I64] * 3 + [_PTR], _c.c_int),
     "evo_linear_f32_ahead": ([_PTR] * 4 + [_I64] * 3 + [_PTR, _I64, _PTR], _c.c_int),
+    "evo_linear_few_f32": ([_PTR] * 4 + [_I64] * 3 + [_PTR], _c.c_int),
     "evo_linear_f32": ([_PTR] * 4 + [_I64] * 3 + [_PTR, _I64, _PTR], _c.c_int),
     "evo_unembed_logprob_bf16": ([_PTR] * 5 + [_I64] * 3 + [_PTR], _c.c_int),
     "evo_rope_append_decode_bf16": ([_PTR] * 4 + [_F32] + [_I64] * 7 + [_F32, _PTR], _c.c_int),
@@ -106,7 +107,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 24         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 25         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):
@@ -336,6 +337,8 @@ class HipOps(MixerOps):
             return self.linear_mfma(x, w, b)
         if x.dtype == torch.float32 and x.shape[0] > 32 and x.dim() == w.dim() == 2 and self._f32_layer_pays(x.shape[0], *w.shape) and self._f32_layer_ok(x, w, b):
             return self._linear_f32(x, w, b)
+        if x.dtype == torch.float32 and x.dim() == 2 and 1 <= x.shape[0] <= 4 and self._f32_few_ok(x, w, b):
+            return self._linear_few_f32(x, w, b)
         with self._t("gemm"):
             if b is not None:
                 return torch.addmm(b, x, w.t())
@@ -359,15 +362,31 @@ class HipOps(MixerOps):
         return M * N >= 1350000 or M * N * K >= 2200000000
 
     def _f32_layer_ok(self, x, w, b) -> bool:
-        """What csrc/gemm_f32.hip takes, from 33 rows on; below, the weight's own bytes bound the layer and the library reads them at 2.5 to 4.6 TB/s.  What is
+        """What csrc/gemm_f32.hip takes, from 33 rows on; 5 to 32 stay with the library, which reads the weight at 2.5 to 5 TB/s there.  What is
         traced or differentiated stays with torch, and so does what lies on another device than the current one, whose stream the launch goes to."""
+        return (x.dim() == 2 and w.dim() == 2 and x.shape[0] > 32 and x.shape[1] == w.shape[1] and x.shape[1] % 32 == 0 and x.shape[1] >= 256
+                and w.shape[0] % 4 == 0 and w.shape[0] >= 256 and self._f32_plain(x, w, b))
+
+    def _f32_few_ok(self, x, w, b) -> bool:
+        """What csrc/gemv_f32.hip takes, one to four rows."""
+        return (x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1] and x.shape[1] % 32 == 0 and 32 <= x.shape[1] <= 16384 and w.shape[0] >= 1
+                and self._f32_plain(x, w, b))
+
+    def _f32_plain(self, x, w, b) -> bool:
         ts = (x, w) if b is None else (x, w, b)
         return (self.all_gemm_mfma and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()
                                            and t.device == x.device and t.data_ptr() % 16 == 0 for t in ts)
-                and x.device.index == torch.cuda.current_device() and x.dim() == 2 and w.dim() == 2 and x.shape[0] > 32 and x.shape[1] == w.shape[1] and x.shape[1] % 32 == 0 and x.shape[1] >= 256
-                and w.shape[0] % 4 == 0 and w.shape[0] >= 256 and (b is None or b.shape == (w.shape[0],))
+                and x.device.index == torch.cuda.current_device() and (b is None or b.shape == (w.shape[0],))
                 and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts))
                 and torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None and not self._watched())
+
+    def _linear_few_f32(self, x, w, b):
+        M, K = x.shape
+        N = w.shape[0]
+        y = torch.empty(M, N, dtype=torch.float32, device=x.device)
+        with self._t("gemv_f32"):
+            _check(self.lib.evo_linear_few_f32(x.data_ptr(), w.data_ptr(), _ptr(b), y.data_ptr(), M, N, K, _stream()), "evo_linear_few_f32")
+        return y
 
     def _linear_f32(self, x, w, b):
         M, K = x.shape

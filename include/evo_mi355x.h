@@ -65,8 +65,9 @@ extern "C" {
  *  21: evo_linear_ring_share added.
  *  22: evo_lightning_chunk_bf16 and evo_rglru_chunk_bf16 keep the states of cut sequences only: `seg` by the rows, not by the sequences.
  *  23: evo_attn_fwd_packed_bf16 gained `form`.
- *  24: evo_linear_f32_ahead and evo_linear_f32_ahead_plan added. */
-#define EVO_ABI_VERSION 24
+ *  24: evo_linear_f32_ahead and evo_linear_f32_ahead_plan added.
+ *  25: evo_linear_few_f32 added. */
+#define EVO_ABI_VERSION 25
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
@@ -440,6 +441,8 @@ int evo_linear_f32(const float* x, const float* w, const float* bias, float* y, 
  * workgroup each, tiles shared out, the workgroups they are shared by (0: none), bytes of the workspace. */
 int evo_linear_f32_ahead_plan(int64_t M, int64_t N, int64_t K, int64_t* out);
 int evo_linear_f32_ahead(const float* x, const float* w, const float* bias, float* y, int64_t M, int64_t N, int64_t K, void* ws, int64_t ws_bytes, void* stream);
+/* The same for M = 1 .. 4 rows, K % 32 == 0, K <= 16,384, any N (csrc/gemv_f32.hip): fp32 products and sums, x and w 16-byte aligned. */
+int evo_linear_few_f32(const float* x, const float* w, const float* bias, float* y, int64_t M, int64_t N, int64_t K, void* stream);
 
 /* ---- fused scoring tail: unembed + log_softmax + gather (+ entropy) ---------------------------------
  * replaces  logits = x @ E^T ; log_softmax(logits) ; gather(next token) ; -sum p log p
