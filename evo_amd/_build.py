@@ -28,7 +28,7 @@ ARCH = "gfx950"
 
 # component -> (suffix of the library's name, sources, headers beside common.h, the symbols of include/evo_mi355x.h it exports)
 COMPONENTS = {
-    "core": ("", ["elementwise", "gemm", "gemm_tile", "gemm_f32", "gemm_f32_ahead", "gemv", "gemv_f32", "score_tail", "probe"], ["gemm_args.h", "gemm_f32.h"], [
+    "core": ("", ["elementwise", "gemm", "gemm_rows160", "gemm_rows192", "gemm_rows224", "gemm_tile", "gemm_f32", "gemm_f32_ahead", "gemv", "gemv_f32", "score_tail", "probe"], ["gemm_args.h", "gemm_kernel.h", "gemm_f32.h"], [
         "evo_abi_version", "evo_embed_bf16", "evo_rmsnorm_bf16", "evo_rmsnorm_rows_bf16", "evo_rms_finalize_f32", "evo_rope_qk_bf16",
         "evo_rope_append_decode_bf16", "evo_gelu_gate_bf16", "evo_logprob_entropy", "evo_unembed_logprob_bf16",
         "evo_linear_small_m_bf16", "evo_norm_linear_small_m_bf16", "evo_mlp_gate_small_m_bf16", "evo_norm_mlp_gate_small_m_bf16",

@@ -1,0 +1,11 @@
+// The persistent dense-layer kernel on tiles of 160 x 256 (gemm_kernel.h; gemm_tile.hip chooses).
+#include "gemm_kernel.h"
+
+int gemmr_rows160(const GemmArgs& args, int mode, int act, hipStream_t st) {
+    GemmArgs a = args;
+    a.tiles_m = (int)((a.M + 159) / 160);
+    a.tiles_n = a.N / GBN;
+    a.n_tiles = a.tiles_m * a.tiles_n;
+    a.group_m = (mode == 3 ? a.tiles_m : a.tiles_n) >= 32 ? 8 : 4;
+    return gemmr_launch<5>(a, mode, act, st);
+}

@@ -349,7 +349,7 @@ int evo_mlp_gate_mfma_nf_bf16(const void* x, const float* row_scale, const void*
 int evo_linear_t_mfma_nf_bf16(const void* x, const float* row_scale, const void* w, const void* bias, void* zt, int64_t Mp, int64_t N,
                               int64_t K, int64_t x_rows, int64_t Tm, int64_t row_skip, void* stream);
 
-/* Any of the dense layers above, on the tiles that its size asks for: the persistent kernel where 256 x 256 tiles fill the chip, otherwise smaller tiles
+/* Any of the dense layers above, on the tiles that its size asks for: the persistent kernel where its tiles of 160 to 256 rows and 256 columns fill the chip, otherwise smaller tiles
  * and, where those are still too few, parts of K whose fp32 sums a second launch adds in the order of k (csrc/gemm_tile.hip has the rule).
  *   mode 0: y [M, N] = act(x w^T + bias) (+ residual); x row-major, or blocked with xblk != 0 (evo_linear_xblk_mfma_bf16); row_scale, sumsq as in the
  *           nf entries; act on columns [0, act_cols) as in evo_linear_act_mfma_bf16 (without residual and row_scale)
