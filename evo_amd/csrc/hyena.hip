@@ -630,55 +630,59 @@ __global__ __launch_bounds__(512, 4) void hyena_short_kernel(const unsigned char
 }
 
 // ------------------------------------------------------------------------------------------------ decode step
-// one thread per (b, channel pair): FIR step with the 2-sample history, roll, modal update, gate.
-__global__ __launch_bounds__(256) void hyena_step_kernel(
-    const uint32_t* __restrict__ z_t, uint16_t* __restrict__ fir_state, float* __restrict__ iir_state,
-    const uint16_t* __restrict__ fir_w, const uint16_t* __restrict__ fir_b, const float* __restrict__ poles,
-    const float* __restrict__ residues, const uint16_t* __restrict__ dskip, uint32_t* __restrict__ y, int B, int D,
-    int H) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;      // over B * D/2
-    if (i >= (int64_t)B * (D / 2)) return;
-    const int b = (int)(i / (D / 2));
-    const int dp = (int)(i - (int64_t)b * (D / 2));                  // channel pair index within D
-    const int h = dp / (HD / 2), j2 = dp - h * (HD / 2);
-    float f[3][2];
+// One thread per (b, channel): FIR step with the 2-sample history, roll, modal update, gate.  Latency bounds it: 64 bytes of state a channel (4 MB at 16 sequences of 4,096
+// channels) and one wait for all of it, so everything is requested at once in 16-byte pieces, and 128 threads a block spread a small batch over the CUs.  A thread per channel
+// PAIR, its states read and written one by one, took 6.3, 7.0, 8.5 and 10.5 us at 1, 7, 16 and 32 sequences; this: 2.3, 2.7, 4.8 and 7.5.
+#define HS_T 128
+typedef float hs_f32x4 __attribute__((ext_vector_type(4), aligned(8)));      // (states, poles: views of complex values)
+typedef uint32_t hs_u32 __attribute__((aligned(2)));
+__global__ __launch_bounds__(HS_T) void hyena_step_kernel(
+    const uint16_t* __restrict__ z_t, hs_u32* __restrict__ fir_state, hs_f32x4* __restrict__ iir_state,
+    const uint16_t* __restrict__ fir_w, const uint16_t* __restrict__ fir_b, const hs_f32x4* __restrict__ poles,
+    const hs_f32x4* __restrict__ residues, const uint16_t* __restrict__ dskip, uint16_t* __restrict__ y, int B, int D) {
+    const int64_t i = (int64_t)blockIdx.x * HS_T + threadIdx.x;     // over B * D
+    if (i >= (int64_t)B * D) return;
+    const int b = (int)(i / D), d = (int)(i - (int64_t)b * D);
+    const int c0 = d / HD * 3 * HD + d % HD;                         // the channel's column of x2 in the 3D row; x1, v: 128 and 256 further
+    uint16_t z[3], w[3][3], bias[3];
+    uint32_t h[3];
 #pragma unroll
     for (int g = 0; g < 3; ++g) {
-        const int cdw = (h * 3 * HD + g * HD) / 2 + j2;              // dword column in the 3D row
-        const uint32_t zr = z_t[(int64_t)b * (3 * D / 2) + cdw];
-        const float zc[2] = {bf_lo(zr), bf_hi(zr)};
+        const int c = c0 + g * HD;
+        z[g] = z_t[(int64_t)b * 3 * D + c];
+        h[g] = fir_state[(int64_t)b * 3 * D + c];
+        bias[g] = fir_b[c];
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int c = 2 * cdw + e;
-            uint16_t* fs = fir_state + ((int64_t)b * 3 * D + c) * 2;
-            const float o0 = bf_to_f(fs[0]), o1 = bf_to_f(fs[1]);
-            const uint16_t zraw = (uint16_t)(e ? (zr >> 16) : (zr & 0xffffu));
-            f[g][e] = fmaf(bf_to_f(fir_w[c * 3 + 2]), zc[e],
-                           fmaf(bf_to_f(fir_w[c * 3 + 1]), o1, fmaf(bf_to_f(fir_w[c * 3]), o0, bf_to_f(fir_b[c]))));
-            fs[0] = fs[1];
-            fs[1] = zraw;
-        }
+        for (int k = 0; k < 3; ++k) w[g][k] = fir_w[c * 3 + k];
     }
-    float out[2];
+    hs_f32x4 p[NS / 2], r[NS / 2], v[NS / 2];                        // (two modes each)
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        const int d = 2 * dp + e;
-        const float x = f[1][e] * f[2][e];
-        float2* st = (float2*)iir_state + ((int64_t)b * D + d) * NS;
-        const float2* pp = (const float2*)poles + (int64_t)d * NS;
-        const float2* rp = (const float2*)residues + (int64_t)d * NS;
-        float acc = 0.f;
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            const float2 p = pp[s], r = rp[s], sv = st[s];
-            const float nr = fmaf(p.x, sv.x, fmaf(-p.y, sv.y, x));
-            const float ni = fmaf(p.x, sv.y, p.y * sv.x);
-            st[s] = make_float2(nr, ni);
-            acc = fmaf(r.x, nr, fmaf(-r.y, ni, acc));
-        }
-        out[e] = fmaf(x, bf_to_f(dskip[d]), acc) * f[0][e];
+    for (int s = 0; s < NS / 2; ++s) {
+        v[s] = iir_state[i * (NS / 2) + s];
+        p[s] = poles[(int64_t)d * (NS / 2) + s];
+        r[s] = residues[(int64_t)d * (NS / 2) + s];
     }
-    y[i] = pack_bf2(out[0], out[1]);
+    const float skip = bf_to_f(dskip[d]);
+    float f[3];
+#pragma unroll
+    for (int g = 0; g < 3; ++g) {
+        f[g] = fmaf(bf_to_f(w[g][2]), bf_to_f(z[g]), fmaf(bf_to_f(w[g][1]), bf_hi(h[g]), fmaf(bf_to_f(w[g][0]), bf_lo(h[g]), bf_to_f(bias[g]))));
+        fir_state[(int64_t)b * 3 * D + c0 + g * HD] = h[g] >> 16 | (uint32_t)z[g] << 16;
+    }
+    const float x = f[1] * f[2];
+    float acc = 0.f;
+#pragma unroll
+    for (int s = 0; s < NS / 2; ++s) {
+        hs_f32x4 to;
+#pragma unroll
+        for (int e = 0; e < 4; e += 2) {
+            to[e] = fmaf(p[s][e], v[s][e], fmaf(-p[s][e + 1], v[s][e + 1], x));
+            to[e + 1] = fmaf(p[s][e], v[s][e + 1], p[s][e + 1] * v[s][e]);
+            acc = fmaf(r[s][e], to[e], fmaf(-r[s][e + 1], to[e + 1], acc));
+        }
+        iir_state[i * (NS / 2) + s] = to;
+    }
+    y[i] = f_to_bf(fmaf(x, skip, acc) * f[0]);
 }
 
 // ------------------------------------------------------------------------------------------------ C ABI
@@ -772,10 +776,8 @@ extern "C" int evo_hyena_step(const void* z_t, void* fir_state, float* iir_state
                               const float* poles, const float* residues, const void* dskip, void* y, int64_t B,
                               int64_t D, int64_t n_heads, void* stream) {
     if (B <= 0 || D != n_heads * HD) return -1;
-    const int64_t n = B * (D / 2);
-    hipLaunchKernelGGL(hyena_step_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                       (const uint32_t*)z_t, (uint16_t*)fir_state, iir_state, (const uint16_t*)fir_w,
-                       (const uint16_t*)fir_b, poles, residues, (const uint16_t*)dskip, (uint32_t*)y, (int)B, (int)D,
-                       (int)n_heads);
+    hipLaunchKernelGGL(hyena_step_kernel, dim3((unsigned)((B * D + HS_T - 1) / HS_T)), dim3(HS_T), 0, (hipStream_t)stream, (const uint16_t*)z_t, (hs_u32*)fir_state,
+                       (hs_f32x4*)iir_state, (const uint16_t*)fir_w, (const uint16_t*)fir_b, (const hs_f32x4*)poles, (const hs_f32x4*)residues, (const uint16_t*)dskip,
+                       (uint16_t*)y, (int)B, (int)D);
     return evo_launch_status();
 }
