@@ -393,7 +393,7 @@ __global__ __launch_bounds__(256) void lightning_recur_kernel(LightArgs a, const
 }
 
 // Prompts the same way, LT tokens between barriers: their q, k, v rows are staged together (the next LT's are in flight meanwhile), the slices' shares of
-// LT rows of o meet in LDS at the end of the block, summed in the order of the slices.  R: the state rows of a thread, in registers (dk <= 32 R); 0: in LDS.
+// LT rows of o meet in LDS at the end of the block, summed in the order of the slices.  (fp32 heads of 64 or 128 rows: lightning_f32_kernel.)  R: the state rows of a thread, in registers (dk <= 32 R); 0: in LDS.
 // Bound by issue and latency: 70 instructions a token and wave in sequence.  (3 prompts of up to 500 tokens, 32 heads of 128 x 128, fp32, MI355X: 288 us;
 // one token between barriers, its rows requested when they were needed and the state in LDS, 685 us.)
 // The state in LDS is read and written in 16-byte requests (200 tokens, 4 heads of 512 x 64, fp32: 367 us; element by element 573, the form before 471).
@@ -528,6 +528,164 @@ __global__ __launch_bounds__(256) void lightning_tokens_kernel(LightArgs a, cons
     }
 }
 
+// fp32 prompts of heads of 64 or 128 rows, 32 tokens at a time on v_mfma_f32_16x16x4_f32: with A the decay, inside a chunk that starts from S
+//     o_i = A^{i+1} S^T q_i + sum_{j <= i} A^{i-j} (q_i . k_j) v_j          S' = A^n S + sum_j A^{n-1-j} k_j v_j^T
+// in fp32 throughout; the powers are rounded once, from fp64.  A workgroup owns 32 value columns of one head and sequence; S stays in the accumulators (wave w: rows
+// 16 RT w on) and goes through LDS transposed, so that every operand but k's in the state's sum is read as four consecutive values.  Latency bounds it: three barriers
+// a chunk, 104 matrix instructions a wave between them.  The next chunk's rows are requested behind the first barrier.
+// 32 heads of 128 x 128, eight tokens between barriers on the vector units (lightning_tokens_kernel) -> this: prompts of 500, 325 and 325 tokens 237 -> 86 us, one of
+// 150 77 -> 24, of 2,000 950 -> 250, of 4 9 -> 9; against 64 bits 3.0e-7 -> 1.5e-7 (outputs) and 3.6e-7 -> 1.4e-7 (states) of the first.
+// A product with a masked score is 0 v_j: where v is not finite that would reach the tokens before j, and the chunk's sum is taken term by term.
+typedef float lf_f32x4 __attribute__((ext_vector_type(4)));
+template <int RT>
+__global__ __launch_bounds__(256) void lightning_f32_kernel(LightArgs a, const float* __restrict__ decay) {
+    constexpr int C = 32, DK = 64 * RT, PQ = DK + 4, PT = C + 4, QN = DK / 32;        // pitches; float4 of q and of k a thread stages
+    __shared__ __attribute__((aligned(16))) float q[C * PQ], k[C * PQ], s[32 * PQ], vt[32 * PT], p[C * PT];     // s, vt: [column][..]
+    __shared__ float pw[C + 1];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
+    const int h = blockIdx.x, b = blockIdx.z, dv = a.dv, c0 = blockIdx.y * 32, cols = dv - c0 < 32 ? dv - c0 : 32;
+    const int row0 = a.cu[b], n = a.cu[b + 1] - row0;
+    if (tid <= C) pw[tid] = tid ? (float)pow((double)decay[h], (double)tid) : 1.f;
+    float* st = a.state ? a.state + ((int64_t)b * a.H + h) * DK * dv + c0 : nullptr;
+    const bool keep = st && a.resume && a.resume[b];
+    const int srow = 16 * RT * wave + 4 * g;                      // this lane's state rows: srow + 16 rt + r, columns 16 ct + c
+    lf_f32x4 S[RT][2];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[rt][ct][r] = keep && 16 * ct + c < cols ? st[(int64_t)(srow + 16 * rt + r) * dv + 16 * ct + c] : 0.f;
+    const float* zr = (const float*)a.z + (int64_t)row0 * a.ld;
+    const int64_t hq = (int64_t)h * DK, hk = (int64_t)(a.H + h) * DK, hv = (int64_t)2 * a.H * DK + (int64_t)h * dv + c0;
+    const int vtok = tid >> 3, vcol = 4 * (tid & 7);
+    lf_f32x4 zq[QN], zk[QN], zv;
+    auto request = [&](int t0) {
+#pragma unroll
+        for (int j = 0; j < QN; ++j) {
+            const int i = tid + 256 * j, t = t0 + i / (DK / 4);
+            const float* z = zr + (int64_t)(t < n ? t : n - 1) * a.ld + 4 * (i % (DK / 4));
+            zq[j] = *(const lf_f32x4*)(z + hq);
+            zk[j] = *(const lf_f32x4*)(z + hk);
+        }
+        zv = *(const lf_f32x4*)(zr + (int64_t)(t0 + vtok < n ? t0 + vtok : n - 1) * a.ld + hv + (vcol < cols ? vcol : 0));
+    };
+    auto act = [&](float x) { return a.act ? silu_t<float>(x) : x; };
+    if (n > 0) request(0);
+    __syncthreads();
+    const int ti = wave >> 1, tj = wave & 1;                      // this wave's tile of the scores, and of o (tokens 16 ti, columns 16 tj)
+    float wm[4], wr[4];                                          // A^(i - j), A^(i + 1) of its values i = 16 ti + 4 g + r, j = 16 tj + c
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int i = 16 * ti + 4 * g + r, d = i - 16 * tj - c;
+        wm[r] = d >= 0 ? pw[d] : 0.f;
+        wr[r] = pw[i + 1];
+    }
+    for (int t0 = 0; t0 < n; t0 += C) {
+        const int nb = n - t0 < C ? n - t0 : C;
+        bool odd = false;
+#pragma unroll
+        for (int j = 0; j < QN; ++j) {
+            const int i = tid + 256 * j, t = i / (DK / 4), at = t * PQ + 4 * (i % (DK / 4));
+            lf_f32x4 u = {0.f, 0.f, 0.f, 0.f}, w = u;
+            if (t < nb) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { u[e] = act(zq[j][e]); w[e] = act(zk[j][e]); }
+            }
+            *(lf_f32x4*)(q + at) = u;
+            *(lf_f32x4*)(k + at) = w;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float x = vtok < nb && vcol < cols ? act(zv[e]) : 0.f;
+            odd |= !(fabsf(x) <= 3.402823466e38f);
+            vt[(vcol + e) * PT + vtok] = x;
+        }
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int ct = 0; ct < 2; ++ct) *(lf_f32x4*)(s + (16 * ct + c) * PQ + srow + 16 * rt) = S[rt][ct];
+        const bool apart = __syncthreads_or(odd);
+        if (t0 + C < n) request(t0 + C);
+        const lf_f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        lf_f32x4 sc8[8], o8[8], o = zero;                        // (sums of their own: an eighth of the roundings in a row)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sc8[e] = o8[e] = zero;
+#pragma unroll
+        for (int u = 0; u < DK / 16; ++u) {
+            const lf_f32x4 x = *(const lf_f32x4*)(q + (16 * ti + c) * PQ + 16 * u + 4 * g), y = *(const lf_f32x4*)(k + (16 * tj + c) * PQ + 16 * u + 4 * g),
+                           z = *(const lf_f32x4*)(s + (16 * tj + c) * PQ + 16 * u + 4 * g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                sc8[e + 4 * (u & 1)] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], y[e], sc8[e + 4 * (u & 1)], 0, 0, 0);
+                o8[e + 4 * (u & 1)] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], z[e], o8[e + 4 * (u & 1)], 0, 0, 0);
+            }
+        }
+        const lf_f32x4 sc = ((sc8[0] + sc8[1]) + (sc8[2] + sc8[3])) + ((sc8[4] + sc8[5]) + (sc8[6] + sc8[7])),
+                       past = ((o8[0] + o8[1]) + (o8[2] + o8[3])) + ((o8[4] + o8[5]) + (o8[6] + o8[7]));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int i = 16 * ti + 4 * g + r;
+            p[i * PT + 16 * tj + c] = i >= 16 * tj + c ? sc[r] * wm[r] : 0.f;
+        }
+        __syncthreads();
+        if (!apart) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const lf_f32x4 x = *(const lf_f32x4*)(p + (16 * ti + c) * PT + 16 * u + 4 * g), y = *(const lf_f32x4*)(vt + (16 * tj + c) * PT + 16 * u + 4 * g);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], y[e], o, 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                for (int j = 0; j <= 16 * ti + 4 * g + r; ++j) o[r] = fmaf(p[(16 * ti + 4 * g + r) * PT + j], vt[(16 * tj + c) * PT + j], o[r]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int i = 16 * ti + 4 * g + r;
+            if (i < nb && 16 * tj + c < cols) ((float*)a.o)[(int64_t)(row0 + t0 + i) * a.H * dv + (int64_t)h * dv + c0 + 16 * tj + c] = fmaf(wr[r], past[r], o[r]);
+        }
+        const float all = pw[nb];
+        lf_f32x4 add[2][RT][2];                                  // (the chunk's own sum, in halves, added to the state in one rounding)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) add[0][rt][0] = add[0][rt][1] = add[1][rt][0] = add[1][rt][1] = zero;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            lf_f32x4 y[2];
+#pragma unroll
+            for (int ct = 0; ct < 2; ++ct) y[ct] = *(const lf_f32x4*)(vt + (16 * ct + c) * PT + 16 * u + 4 * g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int j = 16 * u + 4 * g + e;
+                const float w = pw[j < nb ? nb - 1 - j : 0];      // (behind the last token k and v are zeros)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    const float x = k[j * PQ + 16 * RT * wave + 16 * rt + c];
+#pragma unroll
+                    for (int ct = 0; ct < 2; ++ct) add[u][rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, y[ct][e] * w, add[u][rt][ct], 0, 0, 0);
+                }
+            }
+        }
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) S[rt][ct][r] = fmaf(all, S[rt][ct][r], add[0][rt][ct][r] + add[1][rt][ct][r]);
+        __syncthreads();
+    }
+    if (st) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int ct = 0; ct < 2; ++ct)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (16 * ct + c < cols) st[(int64_t)(srow + 16 * rt + r) * dv + 16 * ct + c] = S[rt][ct][r];
+    }
+}
+
 template <typename T, int CW>
 static int recur_launch(LightArgs a, const float* decay, int64_t B, hipStream_t s) {
     const size_t lds = (size_t)(2 * a.dk + 32 + 32 * 33) * 4;
@@ -553,6 +711,12 @@ extern "C" int evo_lightning_recurrent(const void* z, int64_t ld, void* o, float
     LightArgs a = {z, o, state, nullptr, cu, resume, nullptr, ld, (int)H, (int)dk, (int)dv, 1, 0, act != 0};
     hipStream_t s = (hipStream_t)stream;
     const bool quad = dv % 4 == 0;
+    if (f32 && cu && (dk == 64 || dk == 128) && dv % 4 == 0 && ld % 4 == 0 && ((uintptr_t)z & 15) == 0) {      // (16-byte requests)
+        const dim3 grid((unsigned)H, (unsigned)((dv + 31) / 32), (unsigned)B);
+        if (dk == 64) hipLaunchKernelGGL(lightning_f32_kernel<1>, grid, dim3(256), 0, s, a, decay);
+        else hipLaunchKernelGGL(lightning_f32_kernel<2>, grid, dim3(256), 0, s, a, decay);
+        return evo_launch_status();
+    }
     // (up to 128 rows the state is in registers and eight tokens share a barrier; wider heads have room for one token's rows beside the state)
 #define LP(T) (dk <= 128 ? (quad ? tokens_launch<T, 4, 4, 8>(a, decay, B, s) : tokens_launch<T, 1, 4, 8>(a, decay, B, s))                                   \
                          : (quad && dk <= 1024 ? tokens_launch<T, 4, 0, 1>(a, decay, B, s) : tokens_launch<T, 1, 0, 1>(a, decay, B, s)))
