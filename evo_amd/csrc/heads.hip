@@ -454,9 +454,8 @@ __global__ __launch_bounds__(256) void heads_decode_kernel(HDecArgs a) {
     }
 }
 
-// Any sizes, both storage types: one wave per (split, head and map, sequence).  V = 4: fp32 rows in 16-byte requests (190 us for 3 sequences x 16 heads
-// of two maps behind 500 tokens element by element, 61 with a lane per key row, 38 with four lanes a row and a wave per 64 slots)
-template <typename T, int V>
+// Any sizes, both storage types: one wave per (split, head and map, sequence).
+template <typename T>
 __global__ __launch_bounds__(64) void heads_decode_any_kernel(HDecArgs a, int maps) {
     extern __shared__ __attribute__((aligned(16))) float qs[];
     const int split = blockIdx.x, hm = blockIdx.y, b = blockIdx.z, lane = threadIdx.x;
@@ -474,10 +473,7 @@ __global__ __launch_bounds__(64) void heads_decode_any_kernel(HDecArgs a, int ma
     for (int s0 = split * 64; s0 < used; s0 += a.n_split * 64) {
         const int slot = s0 + lane;
         float s = -INFINITY;
-        if constexpr (V == 4) {
-            const float dot = dot_rows((const float*)k + (int64_t)s0 * a.rs, a.rs, qs, a.dim, used - s0, lane);
-            if (slot < used) s = dot * a.sc2;
-        } else if (slot < used) {
+        if (slot < used) {
             s = 0.f;
             for (int d = 0; d < a.dim; ++d) s = fmaf(qs[d], ld1(k + (int64_t)slot * a.rs + d), s);
             s *= a.sc2;
@@ -488,33 +484,56 @@ __global__ __launch_bounds__(64) void heads_decode_any_kernel(HDecArgs a, int ma
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[e] *= f;
         const int n = used - s0 < 64 ? used - s0 : 64;
-        if constexpr (V == 4) {                                  // (a lane's eight columns: two runs of four)
-#pragma unroll 8
-            for (int u = 0; u < n; ++u) {
-                const float pu = __shfl(p, u, 64);
+        for (int u = 0; u < n; ++u) {
+            const float pu = __shfl(p, u, 64);
 #pragma unroll
-                for (int e = 0; e < 8; e += 4)
-                    if (4 * lane + 64 * e < a.dv) {
-                        const f32x4_t x = *(const f32x4_t*)((const float*)v + (int64_t)(s0 + u) * a.rs + 4 * lane + 64 * e);
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) o[e + i] = fmaf(pu, x[i], o[e + i]);
-                    }
-            }
-        } else
-            for (int u = 0; u < n; ++u) {
-                const float pu = __shfl(p, u, 64);
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (lane + 64 * e < a.dv) o[e] = fmaf(pu, ld1(v + (int64_t)(s0 + u) * a.rs + lane + 64 * e), o[e]);
-            }
+            for (int e = 0; e < 8; ++e)
+                if (lane + 64 * e < a.dv) o[e] = fmaf(pu, ld1(v + (int64_t)(s0 + u) * a.rs + lane + 64 * e), o[e]);
+        }
     }
     const int64_t p = ((int64_t)b * a.H * maps + hm) * a.n_split + split;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int d = V == 4 ? 4 * lane + 64 * (e & 4) + (e & 3) : lane + 64 * e;
-        if (d < a.dv) a.part_o[p * a.dv + d] = o[e];
-    }
+    for (int e = 0; e < 8; ++e)
+        if (lane + 64 * e < a.dv) a.part_o[p * a.dv + lane + 64 * e] = o[e];
     if (lane == 0) { a.part_ml[2 * p] = m; a.part_ml[2 * p + 1] = l; }
+}
+
+// fp32 rows in 16-byte requests: four waves per (split, head and map, sequence), each 16 of a tile's 64 slots.  Latency bounds it, a wave's requests one behind the other.
+// 3 sequences x 16 heads of two maps behind 500 tokens: one wave per 64 slots 28.0 us, this 13.0 (32 heads over 8 key heads 13.1 -> 7.8; one sequence of 60, two maps, 12.0 -> 6.2)
+__global__ __launch_bounds__(256) void heads_decode_f32_kernel(HDecArgs a, int maps) {
+    extern __shared__ __attribute__((aligned(16))) float qs[];   // [dim]
+    __shared__ float sc[64];
+    __shared__ __attribute__((aligned(16))) float po[4][512];
+    const int split = blockIdx.x, hm = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int hk = hm / maps / (a.H / a.G), m_ = hm % maps;
+    const float* q = (const float*)a.z + (int64_t)b * a.ld + (int64_t)hm * a.dim;
+    for (int d = tid; d < a.dim; d += 256) qs[d] = q[d];
+    const int64_t pos = a.pos[b];
+    const int used = pos + 1 < a.ring ? (int)pos + 1 : a.ring;
+    const float* k = (const float*)a.cache + (int64_t)b * a.ring * a.rs + (int64_t)(hk * maps + m_) * a.dim;
+    const float* v = (const float*)a.cache + (int64_t)b * a.ring * a.rs + (int64_t)a.G * maps * a.dim + (int64_t)hk * a.dv;
+    float m = FLOOR, l = 0.f, o[8];                              // (m, l: the same in every wave)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = 0.f;
+    for (int s0 = split * 64; s0 < used; s0 += a.n_split * 64) {
+        __syncthreads();                                         // (q is there, the scores before are read)
+        const int n = used - s0 < 64 ? used - s0 : 64, left = n - 16 * wave;
+        const float dot = dot_rows16(k + (int64_t)(left > 0 ? s0 + 16 * wave : s0) * a.rs, a.rs, qs, a.dim, left > 0 ? left : 1, lane);
+        if ((lane & 3) == 0) sc[16 * wave + (lane >> 2)] = lane >> 2 < left ? dot * a.sc2 : -INFINITY;
+        __syncthreads();
+        const float s = sc[lane], top = fmaxf(m, wave_max(s)), f = exp2f(m - top), p = exp2f(s - top);
+        m = top;
+        l = l * f + wave_sum(p);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] *= f;
+        sum_rows16(o, v + (int64_t)s0 * a.rs, a.rs, p, 16 * wave, n, a.dv, lane);
+    }
+    const int64_t p = ((int64_t)b * a.H * maps + hm) * a.n_split + split;
+#pragma unroll
+    for (int e = 0; e < 8; e += 4) *(f32x4_t*)(po[wave] + 4 * lane + 64 * e) = f32x4_t{o[e], o[e + 1], o[e + 2], o[e + 3]};
+    __syncthreads();
+    for (int d = tid; d < a.dv; d += 256) a.part_o[p * a.dv + d] = (po[0][d] + po[1][d]) + (po[2][d] + po[3][d]);
+    if (tid == 0) { a.part_ml[2 * p] = m; a.part_ml[2 * p + 1] = l; }
 }
 
 static int heads_decode(void* o, float lam, float gain, float eps, const void* z, int64_t ld, const void* cache, const int64_t* pos, float* part_o, float* part_ml, int64_t B, int64_t H,
@@ -546,9 +565,9 @@ static int heads_decode(void* o, float lam, float gain, float eps, const void* z
     if (o) return -1;
     const dim3 grid((unsigned)n_split, (unsigned)(H * maps), (unsigned)B);
     if (f32 && dim % 4 == 0 && dv % 4 == 0 && rs % 4 == 0 && ((uintptr_t)cache & 15) == 0)
-        hipLaunchKernelGGL((heads_decode_any_kernel<float, 4>), grid, dim3(64), (size_t)dim * 4, s, a, (int)maps);
-    else if (f32) hipLaunchKernelGGL((heads_decode_any_kernel<float, 1>), grid, dim3(64), (size_t)dim * 4, s, a, (int)maps);
-    else hipLaunchKernelGGL((heads_decode_any_kernel<uint16_t, 1>), grid, dim3(64), (size_t)dim * 4, s, a, (int)maps);
+        hipLaunchKernelGGL(heads_decode_f32_kernel, grid, dim3(256), (size_t)dim * 4, s, a, (int)maps);
+    else if (f32) hipLaunchKernelGGL((heads_decode_any_kernel<float>), grid, dim3(64), (size_t)dim * 4, s, a, (int)maps);
+    else hipLaunchKernelGGL((heads_decode_any_kernel<uint16_t>), grid, dim3(64), (size_t)dim * 4, s, a, (int)maps);
     return evo_launch_status();
 }
 

@@ -332,9 +332,8 @@ __global__ __launch_bounds__(512, 2) void latent_decode_kernel(DecArgs a) {
         }
 }
 
-// Any sizes, both storage types: one wave per (split, head, sequence).  V = 4: fp32 rows in 16-byte requests (a lane's key row element by element was one
-// 4-byte request of 64 lines per product: 154 us for 3 sequences x 32 heads behind 500 tokens of 576, 45 in 16-byte ones, 36 with four lanes a row).
-template <typename T, int V>
+// Any sizes, both storage types: one wave per (split, head, sequence).
+template <typename T>
 __global__ __launch_bounds__(64) void latent_decode_any_kernel(DecArgs a, int dq) {
     extern __shared__ __attribute__((aligned(16))) float qf[];
     const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z, lane = threadIdx.x;
@@ -356,11 +355,7 @@ __global__ __launch_bounds__(64) void latent_decode_any_kernel(DecArgs a, int dq
         for (int s0 = split * 64; s0 < used; s0 += a.n_split * 64) {
             const int slot = s0 + lane;
             float s = -INFINITY;
-            const bool seen = slot < used && slot_seen(slot, pos, cur, a);
-            if constexpr (V == 4) {
-                const float dot = dot_rows((const float*)base + (int64_t)s0 * a.rs, a.rs, qf, dq, used - s0, lane);
-                if (seen) s = dot * a.sc2;
-            } else if (seen) {
+            if (slot < used && slot_seen(slot, pos, cur, a)) {
                 s = 0.f;
                 for (int d = 0; d < dq; ++d) s = fmaf(qf[d], ld1(base + (int64_t)slot * a.rs + d), s);
                 s *= a.sc2;
@@ -373,37 +368,65 @@ __global__ __launch_bounds__(64) void latent_decode_any_kernel(DecArgs a, int dq
 #pragma unroll
             for (int e = 0; e < 8; ++e) o[e] *= f;
             const int n = used - s0 < 64 ? used - s0 : 64;
-            if constexpr (V == 4) {                              // (a lane's eight columns: two runs of four)
-#pragma unroll 4
-                for (int u = 0; u < n; ++u) {
-                    const float pu = __shfl(pr, u, 64);
+            for (int u = 0; u < n; ++u) {
+                const float pu = __shfl(pr, u, 64);
 #pragma unroll
-                    for (int e = 0; e < 8; e += 4) {
-                        const int r = pass * 512 + 4 * lane + 64 * e;
-                        if (r < a.R) {
-                            const f32x4_t x = *(const f32x4_t*)((const float*)base + (int64_t)(s0 + u) * a.rs + r);
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) o[e + i] = fmaf(pu, x[i], o[e + i]);
-                        }
-                    }
+                for (int e = 0; e < 8; ++e) {
+                    const int r = pass * 512 + lane + 64 * e;
+                    if (r < a.R) o[e] = fmaf(pu, ld1(base + (int64_t)(s0 + u) * a.rs + r), o[e]);
                 }
-            } else
-                for (int u = 0; u < n; ++u) {
-                    const float pu = __shfl(pr, u, 64);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const int r = pass * 512 + lane + 64 * e;
-                        if (r < a.R) o[e] = fmaf(pu, ld1(base + (int64_t)(s0 + u) * a.rs + r), o[e]);
-                    }
-                }
+            }
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const int r = pass * 512 + (V == 4 ? 4 * lane + 64 * (e & 4) + (e & 3) : lane + 64 * e);
+            const int r = pass * 512 + lane + 64 * e;
             if (r < a.R) po[r] = o[e];
         }
     }
     if (lane == 0) { a.part_ml[2 * p] = m; a.part_ml[2 * p + 1] = l; }
+}
+
+// fp32 rows in 16-byte requests: four waves per (split, head, sequence), each 16 of a tile's 64 slots.  Latency bounds it, a wave's requests one behind the other (the rows
+// themselves come from L2, every head reads them).  Behind 500 tokens of 576, 3 sequences x 32 heads: one wave per 64 slots 25.8 us, this 12.3 (2 x 1,000 slots 25.4 -> 14.0, 8 x 1,000 54 -> 47, one of 60 23.7 -> 8.3)
+__global__ __launch_bounds__(256) void latent_decode_f32_kernel(DecArgs a, int dq) {
+    extern __shared__ __attribute__((aligned(16))) float qf[];   // [dq]
+    __shared__ float sc[64];
+    __shared__ __attribute__((aligned(16))) float po[4][512];
+    const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const float* q = (const float*)a.q + ((int64_t)b * a.H + h) * a.rs;
+    for (int d = tid; d < dq; d += 256) qf[d] = q[d];
+    const int64_t pos = a.pos[b];
+    const int cur = (int)(pos % a.ring);
+    const float* base = (const float*)a.cache + (int64_t)b * a.ring * a.rs;
+    const int64_t p = ((int64_t)b * a.H + h) * a.n_split + split;
+    const int used = pos + 1 < a.ring ? (int)pos + 1 : a.ring;
+    float m = -INFINITY, l = 0.f;                                // (the same in every wave)
+    for (int first = 0; first < a.R; first += 512) {             // 512 latent columns per pass (the scores are recomputed per pass)
+        float o[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = 0.f;
+        m = -INFINITY; l = 0.f;
+        for (int s0 = split * 64; s0 < used; s0 += a.n_split * 64) {
+            __syncthreads();                                     // (q is there, the scores before and the partial sums of the pass before are read)
+            const int n = used - s0 < 64 ? used - s0 : 64, slot = s0 + 16 * wave + (lane >> 2), left = n - 16 * wave;
+            const float dot = dot_rows16(base + (int64_t)(left > 0 ? s0 + 16 * wave : s0) * a.rs, a.rs, qf, dq, left > 0 ? left : 1, lane);
+            if ((lane & 3) == 0) sc[16 * wave + (lane >> 2)] = slot < used && slot_seen(slot, pos, cur, a) ? dot * a.sc2 : -INFINITY;
+            __syncthreads();
+            const float s = sc[lane], top = fmaxf(m, wave_max(s));
+            if (top == -INFINITY) continue;
+            const float f = exp2f(m - top), pr = exp2f(s - top);
+            m = top;
+            l = l * f + wave_sum(pr);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] *= f;
+            sum_rows16(o, base + (int64_t)s0 * a.rs + first, a.rs, pr, 16 * wave, n, a.R - first, lane);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) *(f32x4_t*)(po[wave] + 4 * lane + 64 * e) = f32x4_t{o[e], o[e + 1], o[e + 2], o[e + 3]};
+        __syncthreads();
+        for (int r = tid; r < 512 && first + r < a.R; r += 256) a.part_o[p * a.R + first + r] = (po[0][r] + po[1][r]) + (po[2][r] + po[3][r]);
+    }
+    if (tid == 0) { a.part_ml[2 * p] = m; a.part_ml[2 * p + 1] = l; }
 }
 
 extern "C" int evo_latent_decode(const void* q, const void* cache, const int64_t* pos, float* part_o, float* part_ml, int64_t B, int64_t H, int64_t R,
@@ -445,9 +468,9 @@ extern "C" int evo_latent_decode(const void* q, const void* cache, const int64_t
     }
     const dim3 grid((unsigned)n_split, (unsigned)H, (unsigned)B);
     if (f32 && R % 4 == 0 && dr % 4 == 0 && rs % 4 == 0 && ((uintptr_t)cache & 15) == 0)
-        hipLaunchKernelGGL((latent_decode_any_kernel<float, 4>), grid, dim3(64), (size_t)(R + dr) * 4, s, a, (int)(R + dr));
-    else if (f32) hipLaunchKernelGGL((latent_decode_any_kernel<float, 1>), grid, dim3(64), (size_t)(R + dr) * 4, s, a, (int)(R + dr));
-    else hipLaunchKernelGGL((latent_decode_any_kernel<uint16_t, 1>), grid, dim3(64), (size_t)(R + dr) * 4, s, a, (int)(R + dr));
+        hipLaunchKernelGGL(latent_decode_f32_kernel, grid, dim3(256), (size_t)(R + dr) * 4, s, a, (int)(R + dr));
+    else if (f32) hipLaunchKernelGGL((latent_decode_any_kernel<float>), grid, dim3(64), (size_t)(R + dr) * 4, s, a, (int)(R + dr));
+    else hipLaunchKernelGGL((latent_decode_any_kernel<uint16_t>), grid, dim3(64), (size_t)(R + dr) * 4, s, a, (int)(R + dr));
     return evo_launch_status();
 }
 

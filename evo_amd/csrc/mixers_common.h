@@ -106,32 +106,36 @@ __device__ __forceinline__ mx_frag frag_split(const uint16_t* p) {
     return frag_of(a.x, a.y, b.x, b.y);
 }
 __device__ __forceinline__ f32x4_t mfma16(mx_frag a, mx_frag b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
-// A wave's products of q [dim] (LDS) with 64 fp32 rows, row r at rows + r ld (r >= n: row n - 1 again); -> lane r has row r's.  Four lanes share a row, 16
-// bytes of it each: a request touches 16 rows' 64 bytes instead of 64 rows' 16, and four rows a lane keep four chains going.  dim % 4 == 0, 16-byte aligned.
-__device__ __forceinline__ float dot_rows(const float* rows, int64_t ld, const float* q, int dim, int n, int lane) {
+// fp32 decode attention, 64 slots of a cache by four waves.  Every wave: the products of q [dim] (LDS) with 16 of the rows, row r at rows + r ld (r >= n: row n - 1
+// again); -> lanes 4 r .. 4 r + 3 have row r's.  Four lanes share a row, 16 bytes of it each: a request touches 16 rows' 64 bytes instead of 64 rows' 16.
+// dim % 4 == 0, 16-byte aligned.
+__device__ __forceinline__ float dot_rows16(const float* rows, int64_t ld, const float* q, int dim, int n, int lane) {
     const int part = lane & 3, kq = lane >> 2;
-    const float* r[4];
-    float s[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int g = 0; g < 4; ++g) r[g] = rows + (int64_t)(16 * g + kq < n ? 16 * g + kq : n - 1) * ld;
-#pragma unroll 4
+    const float* r = rows + (int64_t)(kq < n ? kq : n - 1) * ld;
+    float s = 0.f;
+#pragma unroll 12
     for (int d = 4 * part; d < dim; d += 16) {
-        const f32x4_t y = *(const f32x4_t*)(q + d);
-        f32x4_t x[4];
+        const f32x4_t x = *(const f32x4_t*)(r + d), y = *(const f32x4_t*)(q + d);
 #pragma unroll
-        for (int g = 0; g < 4; ++g) x[g] = *(const f32x4_t*)(r[g] + d);
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) s[g] = fmaf(y[e], x[g][e], s[g]);
+        for (int e = 0; e < 4; ++e) s = fmaf(y[e], x[e], s);
     }
-    float out = 0.f;
+    s += __shfl_xor(s, 1, 64);
+    return s + __shfl_xor(s, 2, 64);
+}
+// o[0 .. 7] += sum over this wave's 16 rows u < n of p[u] x the row's columns 4 lane .. and 256 + 4 lane .. (those under `cols`); lane u of `p` has row u's factor
+__device__ __forceinline__ void sum_rows16(float (&o)[8], const float* rows, int64_t ld, float p, int first, int n, int cols, int lane) {
+    auto add = [&](int u, float pu) __attribute__((always_inline)) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        s[g] += __shfl_xor(s[g], 1, 64);
-        s[g] += __shfl_xor(s[g], 2, 64);
-        const float t = __shfl(s[g], 4 * (lane & 15), 64);
-        out = (lane >> 4) == g ? t : out;
-    }
-    return out;
+        for (int e = 0; e < 8; e += 4)
+            if (4 * lane + 64 * e < cols) {
+                const f32x4_t x = *(const f32x4_t*)(rows + (int64_t)u * ld + 4 * lane + 64 * e);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[e + i] = fmaf(pu, x[i], o[e + i]);
+            }
+    };
+    if (first + 16 <= n) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) add(first + u, __shfl(p, first + u, 64));
+    } else
+        for (int u = first; u < n; ++u) add(u, __shfl(p, u, 64));
 }
