@@ -107,9 +107,9 @@ static_assert(!GE_FULL || GE_ORDER == 1, "GE_FULL pairs the strips of GE_ORDER 1
 //   power limit leaves: that bounds 224 and 256 rows, the arrival of the operands the lower ones.
 // WF: a stage's W slab is fetched before its X slab.  The ring holds two stages and a half; the half in front is the slab that has longest to arrive, and the weights come
 //   from HBM (each line read once per XCD), the rows of x from the L2 that eight column tiles share.  us, X first -> W first: 22,016 gated columns at K = 4,096, 256 rows a
-//   tile, 86.5 -> 81 at 300 rows, 170 -> 166 at 1,100, 1.01x at 11,800; 160 rows a tile 73 -> 66 at 300, 12,288 columns 70 -> 63 at 700.  Not in mode 3, whose
-//   "X" is the weight, and not where 256 rows run in mode 0 (the same within noise from 2,000 rows on, 4,096 columns 1 - 2 % behind).
-template <bool BIAS, bool RES, int MODE, bool XB = false, int NF = 0, int ACT = 0, int MT = 8, bool WF = MODE == 1 || (MODE == 0 && MT < 8)>
+//   tile, 86.5 -> 81 at 300 rows, 170 -> 166 at 1,100; 160 rows a tile 73 -> 66 at 300, 12,288 columns 70 -> 63 at 700.  Not in mode 3, whose
+//   "X" is the weight, and of 256 rows in gated launches of few rounds only (gemm.hip; mode 0: the same within noise from 2,000 rows on, 4,096 columns 1 - 2 % behind).
+template <bool BIAS, bool RES, int MODE, bool XB = false, int NF = 0, int ACT = 0, int MT = 8, bool WF = MODE != 3 && MT < 8>
 __global__ __launch_bounds__(256, 1) void gemmr_bf16_kernel(GemmArgs a) {
     constexpr bool STATS = (NF & 1) != 0, SCALE = (NF & 2) != 0;
     static_assert(!STATS || (RES && MODE == 0), "the statistic rides on the launches that write the residual stream");

@@ -492,7 +492,8 @@ static const TileKind kinds[] = {{64, 64, 0.255}, {128, 64, 0.435}, {128, 128, 0
 // (160), 159 -> 124 at 770 (160), 163 -> 147 at 1,025 (224), 247 -> 221 at 1,600 (224), 502 -> 469 at 3,600 (224); 12,288 columns 82 -> 69 at 930 (192), 136 -> 115 at 1,300 (160);
 // K = 11,008, 4,096 columns 193 -> 145 at 2,100 (160), 402 -> 353 at 6,000 (192).
 static const int short_rows[] = {160, 192, 224};
-static const double short_us[] = {0.907, 1.017, 1.105};
+static const double short_us[] = {0.895, 1.022, 1.107};
+static const double short_power[] = {1.11, 1.01, 1.01};  // time at the power limit, by the square tiles'
 #define T_SHORT 96                           // first of them
 #define T_PERSISTENT 99
 
@@ -556,20 +557,21 @@ static int tile_plan_square(int64_t M, int64_t N, int64_t K, int mode, bool stat
     return 1;
 }
 
-// ... or one launch of the persistent kernel on 160, 192 or 224 rows.  Over 8 layers of 2,048 to 16,384 k and 30 sizes of 260 to 6,000 rows, and 3 layers to 11,000, the choice is 0.1 %
-// off the fastest of all plans on average (6.1 % without them) and nowhere more than 5 %.  A tail launch finds its weights in the caches: 7/8 of its time by itself.  Below 2,048 k
-// the plans are as they were (4,096 columns at K = 1,024 could still go from 41 to 37 us at 4,700 rows: layers that small are launches more than work).  Below 256 rows
-// neighbouring tiles start one k-step apart, which these do not; and their padding is most of a tile.
+// ... or one launch of the persistent kernel on 160, 192 or 224 rows.  Over 330 layers and sizes (K = 2,048 to 16,384, 260 to 32,768 rows) the choice is 0.2 % off the fastest of all
+// plans on average (5.3 % without them).  Where many rounds run at the power limit, 256 rows are ahead (32,768 rows, 22,016 gated columns: 4.01 ms, 4.31 on 224, 4.34 on 192, 4.48 on
+// 160).  A tail launch finds its weights in the caches: nine tenths of its time by itself.  Below 2,048 k the plans are as they were (4,096 columns at K = 1,024 could
+// still go from 41 to 37 us at 4,700 rows: layers that small are launches more than work).  Below 256 rows neighbouring tiles start one k-step apart, which these do not; and
+// their padding is most of a tile.
 static int tile_plan(int64_t M, int64_t N, int64_t K, int mode, bool stats, bool splits_ok, bool persistent_ok, bool short_ok, TilePlan (&out)[2]) {
     const int n = tile_plan_square(M, N, K, mode, stats, splits_ok, persistent_ok, out);
     if (!persistent_ok || !short_ok || M < 256 || K < 2048) return n;
-    const double cus = tile_cus(), least = 0.97 * 2.0 * M * N * K / 1.56e9, memory = (2.0 * (M * K + N * K) + 2.0 * M * N) / 4.9e6;
-    double us = n == 2 ? out[0].us + 0.875 * out[1].us + 4.0 : out[0].us;
+    const double cus = tile_cus(), power = 2.0 * M * N * K / 1.56e9, memory = (2.0 * (M * K + N * K) + 2.0 * M * N) / 4.9e6;
+    double us = n == 2 ? out[0].us + 0.9 * out[1].us + 4.0 : out[0].us;
     int kind = -1;
     for (int i = 0; i < 3; ++i) {
         const int64_t rows = mode == 3 ? N : M, cols = mode == 3 ? M : N;      // (mode 3: the tokens are the columns of the launch)
-        double t = ceil((double)((rows + short_rows[i] - 1) / short_rows[i]) * (double)(cols / 256) / cus) * ((double)(K / 64) * short_us[i] + 2.25);
-        if (t < least) t = least;
+        double t = ceil((double)((rows + short_rows[i] - 1) / short_rows[i]) * (double)(cols / 256) / cus) * ((double)(K / 64) * short_us[i] + 2.43);
+        if (t < short_power[i] * power) t = short_power[i] * power;
         if (t < memory) t = memory;
         if (t < us) { us = t; kind = T_SHORT + i; }
     }
