@@ -543,9 +543,15 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         return f._tab_prec <= TABLE_TOL
 
     def _hyena_ct_ok(self, x2d, blk, B, T) -> bool:
+        """Whether the layer goes channel-major.  Below 1,024 rows it does not: z^T and the blocked y are rows padded to multiples of 64 and 256, gathers and a launch for the
+        remainder, and the operator is 16 channels a CU; token-major it is one launch (csrc/hyena.hip hyena_short_kernel) or three.  (Four layers, us, channel- ->
+        token-major.  Width 4,096: 1 x 261 992 -> 898, 4 x 77 1,048 -> 942, 1 x 521 1,425 -> 1,333, 16 x 42 1,587 -> 1,405, 1 x 1,001 1,834 -> 1,785, with end states 1,137 -> 926
+        and 1,991 -> 1,833 of the first and last; 1,024: 509 -> 400, 497 -> 412; 8,192: 2,876 -> 2,676, 5,491 -> 5,548.)  A token behind
+        whole tiles of 512 (1 x 513: 1,470, token-major 1,325) stays with its split below.  From 1,024 rows on, 1.00 to 1.17 by the rows' lengths, a row has the same bits in every
+        batch that way."""
         ops = self.ops
         w = blk.projections.weight
-        return (getattr(ops, "hyena_ct_flag", False) and hasattr(ops, "hyena_ct") and x2d.is_cuda and w.dtype == torch.bfloat16
+        return ((B * T >= 1024 or ops.zt_layout(B, T)[3] == 1) and getattr(ops, "hyena_ct_flag", False) and hasattr(ops, "hyena_ct") and x2d.is_cuda and w.dtype == torch.bfloat16
                 and w.is_contiguous() and ops.zt_shape_ok(B, T, w.shape[0], w.shape[1]))
 
     def _hyena_block(self, i, blk, x2d, B, T, cache: Optional[RecurrentInferenceParams], mask=None, rs=None):
