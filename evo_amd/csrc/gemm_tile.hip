@@ -10,9 +10,10 @@
 // meet in the same L2 channels.  us at 65 / 161 rows, K = 4,096: 22,016 gated columns 47.1 / 56.8 -> 39.3 / 51.5, 12,288 columns 31.6 / 35.8 -> 26.7 / 33.3;
 // K = 11,008, 4,096 columns 30.8 / 34.6 -> 27.4 / 32.9.  (From 256 rows on, where it gives 3 to 6 %, the gated, the ungated and the blocked forms of a layer agree bit
 // for bit, whichever tiles they take.)
-// Inner loop: a ring of NS stages of 64 k, LDS-DMA pieces spread between the products of the first half step (a burst blocks the wave on the
+// Inner loop (another where X and W come in phases): a ring of NS stages of 64 k, LDS-DMA pieces spread between the products of the first half step (a burst blocks the wave on the
 // vector-memory queue), the next half's fragments requested under the products of the current one, one barrier per stage.
 #include <math.h>
+#include <type_traits>
 #include "gemm_kernel.h"
 #include "../../include/evo_mi355x.h"
 
@@ -80,7 +81,11 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
     static_assert(MODE != 1 || SPLIT || WN % 64 == 0 || (ODD && WN % 32 == 0), "a wave holds both halves of its gated columns");
     static_assert(!ODD || (MODE <= 1 && !SPLIT && !XB), "the launches that take such tiles");
     constexpr bool STATS = MODE == 0 && !SPLIT && BN == 128;     // (a strip of the statistic is 128 columns)
-    __shared__ __attribute__((aligned(16))) unsigned char smem[NS * STAGE];
+    // PHASES (NS = 10 + n): rings of their own for X (four slots) and W (n), two stages of X fetched at even k-steps and two of W at odd ones
+    constexpr bool PHASES = NS > 10;
+    constexpr int NX = 4, NWS = NS - 10, SLAB_W = BN * T_ROW, W_AT = PHASES ? NX * SLAB_X : SLAB_X;      // (first of the W slots)
+    static_assert(!PHASES || NWS >= 5, "W is three stages ahead");
+    __shared__ __attribute__((aligned(16))) unsigned char smem[PHASES ? NX * SLAB_X + NWS * SLAB_W : NS * STAGE];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
@@ -172,7 +177,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
                          ::"s"(dst + i * NW * 1024), "v"(xoff[i < PX ? i : 0]), "s"(rx), "s"((uint32_t)s * (XB ? 16384u : 128u)) : "memory", "m0");
         else
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                         ::"s"(dst + SLAB_X + (i - PX) * NW * 1024), "v"(woff[i < PX ? 0 : i - PX]), "s"(rw), "s"((uint32_t)s * 128u) : "memory", "m0");
+                         ::"s"(dst + W_AT + (i - PX) * NW * 1024), "v"(woff[i < PX ? 0 : i - PX]), "s"(rw), "s"((uint32_t)s * 128u) : "memory", "m0");
     };
 
     uint32_t x_rd[2], w_rd[2];
@@ -180,7 +185,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
     for (int kh = 0; kh < 2; ++kh) {
         const int xr = wm * WM + l15, wr = wn * WN + l15;
         x_rd[kh] = lds0 + (uint32_t)(xr * T_ROW + (((4 * kh + lq) ^ xr) & 7) * 16);
-        w_rd[kh] = lds0 + (uint32_t)(SLAB_X + wr * T_ROW + (((4 * kh + lq) ^ wr) & 7) * 16);
+        w_rd[kh] = lds0 + (uint32_t)(W_AT + wr * T_ROW + (((4 * kh + lq) ^ wr) & 7) * 16);
     }
     f32x4_t acc[NT][MT];
 #pragma unroll
@@ -196,6 +201,80 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
 #pragma unroll
         for (int j = 0; j < MT; ++j) T_DSR(xf[kh][j], xa_, j * 16 * T_ROW);
     };
+    if constexpr (PHASES) {
+        // A CU has at most 512 lines under way and they come back in order: 57 GB/s while any of them comes from HBM (1.1 us), 129 where all hit the L2, and x behind w waits
+        // with it.  Phases of the one and of the other, a barrier between them, took a probe of that intake (w : x 1 : 2) from 65 to 84 GB/s.  Even step k: X of stages
+        // k + 2 and k + 3; odd step: W of stages k + n - 2 and k + n - 1 (the slots were read before the last barrier).  At the middle of a step what may still be out is all of
+        // the last two phases (even), all but the first stage of the X phase (odd): the next stage's slabs are then here.
+        int xk = at, wk = at, xl = nk - 1, wl = nk - 1;          // k-step of the next stage to fetch, stages left behind it
+        auto on = [&](int& kk, int& left) { if (left > 0) { --left; kk = kk + 1 == k0 + nk ? k0 : kk + 1; } };        // (past the last: the same again, into a slot nobody reads)
+        uint32_t xf_slot = 0, wf_slot = 0;                       // slot of the next stage to fetch
+        auto one_x = [&](int i) { fetch1(xk, xf_slot, i); };
+        auto one_w = [&](int i) { fetch1(wk, wf_slot, PX + i); };
+        auto end_x = [&] { on(xk, xl); xf_slot = xf_slot + SLAB_X == NX * SLAB_X ? 0 : xf_slot + SLAB_X; };
+        auto end_w = [&] { on(wk, wl); wf_slot = wf_slot + SLAB_W == NWS * SLAB_W ? 0 : wf_slot + SLAB_W; };
+        auto some_x = [&] {
+#pragma unroll
+            for (int i = 0; i < PX; ++i) one_x(i);
+            end_x();
+        };
+        auto some_w = [&] {
+#pragma unroll
+            for (int i = 0; i < PW; ++i) one_w(i);
+            end_w();
+        };
+        auto read2 = [&](uint32_t xs, uint32_t ws_, int kh) {
+#pragma unroll
+            for (int i = 0; i < NT; ++i) T_DSR(wf[kh][i], ws_ + w_rd[kh], i * 16 * T_ROW);
+#pragma unroll
+            for (int j = 0; j < MT; ++j) T_DSR(xf[kh][j], xs + x_rd[kh], j * 16 * T_ROW);
+        };
+        auto mma2 = [&](int kh, auto phase) {                    // phase: pieces between the products, 2 stages of them (0: none, 1: X, 2: W)
+            constexpr int PH_ = decltype(phase)::value, TOTAL = NT * MT, EACH = PH_ == 1 ? PX : PW, D = PH_ ? 2 * EACH : 0;
+#pragma unroll
+            for (int u = 0; u < TOTAL; ++u) {
+                const int i = u / MT, j = u % MT;
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, wf[kh][i]), __builtin_bit_cast(bf16x8_t, xf[kh][j]), acc[i][j], 0, 0, 0);
+#pragma unroll
+                for (int d = u * D / TOTAL; d < (u + 1) * D / TOTAL; ++d) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (PH_ == 1) { one_x(d % EACH); if (d % EACH == EACH - 1) end_x(); }
+                    else { one_w(d % EACH); if (d % EACH == EACH - 1) end_w(); }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        };
+        uint32_t xs = 0, ws_ = 0;
+        auto step = [&](auto phase) {
+            constexpr int PH_ = decltype(phase)::value;
+            read2(xs, ws_, 1);
+            t_lgkm<NT + MT>(wf[0]);
+            t_lgkm<NT + MT>(xf[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            mma2(0, phase);
+            __builtin_amdgcn_sched_barrier(0);
+            t_lgkm<0>(wf[1]);
+            t_lgkm<0>(xf[1]);
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PH_ == 1 ? 2 * PW + 2 * PX : PX + 2 * PW) : "memory");
+            asm volatile("s_barrier" ::: "memory");
+            xs = xs + SLAB_X == NX * SLAB_X ? 0 : xs + SLAB_X;
+            ws_ = ws_ + SLAB_W == NWS * SLAB_W ? 0 : ws_ + SLAB_W;
+            read2(xs, ws_, 0);                                   // (behind the last stage: slots that are not used any more)
+            __builtin_amdgcn_sched_barrier(0);
+            mma2(1, std::integral_constant<int, 0>{});
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        some_w(); some_w(); some_x(); some_x();
+#pragma unroll
+        for (int i = 2; i < NWS - 1; ++i) some_w();
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PX + (NWS - 3) * PW) : "memory");       // (W 0, W 1, X 0)
+        asm volatile("s_barrier" ::: "memory");
+        read2(0, 0, 0);
+        for (int k = 0; k < nk; k += 2) {
+            step(std::integral_constant<int, 1>{});
+            if (k + 1 < nk) step(std::integral_constant<int, 2>{});
+        }
+    } else {
     // the products of one half of a k-step; `dma`: with the P pieces of k-step `s` between them
     auto mma = [&](int kh, bool dma, int s, uint32_t fslot) {
         constexpr int TOTAL = NT * MT;
@@ -248,6 +327,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU * WGM * WGN / 4) void gemm_t
         fslot = slot;
         slot = nslot;
         nslot = nslot + STAGE == NS * STAGE ? 0 : nslot + STAGE;
+    }
     }
     t_lgkm<0>(wf[0]);
     t_lgkm<0>(xf[0]);
@@ -587,6 +667,16 @@ static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, flo
     a.group_m = 8;
     a.n_tiles = a.tiles_m * a.tiles_n * splits;
     const dim3 grid((unsigned)a.n_tiles), block(64 * WGM * WGN);
+    // X and W in phases (gemm_tile_kernel) where seven eighths of the tiles' rows are there, and from 150 rows on 192, 80 on 96: rows that are not cost no intake, and W is further
+    // ahead without.  us, in turn -> in phases: 12,288 columns, K = 4,096, 43.6 -> 37.9 at 256 rows, 41.6 -> 37.2 at 128, 39.3 -> 36.7 at 112, 33.0 -> 35.9 at 161; 4,096 columns,
+    // K = 11,008, 104 -> 93 at 1,024; 22,016 gated columns 48.0 -> 44.9 at 161, 52.5 -> 46.6 at 192, 47.9 -> 50.5 at 129 (192 rows), 39.3 -> 38.0 at 90 (96).  Parts of K: 0.94 to 1.03.
+    if constexpr (BM == 128 && BN == 128) {
+        if (splits == 1 && !xblk && mode <= 1 && 8 * a.M >= 7 * (int64_t)BM * a.tiles_m) {
+            if (mode == 1) hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, 16, PER_CU, 1, false, false>), grid, block, 0, st, a, act, ws, splits);
+            else hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, 16, PER_CU, 0, false, false>), grid, block, 0, st, a, act, ws, splits);
+            return evo_launch_status();
+        }
+    }
 #define T_GO(MODE, XB, SPLIT) hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, NS, PER_CU, MODE, XB, SPLIT>), grid, block, 0, st, a, act, ws, splits)
     if (splits == 1) {
         if (mode == 3) T_GO(3, false, false);
@@ -721,8 +811,8 @@ extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const voi
             else if (t.kind == 4) rc = tile_launch<256, 128, 4, 2, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
             else if (t.kind == 5) rc = tile_launch<128, 256, 2, 4, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
             else if (xblk || tm > 1 || (tm == 1) != (t.kind < T_ODD + 2)) rc = -1;
-            else if (t.kind == T_ODD) rc = tile_launch_odd<96, 96, 2, 3, 6, 1>(a, (int)act, st);
-            else if (t.kind == T_ODD + 1) rc = tile_launch_odd<192, 96, 4, 3, 4, 1>(a, (int)act, st);
+            else if (t.kind == T_ODD) rc = a.M >= 80 ? tile_launch_odd<96, 96, 2, 3, 18, 1>(a, (int)act, st) : tile_launch_odd<96, 96, 2, 3, 6, 1>(a, (int)act, st);
+            else if (t.kind == T_ODD + 1) rc = a.M >= 150 ? tile_launch_odd<192, 96, 4, 3, 15, 1>(a, (int)act, st) : tile_launch_odd<192, 96, 4, 3, 4, 1>(a, (int)act, st);
             else rc = tile_launch_odd<96, 48, 3, 1, 8, 0>(a, (int)act, st);
         }
         if (rc != 0) return rc;
