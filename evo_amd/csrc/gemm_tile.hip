@@ -647,11 +647,13 @@ static int tile_plan(int64_t M, int64_t N, int64_t K, int mode, bool stats, bool
     if (!persistent_ok || !short_ok || M < 256 || K < 2048) return n;
     const double cus = tile_cus(), power = 2.0 * M * N * K / 1.56e9, memory = (2.0 * (M * K + N * K) + 2.0 * M * N) / 4.9e6;
     double us = n == 2 ? out[0].us + 0.9 * out[1].us + 4.0 : out[0].us;
+    if (mode == 1 && n == 1 && out[0].kind != T_PERSISTENT) us -= 3.0;       // (one tile's closing with the gate: 11,008 gated columns at 390 rows 51.9 on 256 x 128, 58.8 on 160)
     int kind = -1;
     for (int i = 0; i < 3; ++i) {
         const int64_t rows = mode == 3 ? N : M, cols = mode == 3 ? M : N;      // (mode 3: the tokens are the columns of the launch)
         double t = ceil((double)((rows + short_rows[i] - 1) / short_rows[i]) * (double)(cols / 256) / cus) * ((double)(K / 64) * short_us[i] + 2.43);
         if (t < short_power[i] * power) t = short_power[i] * power;
+        if (K >= 16384) t *= 1.08;                               // (4,096 columns 489 us in two launches, 523 on 160, at 4,928 rows; 269 and 206 at 2,100)
         if (t < memory) t = memory;
         if (t < us) { us = t; kind = T_SHORT + i; }
     }
@@ -667,11 +669,13 @@ static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, flo
     a.group_m = 8;
     a.n_tiles = a.tiles_m * a.tiles_n * splits;
     const dim3 grid((unsigned)a.n_tiles), block(64 * WGM * WGN);
-    // X and W in phases (gemm_tile_kernel) where seven eighths of the tiles' rows are there, and from 150 rows on 192, 80 on 96: rows that are not cost no intake, and W is further
-    // ahead without.  us, in turn -> in phases: 12,288 columns, K = 4,096, 43.6 -> 37.9 at 256 rows, 41.6 -> 37.2 at 128, 39.3 -> 36.7 at 112, 33.0 -> 35.9 at 161; 4,096 columns,
+    // X and W in phases (gemm_tile_kernel) where the last row tile has 96 of its 128 rows (120 of more than four tiles), and at 150 to 192 rows on 192, 80 to 96 on 96: rows that are not there cost no intake,
+    // a tile without them runs ahead of those that share its weights (4,096 columns, K = 11,008: 102.6 -> 91.7 at 896 rows, 81.1 -> 92.4 at 912), and W is further
+    // ahead without.  us, in turn -> in phases: 12,288 columns, K = 4,096, 43.6 -> 37.9 at 256 rows, 41.6 -> 37.2 at 128, 38.6 -> 36.9 at 104, 33.0 -> 35.9 at 161; 4,096 columns,
     // K = 11,008, 104 -> 93 at 1,024; 22,016 gated columns 48.0 -> 44.9 at 161, 52.5 -> 46.6 at 192, 47.9 -> 50.5 at 129 (192 rows), 39.3 -> 38.0 at 90 (96).  Parts of K: 0.94 to 1.03.
+    // Not where x is what comes from HBM (512 columns at 8,190 rows 34.2 -> 37.5): from four columns a row on; nor below 1,024 k (4,096 columns at 757 rows, K = 512 7.4 -> 7.9).
     if constexpr (BM == 128 && BN == 128) {
-        if (splits == 1 && !xblk && mode <= 1 && 8 * a.M >= 7 * (int64_t)BM * a.tiles_m) {
+        if (splits == 1 && !xblk && mode <= 1 && a.K >= 1024 && 4 * a.M <= a.N && (a.M - 1) % BM >= (a.tiles_m > 4 ? 119 : 95)) {
             if (mode == 1) hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, 16, PER_CU, 1, false, false>), grid, block, 0, st, a, act, ws, splits);
             else hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, 16, PER_CU, 0, false, false>), grid, block, 0, st, a, act, ws, splits);
             return evo_launch_status();
@@ -811,8 +815,8 @@ extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const voi
             else if (t.kind == 4) rc = tile_launch<256, 128, 4, 2, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
             else if (t.kind == 5) rc = tile_launch<128, 256, 2, 4, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
             else if (xblk || tm > 1 || (tm == 1) != (t.kind < T_ODD + 2)) rc = -1;
-            else if (t.kind == T_ODD) rc = a.M >= 80 ? tile_launch_odd<96, 96, 2, 3, 18, 1>(a, (int)act, st) : tile_launch_odd<96, 96, 2, 3, 6, 1>(a, (int)act, st);
-            else if (t.kind == T_ODD + 1) rc = a.M >= 150 ? tile_launch_odd<192, 96, 4, 3, 15, 1>(a, (int)act, st) : tile_launch_odd<192, 96, 4, 3, 4, 1>(a, (int)act, st);
+            else if (t.kind == T_ODD) rc = a.M >= 80 && a.M <= 96 && a.K >= 4096 ? tile_launch_odd<96, 96, 2, 3, 18, 1>(a, (int)act, st) : tile_launch_odd<96, 96, 2, 3, 6, 1>(a, (int)act, st);
+            else if (t.kind == T_ODD + 1) rc = a.M >= 150 && a.M <= 192 && a.K >= 1024 ? tile_launch_odd<192, 96, 4, 3, 15, 1>(a, (int)act, st) : tile_launch_odd<192, 96, 4, 3, 4, 1>(a, (int)act, st);
             else rc = tile_launch_odd<96, 48, 3, 1, 8, 0>(a, (int)act, st);
         }
         if (rc != 0) return rc;

@@ -1,5 +1,5 @@
-"""128 x 128 tiles whose operands come in phases (csrc/gemm_tile.hip PHASES): one to seventeen k-steps, even and odd, full last row tiles and ones an eighth short; the persistent
-kernel's bits in every form, and rows behind the last untouched.  (192 x 96 and 96 x 96: test_gpu_dense_tiles.py at 161, 192 and 96 rows.)"""
+"""128 x 128 tiles whose operands come in phases (csrc/gemm_tile.hip PHASES): sixteen k-steps and seventeen, full last row tiles and ones a quarter short; below, and one row
+fewer, the other inner loop (K up to 2,048: above, tiles of fewer than 256 rows start a k-step apart and sum in another order).  The persistent kernel's bits in every form, and rows behind the last untouched.  (192 x 96 and 96 x 96: test_gpu_dense_tiles.py at 161, 192 and 96 rows.)"""
 import pytest
 import torch
 
@@ -8,8 +8,8 @@ from test_dense_plan import launches
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 1088])
-@pytest.mark.parametrize("M,N", [(224, 12288), (256, 11008), (384, 6912), (481, 8192)])
+@pytest.mark.parametrize("K", [64, 320, 1024, 1088, 2048])
+@pytest.mark.parametrize("M,N", [(223, 12288), (224, 12288), (256, 11008), (384, 6912), (481, 8192)])
 def test_phases(M, N, K):
     from test_gpu_dense_tiles import _data, _ops
     from evo_amd.ops import _stream
