@@ -47,11 +47,11 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(PrepArgs a) {
         if (h < a.H) {
             T* x = q + h * dh + a.dn;
             const float u = ld1(x + i), v = ld1(x + i + half);
-            st1(x + i, u * cs - v * sn);
-            st1(x + i + half, v * cs + u * sn);
+            st1(x + i, fmaf(u, cs, -(v * sn)));
+            st1(x + i + half, fmaf(u, sn, v * cs));
         } else {
             const float u = ld1(dkv + a.R + i), v = ld1(dkv + a.R + i + half);
-            const float x = u * cs - v * sn, y = v * cs + u * sn;
+            const float x = fmaf(u, cs, -(v * sn)), y = fmaf(u, sn, v * cs);
             if (a.kr) { st1((T*)a.kr + (int64_t)m * a.dr + i, x); st1((T*)a.kr + (int64_t)m * a.dr + i + half, y); }
             if (slot) { st1(slot + a.R + i, x); st1(slot + a.R + i + half, y); }
         }
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(PrepArgs a) {
 }
 
 // The same in 16-byte requests (8 bf16 or 4 fp32 at a time twice) where every part is whole ones: three waves rotate, the fourth norms, and what a thread needs is asked for
-// before the angles.  A decode step waits for one round of requests where it waited for one each pair of elements after the other, a prompt is a fifth of the instructions.
+// before the angles; the roundings and the order of the sums are latent_prep_kernel's.  A decode step waits for one round of requests where it waited for one each pair of elements after the other, a prompt is a fifth of the instructions.
 // 32 heads of 128 + 64, R = 512, pair by pair -> this: 8 tokens decoded 4.4 -> 2.9 us, 329 of a prompt 5.2 -> 3.4, 1,500 8.3 -> 5.3, 11,877 41 -> 23.
 template <typename T>
 __global__ __launch_bounds__(256) void latent_prep_vec_kernel(PrepArgs a) {
@@ -92,17 +92,31 @@ __global__ __launch_bounds__(256) void latent_prep_vec_kernel(PrepArgs a) {
     for (int i = tid; i < half; i += 256) sincosf((float)pos * a.inv_freq[i], &turn[i].y, &turn[i].x);
     __syncthreads();
     if (norms) {
-        float ss = 0.f;
-        for (int r = 8 * lane; r < a.R; r += 512) {
+        // the squares' sum in latent_prep_kernel's order, so that a row has the same bits on either path: thread t there adds columns t, t + 256, .. one after the other
+        // (lanes l and l + 32 here hold columns t and t + 256 of the same eight threads), then eight, 64 and 256 threads' sums meet
+        float ss[8] = {};
+        for (int r0 = 0; r0 < a.R; r0 += 512) {
             float x[8];
-            if (r < 512) {
+            const int r = r0 + 8 * lane;
+            if (r0 == 0) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) x[e] = u[e];
-            } else vec_io<T, 8>::load(dkv + r, x);
+            } else vec_io<T, 8>::load(dkv + (r < a.R ? r : 0), x);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t own = r < a.R ? __float_as_uint(x[e]) : 0u;
+                const auto both = __builtin_amdgcn_permlane32_swap(own, own, false, false);      // lane l % 32's value and lane l % 32 + 32's
+                ss[e] = fmaf(__uint_as_float(both[0]), __uint_as_float(both[0]), ss[e]);
+                ss[e] = fmaf(__uint_as_float(both[1]), __uint_as_float(both[1]), ss[e]);
+            }
         }
-        const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)a.R + a.eps);
+        float sum = ((ss[0] + ss[1]) + (ss[2] + ss[3])) + ((ss[4] + ss[5]) + (ss[6] + ss[7]));
+        sum += dpp_fetch<EVO_DPP_XOR1>(sum);
+        sum += dpp_fetch<EVO_DPP_XOR2>(sum);
+        sum += dpp_fetch<EVO_DPP_HALF_MIRROR>(sum);
+        auto of = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sum), l)); };
+        sum = of(0) + of(8) + of(16) + of(24);
+        const float inv = 1.0f / sqrtf(sum / (float)a.R + a.eps);
         for (int r = 8 * lane; r < a.R; r += 512) {
             float x[8], w[8];
             if (r < 512) {
@@ -136,8 +150,8 @@ __global__ __launch_bounds__(256) void latent_prep_vec_kernel(PrepArgs a) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const float2 t = turn[i + e];
-            p[e] = u[e] * t.x - v[e] * t.y;
-            r[e] = v[e] * t.x + u[e] * t.y;
+            p[e] = fmaf(u[e], t.x, -(v[e] * t.y));               // (latent_prep_kernel's roundings)
+            r[e] = fmaf(u[e], t.y, v[e] * t.x);
         }
         if (h < a.H) { vec_io<T, 8>::store(x, p); vec_io<T, 8>::store(x + half, r); }
         else {
