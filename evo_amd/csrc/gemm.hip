@@ -406,23 +406,20 @@ extern "C" int evo_linear_xblk_mfma_nf_bf16(const void* x_blk, const void* w, co
 // Gated MLP, first half: a[M, I] = act(x W1^T) * (x W2^T), act = gelu (0) or silu (1), in ONE launch of the persistent kernel -- the [M, 2 I] intermediate
 // never reaches memory [REF stripedhyena/layers.py ParallelGatedMLP.forward].  w12g = the rows of [W1; W2] regrouped as blocks
 // of 64: 32 rows of W1 followed by the same 32 rows of W2 (evo_amd/ops.py pack_gate_weights), 2 I rows in all.
-static int mlp_gate_mfma(const void* x, const float* row_scale, const void* w12g, void* a_out, int64_t M, int64_t I, int64_t K, int64_t act, void* stream);
-
 extern "C" int evo_mlp_gate_mfma_bf16(const void* x, const void* w12g, void* a_out, int64_t M, int64_t I, int64_t K, int64_t act, void* stream) {
-    return mlp_gate_mfma(x, nullptr, w12g, a_out, M, I, K, act, stream);
+    return gemmr_gate(x, nullptr, w12g, a_out, M, I, K, act, stream);
 }
 
 // ... with the post-mixer RMSNorm folded in: x = the residual stream itself, row_scale [ceil(M / 256) * 256] = 1 / (rms + eps) per row,
 // w12g = the regrouped rows of [W1 diag(g); W2 diag(g)] (see evo_linear_mfma_nf_bf16)
 extern "C" int evo_mlp_gate_mfma_nf_bf16(const void* x, const float* row_scale, const void* w12g, void* a_out, int64_t M, int64_t I, int64_t K,
                                          void* stream) {
-    return mlp_gate_mfma(x, row_scale, w12g, a_out, M, I, K, 0, stream);
+    return gemmr_gate(x, row_scale, w12g, a_out, M, I, K, 0, stream);
 }
 
-static int mlp_gate_mfma(const void* x, const float* row_scale, const void* w12g, void* a_out, int64_t M, int64_t I, int64_t K, int64_t act,
-                         void* stream) {
+int gemmr_gate(const void* x, const float* row_scale, const void* w12g, void* a_out, int64_t M, int64_t I, int64_t K, int64_t act, void* stream) {
     const int64_t N = 2 * I;
-    if ((act != 0 && act != 1) || (act && row_scale)) return -1;
+    if (act != 0 && act != 1) return -1;
     if (M <= 0 || I <= 0 || K <= 0 || N % GBN != 0 || K % GBK != 0 || K < 2 * GBK || N > 0x7fffffff / 2) return -1;
     if (M * K * 2 >= 0xffffffffll || N * K * 2 >= 0xffffffffll) return -1;
     GemmArgs a;
@@ -448,7 +445,8 @@ static int mlp_gate_mfma(const void* x, const float* row_scale, const void* w12g
         if (a.n_tiles <= 16 * n_cu) hipLaunchKernelGGL((gemmr_bf16_kernel<false, false, 1, false, NF, ACT, 8, true>), dim3((unsigned)n_cu), dim3(256), 0, (hipStream_t)stream, a); \
         else hipLaunchKernelGGL((gemmr_bf16_kernel<false, false, 1, false, NF, ACT, 8, false>), dim3((unsigned)n_cu), dim3(256), 0, (hipStream_t)stream, a); \
     } while (0)
-    if (row_scale) EVO_GATE(2, 0);
+    if (row_scale && act) EVO_GATE(2, 1);
+    else if (row_scale) EVO_GATE(2, 0);
     else if (act) EVO_GATE(0, 1);
     else EVO_GATE(0, 0);
 #undef EVO_GATE

@@ -706,7 +706,8 @@ static int gemmr_launch(const GemmArgs& a, int mode, int act, hipStream_t st) {
 #define GL_GO(...) hipLaunchKernelGGL((gemmr_bf16_kernel<__VA_ARGS__, MT>), dim3((unsigned)n_cu), dim3(256), 0, st, a)
     const bool bias = a.bias != nullptr, res = a.res != nullptr;
     if (mode == 1) {
-        if (a.rs) GL_GO(false, false, 1, false, 2, 0);
+        if (a.rs && act) GL_GO(false, false, 1, false, 2, 1);
+        else if (a.rs) GL_GO(false, false, 1, false, 2, 0);
         else if (act) GL_GO(false, false, 1, false, 0, 1);
         else GL_GO(false, false, 1, false, 0, 0);
     } else if (mode == 3) {
@@ -730,3 +731,6 @@ static int gemmr_launch(const GemmArgs& a, int mode, int act, hipStream_t st) {
 int gemmr_rows160(const GemmArgs& a, int mode, int act, hipStream_t st);
 int gemmr_rows192(const GemmArgs& a, int mode, int act, hipStream_t st);
 int gemmr_rows224(const GemmArgs& a, int mode, int act, hipStream_t st);
+
+// The gated layer on 256 rows a tile, with or without row factors, either gate (gemm.hip).
+int gemmr_gate(const void* x, const float* row_scale, const void* w12g, void* a_out, int64_t M, int64_t I, int64_t K, int64_t act, void* stream);

@@ -787,7 +787,7 @@ extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const voi
         float* qi = sumsq ? sumsq + m0 : nullptr;
         int rc;
         if (t.kind == T_PERSISTENT) {
-            if (mode == 1) rc = row_scale ? evo_mlp_gate_mfma_nf_bf16(xi, si, w, yi, t.rows, N / 2, K, stream) : evo_mlp_gate_mfma_bf16(xi, w, yi, t.rows, N / 2, K, act, stream);
+            if (mode == 1) rc = gemmr_gate(xi, si, w, yi, t.rows, N / 2, K, act, stream);
             else if (mode == 3) rc = row_scale ? evo_linear_t_mfma_nf_bf16(x, row_scale, w, bias, y, M, N, K, x_rows, Tm, row_skip, stream)
                                                : evo_linear_t_mfma_bf16(x, w, bias, y, M, N, K, stream);
             else if (xblk) rc = evo_linear_xblk_mfma_nf_bf16(xi, w, bias, ri, yi, qi, ss_ld, t.rows, N, K, stream);
