@@ -717,18 +717,19 @@ static bool dense_shape(int64_t mode, int64_t M, int64_t N, int64_t K) {
            && (mode != 3 || M % 256 == 0) && (mode != 2 || N * K * 2 < 0xffffffffll);
 }
 
-static int dense_plan(int64_t mode, bool stats, int64_t M, int64_t N, int64_t K, bool splits_ok, bool xblk, TilePlan (&plan)[2]) {
+// `square`: without tiles of 160 to 224 rows
+static int dense_plan(int64_t mode, bool stats, int64_t M, int64_t N, int64_t K, bool splits_ok, bool square, TilePlan (&plan)[2]) {
     splits_ok = splits_ok && M < 1024;                           // (from 1,024 rows on a row's result is the same bits in every batch: passes may be run in row groups)
     const bool persistent_ok = mode != 2 && K >= 128 && M * K * 2 < 0xffffffffll && N * K * 2 < 0xffffffffll;
-    return tile_plan(M, N, K, mode == 2 ? 1 : (int)mode, stats, splits_ok, persistent_ok, !xblk, plan);      // (blocks of 128 rows lie whole in a tile)
+    return tile_plan(M, N, K, mode == 2 ? 1 : (int)mode, stats, splits_ok, persistent_ok, !square, plan);
 }
 
 extern "C" int evo_dense_ws(int64_t mode, int64_t stats, int64_t M, int64_t N, int64_t K) {
     if (!dense_shape(mode, M, N, K)) return -1;
     int64_t most = 0;
-    for (const bool xblk : {false, true}) {                      // (either form of x)
+    for (const bool square : {false, true}) {                    // (whichever form the call has)
         TilePlan plan[2];
-        const int n = dense_plan(mode, stats != 0, M, N, K, true, xblk, plan);
+        const int n = dense_plan(mode, stats != 0, M, N, K, true, square, plan);
         for (int i = 0; i < n; ++i)
             if (plan[i].splits > 1 && plan[i].splits * plan[i].rows * N * 4 > most) most = plan[i].splits * plan[i].rows * N * 4;
     }
@@ -767,11 +768,13 @@ extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const voi
     if (xblk && (M % 256 != 0 || row_scale || act)) return -1;
     if (mode == 3 && row_scale ? (Tm <= 0 || Tm % 256 != 0 || M % Tm != 0 || row_skip < 0 || row_skip > 0x7fff || x_rows < M + (M / Tm - 1) * row_skip)
                                : (x_rows != 0 || Tm != 0 || row_skip != 0)) return -1;
+    // blocks of 128 rows of x lie whole in a tile; the persistent kernel has 32 bits for an operand's bytes, and tokens that are skipped between rows count (256 rows refuse)
+    const bool square = xblk || (mode == 3 && row_scale && x_rows * K * 2 >= 0xffffffffll);
     TilePlan plan[2];
-    int n = dense_plan(mode, sumsq != nullptr, M, N, K, true, xblk != 0, plan);
+    int n = dense_plan(mode, sumsq != nullptr, M, N, K, true, square, plan);
     for (int i = 0; i < n; ++i)
         if (plan[i].splits > 1 && (!ws || ws_bytes < plan[i].splits * plan[i].rows * N * 4)) {
-            n = dense_plan(mode, sumsq != nullptr, M, N, K, false, xblk != 0, plan);
+            n = dense_plan(mode, sumsq != nullptr, M, N, K, false, square, plan);
             break;
         }
     // (from 256 rows on the order of k is the persistent kernel's.  us, in step -> in turn: K = 2,048, 4,096 columns 8.5 -> 9.1 at 65 rows, 22,016 24.8 -> 23.4; [W1; W2] as it is
