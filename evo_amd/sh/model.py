@@ -899,10 +899,8 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
     packed_rows = 64 * 1024      # rows of one such pass
 
     def _prompt_groups(self, lens: List[int]) -> List[List[int]]:
-        """Prompts that share a pass: those of 4 to 4,096 tokens, as many as fit, when the matrix-core operator takes every Hyena layer; longer ones fill the dense
-        layers by themselves.  (Four layers of width 4,096, us, one by one -> together: 16 prompts of 4 tokens 7,180 -> 2,410, of 31 7,870 -> 2,480, of 100 10,800 -> 3,510;
-        3 of 8 1,405 -> 1,180.  Two of fewer than 32 tokens stay alone: 2 of 8 950 -> 1,150, of 31 1,040 -> 1,190, of 40 1,080 -> 1,150, of 64 1,140 -> 1,160,
-        of 200 1,650 -> 1,430.)"""
+        """Prompts that share a pass: those of 32 to 4,096 tokens, as many as fit, when the matrix-core operator takes every Hyena layer.  (Shorter
+        ones take the modal kernels; longer ones fill the dense layers by themselves.)"""
         if not self._packed:
             self._pack()
         ops = self.ops
@@ -910,19 +908,17 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
               and self.hidden_size == self.num_heads * 128 and ops.zt_shape_ok(1, self.packed_rows, 3 * self.hidden_size, self.hidden_size) and getattr(self, "block_taps", None) is None
               and all(isinstance(b, _AttentionBlock) or (b.projections.weight.is_contiguous() and b.projections.weight.dtype == torch.bfloat16
                                                          and self._table_ok(b)) for b in self.blocks))
-        groups, open_, rows = [], None, 0                         # (the pass that still takes prompts, its rows)
+        groups, rows = [], 0
         for n, m in enumerate(lens):
             need = (m + 63) // 64 * 64
-            if not (ok and max(4, self.short_filter_length - 1) <= m <= 4096):
-                groups.append([n])
-            elif open_ is not None and rows + need <= self.packed_rows:
-                open_.append(n)
+            share = ok and 32 <= m <= 4096
+            if share and rows and rows + need <= self.packed_rows:
+                groups[-1].append(n)
                 rows += need
             else:
-                open_, rows = [n], need
-                groups.append(open_)
-        few = [g for g in groups if len(g) == 2 and max(lens[n] for n in g) < 32]
-        return [g for g in groups if g not in few] + [[n] for g in few for n in g]
+                groups.append([n])
+                rows = need if share else 0
+        return groups
 
     def _prefill_packed(self, prompts: List[torch.Tensor]):
         """Prompts behind each other as ONE stream of rows, each from a multiple of 64 on (the rows between are token 0 and reach nobody: every
@@ -1001,7 +997,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
     def prefill_rows(self, prompts: List[torch.Tensor], want: Optional[List[List[int]]] = None):
         """Prompts ([P] ids) of any lengths -> [(logits [wanted, V], caches, row of the caches)], several in a pass where they can share one
         (_prompt_groups); `want`: the places whose logits are returned (the last token's by default)."""
-        out = [None] * len(prompts)
+        out = []
         for group in self._prompt_groups([p.numel() for p in prompts]):
             if len(group) > 1:
                 h, first, caches = self._prefill_packed([prompts[n] for n in group])
@@ -1012,8 +1008,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             at = [[prompts[n].numel() - 1] if want is None else [self._place(t, prompts[n].numel()) for t in want[n]] for n in group]
             rows = torch.tensor([f + t for f, ts in zip(first, at) for t in ts], dtype=torch.int64, device=h.device)
             logits = self.ops.linear(h[rows].contiguous(), self.unembed.weight, None) if rows.numel() else h.new_empty(0, self.vocab_size)
-            for n, lg, ipd in zip(group, logits.split([len(ts) for ts in at]), caches):
-                out[n] = (lg, ipd, 0)
+            out += [(lg, ipd, 0) for lg, ipd in zip(logits.split([len(ts) for ts in at]), caches)]
         return out
 
     # upstream names, kept for callers that reach for them
