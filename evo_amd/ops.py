@@ -395,10 +395,14 @@ class HipOps(MixerOps):
         y = torch.empty(M, N, dtype=torch.float32, device=x.device)
         plan = (_c.c_int64 * 6)()
         if self.lib.evo_linear_f32_ahead_plan(M, N, K, _c.cast(plan, _PTR)) == 1:
-            ws = torch.empty(plan[5], dtype=torch.uint8, device=x.device)
-            with self._t("gemm_f32"):
-                _check(self.lib.evo_linear_f32_ahead(x.data_ptr(), w.data_ptr(), _ptr(b), y.data_ptr(), M, N, K, ws.data_ptr(), plan[5], _stream()), "evo_linear_f32_ahead")
-            return y
+            try:
+                ws = torch.empty(plan[5], dtype=torch.uint8, device=x.device)
+            except torch.cuda.OutOfMemoryError:                  # (up to 1 GiB: a card with less left takes the form that splits as it goes)
+                ws = None
+            if ws is not None:
+                with self._t("gemm_f32"):
+                    _check(self.lib.evo_linear_f32_ahead(x.data_ptr(), w.data_ptr(), _ptr(b), y.data_ptr(), M, N, K, ws.data_ptr(), plan[5], _stream()), "evo_linear_f32_ahead")
+                return y
         n = self.lib.evo_linear_f32_ws(M, N, K)
         ws = torch.empty(n * M * N, dtype=torch.float32, device=x.device) if n > 0 else None
         with self._t("gemm_f32"):
