@@ -662,6 +662,20 @@ static int tile_plan(int64_t M, int64_t N, int64_t K, int mode, bool stats, bool
     return 1;
 }
 
+// X and W in phases (gemm_tile_kernel) where the last row tile has 96 of its 128 rows (120 of more than four tiles), and at 150 to 192 rows on 192, 80 to 96 on 96: rows that are not there cost no intake,
+// a tile without them runs ahead of those that share its weights (4,096 columns, K = 11,008: 102.6 -> 91.7 at 896 rows, 81.1 -> 92.4 at 912), and W is further
+// ahead without.  us, in turn -> in phases: 12,288 columns, K = 4,096, 43.6 -> 37.9 at 256 rows, 41.6 -> 37.2 at 128, 38.6 -> 36.9 at 104, 33.0 -> 35.9 at 161; 4,096 columns,
+// K = 11,008, 104 -> 93 at 1,024; 22,016 gated columns 48.0 -> 44.9 at 161, 52.5 -> 46.6 at 192, 47.9 -> 50.5 at 129 (192 rows), 39.3 -> 38.0 at 90 (96).  Parts of K: 0.94 to 1.03.
+// Not where x is what comes from HBM (512 columns at 8,190 rows 34.2 -> 37.5): from four columns a row on; nor below 1,024 k (4,096 columns at 757 rows, K = 512 7.4 -> 7.9).
+// -> W slots of the loop in phases, 0: the other loop.
+static int tile_phases(int kind, int mode, bool xblk, int splits, int64_t M, int64_t N, int64_t K) {
+    if (splits != 1 || xblk || mode > 2) return 0;
+    if (kind == 2) return K >= 1024 && 4 * M <= N && (M - 1) % 128 >= (M > 512 ? 119 : 95) ? 6 : 0;
+    if (kind == T_ODD) return M >= 80 && M <= 96 && K >= 4096 ? 8 : 0;
+    if (kind == T_ODD + 1) return M >= 150 && M <= 192 && K >= 1024 ? 5 : 0;
+    return 0;
+}
+
 template <int BM, int BN, int WGM, int WGN, int NS, int PER_CU, bool GATE>
 static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, float* ws, hipStream_t st) {
     a.tiles_m = (int)((a.M + BM - 1) / BM);
@@ -669,13 +683,8 @@ static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, flo
     a.group_m = 8;
     a.n_tiles = a.tiles_m * a.tiles_n * splits;
     const dim3 grid((unsigned)a.n_tiles), block(64 * WGM * WGN);
-    // X and W in phases (gemm_tile_kernel) where the last row tile has 96 of its 128 rows (120 of more than four tiles), and at 150 to 192 rows on 192, 80 to 96 on 96: rows that are not there cost no intake,
-    // a tile without them runs ahead of those that share its weights (4,096 columns, K = 11,008: 102.6 -> 91.7 at 896 rows, 81.1 -> 92.4 at 912), and W is further
-    // ahead without.  us, in turn -> in phases: 12,288 columns, K = 4,096, 43.6 -> 37.9 at 256 rows, 41.6 -> 37.2 at 128, 38.6 -> 36.9 at 104, 33.0 -> 35.9 at 161; 4,096 columns,
-    // K = 11,008, 104 -> 93 at 1,024; 22,016 gated columns 48.0 -> 44.9 at 161, 52.5 -> 46.6 at 192, 47.9 -> 50.5 at 129 (192 rows), 39.3 -> 38.0 at 90 (96).  Parts of K: 0.94 to 1.03.
-    // Not where x is what comes from HBM (512 columns at 8,190 rows 34.2 -> 37.5): from four columns a row on; nor below 1,024 k (4,096 columns at 757 rows, K = 512 7.4 -> 7.9).
     if constexpr (BM == 128 && BN == 128) {
-        if (splits == 1 && !xblk && mode <= 1 && a.K >= 1024 && 4 * a.M <= a.N && (a.M - 1) % BM >= (a.tiles_m > 4 ? 119 : 95)) {
+        if (tile_phases(2, mode, xblk, splits, a.M, a.N, a.K)) {
             if (mode == 1) hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, 16, PER_CU, 1, false, false>), grid, block, 0, st, a, act, ws, splits);
             else hipLaunchKernelGGL((gemm_tile_kernel<BM, BN, WGM, WGN, 16, PER_CU, 0, false, false>), grid, block, 0, st, a, act, ws, splits);
             return evo_launch_status();
@@ -736,10 +745,10 @@ extern "C" int evo_dense_ws(int64_t mode, int64_t stats, int64_t M, int64_t N, i
     return (int)most;
 }
 
-extern "C" int evo_dense_plan(int64_t mode, int64_t stats, int64_t M, int64_t N, int64_t K, int64_t* out) {
-    if (!dense_shape(mode, M, N, K) || !out) return -1;
+extern "C" int evo_dense_launches(int64_t mode, int64_t stats, int64_t xblk, int64_t M, int64_t N, int64_t K, int64_t* out) {
+    if (!dense_shape(mode, M, N, K) || !out || (xblk && (mode != 0 || M % 256 != 0))) return -1;
     TilePlan plan[2];
-    const int n = dense_plan(mode, stats != 0, M, N, K, true, false, plan);
+    const int n = dense_plan(mode, stats != 0, M, N, K, true, xblk != 0, plan);
     int64_t m0 = 0;
     for (int i = 0; i < n; ++i) {
         const TilePlan& t = plan[i];
@@ -750,10 +759,18 @@ extern "C" int evo_dense_plan(int64_t mode, int64_t stats, int64_t M, int64_t N,
         a.ss_ld = (M + 255) / 256 * 256;
         const int64_t tiles_end = (t.rows + bm - 1) / bm * bm;   // (the persistent kernel stores the statistic of whole tiles)
         const int64_t stored = !stats ? 0 : t.kind != T_PERSISTENT && t_stat_rows(a) < tiles_end ? t_stat_rows(a) : tiles_end;
-        const int64_t row[7] = {m0, t.rows, bm, bn, t.splits, t.kind >= T_SHORT, m0 + stored};
-        for (int k = 0; k < 7; ++k) out[7 * i + k] = row[k];
+        const int64_t row[8] = {m0, t.rows, bm, bn, t.splits, t.kind >= T_SHORT, m0 + stored, tile_phases(t.kind, (int)mode, xblk != 0, t.splits, t.rows, N, K)};
+        for (int k = 0; k < 8; ++k) out[8 * i + k] = row[k];
         m0 += t.rows;
     }
+    return n;
+}
+
+extern "C" int evo_dense_plan(int64_t mode, int64_t stats, int64_t M, int64_t N, int64_t K, int64_t* out) {
+    int64_t row[16];
+    const int n = out ? evo_dense_launches(mode, stats, 0, M, N, K, row) : -1;
+    for (int i = 0; i < n; ++i)
+        for (int k = 0; k < 7; ++k) out[7 * i + k] = row[8 * i + k];
     return n;
 }
 
@@ -807,7 +824,7 @@ extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const voi
                 a.M = N; a.N = (int)M;
                 if (row_scale) { a.w_rows = x_rows; a.tm_tiles = (int)(Tm / 256); a.row_skip = (int)row_skip; }
             }
-            const int tm = mode == 2 ? 1 : (int)mode;
+            const int tm = mode == 2 ? 1 : (int)mode, phases = tile_phases(t.kind, tm, xblk != 0, t.splits, a.M, a.N, a.K);
             float* f = (float*)ws;
             hipStream_t st = (hipStream_t)stream;
             if (t.kind >= T_SHORT) rc = t.kind == T_SHORT ? gemmr_rows160(a, tm, (int)act, st) : t.kind == T_SHORT + 1 ? gemmr_rows192(a, tm, (int)act, st) : gemmr_rows224(a, tm, (int)act, st);
@@ -818,8 +835,8 @@ extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const voi
             else if (t.kind == 4) rc = tile_launch<256, 128, 4, 2, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
             else if (t.kind == 5) rc = tile_launch<128, 256, 2, 4, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
             else if (xblk || tm > 1 || (tm == 1) != (t.kind < T_ODD + 2)) rc = -1;
-            else if (t.kind == T_ODD) rc = a.M >= 80 && a.M <= 96 && a.K >= 4096 ? tile_launch_odd<96, 96, 2, 3, 18, 1>(a, (int)act, st) : tile_launch_odd<96, 96, 2, 3, 6, 1>(a, (int)act, st);
-            else if (t.kind == T_ODD + 1) rc = a.M >= 150 && a.M <= 192 && a.K >= 1024 ? tile_launch_odd<192, 96, 4, 3, 15, 1>(a, (int)act, st) : tile_launch_odd<192, 96, 4, 3, 4, 1>(a, (int)act, st);
+            else if (t.kind == T_ODD) rc = phases ? tile_launch_odd<96, 96, 2, 3, 18, 1>(a, (int)act, st) : tile_launch_odd<96, 96, 2, 3, 6, 1>(a, (int)act, st);
+            else if (t.kind == T_ODD + 1) rc = phases ? tile_launch_odd<192, 96, 4, 3, 15, 1>(a, (int)act, st) : tile_launch_odd<192, 96, 4, 3, 4, 1>(a, (int)act, st);
             else rc = tile_launch_odd<96, 48, 3, 1, 8, 0>(a, (int)act, st);
         }
         if (rc != 0) return rc;

@@ -56,6 +56,7 @@ _SIGNATURES = {
     "evo_hyena_ct_packed": ([_PTR] * 9 + [_I64] * 5 + [_PTR], _c.c_int),
     "evo_attn_fwd_packed_bf16": ([_PTR] * 4 + [_I64] * 9 + [_PTR] * 2 + [_I64, _PTR, _F32, _PTR, _PTR], _c.c_int),
     "evo_dense_ws": ([_I64] * 5, _c.c_int),
+    "evo_dense_launches": ([_I64] * 6 + [_PTR], _c.c_int),
     "evo_dense_plan": ([_I64] * 5 + [_PTR], _c.c_int),
     "evo_dense_bf16": ([_I64] * 3 + [_PTR] * 7 + [_I64] * 8 + [_PTR, _I64, _PTR], _c.c_int),
     "evo_linear_t_mfma_nf_bf16": ([_PTR] * 5 + [_I64] * 6 + [_PTR], _c.c_int),
@@ -107,7 +108,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 25         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 26         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):

@@ -66,8 +66,9 @@ extern "C" {
  *  22: evo_lightning_chunk_bf16 and evo_rglru_chunk_bf16 keep the states of cut sequences only: `seg` by the rows, not by the sequences.
  *  23: evo_attn_fwd_packed_bf16 gained `form`.
  *  24: evo_linear_f32_ahead and evo_linear_f32_ahead_plan added.
- *  25: evo_linear_few_f32 added. */
-#define EVO_ABI_VERSION 25
+ *  25: evo_linear_few_f32 added.
+ *  26: evo_dense_launches added. */
+#define EVO_ABI_VERSION 26
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
@@ -357,9 +358,11 @@ int evo_linear_t_mfma_nf_bf16(const void* x, const float* row_scale, const void*
  *   mode 3: z^T of evo_linear_t_mfma_nf_bf16, M = Mp; x_rows, Tm, row_skip as there with row_scale, 0 without
  * N % 256 == 0, K % 64 == 0; M % 256 == 0 for mode 3 and xblk; N K 2 < 4 GiB for mode 2.  `ws`: evo_dense_ws(mode, sumsq != NULL, M, N, K) bytes, 16-byte
  * aligned; NULL or fewer: the same product without parts of K.
- * evo_dense_plan: the one or two launches (the result) that evo_dense_bf16 makes with that workspace, needs no GPU; seven values each in `out` [14], a HOST array:
- * first row, rows, rows of a tile, columns of a tile (tokens, weight rows for mode 3), parts of K, 1 for the persistent kernel, and the row behind the last whose
- * sum of squares it stores (at most M rounded up to 256). */
+ * evo_dense_launches: the one or two launches (the result) that evo_dense_bf16 makes with that workspace, needs no GPU; eight values each in `out` [16], a HOST
+ * array: first row, rows, rows of a tile, columns of a tile (tokens, weight rows for mode 3), parts of K, 1 for the persistent kernel, the row behind the last whose
+ * sum of squares it stores (at most M rounded up to 256), and the slots of w of the loop that takes its operands in phases (0: the other loop).
+ * evo_dense_plan: the first seven of them, out [14], x row-major. */
+int evo_dense_launches(int64_t mode, int64_t stats, int64_t xblk, int64_t M, int64_t N, int64_t K, int64_t* out);
 int evo_dense_plan(int64_t mode, int64_t stats, int64_t M, int64_t N, int64_t K, int64_t* out);
 int evo_dense_ws(int64_t mode, int64_t stats, int64_t M, int64_t N, int64_t K);
 int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const void* x, const void* w, const void* bias, const void* residual, void* y,

@@ -1,8 +1,10 @@
-"""128 x 128 tiles whose operands come in phases (csrc/gemm_tile.hip PHASES): sixteen k-steps and seventeen, full last row tiles and ones a quarter short; below, and one row
-fewer, the other inner loop (K up to 2,048: above, tiles of fewer than 256 rows start a k-step apart and sum in another order).  The persistent kernel's bits in every form, and rows behind the last untouched.  (192 x 96 and 96 x 96: test_gpu_dense_tiles.py at 161, 192 and 96 rows.)"""
+"""Tiles of 128 x 128, 192 x 96 and 96 x 96 whose operands come in phases (csrc/gemm_tile.hip PHASES): full last row tiles and ones a quarter short; below, and one row
+fewer, the other inner loop.  128 x 128: sixteen k-steps and seventeen (K up to 2,048: above, tiles of fewer than 256 rows start a k-step apart and sum in another order), the
+persistent kernel's bits in every form.  The narrow tiles: odd counts of k-steps, against fp64 sums.  Rows behind the last untouched."""
 import pytest
 import torch
 
+from test_dense_launches import all_launches
 from test_dense_plan import launches
 
 pytestmark = pytest.mark.gpu
@@ -14,6 +16,7 @@ def test_phases(M, N, K):
     from test_gpu_dense_tiles import _data, _ops
     from evo_amd.ops import _stream
     assert all([(p["tile_rows"], p["tile_cols"], p["parts"]) for p in launches(m, s, M, N, K)] == [(128, 128, 1)] for m, s in ((0, False), (0, True), (1, False)))
+    assert all([p["slots"] for p in all_launches(m, s, False, M, N, K)] == [6 if K >= 1024 and M != 223 else 0] for m, s in ((0, False), (0, True), (1, False)))
     ops, ld = _ops(), (M + 255) // 256 * 256
     g, x, w = _data(M, N, K, 12)
     b, r = (torch.randn(*s, device="cuda", generator=g).bfloat16() for s in ((N,), (M, N)))
@@ -41,3 +44,13 @@ def test_phases(M, N, K):
     assert ops.lib.evo_mlp_gate_mfma_bf16(x.data_ptr(), w.data_ptr(), want.data_ptr(), M, N // 2, K, 0, _stream()) == 0
     ops._dense_layer(1, x, w, got, M, N, K)
     assert torch.equal(got, want) and bool((got[M:] == 7).all())
+
+
+@pytest.mark.parametrize("M,N,K,tile,slots", [(80, 22016, 4096, 96, 8), (96, 20992, 4160, 96, 8), (79, 22016, 4096, 96, 0), (96, 20992, 4032, 96, 0),
+                                              (192, 24576, 1024, 192, 5), (150, 22016, 1088, 192, 5), (149, 22016, 1088, 192, 0), (161, 21760, 960, 192, 0)])
+def test_narrow_tiles(M, N, K, tile, slots):
+    """96 gated columns: eight or five slots of w, first and last row of the ranges; one row or one k-step outside them the loop in turn."""
+    from test_gpu_dense_tiles import test_tiles_of_odd_widths as compare
+    for mode in (1, 2):
+        assert [(p["tile_rows"], p["tile_cols"], p["parts"], p["slots"]) for p in all_launches(mode, False, False, M, N, K)] == [(tile, 96, 1, slots)]
+    compare(M, N, K, (tile, 96))
