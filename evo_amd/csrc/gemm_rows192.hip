@@ -6,6 +6,6 @@ int gemmr_rows192(const GemmArgs& args, int mode, int act, hipStream_t st) {
     a.tiles_m = (int)((a.M + 191) / 192);
     a.tiles_n = a.N / GBN;
     a.n_tiles = a.tiles_m * a.tiles_n;
-    a.group_m = (mode == 3 ? a.tiles_m : a.tiles_n) >= 32 ? 8 : 4;
+    a.group_m = mode == 3 ? gemmr_group(a.tiles_n, a.tiles_m) : gemmr_group(a.tiles_m, a.tiles_n);
     return gemmr_launch<6>(a, mode, act, st);
 }
