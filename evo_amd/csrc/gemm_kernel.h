@@ -729,7 +729,7 @@ static int gemmr_launch(const GemmArgs& a, int mode, int act, hipStream_t st) {
 
 // How many tiles along the tokens come next to each other before the next one along the weight: 4, or 8 where the weight is 32 tiles and wider; one or two more where the last
 // group would be a single tile, all of whose neighbours are at other weight rows (at K = 16,384, whose rows are 32 KiB apart, 1,700 rows x 6,912 columns took 374 us on nine
-// tiles of 192 rows as 4 + 4 + 1, 270 as 5 + 4; 249 layers of 2 to 41 such tiles: 0.99 in the mean, at most 1.02).
+// tiles of 192 rows as 4 + 4 + 1, 286 as 5 + 4; 249 layers of 2 to 41 such tiles: 0.99 in the mean, at most 1.02).
 static inline int gemmr_group(int tokens, int weight) {
     int g = weight >= 32 ? 8 : 4;
     while (tokens > g && tokens % g == 1) ++g;

@@ -572,8 +572,13 @@ static const TileKind kinds[] = {{64, 64, 0.255}, {128, 64, 0.435}, {128, 128, 0
 // (160), 159 -> 124 at 770 (160), 163 -> 147 at 1,025 (224), 247 -> 221 at 1,600 (224), 502 -> 469 at 3,600 (224); 12,288 columns 82 -> 69 at 930 (192), 136 -> 115 at 1,300 (160);
 // K = 11,008, 4,096 columns 193 -> 145 at 2,100 (160), 402 -> 353 at 6,000 (192).
 static const int short_rows[] = {160, 192, 224};
-static const double short_us[] = {0.895, 1.022, 1.107};
-static const double short_power[] = {1.11, 1.01, 1.01};  // time at the power limit, by the square tiles'
+// A step of 64 k of those tiles, and of 256 rows beside them: `us`, and `more` for each unit of the chip's rounds beyond `from` that is rows of the result (power).  Measured, us
+// at under half, three quarters and all of a round: 160 rows 0.80, 0.90, 0.99; 192 0.86, 1.02, 1.11; 224 0.93, 1.16, 1.27; 256 1.19, 1.25, 1.43, in one round as in nine and at
+// K = 2,048 to 22,528 (3,587 layers of 256 to 10,000 rows, 3 to 6 % about these; 256 rows are taken at 2 % less, which the plans of before had).  `end`: a round's first
+// operands and results.
+struct StepUs { int rows; double us, from, more, end; };
+static const StepUs short_steps[] = {{160, 0.895, 0.76, 0.45, 2.43}, {192, 1.022, 0.76, 0.47, 2.43}, {224, 1.107, 0.66, 0.62, 2.43}};
+static const StepUs whole_steps = {256, 1.16, 0.68, 0.85, 4.5};
 #define T_SHORT 96                           // first of them
 #define T_PERSISTENT 99
 
@@ -637,24 +642,29 @@ static int tile_plan_square(int64_t M, int64_t N, int64_t K, int mode, bool stat
     return 1;
 }
 
-// ... or one launch of the persistent kernel on 160, 192 or 224 rows.  Over 330 layers and sizes (K = 2,048 to 16,384, 260 to 32,768 rows) the choice is 0.2 % off the fastest of all
-// plans on average (5.3 % without them).  Where many rounds run at the power limit, 256 rows are ahead (32,768 rows, 22,016 gated columns: 4.01 ms, 4.31 on 224, 4.34 on 192, 4.48 on
-// 160).  A tail launch finds its weights in the caches: nine tenths of its time by itself.  Below 2,048 k the plans are as they were (4,096 columns at K = 1,024 could
+static double steps_us(const StepUs& s, double rows, double cols, double nk) {
+    const double cus = tile_cus(), rounds = ceil(ceil(rows / s.rows) * cols / cus), full = rows / s.rows * cols / (rounds * cus);
+    return rounds * (nk * (s.us + s.more * fmax(0.0, full - s.from)) + s.end);
+}
+
+// ... or one launch of the persistent kernel on 160, 192 or 224 rows.  Over 3,587 layers and sizes (K = 2,048 to 22,528, 256 to 10,000 rows) the choice is 0.4 % off the fastest of
+// all plans on average (4.8 % without them), and more than 3 % behind the plan without them at seven (at most 9 %: 224 rows in a full round at K = 16,384).  Where many rounds run at
+// the power limit, 256 rows are ahead (32,768 rows, 22,016 gated columns: 4.01 ms, 4.31 on 224, 4.34 on 192, 4.48 on 160).  Two launches take 3 to 9 % more than their sum, a tail
+// that finds its weights in the caches nine tenths of its time.  Below 2,048 k the plans are as they were (4,096 columns at K = 1,024 could
 // still go from 41 to 37 us at 4,700 rows: layers that small are launches more than work).  Below 256 rows neighbouring tiles start one k-step apart, which these do not; and
 // their padding is most of a tile.
 static int tile_plan(int64_t M, int64_t N, int64_t K, int mode, bool stats, bool splits_ok, bool persistent_ok, bool short_ok, TilePlan (&out)[2]) {
     const int n = tile_plan_square(M, N, K, mode, stats, splits_ok, persistent_ok, out);
     if (!persistent_ok || !short_ok || M < 256 || K < 2048) return n;
-    const double cus = tile_cus(), power = 2.0 * M * N * K / 1.56e9, memory = (2.0 * (M * K + N * K) + 2.0 * M * N) / 4.9e6;
-    double us = n == 2 ? out[0].us + 0.9 * out[1].us + 4.0 : out[0].us;
-    if (mode == 1 && n == 1 && out[0].kind != T_PERSISTENT) us -= 3.0;       // (one tile's closing with the gate: 11,008 gated columns at 390 rows 51.9 on 256 x 128, 58.8 on 160)
+    const double memory = (2.0 * (M * K + N * K) + 2.0 * M * N) / 4.9e6, nk = (double)(K / 64);
+    const double rows = (double)(mode == 3 ? N : M), cols = (double)((mode == 3 ? M : N) / 256);       // (mode 3: the tokens are the columns of the launch)
+    double us = out[0].us;
+    if (n == 2) us = 1.03 * (us + 0.9 * out[1].us + 4.0);
+    else if (out[0].kind == T_PERSISTENT) us = fmax(steps_us(whole_steps, rows, cols, nk), memory);
+    else if (mode == 1 && out[0].splits == 1) us -= 3.0;         // (one tile's closing with the gate: 11,008 gated columns at 390 rows 51.9 on 256 x 128, 58.8 on 160)
     int kind = -1;
     for (int i = 0; i < 3; ++i) {
-        const int64_t rows = mode == 3 ? N : M, cols = mode == 3 ? M : N;      // (mode 3: the tokens are the columns of the launch)
-        double t = ceil((double)((rows + short_rows[i] - 1) / short_rows[i]) * (double)(cols / 256) / cus) * ((double)(K / 64) * short_us[i] + 2.43);
-        if (t < short_power[i] * power) t = short_power[i] * power;
-        if (K >= 16384) t *= 1.08;                               // (4,096 columns 489 us in two launches, 523 on 160, at 4,928 rows; 269 and 206 at 2,100)
-        if (t < memory) t = memory;
+        const double t = fmax(steps_us(short_steps[i], rows, cols, nk), memory);
         if (t < us) { us = t; kind = T_SHORT + i; }
     }
     if (kind < 0) return n;

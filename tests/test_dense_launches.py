@@ -44,3 +44,15 @@ def test_the_short_form():
                                                    (1, 149, 22016, 4096, 192, 0), (1, 161, 21760, 960, 192, 0)])
 def test_which_loop(mode, M, N, K, tile, slots):
     assert [(p["tile_rows"], p["slots"]) for p in all_launches(mode, False, False, M, N, K)] == [(tile, slots)]
+
+
+def test_the_tile_hangs_on_the_size_and_not_on_one_width():
+    """No width of K where tiles change all at once: neighbouring ones take the same launches at 98.5 of 100 sizes."""
+    for mode in (0, 1):
+        for K in (2112, 4096, 8192, 11008, 16320, 16384):
+            other = total = 0
+            for N in range(2048, 13000, 512):
+                for M in range(256, 6000, 91):
+                    total += 1
+                    other += [tuple(p[k] for k in KEYS) for p in launches(mode, False, M, N, K)] != [tuple(p[k] for k in KEYS) for p in launches(mode, False, M, N, K - 64)]
+            assert other <= 0.015 * total, (mode, K, other, total)
