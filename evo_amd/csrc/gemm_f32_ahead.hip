@@ -120,7 +120,7 @@ __device__ __forceinline__ void fa_again(uint64_t odd, const float* x, const flo
     }
 }
 
-// Workgroup = BM = 16 TM rows x 256 columns of y, four waves of 64 columns each in 16 x 16 x 32 products, D stages of 32 k ahead.
+// Workgroup = BM = 16 TM rows x 256 columns of y, eight waves of 32 columns each in 16 x 16 x 32 products, D stages of 32 k ahead.
 template <int TM, int D>
 __global__ __launch_bounds__(512, 2) void gemm_f32_ahead_kernel(FaArgs a) {
     constexpr int CN = 2, NW = 8, BM = 16 * TM, NX = 3 * TM, PX = (NX + NW - 1) / NW, PW = 2 * CN, P = PX + PW, XS = NX * 1024, WS = 32768, XB = (D + 1) * XS;

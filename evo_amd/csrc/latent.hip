@@ -65,7 +65,7 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(PrepArgs a) {
 
 // The same in 16-byte requests (8 bf16 or 4 fp32 at a time twice) where every part is whole ones: three waves rotate, the fourth norms, and what a thread needs is asked for
 // before the angles; the roundings and the order of the sums are latent_prep_kernel's.  A decode step waits for one round of requests where it waited for one each pair of elements after the other, a prompt is a fifth of the instructions.
-// 32 heads of 128 + 64, R = 512, pair by pair -> this: 8 tokens decoded 4.4 -> 2.9 us, 329 of a prompt 5.2 -> 3.4, 1,500 8.3 -> 5.3, 11,877 41 -> 23.
+// 32 heads of 128 + 64, R = 512, pair by pair -> this: 8 tokens decoded 4.1 -> 2.6 us, 11,877 of a prompt 38.2 -> 22.2.
 template <typename T>
 __global__ __launch_bounds__(256) void latent_prep_vec_kernel(PrepArgs a) {
     extern __shared__ float2 turn[];                             // [n_rot / 2] cosine and sine of this token's angles
@@ -491,7 +491,8 @@ __global__ __launch_bounds__(64) void latent_decode_any_kernel(DecArgs a, int dq
 }
 
 // fp32 rows in 16-byte requests: four waves per (split, head, sequence), each 16 of a tile's 64 slots.  Latency bounds it, a wave's requests one behind the other (the rows
-// themselves come from L2, every head reads them).  Behind 500 tokens of 576, 3 sequences x 32 heads: one wave per 64 slots 25.8 us, this 12.3 (2 x 1,000 slots 25.4 -> 14.0, 8 x 1,000 54 -> 47, one of 60 23.7 -> 8.3)
+// themselves come from L2, every head reads them).  Behind 500 tokens of 576, 3 sequences x 32 heads: one wave per 64 slots 25.8 us, this 12.3 by itself (36.1 -> 22.6 in the trace of such a
+// decode, where eight of the ring's sixteen parts have no slot; 2 x 1,000 slots 25.4 -> 14.0, 8 x 1,000 54 -> 47, one of 60 23.7 -> 8.3)
 __global__ __launch_bounds__(256) void latent_decode_f32_kernel(DecArgs a, int dq) {
     extern __shared__ __attribute__((aligned(16))) float qf[];   // [dq]
     __shared__ float sc[64];

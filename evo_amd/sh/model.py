@@ -514,7 +514,8 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
     def _mfma_hyena_ok(self, B: int, T: int) -> bool:
         """The single-pass matrix-core operator (csrc/hyena_ct.hip) serves every parallel (T > 1) Hyena call without a padding mask on
         the HIP backend -- scoring, cached prefill with carry-in / end state, sequence-parallel shards -- when the shape fits its launch
-        contract; masks and very short inputs take the modal kernels.  (Shape part only: _hyena_ct_ok adds the tensors' checks.)"""
+        contract; masks and very short inputs take the modal kernels.  (That contract only: below 1,024 rows _hyena_ct_ok leaves most layers token-major, on the modal kernels;
+        sequence-parallel shards go by this contract alone.)"""
         ops = self.ops
         D, H = self.hidden_size, self.num_heads
         if not getattr(ops, "hyena_mfma", False) or not hasattr(ops, "hyena_ct") or D != H * 128:
@@ -545,10 +546,11 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
     def _hyena_ct_ok(self, x2d, blk, B, T) -> bool:
         """Whether the layer goes channel-major.  Below 1,024 rows it does not: z^T and the blocked y are rows padded to multiples of 64 and 256, gathers and a launch for the
         remainder, and the operator is 16 channels a CU; token-major it is one launch (csrc/hyena.hip hyena_short_kernel) or three.  (Four layers, us, channel- ->
-        token-major.  Width 4,096: 1 x 261 992 -> 898, 4 x 77 1,048 -> 942, 1 x 521 1,425 -> 1,333, 16 x 42 1,587 -> 1,405, 1 x 1,001 1,834 -> 1,785, with end states 1,137 -> 926
-        and 1,991 -> 1,833 of the first and last; 1,024: 509 -> 400, 497 -> 412; 8,192: 2,876 -> 2,676, 5,491 -> 5,548.)  A token behind
-        whole tiles of 512 (1 x 513: 1,470, token-major 1,325) stays with its split below.  From 1,024 rows on, 1.00 to 1.17 by the rows' lengths, a row has the same bits in every
-        batch that way."""
+        token-major, at 1 x 261, 8 x 77, 1 x 1,001 and 1 x 1,023: width 1,024 477 -> 375, 460 -> 355, 464 -> 381, 461 -> 380; 2,048 510 -> 440, 651 -> 576, 768 -> 751, 776 -> 759;
+        4,096 947 -> 849, 1,482 -> 1,350, 1,795 -> 1,765, 1,780 -> 1,759; 8,192 2,845 -> 2,649, 4,395 -> 4,131, 5,559 -> 5,556, 5,571 -> 5,600.  With end states at 4,096 1 x 261
+        1,137 -> 926, 1 x 1,001 1,991 -> 1,833.)  A token behind
+        whole tiles of 512 (1 x 513: 1,470, token-major 1,325) stays with its split below.  From 1,024 rows on, 0.98 to 1.09 by width and the rows' lengths, a row has the same bits
+        in every batch that way."""
         ops = self.ops
         w = blk.projections.weight
         return ((B * T >= 1024 or ops.zt_layout(B, T)[3] == 1) and getattr(ops, "hyena_ct_flag", False) and hasattr(ops, "hyena_ct") and x2d.is_cuda and w.dtype == torch.bfloat16
