@@ -358,7 +358,7 @@ int evo_linear_t_mfma_nf_bf16(const void* x, const float* row_scale, const void*
  *   mode 3: z^T of evo_linear_t_mfma_nf_bf16, M = Mp; x_rows, Tm, row_skip as there with row_scale, 0 without
  * N % 256 == 0, K % 64 == 0; M % 256 == 0 for mode 3 and xblk; N K 2 < 4 GiB for mode 2.  `ws`: evo_dense_ws(mode, sumsq != NULL, M, N, K) bytes, 16-byte
  * aligned; NULL or fewer: the same product without parts of K.
- * evo_dense_launches: the one or two launches (the result) that evo_dense_bf16 makes with that workspace, needs no GPU; eight values each in `out` [16], a HOST
+ * evo_dense_launches: the one or two launches (the result) that evo_dense_bf16 makes with that workspace (mode 3 with row factors: token matrices below 4 GiB), needs no GPU; eight values each in `out` [16], a HOST
  * array: first row, rows, rows of a tile, columns of a tile (tokens, weight rows for mode 3), parts of K, 1 for the persistent kernel, the row behind the last whose
  * sum of squares it stores (at most M rounded up to 256), and the slots of w of the loop that takes its operands in phases (0: the other loop).
  * evo_dense_plan: the first seven of them, out [14], x row-major. */
