@@ -43,7 +43,7 @@ COMPONENTS = {
         "evo_attn_fwd_causal_bf16", "evo_attn_fwd_packed_bf16", "evo_attn_decode_bf16",
     ]),
     "mixers": ("_mixers", ["stream", "window_attn"], ["mixers_common.h"], [
-        "evo_embed_stream", "evo_postnorm_residual", "evo_sum_norm", "evo_closing_parts", "evo_rmsnorm_stream", "evo_gated_norm", "evo_silu_gate", "evo_act_cols",
+        "evo_embed_stream", "evo_postnorm_residual", "evo_sum_norm", "evo_closing_parts", "evo_closing_final", "evo_rmsnorm_stream", "evo_gated_norm", "evo_silu_gate", "evo_act_cols",
         "evo_window_attn",
     ]),
     "lightning": ("_lightning", ["lightning"], ["mixers_common.h"], ["evo_lightning_chunk_bf16", "evo_lightning_recurrent"]),

@@ -18,6 +18,24 @@
         return evo_launch_status();                                                                                        \
     } while (0)
 
+// The same for kernels of one workgroup a row: rows of whole runs of eight a thread (2,048, 4,096 and 8,192 elements) have forms without a condition
+#define ROW_DISPATCH(KERNEL, VECOK, D_, GRID, ...)                                                                          \
+    do {                                                                                                                   \
+        const dim3 g_(GRID), b_(256);                                                                                      \
+        hipStream_t s_ = (hipStream_t)stream;                                                                              \
+        const int runs_ = (VECOK) ? ((D_) == 2048 ? 1 : (D_) == 4096 ? 2 : (D_) == 8192 ? 4 : 0) : -1;                     \
+        if (f32) { ROW_LAUNCH(KERNEL, float, __VA_ARGS__); } else { ROW_LAUNCH(KERNEL, uint16_t, __VA_ARGS__); }           \
+        return evo_launch_status();                                                                                        \
+    } while (0)
+#define ROW_LAUNCH(KERNEL, T, ...)                                                                                         \
+    switch (runs_) {                                                                                                       \
+        case 1: hipLaunchKernelGGL((KERNEL<T, 8, 1>), g_, b_, 0, s_, __VA_ARGS__); break;                                  \
+        case 2: hipLaunchKernelGGL((KERNEL<T, 8, 2>), g_, b_, 0, s_, __VA_ARGS__); break;                                  \
+        case 4: hipLaunchKernelGGL((KERNEL<T, 8, 4>), g_, b_, 0, s_, __VA_ARGS__); break;                                  \
+        case 0: hipLaunchKernelGGL((KERNEL<T, 8, 0>), g_, b_, 0, s_, __VA_ARGS__); break;                                  \
+        default: hipLaunchKernelGGL((KERNEL<T, 1, 0>), g_, b_, 0, s_, __VA_ARGS__);                                        \
+    }
+
 // ---------------------------------------------------------------------------------------------- embedding
 // x = scale * w[id]; an id outside the table gives a zero row and raises *bad_flag
 template <typename T, int V>
@@ -50,29 +68,82 @@ extern "C" int evo_embed_stream(const int64_t* ids, const void* w, float* x, voi
 // y stays in registers between the two passes (rows up to 4,096 elements); x is written in fp32 and, for the next sublayer's matrix
 // product, once more in bf16.
 // PARTS: y is the sum of `parts` fp32 planes [gridDim.x, D] one behind the other, added in their order and rounded to bf16 (what evo_linear_small_m_bf16 stores).
-template <typename T, int V, bool SUM, bool PARTS = false>
-__device__ __forceinline__ void closing_norm(const void* __restrict__ y_, const void* __restrict__ w_, float* __restrict__ x,
-                                             uint16_t* __restrict__ xb, int D, float alpha, float eps, float off, int parts = 0) {
-    constexpr int KEEP = V == 8 ? 2 : 4;                         // runs of V elements a thread keeps in registers (D <= 256 V KEEP)
-    __shared__ float red[4];
+//
+// RUNS > 0: the row is exactly RUNS runs of V elements a thread.  Everything a row needs -- y or its parts four at a time, x, the norm's weight -- is then requested
+// together, without a condition among the requests.  A decode step's launch is a chain of latencies: with the weight (cold: a whole step's weights went by since) and x
+// asked for behind the reduction there were two of them: rows of 4,096 in a step of four layers 3.5 -> 2.8 us at 8 rows, on the parts of 24 rows 5.2 -> 3.8, the gated norm
+// 3.9 -> 2.4 (an empty launch is 1.6).
+template <typename T, int V, bool PARTS>
+__device__ __forceinline__ void closing_load(const void* __restrict__ y_, int64_t row, int c, int D, int parts, float* f) {
+    if constexpr (PARTS) {
+        const float* p = (const float*)y_ + row * D + c;
+        const int64_t plane = (int64_t)gridDim.x * D;
+        vec_io<float, V>::load(p, f);
+        for (int s = 1; s < parts; s += 3) {                     // (three requests at once; a plane behind the last is the last again, and not added)
+            float q[3][V];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) vec_io<float, V>::load(p + (s + k < parts ? s + k : parts - 1) * plane, q[k]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+#pragma unroll
+                for (int e = 0; e < V; ++e) f[e] = s + k < parts ? f[e] + q[k][e] : f[e];
+        }
+#pragma unroll
+        for (int e = 0; e < V; ++e) f[e] = bf_to_f(f_to_bf(f[e]));
+    } else vec_io<T, V>::load((const T*)y_ + row * D + c, f);
+}
+
+template <typename T, int V, bool SUM, bool PARTS, int RUNS>
+__device__ __forceinline__ void closing_row(const void* __restrict__ y_, const void* __restrict__ w_, const float* __restrict__ x, int D, float alpha, float eps, float off,
+                                            int parts, float* red, float (&r)[RUNS][V]) {   // -> the row's new x in r
     const T* w = (const T*)w_;
     const int64_t row = blockIdx.x;
-    const T* y = (const T*)y_ + row * D;
+    float f[RUNS][V], g[RUNS][V];
+#pragma unroll
+    for (int i = 0; i < RUNS; ++i) {
+        const int c = (threadIdx.x + 256 * i) * V;
+        vec_io<float, V>::load(x + row * D + c, r[i]);
+        vec_io<T, V>::load(w + c, g[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < RUNS; ++i) closing_load<T, V, PARTS>(y_, row, (threadIdx.x + 256 * i) * V, D, parts, f[i]);
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < RUNS; ++i)
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            if (SUM) f[i][e] = fmaf(alpha, r[i][e], f[i][e]);
+            ss = fmaf(f[i][e], f[i][e], ss);
+        }
+    const float inv = 1.0f / sqrtf(block_sum_256(ss, red) / (float)D + eps);
+#pragma unroll
+    for (int i = 0; i < RUNS; ++i)
+#pragma unroll
+        for (int e = 0; e < V; ++e) r[i][e] = SUM ? f[i][e] * inv * (off + g[i][e]) : fmaf(f[i][e] * inv, off + g[i][e], r[i][e]);
+}
+
+template <typename T, int V, bool SUM, bool PARTS = false, int RUNS = 0>
+__device__ __forceinline__ void closing_norm(const void* __restrict__ y_, const void* __restrict__ w_, float* __restrict__ x,
+                                             uint16_t* __restrict__ xb, int D, float alpha, float eps, float off, int parts = 0) {
+    __shared__ float red[4];
+    const int64_t row = blockIdx.x;
+    if constexpr (RUNS > 0) {
+        float r[RUNS][V];
+        closing_row<T, V, SUM, PARTS, RUNS>(y_, w_, x, D, alpha, eps, off, parts, red, r);
+#pragma unroll
+        for (int i = 0; i < RUNS; ++i) {
+            const int c = (threadIdx.x + 256 * i) * V;
+            vec_io<float, V>::store(x + row * D + c, r[i]);
+            if (xb) vec_io<uint16_t, V>::store(xb + row * D + c, r[i]);
+        }
+        return;
+    }
+    constexpr int KEEP = V == 8 ? 2 : 4;                         // runs of V elements a thread keeps in registers (D <= 256 V KEEP)
+    const T* w = (const T*)w_;
     float keep[KEEP][V];
     float ss = 0.f;
     auto load = [&](int c, float* f) {
-        if constexpr (PARTS) {
-            const float* p = (const float*)y_ + row * D + c;
-            vec_io<float, V>::load(p, f);
-            for (int s = 1; s < parts; ++s) {
-                float q[V];
-                vec_io<float, V>::load(p + s * ((int64_t)gridDim.x * D), q);
-#pragma unroll
-                for (int e = 0; e < V; ++e) f[e] += q[e];
-            }
-#pragma unroll
-            for (int e = 0; e < V; ++e) f[e] = bf_to_f(f_to_bf(f[e]));
-        } else vec_io<T, V>::load(y + c, f);
+        closing_load<T, V, PARTS>(y_, row, c, D, parts, f);
         if constexpr (SUM) {
             float r[V];
             vec_io<float, V>::load(x + row * D + c, r);
@@ -117,36 +188,36 @@ __device__ __forceinline__ void closing_norm(const void* __restrict__ y_, const 
     }
 }
 
-template <typename T, int V>
+template <typename T, int V, int RUNS>
 __global__ __launch_bounds__(256) void postnorm_residual_kernel(const void* __restrict__ y, const void* __restrict__ w, float* __restrict__ x,
                                                                 uint16_t* __restrict__ xb, int D, float eps, float off) {
-    closing_norm<T, V, false>(y, w, x, xb, D, 1.f, eps, off);
+    closing_norm<T, V, false, false, RUNS>(y, w, x, xb, D, 1.f, eps, off);
 }
-template <typename T, int V>
+template <typename T, int V, int RUNS>
 __global__ __launch_bounds__(256) void sum_norm_kernel(const void* __restrict__ y, const void* __restrict__ w, float* __restrict__ x,
                                                        uint16_t* __restrict__ xb, int D, float alpha, float eps, float off) {
-    closing_norm<T, V, true>(y, w, x, xb, D, alpha, eps, off);
+    closing_norm<T, V, true, false, RUNS>(y, w, x, xb, D, alpha, eps, off);
 }
 
 extern "C" int evo_postnorm_residual(const void* y, const void* w, float* x, void* xb, int64_t M, int64_t D, float eps, float w_offset,
                                      int64_t f32, void* stream) {
     if (M < 0 || M > 0x7fffffff || D <= 0 || D > 0x3fffffff) return -1;
     if (M == 0) return 0;
-    STREAM_DISPATCH(postnorm_residual_kernel, D % 8 == 0, (unsigned)M, y, w, x, (uint16_t*)xb, (int)D, eps, w_offset);
+    ROW_DISPATCH(postnorm_residual_kernel, D % 8 == 0, D, (unsigned)M, y, w, x, (uint16_t*)xb, (int)D, eps, w_offset);
 }
 
 extern "C" int evo_sum_norm(const void* y, const void* w, float* x, void* xb, int64_t M, int64_t D, float alpha, float eps, float w_offset,
                             int64_t f32, void* stream) {
     if (!y || !w || !x || M < 0 || M > 0x7fffffff || D <= 0 || D > 0x3fffffff) return -1;
     if (M == 0) return 0;
-    STREAM_DISPATCH(sum_norm_kernel, D % 8 == 0, (unsigned)M, y, w, x, (uint16_t*)xb, (int)D, alpha, eps, w_offset);
+    ROW_DISPATCH(sum_norm_kernel, D % 8 == 0, D, (unsigned)M, y, w, x, (uint16_t*)xb, (int)D, alpha, eps, w_offset);
 }
 
 // Both on the parts of a dense layer's sum (evo_linear_parts_bf16): the launch that added and rounded them was 4.7 us of its own, a decode layer of 17 to 64 rows.
-template <bool SUM>
+template <bool SUM, int RUNS>
 __global__ __launch_bounds__(256) void closing_parts_kernel(const float* __restrict__ y, const void* __restrict__ w, float* __restrict__ x, uint16_t* __restrict__ xb, int D,
                                                             float alpha, float eps, float off, int parts) {
-    closing_norm<uint16_t, 8, SUM, true>(y, w, x, xb, D, alpha, eps, off, parts);
+    closing_norm<uint16_t, 8, SUM, true, RUNS>(y, w, x, xb, D, alpha, eps, off, parts);
 }
 
 extern "C" int evo_closing_parts(const float* y, int64_t parts, const void* w, float* x, void* xb, int64_t M, int64_t D, int64_t sum, float alpha, float eps, float w_offset,
@@ -154,13 +225,17 @@ extern "C" int evo_closing_parts(const float* y, int64_t parts, const void* w, f
     if (!y || !w || !x || !xb || parts < 1 || parts > 64 || M < 0 || M > 0x7fffffff || D <= 0 || D > 0x3fffffff || D % 8 != 0) return -1;
     if (((uintptr_t)y | (uintptr_t)w | (uintptr_t)x | (uintptr_t)xb) & 15) return -1;
     if (M == 0) return 0;
-    if (sum) hipLaunchKernelGGL(closing_parts_kernel<true>, dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream, y, w, x, (uint16_t*)xb, (int)D, alpha, eps, w_offset, (int)parts);
-    else hipLaunchKernelGGL(closing_parts_kernel<false>, dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream, y, w, x, (uint16_t*)xb, (int)D, 1.f, eps, w_offset, (int)parts);
+#define CP(SUM, RUNS) hipLaunchKernelGGL((closing_parts_kernel<SUM, RUNS>), dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream, y, w, x, (uint16_t*)xb, (int)D,   \
+                                         sum ? alpha : 1.f, eps, w_offset, (int)parts)
+    if (D == 4096) { if (sum) CP(true, 2); else CP(false, 2); }
+    else if (sum) CP(true, 0); else CP(false, 0);
+#undef CP
     return evo_launch_status();
 }
 
 // ---------------------------------------------------------------------------------------------- out = norm(x) * (off + w), x the stream
-template <typename T, int V>
+// RUNS: as in closing_norm
+template <typename T, int V, int RUNS>
 __global__ __launch_bounds__(256) void rmsnorm_stream_kernel(const float* __restrict__ x_, const void* __restrict__ w_, void* __restrict__ out_, int D,
                                                              float eps, float off) {
     __shared__ float red[4];
@@ -169,6 +244,27 @@ __global__ __launch_bounds__(256) void rmsnorm_stream_kernel(const float* __rest
     const float* x = x_ + row * D;
     T* out = (T*)out_ + row * D;
     float ss = 0.f;
+    if constexpr (RUNS > 0) {
+        float f[RUNS][V], g[RUNS][V];
+#pragma unroll
+        for (int i = 0; i < RUNS; ++i) {
+            const int c = (threadIdx.x + 256 * i) * V;
+            vec_io<float, V>::load(x + c, f[i]);
+            vec_io<T, V>::load(w + c, g[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < RUNS; ++i)
+#pragma unroll
+            for (int e = 0; e < V; ++e) ss = fmaf(f[i][e], f[i][e], ss);
+        const float inv = 1.0f / sqrtf(block_sum_256(ss, red) / (float)D + eps);
+#pragma unroll
+        for (int i = 0; i < RUNS; ++i) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) f[i][e] = f[i][e] * inv * (off + g[i][e]);
+            vec_io<T, V>::store(out + (threadIdx.x + 256 * i) * V, f[i]);
+        }
+        return;
+    }
     for (int c = threadIdx.x * V; c < D; c += 256 * V) {
         float f[V];
         vec_io<float, V>::load(x + c, f);
@@ -190,11 +286,55 @@ extern "C" int evo_rmsnorm_stream(const float* x, const void* w, void* out, int6
                                   void* stream) {
     if (M < 0 || M > 0x7fffffff || D <= 0 || D > 0x3fffffff) return -1;
     if (M == 0) return 0;
-    STREAM_DISPATCH(rmsnorm_stream_kernel, D % 8 == 0, (unsigned)M, x, w, out, (int)D, eps, w_offset);
+    ROW_DISPATCH(rmsnorm_stream_kernel, D % 8 == 0, D, (unsigned)M, x, w, out, (int)D, eps, w_offset);
+}
+
+// ---------------------------------------------------------------------------------------------- the last closing norm and the final one
+// out = norm(x') * (off + wf) of the x' that a closing norm makes, which nothing reads any more: neither it nor its copy is stored.  The same bits as the two launches.
+template <typename T, bool SUM, bool PARTS, int RUNS>
+__global__ __launch_bounds__(256) void closing_final_kernel(const void* __restrict__ y, const void* __restrict__ w, const float* __restrict__ x, const void* __restrict__ wf_,
+                                                            void* __restrict__ out_, int D, float alpha, float eps, float off, int parts) {
+    constexpr int V = 8;
+    __shared__ float red[4], red2[4];
+    const T* wf = (const T*)wf_;
+    T* out = (T*)out_ + (int64_t)blockIdx.x * D;
+    float g[RUNS][V], r[RUNS][V], ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < RUNS; ++i) vec_io<T, V>::load(wf + (threadIdx.x + 256 * i) * V, g[i]);
+    closing_row<T, V, SUM, PARTS, RUNS>(y, w, x, D, alpha, eps, off, parts, red, r);
+#pragma unroll
+    for (int i = 0; i < RUNS; ++i)
+#pragma unroll
+        for (int e = 0; e < V; ++e) ss = fmaf(r[i][e], r[i][e], ss);
+    const float inv = 1.0f / sqrtf(block_sum_256(ss, red2) / (float)D + eps);
+#pragma unroll
+    for (int i = 0; i < RUNS; ++i) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) r[i][e] = r[i][e] * inv * (off + g[i][e]);
+        vec_io<T, V>::store(out + (threadIdx.x + 256 * i) * V, r[i]);
+    }
+}
+
+extern "C" int evo_closing_final(const void* y, int64_t parts, const void* w, const float* x, const void* wf, void* out, int64_t M, int64_t D, int64_t sum, float alpha, float eps,
+                                 float w_offset, int64_t f32, void* stream) {
+    if (!y || !w || !x || !wf || !out || parts < 0 || parts > 64 || M < 0 || M > 0x7fffffff || (D != 2048 && D != 4096 && D != 8192)) return -1;
+    if (parts && (f32 || D != 4096)) return -1;
+    if (((uintptr_t)y | (uintptr_t)w | (uintptr_t)x | (uintptr_t)wf | (uintptr_t)out) & 15) return -1;
+    if (M == 0) return 0;
+#define CF(T, SUM, PARTS, RUNS) hipLaunchKernelGGL((closing_final_kernel<T, SUM, PARTS, RUNS>), dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream, y, w, x, wf, out, (int)D, \
+                                                   alpha, eps, w_offset, (int)parts)
+#define CF_RUNS(T, SUM) do { if (D == 2048) CF(T, SUM, false, 1); else if (D == 4096) CF(T, SUM, false, 2); else CF(T, SUM, false, 4); } while (0)
+    if (parts) { if (sum) CF(uint16_t, true, true, 2); else CF(uint16_t, false, true, 2); }
+    else if (f32) { if (sum) CF_RUNS(float, true); else CF_RUNS(float, false); }
+    else if (sum) CF_RUNS(uint16_t, true); else CF_RUNS(uint16_t, false);
+#undef CF_RUNS
+#undef CF
+    return evo_launch_status();
 }
 
 // ---------------------------------------------------------------------------------------------- out = norm(o) * w * sigmoid(g)
-template <typename T, int V>
+// RUNS: as in closing_norm
+template <typename T, int V, int RUNS>
 __global__ __launch_bounds__(256) void gated_norm_kernel(const void* __restrict__ o_, const void* __restrict__ g_, int64_t ldg,
                                                          const void* __restrict__ w_, void* __restrict__ out_, int D, float eps) {
     constexpr int KEEP = V == 8 ? 2 : 4;
@@ -204,6 +344,28 @@ __global__ __launch_bounds__(256) void gated_norm_kernel(const void* __restrict_
     const T* o = (const T*)o_ + row * D;
     const T* g = (const T*)g_ + row * ldg;
     T* out = (T*)out_ + row * D;
+    if constexpr (RUNS > 0) {
+        float f[RUNS][V], gg[RUNS][V], ww[RUNS][V], ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < RUNS; ++i) {
+            const int c = (threadIdx.x + 256 * i) * V;
+            vec_io<T, V>::load(o + c, f[i]);
+            vec_io<T, V>::load(g + c, gg[i]);
+            vec_io<T, V>::load(w + c, ww[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < RUNS; ++i)
+#pragma unroll
+            for (int e = 0; e < V; ++e) ss = fmaf(f[i][e], f[i][e], ss);
+        const float inv = 1.0f / sqrtf(block_sum_256(ss, red) / (float)D + eps);
+#pragma unroll
+        for (int i = 0; i < RUNS; ++i) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) f[i][e] = f[i][e] * inv * ww[i][e] * sigmoid_t<T>(gg[i][e]);
+            vec_io<T, V>::store(out + (threadIdx.x + 256 * i) * V, f[i]);
+        }
+        return;
+    }
     float keep[KEEP][V];
     float ss = 0.f;
 #pragma unroll
@@ -247,7 +409,7 @@ extern "C" int evo_gated_norm(const void* o, const void* g, int64_t ldg, const v
     if (M < 0 || M > 0x7fffffff || D <= 0 || D > 0x3fffffff || ldg < D) return -1;
     if (M == 0) return 0;
     const bool vec = D % 8 == 0 && ldg % 8 == 0 && ((uintptr_t)g & 15) == 0;
-    STREAM_DISPATCH(gated_norm_kernel, vec, (unsigned)M, o, g, ldg, w, out, (int)D, eps);
+    ROW_DISPATCH(gated_norm_kernel, vec, D, (unsigned)M, o, g, ldg, w, out, (int)D, eps);
 }
 
 // ---------------------------------------------------------------------------------------------- a = silu(z[:, :I]) * z[:, I:]

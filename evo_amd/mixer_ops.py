@@ -44,8 +44,9 @@ class TokenBatch:
 
 
 class Stream:
-    """The fp32 residual stream x [M, D] of one pass, its storage-type copy, and at most one sublayer output that has not been added yet: for a
-    few rows of bf16 the next layer's launch adds it (ops.postnorm_linear / postnorm_gate), otherwise it is added at once.
+    """The fp32 residual stream x [M, D] of one pass, its storage-type copy, and at most one sublayer output that has not been added yet: for one
+    row of bf16 the next layer's launch adds it (ops.postnorm_linear / postnorm_gate), the last of a pass the final norm's (ops.closing_final),
+    otherwise it is added before the next layer.
 
     The norm of a sublayer's output y comes before the addition, x <- x + norm(y), or -- with `alpha` -- behind it, x <- norm(alpha x + y);
     norm(t) = t / rms(t) * (w_offset + w)."""
@@ -64,18 +65,20 @@ class Stream:
 
     def add(self, y: torch.Tensor, w: torch.Tensor) -> None:
         self.flush()
-        if y.dim() == 3:                                         # (parts)
-            self.ops.closing_parts_(self.x, self.xb, y, w, self.alpha, self.eps, self.w_offset)
-            self.behind = False
-            return
         self.open = (y, w)
-        if not self.ops.fuse_postnorm_ok(y):
-            self.flush()
+
+    def _next_adds(self) -> bool:
+        """Whether the next layer's launch adds the open output."""
+        return self.open is not None and self.open[0].dim() == 2 and self.ops.fuse_postnorm_ok(self.open[0])
 
     def flush(self) -> None:
         if self.open is not None:
             y, w = self.open
             self.open = None
+            if y.dim() == 3:                                     # (parts)
+                self.ops.closing_parts_(self.x, self.xb, y, w, self.alpha, self.eps, self.w_offset)
+                self.behind = False
+                return
             if self.xb.dtype == self.x.dtype:
                 self.xb = self.x
             if self.alpha is None:
@@ -101,16 +104,20 @@ class Stream:
         return y, w, old, new
 
     def linear(self, w: torch.Tensor, act: Optional[str] = None) -> torch.Tensor:
-        if self.open is None:
+        if not self._next_adds():
             return self.ops.linear(self.input(), w) if act is None else self.ops.linear_act(self.input(), w, act, w.shape[0])
         return self.ops.postnorm_linear(*self._swap(), w, self.eps, self.w_offset, alpha=self.alpha, act=act)
 
     def gate(self, w12: torch.Tensor, grouped: bool, act: str) -> torch.Tensor:
-        if self.open is None:
+        if not self._next_adds():
             return self.ops.mlp_gate(self.input(), None if grouped else w12, w12g=w12 if grouped else None, act=act)
         return self.ops.postnorm_gate(*self._swap(), w12, grouped, act, self.eps, self.w_offset, alpha=self.alpha)
 
     def final(self, w: torch.Tensor) -> torch.Tensor:
+        """The final norm; nothing reads the stream behind it."""
+        if self.open is not None and hasattr(self.ops, "closing_final_ok") and self.ops.closing_final_ok(*self.open, self.x, w):
+            (y, g), self.open = self.open, None
+            return self.ops.closing_final(self.x, y, g, w, self.alpha, self.eps, self.w_offset)
         self.flush()
         return self.ops.rmsnorm_stream(self.x, w, self.eps, self.w_offset)
 
@@ -240,6 +247,24 @@ class MixerOps:
         assert x.dtype == torch.float32 and x.is_cuda
         out = torch.empty(M, D, dtype=w.dtype, device=x.device)
         self._call("evo_rmsnorm_stream", x.data_ptr(), w.data_ptr(), out.data_ptr(), M, D, float(eps), float(w_offset), f32)
+        return out
+
+    def closing_final_ok(self, y: torch.Tensor, w: torch.Tensor, x: torch.Tensor, wf: torch.Tensor) -> bool:
+        """Rows that closing_final's kernel holds in registers."""
+        D = x.shape[1]
+        return (D in (2048, 4096, 8192) and (y.dim() == 2 or D == 4096) and w.dtype == wf.dtype and w.is_contiguous() and wf.is_contiguous()
+                and (y.data_ptr() | w.data_ptr() | x.data_ptr() | wf.data_ptr()) % 16 == 0)
+
+    def closing_final(self, x: torch.Tensor, y: torch.Tensor, w: torch.Tensor, wf: torch.Tensor, alpha: Optional[float], eps: float, w_offset: float) -> torch.Tensor:
+        """rmsnorm_stream(x', wf) of the x' that postnorm_residual_, sum_norm_ or closing_parts_ (y of three dimensions) would store; x itself stays."""
+        parts = y.shape[0] if y.dim() == 3 else 0
+        f32 = self._store(w, wf) if parts else self._store(y, w, wf)
+        M, D = x.shape
+        self._dense(y, ((parts,) if parts else ()) + (M, D), "y"), self._dense(x, (M, D), "x"), self._dense(w, (D,), "w"), self._dense(wf, (D,), "wf")
+        assert x.dtype == torch.float32 and x.is_cuda and (not parts or (y.dtype == torch.float32 and y.is_cuda))
+        out = torch.empty(M, D, dtype=w.dtype, device=x.device)
+        self._call("evo_closing_final", y.data_ptr(), parts, w.data_ptr(), x.data_ptr(), wf.data_ptr(), out.data_ptr(), M, D, int(alpha is not None), float(alpha or 0.0),
+                   float(eps), float(w_offset), f32)
         return out
 
     def gated_norm(self, o: torch.Tensor, g: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:

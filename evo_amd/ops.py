@@ -88,6 +88,7 @@ _SIGNATURES = {
     "evo_linear_ring_share": ([_I64] * 3 + [_PTR], _c.c_int),
     "evo_linear_parts": ([_I64] * 3, _c.c_int),
     "evo_linear_parts_bf16": ([_PTR] * 3 + [_I64] * 4 + [_PTR], _c.c_int),
+    "evo_closing_final": ([_PTR, _I64] + [_PTR] * 4 + [_I64] * 3 + [_F32] * 3 + [_I64, _PTR], _c.c_int),
     "evo_closing_parts": ([_PTR, _I64] + [_PTR] * 3 + [_I64] * 3 + [_F32] * 3 + [_PTR], _c.c_int),
     "evo_sum_norm": ([_PTR] * 4 + [_I64] * 2 + [_F32] * 3 + [_I64, _PTR], _c.c_int),
     "evo_act_cols": ([_PTR] + [_I64] * 5 + [_PTR], _c.c_int),
@@ -108,7 +109,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 26         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 27         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):

@@ -67,8 +67,9 @@ extern "C" {
  *  23: evo_attn_fwd_packed_bf16 gained `form`.
  *  24: evo_linear_f32_ahead and evo_linear_f32_ahead_plan added.
  *  25: evo_linear_few_f32 added.
- *  26: evo_dense_launches added. */
-#define EVO_ABI_VERSION 26
+ *  26: evo_dense_launches added.
+ *  27: evo_closing_final added. */
+#define EVO_ABI_VERSION 27
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
@@ -486,6 +487,11 @@ int evo_sum_norm(const void* y, const void* w, float* x, void* xb, int64_t M, in
  * evo_linear_small_m_bf16 in front of them.  bf16 weights and xb, D % 8 == 0, everything 16-byte aligned. */
 int evo_closing_parts(const float* y, int64_t parts, const void* w, float* x, void* xb, int64_t M, int64_t D, int64_t sum, float alpha, float eps, float w_offset,
                       void* stream);
+/* out = x' / sqrt(mean(x'^2) + eps) * (w_offset + wf) of the x' that evo_sum_norm (`sum`) or evo_postnorm_residual would store, or, with `parts` > 0, evo_closing_parts (y its
+ * fp32 planes): the last closing norm and the final norm, in one launch and with the bits of two; x is not written.  D 2,048, 4,096 or 8,192 (parts: 4,096 and bf16),
+ * everything 16-byte aligned. */
+int evo_closing_final(const void* y, int64_t parts, const void* w, const float* x, const void* wf, void* out, int64_t M, int64_t D, int64_t sum, float alpha, float eps,
+                      float w_offset, int64_t f32, void* stream);
 /* out = x / sqrt(mean(x^2) + eps) * (w_offset + w) */
 int evo_rmsnorm_stream(const float* x, const void* w, void* out, int64_t M, int64_t D, float eps, float w_offset, int64_t f32, void* stream);
 /* out = o / sqrt(mean(o^2) + eps) * w * sigmoid(g); g rows have pitch ldg. */

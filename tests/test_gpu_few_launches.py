@@ -36,6 +36,62 @@ def test_closing_norm_of_parts(ops, M, N, K, alpha):
         assert torch.equal(x, x2) and torch.equal(xb, xb2)
 
 
+@pytest.mark.parametrize("M,D,dtype", [(1, 2048, BF), (3, 4096, torch.float32), (5, 4096, BF), (2, 8192, torch.float32), (300, 8192, BF)])
+@pytest.mark.parametrize("alpha", [None, 2.0])
+def test_last_closing_norm_with_the_final_one(ops, M, D, dtype, alpha):
+    """The same bits as the closing norm and the final norm in launches of their own; the stream stays as it was."""
+    x, y, g, wf = (rnd(*s, seed=i).to(DEV, t) for i, (s, t) in enumerate((((M, D), torch.float32), ((M, D), dtype), ((D,), dtype), ((D,), dtype))))
+    was = x.clone()
+    assert ops.closing_final_ok(y, g, x, wf)
+    got = ops.closing_final(x, y, g, wf, alpha, 1e-6, 1.0)
+    assert torch.equal(x, was)
+    xb = x if dtype == torch.float32 else torch.zeros(M, D, device=DEV, dtype=BF)
+    if alpha is None:
+        ops.postnorm_residual_(x, xb, y, g, 1e-6, 1.0)
+    else:
+        ops.sum_norm_(x, xb, y, g, alpha, 1e-6, 1.0)
+    assert torch.equal(got, ops.rmsnorm_stream(x, wf, 1e-6, 1.0))
+    assert not ops.closing_final_ok(y[:, 8:].contiguous(), g[8:], x[:, 8:].contiguous(), wf[8:])
+    parts = rnd(7, M, 4096, seed=9).to(DEV)
+    x, xb, g, wf = (t[..., :4096].contiguous() if t.shape[-1] > 4096 else torch.nn.functional.pad(t, (0, 4096 - t.shape[-1])) for t in (was, xb.to(BF), g.to(BF), wf.to(BF)))
+    for n in (1, 2, 3, 4, 7):
+        x2, xb2 = x.clone(), torch.zeros_like(xb)
+        got = ops.closing_final(x, parts[:n], g, wf, alpha, 1e-6, 1.0)
+        ops.closing_parts_(x2, xb2, parts[:n], g, alpha, 1e-6, 1.0)
+        assert torch.equal(got, ops.rmsnorm_stream(x2, wf, 1e-6, 1.0))
+
+
+@pytest.mark.parametrize("D", [2048, 4096, 8192])
+@pytest.mark.parametrize("dtype", [BF, torch.float32])
+def test_rows_of_whole_runs(ops, D, dtype):
+    """Rows that a thread requests whole against rows that it walks: D elements with a zero behind every other one are 2 D elements of half the mean square, in the order of
+    the walk.  The runs are other threads', so sums differ by their order: at most D additions of 2^-24, in a root, and bf16's rounding on top."""
+    M = 5
+    x, y, g = (rnd(*s, seed=i).to(DEV, t) for i, (s, t) in enumerate((((M, D), torch.float32), ((M, D), dtype), ((D,), dtype))))
+    tol = D * 2.0 ** -24 + (2.0 ** -8 if dtype == BF else 0.0)
+
+    def wide(t):
+        return torch.nn.functional.pad(t, (0, 3 * D))
+    for alpha in (None, 2.0):
+        a, b = x.clone(), wide(x)
+        ab, bb = (a, b) if dtype == torch.float32 else (torch.zeros_like(y), torch.zeros_like(wide(y)))
+        if alpha is None:
+            ops.postnorm_residual_(a, ab, y, g, 1e-6, 1.0)
+            ops.postnorm_residual_(b, bb, wide(y), wide(g), 1e-6 / 4, 1.0)
+            want = x.double() + (b[:, :D].double() - x.double()) / 2             # (a mean over four times the elements)
+        else:
+            ops.sum_norm_(a, ab, y, g, alpha, 1e-6, 1.0)
+            ops.sum_norm_(b, bb, wide(y), wide(g), alpha, 1e-6 / 4, 1.0)
+            want = b[:, :D].double() / 2
+        assert ((a.double() - want).abs() <= 8 * D * 2.0 ** -24 * (want.abs() + x.double().abs())).all()
+        assert torch.equal(ab, a.to(dtype))
+    n, nw = ops.rmsnorm_stream(x, g, 1e-6, 1.0), ops.rmsnorm_stream(wide(x), wide(g), 1e-6 / 4, 1.0)[:, :D]
+    assert ((n.double() - nw.double() / 2).abs() <= 2 * tol * n.double().abs() + 1e-30).all()
+    z = rnd(M, D, seed=7).to(DEV, dtype)
+    n, nw = ops.gated_norm(y, z, g, 1e-6), ops.gated_norm(wide(y), wide(z), wide(g), 1e-6 / 4)[:, :D]
+    assert ((n.double() - nw.double() / 2).abs() <= 2 * tol * n.double().abs() + 1e-30).all()
+
+
 def test_one_sum_stays_one_sum(ops):
     for M, N, K in ((16, 4096, 16384), (24, 4096, 4096), (65, 4096, 16384), (24, 4160, 16384), (24, 4096, 16416), (24, 512, 16384)):
         assert ops.linear_parts(torch.zeros(M, K, device=DEV, dtype=BF), torch.zeros(N, K, device=DEV, dtype=BF)) is None
