@@ -814,7 +814,10 @@ __global__ __launch_bounds__(256) void attn_decode_stream_kernel(AttnArgs a, int
 // 512 threads = 4 groups x 128 output dims; the statistics are read once into LDS (coalesced) and turned into weights, then
 // group g sums splits g, g + 4, ... with eight independent row loads in flight (the first version walked the splits one
 // dependent L2 round trip at a time: 7 us at 16 splits, ~30 us at the 64 the streaming kernel uses).
+// FEW: up to 31 splits.  A thread's rows -- at most eight, one latency each in the loop for what eight at a time leave over -- are then asked for with the statistics, before
+// the weights are known (16 / 20 splits 15.5 -> 14.8 and 40.8 -> 40.3 us with the streaming kernel at 2 x 1,000 and 16 x 700 keys; 32 splits 16.5 : 16.7, which stay).
 #define ATTN_MAX_SPLITS 1024
+template <bool FEW>
 __global__ __launch_bounds__(512) void attn_decode_combine_kernel(const float* __restrict__ part_o,
                                                                   const float* __restrict__ part_ml,
                                                                   uint16_t* __restrict__ o, int H, int n_splits) {
@@ -823,6 +826,11 @@ __global__ __launch_bounds__(512) void attn_decode_combine_kernel(const float* _
     __shared__ float acc_s[4][DH];
     const int tid = threadIdx.x, d = tid & (DH - 1), g = tid >> 7, head = blockIdx.x, bat = blockIdx.y;
     const int64_t base = ((int64_t)bat * H + head) * n_splits;
+    float r[8];
+    if constexpr (FEW) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) r[u] = part_o[(base + (g + 4 * u < n_splits ? g + 4 * u : n_splits - 1)) * DH + d];
+    }
     // pass 1: maxima
     float M = -INFINITY;
     for (int s = tid; s < n_splits; s += 512) M = fmaxf(M, part_ml[(base + s) * 2]);
@@ -848,15 +856,19 @@ __global__ __launch_bounds__(512) void attn_decode_combine_kernel(const float* _
     for (int i = 0; i < 8; ++i) L += red[8 + i];
     // pass 3: weighted rows
     float acc = 0.f;
-    int s = g;
-    for (; s + 28 < n_splits; s += 32) {
-        float r[8];
+    if constexpr (FEW) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) r[u] = part_o[(base + s + 4 * u) * DH + d];
+        for (int u = 0; u < 8; ++u) acc = g + 4 * u < n_splits ? fmaf(r[u], w_s[g + 4 * u], acc) : acc;
+    } else {
+        int s = g;
+        for (; s + 28 < n_splits; s += 32) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) acc = fmaf(r[u], w_s[s + 4 * u], acc);
+            for (int u = 0; u < 8; ++u) r[u] = part_o[(base + s + 4 * u) * DH + d];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) acc = fmaf(r[u], w_s[s + 4 * u], acc);
+        }
+        for (; s < n_splits; s += 4) acc = fmaf(part_o[(base + s) * DH + d], w_s[s], acc);
     }
-    for (; s < n_splits; s += 4) acc = fmaf(part_o[(base + s) * DH + d], w_s[s], acc);
     acc_s[g][d] = acc;
     __syncthreads();
     if (g == 0) {
@@ -972,7 +984,9 @@ extern "C" int evo_attn_decode_bf16(const void* q, const void* k, const void* v,
     }
     else
         hipLaunchKernelGGL(attn_fwd_kernel<true>, dim3((unsigned)n_splits, (unsigned)H, (unsigned)B), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(attn_decode_combine_kernel, dim3((unsigned)H, (unsigned)B), dim3(512), 0, s, part_o, part_ml,
-                       (uint16_t*)o, (int)H, (int)n_splits);
+    if (n_splits < 32)
+        hipLaunchKernelGGL(attn_decode_combine_kernel<true>, dim3((unsigned)H, (unsigned)B), dim3(512), 0, s, part_o, part_ml, (uint16_t*)o, (int)H, (int)n_splits);
+    else
+        hipLaunchKernelGGL(attn_decode_combine_kernel<false>, dim3((unsigned)H, (unsigned)B), dim3(512), 0, s, part_o, part_ml, (uint16_t*)o, (int)H, (int)n_splits);
     return evo_launch_status();
 }

@@ -43,46 +43,53 @@ __device__ __forceinline__ void fill_turns(float2* turn, const HeadsArgs& a, int
 }
 
 // LG lanes per vector, 16 elements each: a run of eight and its partners half a rotation further, or two runs that are not rotated.
-// n_rot % 16 == 0, dim % 8 == 0, 16-byte aligned rows.
+// n_rot % 16 == 0, dim % 8 == 0, 16-byte aligned rows.  What a thread's first vector needs, its norm's weight and its values are asked for before the angles, and few
+// tokens' vectors are shared out over gridDim.y workgroups: a decode step's launch is a chain of latencies (24 tokens of 40 and 64
+// vectors of 128 in a step of four layers 5.5 -> 4.2 us)
 template <typename T, int LG>
 __global__ __launch_bounds__(256) void heads_prep_kernel(HeadsArgs a) {
     extern __shared__ float2 turn[];                             // [n_rot / 2] cosine and sine of this token's angles, times the amplitude
-    const int m = blockIdx.x, tid = threadIdx.x, u = tid % LG;
-    const int64_t pos = a.pos[m];
+    constexpr int PER = 256 / LG;
+    const int m = blockIdx.x, tid = threadIdx.x, u = tid % LG, nh = a.nq + a.nk, h_first = blockIdx.y * PER + tid / LG, step = gridDim.y * PER;
     T* z = (T*)a.z + (int64_t)m * a.ld;
-    T* slot = cache_row<T>(a, m, pos);
     const int half = a.n_rot / 2, rot = a.n_rot / 16;
     const int oa = u < rot ? 8 * u : a.n_rot + 16 * (u - rot), ob = u < rot ? half + 8 * u : oa + 8;
     const bool ha = oa < a.dim, hb = ob < a.dim;                 // (lanes past the vector idle)
+    const int la = ha ? oa : 0, lb = hb ? ob : 0;                // (and read its start)
+    const T* values = z + (int64_t)nh * a.dim;
+    const int vi = (blockIdx.y * 256 + tid) * 8;
+    float x[8], y[8], gx[8], gy[8], val[8];
+    auto fetch = [&](int h) __attribute__((always_inline)) {
+        const T* v = z + (int64_t)(h < nh ? h : nh - 1) * a.dim;
+        vec_io<T, 8>::load(v + la, x);
+        vec_io<T, 8>::load(v + lb, y);
+        if (a.qw) {
+            const T* w = (const T*)(h < a.nq ? a.qw : a.kw);
+            vec_io<T, 8>::load(w + la, gx);
+            vec_io<T, 8>::load(w + lb, gy);
+        }
+    };
+    fetch(h_first);
+    if (vi + 7 < a.nv) vec_io<T, 8>::load(values + vi, val);
+    const int64_t pos = a.pos[m];
+    T* slot = cache_row<T>(a, m, pos);
     fill_turns(turn, a, pos);
     __syncthreads();
-    for (int h = tid / LG; h < a.nq + a.nk; h += 256 / LG) {
+    for (int h = h_first; h < nh; h += step) {
+        if (h != h_first) fetch(h);
         T* v = z + (int64_t)h * a.dim;
-        float x[8], y[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = y[e] = 0.f;
-        if (ha) vec_io<T, 8>::load(v + oa, x);
-        if (hb) vec_io<T, 8>::load(v + ob, y);
-        const T* w = (const T*)(h < a.nq ? a.qw : a.kw);
+        for (int e = 0; e < 8; ++e) { x[e] = ha ? x[e] : 0.f; y[e] = hb ? y[e] : 0.f; }
         auto inv_rms = [&]() {
             float ss = 0.f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], fmaf(y[e], y[e], ss));
             return 1.0f / sqrtf(lanes_sum<LG>(ss) / (float)a.dim + a.eps);
         };
-        if (w) {
+        if (a.qw) {
             const float inv = inv_rms();
-            float g[8];
-            if (ha) {
-                vec_io<T, 8>::load(w + oa, g);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) x[e] *= inv * g[e];
-            }
-            if (hb) {
-                vec_io<T, 8>::load(w + ob, g);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) y[e] *= inv * g[e];
-            }
+            for (int e = 0; e < 8; ++e) { x[e] *= inv * gx[e]; y[e] *= inv * gy[e]; }
         }
         if (u < rot) {
 #pragma unroll
@@ -107,14 +114,14 @@ __global__ __launch_bounds__(256) void heads_prep_kernel(HeadsArgs a) {
         }
     }
     if (slot) {
-        const T* v = z + (int64_t)(a.nq + a.nk) * a.dim;
         T* d = slot + (int64_t)a.nk * a.dim;
-        for (int i = tid * 8; i + 7 < a.nv; i += 2048) {
-            float x[8];
-            vec_io<T, 8>::load(v + i, x);
-            vec_io<T, 8>::store(d + i, x);
+        if (vi + 7 < a.nv) vec_io<T, 8>::store(d + vi, val);
+        for (int i = vi + gridDim.y * 2048; i + 7 < a.nv; i += gridDim.y * 2048) {
+            vec_io<T, 8>::load(values + i, val);
+            vec_io<T, 8>::store(d + i, val);
         }
-        for (int i = a.nv / 8 * 8 + tid; i < a.nv; i += 256) d[i] = v[i];
+        if (blockIdx.y == 0)
+            for (int i = a.nv / 8 * 8 + tid; i < a.nv; i += 256) d[i] = values[i];
     }
 }
 
@@ -176,8 +183,11 @@ extern "C" int evo_heads_prep(void* z, int64_t ld, void* cache, const void* qw, 
     const dim3 grid((unsigned)M), block(256);
     const int64_t lanes = n_rot / 16 + (dim - n_rot + 15) / 16;
     if (n_rot % 16 == 0 && dim % 8 == 0 && lanes <= 64 && ld % 8 == 0 && rs % 8 == 0 && (((uintptr_t)z | (uintptr_t)cache | (uintptr_t)qw | (uintptr_t)kw) & 15) == 0) {
-#define HP(LG) do { if (f32) hipLaunchKernelGGL((heads_prep_kernel<float, LG>), grid, block, lds, s, a);                   \
-                    else hipLaunchKernelGGL((heads_prep_kernel<uint16_t, LG>), grid, block, lds, s, a); } while (0)
+        // (a workgroup's vectors in one round each while that leaves them a CU of their own)
+#define HP(LG) do { const int64_t rounds = ((nq + nk) * LG + 255) / 256, parts = 256 / M < 1 ? 1 : 256 / M;                \
+                    const dim3 g2((unsigned)M, (unsigned)(rounds < parts ? rounds : parts));                               \
+                    if (f32) hipLaunchKernelGGL((heads_prep_kernel<float, LG>), g2, block, lds, s, a);                     \
+                    else hipLaunchKernelGGL((heads_prep_kernel<uint16_t, LG>), g2, block, lds, s, a); } while (0)
         if (lanes <= 1) HP(1); else if (lanes <= 2) HP(2); else if (lanes <= 4) HP(4); else if (lanes <= 8) HP(8);
         else if (lanes <= 16) HP(16); else if (lanes <= 32) HP(32); else HP(64);
 #undef HP

@@ -78,6 +78,15 @@ def test_heads_prep(ops, dt, nq, nk, dim, nv, n_rot, keep, window, norm):
         at += n
 
 
+@TYPES
+@pytest.mark.parametrize("nq,nk,dim,nv,n_rot,keep,window", [(40, 25, 128, 4203, 64, 2, 9), (33, 32, 64, 8200, 64, 0, 100), (60, 9, 256, 2049, 16, 1, 300), (40, 25, 128, 4200, 128, 2, 500)])
+@pytest.mark.parametrize("norm", ["both", "none"])
+def test_heads_prep_shared_out(ops, dt, nq, nk, dim, nv, n_rot, keep, window, norm):
+    """Vectors and values of more than one round of a workgroup, shared out over several (few tokens) or walked by one."""
+    test_heads_prep(ops, dt, nq, nk, dim, nv, n_rot, keep, window, norm)
+
+
+
 # ------------------------------------------------------------------------------------------------ prompts
 def combine(q, k, v, maps, scale, lam, gain, eps, mask):
     if maps == 1:
