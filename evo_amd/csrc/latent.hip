@@ -63,6 +63,34 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(PrepArgs a) {
     }
 }
 
+// One wave: the sum of the squares of a row of R latents (R % 8 == 0); u: this lane's run of eight of the first 512 (lane 0's where there is none).
+template <typename T> __device__ __forceinline__ float latent_sumsq(const T* dkv, int R, int lane, const float* u) {
+    // in latent_prep_kernel's order, so that a row has the same bits on either path: thread t there adds columns t, t + 256, .. one after the other
+    // (lanes l and l + 32 here hold columns t and t + 256 of the same eight threads), then eight, 64 and 256 threads' sums meet
+    float ss[8] = {};
+    for (int r0 = 0; r0 < R; r0 += 512) {
+        float x[8];
+        const int r = r0 + 8 * lane;
+        if (r0 == 0) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = u[e];
+        } else vec_io<T, 8>::load(dkv + (r < R ? r : 0), x);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t own = r < R ? __float_as_uint(x[e]) : 0u;
+            const auto both = __builtin_amdgcn_permlane32_swap(own, own, false, false);      // lane l % 32's value and lane l % 32 + 32's
+            ss[e] = fmaf(__uint_as_float(both[0]), __uint_as_float(both[0]), ss[e]);
+            ss[e] = fmaf(__uint_as_float(both[1]), __uint_as_float(both[1]), ss[e]);
+        }
+    }
+    float sum = ((ss[0] + ss[1]) + (ss[2] + ss[3])) + ((ss[4] + ss[5]) + (ss[6] + ss[7]));
+    sum += dpp_fetch<EVO_DPP_XOR1>(sum);
+    sum += dpp_fetch<EVO_DPP_XOR2>(sum);
+    sum += dpp_fetch<EVO_DPP_HALF_MIRROR>(sum);
+    auto of = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sum), l)); };
+    return of(0) + of(8) + of(16) + of(24);
+}
+
 // The same in 16-byte requests (8 bf16 or 4 fp32 at a time twice) where every part is whole ones: three waves rotate, the fourth norms, and what a thread needs is asked for
 // before the angles; the roundings and the order of the sums are latent_prep_kernel's.  A decode step waits for one round of requests where it waited for one each pair of elements after the other, a prompt is a fifth of the instructions.
 // 32 heads of 128 + 64, R = 512, pair by pair -> this: 8 tokens decoded 4.1 -> 2.6 us, 11,877 of a prompt 38.2 -> 22.2.
@@ -92,30 +120,7 @@ __global__ __launch_bounds__(256) void latent_prep_vec_kernel(PrepArgs a) {
     for (int i = tid; i < half; i += 256) sincosf((float)pos * a.inv_freq[i], &turn[i].y, &turn[i].x);
     __syncthreads();
     if (norms) {
-        // the squares' sum in latent_prep_kernel's order, so that a row has the same bits on either path: thread t there adds columns t, t + 256, .. one after the other
-        // (lanes l and l + 32 here hold columns t and t + 256 of the same eight threads), then eight, 64 and 256 threads' sums meet
-        float ss[8] = {};
-        for (int r0 = 0; r0 < a.R; r0 += 512) {
-            float x[8];
-            const int r = r0 + 8 * lane;
-            if (r0 == 0) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) x[e] = u[e];
-            } else vec_io<T, 8>::load(dkv + (r < a.R ? r : 0), x);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint32_t own = r < a.R ? __float_as_uint(x[e]) : 0u;
-                const auto both = __builtin_amdgcn_permlane32_swap(own, own, false, false);      // lane l % 32's value and lane l % 32 + 32's
-                ss[e] = fmaf(__uint_as_float(both[0]), __uint_as_float(both[0]), ss[e]);
-                ss[e] = fmaf(__uint_as_float(both[1]), __uint_as_float(both[1]), ss[e]);
-            }
-        }
-        float sum = ((ss[0] + ss[1]) + (ss[2] + ss[3])) + ((ss[4] + ss[5]) + (ss[6] + ss[7]));
-        sum += dpp_fetch<EVO_DPP_XOR1>(sum);
-        sum += dpp_fetch<EVO_DPP_XOR2>(sum);
-        sum += dpp_fetch<EVO_DPP_HALF_MIRROR>(sum);
-        auto of = [&](int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sum), l)); };
-        sum = of(0) + of(8) + of(16) + of(24);
+        const float sum = latent_sumsq<T>(dkv, a.R, lane, u);
         const float inv = 1.0f / sqrtf(sum / (float)a.R + a.eps);
         for (int r = 8 * lane; r < a.R; r += 512) {
             float x[8], w[8];
@@ -181,15 +186,51 @@ extern "C" int evo_latent_prep(void* q, int64_t ldq, void* c, void* kr, void* ca
 // ------------------------------------------------------------------------------------------------ decode: query side of the key map
 // out[b][h] = [W_uk,h^T q_n (R) | rotated q (dr) | zeros up to rs].  Workgroup: 64 V latent columns of one head, NB sequences; eight waves
 // share the dn rows of the map, a lane owns V adjacent columns.  Latency bounds it (4 MB of map at 32 heads of 128 x 512): a wave asks for its first 16 rows
-// before anything else, and columns are halved where that leaves fewer than 128 workgroups.
-template <typename T, int NB, int V>
+// before anything else, and columns are halved while that leaves fewer than 256 workgroups.
+// PREP: q comes as the projection wrote it.  The heads' first workgroups rotate (the queries stay as they are), and one more "head" norms and rotates the tokens' own rows
+// for the cache, a wave a token: latent_prep and this in one launch, with the bits of two.  In a step of four layers, 8 sequences, 32 heads of 128 x 512: 11.8 us in two
+// launches with 128 workgroups' columns here, 7.4 so (3.1 of them the requests' latency, the map being cold); columns halved to 256 instead of 128 workgroups 0.4 to 1.3
+// (3 / 4 / 8 sequences 23.4 / 24.9 / 26.0 -> 22.2 / 23.6 / 25.6, all launches of the layer).
+template <typename T, int NB, int V, bool PREP>
 __global__ __launch_bounds__(512) void latent_absorb_kernel(const void* __restrict__ q_, int64_t ldq, const void* __restrict__ w_, void* __restrict__ out_,
-                                                            int B, int H, int dn, int dr, int R, int rs) {
+                                                            int B, int H, int dn, int dr, int R, int rs, PrepArgs a) {
     extern __shared__ float sm[];                                // q parts [NB][dn], partial sums [8][NB][64 V]
     constexpr int U = 16;                                        // rows of a wave in flight
     float* part = sm + NB * dn;
     const int h = blockIdx.y, b0 = blockIdx.z * NB, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int nb = B - b0 < NB ? B - b0 : NB, dh = dn + dr;
+    const int nb = B - b0 < NB ? B - b0 : NB, dh = dn + dr, half = PREP ? a.n_rot / 2 : 0;
+    if (PREP && h == H) {                                        // the cache's rows
+        if (wave >= nb || blockIdx.x) return;
+        const int b = b0 + wave;
+        const T* dkv = (const T*)q_ + (int64_t)b * ldq + (int64_t)H * dh;
+        float u[8], w[8];
+        vec_io<T, 8>::load(dkv + (8 * lane < R ? 8 * lane : 0), u);
+        vec_io<T, 8>::load((const T*)a.w + (8 * lane < R ? 8 * lane : 0), w);
+        const int i0 = lane < dr ? lane : 0, ip = lane < half ? lane + half : i0;
+        const float x0 = ld1(dkv + R + i0), x1 = ld1(dkv + R + ip), f0 = a.inv_freq[lane < half ? lane : 0];
+        const int64_t pos = a.pos[b];
+        T* slot = (T*)a.cache + ((int64_t)b * a.ring + pos % a.ring) * rs;
+        const float sum = latent_sumsq<T>(dkv, R, lane, u), inv = 1.0f / sqrtf(sum / (float)R + a.eps);
+        for (int r = 8 * lane; r < R; r += 512) {
+            if (r >= 512) {
+                vec_io<T, 8>::load(dkv + r, u);
+                vec_io<T, 8>::load((const T*)a.w + r, w);
+            }
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = u[e] * inv * w[e];
+            vec_io<T, 8>::store(slot + r, x);
+        }
+        for (int i = lane; i < half; i += 64) {
+            const float p = i == lane ? x0 : ld1(dkv + R + i), v = i == lane ? x1 : ld1(dkv + R + i + half);
+            float sn, cs;
+            sincosf((float)pos * (i == lane ? f0 : a.inv_freq[i]), &sn, &cs);
+            st1(slot + R + i, fmaf(p, cs, -(v * sn)));
+            st1(slot + R + i + half, fmaf(p, sn, v * cs));
+        }
+        for (int i = 2 * half + lane; i < dr; i += 64) st1(slot + R + i, ld1(dkv + R + i));
+        return;
+    }
     const int r0 = blockIdx.x * 64 * V, r = r0 + lane * V;
     const T* w = (const T*)w_ + (int64_t)h * dn * R + (r < R ? r : 0);       // (lanes behind the last column read the first ones and store nothing)
     float f[U][V];
@@ -198,6 +239,20 @@ __global__ __launch_bounds__(512) void latent_absorb_kernel(const void* __restri
         for (int u = 0; u < U; ++u) vec_io<T, V>::load(w + (int64_t)(n + 8 * u < dn ? n + 8 * u : dn - 1) * R, f[u]);
     };
     fetch(wave);                                                 // (no need of the queries: on their way behind each other)
+    // the part behind the latents: element c, its partner in the rotation, the pair's frequency and the position of this thread's first one, asked for with the rest
+    const int tail = rs - R, per = tail > 0 ? tail : 1, c_first = tid < NB * tail ? tid : 0, i_first = c_first / per, c_in = c_first - i_first * per;
+    const int b_first = b0 + (i_first < nb ? i_first : 0);
+    const T* q_first = (const T*)q_ + (int64_t)b_first * ldq + (int64_t)h * dh + dn;
+    float tx = 0.f, ty = 0.f, tf = 0.f;
+    int64_t tp = 0;
+    if (blockIdx.x == 0 && dr > 0) {
+        tx = ld1(q_first + (c_in < dr ? c_in : 0));
+        if constexpr (PREP) {
+            ty = ld1(q_first + (c_in < half ? c_in + half : c_in < 2 * half ? c_in - half : 0));
+            tf = a.inv_freq[c_in < half ? c_in : c_in < 2 * half ? c_in - half : 0];
+            tp = a.pos[b_first];
+        }
+    }
 #pragma unroll
     for (int i = 0; i < NB; ++i)
         for (int n = tid; n < dn; n += 512) sm[i * dn + n] = i < nb ? ld1((const T*)q_ + (int64_t)(b0 + i) * ldq + (int64_t)h * dh + n) : 0.f;
@@ -222,43 +277,72 @@ __global__ __launch_bounds__(512) void latent_absorb_kernel(const void* __restri
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) vec_io<float, V>::store(part + ((wave * NB + i) * 64 + lane) * V, acc[i]);
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-        if (i >= nb) break;
-        T* out = (T*)out_ + ((int64_t)(b0 + i) * H + h) * rs;
-        for (int c = tid; c < 64 * V; c += 512) {
-            float v = 0.f;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) v += part[(k * NB + i) * 64 * V + c];
-            if (r0 + c < R) st1(out + r0 + c, v);
+    if (blockIdx.x == 0)
+        for (int it = tid; it < NB * tail; it += 512) {
+            const int i = it / per, c = it - i * per;
+            if (i >= nb) break;
+            const bool again = it != tid;
+            const T* qt = (const T*)q_ + (int64_t)(b0 + i) * ldq + (int64_t)h * dh + dn;
+            float x = 0.f;
+            if (c < dr) {
+                x = again ? ld1(qt + c) : tx;
+                if (PREP && c < 2 * half) {
+                    const int k = c < half ? c : c - half;
+                    const float y = again ? ld1(qt + (c < half ? c + half : k)) : ty;
+                    float sn, cs;
+                    sincosf((float)(again ? a.pos[b0 + i] : tp) * (again ? a.inv_freq[k] : tf), &sn, &cs);
+                    x = c < half ? fmaf(x, cs, -(y * sn)) : fmaf(y, sn, x * cs);
+                }
+            }
+            st1((T*)out_ + ((int64_t)(b0 + i) * H + h) * rs + R + c, x);
         }
-        if (blockIdx.x == 0)
-            for (int c = R + tid; c < rs; c += 512)
-                st1(out + c, c < R + dr ? ld1((const T*)q_ + (int64_t)(b0 + i) * ldq + (int64_t)h * dh + dn + c - R) : 0.f);
+    __syncthreads();
+    for (int it = tid; it < NB * 64 * V; it += 512) {
+        const int i = it / (64 * V), c = it % (64 * V);
+        float v = 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v += part[(k * NB + i) * 64 * V + c];
+        if (i < nb && r0 + c < R) st1((T*)out_ + ((int64_t)(b0 + i) * H + h) * rs + r0 + c, v);
     }
+}
+
+// prep: null, or the preparation's arguments
+static int latent_absorb(const void* q, int64_t ldq, const void* wuk, void* out, int64_t B, int64_t H, int64_t dn, int64_t dr, int64_t R, int64_t rs, const PrepArgs* prep,
+                         int64_t f32, void* stream) {
+    if (!q || !wuk || !out || B <= 0 || H <= 0 || H > 65534 || dn <= 0 || dn > 4096 || dr < 0 || R <= 0 || rs < R + dr || ldq < H * (dn + dr)) return -1;
+    const int nb = B > 2 ? 4 : (int)B;
+    int v = R % 8 == 0 && ((uintptr_t)wuk & 15) == 0 ? 8 : 1;
+    while (v > 2 && ((R + 64 * v - 1) / (64 * v)) * H * ((B + nb - 1) / nb) < 256) v /= 2;
+    const dim3 grid((unsigned)((R + 64 * v - 1) / (64 * v)), (unsigned)(H + (prep ? 1 : 0)), (unsigned)((B + nb - 1) / nb)), block(512);
+    const size_t lds = (size_t)nb * (dn + 512 * v) * 4;          // (<= 128 KB)
+    hipStream_t s = (hipStream_t)stream;
+    const PrepArgs a = prep ? *prep : PrepArgs{};
+#define AB(T, NB, V, P)                                                                                                    \
+    do {                                                                                                                   \
+        if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)latent_absorb_kernel<T, NB, V, P>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+        hipLaunchKernelGGL((latent_absorb_kernel<T, NB, V, P>), grid, block, lds, s, q, ldq, wuk, out, (int)B, (int)H, (int)dn, (int)dr, (int)R, (int)rs, a); \
+    } while (0)
+#define ABP(T, NB, V) do { if (prep) AB(T, NB, V, true); else AB(T, NB, V, false); } while (0)
+#define ABV(T, V) do { if (nb == 1) ABP(T, 1, V); else if (nb == 2) ABP(T, 2, V); else ABP(T, 4, V); } while (0)
+    if (f32) { if (v == 8) ABV(float, 8); else if (v == 4) ABV(float, 4); else if (v == 2) ABV(float, 2); else ABV(float, 1); }
+    else { if (v == 8) ABV(uint16_t, 8); else if (v == 4) ABV(uint16_t, 4); else if (v == 2) ABV(uint16_t, 2); else ABV(uint16_t, 1); }
+#undef ABV
+#undef ABP
+#undef AB
+    return evo_launch_status();
 }
 
 extern "C" int evo_latent_absorb(const void* q, int64_t ldq, const void* wuk, void* out, int64_t B, int64_t H, int64_t dn, int64_t dr, int64_t R,
                                  int64_t rs, int64_t f32, void* stream) {
-    if (!q || !wuk || !out || B <= 0 || H <= 0 || H > 65535 || dn <= 0 || dn > 4096 || dr < 0 || R <= 0 || rs < R + dr || ldq < H * (dn + dr)) return -1;
-    const int nb = B > 2 ? 4 : (int)B;
-    int v = R % 8 == 0 && ((uintptr_t)wuk & 15) == 0 ? 8 : 1;
-    if (v == 8 && ((R + 511) / 512) * H * ((B + nb - 1) / nb) < 128) v = 4;
-    const dim3 grid((unsigned)((R + 64 * v - 1) / (64 * v)), (unsigned)H, (unsigned)((B + nb - 1) / nb)), block(512);
-    const size_t lds = (size_t)nb * (dn + 512 * v) * 4;          // (<= 128 KB)
-    hipStream_t s = (hipStream_t)stream;
-#define AB(T, NB, V)                                                                                                       \
-    do {                                                                                                                   \
-        if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)latent_absorb_kernel<T, NB, V>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
-        hipLaunchKernelGGL((latent_absorb_kernel<T, NB, V>), grid, block, lds, s, q, ldq, wuk, out, (int)B, (int)H, (int)dn, (int)dr, (int)R, (int)rs); \
-    } while (0)
-#define ABV(T, V) do { if (nb == 1) AB(T, 1, V); else if (nb == 2) AB(T, 2, V); else AB(T, 4, V); } while (0)
-    if (f32) { if (v == 8) ABV(float, 8); else if (v == 4) ABV(float, 4); else ABV(float, 1); }
-    else { if (v == 8) ABV(uint16_t, 8); else if (v == 4) ABV(uint16_t, 4); else ABV(uint16_t, 1); }
-#undef ABV
-#undef AB
-    return evo_launch_status();
+    return latent_absorb(q, ldq, wuk, out, B, H, dn, dr, R, rs, nullptr, f32, stream);
+}
+
+extern "C" int evo_latent_prep_absorb(const void* q, int64_t ldq, const void* wuk, void* out, void* cache, const void* w, const float* inv_freq, const int64_t* pos, int64_t B,
+                                      int64_t H, int64_t dn, int64_t dr, int64_t R, int64_t n_rot, int64_t ring, int64_t rs, float eps, int64_t f32, void* stream) {
+    if (!q || !cache || !w || !pos || !inv_freq || ring <= 0 || n_rot <= 0 || n_rot > dr || n_rot % 2 || ldq < H * (dn + dr) + R + dr) return -1;
+    if (ldq % 8 || (dn + dr) * H % 8 || R % 8 || rs % 8 || (((uintptr_t)q | (uintptr_t)cache | (uintptr_t)w) & 15)) return -1;
+    const PrepArgs a = {nullptr, ldq, nullptr, nullptr, cache, w, inv_freq, pos, nullptr, nullptr, (int)H, (int)dn, (int)dr, (int)R, (int)n_rot, (int)ring, (int)rs, eps};
+    return latent_absorb(q, ldq, wuk, out, B, H, dn, dr, R, rs, &a, f32, stream);
 }
 
 // ------------------------------------------------------------------------------------------------ decode: scores and sum on the latents
@@ -423,6 +507,13 @@ __global__ __launch_bounds__(512, 2) void latent_decode_kernel(DecArgs a) {
             const int grp = wave + 8 * i, h = h0 + 16 * cb + c16;
             if (grp < NR && h < a.H) {
                 float* po = a.part_o + (((int64_t)b * a.H + h) * a.n_split + split) * a.R;
+                if ((a.R & 7) == 0) {                            // (a lane's eight columns are neighbours)
+                    if (32 * grp + 8 * g < a.R) {
+                        *(f32x4_t*)(po + 32 * grp + 8 * g) = f32x4_t{o[i][0][cb][0], o[i][1][cb][0], o[i][0][cb][1], o[i][1][cb][1]};
+                        *(f32x4_t*)(po + 32 * grp + 8 * g + 4) = f32x4_t{o[i][0][cb][2], o[i][1][cb][2], o[i][0][cb][3], o[i][1][cb][3]};
+                    }
+                    continue;
+                }
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int col = 32 * grp + 8 * g + 2 * r;
@@ -660,55 +751,82 @@ __global__ __launch_bounds__(512) void latent_up_kernel(const float* __restrict_
     }
 }
 
-// The same on the matrix cores (bf16, R % 32 == 0): 128 value rows of one head and NS sequences, a wave owns 16 of the rows.  Latency and the pace of one CU bound
-// it: at 8 sequences of 16 parts a head's merge reads 262 KB, its rows 131 KB.  So sequences are spread over up to 256 workgroups (a head's rows are read by
-// several), and the first 512 columns of the rows are asked for before the parts.
+// The same on the matrix cores (bf16, R % 32 == 0): VR value rows of one head and NS sequences, a wave owns 16 of the rows.  Latency and the pace of one CU bound
+// it: at 8 sequences of 16 parts a head's merge reads 262 KB, its rows 131 KB.  So sequences, then rows, are spread over up to 256 workgroups (a head's rows and parts are
+// read by several), and everything a thread needs is asked for together: statistics, its first 16 parts, the first 512 columns of the rows.
 // latent_absorb to here, 32 heads, R = 512, 900 slots, in a graph: 3 / 8 / 16 / 32 sequences 28.0 / 34.9 / 39.4 / 48.0 -> 23.8 / 27.9 / 29.9 / 36.7 us; of 64 x 128
-// 14.4 / 16.4 / 19.2 / 22.3 -> 14.4 / 15.9 / 17.4 / 20.3.
-template <int NS>
+// 14.4 / 16.4 / 19.2 / 22.3 -> 14.4 / 15.9 / 17.4 / 20.3.  With the rows spread, the requests together and the preparation in
+// latent_absorb's launch, caches and maps cold, latent_prep to here: 1 / 3 / 8 / 16 / 32 sequences 21.9 / 27.7 / 32.2 / 34.5 / 39.9 -> 17.8 / 22.2 / 25.7 / 29.5 / 38.8 us.
+template <int NS, int VR>
 __global__ __launch_bounds__(512) void latent_up_mfma_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, const float* __restrict__ sink,
                                                              const uint16_t* __restrict__ w, uint16_t* __restrict__ o, int B, int H, int R, int dv, int n_split) {
     extern __shared__ __attribute__((aligned(16))) uint16_t lat[];   // [NS][R + 8] merged latents, then [NS][n_split] weights of the parts
+    constexpr int PF = 16;                                       // parts of a thread's item in flight
     const int h = blockIdx.y, b0 = blockIdx.z * NS, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int pr = R + 8, c16 = lane & 15, g = lane >> 4;
     float* wt = (float*)(lat + NS * pr);
-    const int v0 = blockIdx.x * 128 + 16 * wave;
-    const uint16_t* wr = w + ((int64_t)h * dv + (v0 + c16 < dv ? v0 + c16 : dv - 1)) * R + 8 * g;
-    mx_u32x4 first[16];
+    const int v0 = blockIdx.x * VR + 16 * wave;
+    const bool rows = 16 * wave < VR && v0 < dv;                 // (the same in a whole wave)
+    constexpr int SW = (NS + 7) / 8;                             // sequences of a wave
+    float m[SW], d[SW];
+    const float sk = sink[h] * LOG2E;
 #pragma unroll
-    for (int k = 0; k < 16; ++k)
-        if (32 * k < R) first[k] = *(const mx_u32x4*)(wr + 32 * k);
-    for (int i = wave; i < NS; i += 8) {
-        const int b = b0 + i < B ? b0 + i : B - 1;
-        const float* ml = part_ml + ((int64_t)b * H + h) * n_split * 2;
-        const float m = lane < n_split ? ml[2 * lane] : -INFINITY, d = lane < n_split ? ml[2 * lane + 1] : 0.f;     // (n_split <= 64)
-        const float sk = sink[h] * LOG2E, top = fmaxf(sk, wave_max(m)), f = exp2f(m - top);
-        const float l = wave_sum(d * f) + exp2f(sk - top);
+    for (int k = 0; k < SW; ++k) {
+        const int i = wave + 8 * k, b = b0 + i < B ? b0 + i : B - 1;
+        const float* ml = part_ml + (((int64_t)b * H + h) * n_split + (lane < n_split ? lane : 0)) * 2;     // (n_split <= 64)
+        m[k] = ml[0];
+        d[k] = ml[1];
+    }
+    const int items = NS * (R / 4);
+    auto part_of = [&](int it) {                                 // an item's first part
+        const int i = it / (R / 4), r = it % (R / 4) * 4, b = b0 + i < B ? b0 + i : B - 1;
+        return part_o + ((int64_t)b * H + h) * n_split * R + r;
+    };
+    f32x4_t x[PF];
+    {
+        const float* po = part_of(tid < items ? tid : 0);
+#pragma unroll
+        for (int u = 0; u < PF; ++u) x[u] = *(const f32x4_t*)(po + (int64_t)(u < n_split ? u : n_split - 1) * R);
+    }
+    const uint16_t* wr = w + ((int64_t)h * dv + (rows && v0 + c16 < dv ? v0 + c16 : dv - 1)) * R + 8 * g;
+    mx_u32x4 first[16];
+    if (rows) {
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+            if (32 * k < R) first[k] = *(const mx_u32x4*)(wr + 32 * k);
+    }
+#pragma unroll
+    for (int k = 0; k < SW; ++k) {
+        const int i = wave + 8 * k;
+        if (i >= NS) break;
+        const float mk = lane < n_split ? m[k] : -INFINITY, top = fmaxf(sk, wave_max(mk)), f = exp2f(mk - top);
+        const float l = wave_sum((lane < n_split ? d[k] : 0.f) * f) + exp2f(sk - top);
         if (lane < n_split) wt[i * n_split + lane] = f / l;
     }
     __syncthreads();
-    for (int it = tid; it < NS * (R / 4); it += 512) {
-        const int i = it / (R / 4), r = it % (R / 4) * 4, b = b0 + i < B ? b0 + i : B - 1;
-        const float* po = part_o + ((int64_t)b * H + h) * n_split * R + r;
+    for (int it = tid; it < items; it += 512) {
+        const int i = it / (R / 4), r = it % (R / 4) * 4;
+        const float* po = part_of(it);
         f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-        for (int s = 0; s < n_split; s += 8) {                   // (eight requests on their way together: left to itself the compiler waits for each)
-            f32x4_t x[8];
+        for (int s = 0; s < n_split; s += PF) {                  // (a round's requests on their way together: left to itself the compiler waits for each)
+            if (s || it != tid) {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) x[u] = *(const f32x4_t*)(po + (int64_t)(s + u < n_split ? s + u : n_split - 1) * R);
+                for (int u = 0; u < PF; ++u) x[u] = *(const f32x4_t*)(po + (int64_t)(s + u < n_split ? s + u : n_split - 1) * R);
+            }
 #pragma unroll
-            for (int u = 0; u < 8; ++u) asm volatile("" : "+v"(x[u]));
+            for (int u = 0; u < PF; ++u) asm volatile("" : "+v"(x[u]));
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                if (s + u >= n_split) break;
-                const float f = wt[i * n_split + s + u];
+            for (int u = 0; u < PF; ++u) {
+                const bool on = s + u < n_split;
+                const float f = wt[i * n_split + (on ? s + u : n_split - 1)];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc[e] = fmaf(x[u][e], f, acc[e]);
+                for (int e = 0; e < 4; ++e) acc[e] = on ? fmaf(x[u][e], f, acc[e]) : acc[e];
             }
         }
         *(uint2*)(lat + i * pr + r) = make_uint2(pack_bf2(acc[0], acc[1]), pack_bf2(acc[2], acc[3]));
     }
     __syncthreads();
-    if (v0 >= dv) return;
+    if (!rows) return;
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
     const int cl = c16 < NS ? c16 : 0;                           // (columns beyond NS repeat the first and are not stored)
 #pragma unroll
@@ -729,17 +847,20 @@ extern "C" int evo_latent_up(const float* part_o, const float* part_ml, const fl
                              int64_t dv, int64_t n_split, int64_t f32, int64_t mfma, void* stream) {
     if (!part_o || !part_ml || !sink || !wuv || !o || B <= 0 || H <= 0 || H > 65535 || R <= 0 || R > 8192 || dv <= 0 || n_split <= 0 || n_split > 64) return -1;
     if (!f32 && mfma && B > 2 && R % 32 == 0 && R <= 1024 && (((uintptr_t)wuv | (uintptr_t)part_o) & 15) == 0) {
-        int ns = 2;                                              // as many workgroups as there are CUs, if there are that many heads and sequences
+        int ns = 2, vr = 128;                                    // as many workgroups as there are CUs, if there are that many heads and sequences
         const int64_t per = H * ((dv + 127) / 128);
         while (ns < 16 && per * ((B + ns - 1) / ns) > 256) ns *= 2;
-        const dim3 grid((unsigned)((dv + 127) / 128), (unsigned)H, (unsigned)((B + ns - 1) / ns));
+        while (ns == 2 && vr > 32 && H * ((dv + vr / 2 - 1) / (vr / 2)) * ((B + 1) / 2) <= 256) vr /= 2;
+        const dim3 grid((unsigned)((dv + vr - 1) / vr), (unsigned)H, (unsigned)((B + ns - 1) / ns));
         const size_t lds = (size_t)ns * ((R + 8) * 2 + n_split * 4);
-#define UPM(NS) hipLaunchKernelGGL((latent_up_mfma_kernel<NS>), grid, dim3(512), lds, (hipStream_t)stream, part_o, part_ml, sink, (const uint16_t*)wuv, \
-                                   (uint16_t*)o, (int)B, (int)H, (int)R, (int)dv, (int)n_split)
-        if (ns == 2) UPM(2);
-        else if (ns == 4) UPM(4);
-        else if (ns == 8) UPM(8);
-        else UPM(16);
+#define UPM(NS, VR) hipLaunchKernelGGL((latent_up_mfma_kernel<NS, VR>), grid, dim3(512), lds, (hipStream_t)stream, part_o, part_ml, sink, (const uint16_t*)wuv, \
+                                       (uint16_t*)o, (int)B, (int)H, (int)R, (int)dv, (int)n_split)
+        if (vr == 32) UPM(2, 32);
+        else if (vr == 64) UPM(2, 64);
+        else if (ns == 2) UPM(2, 128);
+        else if (ns == 4) UPM(4, 128);
+        else if (ns == 8) UPM(8, 128);
+        else UPM(16, 128);
 #undef UPM
         return evo_launch_status();
     }

@@ -55,6 +55,19 @@ template <> struct vec_io<float, 4> {
     }
     static __device__ __forceinline__ void store(float* p, const float* f) { *(float4*)p = make_float4(f[0], f[1], f[2], f[3]); }
 };
+template <> struct vec_io<uint16_t, 2> {
+    static __device__ __forceinline__ void load(const uint16_t* p, float* f) {
+        const uint32_t v = *(const uint32_t*)p;
+        f[0] = bf_lo(v); f[1] = bf_hi(v);
+    }
+};
+template <> struct vec_io<float, 2> {
+    static __device__ __forceinline__ void load(const float* p, float* f) {
+        const float2 a = *(const float2*)p;
+        f[0] = a.x; f[1] = a.y;
+    }
+    static __device__ __forceinline__ void store(float* p, const float* f) { *(float2*)p = make_float2(f[0], f[1]); }
+};
 template <typename T> struct vec_io<T, 1> {
     static __device__ __forceinline__ void load(const T* p, float* f) { f[0] = ld1(p); }
     static __device__ __forceinline__ void store(T* p, const float* f) { st1(p, f[0]); }

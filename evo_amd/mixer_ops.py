@@ -439,9 +439,16 @@ class MixerOps:
             return n, 16
         return parts((heads + 31) // 32), 32
 
+    @staticmethod
+    def latent_prep_fits(qd: torch.Tensor, cache: torch.Tensor, norm_w: torch.Tensor, inv_freq: torch.Tensor, heads: int, dn: int, dr: int, R: int) -> bool:
+        """What latent_decode's `prep` takes: rows of whole 16-byte pieces."""
+        return (qd.stride(0) % 8 == 0 and heads * (dn + dr) % 8 == 0 and R % 8 == 0 and cache.shape[2] % 8 == 0 and 0 < 2 * inv_freq.numel() <= dr and dn <= 4096
+                and norm_w.dtype == qd.dtype and (qd.data_ptr() | cache.data_ptr() | norm_w.data_ptr()) % 16 == 0)
+
     def latent_decode(self, qd: torch.Tensor, cache: torch.Tensor, pos: torch.Tensor, wuk: torch.Tensor, wuv: torch.Tensor, sink: torch.Tensor,
-                      heads: int, dn: int, dr: int, dv: int, R: int, window: int, scale: float, n_split: Optional[int] = None) -> torch.Tensor:
-        """One token per cache row (already appended by latent_prep) against the ring cache -> [B, heads dv]."""
+                      heads: int, dn: int, dr: int, dv: int, R: int, window: int, scale: float, n_split: Optional[int] = None, prep=None) -> torch.Tensor:
+        """One token per cache row against the ring cache -> [B, heads dv].  The rows are already appended by latent_prep or, with `prep` = (norm weight, inv_freq, eps),
+        are appended here, by the first launch; qd's queries then stay as they are."""
         f32 = self._store(qd, cache, wuk, wuv)
         B = qd.shape[0]
         rows, ring, rs = cache.shape
@@ -449,7 +456,14 @@ class MixerOps:
         self._dense(wuk, (heads * dn, R), "wuk"), self._dense(wuv, (heads * dv, R), "wuv")
         assert rows >= B and qd.shape[1] >= heads * (dn + dr) and window <= ring and sink.numel() == heads
         q = torch.empty(B, heads, rs, dtype=qd.dtype, device=qd.device)
-        self._call("evo_latent_absorb", qd.data_ptr(), qd.stride(0), wuk.data_ptr(), q.data_ptr(), B, heads, dn, dr, R, rs, f32)
+        if prep is None:
+            self._call("evo_latent_absorb", qd.data_ptr(), qd.stride(0), wuk.data_ptr(), q.data_ptr(), B, heads, dn, dr, R, rs, f32)
+        else:
+            norm_w, inv_freq, eps = prep
+            assert norm_w.dtype == qd.dtype and norm_w.is_cuda and norm_w.is_contiguous() and norm_w.numel() == R and qd.shape[1] >= heads * (dn + dr) + R + dr
+            self._call("evo_latent_prep_absorb", qd.data_ptr(), qd.stride(0), wuk.data_ptr(), q.data_ptr(), cache.data_ptr(), norm_w.data_ptr(),
+                       self._ix(inv_freq, torch.float32, 0, "inv_freq"), self._ix(pos, torch.int64, B, "pos"), B, heads, dn, dr, R, 2 * inv_freq.numel(), ring, rs,
+                       float(eps), f32)
         group = 1
         if n_split is None:
             n_split, group = self.latent_split(B, heads, (ring + 63) // 64)

@@ -154,8 +154,12 @@ class LatentAttention(Sublayer):
         H, dn, dr, dv, R = self.heads, self.dn, self.dr, self.dv, self.R
         qd = stream.linear(self.w_in)                             # [queries | latent, shared key]
         if batch.decode:
-            ops.latent_prep(qd, H, dn, dr, R, self.w_norm, self.inv_freq, self.eps, batch, cache, want_kv=False)
-            a = ops.latent_decode(qd, cache, batch.pos, self.w_kv[:H * dn], self.w_kv[H * dn:], self.sink, H, dn, dr, dv, R, self.window, self.scale)
+            more = {}
+            if hasattr(ops, "latent_prep_fits") and ops.latent_prep_fits(qd, cache, self.w_norm, self.inv_freq, H, dn, dr, R):
+                more["prep"] = (self.w_norm, self.inv_freq, self.eps)
+            else:
+                ops.latent_prep(qd, H, dn, dr, R, self.w_norm, self.inv_freq, self.eps, batch, cache, want_kv=False)
+            a = ops.latent_decode(qd, cache, batch.pos, self.w_kv[:H * dn], self.w_kv[H * dn:], self.sink, H, dn, dr, dv, R, self.window, self.scale, **more)
             return stream.product(a, self.w_o)
         old, seen = (None, None) if batch.resume is None else self._earlier(batch, cache)   # (read before the ring moves on)
         c, kr = ops.latent_prep(qd, H, dn, dr, R, self.w_norm, self.inv_freq, self.eps, batch, cache, want_kv=True)

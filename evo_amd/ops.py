@@ -103,6 +103,7 @@ _SIGNATURES = {
     "evo_rglru_chunk_bf16": ([_PTR, _I64] + [_PTR] * 13 + [_I64] * 6 + [_PTR], _c.c_int),
     "evo_rglru_step_bf16": ([_PTR, _I64] + [_PTR] * 11 + [_I64] * 5 + [_PTR], _c.c_int),
     "evo_rglru_any": ([_PTR, _I64] + [_PTR] * 15 + [_I64] * 7 + [_PTR], _c.c_int),
+    "evo_latent_prep_absorb": ([_PTR, _I64] + [_PTR] * 6 + [_I64] * 8 + [_F32, _I64, _PTR], _c.c_int),
     "evo_latent_absorb": ([_PTR, _I64] + [_PTR] * 2 + [_I64] * 7 + [_PTR], _c.c_int),
     "evo_latent_decode": ([_PTR] * 5 + [_I64] * 8 + [_F32] + [_I64] * 2 + [_PTR], _c.c_int),
     "evo_latent_up": ([_PTR] * 5 + [_I64] * 7 + [_PTR], _c.c_int),

@@ -68,7 +68,7 @@ extern "C" {
  *  24: evo_linear_f32_ahead and evo_linear_f32_ahead_plan added.
  *  25: evo_linear_few_f32 added.
  *  26: evo_dense_launches added.
- *  27: evo_closing_final added. */
+ *  27: evo_closing_final and evo_latent_prep_absorb added. */
 #define EVO_ABI_VERSION 27
 int evo_abi_version(void);
 
@@ -583,6 +583,10 @@ int evo_latent_prep(void* q, int64_t ldq, void* c, void* kr, void* cache, const 
  *   16 (mfma 16, or up to 16 heads) or 32 heads per workgroup);  o [B, H dv] = W_uv,h of the merged, sink-normalised latent. */
 int evo_latent_absorb(const void* q, int64_t ldq, const void* wuk, void* out, int64_t B, int64_t H, int64_t dn, int64_t dr, int64_t R, int64_t rs,
                       int64_t f32, void* stream);
+/* evo_latent_absorb on a projection's rows as they are (R + dr more elements behind the queries), and evo_latent_prep's rows of the cache, in one launch with the bits of two;
+ * q is not written.  0 < n_rot <= dr, and ldq, H (dn + dr), R and rs whole 16-byte pieces of bf16. */
+int evo_latent_prep_absorb(const void* q, int64_t ldq, const void* wuk, void* out, void* cache, const void* w, const float* inv_freq, const int64_t* pos, int64_t B,
+                           int64_t H, int64_t dn, int64_t dr, int64_t R, int64_t n_rot, int64_t ring, int64_t rs, float eps, int64_t f32, void* stream);
 int evo_latent_decode(const void* q, const void* cache, const int64_t* pos, float* part_o, float* part_ml, int64_t B, int64_t H, int64_t R,
                       int64_t dr, int64_t rs, int64_t ring, int64_t window, int64_t n_split, float scale, int64_t f32, int64_t mfma, void* stream);
 int evo_latent_up(const float* part_o, const float* part_ml, const float* sink, const void* wuv, void* o, int64_t B, int64_t H, int64_t R,

@@ -34,3 +34,29 @@ def test_the_bits_of_the_element_kernel(ops, dt, H, dn, dr, R, n_rot):  # noqa: 
         out.append((z[:, :width], c, kr, cache))
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+@TYPES
+@pytest.mark.parametrize("B,H,dn,dr,R,n_rot,ring", [(1, 32, 128, 64, 512, 64, 1024), (2, 5, 16, 24, 64, 16, 7), (3, 2, 40, 72, 1032, 72, 9), (5, 3, 24, 200, 72, 130, 3),
+                                                    (8, 32, 128, 64, 512, 64, 64), (13, 3, 200, 8, 520, 2, 40)])
+def test_preparation_with_the_query_side(ops, dt, B, H, dn, dr, R, n_rot, ring):  # noqa: F811
+    """latent_decode with `prep` against latent_prep in front of it: the same cached rows and the same result, bit for bit; queries as they were, other rows untouched."""
+    from evo_amd.mixer_ops import MixerOps, TokenBatch
+    g = torch.Generator(device="cuda").manual_seed(B)
+
+    def rnd(*s):
+        return torch.randn(*s, device="cuda", generator=g).to(dt)
+    rs, dv, width = MixerOps.latent_row(R, dr), 24, H * (dn + dr) + R + dr
+    qd, w, wuk, wuv, cache = rnd(B, (width + 7) // 8 * 8 + 8), rnd(R), rnd(H * dn, R), rnd(H * dv, R), rnd(B + 1, ring, rs)
+    inv = 10000.0 ** (-torch.arange(0, n_rot, 2, device="cuda") / n_rot)
+    sink, pos = torch.randn(H, device="cuda", generator=g), torch.arange(B, device="cuda") * 131 + 5
+    sizes = (H, dn, dr, dv, R, ring, 0.05)
+    if H * (dn + dr) % 8 or rs % 8:
+        assert not ops.latent_prep_fits(qd, cache, w, inv, H, dn, dr, R)
+        return
+    assert ops.latent_prep_fits(qd, cache, w, inv, H, dn, dr, R)
+    q2, c2, was = qd.clone(), cache.clone(), qd.clone()
+    got = ops.latent_decode(qd, cache, pos, wuk, wuv, sink, *sizes, prep=(w, inv, 1e-6))
+    ops.latent_prep(q2, H, dn, dr, R, w, inv, 1e-6, TokenBatch.of_decode(pos), c2, want_kv=False)
+    want = ops.latent_decode(q2, c2, pos, wuk, wuv, sink, *sizes)
+    assert torch.equal(qd, was) and torch.equal(cache, c2) and torch.equal(got, want)
