@@ -190,11 +190,12 @@ extern "C" int evo_latent_prep(void* q, int64_t ldq, void* c, void* kr, void* ca
 // PREP: q comes as the projection wrote it.  The heads' first workgroups rotate (the queries stay as they are), and one more "head" norms and rotates the tokens' own rows
 // for the cache, a wave a token: latent_prep and this in one launch, with the bits of two.  In a step of four layers, 8 sequences, 32 heads of 128 x 512: 11.8 us in two
 // launches with 128 workgroups' columns here, 7.4 so (3.1 of them the requests' latency, the map being cold); columns halved to 256 instead of 128 workgroups 0.4 to 1.3
-// (3 / 4 / 8 sequences 23.4 / 24.9 / 26.0 -> 22.2 / 23.6 / 25.6, all launches of the layer).
+// (3 / 4 / 8 sequences 23.4 / 24.9 / 26.0 -> 22.2 / 23.6 / 25.6, all launches of the layer).  Queries lie [dn][NB]: a row's are one LDS request instead of
+// NB (8 / 16 / 32 sequences 25.6 / 29.3 / 38.7 -> 25.2 / 28.6 / 38.3).
 template <typename T, int NB, int V, bool PREP>
 __global__ __launch_bounds__(512) void latent_absorb_kernel(const void* __restrict__ q_, int64_t ldq, const void* __restrict__ w_, void* __restrict__ out_,
                                                             int B, int H, int dn, int dr, int R, int rs, PrepArgs a) {
-    extern __shared__ float sm[];                                // q parts [NB][dn], partial sums [8][NB][64 V]
+    extern __shared__ __attribute__((aligned(16))) float sm[];   // q parts [dn][NB], partial sums [8][NB][64 V]
     constexpr int U = 16;                                        // rows of a wave in flight
     float* part = sm + NB * dn;
     const int h = blockIdx.y, b0 = blockIdx.z * NB, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -255,7 +256,7 @@ __global__ __launch_bounds__(512) void latent_absorb_kernel(const void* __restri
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i)
-        for (int n = tid; n < dn; n += 512) sm[i * dn + n] = i < nb ? ld1((const T*)q_ + (int64_t)(b0 + i) * ldq + (int64_t)h * dh + n) : 0.f;
+        for (int n = tid; n < dn; n += 512) sm[n * NB + i] = i < nb ? ld1((const T*)q_ + (int64_t)(b0 + i) * ldq + (int64_t)h * dh + n) : 0.f;
     __syncthreads();
     float acc[NB][V];
 #pragma unroll
@@ -266,12 +267,12 @@ __global__ __launch_bounds__(512) void latent_absorb_kernel(const void* __restri
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (n + 8 * u >= dn) break;
+            float q[NB];
+            vec_io<float, NB>::load(sm + (n + 8 * u) * NB, q);
 #pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                const float q = sm[i * dn + n + 8 * u];
+            for (int i = 0; i < NB; ++i)
 #pragma unroll
-                for (int e = 0; e < V; ++e) acc[i][e] = fmaf(f[u][e], q, acc[i][e]);
-            }
+                for (int e = 0; e < V; ++e) acc[i][e] = fmaf(f[u][e], q[i], acc[i][e]);
         }
         if (n + 8 * U < dn) fetch(n + 8 * U);
     }
@@ -756,7 +757,7 @@ __global__ __launch_bounds__(512) void latent_up_kernel(const float* __restrict_
 // read by several), and everything a thread needs is asked for together: statistics, its first 16 parts, the first 512 columns of the rows.
 // latent_absorb to here, 32 heads, R = 512, 900 slots, in a graph: 3 / 8 / 16 / 32 sequences 28.0 / 34.9 / 39.4 / 48.0 -> 23.8 / 27.9 / 29.9 / 36.7 us; of 64 x 128
 // 14.4 / 16.4 / 19.2 / 22.3 -> 14.4 / 15.9 / 17.4 / 20.3.  With the rows spread, the requests together and the preparation in
-// latent_absorb's launch, caches and maps cold, latent_prep to here: 1 / 3 / 8 / 16 / 32 sequences 21.9 / 27.7 / 32.2 / 34.5 / 39.9 -> 17.8 / 22.2 / 25.7 / 29.5 / 38.8 us.
+// latent_absorb's launch, caches and maps cold, latent_prep to here: 1 / 3 / 8 / 16 / 32 sequences 21.9 / 27.7 / 32.2 / 34.5 / 39.9 -> 17.7 / 21.6 / 25.2 / 28.6 / 38.3 us.
 template <int NS, int VR>
 __global__ __launch_bounds__(512) void latent_up_mfma_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, const float* __restrict__ sink,
                                                              const uint16_t* __restrict__ w, uint16_t* __restrict__ o, int B, int H, int R, int dv, int n_split) {
