@@ -246,12 +246,12 @@ class LayeredDecoder(DecodeGraphMixin, nn.Module):
         return all(self.ops.small_m_shape_ok(B, n, k) for n, k in shapes)
 
     # ------------------------------------------------------------------ forward
-    def _run(self, ids: torch.Tensor, batch: TokenBatch, ipd: Optional[dict]) -> torch.Tensor:
+    def _run(self, ids: torch.Tensor, batch: TokenBatch, ipd: Optional[dict], ids_known: bool = False) -> torch.Tensor:
         """Packed ids [M] -> final-norm hidden states [M, width] (logits = hidden @ head^T)."""
         if not self._loaded:
             raise RuntimeError(f"{type(self).__name__} has no weights: call load_state_dict first")
         ops = self.ops
-        stream = Stream(ops, ids.to(self.device), self.embed, self.embed_scale, self.eps, self.NORM_OFFSET, self.alpha)
+        stream = Stream(ops, ids.to(self.device), self.embed, self.embed_scale, self.eps, self.NORM_OFFSET, self.alpha, ids_known)
         taps = getattr(self, "block_taps", None)     # debugging / parity hook: residual stream entering every layer, then the final one
         for i, layer in enumerate(self.layers):
             if taps is not None:
@@ -265,8 +265,13 @@ class LayeredDecoder(DecodeGraphMixin, nn.Module):
             taps.append(stream.x.clone())
         return stream.final(self.final_norm)
 
-    def hidden_states(self, x: torch.Tensor, inference_params_dict=None, padding_mask=None) -> torch.Tensor:
-        """ids [B, T] -> final-norm hidden states [B T, width].  With records: the T tokens go on from `seqlen_offset`; one token per
+    @property
+    def embedding_rows(self) -> int:
+        """Rows of the embedding table: ids below are the ones that hidden_states takes."""
+        return self.embed.shape[0] if self._loaded else 0
+
+    def hidden_states(self, x: torch.Tensor, inference_params_dict=None, padding_mask=None, ids_known: bool = False) -> torch.Tensor:
+        """ids [B, T] -> final-norm hidden states [B T, width].  `ids_known`: the caller has checked that they lie in [0, embedding_rows).  With records: the T tokens go on from `seqlen_offset`; one token per
         row at the rows' own positions when the KV record carries a `pos_tensor`."""
         if x.dim() != 2:
             raise ValueError("input_ids must be [batch, length]")
@@ -274,7 +279,7 @@ class LayeredDecoder(DecodeGraphMixin, nn.Module):
             raise ValueError(f"{type(self).__name__} takes no padding mask: unequal prompts are packed (prefill_rows), pads behind a prompt are never seen by it")
         B, T = x.shape
         if inference_params_dict is None:
-            return self._run(x.reshape(-1), TokenBatch.of_prompts([T] * B, [0] * B, self.device), None)
+            return self._run(x.reshape(-1), TokenBatch.of_prompts([T] * B, [0] * B, self.device), None, ids_known)
         mha = inference_params_dict["mha"]
         pos = getattr(mha, "pos_tensor", None)
         off = int(mha.seqlen_offset)

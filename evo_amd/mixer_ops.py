@@ -51,9 +51,10 @@ class Stream:
     The norm of a sublayer's output y comes before the addition, x <- x + norm(y), or -- with `alpha` -- behind it, x <- norm(alpha x + y);
     norm(t) = t / rms(t) * (w_offset + w)."""
 
-    def __init__(self, ops, ids: torch.Tensor, weight: torch.Tensor, scale: float, eps: float, w_offset: float, alpha: Optional[float] = None):
+    def __init__(self, ops, ids: torch.Tensor, weight: torch.Tensor, scale: float, eps: float, w_offset: float, alpha: Optional[float] = None,
+                 ids_known: bool = False):
         self.ops, self.eps, self.w_offset, self.alpha = ops, eps, w_offset, alpha
-        self.x, self.xb = ops.embed_stream(ids, weight, scale)
+        self.x, self.xb = ops.embed_stream(ids, weight, scale, **({"validate": False} if ids_known else {}))
         self.open = None                                         # (y, w): still to be added
         self.spare = None                                        # the buffer the next such launch writes x to
         self.behind = False                                      # xb does not hold the current x
@@ -159,15 +160,15 @@ class MixerOps:
             _check(getattr(self.lib, name)(*args, _stream()), name)
 
     # ---- residual stream ------------------------------------------------------------------------------------------------
-    def embed_stream(self, ids: torch.Tensor, weight: torch.Tensor, scale: float) -> Tuple[torch.Tensor, torch.Tensor]:
-        """(x fp32 [M, D] = scale * weight[ids], the same in the storage type: x itself for fp32)."""
+    def embed_stream(self, ids: torch.Tensor, weight: torch.Tensor, scale: float, validate: bool = True) -> Tuple[torch.Tensor, torch.Tensor]:
+        """(x fp32 [M, D] = scale * weight[ids], the same in the storage type: x itself for fp32).  `validate=False`: the caller has checked the ids."""
         ids = ids.reshape(-1).to(torch.int64).contiguous()
         f32 = self._store(weight)
         V, D = weight.shape
         self._dense(weight, (V, D), "embedding table")
         x = torch.empty(ids.numel(), D, dtype=torch.float32, device=weight.device)
         xb = x if f32 else torch.empty(ids.numel(), D, dtype=torch.bfloat16, device=weight.device)
-        flag = None if torch.cuda.is_current_stream_capturing() or not self.validate_ids else \
+        flag = None if torch.cuda.is_current_stream_capturing() or not (self.validate_ids and validate) else \
             torch.zeros(1, dtype=torch.int32, device=weight.device)
         self._call("evo_embed_stream", self._ix(ids, torch.int64, ids.numel(), "ids"), weight.data_ptr(), x.data_ptr(), None if f32 else xb.data_ptr(),
                    ids.numel(), D, V, float(scale), None if flag is None else flag.data_ptr(), f32)

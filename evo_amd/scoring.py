@@ -19,6 +19,12 @@ def prepare_batch(seqs: List[str], tokenizer: CharLevelTokenizer, prepend_bos: b
                   device: str = "cuda:0") -> Tuple[torch.Tensor, List[int]]:
     """Tokenise, (optionally) prepend BOS = eod_id, right-pad with pad_id to the longest sequence.
     Returns (input_ids [B, T] int64 on `device`, list of sequence lengths)."""
+    ids, seq_lengths = _batch_ids(seqs, tokenizer, prepend_bos)
+    return torch.from_numpy(ids).to(device), seq_lengths
+
+
+def _batch_ids(seqs: List[str], tokenizer: CharLevelTokenizer, prepend_bos: bool) -> Tuple[np.ndarray, List[int]]:
+    """prepare_batch's ids, on the host."""
     seq_lengths = [len(s) for s in seqs]
     longest = max(seq_lengths)
     bos = int(prepend_bos)
@@ -34,7 +40,17 @@ def prepare_batch(seqs: List[str], tokenizer: CharLevelTokenizer, prepend_bos: b
         ids[:, 0] = tokenizer.eod_id
     for i, r in enumerate(rows):
         ids[i, bos:bos + r.size] = r
-    return torch.from_numpy(ids).to(device), seq_lengths
+    return ids, seq_lengths
+
+
+def _scorer_batch(seqs: List[str], model, tokenizer: CharLevelTokenizer, device: str):
+    """A scorer's batch -> (ids on the device, sequence lengths, whether every id has a row of the model's embedding table).  Ids that the host has looked at
+    need no flag of the embedding's launch, whose read-back is a wait before the first layer: a pass over 161 tokens of four
+    layers 748 -> 727 us (its launches of the flag, and of the targets that entropies do not need, among it)."""
+    ids, seq_lengths = _batch_ids(seqs, tokenizer, True)
+    rows = getattr(model, "embedding_rows", None)
+    known = rows is not None and ids.size > 0 and int(ids.min()) >= 0 and int(ids.max()) < rows
+    return torch.from_numpy(ids).to(device), seq_lengths, known
 
 
 def _ops_for(t: torch.Tensor):
@@ -69,20 +85,22 @@ def _fused_tail_ok(model, input_ids) -> bool:
             and ops.unembed_logprob_ok(model.unembed.weight.new_empty(1, model.hidden_size), model.unembed.weight))
 
 
-def score_logprobs_device(model, input_ids: torch.Tensor, want_entropy: bool = False):
+def score_logprobs_device(model, input_ids: torch.Tensor, want_entropy: bool = False, ids_known: bool = False):
     """What `score_sequences` / `positional_entropies` compute on the device for a BOS-prefixed id matrix [B, T]:
     (log-prob of token t+1 at position t  [B, T-1] f32 | None, entropy of the next-token distribution [B, T-1] f32 |
     None).  On the MI355X engine the unembedding and then the log-softmax, the gather
     and the entropy run over chunks of rows and the [B, T, 512] logits are never held as a whole; any other model object takes
-    model(ids) -> logits_to_logprobs like the reference [REF evo/scoring.py:80-84,116-121]."""
+    model(ids) -> logits_to_logprobs like the reference [REF evo/scoring.py:80-84,116-121].  `ids_known`: the caller has checked them."""
     B, T = input_ids.shape
     if _fused_tail_ok(model, input_ids):
         with torch.no_grad():
-            hid = model.hidden_states(input_ids)                       # [B*T, D] final-norm output
-            tgt = torch.full((B, T), -1, dtype=torch.int64, device=hid.device)
-            tgt[:, :-1] = input_ids[:, 1:].to(hid.device)
-            lp, en = model.ops.unembed_logprob(hid, model.unembed.weight, tgt.reshape(-1),
-                                               want_logprob=not want_entropy, want_entropy=want_entropy)
+            hid = model.hidden_states(input_ids, **({"ids_known": True} if ids_known else {}))      # [B*T, D] final-norm output
+            tgt = None
+            if not want_entropy:
+                tgt = torch.full((B, T), -1, dtype=torch.int64, device=hid.device)
+                tgt[:, :-1] = input_ids[:, 1:].to(hid.device)
+                tgt = tgt.reshape(-1)
+            lp, en = model.ops.unembed_logprob(hid, model.unembed.weight, tgt, want_logprob=not want_entropy, want_entropy=want_entropy)
         return (None if lp is None else lp.view(B, T)[:, :-1]), (None if en is None else en.view(B, T)[:, :-1])
     logits, _ = model(input_ids)
     if not want_entropy:
@@ -112,20 +130,20 @@ def score_sequences(seqs: List[str], model, tokenizer: CharLevelTokenizer, reduc
     """Mean (or sum) per-token log-likelihood of each sequence under the model."""
     if reduce_method not in ("mean", "sum"):
         raise ValueError(f"Invalid reduce_method {reduce_method}")
-    input_ids, seq_lengths = prepare_batch(seqs, tokenizer, device=device, prepend_bos=True)
+    input_ids, seq_lengths, known = _scorer_batch(seqs, model, tokenizer, device)
     assert len(seq_lengths) == input_ids.shape[0]
     with torch.inference_mode():
-        logprobs, _ = score_logprobs_device(model, input_ids)          # (batch, length - 1)
+        logprobs, _ = score_logprobs_device(model, input_ids, ids_known=known)          # (batch, length - 1)
     return _reduce(logprobs.float().cpu().numpy(), seq_lengths, reduce_method)
 
 
 def positional_entropies(seqs: List[str], model, tokenizer: CharLevelTokenizer,
                          device: str = "cuda:0") -> List[np.ndarray]:
     """Per-position entropy of the next-token distribution, one array (len(seq)) per sequence."""
-    input_ids, seq_lengths = prepare_batch(seqs, tokenizer, device=device, prepend_bos=True)
+    input_ids, seq_lengths, known = _scorer_batch(seqs, model, tokenizer, device)
     assert len(seq_lengths) == input_ids.shape[0]
     with torch.inference_mode():
-        _, ent = score_logprobs_device(model, input_ids, want_entropy=True)
+        _, ent = score_logprobs_device(model, input_ids, want_entropy=True, ids_known=known)
     ent = ent.float().cpu().numpy()
     out = [ent[i][: seq_lengths[i]] for i in range(len(seq_lengths))]
     assert all(len(s) == len(e) for s, e in zip(seqs, out))

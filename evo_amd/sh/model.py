@@ -760,8 +760,13 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             n += 1
         return split(n0)
 
-    def hidden_states(self, x: torch.Tensor, inference_params_dict=None, padding_mask=None) -> torch.Tensor:
-        """ids [B,T] -> final-norm hidden states [B*T, D] (logits = hidden @ E^T)."""
+    @property
+    def embedding_rows(self) -> int:
+        """Rows of the embedding table: ids below are the ones that hidden_states takes."""
+        return self.embedding_layer.weight.shape[0]
+
+    def hidden_states(self, x: torch.Tensor, inference_params_dict=None, padding_mask=None, ids_known: bool = False) -> torch.Tensor:
+        """ids [B,T] -> final-norm hidden states [B*T, D] (logits = hidden @ E^T).  `ids_known`: the caller has checked that they lie in [0, embedding_rows)."""
         if not self._packed:
             self._pack()
         if x.dim() != 2:
@@ -775,13 +780,13 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             out, b0 = None, 0
             for nb in groups:
                 pm = None if padding_mask is None else padding_mask[b0:b0 + nb]
-                hg = self.hidden_states(x[b0:b0 + nb], None, pm)
+                hg = self.hidden_states(x[b0:b0 + nb], None, pm, ids_known)
                 if out is None:
                     out = torch.empty(B * T, hg.shape[1], dtype=hg.dtype, device=hg.device)
                 out[b0 * T:(b0 + nb) * T] = hg
                 b0 += nb
             return out
-        h = ops.embed(x.to(self.device), self.embedding_layer.weight)             # [B*T, D]
+        h = ops.embed(x.to(self.device), self.embedding_layer.weight, **({"validate": False} if ids_known else {}))             # [B*T, D]
         mask = None
         if padding_mask is not None:
             pm = padding_mask.to(self.device) != 0

@@ -107,3 +107,25 @@ def test_fixes_over_reference():
     assert a == b == c
     np.testing.assert_allclose(sa, sb, rtol=1e-6)
     np.testing.assert_allclose(sb, sc, rtol=1e-6)
+
+
+@pytest.mark.parametrize("rows,known", [(512, True), (85, True), (84, False), (None, False)])
+def test_scorers_look_at_ids_on_the_host(rows, known):
+    """Ids below the embedding table's rows need no check on the device; others, and models that do not say how many rows there are, keep it."""
+    import types
+    from evo_amd import scoring
+    asked = []
+
+    class Model(types.SimpleNamespace):
+        def hidden_states(self, ids, **kw):
+            asked.append(kw)
+            return torch.zeros(ids.numel(), 4)
+    ops = types.SimpleNamespace(name="hip-gfx950", unembed_logprob_ok=lambda h, e: True,
+                                unembed_logprob=lambda h, e, t, want_logprob, want_entropy: (torch.zeros(len(h)), torch.zeros(len(h)) if want_entropy else None))
+    m = Model(ops=ops, hidden_size=4, unembed=types.SimpleNamespace(weight=torch.zeros(512, 4)))
+    if rows is not None:
+        m.embedding_rows = rows
+    tok = CharLevelTokenizer(512)
+    assert [len(e) for e in scoring.positional_entropies(["ACGT", "AC"], m, tok, device="cpu")] == [4, 2]
+    assert len(scoring.score_sequences(["ACGT", "AC"], m, tok, device="cpu")) == 2
+    assert asked == [{"ids_known": True} if known else {}] * 2
