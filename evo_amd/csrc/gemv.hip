@@ -1197,37 +1197,45 @@ static int ring_go(dim3 grid, const void* x, const void* w, const void* bias, co
                        (const uint16_t*)res, (uint16_t*)y, (int)M, (int)N, (int)K, act, layout, ws);
     return evo_launch_status();
 }
-static int64_t ring_groups(int64_t N) {
+// 4,097 to 7,680 columns from K = 4,096 on (to 7,168: from 2,048): a workgroup per CU here too, of 17 to 30 columns in two waves.  A CU takes in 45 to 55 GB/s while lines come
+// from memory, however many are under way, and 132 to 240 workgroups left the others idle (and, to 16 rows, six stages of their 12 KB: 36 KB under way are too few).  Four
+// stages and 32 columns -> this, us at 5 / 16 / 24 / 32 rows: 4,224 x 4,096 11.1 / 11.0 / 12.1 / 12.5 -> 10.4 / 10.3 / 12.2 / 12.3, 6,144 x 4,096 13.2 / 13.1 / 12.9 / 13.5 ->
+// 11.0 / 11.4 / 12.5 / 12.7, 6,720 x 4,096 13.5 / 13.1 / 13.4 / 14.0 -> 11.5 / 11.9 / 12.6 / 13.2, x 11,008 29.3 / 30.1 / 32.6 / 32.1 -> 26.4 / 27.4 / 31.0 / 32.7; 33 to 64 rows
+// 1.00 to 1.04.  Beyond, 31 and 32 columns a workgroup are as good (8,000 x 4,096 14.2 : 14.6), and at small K nothing is gained (6,144 x 1,024 4.9 : 5.0,
+// 7,680 x 2,048 7.5 : 7.7).
+static bool ring_spread(int64_t N, int64_t K) { return N > 4096 && (N <= 7168 ? K >= 2048 : N <= 7680 && K >= 4096); }
+static int64_t ring_groups(int64_t N, int64_t K) {
     const int64_t share = (N + 31) / 32;
-    return share < 256 ? share : N <= 256 * 96 ? 256 : 256 * ((N + 256 * 64 - 1) / (256 * 64));
+    return ring_spread(N, K) ? 256 : share < 256 ? share : N <= 256 * 96 ? 256 : 256 * ((N + 256 * 64 - 1) / (256 * 64));
 }
-static int ring_waves(int64_t N) {
-    const int64_t groups = ring_groups(N), rows = (N + groups - 1) / groups;
+static int ring_waves(int64_t N, int64_t K) {
+    const int64_t groups = ring_groups(N, K), rows = (N + groups - 1) / groups;
     return rows <= 32 ? 2 : rows <= 48 ? 3 : rows <= 64 ? 4 : 6;
 }
 // What workgroup `block` of N weight rows (gated: N / 2 result columns) takes: out = workgroups, its first column, the next one's, columns that it has room for
 extern "C" int evo_linear_ring_share(int64_t N, int64_t gated, int64_t block, int64_t* out) {
     if (!out || N <= 0 || N > 0x7fffffff - 16 || (gated && N % 2)) return -1;
-    const int64_t groups = ring_groups(N), cols = gated ? N / 2 : N;
+    const int64_t K = 4096, groups = ring_groups(N, K), cols = gated ? N / 2 : N;     // (any K from 4,096 on)
     if (block < 0 || block >= groups) return -1;
     out[0] = groups;
     out[1] = ring_edge((uint32_t)cols, (uint32_t)groups, (uint32_t)block);
     out[2] = ring_edge((uint32_t)cols, (uint32_t)groups, (uint32_t)block + 1);
-    out[3] = (gated ? 8 : 16) * ring_waves(N);
+    out[3] = (gated ? 8 : 16) * ring_waves(N, K);
     return 0;
 }
 // parts > 0: MODE 2, 64 rows a workgroup (N a multiple of 64)
 template <int MODE>
 static int ring_launch(const void* x, const void* w, const void* bias, const void* res, void* y, int64_t M, int64_t N, int64_t K, int act, int layout, float* ws, int parts,
                        hipStream_t s) {
-    const int waves = ring_waves(N);
-    const dim3 grid((unsigned)(parts ? N / 64 : ring_groups(N)), (unsigned)(parts ? parts : 1));
+    const int waves = ring_waves(N, K);
+    const dim3 grid((unsigned)(parts ? N / 64 : ring_groups(N, K)), (unsigned)(parts ? parts : 1));
 #define EVO_RG(XR, T, NB) ring_go<XR, T, MODE, NB>(grid, x, w, bias, res, y, M, N, K, act, layout, ws, s)
 #define EVO_RG1(T) (M <= 16 ? EVO_RG(16, T, 4) : M <= 32 ? EVO_RG(32, T, 4) : EVO_RG(64, T, (T == 6 ? 3 : 4)))
 #define EVO_RGN(T) (M <= 16 ? EVO_RG(16, T, 3) : M <= 32 ? EVO_RG(32, T, 3) : EVO_RG(64, T, 2))
     if constexpr (MODE == 2) return EVO_RG1(4);
     else {
         if (grid.x > 256) return waves == 3 ? EVO_RGN(3) : EVO_RGN(4);         // (33 to 64 rows)
+        if (M <= 16 && ring_spread(N, K)) return EVO_RG(16, 2, 6);
         return waves == 2 ? EVO_RG1(2) : waves == 3 ? EVO_RG1(3) : waves == 4 ? EVO_RG1(4) : EVO_RG1(6);
     }
 #undef EVO_RGN

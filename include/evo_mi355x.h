@@ -293,7 +293,7 @@ int evo_attn_decode_bf16(const void* q, const void* k, const void* v, void* o,
 int evo_linear_small_m_bf16(const void* x, const void* w, const void* bias, const void* residual, void* y,
                             int64_t M, int64_t N, int64_t K, void* ws, int64_t ws_bytes, int64_t act, void* stream);
 
-/* Columns per workgroup of that launch on a wide layer (N > 4096, K % 128 == 0) and of the gated one (`gated`: N = 2 I, I columns): out [4] = workgroups, first column of workgroup
+/* Columns per workgroup of that launch on a wide layer (N > 4096, K % 128 == 0 and, for 4,097 to 7,680 columns, K >= 4096) and of the gated one (`gated`: N = 2 I, I columns): out [4] = workgroups, first column of workgroup
  * `block`, first behind it, columns that a workgroup has room for.  On the host, no launch; -1: no such workgroup. */
 int evo_linear_ring_share(int64_t N, int64_t gated, int64_t block, int64_t* out);
 

@@ -52,6 +52,19 @@ def test_linear_in_rounds_and_parts(M, N, K, few, many):
     assert torch.equal(r[M], keep[M]) and bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + 1e-3).all())
 
 
+# a workgroup per CU on 4,097 to 7,680 columns: shares of 16 and 17, 28, 29 and 30 columns, stages that outnumber nothing, chunks that are few against the starts; the sizes beside
+@pytest.mark.parametrize("M", [5, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(4097, 2048), (4112, 2176), (7168, 2048), (7169, 2048), (7169, 4096), (7680, 4096), (7681, 4096), (6721, 1920)])
+def test_linear_spread(M, N, K):
+    test_linear(M, N, K, True)
+
+
+@pytest.mark.parametrize("M", [5, 16, 17, 64])
+@pytest.mark.parametrize("I,K", [(2064, 2048), (2080, 4096), (3584, 2048), (3616, 4096), (3840, 4096)])
+def test_gate_spread(M, I, K):
+    test_gate(M, I, K, I % 32 == 0)
+
+
 @pytest.mark.parametrize("M", [3, 5, 16, 17, 33, 64])
 @pytest.mark.parametrize("I,K", [(32, 128), (96, 384), (2080, 256), (5504, 1152), (8224, 2176), (12320, 1408), (16416, 256)])
 @pytest.mark.parametrize("grouped", [False, True])
