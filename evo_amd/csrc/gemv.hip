@@ -881,7 +881,7 @@ __global__ __launch_bounds__(512) void skinny_mfma_kernel(const uint4* __restric
 // K = 16,384 [22.0] 28.5 / 29.9 / 33.3 -> 22.8 / 22.3 / 29.3.
 // XR: batch rows loaded (8, 16 or 32; rows behind M read as zero or are a repeated row, and are never stored).
 #define KW_WAIT(N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory")
-template <int XR, int WAVES, int CH, int NB>
+template <int XR, int WAVES, int CH, int NB, int EP>
 __global__ __launch_bounds__(64 * WAVES) void skinny_kw_kernel(const unsigned char* __restrict__ x, const unsigned char* __restrict__ w,
                                                                const uint16_t* __restrict__ bias, const uint16_t* res, uint16_t* y, int M, int N, int K,
                                                                int act) {   // res may alias y
@@ -903,6 +903,23 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kw_kernel(const unsigned ch
     for (int i = 0; i < (PX > PW ? PX : PW); ++i) {
         const int r = i * RPI + lane / GR;
         off[i] = (uint32_t)r * rowb + (uint32_t)((lane % GR) ^ (r & 15 & (GR - 1))) * 16u;
+    }
+    // EP: bias and residual values of the waves that end with results, requested ahead of everything (from places that are there; `EP` 2: four at a time) and looked at behind the
+    // last product: asked for there they were a memory latency of their own at the end (4,096 x 4,096 with both, 5 / 16 / 32 rows 8.4 / 9.3 / 11.4 -> 7.5 / 8.1 / 10.0 us, K = 11,008
+    // 17.8 / 18.9 -> 16.7 / 17.7; one value a request 7.7 / 8.4 / 10.3, behind the first chunks 8.1 / 9.0 / 10.8).  Without either they are not in the code: 7.25 -> 7.1.
+    uint2 pb = {}, pr = {};
+    if (EP && wave < MT) {
+        const int m = 16 * wave + r16, nq = n0 + 4 * kb;
+        const uint16_t* from = res + (int64_t)(m < M ? m : M - 1) * N;
+        auto four = [&](const uint16_t* p) {
+            if constexpr (EP == 2) return *(const uint2*)(p + (nq < N ? nq : 0));
+            uint32_t v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = p[nq + r < N ? nq + r : N - 1];
+            return make_uint2(v[0] | v[1] << 16, v[2] | v[3] << 16);
+        };
+        if (bias) pb = four(bias);
+        if (res) pr = four(from);
     }
     const int chunks = K / CH, mine = (chunks - wave + WAVES - 1) / WAVES;
     const int start = mine > 4 && gridDim.x >= 128 ? (int)(blockIdx.x >> 3) * 3 % mine : 0;       // (workgroups of an XCD don't walk K in step: skinny_ring_kernel)
@@ -971,8 +988,9 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kw_kernel(const unsigned ch
             for (int r = 0; r < 4; ++r) {
                 const int n = n0 + 4 * kb + r;
                 if (n < N) {
-                    float o = a_[r] + (bias ? bf_to_f(bias[n]) : 0.f);
-                    if (res) o += bf_to_f(res[(int64_t)m * N + n]);
+                    auto one = [&](uint2 v) { const uint32_t h = r < 2 ? v.x : v.y; return r & 1 ? bf_hi(h) : bf_lo(h); };
+                    float o = a_[r] + (EP && bias ? one(pb) : 0.f);
+                    if (EP && res) o += one(pr);
                     y[(int64_t)m * N + n] = f_to_bf(out_act(o, act));
                 }
             }
@@ -980,14 +998,21 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kw_kernel(const unsigned ch
     }
 }
 
-template <int XR, int WAVES, int CH, int NB>
-static int kw_launch(const void* x, const void* w, const void* bias, const void* residual, void* y, int64_t M, int64_t N, int64_t K, int act, hipStream_t s) {
+template <int XR, int WAVES, int CH, int NB, int EP>
+static int kw_go(const void* x, const void* w, const void* bias, const void* residual, void* y, int64_t M, int64_t N, int64_t K, int act, hipStream_t s) {
     constexpr size_t lds = (size_t)WAVES * NB * (16 + XR) * 2 * CH;
     static_assert(lds <= 160 * 1024, "the CU's LDS");
-    if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)skinny_kw_kernel<XR, WAVES, CH, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL((skinny_kw_kernel<XR, WAVES, CH, NB>), dim3((unsigned)((N + 15) / 16)), dim3(64 * WAVES), lds, s, (const unsigned char*)x,
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)skinny_kw_kernel<XR, WAVES, CH, NB, EP>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL((skinny_kw_kernel<XR, WAVES, CH, NB, EP>), dim3((unsigned)((N + 15) / 16)), dim3(64 * WAVES), lds, s, (const unsigned char*)x,
                        (const unsigned char*)w, (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)K, act);
     return evo_launch_status();
+}
+// (a form of its own for layers without bias and residual: the requests in front of their loop cost 0.2 to 0.3 us there)
+template <int XR, int WAVES, int CH, int NB>
+static int kw_launch(const void* x, const void* w, const void* bias, const void* residual, void* y, int64_t M, int64_t N, int64_t K, int act, hipStream_t s) {
+    if (!bias && !residual) return kw_go<XR, WAVES, CH, NB, 0>(x, w, bias, residual, y, M, N, K, act, s);
+    if (N % 4 == 0 && (((uintptr_t)bias | (uintptr_t)residual) & 7) == 0) return kw_go<XR, WAVES, CH, NB, 2>(x, w, bias, residual, y, M, N, K, act, s);
+    return kw_go<XR, WAVES, CH, NB, 1>(x, w, bias, residual, y, M, N, K, act, s);
 }
 
 // ---- 3 to 64 rows on the wide layers (and, with parts of K, on those of up to 8,192 columns from 17 rows on): a workgroup owns N / gridDim.x weight rows (any number up to

@@ -127,3 +127,27 @@ def test_rows_off_16_bytes():
     gate = torch.nn.functional.gelu(u) * v
     assert ((ops.mlp_gate(x, w).double() - gate).norm() / gate.norm()).item() < 4e-3
     assert torch.equal(ops.mlp_gate(x, None, w12g=ops.pack_gate_weights(w)), ops.mlp_gate(x.clone(), w))     # (copied to a place that they can)
+
+
+# layers of up to 4,096 columns at 3 to 32 rows: bias and residual four values a request, and one (odd columns, addresses two bytes on), each without the other
+@pytest.mark.parametrize("M", [3, 8, 9, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(4096, 2048), (4094, 2048), (2052, 2176), (2049, 4096), (516, 1024), (20, 256)])
+@pytest.mark.parametrize("odd", [0, 1])
+def test_narrow_epilogue(M, N, K, odd):
+    from evo_amd.ops import default_ops
+    ops = default_ops()
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x, w = _framed(M, K, g), _framed(N, K, g, K ** -0.5)
+    plain = x.double() @ w.double().T
+    b = torch.randn(N + 1, device=DEV, generator=g).bfloat16()[odd:odd + N]
+    for bias in (None, b):
+        for with_res in (False, True):
+            if not with_res and bias is None:
+                continue
+            r = torch.randn(M * N + N + 1, device=DEV, generator=g).bfloat16()
+            keep, res = r.clone(), r[odd:odd + M * N].view(M, N) if with_res else None
+            want = plain + (0 if bias is None else bias.double()) + (keep[odd:odd + M * N].view(M, N).double() if with_res else 0)
+            got = ops._linear_small_m(x, w, bias, res)
+            assert bool(((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + 1e-3).all())
+            if with_res:
+                assert got.data_ptr() == res.data_ptr() and torch.equal(r[odd + M * N:], keep[odd + M * N:]) and torch.equal(r[:odd], keep[:odd])
