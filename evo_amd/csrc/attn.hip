@@ -665,8 +665,10 @@ __global__ __launch_bounds__(256) void attn_decode_stream_kernel(AttnArgs a, int
     const gptr_t vp = (gptr_t)(uint64_t)(a.v + bat * a.v_sb + head * a.v_sh);
     const uint32_t kst = (uint32_t)(a.k_st * 2), vst = (uint32_t)(a.v_st * 2), dco = (uint32_t)dc * 16;
     typedef unsigned int attn_u32x4 __attribute__((ext_vector_type(4)));
+    // (non-temporal: whole rows that nobody reads again.  us with the merge: 1 x 3,000 / 30,000 / 131,000 keys 16.6 / 90.6 / 364 -> 14.8 / 81.7 / 331, 16 x 700 40.4 -> 36.0, 5 x 100
+    // 9.0 -> 8.3)
     auto ld16 = [](gptr_t base, uint32_t off) {
-        const attn_u32x4 t = *(const __attribute__((address_space(1))) attn_u32x4*)(base + off);
+        const attn_u32x4 t = __builtin_nontemporal_load((const __attribute__((address_space(1))) attn_u32x4*)(base + off));
         return make_uint4(t[0], t[1], t[2], t[3]);
     };
     float m_run = -INFINITY, l_run = 0.f;

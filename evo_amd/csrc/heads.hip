@@ -267,11 +267,13 @@ __global__ __launch_bounds__(256) void heads_decode_kernel(HDecArgs a) {
                 }
         }
     };
-    auto load_v = [&](int s0) __attribute__((always_inline)) {   // item: eight values of a slot
+    // item: eight values of a slot.  A request is whole lines that nobody reads again (non-temporal: 239 / 526 MB of keys and values 58.7 / 104 -> 56.8 / 97.9 us, one map 17.0 /
+    // 28.9 -> 16.1 / 26.7 at 60 / 119 MB); the keys' requests are halves of lines, which have to be there for the other half (the same for them: 2 to 17 % slower)
+    auto load_v = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 2 * NG; ++i) {
             const int it = lane + 64 * i, r = s0 + it / (4 * NG), d = 8 * (it % (4 * NG));
-            rv[i] = *(const mx_u32x4*)(vbase + (int64_t)(r < used ? r : last) * a.rs + (d < dv ? d : dv - 8));
+            rv[i] = __builtin_nontemporal_load((const mx_u32x4*)(vbase + (int64_t)(r < used ? r : last) * a.rs + (d < dv ? d : dv - 8)));
         }
     };
     const int step = a.n_split * 128;
