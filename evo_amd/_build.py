@@ -29,12 +29,12 @@ ARCH = "gfx950"
 # component -> (suffix of the library's name, sources, headers beside common.h, the symbols of include/evo_mi355x.h it exports)
 COMPONENTS = {
     "core": ("", ["elementwise", "gemm", "gemm_rows160", "gemm_rows192", "gemm_rows224", "gemm_tile", "gemm_f32", "gemm_f32_ahead", "gemv", "gemv_f32", "score_tail", "probe"], ["gemm_args.h", "gemm_kernel.h", "gemm_f32.h"], [
-        "evo_abi_version", "evo_embed_bf16", "evo_rmsnorm_bf16", "evo_rmsnorm_rows_bf16", "evo_rms_finalize_f32", "evo_rope_qk_bf16",
+        "evo_abi_version", "evo_embed_bf16", "evo_rmsnorm_bf16", "evo_rmsnorm_rows_bf16", "evo_rmsnorm_parts_bf16", "evo_rms_finalize_f32", "evo_rope_qk_bf16",
         "evo_rope_append_decode_bf16", "evo_gelu_gate_bf16", "evo_logprob_entropy", "evo_unembed_logprob_bf16",
         "evo_linear_small_m_bf16", "evo_norm_linear_small_m_bf16", "evo_mlp_gate_small_m_bf16", "evo_norm_mlp_gate_small_m_bf16",
         "evo_hyena_decode_fused_small_m", "evo_linear_mfma_bf16", "evo_linear_mfma_nf_bf16", "evo_mlp_gate_mfma_bf16",
         "evo_mlp_gate_mfma_nf_bf16", "evo_linear_xblk_mfma_bf16", "evo_linear_xblk_mfma_nf_bf16", "evo_linear_t_mfma_bf16",
-        "evo_linear_t_mfma_nf_bf16", "evo_linear_act_mfma_bf16", "evo_dense_ws", "evo_dense_launches", "evo_dense_plan", "evo_dense_bf16", "evo_linear_f32_ws", "evo_linear_f32_plan", "evo_linear_f32", "evo_linear_f32_ahead_plan", "evo_linear_f32_ahead", "evo_linear_few_f32", "evo_put_tokens",
+        "evo_linear_t_mfma_nf_bf16", "evo_linear_act_mfma_bf16", "evo_dense_ws", "evo_dense_parts", "evo_dense_parts_bf16", "evo_dense_launches", "evo_dense_plan", "evo_dense_bf16", "evo_linear_f32_ws", "evo_linear_f32_plan", "evo_linear_f32", "evo_linear_f32_ahead_plan", "evo_linear_f32_ahead", "evo_linear_few_f32", "evo_put_tokens",
         "evo_advance_positions", "evo_step_out", "evo_copy_rows", "evo_linear_ring_share", "evo_linear_parts", "evo_linear_parts_bf16", "evo_postnorm_linear_small_m_bf16",
         "evo_postnorm_mlp_gate_small_m_bf16", "evo_probe_copy_f4", "evo_probe_mfma_bf16",
     ]),

@@ -686,8 +686,9 @@ static int tile_phases(int kind, int mode, bool xblk, int splits, int64_t M, int
     return 0;
 }
 
+// `add`: the launch that adds the parts too
 template <int BM, int BN, int WGM, int WGN, int NS, int PER_CU, bool GATE>
-static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, float* ws, hipStream_t st) {
+static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, float* ws, hipStream_t st, bool add = true) {
     a.tiles_m = (int)((a.M + BM - 1) / BM);
     a.tiles_n = (a.N + BN - 1) / BN;
     a.group_m = 8;
@@ -713,6 +714,7 @@ static int tile_launch(GemmArgs a, int mode, int act, bool xblk, int splits, flo
     else if (xblk) T_GO(0, true, true);
     else T_GO(0, false, true);
 #undef T_GO
+    if (!add) return evo_launch_status();
     const int64_t threads = a.M * ((mode == 1 ? a.N / 2 : a.N) / 8);
     const dim3 rgrid((unsigned)((threads + 255) / 256)), rblock(256);
     if (mode == 3) hipLaunchKernelGGL(gemm_parts_kernel<3>, rgrid, rblock, 0, st, a, act, ws, splits);
@@ -782,6 +784,48 @@ extern "C" int evo_dense_plan(int64_t mode, int64_t stats, int64_t M, int64_t N,
     for (int i = 0; i < n; ++i)
         for (int k = 0; k < 7; ++k) out[7 * i + k] = row[8 * i + k];
     return n;
+}
+
+// Parts of K that the norm behind a layer adds (rmsnorm_parts_kernel, closing_parts_kernel), 65 to 1,023 rows and up to 8,192 columns: without a launch of their own (5.5 us at 161 rows)
+// parts pay in more layers and in larger numbers.  us, layer and norm in their own launches -> parts and norm, K = 4,096, 11,008 and 16,384 of 4,096 columns: 65 rows 20.5 -> 17.0,
+// 33.9 -> 28.6, 39.3 -> 35.0; 161 rows 23.2 -> 22.3, 38.6 -> 36.3, 46.8 -> 44.2; 512 rows 39.1 -> 33.8, 64.3 -> 63, 81.5 -> 78.5; 8,192 x 8,192 56.4 -> 45.8 at 161 rows, 84 -> 81 at 512; over 400
+// layers of 512 to 8,192 columns 1.12 x with rmsnorm_parts_kernel, over 169 1.11 x with closing_parts_kernel, 11 of them 1 to 3 % behind (4,096 x 4,096 at 540 rows 38.2 : 39.1).
+// `parts_us`, fitted to 2,100 launches (5 % off them): the k-steps of a part, the parts' bytes, written and read, and the weights'; two, four and eight parts start a power of two
+// apart and meet in the L2's channels.  One round of the chip; parts of 64 x 64 tiles as far as they have a CU each, eight of 192 rows on never (7 : 8 at K = 16,384 44 : 50).
+struct PartsUs { int kind; double us, base; };
+static const PartsUs parts_us[] = {{0, 0.21, 6.0}, {2, 0.43, 6.6}, {3, 0.55, 5.5}, {4, 0.665, 4.4}};
+static TilePlan parts_plan(int64_t M, int64_t N, int64_t K) {
+    TilePlan best = {-1, 0, 1e30, M}, own[2];
+    // (narrow rows leave the norm's threads idle: 512 x 1,024 8.8 -> 10.4 at 540 rows, 1,024 x 4,096 18.8 -> 21.8 at 870)
+    if (M < 65 || M >= 1024 || N > 8192 || (N < 2048 && 2 * M > N) || !dense_shape(0, M, N, K)) return best;
+    const double cus = tile_cus(), nk = (double)(K / 64), power = 2.2e-9 * (double)M * N * K / 1.56;
+    for (const PartsUs& p : parts_us) {
+        const double tiles = (double)((M + kinds[p.kind].bm - 1) / kinds[p.kind].bm) * (double)((N + kinds[p.kind].bn - 1) / kinds[p.kind].bn);
+        for (int s = 2; s <= 8 && tiles * s <= cus && nk / s >= 8 && (s < 8 || p.kind < 3); ++s) {
+            const double us = ceil(nk / s) * p.us + p.base + 0.58e-6 * (double)(s * M * N * 4) + ((s & (s - 1)) == 0 ? 0.081e-6 : 0.066e-6) * (double)(N * K * 2);
+            if (us < best.us) best = {p.kind, s, us, M};
+        }
+    }
+    const int n = dense_plan(0, false, M, N, K, true, false, own);
+    const double apart = 1.1 * (n == 2 ? own[0].us + own[1].us + 4.0 : own[0].us) + 1.3 + 0.47e-6 * (double)(M * N * 2);
+    if (fmax(best.us, power) > 0.97 * apart) best.splits = 0;
+    return best;
+}
+
+extern "C" int evo_dense_parts(int64_t M, int64_t N, int64_t K) { return parts_plan(M, N, K).splits; }
+
+extern "C" int evo_dense_parts_bf16(const void* x, const void* w, float* ws, int64_t M, int64_t N, int64_t K, int64_t parts, void* stream) {
+    const TilePlan t = parts_plan(M, N, K);
+    if (!x || !w || !ws || parts < 2 || parts != t.splits || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)ws) & 15)) return -1;
+    GemmArgs a;
+    a.x = (const unsigned char*)x; a.w = (const unsigned char*)w; a.bias = nullptr; a.res = nullptr; a.y = nullptr;
+    a.M = M; a.N = (int)N; a.K = (int)K;
+    a.turn = M < 256 && K > 2048 ? 1 : 0;
+    hipStream_t st = (hipStream_t)stream;
+    if (t.kind == 0) return tile_launch<64, 64, 2, 2, 5, 2, false>(a, 0, 0, false, t.splits, ws, st, false);
+    if (t.kind == 2) return tile_launch<128, 128, 4, 2, 5, 1, true>(a, 0, 0, false, t.splits, ws, st, false);
+    if (t.kind == 3) return tile_launch<192, 128, 4, 2, 4, 1, true>(a, 0, 0, false, t.splits, ws, st, false);
+    return tile_launch<256, 128, 4, 2, 3, 1, true>(a, 0, 0, false, t.splits, ws, st, false);
 }
 
 extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const void* x, const void* w, const void* bias, const void* residual, void* y,

@@ -310,7 +310,7 @@ __global__ __launch_bounds__(512) void latent_absorb_kernel(const void* __restri
 // prep: null, or the preparation's arguments
 static int latent_absorb(const void* q, int64_t ldq, const void* wuk, void* out, int64_t B, int64_t H, int64_t dn, int64_t dr, int64_t R, int64_t rs, const PrepArgs* prep,
                          int64_t f32, void* stream) {
-    if (!q || !wuk || !out || B <= 0 || H <= 0 || H > 65534 || dn <= 0 || dn > 4096 || dr < 0 || R <= 0 || rs < R + dr || ldq < H * (dn + dr)) return -1;
+    if (!q || !wuk || !out || B <= 0 || H <= 0 || H > (prep ? 65534 : 65535) || dn <= 0 || dn > 4096 || dr < 0 || R <= 0 || rs < R + dr || ldq < H * (dn + dr)) return -1;
     const int nb = B > 2 ? 4 : (int)B;
     int v = R % 8 == 0 && ((uintptr_t)wuk & 15) == 0 ? 8 : 1;
     while (v > 2 && ((R + 64 * v - 1) / (64 * v)) * H * ((B + nb - 1) / nb) < 256) v /= 2;

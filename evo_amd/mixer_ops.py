@@ -60,8 +60,8 @@ class Stream:
         self.behind = False                                      # xb does not hold the current x
 
     def product(self, a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-        """a @ w^T of a sublayer, for `add` -- or its parts over K [parts, M, N], where a few rows' layer is summed in parts: the closing norm adds them."""
-        parts = self.ops.linear_parts(a, w) if self.xb.dtype == torch.bfloat16 and hasattr(self.ops, "linear_parts") else None
+        """a @ w^T of a sublayer, for `add` -- or its parts over K [parts, M, N], where the layer is summed in parts: the closing norm adds them."""
+        parts = self.ops.layer_parts(a, w) if self.xb.dtype == torch.bfloat16 and w.shape[0] <= 4096 and hasattr(self.ops, "layer_parts") else None
         return self.ops.linear(a, w) if parts is None else parts
 
     def add(self, y: torch.Tensor, w: torch.Tensor) -> None:

@@ -44,6 +44,7 @@ _SIGNATURES = {
     "evo_mlp_gate_mfma_bf16": ([_PTR] * 3 + [_I64] * 4 + [_PTR], _c.c_int),
     "evo_hyena_ct": ([_PTR] * 9 + [_I64] * 13 + [_PTR], _c.c_int),
     "evo_linear_t_mfma_bf16": ([_PTR] * 4 + [_I64] * 3 + [_PTR], _c.c_int),
+    "evo_rmsnorm_parts_bf16": ([_PTR, _PTR, _I64] + [_PTR] * 3 + [_I64] * 2 + [_F32, _PTR], _c.c_int),
     "evo_rmsnorm_rows_bf16": ([_PTR, _PTR, _PTR, _PTR, _I64, _I64, _F32, _I64, _I64, _I64, _I64, _PTR], _c.c_int),
     "evo_linear_xblk_mfma_bf16": ([_PTR] * 5 + [_I64] * 3 + [_PTR], _c.c_int),
     "evo_linear_mfma_nf_bf16": ([_PTR] * 7 + [_I64] * 4 + [_PTR], _c.c_int),
@@ -56,6 +57,8 @@ _SIGNATURES = {
     "evo_hyena_ct_packed": ([_PTR] * 9 + [_I64] * 5 + [_PTR], _c.c_int),
     "evo_attn_fwd_packed_bf16": ([_PTR] * 4 + [_I64] * 9 + [_PTR] * 2 + [_I64, _PTR, _F32, _PTR, _PTR], _c.c_int),
     "evo_dense_ws": ([_I64] * 5, _c.c_int),
+    "evo_dense_parts": ([_I64] * 3, _c.c_int),
+    "evo_dense_parts_bf16": ([_PTR] * 3 + [_I64] * 4 + [_PTR], _c.c_int),
     "evo_dense_launches": ([_I64] * 6 + [_PTR], _c.c_int),
     "evo_dense_plan": ([_I64] * 5 + [_PTR], _c.c_int),
     "evo_dense_bf16": ([_I64] * 3 + [_PTR] * 7 + [_I64] * 8 + [_PTR, _I64, _PTR], _c.c_int),
@@ -110,7 +113,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 27         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 28         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):
@@ -486,6 +489,39 @@ class HipOps(MixerOps):
         with self._t("gemv"):
             _check(self.lib.evo_linear_parts_bf16(x.data_ptr(), w.data_ptr(), ws.data_ptr(), M, w.shape[0], K, n, _stream()), "evo_linear_parts_bf16")
         return ws
+
+    def layer_parts(self, x, w, mfma: bool = False) -> Optional[torch.Tensor]:
+        """linear_parts, and the parts of 65 to 1,023 rows that the norm behind a layer is to add (evo_dense_parts): [parts, M, N] fp32, or None."""
+        M, K = x.shape
+        if M <= 64:
+            return self.linear_parts(x, w)
+        if M >= 1024 or not self._take_mfma(mfma) or not self.mfma_linear_ok(x, w) or (x.data_ptr() | w.data_ptr()) % 16:
+            return None
+        n = self.lib.evo_dense_parts(M, w.shape[0], K)
+        if n <= 0:
+            return None
+        ws = torch.empty(n, M, w.shape[0], dtype=torch.float32, device=x.device)
+        with self._t("gemm_mfma"):
+            _check(self.lib.evo_dense_parts_bf16(x.data_ptr(), w.data_ptr(), ws.data_ptr(), M, w.shape[0], K, n, _stream()), "evo_dense_parts_bf16")
+        return ws
+
+    def linear_residual_norm_(self, res: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], scale: torch.Tensor, eps: float,
+                              mfma: bool = False) -> Optional[torch.Tensor]:
+        """res += x @ w^T (+ bias) in place, as linear_residual_, and rmsnorm(res) * scale -- where the layer is summed in parts that the norm's launch can add; elsewhere
+        None, and nothing is done."""
+        M, D = res.shape
+        if not (17 <= M < 1024 and 8 <= D <= 8192 and res.dtype == scale.dtype == torch.bfloat16 and res.is_contiguous() and scale.is_contiguous() and w.shape[0] == D
+                and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous()))
+                and (res.data_ptr() | scale.data_ptr() | (0 if bias is None else bias.data_ptr())) % 16 == 0):
+            return None
+        parts = self.layer_parts(x, w, mfma)
+        if parts is None:
+            return None
+        out = torch.empty_like(res)
+        with self._t("rmsnorm"):
+            _check(self.lib.evo_rmsnorm_parts_bf16(res.data_ptr(), parts.data_ptr(), parts.shape[0], _ptr(bias), scale.data_ptr(), out.data_ptr(), M, D, float(eps), _stream()),
+                   "evo_rmsnorm_parts_bf16")
+        return out
 
     @staticmethod
     def mfma_linear_ok(x, w):
@@ -1069,18 +1105,18 @@ class HipOps(MixerOps):
         return y
 
     def hyena_decode_fused(self, x, norm_scale, eps, proj_w, proj_b, fir_state, iir_state, fir_w, fir_b, poles,
-                           residues, dskip, n_heads: int, one_launch: bool = False) -> torch.Tensor:
+                           residues, dskip, n_heads: int, one_launch: bool = False, normed: Optional[torch.Tensor] = None) -> torch.Tensor:
         """One decode token through pre-norm + projections + FIR/modal step + gate in ONE launch (M = batch <= 4, or <= 6 at D = 4096: 23.5 us
         against 23 in three launches, 26.8 against 23 at 8); states are updated in place.  Falls back to the separate kernels otherwise.  `one_launch`: up to 8 rows
-        (the last tokens of a scoring batch, whose launches are few beside the batch's own)."""
+        (the last tokens of a scoring batch, whose launches are few beside the batch's own).  `normed`: x behind the pre-norm, where that is there already."""
         M, D = x.shape
-        ok = ((1 <= M <= 4 or (M <= (8 if one_launch else 6) and D == 4096)) and x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and proj_w.is_contiguous()
+        ok = (normed is None and (1 <= M <= 4 or (M <= (8 if one_launch else 6) and D == 4096)) and x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and proj_w.is_contiguous()
               and proj_w.dtype == torch.bfloat16 and norm_scale.dtype == torch.bfloat16 and proj_b is not None
               and fir_state.dtype == torch.bfloat16 and fir_state.is_contiguous() and fir_state.shape[0] == M
               and iir_state.dtype == torch.complex64 and iir_state.is_contiguous() and iir_state.shape[0] == M
               and D == n_heads * 128)
         if not ok:
-            z = self.norm_linear(x, norm_scale, eps, proj_w, proj_b)
+            z = self.norm_linear(x, norm_scale, eps, proj_w, proj_b) if normed is None else self.linear(normed, proj_w, proj_b)
             return self.hyena_step(z, fir_state, iir_state, fir_w, fir_b, poles, residues, dskip, n_heads)
         y = torch.empty(M, D, dtype=torch.bfloat16, device=x.device)
         sr = torch.view_as_real(iir_state)

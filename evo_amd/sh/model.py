@@ -14,7 +14,7 @@ There is no CPU fallback here: with no `ops` injected and no usable HIP library 
 from __future__ import annotations
 
 import math
-from typing import Dict, List, Optional, Tuple
+from typing import Dict, List, NamedTuple, Optional, Tuple
 
 import torch
 import torch.nn as nn
@@ -71,6 +71,11 @@ class _MHA(nn.Module):
         self.out_proj = _Params(weight=((D, D), bf), bias=((D,), bf))
         self.rotary_emb = nn.Module()
         self.rotary_emb.register_buffer("inv_freq", torch.empty(hd // 2, dtype=torch.float32), persistent=True)
+
+
+class _Normed(NamedTuple):
+    """The stream behind the next norm, handed from block to block in the place of row factors."""
+    rows: torch.Tensor
 
 
 class _AttentionBlock(nn.Module):
@@ -441,6 +446,26 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         self.ops.linear_residual_(x2d, y, w, mfma=mfma, bias=bias)
         return None
 
+    def _mixer_out_norm_(self, blk, x2d, y, w, bias, mask=None, mfma=False):
+        """_mixer_out_, and the post-mixer norm of the new stream where the projection is summed in parts that the norm's launch adds; else None."""
+        if mask is None and y.dim() == 2 and hasattr(self.ops, "linear_residual_norm_"):
+            n2 = self.ops.linear_residual_norm_(x2d, y, w, bias, blk.post_norm.scale, self.eps, mfma)
+            if n2 is not None:
+                return n2
+        self._mixer_out_(blk, x2d, y, w, bias, mfma=mfma)
+        return None
+
+    def _next_norm(self, i: int, x2d, B: int, T: int, mask):
+        """Scale of the norm behind block i's MLP, if what takes it reads normed rows (a Hyena block that goes channel-major norms into its own layout); else None."""
+        if mask is not None or not 17 <= B * T < 1024:
+            return None
+        if i + 1 == len(self.blocks):
+            return None if self.norm is None else self.norm.scale
+        nxt = self.blocks[i + 1]
+        if not isinstance(nxt, _AttentionBlock) and T > 1 and self._channel_major(nxt, x2d, B, T, mask):
+            return None
+        return nxt.pre_norm.scale
+
     # ---- RMSNorm folded into the dense layers around it (round 5; csrc/gemm.hip NF, include/evo_mi355x.h) ---------------------------
     # The dense layer that writes the residual stream (mixer output projection, l3) also emits every row's 1 / (rms + eps) -- `rs` below,
     # handed from block to block --, and the layer that consumes the norm (Hyena projections, Wqkv, l1 | l2) reads the stream itself and
@@ -492,7 +517,9 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             mlp._w12g = self.ops.pack_gate_weights(mlp._w12)
         return mlp._w12g
 
-    def _mlp_residual_(self, blk, x2d, bias, mask=None):
+    def _mlp_residual_(self, blk, x2d, bias, mask=None, n2=None, nxt=None):
+        """The block's MLP, residual added in place.  `n2`: the post-mixer norm of x2d, where it is there already.  `nxt`: scale of the norm behind the block; returns
+        that norm's rows (_Normed) if l3 is summed in parts that the norm's launch adds, else None."""
         ops = self.ops
         self._gate_pack(blk, x2d.shape[0])
         if mask is not None:                                             # upstream: (mixer out + u) * padding_mask
@@ -503,13 +530,20 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             n2 = ops.rmsnorm(x2d, None, blk.post_norm.scale, self.eps)
             a = ops.mlp_gate(n2, blk.mlp._w12, w12g=blk.mlp._w12g)
             ops.linear_residual_(x2d, a, blk.mlp._w3)
-            return
-        if bias is None:                                                 # decode: norm + l1/l2 + gate in one launch
+            return None
+        if n2 is not None:
+            a = ops.mlp_gate(n2, blk.mlp._w12, w12g=blk.mlp._w12g)
+        elif bias is None:                                               # decode: norm + l1/l2 + gate in one launch
             a = ops.mlp_gate(x2d, blk.mlp._w12, blk.post_norm.scale, self.eps, w12g=blk.mlp._w12g)
         else:
             n2 = ops.rmsnorm(x2d, bias, blk.post_norm.scale, self.eps)   # x += bias (in place); n2 = norm(x)
             a = ops.mlp_gate(n2, blk.mlp._w12, w12g=blk.mlp._w12g)
+        if nxt is not None and hasattr(ops, "linear_residual_norm_"):
+            n1 = ops.linear_residual_norm_(x2d, a, blk.mlp._w3, None, nxt, self.eps)
+            if n1 is not None:
+                return _Normed(n1)
         ops.linear_residual_(x2d, a, blk.mlp._w3)
+        return None
 
     def _mfma_hyena_ok(self, B: int, T: int) -> bool:
         """The single-pass matrix-core operator (csrc/hyena_ct.hip) serves every parallel (T > 1) Hyena call without a padding mask on
@@ -556,6 +590,9 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         return ((B * T >= 1024 or ops.zt_layout(B, T)[3] == 1) and getattr(ops, "hyena_ct_flag", False) and hasattr(ops, "hyena_ct") and x2d.is_cuda and w.dtype == torch.bfloat16
                 and w.is_contiguous() and ops.zt_shape_ok(B, T, w.shape[0], w.shape[1]))
 
+    def _channel_major(self, blk, x2d, B: int, T: int, mask) -> bool:
+        return mask is None and self._mfma_hyena_ok(B, T) and self._hyena_ct_ok(x2d, blk, B, T) and self._table_ok(blk)
+
     def _hyena_block(self, i, blk, x2d, B, T, cache: Optional[RecurrentInferenceParams], mask=None, rs=None):
         """`mask` = (flat [B*T,1] bf16, [B,T] uint8) of upstream's padding_mask, or None: the projections output, the FIR
         output and the mixer output + residual are multiplied by it, as upstream's ParallelGatedConvBlock /
@@ -563,13 +600,15 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         ops = self.ops
         D, H = self.hidden_size, self.num_heads
         f = blk.filter
+        n1 = rs.rows if isinstance(rs, _Normed) else None            # the pre-norm's rows
+        rs = None if n1 is not None else rs
         have_state = cache is not None and i in cache.fir_state_dict
         K1 = self.short_filter_length - 1
         if have_state and T == 1:                 # decode: norm + projections + FIR/modal step + gate in one launch
             y = ops.hyena_decode_fused(x2d, blk.pre_norm.scale, self.eps, blk.projections.weight, blk.projections.bias,
                                        cache.fir_state_dict[i], cache.state_dict[i], f._fir_w, f.short_filter_bias,
-                                       f._poles, f._residues, f.D, H)
-        elif mask is None and self._mfma_hyena_ok(B, T) and self._hyena_ct_ok(x2d, blk, B, T) and self._table_ok(blk):
+                                       f._poles, f._residues, f.D, H, **({} if n1 is None else {"normed": n1}))
+        elif n1 is None and self._channel_major(blk, x2d, B, T, mask):
             # the whole operator in ONE pass on the matrix cores (csrc/hyena_ct.hip) -- scoring and cached prefill (carry-in state + FIR
             # history in, end state out) alike.
             # z CHANNEL-MAJOR.  The pre-norm writes its rows in z^T's position order (HipOps.zt_layout: batch
@@ -620,7 +659,8 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             self._mlp_residual_(blk, x2d, self._mixer_out_(blk, x2d, y, blk.out_filter_dense.weight, blk.out_filter_dense.bias), None)
             return None
         else:
-            z = ops.norm_linear(x2d, blk.pre_norm.scale, self.eps, blk.projections.weight, blk.projections.bias)   # [B*T, 3D]
+            z = (ops.norm_linear(x2d, blk.pre_norm.scale, self.eps, blk.projections.weight, blk.projections.bias) if n1 is None      # [B*T, 3D]
+                 else ops.linear(n1, blk.projections.weight, blk.projections.bias))
             if mask is not None:
                 z.mul_(mask[0])
             z3 = z.view(B, T, 3 * D)
@@ -640,9 +680,8 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
                     tail = torch.cat([z3.new_zeros(B, K1 - T, 3 * D), tail], dim=1)
                 cache.fir_state_dict[i] = tail.transpose(1, 2).contiguous()      # [B, 3D, 2]
                 cache.state_dict[i] = state
-        self._mlp_residual_(blk, x2d, self._mixer_out_(blk, x2d, y, blk.out_filter_dense.weight, blk.out_filter_dense.bias),
-                            None if mask is None else mask[0])
-        return None
+        n2 = self._mixer_out_norm_(blk, x2d, y, blk.out_filter_dense.weight, blk.out_filter_dense.bias, mask)
+        return self._mlp_residual_(blk, x2d, None, None if mask is None else mask[0], n2, self._next_norm(i, x2d, B, T, mask))
 
     def _tail_split_index(self, B: int, T: int, device):
         """Index tensors of the tail-split routing (_hyena_block), cached per (B, T): the z^T block holding the last two main steps of every
@@ -678,8 +717,11 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         mha = blk.inner_mha_cls
         if mask is not None:                      # upstream AttentionBlock: u * padding_mask before and after the mixer
             x2d.mul_(mask[0])
+        n1 = rs.rows if isinstance(rs, _Normed) else None            # the pre-norm's rows
         nf = T > 1 and self._nf_ok(B * T, mask)
-        if nf and rs is not None:
+        if n1 is not None:
+            qkv = ops.linear(n1, mha.Wqkv.weight, mha.Wqkv.bias, mfma=True).view(B, T, 3, H, hd)
+        elif nf and rs is not None:
             wqkv_f = self._folded(mha, "_wqkv_f", mha.Wqkv.weight, blk.pre_norm.scale)
             qkv = ops.linear_rs(x2d, rs, wqkv_f, mha.Wqkv.bias, mha.Wqkv.weight, blk.pre_norm.scale, self.eps).view(B, T, 3, H, hd)
         else:
@@ -721,9 +763,8 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
                 a = ops.attention(q, k, v, off, **ak).view(B * T, D)
         if nf:
             return self._mlp_residual_rs_(blk, x2d, self._mixer_out_rs_(blk, x2d, a, mha.out_proj.weight, mha.out_proj.bias))
-        self._mlp_residual_(blk, x2d, self._mixer_out_(blk, x2d, a, mha.out_proj.weight, mha.out_proj.bias, mfma=True),
-                            None if mask is None else mask[0])
-        return None
+        n2 = self._mixer_out_norm_(blk, x2d, a, mha.out_proj.weight, mha.out_proj.bias, mask, mfma=True)
+        return self._mlp_residual_(blk, x2d, None, None if mask is None else mask[0], n2, self._next_norm(i, x2d, B, T, mask))
 
     # ------------------------------------------------------------------ forward
     max_rows_per_pass = 160 * 1024     # rows (B T) of one stateless pass; larger batches run in row groups (hidden_states)
@@ -803,7 +844,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             for i, blk in enumerate(self.blocks):
                 if taps is not None and (tap_idxs is None or i in tap_idxs):
                     taps.append(h.clone())
-                # rs: 1 / (rms + eps) of every row of h, from the epilogue of the dense layer that wrote it (None: the block norms h itself)
+                # rs: 1 / (rms + eps) of every row of h, from the epilogue of the dense layer that wrote it, or h behind the block's pre-norm (None: the block norms h itself)
                 if isinstance(blk, _AttentionBlock):
                     rs = self._attn_block(i, blk, h, B, T, mha_c, mask, rs)
                 else:
@@ -814,7 +855,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             if dyn:
                 mha_c._rot_dyn = None
         if self.norm is not None:
-            h = ops.rmsnorm(h, None, self.norm.scale, self.eps)
+            h = rs.rows if isinstance(rs, _Normed) else ops.rmsnorm(h, None, self.norm.scale, self.eps)
         return h
 
     @torch.no_grad()

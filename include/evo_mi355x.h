@@ -68,8 +68,9 @@ extern "C" {
  *  24: evo_linear_f32_ahead and evo_linear_f32_ahead_plan added.
  *  25: evo_linear_few_f32 added.
  *  26: evo_dense_launches added.
- *  27: evo_closing_final and evo_latent_prep_absorb added. */
-#define EVO_ABI_VERSION 27
+ *  27: evo_closing_final and evo_latent_prep_absorb added.
+ *  28: evo_dense_parts, evo_dense_parts_bf16 and evo_rmsnorm_parts_bf16 added. */
+#define EVO_ABI_VERSION 28
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
@@ -366,6 +367,13 @@ int evo_linear_t_mfma_nf_bf16(const void* x, const float* row_scale, const void*
 int evo_dense_launches(int64_t mode, int64_t stats, int64_t xblk, int64_t M, int64_t N, int64_t K, int64_t* out);
 int evo_dense_plan(int64_t mode, int64_t stats, int64_t M, int64_t N, int64_t K, int64_t* out);
 int evo_dense_ws(int64_t mode, int64_t stats, int64_t M, int64_t N, int64_t K);
+/* The parts of K of x w^T that the norm behind the layer is to add (evo_rmsnorm_parts_bf16, evo_closing_parts), 65 to 1,023 rows: how many, 0 where layer and norm in launches of
+ * their own are ahead (no GPU needed); ws [parts, M, N] fp32.  Everything 16-byte aligned. */
+int evo_dense_parts(int64_t M, int64_t N, int64_t K);
+int evo_dense_parts_bf16(const void* x, const void* w, float* ws, int64_t M, int64_t N, int64_t K, int64_t parts, void* stream);
+/* x [M, D] += the parts part [parts, M, D] (+ bias), rounded once; out = x / (rms(x) + eps) * scale, with the bits of evo_rmsnorm_bf16.  D % 8 == 0, D <= 8192, at most 64 parts,
+ * everything 16-byte aligned. */
+int evo_rmsnorm_parts_bf16(void* x, const float* part, int64_t parts, const void* bias, const void* scale, void* out, int64_t M, int64_t D, float eps, void* stream);
 int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const void* x, const void* w, const void* bias, const void* residual, void* y,
                    const float* row_scale, float* sumsq, int64_t ss_ld, int64_t M, int64_t N, int64_t K, int64_t act_cols, int64_t x_rows,
                    int64_t Tm, int64_t row_skip, void* ws, int64_t ws_bytes, void* stream);
