@@ -560,12 +560,12 @@ __global__ __launch_bounds__(256) void gemm_parts_kernel(GemmArgs a, int act, co
 // 147 at 2,048; 12,288 columns 76 -> 34 at 161 rows, 78 -> 58 at 512; 22,016 gated columns 82 -> 53 at 161.
 struct TileKind { int bm, bn; double step_us; };
 static const TileKind kinds[] = {{64, 64, 0.255}, {128, 64, 0.435}, {128, 128, 0.515}, {192, 128, 0.70}, {256, 128, 0.84}, {128, 256, 0.86},
-                                 {96, 96, 0.50}, {192, 96, 0.667}, {96, 48, 0.35}};
-// The last three, below 256 rows and without parts, statistics or a transposed result: narrow enough that a layer of 12,288 to 24,576 columns is one round of
+                                 {96, 96, 0.50}, {192, 96, 0.667}, {96, 48, 0.35}, {64, 96, 0.40}};
+// The next three, below 256 rows and without parts, statistics or a transposed result: narrow enough that a layer of 12,288 to 24,576 columns is one round of
 // nearly all CUs.  us, before -> with them: 22,016 gated columns, K = 4,096 (172 tiles of 128 -> 230 of 96) 39.6 -> 37.7 at 65 rows, 42.2 -> 40.8 at 96, 48.0 -> 44.8
 // at 129, 51.7 -> 48.7 at 161, 53.6 -> 51.4 at 192; 12,288 columns (192 tiles of 64 -> 256 of 48) 27.2 -> 24.4 at 65, 29.8 -> 27.8 at 96; 11,264 columns 30.5 -> 23.5 and 33.1 -> 26.7.  Twelve waves for
 // 192 x 96 (six 49.8, four 56.7: a wave alone on its SIMD waits for its own fragments).  Not taken: 128 x 96 (43.4 - 45.1 at 97 - 128 rows, 42.4 - 46.6 with 128 x 128),
-// 256 x 96 (66.5 against 56.5 at 193) and 192 x 48 (35.7 against 34.2).
+// 256 x 96 (66.5 against 56.5 at 193) and 192 x 48 (35.7 against 34.2).  The last: tile_one_round.
 #define T_ODD 6                              // first of them
 // The persistent kernel on tiles of 160, 192 and 224 rows (and 256 columns): a step of 64 k takes nearly as little as its operands do, where 256 rows are a round that
 // leaves a third of the chip idle or a tile that is half padding.  us, the plan without them -> with (rows of the tile): K = 4,096, 22,016 gated columns 89 -> 66 at 300 rows
@@ -604,7 +604,7 @@ static TilePlan tile_best(int64_t M, int64_t N, int64_t K, int mode, bool stats,
         best = {T_PERSISTENT, 1, us > power ? us : power, M};
         if (memory > best.us) best.us = memory;
     }
-    for (int c = 0; c < (int)(sizeof(kinds) / sizeof(kinds[0])); ++c) {
+    for (int c = 0; c < T_ODD + 3; ++c) {
         const int bm = mode == 3 ? kinds[c].bn : kinds[c].bm, bn = mode == 3 ? kinds[c].bm : kinds[c].bn;      // along the tokens, along the weight
         if ((mode == 1 && c == 0) || (mode != 3 && c == 5)) continue;
         if (c >= T_ODD && (M >= 256 || mode == 3 || stats || (mode == 1) != (c < T_ODD + 2))) continue;
@@ -642,6 +642,24 @@ static int tile_plan_square(int64_t M, int64_t N, int64_t K, int mode, bool stat
     return 1;
 }
 
+// Ungated layers of 65 to 255 rows on tiles whose row tiles and column tiles together are nearly one round of the CUs (nine tenths and more), where the tiles above leave a quarter of the
+// chip idle, and in place of 128 x 64 in one round two parts of 128 x 128: half the operand rows a CU takes in, and what a round of 128 x 64 waits for is beyond its cost rule (weights
+// that come from memory; sums included).  us, before -> these, at 112 / 129 / 161 / 192 rows: 96 x 96, 12,288 columns of K = 2,048 21.5 / 20.3 / 20.8 / 22.0 -> 18.5 / 18.9 /
+// 20.6 / 21.2, 4,096 37.9 / 34.4 / 35.7 / 37.8 -> 31.1 / 31.7 / 35.0 / 36.0 (phases from 161 rows on), 8,192 54.9 / 57.7 / 63.4 / 65.9 -> 52.1 / 54.1 / 60.5 / 65.5, 11,264 of 4,096 31.9 / 34.0 /
+// 35.0 / 37.2 -> 31.4 / 31.0 / 34.2 / 34.6; 96 x 48, 6,144 of 4,096 22.4 / 24.5 / 26.4 / 27.9 -> 20.9 / 21.4 / 23.3 / 26.1 (of 6,144 from 145 rows on 2 to 11 % behind: parts of K); 64 x 96 at
+// 193 / 224 / 255 rows there 27.2 / 29.0 / 30.8 -> 23.8 / 26.3 / 28.7; two parts at 65 / 96 / 128 rows, 16,384 of 4,096 41.0 / 39.0 / 40.7 -> 34.9 / 36.1 / 38.7, 13,824 of 5,120 47.9 / 46.6 /
+// 50.1 -> 39.3 / 40.9 / 43.9, 8,192 of 4,096 at 240 36.9 -> 32.5 (of 2,048 behind: 16,384 24.0 : 26.5).
+static void tile_one_round(int64_t M, int64_t N, int64_t K, bool splits_ok, TilePlan& plan) {
+    const int64_t cus = tile_cus();
+    auto round = [&](int kind) {
+        const int64_t tiles = ((M + kinds[kind].bm - 1) / kinds[kind].bm) * ((N + kinds[kind].bn - 1) / kinds[kind].bn);
+        return tiles <= cus && 10 * tiles >= 9 * cus;
+    };
+    const int kind = M <= 96 || K < 2048 ? -1 : M <= 192 && round(T_ODD) ? T_ODD : K > 5120 ? -1 : M <= 192 ? (round(T_ODD + 2) ? T_ODD + 2 : -1) : round(T_ODD + 3) ? T_ODD + 3 : -1;
+    if (kind >= 0) plan = {kind, 1, 0.9 * plan.us, M};
+    else if (plan.kind == 1 && plan.splits == 1 && splits_ok && K >= 4096 && 2 * ((M + 127) / 128) * (N / 128) <= cus) plan = {2, 2, plan.us, M};
+}
+
 static double steps_us(const StepUs& s, double rows, double cols, double nk) {
     const double cus = tile_cus(), rounds = ceil(ceil(rows / s.rows) * cols / cus), full = rows / s.rows * cols / (rounds * cus);
     return rounds * (nk * (s.us + s.more * fmax(0.0, full - s.from)) + s.end);
@@ -655,6 +673,7 @@ static double steps_us(const StepUs& s, double rows, double cols, double nk) {
 // their padding is most of a tile.
 static int tile_plan(int64_t M, int64_t N, int64_t K, int mode, bool stats, bool splits_ok, bool persistent_ok, bool short_ok, TilePlan (&out)[2]) {
     const int n = tile_plan_square(M, N, K, mode, stats, splits_ok, persistent_ok, out);
+    if (mode == 0 && M < 256 && !stats) tile_one_round(M, N, K, splits_ok, out[0]);
     if (!persistent_ok || !short_ok || M < 256 || K < 2048) return n;
     const double memory = (2.0 * (M * K + N * K) + 2.0 * M * N) / 4.9e6, nk = (double)(K / 64);
     const double rows = (double)(mode == 3 ? N : M), cols = (double)((mode == 3 ? M : N) / 256);       // (mode 3: the tokens are the columns of the launch)
@@ -681,7 +700,7 @@ static int tile_plan(int64_t M, int64_t N, int64_t K, int mode, bool stats, bool
 static int tile_phases(int kind, int mode, bool xblk, int splits, int64_t M, int64_t N, int64_t K) {
     if (splits != 1 || xblk || mode > 2) return 0;
     if (kind == 2) return K >= 1024 && 4 * M <= N && (M - 1) % 128 >= (M > 512 ? 119 : 95) ? 6 : 0;
-    if (kind == T_ODD) return M >= 80 && M <= 96 && K >= 4096 ? 8 : 0;
+    if (kind == T_ODD) return mode == 0 ? (M > 160 ? 8 : 0) : M >= 80 && M <= 96 && K >= 4096 ? 8 : 0;
     if (kind == T_ODD + 1) return M >= 150 && M <= 192 && K >= 1024 ? 5 : 0;
     return 0;
 }
@@ -888,7 +907,9 @@ extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const voi
             else if (t.kind == 3) rc = tile_launch<192, 128, 4, 2, 4, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
             else if (t.kind == 4) rc = tile_launch<256, 128, 4, 2, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
             else if (t.kind == 5) rc = tile_launch<128, 256, 2, 4, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
-            else if (xblk || tm > 1 || (tm == 1) != (t.kind < T_ODD + 2)) rc = -1;
+            else if (xblk || tm > 1 || (tm == 1 ? t.kind >= T_ODD + 2 : t.kind == T_ODD + 1)) rc = -1;
+            else if (tm == 0 && t.kind == T_ODD) rc = phases ? tile_launch_odd<96, 96, 2, 3, 18, 0>(a, (int)act, st) : tile_launch_odd<96, 96, 2, 3, 6, 0>(a, (int)act, st);
+            else if (t.kind == T_ODD + 3) rc = tile_launch_odd<64, 96, 2, 2, 7, 0>(a, (int)act, st);
             else if (t.kind == T_ODD) rc = phases ? tile_launch_odd<96, 96, 2, 3, 18, 1>(a, (int)act, st) : tile_launch_odd<96, 96, 2, 3, 6, 1>(a, (int)act, st);
             else if (t.kind == T_ODD + 1) rc = phases ? tile_launch_odd<192, 96, 4, 3, 15, 1>(a, (int)act, st) : tile_launch_odd<192, 96, 4, 3, 4, 1>(a, (int)act, st);
             else rc = tile_launch_odd<96, 48, 3, 1, 8, 0>(a, (int)act, st);
