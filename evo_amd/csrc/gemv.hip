@@ -884,7 +884,7 @@ __global__ __launch_bounds__(512) void skinny_mfma_kernel(const uint4* __restric
 template <int XR, int WAVES, int CH, int NB, int EP>
 __global__ __launch_bounds__(64 * WAVES) void skinny_kw_kernel(const unsigned char* __restrict__ x, const unsigned char* __restrict__ w,
                                                                const uint16_t* __restrict__ bias, const uint16_t* res, uint16_t* y, int M, int N, int K,
-                                                               int act) {   // res may alias y
+                                                               int act, const uint16_t* __restrict__ scale, uint16_t* __restrict__ xg, float* __restrict__ ss) {   // res may alias y
     constexpr int MT = XR > 16 ? 2 : 1, ROW = 2 * CH, RPI = 1024 / ROW, GR = ROW / 16;      // bytes of a row piece, rows per request, granules per row piece
     constexpr int PW = 16 / RPI, PX = XR / RPI, P = PW + PX, BUF = (16 + XR) * ROW;
     extern __shared__ __attribute__((aligned(16))) unsigned char kw_lds[];
@@ -907,12 +907,14 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kw_kernel(const unsigned ch
     // EP: bias and residual values of the waves that end with results, requested ahead of everything (from places that are there; `EP` 2: four at a time) and looked at behind the
     // last product: asked for there they were a memory latency of their own at the end (4,096 x 4,096 with both, 5 / 16 / 32 rows 8.4 / 9.3 / 11.4 -> 7.5 / 8.1 / 10.0 us, K = 11,008
     // 17.8 / 18.9 -> 16.7 / 17.7; one value a request 7.7 / 8.4 / 10.3, behind the first chunks 8.1 / 9.0 / 10.8).  Without either they are not in the code: 7.25 -> 7.1.
-    uint2 pb = {}, pr = {};
+    // EP 3 (N % 16 == 0): for the norm behind the layer, whose scale this is: xg = the new value times scale, and ss [M][N / 16], a row's sum of squares by workgroups.  What takes the
+    // norm multiplies xg by its weights and the sums by 1 / (rms + eps) (skinny_ring_kernel, RS).
+    uint2 pb = {}, pr = {}, pg = {};
     if (EP && wave < MT) {
         const int m = 16 * wave + r16, nq = n0 + 4 * kb;
         const uint16_t* from = res + (int64_t)(m < M ? m : M - 1) * N;
         auto four = [&](const uint16_t* p) {
-            if constexpr (EP == 2) return *(const uint2*)(p + (nq < N ? nq : 0));
+            if constexpr (EP >= 2) return *(const uint2*)(p + (nq < N ? nq : 0));
             uint32_t v[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] = p[nq + r < N ? nq + r : N - 1];
@@ -920,6 +922,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kw_kernel(const unsigned ch
         };
         if (bias) pb = four(bias);
         if (res) pr = four(from);
+        if constexpr (EP == 3) pg = four(scale);
     }
     const int chunks = K / CH, mine = (chunks - wave + WAVES - 1) / WAVES;
     const int start = mine > 4 && gridDim.x >= 128 ? (int)(blockIdx.x >> 3) * 3 % mine : 0;       // (workgroups of an XCD don't walk K in step: skinny_ring_kernel)
@@ -983,6 +986,25 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kw_kernel(const unsigned ch
 #pragma unroll
         for (int q = 1; q < WAVES; ++q) a_ += part[(wave * WAVES + q) * 64 + lane];
         const int m = 16 * wave + r16;
+        if constexpr (EP == 3) {
+            float o[4], q = 0.f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                auto one = [&](uint2 v) { const uint32_t h = r < 2 ? v.x : v.y; return r & 1 ? bf_hi(h) : bf_lo(h); };
+                o[r] = a_[r] + (bias ? one(pb) : 0.f);
+                o[r] = round_bf(o[r] + one(pr));
+                q = fmaf(o[r], o[r], q);
+            }
+            q += __shfl_xor(q, 16, 64);
+            q += __shfl_xor(q, 32, 64);
+            if (m < M) {
+                const int64_t at = (int64_t)m * N + n0 + 4 * kb;
+                *(uint2*)(y + at) = make_uint2(pack_bf2(o[0], o[1]), pack_bf2(o[2], o[3]));
+                *(uint2*)(xg + at) = make_uint2(pack_bf2(o[0] * bf_lo(pg.x), o[1] * bf_hi(pg.x)), pack_bf2(o[2] * bf_lo(pg.y), o[3] * bf_hi(pg.y)));
+                if (kb == 0) ss[(int64_t)m * gridDim.x + blockIdx.x] = q;
+            }
+            return;
+        }
         if (m < M) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -999,12 +1021,13 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kw_kernel(const unsigned ch
 }
 
 template <int XR, int WAVES, int CH, int NB, int EP>
-static int kw_go(const void* x, const void* w, const void* bias, const void* residual, void* y, int64_t M, int64_t N, int64_t K, int act, hipStream_t s) {
+static int kw_go(const void* x, const void* w, const void* bias, const void* residual, void* y, int64_t M, int64_t N, int64_t K, int act, hipStream_t s,
+                 const void* scale = nullptr, void* xg = nullptr, float* ss = nullptr) {
     constexpr size_t lds = (size_t)WAVES * NB * (16 + XR) * 2 * CH;
     static_assert(lds <= 160 * 1024, "the CU's LDS");
     if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)skinny_kw_kernel<XR, WAVES, CH, NB, EP>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     hipLaunchKernelGGL((skinny_kw_kernel<XR, WAVES, CH, NB, EP>), dim3((unsigned)((N + 15) / 16)), dim3(64 * WAVES), lds, s, (const unsigned char*)x,
-                       (const unsigned char*)w, (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)K, act);
+                       (const unsigned char*)w, (const uint16_t*)bias, (const uint16_t*)residual, (uint16_t*)y, (int)M, (int)N, (int)K, act, (const uint16_t*)scale, (uint16_t*)xg, ss);
     return evo_launch_status();
 }
 // (a form of its own for layers without bias and residual: the requests in front of their loop cost 0.2 to 0.3 us there)
@@ -1041,9 +1064,14 @@ static __host__ __device__ __forceinline__ uint32_t ring_edge(uint32_t cols, uin
     const uint32_t each = cols / groups, more = cols % groups;
     return b * each + (groups <= 0x10000 ? b * more / groups : (uint32_t)((uint64_t)b * more / groups));
 }
-template <int XR, int T, int NB, int MODE>
+// RS: x is a row times the scale of its norm, and its products are taken times 1 / (rms + eps) of the row, from the sums of squares ss [M][strips] (skinny_kw_kernel, EP 3): the norm
+// between two layers without a launch.  The sums are asked for ahead of the stream and added up behind it, 0.3 us; the launch was 2.6.  Pools of 5 / 8 / 16 / 24 / 32
+// short prompts, four layers, 32 steps (seven norms a step; three from 17 rows on, whose l3 is summed in parts): 12.88 / 13.46 / 15.11 / 16.88 / 18.33 -> 12.53 / 12.98 / 14.54 / 16.58 /
+// 18.03 ms, logits as far from 64 bits as before (7.9e-3 -> 7.8e-3 to 7.9e-3).
+template <int XR, int T, int NB, int MODE, bool RS = false>
 __global__ __launch_bounds__(64 * T) void skinny_ring_kernel(const unsigned char* __restrict__ x, const unsigned char* __restrict__ w, const uint16_t* __restrict__ bias,
-                                                             const uint16_t* res, uint16_t* y, int M, int N, int K, int act, int layout, float* __restrict__ ws) {   // res may alias y
+                                                             const uint16_t* res, uint16_t* y, int M, int N, int K, int act, int layout, float* __restrict__ ws,
+                                                             const float* __restrict__ ss, int strips, float eps, float inv_sqrt_d) {   // res may alias y
     constexpr int MT = XR / 16, PX = (XR / 4 + T - 1) / T, PW = 4, P = PX + PW;      // requests of 1 KiB (4 rows) per wave and chunk
     constexpr int XOFF = T * 16 * RG_ROWB, BUF = XOFF + T * PX * 1024;
     static_assert(XR % 16 == 0 && NB >= 2 && (NB - 2) * P < 64, "the wait counter has six bits");
@@ -1092,6 +1120,13 @@ __global__ __launch_bounds__(64 * T) void skinny_ring_kernel(const unsigned char
 #pragma unroll
             for (int r = 0; r < 4; ++r) pr[t][r] = from[n0 + r < N ? n0 + r : N - 1];
         }
+    }
+    constexpr int RW = RS ? (XR + T - 1) / T : 1;                // rows whose sums a wave adds: wave, wave + T, ..
+    gv_f32x4 sq[RW];
+    __shared__ float rs_s[RS ? RW * T : 1];
+    if constexpr (RS) {
+#pragma unroll
+        for (int j = 0; j < RW; ++j) sq[j] = *(const gv_f32x4*)(ss + (int64_t)(wave + T * j < M ? wave + T * j : M - 1) * strips + (4 * lane < strips ? 4 * lane : 0));
     }
     const int all = K / 128, c0 = MODE == 2 ? (int)((int64_t)all * blockIdx.y / gridDim.y) : 0;
     const int chunks = (MODE == 2 ? (int)((int64_t)all * (blockIdx.y + 1) / gridDim.y) : all) - c0;
@@ -1144,6 +1179,20 @@ __global__ __launch_bounds__(64 * T) void skinny_ring_kernel(const unsigned char
             }
         }
         buf = buf + BUF == lds0 + NB * BUF ? lds0 : buf + BUF;
+    }
+    if constexpr (RS) {
+#pragma unroll
+        for (int j = 0; j < RW; ++j) {
+            const float sum = wave_sum(4 * lane < strips ? (sq[j][0] + sq[j][1]) + (sq[j][2] + sq[j][3]) : 0.f);
+            if (lane == 0) rs_s[wave + T * j] = 1.0f / (sqrtf(sum) * inv_sqrt_d + eps);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const float f = rs_s[16 * t + r16];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[t][r] *= f;
+        }
     }
     // D[n][m]: lane holds rows 4 kb + r of its wave's tile, m = 16 t + r16
     if constexpr (MODE == 1) {
@@ -1212,14 +1261,15 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const float* __restr
 // rows, rounds of up to 96 rows and four stages -> this: 28,672 x 1,024 11.6 / 12.3 / 15.4 / 20.0 -> 11.4 / 12.2 / 13.7 / 16.7, 50,304 x 1,024 22.4 / 24.1 / 27.1 / 33.0 ->
 // 18.4 / 19.7 / 23.4 / 31.4, 65,536 x 4,096 78 / 80 / 86 / 102 -> 79 / 78 / 80 / 95, 151,936 x 512 34 / 40 / 47 / 59 -> 28 / 32 / 38 / 55 (x 4,096 179 / 192 / 214 / 251 ->
 // 182 / 191 / 216 / 263).
-template <int XR, int T, int MODE, int NB>
+struct RingNorm { const float* ss; int strips; float eps, inv_sqrt_d; };     // RS
+template <int XR, int T, int MODE, int NB, bool RS = false>
 static int ring_go(dim3 grid, const void* x, const void* w, const void* bias, const void* res, void* y, int64_t M, int64_t N, int64_t K, int act, int layout, float* ws,
-                   hipStream_t s) {
+                   hipStream_t s, RingNorm n = {}) {
     constexpr size_t lds = (size_t)NB * T * (16 * RG_ROWB + (XR / 4 + T - 1) / T * 1024);
     static_assert(lds <= 160 * 1024, "the CU's LDS");
-    if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)skinny_ring_kernel<XR, T, NB, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL((skinny_ring_kernel<XR, T, NB, MODE>), grid, dim3(64 * T), lds, s, (const unsigned char*)x, (const unsigned char*)w, (const uint16_t*)bias,
-                       (const uint16_t*)res, (uint16_t*)y, (int)M, (int)N, (int)K, act, layout, ws);
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)skinny_ring_kernel<XR, T, NB, MODE, RS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL((skinny_ring_kernel<XR, T, NB, MODE, RS>), grid, dim3(64 * T), lds, s, (const unsigned char*)x, (const unsigned char*)w, (const uint16_t*)bias,
+                       (const uint16_t*)res, (uint16_t*)y, (int)M, (int)N, (int)K, act, layout, ws, n.ss, n.strips, n.eps, n.inv_sqrt_d);
     return evo_launch_status();
 }
 // 4,097 to 7,680 columns from K = 4,096 on (to 7,168: from 2,048): a workgroup per CU here too, of 17 to 30 columns in two waves.  A CU takes in 45 to 55 GB/s while lines come
@@ -1266,6 +1316,20 @@ static int ring_launch(const void* x, const void* w, const void* bias, const voi
 #undef EVO_RGN
 #undef EVO_RG1
 #undef EVO_RG
+}
+
+// RS, 5 to 32 rows and up to 24,576 weight rows: as many waves and stages as ring_launch takes
+template <int MODE>
+static int ring_factors(const void* x, const void* w, const void* bias, void* y, int64_t M, int64_t N, int64_t K, int layout, RingNorm n, hipStream_t s) {
+    const int waves = ring_waves(N, K);
+    const dim3 grid((unsigned)ring_groups(N, K));
+    if (grid.x > 256) return -1;
+#define EVO_RF(XR, T, NB) ring_go<XR, T, MODE, NB, true>(grid, x, w, bias, nullptr, y, M, N, K, 0, layout, nullptr, s, n)
+#define EVO_RF1(T) (M <= 16 ? EVO_RF(16, T, 4) : EVO_RF(32, T, 4))
+    if (M <= 16 && ring_spread(N, K)) return EVO_RF(16, 2, 6);
+    return waves == 2 ? EVO_RF1(2) : waves == 3 ? EVO_RF1(3) : waves == 4 ? EVO_RF1(4) : EVO_RF1(6);
+#undef EVO_RF1
+#undef EVO_RF
 }
 
 template <int M>
@@ -1494,4 +1558,29 @@ extern "C" int evo_linear_small_m_bf16(const void* x, const void* w, const void*
         default: gemv_launch<8>(x, w, bias, residual, y, N, K, (int)act, s); break;
     }
     return evo_launch_status();
+}
+
+// ---- a norm between two layers without a launch, 5 to 32 rows (skinny_kw_kernel EP 3, skinny_ring_kernel RS)
+extern "C" int evo_linear_residual_scaled_bf16(const void* x, const void* w, const void* bias, void* y, const void* scale, void* xg, float* ss, int64_t M, int64_t N, int64_t K,
+                                               void* stream) {
+    if (!x || !w || !y || !scale || !xg || !ss || M < 5 || M > 32 || N < 2048 || N > 4096 || N % 64 != 0 || K < 1152 || K % 128 != 0 || K > 0x9fffff || small_m_parts(M, N, K)) return -1;
+    if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)ss) & 15) || (((uintptr_t)bias | (uintptr_t)y | (uintptr_t)scale | (uintptr_t)xg) & 7)) return -1;
+    hipStream_t s = (hipStream_t)stream;
+    if (M <= 8) return kw_go<8, 4, 128, 3, 3>(x, w, bias, y, y, M, N, K, 0, s, scale, xg, ss);
+    if (M <= 16) return kw_go<16, 4, 128, 2, 3>(x, w, bias, y, y, M, N, K, 0, s, scale, xg, ss);
+    return kw_go<32, 3, 128, 2, 3>(x, w, bias, y, y, M, N, K, 0, s, scale, xg, ss);
+}
+
+static bool factors_ok(const void* xg, const float* ss, const void* w, int64_t M, int64_t N, int64_t K) {
+    return xg && ss && w && M >= 5 && M <= 32 && N > 4096 && N <= 24576 && K >= 2048 && K <= 4096 && K % 128 == 0 && (((uintptr_t)xg | (uintptr_t)ss | (uintptr_t)w) & 15) == 0;
+}
+
+extern "C" int evo_linear_factors_bf16(const void* xg, const float* ss, float eps, const void* w, const void* bias, void* y, int64_t M, int64_t N, int64_t K, void* stream) {
+    if (!factors_ok(xg, ss, w, M, N, K) || !y) return -1;
+    return ring_factors<0>(xg, w, bias, y, M, N, K, 0, {ss, (int)(K / 16), eps, 1.0f / sqrtf((float)K)}, (hipStream_t)stream);
+}
+
+extern "C" int evo_mlp_gate_factors_bf16(const void* xg, const float* ss, float eps, const void* w12, void* a, int64_t M, int64_t I, int64_t K, int64_t grouped, void* stream) {
+    if (I <= 0 || I > 0x3fffffff || I % 32 != 0 || !factors_ok(xg, ss, w12, M, 2 * I, K) || !a) return -1;
+    return ring_factors<1>(xg, w12, nullptr, a, M, 2 * I, K, grouped ? 1 : 2, {ss, (int)(K / 16), eps, 1.0f / sqrtf((float)K)}, (hipStream_t)stream);
 }

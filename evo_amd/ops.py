@@ -57,6 +57,9 @@ _SIGNATURES = {
     "evo_hyena_ct_packed": ([_PTR] * 9 + [_I64] * 5 + [_PTR], _c.c_int),
     "evo_attn_fwd_packed_bf16": ([_PTR] * 4 + [_I64] * 9 + [_PTR] * 2 + [_I64, _PTR, _F32, _PTR, _PTR], _c.c_int),
     "evo_dense_ws": ([_I64] * 5, _c.c_int),
+    "evo_linear_residual_scaled_bf16": ([_PTR] * 7 + [_I64] * 3 + [_PTR], _c.c_int),
+    "evo_linear_factors_bf16": ([_PTR, _PTR, _F32] + [_PTR] * 3 + [_I64] * 3 + [_PTR], _c.c_int),
+    "evo_mlp_gate_factors_bf16": ([_PTR, _PTR, _F32, _PTR, _PTR] + [_I64] * 4 + [_PTR], _c.c_int),
     "evo_dense_parts": ([_I64] * 3, _c.c_int),
     "evo_dense_parts_bf16": ([_PTR] * 3 + [_I64] * 4 + [_PTR], _c.c_int),
     "evo_dense_launches": ([_I64] * 6 + [_PTR], _c.c_int),
@@ -113,7 +116,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 28         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 29         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):
@@ -522,6 +525,49 @@ class HipOps(MixerOps):
             _check(self.lib.evo_rmsnorm_parts_bf16(res.data_ptr(), parts.data_ptr(), parts.shape[0], _ptr(bias), scale.data_ptr(), out.data_ptr(), M, D, float(eps), _stream()),
                    "evo_rmsnorm_parts_bf16")
         return out
+
+    def factors_ok(self, M: int, w: torch.Tensor, gate: bool = False) -> bool:
+        """Whether linear_factors (mlp_gate_factors) takes w: layers that the weight-streaming launches of 5 to 32 rows take in one round."""
+        N, K = w.shape
+        return (5 <= M <= 32 and 4096 < N <= 24576 and 2048 <= K <= 4096 and K % 128 == 0 and w.is_cuda and w.dtype == torch.bfloat16 and w.is_contiguous()
+                and w.data_ptr() % 16 == 0 and (N % 64 == 0 and self.gate_small_m_mfma if gate else self.lib.evo_linear_parts(M, N, K) == 0))
+
+    def linear_residual_scaled_(self, res: torch.Tensor, x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], scale: torch.Tensor):
+        """res += x @ w^T (+ bias) in place, as linear_residual_, and for a norm of the new rows (res * scale, their sums of squares by 16 columns), which
+        linear_factors and mlp_gate_factors take; None, and nothing is done, for layers that the launch is not for."""
+        M, K = x.shape
+        N = w.shape[0]
+        if not (5 <= M <= 32 and 2048 <= N <= 4096 and N % 64 == 0 and K % 128 == 0 and 1024 < K and self._use_small_m(x, w) and res.dtype == scale.dtype == torch.bfloat16
+                and tuple(res.shape) == (M, N) and res.is_contiguous() and scale.is_contiguous() and scale.numel() == N
+                and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous()))
+                and (x.data_ptr() | w.data_ptr() | res.data_ptr() | scale.data_ptr() | (0 if bias is None else bias.data_ptr())) % 16 == 0 and self.lib.evo_linear_parts(M, N, K) == 0):
+            return None
+        xg, ss = torch.empty_like(res), torch.empty(M, N // 16, dtype=torch.float32, device=res.device)
+        with self._t("gemv"):
+            _check(self.lib.evo_linear_residual_scaled_bf16(x.data_ptr(), w.data_ptr(), _ptr(bias), res.data_ptr(), scale.data_ptr(), xg.data_ptr(), ss.data_ptr(), M, N, K,
+                                                            _stream()), "evo_linear_residual_scaled_bf16")
+        return xg, ss
+
+    def linear_factors(self, xg: torch.Tensor, ss: torch.Tensor, eps: float, w: torch.Tensor, b: Optional[torch.Tensor]) -> torch.Tensor:
+        """linear(rmsnorm(x) * scale, w, b) from linear_residual_scaled_'s results."""
+        M, K = xg.shape
+        assert self.factors_ok(M, w) and w.shape[1] == K and tuple(ss.shape) == (M, K // 16) and (b is None or (b.dtype == torch.bfloat16 and b.is_contiguous()))
+        y = torch.empty(M, w.shape[0], dtype=torch.bfloat16, device=xg.device)
+        with self._t("gemv"):
+            _check(self.lib.evo_linear_factors_bf16(xg.data_ptr(), ss.data_ptr(), float(eps), w.data_ptr(), _ptr(b), y.data_ptr(), M, w.shape[0], K, _stream()),
+                   "evo_linear_factors_bf16")
+        return y
+
+    def mlp_gate_factors(self, xg: torch.Tensor, ss: torch.Tensor, eps: float, w12: torch.Tensor, grouped: bool) -> torch.Tensor:
+        """mlp_gate(rmsnorm(x) * scale, w12) (GELU) from linear_residual_scaled_'s results; `grouped`: w12 in pack_gate_weights' order."""
+        M, K = xg.shape
+        I = w12.shape[0] // 2
+        assert self.factors_ok(M, w12, gate=True) and w12.shape[1] == K and tuple(ss.shape) == (M, K // 16)
+        a = torch.empty(M, I, dtype=torch.bfloat16, device=xg.device)
+        with self._t("gemv_gate"):
+            _check(self.lib.evo_mlp_gate_factors_bf16(xg.data_ptr(), ss.data_ptr(), float(eps), w12.data_ptr(), a.data_ptr(), M, I, K, int(grouped), _stream()),
+                   "evo_mlp_gate_factors_bf16")
+        return a
 
     @staticmethod
     def mfma_linear_ok(x, w):
@@ -1105,18 +1151,18 @@ class HipOps(MixerOps):
         return y
 
     def hyena_decode_fused(self, x, norm_scale, eps, proj_w, proj_b, fir_state, iir_state, fir_w, fir_b, poles,
-                           residues, dskip, n_heads: int, one_launch: bool = False, normed: Optional[torch.Tensor] = None) -> torch.Tensor:
+                           residues, dskip, n_heads: int, one_launch: bool = False) -> torch.Tensor:
         """One decode token through pre-norm + projections + FIR/modal step + gate in ONE launch (M = batch <= 4, or <= 6 at D = 4096: 23.5 us
         against 23 in three launches, 26.8 against 23 at 8); states are updated in place.  Falls back to the separate kernels otherwise.  `one_launch`: up to 8 rows
-        (the last tokens of a scoring batch, whose launches are few beside the batch's own).  `normed`: x behind the pre-norm, where that is there already."""
+        (the last tokens of a scoring batch, whose launches are few beside the batch's own)."""
         M, D = x.shape
-        ok = (normed is None and (1 <= M <= 4 or (M <= (8 if one_launch else 6) and D == 4096)) and x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and proj_w.is_contiguous()
+        ok = ((1 <= M <= 4 or (M <= (8 if one_launch else 6) and D == 4096)) and x.is_cuda and x.dtype == torch.bfloat16 and x.is_contiguous() and proj_w.is_contiguous()
               and proj_w.dtype == torch.bfloat16 and norm_scale.dtype == torch.bfloat16 and proj_b is not None
               and fir_state.dtype == torch.bfloat16 and fir_state.is_contiguous() and fir_state.shape[0] == M
               and iir_state.dtype == torch.complex64 and iir_state.is_contiguous() and iir_state.shape[0] == M
               and D == n_heads * 128)
         if not ok:
-            z = self.norm_linear(x, norm_scale, eps, proj_w, proj_b) if normed is None else self.linear(normed, proj_w, proj_b)
+            z = self.norm_linear(x, norm_scale, eps, proj_w, proj_b)
             return self.hyena_step(z, fir_state, iir_state, fir_w, fir_b, poles, residues, dskip, n_heads)
         y = torch.empty(M, D, dtype=torch.bfloat16, device=x.device)
         sr = torch.view_as_real(iir_state)

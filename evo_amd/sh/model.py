@@ -78,6 +78,12 @@ class _Normed(NamedTuple):
     rows: torch.Tensor
 
 
+class _Scaled(NamedTuple):
+    """The stream times the next norm's scale, and the sums of squares that its rows' factors come from (ops.linear_residual_scaled_), handed on in the same way."""
+    rows: torch.Tensor
+    ss: torch.Tensor
+
+
 class _AttentionBlock(nn.Module):
     def __init__(self, D, inner, hd):
         super().__init__()
@@ -446,25 +452,47 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         self.ops.linear_residual_(x2d, y, w, mfma=mfma, bias=bias)
         return None
 
+    def _residual_norm_(self, x2d, y, w, bias, scale, takes, gate=False, mfma=False):
+        """x2d += y @ w^T (+ bias), and what the norm behind it needs no launch of its own for: _Scaled where `takes`, the weight that reads the norm, takes row factors, _Normed where
+        the layer is summed in parts that the norm's launch adds; else None, and nothing is done."""
+        ops = self.ops
+        M = x2d.shape[0]
+        if takes is not None and M <= 32 and hasattr(ops, "linear_residual_scaled_") and ops.factors_ok(M, takes, gate):
+            got = ops.linear_residual_scaled_(x2d, y, w, bias, scale)
+            if got is not None:
+                return _Scaled(*got)
+        if not 17 <= M < 1024 or not hasattr(ops, "linear_residual_norm_"):
+            return None
+        n = ops.linear_residual_norm_(x2d, y, w, bias, scale, self.eps, mfma)
+        return None if n is None else _Normed(n)
+
     def _mixer_out_norm_(self, blk, x2d, y, w, bias, mask=None, mfma=False):
-        """_mixer_out_, and the post-mixer norm of the new stream where the projection is summed in parts that the norm's launch adds; else None."""
-        if mask is None and y.dim() == 2 and hasattr(self.ops, "linear_residual_norm_"):
-            n2 = self.ops.linear_residual_norm_(x2d, y, w, bias, blk.post_norm.scale, self.eps, mfma)
+        """_mixer_out_, and the post-mixer norm of the new stream where it needs no launch of its own (_residual_norm_); else None."""
+        if mask is None and y.dim() == 2:
+            mlp = blk.mlp
+            n2 = self._residual_norm_(x2d, y, w, bias, blk.post_norm.scale, mlp._w12g if mlp._w12 is None else mlp._w12, True, mfma)
             if n2 is not None:
                 return n2
         self._mixer_out_(blk, x2d, y, w, bias, mfma=mfma)
         return None
 
     def _next_norm(self, i: int, x2d, B: int, T: int, mask):
-        """Scale of the norm behind block i's MLP, if what takes it reads normed rows (a Hyena block that goes channel-major norms into its own layout); else None."""
-        if mask is not None or not 17 <= B * T < 1024:
+        """(scale of the norm behind block i's MLP, the weight that reads the norm or None) if what takes it reads normed rows (a Hyena block that goes channel-major norms
+        into its own layout); else None."""
+        if mask is not None or not 5 <= B * T < 1024:
             return None
         if i + 1 == len(self.blocks):
-            return None if self.norm is None else self.norm.scale
+            return None if self.norm is None else (self.norm.scale, None)
         nxt = self.blocks[i + 1]
-        if not isinstance(nxt, _AttentionBlock) and T > 1 and self._channel_major(nxt, x2d, B, T, mask):
+        if isinstance(nxt, _AttentionBlock):
+            return nxt.pre_norm.scale, nxt.inner_mha_cls.Wqkv.weight
+        if T > 1 and self._channel_major(nxt, x2d, B, T, mask):
             return None
-        return nxt.pre_norm.scale
+        return nxt.pre_norm.scale, nxt.projections.weight
+
+    def _norm_layer(self, n, w, b, mfma=False):
+        """x w^T + b of the normed x."""
+        return self.ops.linear_factors(n.rows, n.ss, self.eps, w, b) if isinstance(n, _Scaled) else self.ops.linear(n.rows, w, b, mfma=mfma)
 
     # ---- RMSNorm folded into the dense layers around it (round 5; csrc/gemm.hip NF, include/evo_mi355x.h) ---------------------------
     # The dense layer that writes the residual stream (mixer output projection, l3) also emits every row's 1 / (rms + eps) -- `rs` below,
@@ -518,8 +546,8 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         return mlp._w12g
 
     def _mlp_residual_(self, blk, x2d, bias, mask=None, n2=None, nxt=None):
-        """The block's MLP, residual added in place.  `n2`: the post-mixer norm of x2d, where it is there already.  `nxt`: scale of the norm behind the block; returns
-        that norm's rows (_Normed) if l3 is summed in parts that the norm's launch adds, else None."""
+        """The block's MLP, residual added in place.  `n2`: the post-mixer norm of x2d, where it is there already (_Normed, _Scaled).  `nxt`: the norm behind the block
+        (_next_norm); returns that norm if it needs no launch of its own (_residual_norm_), else None."""
         ops = self.ops
         self._gate_pack(blk, x2d.shape[0])
         if mask is not None:                                             # upstream: (mixer out + u) * padding_mask
@@ -531,17 +559,19 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             a = ops.mlp_gate(n2, blk.mlp._w12, w12g=blk.mlp._w12g)
             ops.linear_residual_(x2d, a, blk.mlp._w3)
             return None
-        if n2 is not None:
-            a = ops.mlp_gate(n2, blk.mlp._w12, w12g=blk.mlp._w12g)
+        if isinstance(n2, _Scaled):
+            a = ops.mlp_gate_factors(n2.rows, n2.ss, self.eps, blk.mlp._w12g if blk.mlp._w12 is None else blk.mlp._w12, blk.mlp._w12 is None)
+        elif n2 is not None:
+            a = ops.mlp_gate(n2.rows, blk.mlp._w12, w12g=blk.mlp._w12g)
         elif bias is None:                                               # decode: norm + l1/l2 + gate in one launch
             a = ops.mlp_gate(x2d, blk.mlp._w12, blk.post_norm.scale, self.eps, w12g=blk.mlp._w12g)
         else:
             n2 = ops.rmsnorm(x2d, bias, blk.post_norm.scale, self.eps)   # x += bias (in place); n2 = norm(x)
             a = ops.mlp_gate(n2, blk.mlp._w12, w12g=blk.mlp._w12g)
-        if nxt is not None and hasattr(ops, "linear_residual_norm_"):
-            n1 = ops.linear_residual_norm_(x2d, a, blk.mlp._w3, None, nxt, self.eps)
+        if nxt is not None:
+            n1 = self._residual_norm_(x2d, a, blk.mlp._w3, None, *nxt)
             if n1 is not None:
-                return _Normed(n1)
+                return n1
         ops.linear_residual_(x2d, a, blk.mlp._w3)
         return None
 
@@ -600,14 +630,18 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         ops = self.ops
         D, H = self.hidden_size, self.num_heads
         f = blk.filter
-        n1 = rs.rows if isinstance(rs, _Normed) else None            # the pre-norm's rows
+        n1 = rs if isinstance(rs, (_Normed, _Scaled)) else None      # the pre-norm, where it is there already
         rs = None if n1 is not None else rs
         have_state = cache is not None and i in cache.fir_state_dict
         K1 = self.short_filter_length - 1
         if have_state and T == 1:                 # decode: norm + projections + FIR/modal step + gate in one launch
-            y = ops.hyena_decode_fused(x2d, blk.pre_norm.scale, self.eps, blk.projections.weight, blk.projections.bias,
-                                       cache.fir_state_dict[i], cache.state_dict[i], f._fir_w, f.short_filter_bias,
-                                       f._poles, f._residues, f.D, H, **({} if n1 is None else {"normed": n1}))
+            if n1 is not None:
+                y = ops.hyena_step(self._norm_layer(n1, blk.projections.weight, blk.projections.bias), cache.fir_state_dict[i], cache.state_dict[i], f._fir_w,
+                                   f.short_filter_bias, f._poles, f._residues, f.D, H)
+            else:
+                y = ops.hyena_decode_fused(x2d, blk.pre_norm.scale, self.eps, blk.projections.weight, blk.projections.bias,
+                                           cache.fir_state_dict[i], cache.state_dict[i], f._fir_w, f.short_filter_bias,
+                                           f._poles, f._residues, f.D, H)
         elif n1 is None and self._channel_major(blk, x2d, B, T, mask):
             # the whole operator in ONE pass on the matrix cores (csrc/hyena_ct.hip) -- scoring and cached prefill (carry-in state + FIR
             # history in, end state out) alike.
@@ -660,7 +694,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             return None
         else:
             z = (ops.norm_linear(x2d, blk.pre_norm.scale, self.eps, blk.projections.weight, blk.projections.bias) if n1 is None      # [B*T, 3D]
-                 else ops.linear(n1, blk.projections.weight, blk.projections.bias))
+                 else self._norm_layer(n1, blk.projections.weight, blk.projections.bias))
             if mask is not None:
                 z.mul_(mask[0])
             z3 = z.view(B, T, 3 * D)
@@ -717,10 +751,10 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         mha = blk.inner_mha_cls
         if mask is not None:                      # upstream AttentionBlock: u * padding_mask before and after the mixer
             x2d.mul_(mask[0])
-        n1 = rs.rows if isinstance(rs, _Normed) else None            # the pre-norm's rows
+        n1 = rs if isinstance(rs, (_Normed, _Scaled)) else None      # the pre-norm, where it is there already
         nf = T > 1 and self._nf_ok(B * T, mask)
         if n1 is not None:
-            qkv = ops.linear(n1, mha.Wqkv.weight, mha.Wqkv.bias, mfma=True).view(B, T, 3, H, hd)
+            qkv = self._norm_layer(n1, mha.Wqkv.weight, mha.Wqkv.bias, mfma=True).view(B, T, 3, H, hd)
         elif nf and rs is not None:
             wqkv_f = self._folded(mha, "_wqkv_f", mha.Wqkv.weight, blk.pre_norm.scale)
             qkv = ops.linear_rs(x2d, rs, wqkv_f, mha.Wqkv.bias, mha.Wqkv.weight, blk.pre_norm.scale, self.eps).view(B, T, 3, H, hd)

@@ -69,8 +69,9 @@ extern "C" {
  *  25: evo_linear_few_f32 added.
  *  26: evo_dense_launches added.
  *  27: evo_closing_final and evo_latent_prep_absorb added.
- *  28: evo_dense_parts, evo_dense_parts_bf16 and evo_rmsnorm_parts_bf16 added. */
-#define EVO_ABI_VERSION 28
+ *  28: evo_dense_parts, evo_dense_parts_bf16 and evo_rmsnorm_parts_bf16 added.
+ *  29: evo_linear_residual_scaled_bf16, evo_linear_factors_bf16 and evo_mlp_gate_factors_bf16 added. */
+#define EVO_ABI_VERSION 29
 int evo_abi_version(void);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
@@ -293,6 +294,14 @@ int evo_attn_decode_bf16(const void* q, const void* k, const void* v, void* o,
  * act 3: the square of relu before the rounding (0: none). */
 int evo_linear_small_m_bf16(const void* x, const void* w, const void* bias, const void* residual, void* y,
                             int64_t M, int64_t N, int64_t K, void* ws, int64_t ws_bytes, int64_t act, void* stream);
+
+/* A norm between two layers without a launch, 5 to 32 rows.  evo_linear_residual_scaled_bf16: y [M, N] += x w^T (+ bias), rounded once; xg [M, N] = y * scale; ss [M, N / 16] fp32 the
+ * sums of squares of y's rows over 16 columns each.  2,048 <= N <= 4,096, N % 64 == 0, K % 128 == 0, K > 1,024, and a layer that evo_linear_parts takes in one sum.
+ * evo_linear_factors_bf16, evo_mlp_gate_factors_bf16: evo_linear_small_m_bf16 and evo_mlp_gate_small_m_bf16 (GELU) of y / (rms(y) + eps) * scale from those, the rows' factors on the
+ * fp32 sums; K the norm's width, 4,096 < N (2 I) <= 24,576, I % 32 == 0.  x, xg, w and ss 16-byte aligned, the others 8. */
+int evo_linear_residual_scaled_bf16(const void* x, const void* w, const void* bias, void* y, const void* scale, void* xg, float* ss, int64_t M, int64_t N, int64_t K, void* stream);
+int evo_linear_factors_bf16(const void* xg, const float* ss, float eps, const void* w, const void* bias, void* y, int64_t M, int64_t N, int64_t K, void* stream);
+int evo_mlp_gate_factors_bf16(const void* xg, const float* ss, float eps, const void* w12, void* a, int64_t M, int64_t I, int64_t K, int64_t grouped, void* stream);
 
 /* Columns per workgroup of that launch on a wide layer (N > 4096, K % 128 == 0 and, for 4,097 to 7,680 columns, K >= 4096) and of the gated one (`gated`: N = 2 I, I columns): out [4] = workgroups, first column of workgroup
  * `block`, first behind it, columns that a workgroup has room for.  On the host, no launch; -1: no such workgroup. */
