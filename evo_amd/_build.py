@@ -35,7 +35,7 @@ COMPONENTS = {
         "evo_hyena_decode_fused_small_m", "evo_linear_mfma_bf16", "evo_linear_mfma_nf_bf16", "evo_mlp_gate_mfma_bf16",
         "evo_mlp_gate_mfma_nf_bf16", "evo_linear_xblk_mfma_bf16", "evo_linear_xblk_mfma_nf_bf16", "evo_linear_t_mfma_bf16",
         "evo_linear_t_mfma_nf_bf16", "evo_linear_act_mfma_bf16", "evo_dense_ws", "evo_dense_parts", "evo_dense_parts_bf16", "evo_dense_launches", "evo_dense_plan", "evo_dense_bf16", "evo_linear_f32_ws", "evo_linear_f32_plan", "evo_linear_f32", "evo_linear_f32_ahead_plan", "evo_linear_f32_ahead", "evo_linear_few_f32", "evo_put_tokens",
-        "evo_advance_positions", "evo_step_out", "evo_copy_rows", "evo_linear_ring_share", "evo_linear_parts", "evo_linear_parts_bf16", "evo_linear_residual_scaled_bf16", "evo_linear_factors_bf16", "evo_mlp_gate_factors_bf16", "evo_postnorm_linear_small_m_bf16",
+        "evo_token_batch", "evo_advance_positions", "evo_step_out", "evo_copy_rows", "evo_linear_ring_share", "evo_linear_parts", "evo_linear_parts_bf16", "evo_linear_residual_scaled_bf16", "evo_linear_factors_bf16", "evo_mlp_gate_factors_bf16", "evo_postnorm_linear_small_m_bf16",
         "evo_postnorm_mlp_gate_small_m_bf16", "evo_probe_copy_f4", "evo_probe_mfma_bf16",
     ]),
     "stripedhyena": ("_stripedhyena", ["attn", "attn_w64", "hyena", "hyena_ct"], ["attn_common.h"], [

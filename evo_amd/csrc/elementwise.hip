@@ -630,6 +630,47 @@ extern "C" int evo_put_tokens(int64_t* ids, int64_t S, const int64_t* slots, con
     return evo_launch_status();
 }
 
+// A batch of prompts from the lengths as kernel arguments: starts cu [B + 1], sequence and position of every token, sequences that go on from a state (resume, may be null).  It
+// was a blocking copy from host memory, which waits for whatever runs, and eight launches.
+struct BatchArgs { int start[EVO_PUT_MAX + 1]; int64_t past[EVO_PUT_MAX]; };
+__global__ __launch_bounds__(256) void token_batch_kernel(int* __restrict__ cu, int* __restrict__ seq, int64_t* __restrict__ pos, int* __restrict__ resume, BatchArgs a, int B) {
+    __shared__ int start[EVO_PUT_MAX + 1];
+    __shared__ int64_t past[EVO_PUT_MAX];
+    const int tid = threadIdx.x;
+    if (tid <= B) start[tid] = a.start[tid];
+    if (tid < B) past[tid] = a.past[tid];
+    __syncthreads();
+    if (blockIdx.x == 0) {
+        if (tid <= B) cu[tid] = start[tid];
+        if (resume && tid < B) resume[tid] = past[tid] > 0;
+    }
+    const int64_t i = (int64_t)blockIdx.x * 256 + tid;
+    if (i >= start[B]) return;
+    int lo = 0, hi = B;                                          // the last sequence that starts at i or before (empty ones start where the next does)
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (start[mid] <= i) lo = mid; else hi = mid;
+    }
+    seq[i] = lo;
+    pos[i] = past[lo] + (i - start[lo]);
+}
+
+extern "C" int evo_token_batch(int* cu, int* seq, int64_t* pos, int* resume, const int64_t* lens, const int64_t* past, int64_t B, void* stream) {
+    if (!cu || !seq || !pos || !lens || !past || B <= 0 || B > EVO_PUT_MAX) return -1;
+    BatchArgs a;
+    int64_t at = 0;
+    for (int64_t i = 0; i < B; ++i) {
+        if (lens[i] < 0 || past[i] < 0) return -1;
+        a.start[i] = (int)at;
+        a.past[i] = past[i];
+        at += lens[i];
+        if (at > 0x7fffffff) return -1;
+    }
+    a.start[B] = (int)at;
+    hipLaunchKernelGGL(token_batch_kernel, dim3((unsigned)((at + 255) / 256 > 0 ? (at + 255) / 256 : 1)), dim3(256), 0, (hipStream_t)stream, cu, seq, pos, resume, a, (int)B);
+    return evo_launch_status();
+}
+
 __global__ __launch_bounds__(256) void advance_positions_kernel(int64_t* __restrict__ pos, int64_t n, int64_t last) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i < n) pos[i] = pos[i] + 1 < last ? pos[i] + 1 : last;

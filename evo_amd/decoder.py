@@ -201,7 +201,7 @@ class LayeredDecoder(DecodeGraphMixin, nn.Module):
     def prefill_rows(self, prompts: List[torch.Tensor], want: Optional[List[List[int]]] = None):
         """Prompts of any lengths as packed passes -> [(logits [wanted, V], records, row of the records)]; `want`: the places whose logits are
         returned (the last token's by default)."""
-        out, first = [], 0
+        out, first, later = [], 0, [] if hasattr(self.ops, "check_ids") else None
         while first < len(prompts):
             n, tokens = 0, 0
             while first + n < len(prompts) and (n == 0 or tokens + prompts[first + n].numel() <= self.max_rows_per_pass):
@@ -210,14 +210,24 @@ class LayeredDecoder(DecodeGraphMixin, nn.Module):
             group = prompts[first:first + n]
             lens = [p.numel() for p in group]
             ipd = self.allocate_rows(n, max(lens))
-            h = self._run(torch.cat([p.reshape(-1) for p in group]), TokenBatch.of_prompts(lens, [0] * n, self.device), ipd)
+            h = self._run(torch.cat([p.reshape(-1) for p in group]), TokenBatch.of_prompts(lens, [0] * n, self.device, self.ops), ipd, later=later)
             at = [[m - 1] for m in lens] if want is None else want[first:first + n]
-            base = [sum(lens[:i]) for i in range(n)]
-            rows = torch.tensor([b + t for b, ts in zip(base, at) for t in ts], dtype=torch.int64, device=h.device)
-            logits = self.ops.linear(h[rows].contiguous(), self.unembed.weight) if rows.numel() else h.new_empty(0, self.vocab_size)
+            logits = self._logits_at(h, [sum(lens[:i]) for i in range(n)], lens, at)
             out += [(lg, ipd, i) for i, lg in enumerate(logits.split([len(ts) for ts in at]))]
             first += n
+        if later:
+            self.ops.check_ids(later)
         return out
+
+    def _logits_at(self, h: torch.Tensor, first: List[int], lens: List[int], at: List[List[int]]) -> torch.Tensor:
+        """Logits of the places `at` of sequences that lie in h from rows `first` on, one sequence's behind the other's."""
+        if not sum(len(ts) for ts in at):
+            return h.new_empty(0, self.vocab_size)
+        if any(len(ts) != m or list(ts) != list(range(m)) for ts, m in zip(at, lens)):        # (all of them: h as it is)
+            rows = [b + t for b, ts in zip(first, at) for t in ts]
+            rows = self.ops.host_rows(rows, h.device) if h.is_cuda and hasattr(self.ops, "host_rows") else torch.tensor(rows, dtype=torch.int64, device=h.device)
+            h = h[rows].contiguous()
+        return self.ops.linear(h, self.unembed.weight)
 
     # ------------------------------------------------------------------ captured decode step (sh/graph.py)
     def _graph_tensors(self, ipd):
@@ -246,12 +256,12 @@ class LayeredDecoder(DecodeGraphMixin, nn.Module):
         return all(self.ops.small_m_shape_ok(B, n, k) for n, k in shapes)
 
     # ------------------------------------------------------------------ forward
-    def _run(self, ids: torch.Tensor, batch: TokenBatch, ipd: Optional[dict], ids_known: bool = False) -> torch.Tensor:
-        """Packed ids [M] -> final-norm hidden states [M, width] (logits = hidden @ head^T)."""
+    def _run(self, ids: torch.Tensor, batch: TokenBatch, ipd: Optional[dict], ids_known: bool = False, later: Optional[list] = None) -> torch.Tensor:
+        """Packed ids [M] -> final-norm hidden states [M, width] (logits = hidden @ head^T).  `later`: the caller checks the ids behind the launches (ops.check_ids)."""
         if not self._loaded:
             raise RuntimeError(f"{type(self).__name__} has no weights: call load_state_dict first")
         ops = self.ops
-        stream = Stream(ops, ids.to(self.device), self.embed, self.embed_scale, self.eps, self.NORM_OFFSET, self.alpha, ids_known)
+        stream = Stream(ops, ids.to(self.device), self.embed, self.embed_scale, self.eps, self.NORM_OFFSET, self.alpha, ids_known, later)
         taps = getattr(self, "block_taps", None)     # debugging / parity hook: residual stream entering every layer, then the final one
         for i, layer in enumerate(self.layers):
             if taps is not None:
@@ -279,7 +289,7 @@ class LayeredDecoder(DecodeGraphMixin, nn.Module):
             raise ValueError(f"{type(self).__name__} takes no padding mask: unequal prompts are packed (prefill_rows), pads behind a prompt are never seen by it")
         B, T = x.shape
         if inference_params_dict is None:
-            return self._run(x.reshape(-1), TokenBatch.of_prompts([T] * B, [0] * B, self.device), None, ids_known)
+            return self._run(x.reshape(-1), TokenBatch.of_prompts([T] * B, [0] * B, self.device, self.ops), None, ids_known)
         mha = inference_params_dict["mha"]
         pos = getattr(mha, "pos_tensor", None)
         off = int(mha.seqlen_offset)
@@ -293,7 +303,7 @@ class LayeredDecoder(DecodeGraphMixin, nn.Module):
             fresh = self.allocate_rows(max(B, int(mha.max_batch_size or 1)), T + self.spare_positions)
             for i, layer in enumerate(self.layers):
                 layer.mix.store(inference_params_dict)[i] = layer.mix.store(fresh)[i]
-        return self._run(x.reshape(-1), TokenBatch.of_prompts([T] * B, [off] * B, self.device), inference_params_dict)
+        return self._run(x.reshape(-1), TokenBatch.of_prompts([T] * B, [off] * B, self.device, self.ops), inference_params_dict)
 
     @torch.no_grad()
     def forward(self, x, inference_params_dict=None, padding_mask=None):

@@ -28,9 +28,12 @@ class TokenBatch:
     decode: bool = False
 
     @staticmethod
-    def of_prompts(lens: Sequence[int], past: Sequence[int], device) -> "TokenBatch":
+    def of_prompts(lens: Sequence[int], past: Sequence[int], device, ops=None) -> "TokenBatch":
         lens, past = list(lens), list(past)
         B, M, device = len(lens), sum(lens), torch.device(device)
+        if device.type == "cuda" and hasattr(ops, "token_batch") and 0 < B <= ops.MAX_PUT:
+            cu, seq, pos, resume = ops.token_batch(lens, past, device)
+            return TokenBatch(cu, seq, pos, resume, lens, past)
         host = torch.tensor([[0] + lens, [0] + past], dtype=torch.int64).to(device)       # (one copy; the rest is made on the device)
         cu = host[0].cumsum(0)
         seq = torch.repeat_interleave(torch.arange(B, device=device), host[0, 1:], output_size=M)
@@ -52,9 +55,9 @@ class Stream:
     norm(t) = t / rms(t) * (w_offset + w)."""
 
     def __init__(self, ops, ids: torch.Tensor, weight: torch.Tensor, scale: float, eps: float, w_offset: float, alpha: Optional[float] = None,
-                 ids_known: bool = False):
+                 ids_known: bool = False, later: Optional[list] = None):
         self.ops, self.eps, self.w_offset, self.alpha = ops, eps, w_offset, alpha
-        self.x, self.xb = ops.embed_stream(ids, weight, scale, **({"validate": False} if ids_known else {}))
+        self.x, self.xb = ops.embed_stream(ids, weight, scale, **({"validate": False} if ids_known else {} if later is None else {"later": later}))
         self.open = None                                         # (y, w): still to be added
         self.spare = None                                        # the buffer the next such launch writes x to
         self.behind = False                                      # xb does not hold the current x
@@ -160,8 +163,9 @@ class MixerOps:
             _check(getattr(self.lib, name)(*args, _stream()), name)
 
     # ---- residual stream ------------------------------------------------------------------------------------------------
-    def embed_stream(self, ids: torch.Tensor, weight: torch.Tensor, scale: float, validate: bool = True) -> Tuple[torch.Tensor, torch.Tensor]:
-        """(x fp32 [M, D] = scale * weight[ids], the same in the storage type: x itself for fp32).  `validate=False`: the caller has checked the ids."""
+    def embed_stream(self, ids: torch.Tensor, weight: torch.Tensor, scale: float, validate: bool = True, later: Optional[list] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+        """(x fp32 [M, D] = scale * weight[ids], the same in the storage type: x itself for fp32).  `validate=False`: the caller has checked the ids; `later`: it calls
+        check_ids."""
         ids = ids.reshape(-1).to(torch.int64).contiguous()
         f32 = self._store(weight)
         V, D = weight.shape
@@ -172,8 +176,8 @@ class MixerOps:
             torch.zeros(1, dtype=torch.int32, device=weight.device)
         self._call("evo_embed_stream", self._ix(ids, torch.int64, ids.numel(), "ids"), weight.data_ptr(), x.data_ptr(), None if f32 else xb.data_ptr(),
                    ids.numel(), D, V, float(scale), None if flag is None else flag.data_ptr(), f32)
-        if flag is not None and int(flag.item()) != 0:
-            raise IndexError(f"input_ids contain values outside [0, {V}) (embedding table has {V} rows)")
+        if flag is not None:
+            self.raise_bad_ids(flag, V, later)
         return x, xb
 
     def _closing_args(self, x, xb, y, w):

@@ -52,6 +52,7 @@ _SIGNATURES = {
     "evo_mlp_gate_mfma_nf_bf16": ([_PTR] * 4 + [_I64] * 3 + [_PTR], _c.c_int),
     "evo_put_tokens": ([_PTR, _I64, _PTR, _PTR, _I64, _PTR], _c.c_int),
     "evo_advance_positions": ([_PTR, _I64, _I64, _PTR], _c.c_int),
+    "evo_token_batch": ([_PTR] * 6 + [_I64, _PTR], _c.c_int),
     "evo_step_out": ([_PTR] * 2 + [_I64, _PTR] + [_I64] * 2 + [_PTR], _c.c_int),
     "evo_copy_rows": ([_PTR, _I64, _PTR], _c.c_int),
     "evo_hyena_ct_packed": ([_PTR] * 9 + [_I64] * 5 + [_PTR], _c.c_int),
@@ -116,7 +117,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 29         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 30         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):
@@ -589,11 +590,35 @@ class HipOps(MixerOps):
         return y
 
     # ---- kernels -------------------------------------------------------------------------------------
-    def embed(self, ids: torch.Tensor, weight: torch.Tensor, validate: bool = True) -> torch.Tensor:
+    def raise_bad_ids(self, flag: torch.Tensor, vocab: int, later: Optional[list]) -> None:
+        """IndexError if an embedding has raised its flag: at once, or -- `later` -- by check_ids, so that nobody waits for the launches in front."""
+        if later is None:
+            if int(flag.item()) != 0:
+                raise IndexError(f"input_ids contain values outside [0, {vocab}) (embedding table has {vocab} rows)")
+            return
+        host, done = torch.empty(1, dtype=torch.int32, pin_memory=True), torch.cuda.Event()
+        host.copy_(flag, non_blocking=True)
+        done.record()
+        later.append((host, done, vocab))
+
+    @staticmethod
+    def check_ids(later: list) -> None:
+        """raise_bad_ids for embeddings whose layers are on their way: a wait for the embedding alone."""
+        for host, done, vocab in later:
+            done.synchronize()
+            if int(host.item()) != 0:
+                raise IndexError(f"input_ids contain values outside [0, {vocab}) (embedding table has {vocab} rows)")
+
+    @staticmethod
+    def upload(t: torch.Tensor, device) -> torch.Tensor:
+        """A host tensor on the device, by a copy that does not wait for what runs there."""
+        return t.pin_memory().to(device, non_blocking=True) if torch.device(device).type == "cuda" and t.numel() else t.to(device)
+
+    def embed(self, ids: torch.Tensor, weight: torch.Tensor, validate: bool = True, later: Optional[list] = None) -> torch.Tensor:
         """Row gather.  Ids outside [0, vocab) raise IndexError (the reference's F.embedding device-asserts): the
         kernel never indexes the table with them and raises a device flag, which is read back here -- except while a
         hipGraph is being captured (no host read is possible there; the decode loop's ids come from `sample`).  `validate=False`: the
-        caller has checked the ids itself (a sequence-parallel rank checks ALL of them before its first collective)."""
+        caller has checked the ids itself (a sequence-parallel rank checks ALL of them before its first collective).  `later`: the caller calls check_ids."""
         ids = ids.reshape(-1).to(torch.int64).contiguous()
         self._need(ids, torch.int64, "embed ids")
         self._need(weight, torch.bfloat16, "embed weight")
@@ -605,8 +630,8 @@ class HipOps(MixerOps):
             torch.zeros(1, dtype=torch.int32, device=weight.device)
         _check(self.lib.evo_embed_bf16(ids.data_ptr(), weight.data_ptr(), out.data_ptr(), ids.numel(), D, V,
                                        _ptr(flag), _stream()), "evo_embed_bf16")
-        if flag is not None and int(flag.item()) != 0:
-            raise IndexError(f"input_ids contain values outside [0, {V}) (embedding table has {V} rows)")
+        if flag is not None:
+            self.raise_bad_ids(flag, V, later)
         return out
 
     MAX_PUT = 64                 # tokens of one put_tokens launch (csrc/elementwise.hip EVO_PUT_MAX)
@@ -622,6 +647,26 @@ class HipOps(MixerOps):
             tokens = torch.tensor(tokens, dtype=torch.int64).tolist()
         arr = _c.c_int64 * n
         _check(self.lib.evo_put_tokens(ids.data_ptr(), ids.numel(), _c.cast(arr(*slots), _PTR), _c.cast(arr(*tokens), _PTR), n, _stream()), "evo_put_tokens")
+
+    def token_batch(self, lens, past, device):
+        """(cu [B + 1] int32, seq [M] int32, pos [M] int64, resume [B] int32 or None) of TokenBatch.of_prompts for up to MAX_PUT sequences: one launch, no copy from host memory
+        and no wait."""
+        B, M = len(lens), sum(lens)
+        cu, seq = torch.empty(B + 1, dtype=torch.int32, device=device), torch.empty(M, dtype=torch.int32, device=device)
+        pos = torch.empty(M, dtype=torch.int64, device=device)
+        resume = torch.empty(B, dtype=torch.int32, device=device) if any(past) else None
+        arr = _c.c_int64 * B
+        _check(self.lib.evo_token_batch(cu.data_ptr(), seq.data_ptr() or cu.data_ptr(), pos.data_ptr() or cu.data_ptr(), _ptr(resume), _c.cast(arr(*lens), _PTR),
+                                        _c.cast(arr(*past), _PTR), B, _stream()), "evo_token_batch")
+        return cu, seq, pos, resume
+
+    def host_rows(self, rows, device) -> torch.Tensor:
+        """Row numbers from the host as an int64 tensor: up to MAX_PUT of them as kernel arguments, without a copy that waits."""
+        if not 0 < len(rows) <= self.MAX_PUT:
+            return torch.tensor(rows, dtype=torch.int64).to(device)
+        out = torch.empty(len(rows), dtype=torch.int64, device=device)
+        self.put_tokens(out, range(len(rows)), rows)
+        return out
 
     def advance_positions(self, pos: torch.Tensor, last: int) -> None:
         """pos = min(pos + 1, last), in place."""

@@ -840,8 +840,9 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         """Rows of the embedding table: ids below are the ones that hidden_states takes."""
         return self.embedding_layer.weight.shape[0]
 
-    def hidden_states(self, x: torch.Tensor, inference_params_dict=None, padding_mask=None, ids_known: bool = False) -> torch.Tensor:
-        """ids [B,T] -> final-norm hidden states [B*T, D] (logits = hidden @ E^T).  `ids_known`: the caller has checked that they lie in [0, embedding_rows)."""
+    def hidden_states(self, x: torch.Tensor, inference_params_dict=None, padding_mask=None, ids_known: bool = False, later: Optional[list] = None) -> torch.Tensor:
+        """ids [B,T] -> final-norm hidden states [B*T, D] (logits = hidden @ E^T).  `ids_known`: the caller has checked that they lie in [0, embedding_rows); `later`: it
+        checks them behind the launches (ops.check_ids)."""
         if not self._packed:
             self._pack()
         if x.dim() != 2:
@@ -861,7 +862,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
                 out[b0 * T:(b0 + nb) * T] = hg
                 b0 += nb
             return out
-        h = ops.embed(x.to(self.device), self.embedding_layer.weight, **({"validate": False} if ids_known else {}))             # [B*T, D]
+        h = ops.embed(x.to(self.device), self.embedding_layer.weight, **({"validate": False} if ids_known else {} if later is None else {"later": later}))             # [B*T, D]
         mask = None
         if padding_mask is not None:
             pm = padding_mask.to(self.device) != 0
@@ -1002,7 +1003,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
                 rows = need if share else 0
         return groups
 
-    def _prefill_packed(self, prompts: List[torch.Tensor]):
+    def _prefill_packed(self, prompts: List[torch.Tensor], later: Optional[list] = None):
         """Prompts behind each other as ONE stream of rows, each from a multiple of 64 on (the rows between are token 0 and reach nobody: every
         launch is row-independent or keeps to one prompt's rows): the dense layers see all rows at once, the Hyena operator and the attention take
         all prompts in one launch, or one for each kernel that they would take alone.  -> (final-norm rows, first row of every prompt, caches of every prompt, each of its own length)."""
@@ -1017,10 +1018,11 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         for n, (f, m) in enumerate(zip(first, lens)):
             places[f:f + m] = torch.arange(m)
             places[M + K1 * n:M + K1 * (n + 1)] = torch.arange(f + m - K1, f + m)
-        pos, ends = places.to(dev).split([M, K1 * len(lens)])
+        upload = getattr(ops, "upload", torch.Tensor.to)
+        pos, ends = upload(places, dev).split([M, K1 * len(lens)])
         seqs_h = torch.tensor(list(zip(first, lens)), dtype=torch.int32)
         blocks_h, valid = ops.packed_blocks(first, lens, M)
-        blocks, seqs, valid = torch.cat([blocks_h.view(-1), seqs_h.view(-1), valid]).to(dev).split([blocks_h.numel(), seqs_h.numel(), valid.numel()])
+        blocks, seqs, valid = upload(torch.cat([blocks_h.view(-1), seqs_h.view(-1), valid]), dev).split([blocks_h.numel(), seqs_h.numel(), valid.numel()])
         blocks, seqs = blocks.view(-1, 4), seqs.view(-1, 2)
         none, parts = torch.zeros(512, dtype=torch.int64, device=dev), []
         for p, f, end in zip(prompts, first, first[1:] + [M]):
@@ -1031,7 +1033,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         caches = [self.initialize_inference_params() for _ in lens]
         for ipd, m in zip(caches, lens):
             ipd["mha"].max_seqlen = m
-        x = ops.embed(ids, self.embedding_layer.weight)
+        x = ops.embed(ids, self.embedding_layer.weight, **({} if later is None else {"later": later}))
         yb = ops.yblk_empty(M, D, dev).zero_()                     # (the rows between the prompts stay zero)
         nf, rs = self._nf_ok(M, None), None
         for i, blk in enumerate(self.blocks):
@@ -1079,18 +1081,24 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
     def prefill_rows(self, prompts: List[torch.Tensor], want: Optional[List[List[int]]] = None):
         """Prompts ([P] ids) of any lengths -> [(logits [wanted, V], caches, row of the caches)], several in a pass where they can share one
         (_prompt_groups); `want`: the places whose logits are returned (the last token's by default)."""
-        out = []
+        out, later = [], [] if hasattr(self.ops, "check_ids") else None
         for group in self._prompt_groups([p.numel() for p in prompts]):
             if len(group) > 1:
-                h, first, caches = self._prefill_packed([prompts[n] for n in group])
+                h, first, caches = self._prefill_packed([prompts[n] for n in group], later)
             else:
                 caches = [self.initialize_inference_params()]
                 caches[0]["mha"].max_seqlen = prompts[group[0]].numel()
-                h, first = self.hidden_states(prompts[group[0]].reshape(1, -1), caches[0]), [0]
+                h, first = self.hidden_states(prompts[group[0]].reshape(1, -1), caches[0], later=later), [0]
             at = [[prompts[n].numel() - 1] if want is None else [self._place(t, prompts[n].numel()) for t in want[n]] for n in group]
-            rows = torch.tensor([f + t for f, ts in zip(first, at) for t in ts], dtype=torch.int64, device=h.device)
-            logits = self.ops.linear(h[rows].contiguous(), self.unembed.weight, None) if rows.numel() else h.new_empty(0, self.vocab_size)
+            rows = [f + t for f, ts in zip(first, at) for t in ts]
+            if rows and rows != list(range(h.shape[0])):             # (all of them: h as it is)
+                rows = self.ops.host_rows(rows, h.device) if h.is_cuda and hasattr(self.ops, "host_rows") else torch.tensor(rows, dtype=torch.int64, device=h.device)
+                logits = self.ops.linear(h[rows].contiguous(), self.unembed.weight, None)
+            else:
+                logits = self.ops.linear(h, self.unembed.weight, None) if rows else h.new_empty(0, self.vocab_size)
             out += [(lg, ipd, 0) for lg, ipd in zip(logits.split([len(ts) for ts in at]), caches)]
+        if later:
+            self.ops.check_ids(later)
         return out
 
     # upstream names, kept for callers that reach for them

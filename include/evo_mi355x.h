@@ -70,9 +70,14 @@ extern "C" {
  *  26: evo_dense_launches added.
  *  27: evo_closing_final and evo_latent_prep_absorb added.
  *  28: evo_dense_parts, evo_dense_parts_bf16 and evo_rmsnorm_parts_bf16 added.
- *  29: evo_linear_residual_scaled_bf16, evo_linear_factors_bf16 and evo_mlp_gate_factors_bf16 added. */
-#define EVO_ABI_VERSION 29
+ *  29: evo_linear_residual_scaled_bf16, evo_linear_factors_bf16 and evo_mlp_gate_factors_bf16 added.
+ *  30: evo_token_batch added. */
+#define EVO_ABI_VERSION 30
 int evo_abi_version(void);
+
+/* Tokens of B <= 64 sequences, one sequence behind the other: cu [B + 1] their starts, seq and pos [sum of lens] sequence and position (`past` of its sequence on) of every token,
+ * resume [B] (or NULL) past > 0.  lens and past are HOST arrays, read before the call returns. */
+int evo_token_batch(int* cu, int* seq, int64_t* pos, int* resume, const int64_t* lens, const int64_t* past, int64_t B, void* stream);
 
 /* Decode pool: ids[slots[i]] = tokens[i] for i < n <= 64; slots (each below S) and tokens are HOST arrays, read before the call returns.
  * evo_advance_positions: pos[i] = min(pos[i] + 1, last).  evo_step_out: that, and out [n] fp32 = the n bf16 logits. */
