@@ -560,12 +560,12 @@ __global__ __launch_bounds__(256) void gemm_parts_kernel(GemmArgs a, int act, co
 // 147 at 2,048; 12,288 columns 76 -> 34 at 161 rows, 78 -> 58 at 512; 22,016 gated columns 82 -> 53 at 161.
 struct TileKind { int bm, bn; double step_us; };
 static const TileKind kinds[] = {{64, 64, 0.255}, {128, 64, 0.435}, {128, 128, 0.515}, {192, 128, 0.70}, {256, 128, 0.84}, {128, 256, 0.86},
-                                 {96, 96, 0.50}, {192, 96, 0.667}, {96, 48, 0.35}, {64, 96, 0.40}};
+                                 {96, 96, 0.50}, {192, 96, 0.667}, {96, 48, 0.35}, {64, 96, 0.40}, {128, 96, 0.55}};
 // The next three, below 256 rows and without parts, statistics or a transposed result: narrow enough that a layer of 12,288 to 24,576 columns is one round of
 // nearly all CUs.  us, before -> with them: 22,016 gated columns, K = 4,096 (172 tiles of 128 -> 230 of 96) 39.6 -> 37.7 at 65 rows, 42.2 -> 40.8 at 96, 48.0 -> 44.8
 // at 129, 51.7 -> 48.7 at 161, 53.6 -> 51.4 at 192; 12,288 columns (192 tiles of 64 -> 256 of 48) 27.2 -> 24.4 at 65, 29.8 -> 27.8 at 96; 11,264 columns 30.5 -> 23.5 and 33.1 -> 26.7.  Twelve waves for
-// 192 x 96 (six 49.8, four 56.7: a wave alone on its SIMD waits for its own fragments).  Not taken: 128 x 96 (43.4 - 45.1 at 97 - 128 rows, 42.4 - 46.6 with 128 x 128),
-// 256 x 96 (66.5 against 56.5 at 193) and 192 x 48 (35.7 against 34.2).  The last: tile_one_round.
+// 192 x 96 (six 49.8, four 56.7: a wave alone on its SIMD waits for its own fragments).  Not taken: 128 x 96 in step (43.4 - 45.1 at 97 - 128 rows, 42.4 - 46.6 with 128 x 128),
+// 256 x 96 (66.5 against 56.5 at 193) and 192 x 48 (35.7 against 34.2).  The last two: tile_one_round, tile_one_round_gated.
 #define T_ODD 6                              // first of them
 // The persistent kernel on tiles of 160, 192 and 224 rows (and 256 columns): a step of 64 k takes nearly as little as its operands do, where 256 rows are a round that
 // leaves a third of the chip idle or a tile that is half padding.  us, the plan without them -> with (rows of the tile): K = 4,096, 22,016 gated columns 89 -> 66 at 300 rows
@@ -660,6 +660,15 @@ static void tile_one_round(int64_t M, int64_t N, int64_t K, bool splits_ok, Tile
     else if (plan.kind == 1 && plan.splits == 1 && splits_ok && K >= 4096 && 2 * ((M + 127) / 128) * (N / 128) <= cus) plan = {2, 2, plan.us, M};
 }
 
+// Gated layers of 97 to 128 rows: 128 x 96 in phases where column tiles are nearly a round, 96 x 96 where two row tiles of them are.  us at 97 / 112 / 128 rows, before -> these: 22,016 columns of
+// K = 4,096 43.5 / 43.7 / 44.9 -> 41.8 / 41.8 / 42.7 (128 x 128 in phases before: 172 workgroups; 16,384 columns, 171, 40.8 : 41.5), 11,264 of 2,048 20.5 / 20.5 / 20.9 -> 17.0 / 17.9 / 18.4.
+static void tile_one_round_gated(int64_t M, int64_t N, int64_t K, TilePlan& plan) {
+    const int64_t cus = tile_cus(), across = (N + 95) / 96;
+    if (M <= 96 || M > 128 || K < 2048) return;
+    if (across <= cus && 8 * across >= 7 * cus) plan = {T_ODD + 4, 1, 0.95 * plan.us, M};
+    else if (2 * across <= cus && 20 * across >= 9 * cus) plan = {T_ODD, 1, 0.85 * plan.us, M};
+}
+
 static double steps_us(const StepUs& s, double rows, double cols, double nk) {
     const double cus = tile_cus(), rounds = ceil(ceil(rows / s.rows) * cols / cus), full = rows / s.rows * cols / (rounds * cus);
     return rounds * (nk * (s.us + s.more * fmax(0.0, full - s.from)) + s.end);
@@ -674,6 +683,7 @@ static double steps_us(const StepUs& s, double rows, double cols, double nk) {
 static int tile_plan(int64_t M, int64_t N, int64_t K, int mode, bool stats, bool splits_ok, bool persistent_ok, bool short_ok, TilePlan (&out)[2]) {
     const int n = tile_plan_square(M, N, K, mode, stats, splits_ok, persistent_ok, out);
     if (mode == 0 && M < 256 && !stats) tile_one_round(M, N, K, splits_ok, out[0]);
+    if (mode == 1 && M < 256) tile_one_round_gated(M, N, K, out[0]);
     if (!persistent_ok || !short_ok || M < 256 || K < 2048) return n;
     const double memory = (2.0 * (M * K + N * K) + 2.0 * M * N) / 4.9e6, nk = (double)(K / 64);
     const double rows = (double)(mode == 3 ? N : M), cols = (double)((mode == 3 ? M : N) / 256);       // (mode 3: the tokens are the columns of the launch)
@@ -702,6 +712,7 @@ static int tile_phases(int kind, int mode, bool xblk, int splits, int64_t M, int
     if (kind == 2) return K >= 1024 && 4 * M <= N && (M - 1) % 128 >= (M > 512 ? 119 : 95) ? 6 : 0;
     if (kind == T_ODD) return mode == 0 ? (M > 160 ? 8 : 0) : M >= 80 && M <= 96 && K >= 4096 ? 8 : 0;
     if (kind == T_ODD + 1) return M >= 150 && M <= 192 && K >= 1024 ? 5 : 0;
+    if (kind == T_ODD + 4) return 7;
     return 0;
 }
 
@@ -907,7 +918,8 @@ extern "C" int evo_dense_bf16(int64_t mode, int64_t act, int64_t xblk, const voi
             else if (t.kind == 3) rc = tile_launch<192, 128, 4, 2, 4, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
             else if (t.kind == 4) rc = tile_launch<256, 128, 4, 2, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
             else if (t.kind == 5) rc = tile_launch<128, 256, 2, 4, 3, 1, true>(a, tm, (int)act, xblk != 0, t.splits, f, st);
-            else if (xblk || tm > 1 || (tm == 1 ? t.kind >= T_ODD + 2 : t.kind == T_ODD + 1)) rc = -1;
+            else if (xblk || tm > 1 || (tm == 1 ? t.kind == T_ODD + 2 || t.kind == T_ODD + 3 : t.kind == T_ODD + 1 || t.kind == T_ODD + 4)) rc = -1;
+            else if (t.kind == T_ODD + 4) rc = tile_launch_odd<128, 96, 4, 1, 17, 1>(a, (int)act, st);
             else if (tm == 0 && t.kind == T_ODD) rc = phases ? tile_launch_odd<96, 96, 2, 3, 18, 0>(a, (int)act, st) : tile_launch_odd<96, 96, 2, 3, 6, 0>(a, (int)act, st);
             else if (t.kind == T_ODD + 3) rc = tile_launch_odd<64, 96, 2, 2, 7, 0>(a, (int)act, st);
             else if (t.kind == T_ODD) rc = phases ? tile_launch_odd<96, 96, 2, 3, 18, 1>(a, (int)act, st) : tile_launch_odd<96, 96, 2, 3, 6, 1>(a, (int)act, st);

@@ -42,3 +42,28 @@ def test_what_stays(M, N, K):
     out = (ctypes.c_int64 * 16)()
     assert default_ops().lib.evo_dense_launches(0, 0, 0, M, N, K, ctypes.cast(out, ctypes.c_void_p)) == 1
     assert (out[2], out[3]) not in ((96, 96), (64, 96)) and (out[2], out[3], out[4]) != (128, 128, 2) and ((out[2], out[3]) != (96, 48) or M == 96)
+
+
+@pytest.mark.parametrize("M,N,K,tile", [(97, 22016, 4096, (128, 96, 1, 7)), (112, 21760, 2112, (128, 96, 1, 7)), (128, 24576, 2048, (128, 96, 1, 7)), (97, 11264, 2048, (96, 96, 1, 0)),
+                                        (128, 12288, 4096, (96, 96, 1, 0))])
+def test_gated_tiles_of_one_round(M, N, K, tile):
+    """Both gates on either order of the weight, with and without row factors.  A value of z on the edge of two bf16 numbers may round the other way: 2^-8 of it, through a slope of at
+    most 1.13 and the other factor."""
+    from evo_amd.ops import _stream, default_ops
+    ops = default_ops()
+    out = (ctypes.c_int64 * 16)()
+    assert ops.lib.evo_dense_launches(1, 0, 0, M, N, K, ctypes.cast(out, ctypes.c_void_p)) == 1 and (out[2], out[3], out[4], out[7]) == tile
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x, w = torch.randn(M, K, device="cuda", generator=g).bfloat16(), (torch.randn(N, K, device="cuda", generator=g) / K ** 0.5).bfloat16()
+    rs = torch.rand(M, device="cuda", generator=g) + 0.5
+    z = x.double() @ w.double().T
+    for order, act, scale in ((1, 0, False), (2, 0, True), (1, 1, True), (2, 1, False)):
+        wk, y = ops.pack_gate_weights(w) if order == 1 else w, torch.full((M + 3, N // 2), 7.0, device="cuda", dtype=torch.bfloat16)
+        assert ops.lib.evo_dense_bf16(order, act, 0, x.data_ptr(), wk.data_ptr(), None, None, y.data_ptr(), rs.data_ptr() if scale else None, None, 0, M, N, K, 0, 0, 0, 0, None, 0,
+                                      _stream()) == 0
+        zz = (z * rs.double()[:, None] if scale else z).bfloat16().double()
+        z1, z2 = zz[:, :N // 2], zz[:, N // 2:]
+        want = (torch.nn.functional.silu(z1) if act else torch.nn.functional.gelu(z1)) * z2
+        err = (y[:M].double() - want).abs()
+        assert bool((err <= want.abs() * 2.0 ** -7 + (z1.abs() + 0.2) * z2.abs() * 2.0 ** -7 + 1e-3).all()), err.max().item()
+        assert bool((y[M:] == 7).all())
