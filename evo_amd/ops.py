@@ -499,7 +499,7 @@ class HipOps(MixerOps):
         M, K = x.shape
         if M <= 64:
             return self.linear_parts(x, w)
-        if M >= 1024 or not self._take_mfma(mfma) or not self.mfma_linear_ok(x, w) or (x.data_ptr() | w.data_ptr()) % 16:
+        if M >= 1024 or w.shape[1] != K or not self._take_mfma(mfma) or not self.mfma_linear_ok(x, w) or (x.data_ptr() | w.data_ptr()) % 16:
             return None
         n = self.lib.evo_dense_parts(M, w.shape[0], K)
         if n <= 0:
@@ -514,8 +514,8 @@ class HipOps(MixerOps):
         """res += x @ w^T (+ bias) in place, as linear_residual_, and rmsnorm(res) * scale -- where the layer is summed in parts that the norm's launch can add; elsewhere
         None, and nothing is done."""
         M, D = res.shape
-        if not (17 <= M < 1024 and 8 <= D <= 8192 and res.dtype == scale.dtype == torch.bfloat16 and res.is_contiguous() and scale.is_contiguous() and w.shape[0] == D
-                and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous()))
+        if not (17 <= M < 1024 and 8 <= D <= 8192 and res.dtype == scale.dtype == torch.bfloat16 and res.is_contiguous() and scale.is_contiguous() and w.shape[0] == scale.numel() == D
+                and tuple(x.shape) == (M, w.shape[1]) and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous()))
                 and (res.data_ptr() | scale.data_ptr() | (0 if bias is None else bias.data_ptr())) % 16 == 0):
             return None
         parts = self.layer_parts(x, w, mfma)
@@ -538,7 +538,7 @@ class HipOps(MixerOps):
         linear_factors and mlp_gate_factors take; None, and nothing is done, for layers that the launch is not for."""
         M, K = x.shape
         N = w.shape[0]
-        if not (5 <= M <= 32 and 2048 <= N <= 4096 and N % 64 == 0 and K % 128 == 0 and 1024 < K and self._use_small_m(x, w) and res.dtype == scale.dtype == torch.bfloat16
+        if not (5 <= M <= 32 and 2048 <= N <= 4096 and N % 64 == 0 and K % 128 == 0 and 1024 < K and w.shape[1] == K and self._use_small_m(x, w) and res.dtype == scale.dtype == torch.bfloat16
                 and tuple(res.shape) == (M, N) and res.is_contiguous() and scale.is_contiguous() and scale.numel() == N
                 and (bias is None or (bias.dtype == torch.bfloat16 and bias.is_contiguous()))
                 and (x.data_ptr() | w.data_ptr() | res.data_ptr() | scale.data_ptr() | (0 if bias is None else bias.data_ptr())) % 16 == 0 and self.lib.evo_linear_parts(M, N, K) == 0):
