@@ -4,6 +4,7 @@ arithmetic is fp32."""
 from __future__ import annotations
 
 import functools
+import inspect
 from dataclasses import dataclass
 from typing import List, Optional, Sequence, Tuple
 
@@ -12,6 +13,15 @@ import torch
 LC = 64                                     # tokens per chunk of the linear-attention kernel
 ACTIVATIONS = {"silu": 1, "gelu_tanh": 2, "relu2": 3}
 _DECODE_COLUMNS = (1, 2, 3, 4, 6, 8, 12, 16)   # latent widths, in units of 32, the matrix-core decode kernel is built for
+
+
+def takes(method, keyword: str) -> bool:
+    """Whether a method has the keyword, one of those that programs' own versions of it -- a subclass's, an op set's, a wrapper's -- need not have: they are called as before then."""
+    f = getattr(method, "__func__", method)
+    code = getattr(f, "__code__", None)
+    if code is None or not (keyword in code.co_varnames[:code.co_argcount + code.co_kwonlyargcount] or code.co_flags & inspect.CO_VARKEYWORDS):
+        return False
+    return not hasattr(f, "__wrapped__") or takes(f.__wrapped__, keyword)
 
 
 @dataclass
@@ -57,7 +67,8 @@ class Stream:
     def __init__(self, ops, ids: torch.Tensor, weight: torch.Tensor, scale: float, eps: float, w_offset: float, alpha: Optional[float] = None,
                  ids_known: bool = False, later: Optional[list] = None):
         self.ops, self.eps, self.w_offset, self.alpha = ops, eps, w_offset, alpha
-        self.x, self.xb = ops.embed_stream(ids, weight, scale, **({"validate": False} if ids_known else {} if later is None else {"later": later}))
+        more = {"validate": False} if ids_known else {} if later is None else {"later": later}
+        self.x, self.xb = ops.embed_stream(ids, weight, scale, **{k: v for k, v in more.items() if takes(ops.embed_stream, k)})
         self.open = None                                         # (y, w): still to be added
         self.spare = None                                        # the buffer the next such launch writes x to
         self.behind = False                                      # xb does not hold the current x

@@ -13,7 +13,7 @@ from typing import Dict, List, Optional
 import torch
 import torch.nn as nn
 
-from .mixer_ops import Stream, TokenBatch
+from .mixer_ops import Stream, TokenBatch, takes
 
 
 def _need(cfg: dict, key: str, where: str):
@@ -155,7 +155,7 @@ class LatentAttention(Sublayer):
         qd = stream.linear(self.w_in)                             # [queries | latent, shared key]
         if batch.decode:
             more = {}
-            if hasattr(ops, "latent_prep_fits") and ops.latent_prep_fits(qd, cache, self.w_norm, self.inv_freq, H, dn, dr, R):
+            if hasattr(ops, "latent_prep_fits") and takes(ops.latent_decode, "prep") and ops.latent_prep_fits(qd, cache, self.w_norm, self.inv_freq, H, dn, dr, R):
                 more["prep"] = (self.w_norm, self.inv_freq, self.eps)
             else:
                 ops.latent_prep(qd, H, dn, dr, R, self.w_norm, self.inv_freq, self.eps, batch, cache, want_kv=False)

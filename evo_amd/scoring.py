@@ -12,6 +12,7 @@ from typing import List, Tuple
 import numpy as np
 import torch
 
+from .mixer_ops import takes
 from .tokenizer import CharLevelTokenizer
 
 
@@ -94,7 +95,7 @@ def score_logprobs_device(model, input_ids: torch.Tensor, want_entropy: bool = F
     B, T = input_ids.shape
     if _fused_tail_ok(model, input_ids):
         with torch.no_grad():
-            hid = model.hidden_states(input_ids, **({"ids_known": True} if ids_known else {}))      # [B*T, D] final-norm output
+            hid = model.hidden_states(input_ids, **({"ids_known": True} if ids_known and takes(model.hidden_states, "ids_known") else {}))      # [B*T, D] final-norm output
             tgt = None
             if not want_entropy:
                 tgt = torch.full((B, T), -1, dtype=torch.int64, device=hid.device)

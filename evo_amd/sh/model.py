@@ -19,6 +19,7 @@ from typing import Dict, List, NamedTuple, Optional, Tuple
 import torch
 import torch.nn as nn
 
+from ..mixer_ops import takes
 from .cache import InferenceParams, RecurrentInferenceParams
 from .graph import DecodeGraphMixin
 from .utils import dotdict
@@ -856,13 +857,14 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             out, b0 = None, 0
             for nb in groups:
                 pm = None if padding_mask is None else padding_mask[b0:b0 + nb]
-                hg = self.hidden_states(x[b0:b0 + nb], None, pm, ids_known)
+                hg = self.hidden_states(x[b0:b0 + nb], None, pm, **({"ids_known": True} if ids_known and takes(self.hidden_states, "ids_known") else {}))
                 if out is None:
                     out = torch.empty(B * T, hg.shape[1], dtype=hg.dtype, device=hg.device)
                 out[b0 * T:(b0 + nb) * T] = hg
                 b0 += nb
             return out
-        h = ops.embed(x.to(self.device), self.embedding_layer.weight, **({"validate": False} if ids_known else {} if later is None else {"later": later}))             # [B*T, D]
+        more = {"validate": False} if ids_known else {} if later is None else {"later": later}
+        h = ops.embed(x.to(self.device), self.embedding_layer.weight, **{k: v for k, v in more.items() if takes(ops.embed, k)})             # [B*T, D]
         mask = None
         if padding_mask is not None:
             pm = padding_mask.to(self.device) != 0
@@ -1033,7 +1035,7 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         caches = [self.initialize_inference_params() for _ in lens]
         for ipd, m in zip(caches, lens):
             ipd["mha"].max_seqlen = m
-        x = ops.embed(ids, self.embedding_layer.weight, **({} if later is None else {"later": later}))
+        x = ops.embed(ids, self.embedding_layer.weight, **({} if later is None or not takes(ops.embed, "later") else {"later": later}))
         yb = ops.yblk_empty(M, D, dev).zero_()                     # (the rows between the prompts stay zero)
         nf, rs = self._nf_ok(M, None), None
         for i, blk in enumerate(self.blocks):
@@ -1088,7 +1090,8 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
             else:
                 caches = [self.initialize_inference_params()]
                 caches[0]["mha"].max_seqlen = prompts[group[0]].numel()
-                h, first = self.hidden_states(prompts[group[0]].reshape(1, -1), caches[0], later=later), [0]
+                h = self.hidden_states(prompts[group[0]].reshape(1, -1), caches[0], **({"later": later} if later is not None and takes(self.hidden_states, "later") else {}))
+                first = [0]
             at = [[prompts[n].numel() - 1] if want is None else [self._place(t, prompts[n].numel()) for t in want[n]] for n in group]
             rows = [f + t for f, ts in zip(first, at) for t in ts]
             if rows and rows != list(range(h.shape[0])):             # (all of them: h as it is)
