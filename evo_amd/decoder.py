@@ -208,6 +208,8 @@ class LayeredDecoder(DecodeGraphMixin, nn.Module):
                 tokens += prompts[first + n].numel()
                 n += 1
             group = prompts[first:first + n]
+            if later:                                                # (the GPU has the last pass's layers to run meanwhile)
+                self.ops.check_ids(later, keep=1)
             lens = [p.numel() for p in group]
             ipd = self.allocate_rows(n, max(lens))
             h = self._run(torch.cat([p.reshape(-1) for p in group]), TokenBatch.of_prompts(lens, [0] * n, self.device, self.ops), ipd, later=later)

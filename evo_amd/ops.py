@@ -602,9 +602,10 @@ class HipOps(MixerOps):
         later.append((host, done, vocab))
 
     @staticmethod
-    def check_ids(later: list) -> None:
-        """raise_bad_ids for embeddings whose layers are on their way: a wait for the embedding alone."""
-        for host, done, vocab in later:
+    def check_ids(later: list, keep: int = 0) -> None:
+        """raise_bad_ids for embeddings whose layers are on their way, all but the last `keep` of them: a wait for the embeddings alone."""
+        while len(later) > keep:
+            host, done, vocab = later.pop(0)
             done.synchronize()
             if int(host.item()) != 0:
                 raise IndexError(f"input_ids contain values outside [0, {vocab}) (embedding table has {vocab} rows)")

@@ -1085,6 +1085,8 @@ class StripedHyena(DecodeGraphMixin, nn.Module):
         (_prompt_groups); `want`: the places whose logits are returned (the last token's by default)."""
         out, later = [], [] if hasattr(self.ops, "check_ids") else None
         for group in self._prompt_groups([p.numel() for p in prompts]):
+            if later:                                                # (the GPU has the last pass's layers to run meanwhile)
+                self.ops.check_ids(later, keep=1)
             if len(group) > 1:
                 h, first, caches = self._prefill_packed([prompts[n] for n in group], later)
             else:
