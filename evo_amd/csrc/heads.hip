@@ -221,7 +221,7 @@ struct HDecArgs {
 // Heads are the grid's fastest index: workgroup i runs on XCD i % 8, and behind a short sequence's tokens whole parts have nothing to do (parts first, 16 heads of
 // two maps in 5 to 8 parts: 1 / 3 sequences of up to 300 16.6 / 17.7 -> 14.1 / 15.0; key heads of four queries alike).
 // KS: 32-wide steps of a key, NG: 32-wide groups of a value, MAPS: maps per head ([map 1 | map 2] in keys and queries).
-template <int KS, int NG, int MAPS>
+template <int KS, int NG, int MAPS, bool ONCE>
 __global__ __launch_bounds__(256) void heads_decode_kernel(HDecArgs a) {
     constexpr int VP = 32 * NG + 8, AP = 32 * NG + 4;            // pitches of the value tiles and of the meeting place
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
@@ -267,13 +267,16 @@ __global__ __launch_bounds__(256) void heads_decode_kernel(HDecArgs a) {
                 }
         }
     };
-    // item: eight values of a slot.  A request is whole lines that nobody reads again (non-temporal: 239 / 526 MB of keys and values 58.7 / 104 -> 56.8 / 97.9 us, one map 17.0 /
-    // 28.9 -> 16.1 / 26.7 at 60 / 119 MB); the keys' requests are halves of lines, which have to be there for the other half (the same for them: 2 to 17 % slower)
+    // item: eight values of a slot.  ONCE: a key head's query heads are one block, so a request is whole lines that nobody reads again (non-temporal: 239 / 526 MB of keys and
+    // values 58.7 / 104 -> 56.8 / 97.9 us, one map 17.0 / 28.9 -> 16.1 / 26.7 at 60 / 119 MB).  Of several blocks each reads the values: 24 caches of 2,000 slots, 8 key heads of
+    // 64, 32 / 64 query heads each 43.4 / 67.7 us so, 44.8 / 73.1 non-temporal; 4 of 30,000, 2 of two maps, 32 each 86.6 : 87.6.  The keys' requests are halves of lines, which have
+    // to be there for the other half (non-temporal 2 to 17 % slower)
     auto load_v = [&](int s0) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < 2 * NG; ++i) {
             const int it = lane + 64 * i, r = s0 + it / (4 * NG), d = 8 * (it % (4 * NG));
-            rv[i] = __builtin_nontemporal_load((const mx_u32x4*)(vbase + (int64_t)(r < used ? r : last) * a.rs + (d < dv ? d : dv - 8)));
+            const mx_u32x4* p = (const mx_u32x4*)(vbase + (int64_t)(r < used ? r : last) * a.rs + (d < dv ? d : dv - 8));
+            if constexpr (ONCE) rv[i] = __builtin_nontemporal_load(p); else rv[i] = *p;
         }
     };
     const int step = a.n_split * 128;
@@ -561,16 +564,18 @@ static int heads_decode(void* o, float lam, float gain, float eps, const void* z
     if (!f32 && mfma && dim % 8 == 0 && dv % 8 == 0 && ld % 8 == 0 && rs % 8 == 0 && dim <= (maps == 2 ? 128 : 256) && dv <= 256 &&
         (((uintptr_t)z | (uintptr_t)cache | (uintptr_t)part_o | (uintptr_t)o) & 15) == 0 && (!o || maps * (Q < 16 ? Q : 16) <= 16)) {
         const dim3 grid((unsigned)(kv_heads * a.n_qb), (unsigned)n_split, (unsigned)B);
-#define HD(KS, NG, MAPS)                                                                                                   \
+#define HD(KS, NG, MAPS) do { if (a.n_qb == 1) HDO(KS, NG, MAPS, true); else HDO(KS, NG, MAPS, false); } while (0)
+#define HDO(KS, NG, MAPS, ONCE)                                                                                            \
     do {                                                                                                                   \
         constexpr int tiles = 4 * 32 * (32 * NG + 8) * 2, meet = (MAPS == 1 ? 4 : MAPS) * 16 * (32 * NG + 4) * 4, bytes = tiles > meet ? tiles : meet;   \
-        if (bytes > 60 * 1024) (void)hipFuncSetAttribute((const void*)heads_decode_kernel<KS, NG, MAPS>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes); \
-        hipLaunchKernelGGL((heads_decode_kernel<KS, NG, MAPS>), grid, dim3(256), (size_t)bytes, s, a);                     \
+        if (bytes > 60 * 1024) (void)hipFuncSetAttribute((const void*)heads_decode_kernel<KS, NG, MAPS, ONCE>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes); \
+        hipLaunchKernelGGL((heads_decode_kernel<KS, NG, MAPS, ONCE>), grid, dim3(256), (size_t)bytes, s, a);               \
     } while (0)
 #define HDV(KS, MAPS) do { if (dv <= 64) HD(KS, 2, MAPS); else if (dv <= 128) HD(KS, 4, MAPS); else HD(KS, 8, MAPS); } while (0)
         if (maps == 2) { if (dim <= 64) HDV(2, 2); else HDV(4, 2); }
         else if (dim <= 64) HDV(2, 1); else if (dim <= 128) HDV(4, 1); else HDV(8, 1);
 #undef HDV
+#undef HDO
 #undef HD
         return evo_launch_status();
     }

@@ -177,6 +177,19 @@ def test_decode_attention(ops, mfma, dt, H, G, maps, n, dv, keep, window):
             assert rel_err(got[b:b + 1], want.reshape(1, -1)) < tol(dt, 1.5e-2 if maps == 1 else 3e-2, 2e-5), (b, n_split)
 
 
+@pytest.mark.parametrize("maps,n,dv", [(1, 64, 64), (1, 128, 200), (2, 128, 256)])
+def test_blocks_of_query_heads(ops, maps, n, dv):
+    """33 query heads of a key head, in three workgroups that read the values each: the bits of 16, 16 and one, whose values are read once."""
+    ring, B = 200, 3
+    cache, z = rnd(B, ring, maps * n + dv, seed=1, dt=BF).to(DEV), rnd(B, 33 * maps * n, seed=2, dt=BF).to(DEV)
+    pos = torch.tensor([3, 150, 500]).to(DEV)
+
+    def go(first, heads):
+        q = z.view(B, 33, maps * n)[:, first:first + heads].reshape(B, -1)
+        return ops.heads_decode(q, cache, pos, heads, 1, maps, n, dv, n ** -0.5, 0.4, 1.0, 1e-5, n_split=2)
+    assert torch.equal(go(0, 33), torch.cat([go(0, 16), go(16, 16), go(32, 1)], 1))
+
+
 def test_split_covers_the_cache():
     from evo_amd.mixer_ops import MixerOps
     for groups in (1, 8, 300, 5000):
