@@ -43,10 +43,12 @@ __device__ __forceinline__ void fill_turns(float2* turn, const HeadsArgs& a, int
 }
 
 // LG lanes per vector, 16 elements each: a run of eight and its partners half a rotation further, or two runs that are not rotated.
-// n_rot % 16 == 0, dim % 8 == 0, 16-byte aligned rows.  What a thread's first vector needs, its norm's weight and its values are asked for before the angles, and few
+// n_rot % 16 == 0, dim % 8 == 0, 16-byte aligned rows.  AHEAD: what a thread's first vector needs, its norm's weight and its values are asked for before the angles, and few
 // tokens' vectors are shared out over gridDim.y workgroups: a decode step's launch is a chain of latencies (24 tokens of 40 and 64
-// vectors of 128 in a step of four layers 5.5 -> 4.2 us)
-template <typename T, int LG>
+// vectors of 128 in a step of four layers 5.5 -> 4.2 us).  Many tokens' workgroups hide each other's, and there the registers that wait cost a workgroup per CU, and threads
+// without a vector ask for one all the same.  us, requests behind the angles and weights behind the sum -> ahead -> weights with the values, behind the angles: 12,000 tokens of
+// two fp32 vectors of 64 17.6 -> 27.5 -> 16.1; 3,000 of 16 bf16 vectors of 256, rotated 19.1 -> 21.3 -> 18.4; 2,000 of 32 of 64 8.6 -> 9.1 -> 8.0.
+template <typename T, int LG, bool AHEAD>
 __global__ __launch_bounds__(256) void heads_prep_kernel(HeadsArgs a) {
     extern __shared__ float2 turn[];                             // [n_rot / 2] cosine and sine of this token's angles, times the amplitude
     constexpr int PER = 256 / LG;
@@ -69,14 +71,16 @@ __global__ __launch_bounds__(256) void heads_prep_kernel(HeadsArgs a) {
             vec_io<T, 8>::load(w + lb, gy);
         }
     };
-    fetch(h_first);
-    if (vi + 7 < a.nv) vec_io<T, 8>::load(values + vi, val);
+    if constexpr (AHEAD) {
+        fetch(h_first);
+        if (vi + 7 < a.nv) vec_io<T, 8>::load(values + vi, val);
+    }
     const int64_t pos = a.pos[m];
     T* slot = cache_row<T>(a, m, pos);
     fill_turns(turn, a, pos);
     __syncthreads();
     for (int h = h_first; h < nh; h += step) {
-        if (h != h_first) fetch(h);
+        if (!AHEAD || h != h_first) fetch(h);
         T* v = z + (int64_t)h * a.dim;
 #pragma unroll
         for (int e = 0; e < 8; ++e) { x[e] = ha ? x[e] : 0.f; y[e] = hb ? y[e] : 0.f; }
@@ -115,8 +119,8 @@ __global__ __launch_bounds__(256) void heads_prep_kernel(HeadsArgs a) {
     }
     if (slot) {
         T* d = slot + (int64_t)a.nk * a.dim;
-        if (vi + 7 < a.nv) vec_io<T, 8>::store(d + vi, val);
-        for (int i = vi + gridDim.y * 2048; i + 7 < a.nv; i += gridDim.y * 2048) {
+        if (AHEAD && vi + 7 < a.nv) vec_io<T, 8>::store(d + vi, val);
+        for (int i = AHEAD ? vi + gridDim.y * 2048 : vi; i + 7 < a.nv; i += gridDim.y * 2048) {
             vec_io<T, 8>::load(values + i, val);
             vec_io<T, 8>::store(d + i, val);
         }
@@ -184,13 +188,16 @@ extern "C" int evo_heads_prep(void* z, int64_t ld, void* cache, const void* qw, 
     const int64_t lanes = n_rot / 16 + (dim - n_rot + 15) / 16;
     if (n_rot % 16 == 0 && dim % 8 == 0 && lanes <= 64 && ld % 8 == 0 && rs % 8 == 0 && (((uintptr_t)z | (uintptr_t)cache | (uintptr_t)qw | (uintptr_t)kw) & 15) == 0) {
         // (a workgroup's vectors in one round each while that leaves them a CU of their own)
+        // Ahead: up to 512 tokens; fp32 vectors of half the threads and more from 1,000 tokens on again (16 of 256 at 3,000 47.7 -> 41.0 us, 45.8 without; 700 of 16, rotated 10.2 -> 11.1, 10.0)
+#define HPT(T, LG) do { if (M <= 512 || (f32 && M >= 1000 && (nq + nk) * LG >= 128)) hipLaunchKernelGGL((heads_prep_kernel<T, LG, true>), g2, block, lds, s, a); \
+                        else hipLaunchKernelGGL((heads_prep_kernel<T, LG, false>), g2, block, lds, s, a); } while (0)
 #define HP(LG) do { const int64_t rounds = ((nq + nk) * LG + 255) / 256, parts = 256 / M < 1 ? 1 : 256 / M;                \
                     const dim3 g2((unsigned)M, (unsigned)(rounds < parts ? rounds : parts));                               \
-                    if (f32) hipLaunchKernelGGL((heads_prep_kernel<float, LG>), g2, block, lds, s, a);                     \
-                    else hipLaunchKernelGGL((heads_prep_kernel<uint16_t, LG>), g2, block, lds, s, a); } while (0)
+                    if (f32) HPT(float, LG); else HPT(uint16_t, LG); } while (0)
         if (lanes <= 1) HP(1); else if (lanes <= 2) HP(2); else if (lanes <= 4) HP(4); else if (lanes <= 8) HP(8);
         else if (lanes <= 16) HP(16); else if (lanes <= 32) HP(32); else HP(64);
 #undef HP
+#undef HPT
         return evo_launch_status();
     }
     if (f32) hipLaunchKernelGGL((heads_prep_any_kernel<float>), grid, block, lds + (size_t)dim * 16, s, a);

@@ -86,6 +86,26 @@ def test_heads_prep_shared_out(ops, dt, nq, nk, dim, nv, n_rot, keep, window, no
     test_heads_prep(ops, dt, nq, nk, dim, nv, n_rot, keep, window, norm)
 
 
+@TYPES
+@pytest.mark.parametrize("M", [512, 513, 999, 1000, 1500])
+@pytest.mark.parametrize("nq,nk,dim,nv,n_rot", [(1, 1, 64, 24, 32), (16, 16, 64, 2056, 32), (3, 2, 256, 515, 0)])
+@pytest.mark.parametrize("norm", ["weights", "unit"])
+def test_heads_prep_of_many_tokens(ops, dt, M, nq, nk, dim, nv, n_rot, norm):
+    """What many tokens' workgroups ask for first is nothing that their results or the cache show: the bits of the same tokens, at most 500 a call."""
+    from evo_amd.mixer_ops import TokenBatch
+    cols = (nq + nk) * dim + nv
+    z = rnd(M, (cols + 7) // 8 * 8, seed=1, dt=dt).to(DEV)
+    qk = (rnd(dim, seed=2, dt=dt).to(DEV), rnd(dim, seed=3, dt=dt).to(DEV)) if norm == "weights" else None
+    inv = torch.rand(n_rot // 2, generator=torch.Generator().manual_seed(4)).to(DEV)
+    got = []
+    for step in (M, 500):
+        x, cache = z.clone(), torch.full((1, M + 3, (nk * dim + nv + 7) // 8 * 8), 5.0, dtype=dt, device=DEV)
+        for at in range(0, M, step):
+            n = min(step, M - at)
+            ops.heads_prep(x[at:at + n], nq, nk, dim, nv, qk, inv, 1.25, norm == "unit", 1e-5, TokenBatch.of_prompts([n], [at], DEV), cache, 0)
+        got.append((x, cache))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
 
 # ------------------------------------------------------------------------------------------------ prompts
 def combine(q, k, v, maps, scale, lam, gain, eps, mask):
