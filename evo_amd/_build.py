@@ -47,7 +47,7 @@ COMPONENTS = {
         "evo_window_attn",
     ]),
     "lightning": ("_lightning", ["lightning"], ["mixers_common.h"], ["evo_lightning_chunk_bf16", "evo_lightning_recurrent"]),
-    "latent": ("_latent", ["latent"], ["mixers_common.h"], ["evo_latent_prep", "evo_latent_absorb", "evo_latent_prep_absorb", "evo_latent_decode", "evo_latent_up"]),
+    "latent": ("_latent", ["latent"], ["mixers_common.h"], ["evo_latent_prep", "evo_latent_absorb", "evo_latent_prep_absorb", "evo_latent_decode", "evo_latent_forms", "evo_latent_up"]),
     "heads": ("_heads", ["heads"], ["mixers_common.h"], ["evo_heads_prep", "evo_heads_decode", "evo_heads_decode_whole", "evo_heads_merge"]),
     "rglru": ("_rglru", ["rglru"], ["mixers_common.h"], ["evo_rglru_chunk_bf16", "evo_rglru_step_bf16", "evo_rglru_any"]),
 }

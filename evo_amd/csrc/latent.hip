@@ -189,7 +189,8 @@ extern "C" int evo_latent_prep(void* q, int64_t ldq, void* c, void* kr, void* ca
 // before anything else, and columns are halved while that leaves fewer than 256 workgroups.
 // PREP: q comes as the projection wrote it.  The heads' first workgroups rotate (the queries stay as they are), and one more "head" norms and rotates the tokens' own rows
 // for the cache, a wave a token: latent_prep and this in one launch, with the bits of two.  In a step of four layers, 8 sequences, 32 heads of 128 x 512: 11.8 us in two
-// launches with 128 workgroups' columns here, 7.4 so (3.1 of them the requests' latency, the map being cold); columns halved to 256 instead of 128 workgroups 0.4 to 1.3
+// launches with 128 workgroups' columns here, 7.4 so (3.1 of them the requests' latency, the map being cold); 256 columns at most: angles and eight sequences' columns are registers
+// that a CU's other workgroups lack (128 heads at 64 sequences 71 us with 512, 58 so, 38.1 in two launches, which are ahead there: MixerOps.latent_prep_fits); columns halved to 256 instead of 128 workgroups 0.4 to 1.3
 // (3 / 4 / 8 sequences 23.4 / 24.9 / 26.0 -> 22.2 / 23.6 / 25.6, all launches of the layer).  Queries lie [dn][NB]: a row's are one LDS request instead of
 // NB (8 / 16 / 32 sequences 25.6 / 29.3 / 38.7 -> 25.2 / 28.6 / 38.3).
 template <typename T, int NB, int V, bool PREP>
@@ -307,13 +308,20 @@ __global__ __launch_bounds__(512) void latent_absorb_kernel(const void* __restri
     }
 }
 
+// What a workgroup of the query side takes: nb sequences, 64 v columns (wuk aligned to 16 bytes)
+struct AbsorbForm { int nb, v; };
+static AbsorbForm absorb_form(int64_t B, int64_t H, int64_t R, bool aligned, bool prep) {
+    AbsorbForm f = {B > 2 ? 4 : (int)B, R % 8 == 0 && aligned ? (prep ? 4 : 8) : 1};
+    while (f.v > 2 && ((R + 64 * f.v - 1) / (64 * f.v)) * H * ((B + f.nb - 1) / f.nb) < 256) f.v /= 2;
+    return f;
+}
+
 // prep: null, or the preparation's arguments
 static int latent_absorb(const void* q, int64_t ldq, const void* wuk, void* out, int64_t B, int64_t H, int64_t dn, int64_t dr, int64_t R, int64_t rs, const PrepArgs* prep,
                          int64_t f32, void* stream) {
     if (!q || !wuk || !out || B <= 0 || H <= 0 || H > (prep ? 65534 : 65535) || dn <= 0 || dn > 4096 || dr < 0 || R <= 0 || rs < R + dr || ldq < H * (dn + dr)) return -1;
-    const int nb = B > 2 ? 4 : (int)B;
-    int v = R % 8 == 0 && ((uintptr_t)wuk & 15) == 0 ? 8 : 1;
-    while (v > 2 && ((R + 64 * v - 1) / (64 * v)) * H * ((B + nb - 1) / nb) < 256) v /= 2;
+    const AbsorbForm form = absorb_form(B, H, R, ((uintptr_t)wuk & 15) == 0, prep != nullptr);
+    const int nb = form.nb, v = form.v;
     const dim3 grid((unsigned)((R + 64 * v - 1) / (64 * v)), (unsigned)(H + (prep ? 1 : 0)), (unsigned)((B + nb - 1) / nb)), block(512);
     const size_t lds = (size_t)nb * (dn + 512 * v) * 4;          // (<= 128 KB)
     hipStream_t s = (hipStream_t)stream;
@@ -323,7 +331,7 @@ static int latent_absorb(const void* q, int64_t ldq, const void* wuk, void* out,
         if (lds > 64 * 1024) (void)hipFuncSetAttribute((const void*)latent_absorb_kernel<T, NB, V, P>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
         hipLaunchKernelGGL((latent_absorb_kernel<T, NB, V, P>), grid, block, lds, s, q, ldq, wuk, out, (int)B, (int)H, (int)dn, (int)dr, (int)R, (int)rs, a); \
     } while (0)
-#define ABP(T, NB, V) do { if (prep) AB(T, NB, V, true); else AB(T, NB, V, false); } while (0)
+#define ABP(T, NB, V) do { if constexpr (V == 8) AB(T, NB, V, false); else if (prep) AB(T, NB, V, true); else AB(T, NB, V, false); } while (0)
 #define ABV(T, V) do { if (nb == 1) ABP(T, 1, V); else if (nb == 2) ABP(T, 2, V); else ABP(T, 4, V); } while (0)
     if (f32) { if (v == 8) ABV(float, 8); else if (v == 4) ABV(float, 4); else if (v == 2) ABV(float, 2); else ABV(float, 1); }
     else { if (v == 8) ABV(uint16_t, 8); else if (v == 4) ABV(uint16_t, 4); else if (v == 2) ABV(uint16_t, 2); else ABV(uint16_t, 1); }
@@ -754,15 +762,14 @@ __global__ __launch_bounds__(512) void latent_up_kernel(const float* __restrict_
 
 // The same on the matrix cores (bf16, R % 32 == 0): VR value rows of one head and NS sequences, a wave owns 16 of the rows.  Latency and the pace of one CU bound
 // it: at 8 sequences of 16 parts a head's merge reads 262 KB, its rows 131 KB.  So sequences, then rows, are spread over up to 256 workgroups (a head's rows and parts are
-// read by several), and everything a thread needs is asked for together: statistics, its first 16 parts, the first 512 columns of the rows.
+// read by several), and everything a thread needs is asked for together: statistics, its first PF parts, the first 512 columns of the rows.
 // latent_absorb to here, 32 heads, R = 512, 900 slots, in a graph: 3 / 8 / 16 / 32 sequences 28.0 / 34.9 / 39.4 / 48.0 -> 23.8 / 27.9 / 29.9 / 36.7 us; of 64 x 128
 // 14.4 / 16.4 / 19.2 / 22.3 -> 14.4 / 15.9 / 17.4 / 20.3.  With the rows spread, the requests together and the preparation in
 // latent_absorb's launch, caches and maps cold, latent_prep to here: 1 / 3 / 8 / 16 / 32 sequences 21.9 / 27.7 / 32.2 / 34.5 / 39.9 -> 17.7 / 21.6 / 25.2 / 28.6 / 38.3 us.
-template <int NS, int VR>
+template <int NS, int VR, int PF>
 __global__ __launch_bounds__(512) void latent_up_mfma_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml, const float* __restrict__ sink,
                                                              const uint16_t* __restrict__ w, uint16_t* __restrict__ o, int B, int H, int R, int dv, int n_split) {
     extern __shared__ __attribute__((aligned(16))) uint16_t lat[];   // [NS][R + 8] merged latents, then [NS][n_split] weights of the parts
-    constexpr int PF = 16;                                       // parts of a thread's item in flight
     const int h = blockIdx.y, b0 = blockIdx.z * NS, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int pr = R + 8, c16 = lane & 15, g = lane >> 4;
     float* wt = (float*)(lat + NS * pr);
@@ -844,18 +851,35 @@ __global__ __launch_bounds__(512) void latent_up_mfma_kernel(const float* __rest
     }
 }
 
+// As many workgroups as there are CUs, if there are that many heads and sequences
+struct UpForm { int ns, vr, pf; };
+static UpForm up_form(int64_t B, int64_t H, int64_t dv, int64_t n_split) {
+    UpForm f = {2, 128, 16};
+    const int64_t per = H * ((dv + 127) / 128);
+    while (f.ns < 16 && per * ((B + f.ns - 1) / f.ns) > 256) f.ns *= 2;
+    while (f.ns == 2 && f.vr > 32 && H * ((dv + f.vr / 2 - 1) / (f.vr / 2)) * ((B + 1) / 2) <= 256) f.vr /= 2;
+    return f;
+}
+
+extern "C" int evo_latent_forms(int64_t B, int64_t H, int64_t R, int64_t dv, int64_t n_split, int64_t prep, int64_t* out) {
+    if (!out || B <= 0 || H <= 0 || R <= 0 || dv <= 0 || n_split <= 0) return -1;
+    const AbsorbForm a = absorb_form(B, H, R, true, prep != 0);
+    const UpForm u = up_form(B, H, dv, n_split);
+    out[0] = a.nb; out[1] = a.v; out[2] = u.ns; out[3] = u.vr; out[4] = u.pf;
+    return 0;
+}
+
 extern "C" int evo_latent_up(const float* part_o, const float* part_ml, const float* sink, const void* wuv, void* o, int64_t B, int64_t H, int64_t R,
                              int64_t dv, int64_t n_split, int64_t f32, int64_t mfma, void* stream) {
     if (!part_o || !part_ml || !sink || !wuv || !o || B <= 0 || H <= 0 || H > 65535 || R <= 0 || R > 8192 || dv <= 0 || n_split <= 0 || n_split > 64) return -1;
     if (!f32 && mfma && B > 2 && R % 32 == 0 && R <= 1024 && (((uintptr_t)wuv | (uintptr_t)part_o) & 15) == 0) {
-        int ns = 2, vr = 128;                                    // as many workgroups as there are CUs, if there are that many heads and sequences
-        const int64_t per = H * ((dv + 127) / 128);
-        while (ns < 16 && per * ((B + ns - 1) / ns) > 256) ns *= 2;
-        while (ns == 2 && vr > 32 && H * ((dv + vr / 2 - 1) / (vr / 2)) * ((B + 1) / 2) <= 256) vr /= 2;
+        const UpForm f = up_form(B, H, dv, n_split);
+        const int ns = f.ns, vr = f.vr;
         const dim3 grid((unsigned)((dv + vr - 1) / vr), (unsigned)H, (unsigned)((B + ns - 1) / ns));
         const size_t lds = (size_t)ns * ((R + 8) * 2 + n_split * 4);
-#define UPM(NS, VR) hipLaunchKernelGGL((latent_up_mfma_kernel<NS, VR>), grid, dim3(512), lds, (hipStream_t)stream, part_o, part_ml, sink, (const uint16_t*)wuv, \
-                                       (uint16_t*)o, (int)B, (int)H, (int)R, (int)dv, (int)n_split)
+#define UPG(NS, VR, PF) hipLaunchKernelGGL((latent_up_mfma_kernel<NS, VR, PF>), grid, dim3(512), lds, (hipStream_t)stream, part_o, part_ml, sink, (const uint16_t*)wuv, \
+                                           (uint16_t*)o, (int)B, (int)H, (int)R, (int)dv, (int)n_split)
+#define UPM(NS, VR) UPG(NS, VR, 16)
         if (vr == 32) UPM(2, 32);
         else if (vr == 64) UPM(2, 64);
         else if (ns == 2) UPM(2, 128);
@@ -863,6 +887,7 @@ extern "C" int evo_latent_up(const float* part_o, const float* part_ml, const fl
         else if (ns == 8) UPM(8, 128);
         else UPM(16, 128);
 #undef UPM
+#undef UPG
         return evo_launch_status();
     }
     const int nb = B > 2 ? 4 : (int)B;

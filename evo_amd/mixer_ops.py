@@ -457,8 +457,11 @@ class MixerOps:
 
     @staticmethod
     def latent_prep_fits(qd: torch.Tensor, cache: torch.Tensor, norm_w: torch.Tensor, inv_freq: torch.Tensor, heads: int, dn: int, dr: int, R: int) -> bool:
-        """What latent_decode's `prep` takes: rows of whole 16-byte pieces."""
-        return (qd.stride(0) % 8 == 0 and heads * (dn + dr) % 8 == 0 and R % 8 == 0 and cache.shape[2] % 8 == 0 and 0 < 2 * inv_freq.numel() <= dr and dn <= 4096
+        """What latent_decode's `prep` takes, rows of whole 16-byte pieces, and where it is ahead: not where many workgroups split the columns, whose angles are all made by the
+        first of them (us, in two launches : in one.  64 heads, R = 512: 16 / 24 / 64 sequences 11.7 : 11.2, 14.3 : 15.4, 22.7 : 29.3; 16 heads at 100 14.5 : 15.6; 128
+        heads, R = 256, at 100 40.8 : 35.9)."""
+        ahead = R <= 256 or heads * ((qd.shape[0] + 3) // 4) * ((R + 255) // 256) <= 512
+        return (ahead and qd.stride(0) % 8 == 0 and heads * (dn + dr) % 8 == 0 and R % 8 == 0 and cache.shape[2] % 8 == 0 and 0 < 2 * inv_freq.numel() <= dr and dn <= 4096
                 and norm_w.dtype == qd.dtype and (qd.data_ptr() | cache.data_ptr() | norm_w.data_ptr()) % 16 == 0)
 
     def latent_decode(self, qd: torch.Tensor, cache: torch.Tensor, pos: torch.Tensor, wuk: torch.Tensor, wuv: torch.Tensor, sink: torch.Tensor,

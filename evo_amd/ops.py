@@ -113,11 +113,12 @@ _SIGNATURES = {
     "evo_latent_prep_absorb": ([_PTR, _I64] + [_PTR] * 6 + [_I64] * 8 + [_F32, _I64, _PTR], _c.c_int),
     "evo_latent_absorb": ([_PTR, _I64] + [_PTR] * 2 + [_I64] * 7 + [_PTR], _c.c_int),
     "evo_latent_decode": ([_PTR] * 5 + [_I64] * 8 + [_F32] + [_I64] * 2 + [_PTR], _c.c_int),
+    "evo_latent_forms": ([_I64] * 6 + [_PTR], _c.c_int),
     "evo_latent_up": ([_PTR] * 5 + [_I64] * 7 + [_PTR], _c.c_int),
 }
 
 _LIB = None
-ABI_VERSION = 30         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 31         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):

@@ -71,8 +71,9 @@ extern "C" {
  *  27: evo_closing_final and evo_latent_prep_absorb added.
  *  28: evo_dense_parts, evo_dense_parts_bf16 and evo_rmsnorm_parts_bf16 added.
  *  29: evo_linear_residual_scaled_bf16, evo_linear_factors_bf16 and evo_mlp_gate_factors_bf16 added.
- *  30: evo_token_batch added. */
-#define EVO_ABI_VERSION 30
+ *  30: evo_token_batch added.
+ *  31: evo_latent_forms added. */
+#define EVO_ABI_VERSION 31
 int evo_abi_version(void);
 
 /* Tokens of B <= 64 sequences, one sequence behind the other: cu [B + 1] their starts, seq and pos [sum of lens] sequence and position (`past` of its sequence on) of every token,
@@ -611,6 +612,9 @@ int evo_latent_prep_absorb(const void* q, int64_t ldq, const void* wuk, void* ou
                            int64_t H, int64_t dn, int64_t dr, int64_t R, int64_t n_rot, int64_t ring, int64_t rs, float eps, int64_t f32, void* stream);
 int evo_latent_decode(const void* q, const void* cache, const int64_t* pos, float* part_o, float* part_ml, int64_t B, int64_t H, int64_t R,
                       int64_t dr, int64_t rs, int64_t ring, int64_t window, int64_t n_split, float scale, int64_t f32, int64_t mfma, void* stream);
+/* What a workgroup takes in evo_latent_absorb (`prep`: evo_latent_prep_absorb; maps aligned to 16 bytes) and in evo_latent_up on the matrix cores: out [5] = sequences and columns
+ * per lane of the former, sequences, value rows and parts in flight of the latter.  On the host, no launch. */
+int evo_latent_forms(int64_t B, int64_t H, int64_t R, int64_t dv, int64_t n_split, int64_t prep, int64_t* out);
 int evo_latent_up(const float* part_o, const float* part_ml, const float* sink, const void* wuv, void* o, int64_t B, int64_t H, int64_t R,
                   int64_t dv, int64_t n_split, int64_t f32, int64_t mfma, void* stream);
 

@@ -150,3 +150,32 @@ def test_short_rows_by_their_width():
         assert short(1, 5, D) and short(1, 1023, D) and short(12, 41, D) and short(6, 161, D) and short(8, 90, D)
         assert not short(1, 1024, D) and not short(2, 512, D) and not short(32, 41, D) and not short(18, 5, D)
     assert short(1, 500, 8192) and short(2, 161, 8192) and not short(1, 1000, 8192) and not short(12, 41, 8192) and not short(2, 500, 8192)
+
+
+def latent_forms(B, H, R, dv, n_split, prep):
+    out = (ctypes.c_int64 * 5)()
+    assert evo_ops.load_library().evo_latent_forms(B, H, R, dv, n_split, prep, ctypes.cast(out, ctypes.c_void_p)) == 0
+    return tuple(out)
+
+
+@pytest.mark.parametrize("B,H,R,dv,absorb,with_prep,up", [
+    (1, 32, 512, 128, (1, 2), (1, 2), (2, 32)), (2, 32, 512, 128, (2, 2), (2, 2), (2, 32)), (8, 32, 512, 128, (4, 2), (4, 2), (2, 64)), (16, 32, 512, 128, (4, 4), (4, 4), (2, 128)),
+    (32, 32, 512, 128, (4, 8), (4, 4), (4, 128)), (16, 64, 512, 128, (4, 8), (4, 4), (4, 128)), (7, 32, 512, 100, (4, 2), (4, 2), (2, 64)), (100, 128, 256, 64, (4, 8), (4, 4), (16, 128)),
+    (5, 3, 40, 30, (4, 2), (4, 2), (2, 32)), (5, 3, 41, 30, (4, 1), (4, 1), (2, 32)), (33, 8, 512, 256, (4, 2), (4, 2), (4, 128))])
+def test_forms_of_the_latent_maps(B, H, R, dv, absorb, with_prep, up):
+    """Columns of the query side are halved while fewer than 256 workgroups take them, and are 256 at most beside the preparation; value rows while 256 workgroups are not exceeded."""
+    assert latent_forms(B, H, R, dv, 16, 0) == absorb + up + (16,) and latent_forms(B, H, R, dv, 16, 1) == with_prep + up + (16,)
+
+
+def test_preparation_in_the_query_sides_launch_where_it_is_ahead():
+    import torch
+    from evo_amd.mixer_ops import MixerOps
+
+    def fits(B, heads, R, dn=128, dr=64):
+        width = heads * (dn + dr) + R + dr
+        qd, w = torch.empty(B, width, dtype=torch.bfloat16, device="meta"), torch.empty(R, dtype=torch.bfloat16, device="meta")
+        return MixerOps.latent_prep_fits(qd, torch.empty(B, 64, R + dr, dtype=torch.bfloat16, device="meta"), w, torch.empty(dr // 2, device="meta"), heads, dn, dr, R)
+    for B, heads, R in ((1, 32, 512), (32, 32, 512), (16, 64, 512), (64, 16, 512), (8, 128, 512), (100, 128, 256), (100, 32, 128)):
+        assert fits(B, heads, R)
+    for B, heads, R in ((33, 32, 512), (17, 64, 512), (65, 16, 512), (64, 128, 512), (33, 32, 384)):
+        assert not fits(B, heads, R)

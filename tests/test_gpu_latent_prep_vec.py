@@ -60,3 +60,46 @@ def test_preparation_with_the_query_side(ops, dt, B, H, dn, dr, R, n_rot, ring):
     ops.latent_prep(q2, H, dn, dr, R, w, inv, 1e-6, TokenBatch.of_decode(pos), c2, want_kv=False)
     want = ops.latent_decode(q2, c2, pos, wuk, wuv, sink, *sizes)
     assert torch.equal(qd, was) and torch.equal(cache, c2) and torch.equal(got, want)
+
+
+@TYPES
+@pytest.mark.parametrize("B,H,dn,dr,dv,R,forms", [(8, 32, 128, 64, 128, 512, (4, 2, 2, 64)), (16, 32, 128, 64, 128, 512, (4, 4, 2, 128)), (7, 32, 128, 64, 100, 512, (4, 2, 2, 64)),
+                                                  (16, 64, 24, 8, 24, 512, (4, 8, 4, 128)), (70, 64, 8, 8, 16, 256, (4, 8, 16, 128)), (2, 64, 16, 8, 128, 128, (2, 2, 2, 32))])
+def test_decode_by_the_forms_of_its_maps(ops, dt, B, H, dn, dr, dv, R, forms):  # noqa: F811
+    """Every form of the query side and of the value side, as evo_latent_forms names them, against windowed attention on uncompressed keys and values in 64 bits; with the
+    preparation in the same launch the same bits."""
+    import ctypes
+    import math
+    from evo_amd.mixer_ops import MixerOps, TokenBatch
+    from oracle import vozalorn_ref as V
+    out = (ctypes.c_int64 * 5)()
+    assert ops.lib.evo_latent_forms(B, H, R, dv, 3, 0, ctypes.cast(out, ctypes.c_void_p)) == 0 and tuple(out)[:4] == forms
+    g, ring, rs = torch.Generator().manual_seed(B), 20, MixerOps.latent_row(R, dr)
+
+    def rnd(*s, scale=1.0):
+        return (torch.randn(*s, generator=g) * scale).to(dt)
+    width = H * (dn + dr) + R + dr
+    cache, qd = rnd(B, ring, rs), rnd(B, (width + 7) // 8 * 8)
+    cache[:, :, R + dr:] = 0.0
+    wuk, wuv, w = rnd(H * dn, R, scale=1.5 / math.sqrt(R)), rnd(H * dv, R, scale=1 / math.sqrt(R)), rnd(R)
+    sink, scale, pos = torch.randn(H, generator=g), 1.5 / math.sqrt(dn + dr), [3 * b % 50 for b in range(B)]
+    inv = (10000.0 ** (-torch.arange(0, dr, 2) / dr)).cuda()
+    at = torch.tensor(pos).cuda()
+    dev = [t.cuda() for t in (wuk, wuv, sink)]
+    sizes = (H, dn, dr, dv, R, ring, scale)
+    # a token's own row as latent_prep makes it, and the queries as it leaves them
+    q2, c2 = qd.cuda(), cache.cuda()
+    ops.latent_prep(q2, H, dn, dr, R, w.cuda(), inv, 1e-6, TokenBatch.of_decode(at), c2, want_kv=False)
+    q64, c64 = q2.cpu().double(), c2.cpu().double()
+    for n_split in (1, 4, 5, 8, 9, 20):
+        got = ops.latent_decode(q2, c2, at, *dev, *sizes, n_split=n_split)
+        c3 = cache.cuda()
+        assert torch.equal(got, ops.latent_decode(qd.cuda(), c3, at, *dev, *sizes, n_split=n_split, prep=(w.cuda(), inv, 1e-6))) and torch.equal(c3, c2)
+        for b in {0, 1, B // 2, B - 1}:
+            js = range(max(0, pos[b] - ring + 1), pos[b] + 1)
+            rows = torch.stack([c64[b, j % ring, :R + dr] for j in js])
+            k = torch.cat([(rows[:, :R] @ wuk.double().T).view(len(js), H, dn), rows[:, None, R:].expand(len(js), H, dr)], -1)
+            v = (rows[:, :R] @ wuv.double().T).view(len(js), H, dv)
+            want = V.windowed_sink_attention(q64[b:b + 1, :H * (dn + dr)].view(1, H, dn + dr), k, v, scale, ring, sink, torch.tensor([pos[b]]), torch.tensor(list(js))).reshape(1, -1)
+            err = (got[b:b + 1].cpu().double() - want).norm() / want.norm()
+            assert err < (2e-2 if dt == torch.bfloat16 else 1e-5), (b, n_split, float(err))       # (test_latent_decode's bounds)
