@@ -179,3 +179,8 @@ def test_preparation_in_the_query_sides_launch_where_it_is_ahead():
         assert fits(B, heads, R)
     for B, heads, R in ((33, 32, 512), (17, 64, 512), (65, 16, 512), (64, 128, 512), (33, 32, 384)):
         assert not fits(B, heads, R)
+
+
+def test_no_more_parts_in_flight_than_there_are():
+    for n in range(1, 65):
+        assert latent_forms(16, 32, 512, 128, n, 0)[4] == (4 if n <= 4 else 8 if n <= 8 else 16)
