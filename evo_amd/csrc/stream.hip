@@ -18,12 +18,13 @@
         return evo_launch_status();                                                                                        \
     } while (0)
 
-// The same for kernels of one workgroup a row: rows of whole runs of eight a thread (2,048, 4,096 and 8,192 elements) have forms without a condition
-#define ROW_DISPATCH(KERNEL, VECOK, D_, GRID, ...)                                                                          \
+// The same for kernels of one workgroup a row: rows of whole runs of eight a thread (2,048, 4,096 and 8,192 elements) have forms without a condition, for sizes where these are
+// ahead (AHEAD)
+#define ROW_DISPATCH(KERNEL, VECOK, AHEAD, D_, GRID, ...)                                                                   \
     do {                                                                                                                   \
         const dim3 g_(GRID), b_(256);                                                                                      \
         hipStream_t s_ = (hipStream_t)stream;                                                                              \
-        const int runs_ = (VECOK) ? ((D_) == 2048 ? 1 : (D_) == 4096 ? 2 : (D_) == 8192 ? 4 : 0) : -1;                     \
+        const int runs_ = !(VECOK) ? -1 : !(AHEAD) ? 0 : (D_) == 2048 ? 1 : (D_) == 4096 ? 2 : (D_) == 8192 ? 4 : 0;       \
         if (f32) { ROW_LAUNCH(KERNEL, float, __VA_ARGS__); } else { ROW_LAUNCH(KERNEL, uint16_t, __VA_ARGS__); }           \
         return evo_launch_status();                                                                                        \
     } while (0)
@@ -74,9 +75,9 @@ extern "C" int evo_embed_stream(const int64_t* ids, const void* w, float* x, voi
 // asked for behind the reduction there were two of them: rows of 4,096 in a step of four layers 3.5 -> 2.8 us at 8 rows, on the parts of 24 rows 5.2 -> 3.8, the gated norm
 // 3.9 -> 2.4 (an empty launch is 1.6).
 template <typename T, int V, bool PARTS>
-__device__ __forceinline__ void closing_load(const void* __restrict__ y_, int64_t row, int c, int D, int parts, float* f) {
+__device__ __forceinline__ void closing_load(const void* __restrict__ row, int c, int D, int parts, float* f) {
     if constexpr (PARTS) {
-        const float* p = (const float*)y_ + row * D + c;
+        const float* p = (const float*)row + c;
         const int64_t plane = (int64_t)gridDim.x * D;
         vec_io<float, V>::load(p, f);
         for (int s = 1; s < parts; s += 3) {                     // (three requests at once; a plane behind the last is the last again, and not added)
@@ -90,7 +91,7 @@ __device__ __forceinline__ void closing_load(const void* __restrict__ y_, int64_
         }
 #pragma unroll
         for (int e = 0; e < V; ++e) f[e] = bf_to_f(f_to_bf(f[e]));
-    } else vec_io<T, V>::load((const T*)y_ + row * D + c, f);
+    } else vec_io<T, V>::load((const T*)row + c, f);
 }
 
 template <typename T, int V, bool SUM, bool PARTS, int RUNS>
@@ -106,7 +107,7 @@ __device__ __forceinline__ void closing_row(const void* __restrict__ y_, const v
         vec_io<T, V>::load(w + c, g[i]);
     }
 #pragma unroll
-    for (int i = 0; i < RUNS; ++i) closing_load<T, V, PARTS>(y_, row, (threadIdx.x + 256 * i) * V, D, parts, f[i]);
+    for (int i = 0; i < RUNS; ++i) closing_load<T, V, PARTS>(PARTS ? (const void*)((const float*)y_ + row * D) : (const void*)((const T*)y_ + row * D), (threadIdx.x + 256 * i) * V, D, parts, f[i]);
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < RUNS; ++i)
@@ -140,10 +141,11 @@ __device__ __forceinline__ void closing_norm(const void* __restrict__ y_, const 
     }
     constexpr int KEEP = V == 8 ? 2 : 4;                         // runs of V elements a thread keeps in registers (D <= 256 V KEEP)
     const T* w = (const T*)w_;
+    const void* y = PARTS ? (const void*)((const float*)y_ + row * D) : (const void*)((const T*)y_ + row * D);
     float keep[KEEP][V];
     float ss = 0.f;
     auto load = [&](int c, float* f) {
-        closing_load<T, V, PARTS>(y_, row, c, D, parts, f);
+        closing_load<T, V, PARTS>(y, c, D, parts, f);
         if constexpr (SUM) {
             float r[V];
             vec_io<float, V>::load(x + row * D + c, r);
@@ -203,14 +205,15 @@ extern "C" int evo_postnorm_residual(const void* y, const void* w, float* x, voi
                                      int64_t f32, void* stream) {
     if (M < 0 || M > 0x7fffffff || D <= 0 || D > 0x3fffffff) return -1;
     if (M == 0) return 0;
-    ROW_DISPATCH(postnorm_residual_kernel, D % 8 == 0, D, (unsigned)M, y, w, x, (uint16_t*)xb, (int)D, eps, w_offset);
+    ROW_DISPATCH(postnorm_residual_kernel, D % 8 == 0, true, D, (unsigned)M, y, w, x, (uint16_t*)xb, (int)D, eps, w_offset);
 }
 
 extern "C" int evo_sum_norm(const void* y, const void* w, float* x, void* xb, int64_t M, int64_t D, float alpha, float eps, float w_offset,
                             int64_t f32, void* stream) {
     if (!y || !w || !x || M < 0 || M > 0x7fffffff || D <= 0 || D > 0x3fffffff) return -1;
     if (M == 0) return 0;
-    ROW_DISPATCH(sum_norm_kernel, D % 8 == 0, D, (unsigned)M, y, w, x, (uint16_t*)xb, (int)D, alpha, eps, w_offset);
+    // (8,192 columns, the loop : the row at once, us: 256 rows 9.1 : 8.0, 400 10.9 : 10.6, 512 12.1 : 12.4, 600 14.2 : 15.6, 768 16.9 : 17.3, 1,000 22.1 : 21.9, 2,048 49 : 41)
+    ROW_DISPATCH(sum_norm_kernel, D % 8 == 0, D != 8192 || M <= 400 || M > 900, D, (unsigned)M, y, w, x, (uint16_t*)xb, (int)D, alpha, eps, w_offset);
 }
 
 // Both on the parts of a dense layer's sum (evo_linear_parts_bf16): the launch that added and rounded them was 4.7 us of its own, a decode layer of 17 to 64 rows.
@@ -286,7 +289,7 @@ extern "C" int evo_rmsnorm_stream(const float* x, const void* w, void* out, int6
                                   void* stream) {
     if (M < 0 || M > 0x7fffffff || D <= 0 || D > 0x3fffffff) return -1;
     if (M == 0) return 0;
-    ROW_DISPATCH(rmsnorm_stream_kernel, D % 8 == 0, D, (unsigned)M, x, w, out, (int)D, eps, w_offset);
+    ROW_DISPATCH(rmsnorm_stream_kernel, D % 8 == 0, true, D, (unsigned)M, x, w, out, (int)D, eps, w_offset);
 }
 
 // ---------------------------------------------------------------------------------------------- the last closing norm and the final one
@@ -409,7 +412,9 @@ extern "C" int evo_gated_norm(const void* o, const void* g, int64_t ldg, const v
     if (M < 0 || M > 0x7fffffff || D <= 0 || D > 0x3fffffff || ldg < D) return -1;
     if (M == 0) return 0;
     const bool vec = D % 8 == 0 && ldg % 8 == 0 && ((uintptr_t)g & 15) == 0;
-    ROW_DISPATCH(gated_norm_kernel, vec, D, (unsigned)M, o, g, ldg, w, out, (int)D, eps);
+    // (bf16, the loop : the row at once, us.  2,048 columns: 512 rows 3.3 : 3.3, 600 3.4 : 3.6, 1,536 5.0 : 5.5, 4,096 11.2 : 11.6, 8,190 19.5 : 19.1; 4,096 columns: 400 rows
+    // 4.1 : 3.8, 1,000 6.0 : 6.1, 2,048 10.0 : 11.0, 4,096 19.1 : 19.0, 8,190 36.2 : 33.0; 8,192 and fp32 0.95 to 1.3)
+    ROW_DISPATCH(gated_norm_kernel, vec, f32 || D == 8192 || M <= 512 || M > 4096, D, (unsigned)M, o, g, ldg, w, out, (int)D, eps);
 }
 
 // ---------------------------------------------------------------------------------------------- a = silu(z[:, :I]) * z[:, I:]
