@@ -648,25 +648,29 @@ static int tile_plan_square(int64_t M, int64_t N, int64_t K, int mode, bool stat
 // 20.6 / 21.2, 4,096 37.9 / 34.4 / 35.7 / 37.8 -> 31.1 / 31.7 / 35.0 / 36.0 (phases from 161 rows on), 8,192 54.9 / 57.7 / 63.4 / 65.9 -> 52.1 / 54.1 / 60.5 / 65.5, 11,264 of 4,096 31.9 / 34.0 /
 // 35.0 / 37.2 -> 31.4 / 31.0 / 34.2 / 34.6; 96 x 48, 6,144 of 4,096 22.4 / 24.5 / 26.4 / 27.9 -> 20.9 / 21.4 / 23.3 / 26.1 (of 6,144 from 145 rows on 2 to 11 % behind: parts of K); 64 x 96 at
 // 193 / 224 / 255 rows there 27.2 / 29.0 / 30.8 -> 23.8 / 26.3 / 28.7; two parts at 65 / 96 / 128 rows, 16,384 of 4,096 41.0 / 39.0 / 40.7 -> 34.9 / 36.1 / 38.7, 13,824 of 5,120 47.9 / 46.6 /
-// 50.1 -> 39.3 / 40.9 / 43.9, 8,192 of 4,096 at 240 36.9 -> 32.5 (of 2,048 behind: 16,384 24.0 : 26.5).
+// 50.1 -> 39.3 / 40.9 / 43.9, 8,192 of 4,096 at 240 36.9 -> 32.5 (of 2,048 behind: 16,384 24.0 : 26.5).  96 x 48 of short K not where its second row
+// tile is nearly empty (the time before over this, 5,632 to 6,144 columns of 2,048: 97 rows 0.92, 104 0.96, 120 0.96 to 1.02, 129 1.33 to 1.43; of 2,560 1.02 to 1.15 from 97 on, of 2,816 to 4,096
+// 0.96 to 0.98 at 97 and 0.99 to 1.08 at 104), beyond K = 4,608 to 144 (of 5,120: 129 1.05, 145 0.98, 161 0.93, 192 0.92).
+// 0.9: the mean of 96 x 48's and 64 x 96's times above over those before, for parts_plan's comparison (the others are wider than what comes in parts).
 static void tile_one_round(int64_t M, int64_t N, int64_t K, bool splits_ok, TilePlan& plan) {
     const int64_t cus = tile_cus();
     auto round = [&](int kind) {
         const int64_t tiles = ((M + kinds[kind].bm - 1) / kinds[kind].bm) * ((N + kinds[kind].bn - 1) / kinds[kind].bn);
         return tiles <= cus && 10 * tiles >= 9 * cus;
     };
-    const int kind = M <= 96 || K < 2048 ? -1 : M <= 192 && round(T_ODD) ? T_ODD : K > 5120 ? -1 : M <= 192 ? (round(T_ODD + 2) ? T_ODD + 2 : -1) : round(T_ODD + 3) ? T_ODD + 3 : -1;
+    const bool narrow = M >= (K < 2560 ? 129 : 97) && (K <= 4608 || M <= 144);
+    const int kind = M <= 96 || K < 2048 ? -1 : M <= 192 && round(T_ODD) ? T_ODD : K > 5120 ? -1 : M <= 192 ? (narrow && round(T_ODD + 2) ? T_ODD + 2 : -1) : round(T_ODD + 3) ? T_ODD + 3 : -1;
     if (kind >= 0) plan = {kind, 1, 0.9 * plan.us, M};
     else if (plan.kind == 1 && plan.splits == 1 && splits_ok && K >= 4096 && 2 * ((M + 127) / 128) * (N / 128) <= cus) plan = {2, 2, plan.us, M};
 }
 
 // Gated layers of 97 to 128 rows: 128 x 96 in phases where column tiles are nearly a round, 96 x 96 where two row tiles of them are.  us at 97 / 112 / 128 rows, before -> these: 22,016 columns of
-// K = 4,096 43.5 / 43.7 / 44.9 -> 41.8 / 41.8 / 42.7 (128 x 128 in phases before: 172 workgroups; 16,384 columns, 171, 40.8 : 41.5), 11,264 of 2,048 20.5 / 20.5 / 20.9 -> 17.0 / 17.9 / 18.4.
+// K = 4,096 43.5 / 43.7 / 44.9 -> 41.8 / 41.8 / 42.7 (128 x 128 in phases before: 172 workgroups; 16,384 columns, 171, 40.8 : 41.5; of 2,048 0.95 to 1.0, of 2,560 to 6,144 0.97 to 1.17), 11,264 of 2,048 20.5 / 20.5 / 20.9 -> 17.0 / 17.9 / 18.4.
 static void tile_one_round_gated(int64_t M, int64_t N, int64_t K, TilePlan& plan) {
     const int64_t cus = tile_cus(), across = (N + 95) / 96;
     if (M <= 96 || M > 128 || K < 2048) return;
-    if (across <= cus && 8 * across >= 7 * cus) plan = {T_ODD + 4, 1, 0.95 * plan.us, M};
-    else if (2 * across <= cus && 20 * across >= 9 * cus) plan = {T_ODD, 1, 0.85 * plan.us, M};
+    if (across <= cus && 8 * across >= 7 * cus) plan = {T_ODD + 4, 1, plan.us, M};
+    else if (2 * across <= cus && 20 * across >= 9 * cus) plan = {T_ODD, 1, plan.us, M};
 }
 
 static double steps_us(const StepUs& s, double rows, double cols, double nk) {

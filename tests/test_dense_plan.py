@@ -184,3 +184,16 @@ def test_preparation_in_the_query_sides_launch_where_it_is_ahead():
 def test_no_more_parts_in_flight_than_there_are():
     for n in range(1, 65):
         assert latent_forms(16, 32, 512, 128, n, 0)[4] == (4 if n <= 4 else 8 if n <= 8 else 16)
+
+
+def tiles(M, N, K):
+    p, = launches(0, False, M, N, K)
+    return p["tile_rows"], p["tile_cols"], p["parts"]
+
+
+@pytest.mark.parametrize("N", [5632, 5888, 6144])
+def test_narrow_tiles_where_they_are_ahead(N):
+    """96 x 48: not where the second row tile is nearly empty and K is small, nor where parts of a long K are ahead."""
+    for K, first, last in ((2048, 129, 192), (2496, 129, 192), (2560, 97, 192), (4096, 97, 192), (4608, 97, 192), (4672, 97, 144), (5120, 97, 144)):
+        for M in range(97, 193):
+            assert (tiles(M, N, K) == (96, 48, 1)) == (first <= M <= last), (M, K, tiles(M, N, K))
