@@ -197,3 +197,14 @@ def test_narrow_tiles_where_they_are_ahead(N):
     for K, first, last in ((2048, 129, 192), (2496, 129, 192), (2560, 97, 192), (4096, 97, 192), (4608, 97, 192), (4672, 97, 144), (5120, 97, 144)):
         for M in range(97, 193):
             assert (tiles(M, N, K) == (96, 48, 1)) == (first <= M <= last), (M, K, tiles(M, N, K))
+
+
+def test_parts_for_a_norm_where_they_are_ahead():
+    """Layers whose own launch is ahead of parts and their norm, and neighbours whose is not."""
+    parts = evo_ops.load_library().evo_dense_parts
+    for M, N, K in ((900, 4096, 5632), (780, 4096, 5632), (940, 4096, 5632), (660, 4096, 4096), (900, 3072, 3072), (136, 3072, 3072), (145, 3072, 3072),
+                    (136, 4096, 4096), (145, 4096, 4096)):
+        assert parts(M, N, K) == 0, (M, N, K)
+    for M, N, K in ((1000, 4096, 5632), (740, 4096, 5632), (700, 4096, 5632), (600, 4096, 4096), (512, 4096, 4096), (880, 3072, 3072), (128, 3072, 3072), (123, 4096, 4096),
+                    (222, 4096, 5632), (161, 4096, 11008), (90, 6144, 4096), (145, 5120, 5120)):
+        assert parts(M, N, K) >= 2, (M, N, K)
