@@ -1274,10 +1274,11 @@ static int ring_go(dim3 grid, const void* x, const void* w, const void* bias, co
 }
 // 4,097 to 7,680 columns from K = 4,096 on (to 7,168: from 2,048): a workgroup per CU here too, of 17 to 30 columns in two waves.  A CU takes in 45 to 55 GB/s while lines come
 // from memory, however many are under way, and 132 to 240 workgroups left the others idle (and, to 16 rows, six stages of their 12 KB: 36 KB under way are too few).  Four
-// stages and 32 columns -> this, us at 5 / 16 / 24 / 32 rows: 4,224 x 4,096 11.1 / 11.0 / 12.1 / 12.5 -> 10.4 / 10.3 / 12.2 / 12.3, 6,144 x 4,096 13.2 / 13.1 / 12.9 / 13.5 ->
-// 11.0 / 11.4 / 12.5 / 12.7, 6,720 x 4,096 13.5 / 13.1 / 13.4 / 14.0 -> 11.5 / 11.9 / 12.6 / 13.2, x 11,008 29.3 / 30.1 / 32.6 / 32.1 -> 26.4 / 27.4 / 31.0 / 32.7; 33 to 64 rows
-// 1.00 to 1.04.  Beyond, 31 and 32 columns a workgroup are as good (8,000 x 4,096 14.2 : 14.6), and at small K nothing is gained (6,144 x 1,024 4.9 : 5.0,
-// 7,680 x 2,048 7.5 : 7.7).
+// stages and 32 columns -> this, us at 5 / 16 / 24 / 32 rows, weights cold: 4,224 x 4,096 13.3 / 13.7 / 12.7 / 13.3 -> 11.9 / 11.1 / 12.8 / 12.9, 6,144 x 4,096 14.1 / 14.4 / 15.2 /
+// 14.2 -> 11.9 / 12.3 / 14.6 / 13.6, 6,720 x 4,096 14.5 / 14.7 / 15.2 / 16.0 -> 12.5 / 13.0 / 14.8 / 14.0, x 11,008 30.2 / 30.9 / 33.4 / 34.9 -> 27.3 / 28.3 / 32.6 / 33.8.  Over 861
+// layers, plain and gated, K = 2,048 to 16,384: to 16 rows 0.98 to 1.28, 17 to 32 rows 0.97 to 1.15, 33 to 64 rows 0.96 to 1.10; behind at 17 and 24 rows of K = 2,048 and 4,096 and at 40
+// rows, gated, by up to 0.3 and 1.8 us.  Beyond, 31 and 32 columns a workgroup are as good (8,000 x 4,096 14.2 : 14.6), and at small K nothing is gained (6,144 x 1,024 4.9 :
+// 5.0, 7,680 x 2,048 7.5 : 7.7).
 static bool ring_spread(int64_t N, int64_t K) { return N > 4096 && (N <= 7168 ? K >= 2048 : N <= 7680 && K >= 4096); }
 static int64_t ring_groups(int64_t N, int64_t K) {
     const int64_t share = (N + 31) / 32;
@@ -1288,9 +1289,9 @@ static int ring_waves(int64_t N, int64_t K) {
     return rows <= 32 ? 2 : rows <= 48 ? 3 : rows <= 64 ? 4 : 6;
 }
 // What workgroup `block` of N weight rows (gated: N / 2 result columns) takes: out = workgroups, its first column, the next one's, columns that it has room for
-extern "C" int evo_linear_ring_share(int64_t N, int64_t gated, int64_t block, int64_t* out) {
-    if (!out || N <= 0 || N > 0x7fffffff - 16 || (gated && N % 2)) return -1;
-    const int64_t K = 4096, groups = ring_groups(N, K), cols = gated ? N / 2 : N;     // (any K from 4,096 on)
+extern "C" int evo_linear_ring_share(int64_t N, int64_t K, int64_t gated, int64_t block, int64_t* out) {
+    if (!out || N <= 0 || N > 0x7fffffff - 16 || K <= 0 || K % 128 || (gated && N % 2)) return -1;
+    const int64_t groups = ring_groups(N, K), cols = gated ? N / 2 : N;
     if (block < 0 || block >= groups) return -1;
     out[0] = groups;
     out[1] = ring_edge((uint32_t)cols, (uint32_t)groups, (uint32_t)block);

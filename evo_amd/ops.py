@@ -92,7 +92,7 @@ _SIGNATURES = {
     "evo_lightning_chunk_bf16": ([_PTR, _I64] + [_PTR] * 6 + [_I64] * 6 + [_PTR], _c.c_int),
     "evo_postnorm_linear_small_m_bf16": ([_PTR] * 6 + [_I64] * 3 + [_F32, _I64] + [_F32] * 2 + [_I64, _PTR], _c.c_int),
     "evo_postnorm_mlp_gate_small_m_bf16": ([_PTR] * 6 + [_I64] * 3 + [_F32, _I64] + [_F32] * 2 + [_I64] * 2 + [_PTR], _c.c_int),
-    "evo_linear_ring_share": ([_I64] * 3 + [_PTR], _c.c_int),
+    "evo_linear_ring_share": ([_I64] * 4 + [_PTR], _c.c_int),
     "evo_linear_parts": ([_I64] * 3, _c.c_int),
     "evo_linear_parts_bf16": ([_PTR] * 3 + [_I64] * 4 + [_PTR], _c.c_int),
     "evo_closing_final": ([_PTR, _I64] + [_PTR] * 4 + [_I64] * 3 + [_F32] * 3 + [_I64, _PTR], _c.c_int),
@@ -118,7 +118,7 @@ _SIGNATURES = {
 }
 
 _LIB = None
-ABI_VERSION = 31         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
+ABI_VERSION = 32         # must equal EVO_ABI_VERSION in include/evo_mi355x.h (bumped on every signature change)
 
 
 class EvoLibraryError(RuntimeError):

@@ -72,8 +72,9 @@ extern "C" {
  *  28: evo_dense_parts, evo_dense_parts_bf16 and evo_rmsnorm_parts_bf16 added.
  *  29: evo_linear_residual_scaled_bf16, evo_linear_factors_bf16 and evo_mlp_gate_factors_bf16 added.
  *  30: evo_token_batch added.
- *  31: evo_latent_forms added. */
-#define EVO_ABI_VERSION 31
+ *  31: evo_latent_forms added.
+ *  32: evo_linear_ring_share gained K. */
+#define EVO_ABI_VERSION 32
 int evo_abi_version(void);
 
 /* Tokens of B <= 64 sequences, one sequence behind the other: cu [B + 1] their starts, seq and pos [sum of lens] sequence and position (`past` of its sequence on) of every token,
@@ -309,9 +310,9 @@ int evo_linear_residual_scaled_bf16(const void* x, const void* w, const void* bi
 int evo_linear_factors_bf16(const void* xg, const float* ss, float eps, const void* w, const void* bias, void* y, int64_t M, int64_t N, int64_t K, void* stream);
 int evo_mlp_gate_factors_bf16(const void* xg, const float* ss, float eps, const void* w12, void* a, int64_t M, int64_t I, int64_t K, int64_t grouped, void* stream);
 
-/* Columns per workgroup of that launch on a wide layer (N > 4096, K % 128 == 0 and, for 4,097 to 7,680 columns, K >= 4096) and of the gated one (`gated`: N = 2 I, I columns): out [4] = workgroups, first column of workgroup
- * `block`, first behind it, columns that a workgroup has room for.  On the host, no launch; -1: no such workgroup. */
-int evo_linear_ring_share(int64_t N, int64_t gated, int64_t block, int64_t* out);
+/* Columns per workgroup of that launch on a wide layer (N > 4096, K % 128 == 0) and of the gated one (`gated`: N = 2 I, I columns): out [4] = workgroups, first column of
+ * workgroup `block`, first behind it, columns that a workgroup has room for.  On the host, no launch; -1: no such workgroup. */
+int evo_linear_ring_share(int64_t N, int64_t K, int64_t gated, int64_t block, int64_t* out);
 
 /* Parts of K that evo_linear_small_m_bf16 takes for a narrow layer with such a workspace (0: one sum), and the launch that leaves them in ws [parts][M][N]. */
 int evo_linear_parts(int64_t M, int64_t N, int64_t K);

@@ -64,26 +64,32 @@ def test_segments_of_recurrent_mixers():
     assert plan((1459, 1667, 1875, 2084, 2292, 2500), 32) >= 2500 and plan((500,), 32) == 512 and plan((8190,), 32) == 1024 and plan((1000, 2000, 4000), 32) == 1024
 
 
-@pytest.mark.parametrize("N", [96, 4097, 8192, 12289, 22016, 24577, 6291456, 6291458, 6488064, 7000000, 9999998, 200000000, 2147483630])
+@pytest.mark.parametrize("N", [96, 4096, 4097, 4098, 7168, 7169, 7170, 7680, 7681, 7682, 8192, 12289, 22016, 24577, 6291456, 6291458, 6488064, 7000000, 9999998, 200000000, 2147483630])
+@pytest.mark.parametrize("K", [128, 1920, 2048, 3968, 4096, 22016])
 @pytest.mark.parametrize("gated", [0, 1])
-def test_columns_of_weight_streaming_workgroups(N, gated):
+def test_columns_of_weight_streaming_workgroups(N, K, gated):
     """Every column belongs to one workgroup, which has room for all of its own: floor(block cols / workgroups) up to the largest layer that is accepted, where block x
-    columns has more than 32 bits.  The two halves of [W1; W2] have their borders where the gated launch has them."""
+    columns has more than 32 bits.  The two halves of [W1; W2] have their borders where the gated launch has them.  A workgroup per CU for 4,097 to 7,168 columns from K = 2,048
+    on and to 7,680 from 4,096 on; below, one for every 32 columns."""
     lib, out, half = evo_ops.load_library(), (ctypes.c_int64 * 4)(), (ctypes.c_int64 * 4)()
+    share = lib.evo_linear_ring_share
     if gated and N % 2:
-        assert lib.evo_linear_ring_share(N, 1, 0, ctypes.cast(out, ctypes.c_void_p)) == -1
+        assert share(N, K, 1, 0, ctypes.cast(out, ctypes.c_void_p)) == -1
         return
     cols = N // 2 if gated else N
-    assert lib.evo_linear_ring_share(N, gated, 0, ctypes.cast(out, ctypes.c_void_p)) == 0 and out[1] == 0
+    assert share(N, K, gated, 0, ctypes.cast(out, ctypes.c_void_p)) == 0 and out[1] == 0
     groups, room = out[0], out[3]
+    if N <= 8192:
+        assert groups == (256 if 4096 < N <= 7168 and K >= 2048 or 7168 < N <= 7680 and K >= 4096 else -(-N // 32))
     blocks = range(groups) if groups <= 120000 else sorted({0, 1, 65535, 65536, 65537, groups - 2, groups - 1} | {i * 999983 % groups for i in range(20000)})
     for b in blocks:
-        assert lib.evo_linear_ring_share(N, gated, b, ctypes.cast(out, ctypes.c_void_p)) == 0
+        assert share(N, K, gated, b, ctypes.cast(out, ctypes.c_void_p)) == 0
         assert out[0] == groups and out[1] == b * cols // groups and out[2] == (b + 1) * cols // groups and 0 < out[2] - out[1] <= room
         if gated and b % 2 == 0:
-            assert lib.evo_linear_ring_share(N, 0, b // 2, ctypes.cast(half, ctypes.c_void_p)) == 0 and half[1] == out[1]
+            assert share(N, K, 0, b // 2, ctypes.cast(half, ctypes.c_void_p)) == 0 and half[1] == out[1]
     assert out[2] == cols
-    assert lib.evo_linear_ring_share(N, gated, groups, ctypes.cast(out, ctypes.c_void_p)) == -1
+    assert share(N, K, gated, groups, ctypes.cast(out, ctypes.c_void_p)) == -1
+    assert share(N, K + 64, gated, 0, ctypes.cast(out, ctypes.c_void_p)) == share(N, 0, gated, 0, ctypes.cast(out, ctypes.c_void_p)) == -1
 
 
 def test_workspace_of_segments():
