@@ -5,7 +5,6 @@ from __future__ import annotations
 
 import functools
 import inspect
-import operator
 from dataclasses import dataclass
 from typing import List, Optional, Sequence, Tuple
 
@@ -40,7 +39,7 @@ class TokenBatch:
 
     @staticmethod
     def of_prompts(lens: Sequence[int], past: Sequence[int], device, ops=None) -> "TokenBatch":
-        lens, past = [operator.index(n) for n in lens], [operator.index(n) for n in past]
+        lens, past = list(lens), list(past)
         B, M, device = len(lens), sum(lens), torch.device(device)
         if device.type == "cuda" and hasattr(ops, "token_batch") and 0 < B <= ops.MAX_PUT:
             cu, seq, pos, resume = ops.token_batch(lens, past, device)

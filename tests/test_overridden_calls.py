@@ -3,7 +3,6 @@ passes call them as they stand, whatever keywords the framework's own versions h
 import functools
 import types
 
-import numpy as np
 import pytest
 import torch
 
@@ -11,7 +10,7 @@ from golden_common import TINY, tiny_model
 from oracle_ops import OracleOps
 
 from evo_amd import scoring
-from evo_amd.mixer_ops import Stream, TokenBatch, takes
+from evo_amd.mixer_ops import Stream, takes
 from evo_amd.sh.model import StripedHyena
 from evo_amd.tokenizer import CharLevelTokenizer
 
@@ -103,14 +102,3 @@ def test_whether_a_method_takes_a_keyword():
         later = x
         return later
     assert not takes(local, "later")
-
-
-def test_lengths_that_are_not_ints():
-    """Lengths and positions from arrays or tensors are what they were when torch made a tensor of them: kernel arguments are integers of Python."""
-    asked = []
-    ops = types.SimpleNamespace(MAX_PUT=64, token_batch=lambda lens, past, device: asked.append((lens, past)) or (None, None, None, None))
-    for lens, past in ((np.array([3, 5]), np.array([0, 2], dtype=np.int32)), ([np.int64(3), torch.tensor(5)], [0, np.uint8(2)]), (torch.tensor([3, 5]), torch.tensor([0, 2]))):
-        batch = TokenBatch.of_prompts(lens, past, "cuda", ops)
-        assert (batch.lens, batch.past) == asked.pop() == ([3, 5], [0, 2]) and {type(n) for n in batch.lens + batch.past} == {int}
-        cpu = TokenBatch.of_prompts(lens, past, "cpu")
-        assert cpu.cu.tolist() == [0, 3, 8] and cpu.pos.tolist() == [0, 1, 2, 2, 3, 4, 5, 6]
