@@ -353,5 +353,6 @@ def test_latent_decode(ops, mfma, dt, H, dn, dr, dv, R, window, ring):
 @TYPES
 @pytest.mark.parametrize("H,dn,dr,dv,R", [(70, 40, 16, 72, 64), (2, 136, 24, 130, 640), (1, 7, 8, 17, 1024), (100, 16, 8, 16, 64), (200, 16, 8, 24, 32), (300, 8, 8, 16, 32)])
 def test_latent_decode_maps(ops, mfma, dt, H, dn, dr, dv, R):
-    """The maps around the decode kernel: whole and halved columns, more than one run of rows in flight, rows over 512 wide, 2 to 16 sequences a workgroup."""
+    """The maps around the decode kernel: columns a lane's two and eight at a time (four: test_gpu_latent_prep_vec.py), more than one run of rows in flight, rows over 512 wide, 2 to 16
+    sequences a workgroup."""
     test_latent_decode(ops, mfma, dt, H, dn, dr, dv, R, 20, 20)

@@ -118,3 +118,50 @@ def test_decode_steps_of_a_pool(ops, B, monkeypatch):
         model._dgraph = None
         want = steps()
     assert ((got - want).norm() / want.norm()).item() < 12 * 2.0 ** -9     # (six norms a step, each rounded once, 2^-9 at most, on either side)
+
+
+@pytest.mark.parametrize("B,width", [(40, 2048), (24, 4096)])
+def test_decode_steps_that_add_parts(ops, B, width, monkeypatch):
+    """Steps of 17 to 64 rows, whose norms add the parts of the layers in front of them (at 24 rows of 4,096 the mixer's, as row factors, in between): the same bits eagerly and
+    captured, and every norm's rows against its own launch's."""
+    from evo_amd.sh.model import StripedHyena
+    model = StripedHyena(dict(vocab_size=512, hidden_size=width, num_layers=3, attn_layer_idxs=[1], num_attention_heads=width // 128))
+    g = torch.Generator(device=DEV).manual_seed(0)
+    model.to_bfloat16_except_poles_residues()
+    model = model.to(DEV).eval()
+    with torch.no_grad():
+        for name, p in model.named_parameters():
+            if name.endswith(("poles", "residues")):
+                p.uniform_(0.0, 0.5, generator=g)
+            else:
+                p.normal_(1.0 if name.endswith("scale") else 0.0, 0.02 if p.dim() > 1 else 0.1, generator=g)
+    ids = torch.randint(0, 512, (B, 13), generator=g, device=DEV)
+    added, scaled, one = [], [], []
+    norm_, scaled_ = type(ops).linear_residual_norm_, type(ops).linear_residual_scaled_
+
+    def steps(captured):
+        model.decode_graph, model._dgraph, model._dgraph_warm, model.decode_graph_replays = captured, None, None, 0
+        ipd = model.initialize_inference_params()
+        ipd["mha"].max_batch_size = ipd["hyena"].max_batch_size = B
+        ipd["mha"].max_seqlen = 16
+        out = [model(ids[:, :8], inference_params_dict=ipd)[0][:, -1:]]
+        for t in range(8, 13):
+            one.append(1)
+            ipd["mha"].seqlen_offset = ipd["hyena"].seqlen_offset = t
+            out.append(model(ids[:, t:t + 1], inference_params_dict=ipd)[0])
+            if captured:                                             # (eager work between the replays)
+                ops.rmsnorm(out[-1].new_ones(3, 512), None, out[-1].new_ones(512), 1e-6)
+                torch.cuda.synchronize()
+            one.pop()
+        assert not captured or model.decode_graph_replays >= 3
+        return torch.cat(out, 1).float()
+    with torch.inference_mode():
+        monkeypatch.setattr(type(ops), "linear_residual_norm_", lambda self, *a, **k: ((got := norm_(self, *a, **k)), added.append(got) if one and got is not None else None)[0])
+        monkeypatch.setattr(type(ops), "linear_residual_scaled_", lambda self, *a: ((got := scaled_(self, *a)), scaled.append(got) if one and got is not None else None)[0])
+        got = steps(False)
+        assert len(added) >= 5 * 3 and (len(scaled) >= 5 * 3) == (B <= 32)      # (a step: three layers' at least)
+        assert torch.equal(steps(True), got)
+        monkeypatch.setattr(type(ops), "linear_residual_norm_", lambda *a, **k: None)
+        monkeypatch.setattr(type(ops), "linear_residual_scaled_", lambda *a: None)
+        want = steps(False)
+    assert ((got - want).norm() / want.norm()).item() < 12 * 2.0 ** -9     # (as above)

@@ -64,8 +64,10 @@ def test_what_stays_in_launches_of_its_own(ops):
 
 
 @pytest.mark.parametrize("lens", [[160], [90, 31], [299, 200]])
-def test_scored_and_prefilled_rows(ops, lens, monkeypatch):
-    """A model whose layers hand the next norm on, against the same with every norm in its own launch: both within bf16's rounding of each other, layer after layer."""
+@pytest.mark.parametrize("cached", [False, True])
+def test_scored_and_prefilled_rows(ops, lens, cached, monkeypatch):
+    """A model whose layers hand the next norm on, against the same with every norm in its own launch: both within bf16's rounding of each other, layer after layer.  `cached`: a
+    prompt and its continuation on states that the first call left."""
     from evo_amd.sh.model import StripedHyena
     cfg = dict(vocab_size=512, hidden_size=2048, num_layers=3, attn_layer_idxs=[1], num_attention_heads=16)
     model = StripedHyena(cfg)
@@ -82,9 +84,18 @@ def test_scored_and_prefilled_rows(ops, lens, monkeypatch):
     taken = []
     was = type(ops).linear_residual_norm_
     monkeypatch.setattr(type(ops), "linear_residual_norm_", lambda self, *a, **k: taken.append(was(self, *a, **k)) or taken[-1])
+
+    def logits():
+        if not cached:
+            return model(ids)[0].float()
+        ipd, half = model.initialize_inference_params(), ids.shape[1] * 3 // 5
+        ipd["mha"].max_batch_size = ipd["hyena"].max_batch_size = len(lens)
+        first = model(ids[:, :half], inference_params_dict=ipd)[0]
+        ipd["mha"].seqlen_offset = ipd["hyena"].seqlen_offset = half
+        return torch.cat([first, model(ids[:, half:], inference_params_dict=ipd)[0]], 1).float()
     with torch.inference_mode():
-        got = model(ids)[0].float()
-        assert sum(t is not None for t in taken) >= 3
+        got = logits()
+        assert sum(t is not None for t in taken) >= (6 if cached else 3)
         monkeypatch.setattr(type(ops), "linear_residual_norm_", lambda *a, **k: None)
-        want = model(ids)[0].float()
+        want = logits()
     assert ((got - want).norm() / want.norm()).item() < 8 * 2.0 ** -9      # (six roundings of the stream, each 2^-9 of it at most)

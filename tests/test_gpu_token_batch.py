@@ -50,3 +50,26 @@ def test_ids_that_are_not_there():
             pool.prefill(wrong[1:])
     for (a, _, _), (b, _, _) in zip(pool.prefill(prompts), want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_ids_that_are_not_there_in_a_layered_decoder(dtype):
+    """The same of LayeredDecoder's prompts, packed in one pass or several."""
+    import vozalorn_util as U
+    from evo_amd.ops import default_ops
+    cfg = U.CONFIGS["window_64"]
+    model = U.build(cfg, U.weights(cfg), dtype=dtype, device="cuda", ops=default_ops())
+    g = torch.Generator().manual_seed(0)
+    prompts = [torch.randint(0, cfg["vocab"], (n,), generator=g).cuda() for n in (40, 33, 70)]
+    for rows in (1 << 20, 64):
+        model.max_rows_per_pass = rows
+        with torch.inference_mode():
+            want = model.prefill_rows(prompts)
+            for at in range(3):
+                for bad in (cfg["vocab"], -1):
+                    wrong = [p.clone() for p in prompts]
+                    wrong[at][-1] = bad
+                    with pytest.raises(IndexError, match="outside"):
+                        model.prefill_rows(wrong)
+            for (a, _, _), (b, _, _) in zip(model.prefill_rows(prompts), want):
+                assert torch.equal(a, b)
