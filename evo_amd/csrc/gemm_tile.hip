@@ -822,14 +822,14 @@ extern "C" int evo_dense_plan(int64_t mode, int64_t stats, int64_t M, int64_t N,
 
 // Parts of K that the norm behind a layer adds (rmsnorm_parts_kernel, closing_parts_kernel), 65 to 1,023 rows and up to 8,192 columns: without a launch of their own (5.5 us at 161 rows)
 // parts pay in more layers and in larger numbers.  us, layer and norm in their own launches -> parts and norm, K = 4,096, 11,008 and 16,384 of 4,096 columns: 65 rows 20.5 -> 17.0,
-// 33.9 -> 28.6, 39.3 -> 35.0; 161 rows 23.2 -> 22.3, 38.6 -> 36.3, 46.8 -> 44.2; 512 rows 39.1 -> 33.8, 64.3 -> 63, 81.5 -> 78.5; 8,192 x 8,192 56.4 -> 45.8 at 161 rows, 84 -> 81 at 512; over 873
-// layers and sizes of 512 to 8,192 columns 1.13 x with rmsnorm_parts_kernel, over 630 1.10 x with closing_parts_kernel, ten and nine of them 2 to 5 % behind (2,048 x 2,048 at 520 to 660 rows in
-// the latter; one of 10 %, 4,096 columns of 16,384 at 201 rows).
+// 33.9 -> 28.6, 39.3 -> 35.0; 161 rows 23.2 -> 22.3, 38.6 -> 36.3, 46.8 -> 44.2; 512 rows 39.1 -> 33.8, 64.3 -> 63, 81.5 -> 78.5; 8,192 x 8,192 56.4 -> 45.8 at 161 rows, 84 -> 81 at 512; over 842
+// layers and sizes of 1,024 to 8,192 columns 1.17 x with rmsnorm_parts_kernel, over 601 1.12 x with closing_parts_kernel, weights cold, three and six of them 2 to 5 % behind.
 // `parts_us`, fitted to 2,100 launches (5 % off them): the k-steps of a part, the parts' bytes, written and read, and the weights'; two, four and eight parts start a power of two
 // apart and meet in the L2's channels.  One round of the chip; parts of 64 x 64 tiles as far as they have a CU each, eight of 192 rows on never (7 : 8 at K = 16,384 44 : 50).
 // 128 x 128 in one sum and in step beyond 512 rows takes by its last row tile what its own cost rule does not know: 0.89 to 1.03 of that with 4 to 32 rows there, 1.07 to 1.17 with 100 and
-// more, not 1.1 (4,096 columns of 5,632 at 900 rows 51.4 in one sum, 57.7 in two parts; 780 49.0 : 54.4; of 4,096 at 660 37.5 : 39.0, 600 41.2 : 38.2; at 540 it is taken still, 36.1 : 37.3).  And no parts of fewer than 17
-// k-steps of 128 rows and more of up to 4,096 columns that 64 x 64 takes in one round: 3,072 columns of 3,072 at 145 rows 17.9 : 20.7, 4,096 of 4,096 22.0 : 23.7.
+// more, not 1.1 (4,096 columns of 5,632 at 900 rows 51.4 in one sum, 57.7 in two parts; 780 49.0 : 54.4; of 4,096 at 660 37.5 : 39.0, 600 41.2 : 38.2; at 540 it is taken still, 36.1 : 37.3).  And no parts of fewer than 13
+// k-steps on 192 rows and more of up to 4,096 columns that 64 x 64 takes in one round: 3,072 columns of 3,072 at 151 rows 18.3 : 20.3, 4,096 of 4,096 at 138 20.7 : 21.5 (on 128 x 128, 16
+// k-steps, they are ahead there: 145 rows 21.2 -> 19.6, 161 22.2 -> 20.2, all with the fp32 stream's norm).
 struct PartsUs { int kind; double us, base; };
 static const PartsUs parts_us[] = {{0, 0.21, 6.0}, {2, 0.43, 6.6}, {3, 0.55, 5.5}, {4, 0.665, 4.4}};
 static TilePlan parts_plan(int64_t M, int64_t N, int64_t K) {
@@ -848,7 +848,7 @@ static TilePlan parts_plan(int64_t M, int64_t N, int64_t K) {
     const bool tiles128 = n == 1 && own[0].kind == 2 && own[0].splits == 1 && M > 512 && !tile_phases(2, 0, false, 1, M, N, K);
     const double beyond = tiles128 ? 0.93 + 0.27 * (double)((M - 1) % 128 + 1) / 128 : 1.1;
     const double apart = beyond * (n == 2 ? own[0].us + own[1].us + 4.0 : own[0].us) + 1.3 + 0.47e-6 * (double)(M * N * 2);
-    const bool few_steps = N <= 4096 && best.kind >= 2 && own[0].kind == 0 && own[0].splits == 1 && nk / best.splits < 17;
+    const bool few_steps = N <= 4096 && best.kind >= 3 && own[0].kind == 0 && own[0].splits == 1 && nk / best.splits < 13;
     if (few_steps || fmax(best.us, power) > 0.97 * apart) best.splits = 0;
     return best;
 }

@@ -208,9 +208,10 @@ def test_narrow_tiles_where_they_are_ahead(N):
 def test_parts_for_a_norm_where_they_are_ahead():
     """Layers whose own launch is ahead of parts and their norm, and neighbours whose is not."""
     parts = evo_ops.load_library().evo_dense_parts
-    for M, N, K in ((900, 4096, 5632), (780, 4096, 5632), (940, 4096, 5632), (660, 4096, 4096), (900, 3072, 3072), (136, 3072, 3072), (145, 3072, 3072),
-                    (136, 4096, 4096), (145, 4096, 4096)):
+    for M, N, K in ((900, 4096, 5632), (780, 4096, 5632), (940, 4096, 5632), (660, 4096, 4096), (900, 3072, 3072), (136, 3072, 3072), (151, 3072, 3072),
+                    (130, 4096, 4096), (138, 4096, 4096)):
         assert parts(M, N, K) == 0, (M, N, K)
     for M, N, K in ((1000, 4096, 5632), (740, 4096, 5632), (700, 4096, 5632), (600, 4096, 4096), (512, 4096, 4096), (880, 3072, 3072), (128, 3072, 3072), (123, 4096, 4096),
+                    (145, 4096, 4096), (161, 4096, 4096), (181, 3072, 3584), (189, 3072, 4096), (296, 2048, 4096), (435, 1536, 3584), (161, 3584, 4096),
                     (222, 4096, 5632), (161, 4096, 11008), (90, 6144, 4096), (145, 5120, 5120)):
         assert parts(M, N, K) >= 2, (M, N, K)
