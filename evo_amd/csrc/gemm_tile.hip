@@ -649,8 +649,8 @@ static int tile_plan_square(int64_t M, int64_t N, int64_t K, int mode, bool stat
 // 35.0 / 37.2 -> 31.4 / 31.0 / 34.2 / 34.6; 96 x 48, 6,144 of 4,096 22.4 / 24.5 / 26.4 / 27.9 -> 20.9 / 21.4 / 23.3 / 26.1 (of 6,144 from 145 rows on 2 to 11 % behind: parts of K); 64 x 96 at
 // 193 / 224 / 255 rows there 27.2 / 29.0 / 30.8 -> 23.8 / 26.3 / 28.7; two parts at 65 / 96 / 128 rows, 16,384 of 4,096 41.0 / 39.0 / 40.7 -> 34.9 / 36.1 / 38.7, 13,824 of 5,120 47.9 / 46.6 /
 // 50.1 -> 39.3 / 40.9 / 43.9, 8,192 of 4,096 at 240 36.9 -> 32.5 (of 2,048 behind: 16,384 24.0 : 26.5).  96 x 48 of short K not where its second row
-// tile is nearly empty (the time before over this, 5,632 to 6,144 columns of 2,048: 97 rows 0.92, 104 0.96, 120 0.96 to 1.02, 129 1.33 to 1.43; of 2,560 1.02 to 1.15 from 97 on, of 2,816 to 4,096
-// 0.96 to 0.98 at 97 and 0.99 to 1.08 at 104), beyond K = 4,608 to 144 (of 5,120: 129 1.05, 145 0.98, 161 0.93, 192 0.92).
+// tile is nearly empty (the time before over this, 5,632 to 6,144 columns, weights cold: of 2,048 0.91 at 97 rows, 0.92 to 0.96 at 104, 1.0 at 112, 1.02 to 1.04 to 128, 1.21 to 1.45 beyond; of 2,304
+// 0.93, 0.95, 1.04, 1.09; of 2,560 to 4,608 0.96 to 1.03 at 97 and 104), beyond K = 4,608 to 144 (of 5,120: 136 0.98 to 1.02, 145 0.94 to 0.97, 161 and more 0.90 to 0.96).
 // 0.9: the mean of 96 x 48's and 64 x 96's times above over those before, for parts_plan's comparison (the others are wider than what comes in parts).
 static void tile_one_round(int64_t M, int64_t N, int64_t K, bool splits_ok, TilePlan& plan) {
     const int64_t cus = tile_cus();
@@ -658,7 +658,7 @@ static void tile_one_round(int64_t M, int64_t N, int64_t K, bool splits_ok, Tile
         const int64_t tiles = ((M + kinds[kind].bm - 1) / kinds[kind].bm) * ((N + kinds[kind].bn - 1) / kinds[kind].bn);
         return tiles <= cus && 10 * tiles >= 9 * cus;
     };
-    const bool narrow = M >= (K < 2560 ? 129 : 97) && (K <= 4608 || M <= 144);
+    const bool narrow = M >= (K < 2560 ? 112 : 97) && (K <= 4608 || M <= 144);
     const int kind = M <= 96 || K < 2048 ? -1 : M <= 192 && round(T_ODD) ? T_ODD : K > 5120 ? -1 : M <= 192 ? (narrow && round(T_ODD + 2) ? T_ODD + 2 : -1) : round(T_ODD + 3) ? T_ODD + 3 : -1;
     if (kind >= 0) plan = {kind, 1, 0.9 * plan.us, M};
     else if (plan.kind == 1 && plan.splits == 1 && splits_ok && K >= 4096 && 2 * ((M + 127) / 128) * (N / 128) <= cus) plan = {2, 2, plan.us, M};
