@@ -90,20 +90,21 @@ def test_rows_of_whole_runs(ops, D, dtype):
     assert torch.equal(4 * ops.gated_norm(y, z, g, 1e-6), ops.gated_norm(wide(y), wide(z), wide(g), 1e-6 / 16)[:, :D])
 
 
-@pytest.mark.parametrize("D,counts", [(2048, (513, 4096, 4097)), (4096, (513, 4097)), (8192, (401, 900, 901, 513))])
+@pytest.mark.parametrize("D,counts", [(2048, (513, 4096, 4097)), (4096, (513, 4097)), (8192, (256, 257, 401, 900, 901, 513, 1024, 1025))])
 @pytest.mark.parametrize("dtype", [BF, torch.float32])
 def test_rows_of_either_form(ops, D, counts, dtype):
-    """Rows of a count that takes the loop, or the row at once, against the same rows 400 at a time: a thread has the same elements in the same order, so the same bits."""
+    """Rows of a count that takes the loop, or the row at once, against the same rows 200 at a time: a thread has the same elements in the same order, so the same bits."""
     for M in counts:
         x, y, z, g = (rnd(*s, seed=i).to(DEV, t) for i, (s, t) in enumerate((((M, D), torch.float32), ((M, D), dtype), ((M, D), dtype), ((D,), dtype))))
-        a, b = x.clone(), x.clone()
-        ab, bb = (a, b) if dtype == torch.float32 else (torch.zeros_like(y), torch.zeros_like(y))
-        ops.sum_norm_(a, ab, y, g, 2.0, 1e-6, 1.0)
-        for at in range(0, M, 400):
-            bp = b[at:at + 400]
-            ops.sum_norm_(bp, bp if bb is b else bb[at:at + 400], y[at:at + 400], g, 2.0, 1e-6, 1.0)
-        assert torch.equal(a, b) and torch.equal(ab, bb)
-        assert torch.equal(ops.gated_norm(y, z, g, 1e-6), torch.cat([ops.gated_norm(y[at:at + 400], z[at:at + 400], g, 1e-6) for at in range(0, M, 400)]))
+        for norm in (lambda x, xb, y: ops.sum_norm_(x, xb, y, g, 2.0, 1e-6, 1.0), lambda x, xb, y: ops.postnorm_residual_(x, xb, y, g, 1e-6, 1.0)):
+            a, b = x.clone(), x.clone()
+            ab, bb = (a, b) if dtype == torch.float32 else (torch.zeros_like(y), torch.zeros_like(y))
+            norm(a, ab, y)
+            for at in range(0, M, 200):
+                bp = b[at:at + 200]
+                norm(bp, bp if bb is b else bb[at:at + 200], y[at:at + 200])
+            assert torch.equal(a, b) and torch.equal(ab, bb)
+        assert torch.equal(ops.gated_norm(y, z, g, 1e-6), torch.cat([ops.gated_norm(y[at:at + 200], z[at:at + 200], g, 1e-6) for at in range(0, M, 200)]))
 
 
 def test_one_sum_stays_one_sum(ops):
