@@ -665,8 +665,9 @@ __global__ __launch_bounds__(256) void attn_decode_stream_kernel(AttnArgs a, int
     const gptr_t vp = (gptr_t)(uint64_t)(a.v + bat * a.v_sb + head * a.v_sh);
     const uint32_t kst = (uint32_t)(a.k_st * 2), vst = (uint32_t)(a.v_st * 2), dco = (uint32_t)dc * 16;
     typedef unsigned int attn_u32x4 __attribute__((ext_vector_type(4)));
-    // (non-temporal: whole rows that nobody reads again.  us with the merge: 1 x 3,000 / 30,000 / 131,000 keys 16.6 / 90.6 / 364 -> 14.8 / 81.7 / 331, 16 x 700 40.4 -> 36.0, 5 x 100
-    // 9.0 -> 8.3)
+    // (non-temporal: whole rows that nobody reads again.  us with the merge, one after the other: 1 x 3,000 / 30,000 / 131,000 keys 16.6 / 90.6 / 364 -> 14.8 / 81.7 / 331, 16 x 700 40.4 -> 36.0, 5 x 100
+    // 9.0 -> 8.3.  Behind a layer's weight stream this launch itself is slower so, 1 x 3,000 11.4 -> 12.5, 16 of up to 1,100 29.5 -> 32.7, and the layers behind it find more of their weights in
+    // the last-level cache: a step of four layers, 1 / 8 x 3,000 335.6 / 431.6 -> 329.9 / 413.4, 32 x 900 503.6 -> 478.2, 16 x 300 / 1,100 367.5 / 409.6 -> 370.4 / 411.6, 2 x 900 346.6 -> 355.0)
     auto ld16 = [](gptr_t base, uint32_t off) {
         const attn_u32x4 t = __builtin_nontemporal_load((const __attribute__((address_space(1))) attn_u32x4*)(base + off));
         return make_uint4(t[0], t[1], t[2], t[3]);
@@ -816,10 +817,11 @@ __global__ __launch_bounds__(256) void attn_decode_stream_kernel(AttnArgs a, int
 // 512 threads = 4 groups x 128 output dims; the statistics are read once into LDS (coalesced) and turned into weights, then
 // group g sums splits g, g + 4, ... with eight independent row loads in flight (the first version walked the splits one
 // dependent L2 round trip at a time: 7 us at 16 splits, ~30 us at the 64 the streaming kernel uses).
-// FEW: up to 31 splits.  A thread's rows -- at most eight, one latency each in the loop for what eight at a time leave over -- are then asked for with the statistics, before
-// the weights are known (16 / 20 splits 15.5 -> 14.8 and 40.8 -> 40.3 us with the streaming kernel at 2 x 1,000 and 16 x 700 keys; 32 splits 16.5 : 16.7, which stay).
+// ROWS: up to 31 splits, at most ROWS of them a thread's.  Its rows -- one latency each in the loop for what eight at a time leave over -- are then asked for with the statistics, before
+// the weights are known (16 / 20 splits 15.5 -> 14.8 and 40.8 -> 40.3 us with the streaming kernel at 2 x 1,000 and 16 x 700 keys; 32 splits 16.5 : 16.7, which stay), and no more of
+// them than there are (eight everywhere : as many, us with the streaming kernel: 32 x 30 / 60 / 200 keys 11.5 / 14.2 / 25.8 -> 10.6 / 13.5 / 25.1, 16 x 100 12.1 -> 11.6, 1 x 60 7.4 -> 7.1).
 #define ATTN_MAX_SPLITS 1024
-template <bool FEW>
+template <int ROWS>
 __global__ __launch_bounds__(512) void attn_decode_combine_kernel(const float* __restrict__ part_o,
                                                                   const float* __restrict__ part_ml,
                                                                   uint16_t* __restrict__ o, int H, int n_splits) {
@@ -828,10 +830,10 @@ __global__ __launch_bounds__(512) void attn_decode_combine_kernel(const float* _
     __shared__ float acc_s[4][DH];
     const int tid = threadIdx.x, d = tid & (DH - 1), g = tid >> 7, head = blockIdx.x, bat = blockIdx.y;
     const int64_t base = ((int64_t)bat * H + head) * n_splits;
-    float r[8];
-    if constexpr (FEW) {
+    float r[ROWS > 0 ? ROWS : 8];
+    if constexpr (ROWS > 0) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) r[u] = part_o[(base + (g + 4 * u < n_splits ? g + 4 * u : n_splits - 1)) * DH + d];
+        for (int u = 0; u < ROWS; ++u) r[u] = part_o[(base + (g + 4 * u < n_splits ? g + 4 * u : n_splits - 1)) * DH + d];
     }
     // pass 1: maxima
     float M = -INFINITY;
@@ -858,9 +860,9 @@ __global__ __launch_bounds__(512) void attn_decode_combine_kernel(const float* _
     for (int i = 0; i < 8; ++i) L += red[8 + i];
     // pass 3: weighted rows
     float acc = 0.f;
-    if constexpr (FEW) {
+    if constexpr (ROWS > 0) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) acc = g + 4 * u < n_splits ? fmaf(r[u], w_s[g + 4 * u], acc) : acc;
+        for (int u = 0; u < ROWS; ++u) acc = g + 4 * u < n_splits ? fmaf(r[u], w_s[g + 4 * u], acc) : acc;
     } else {
         int s = g;
         for (; s + 28 < n_splits; s += 32) {
@@ -986,9 +988,12 @@ extern "C" int evo_attn_decode_bf16(const void* q, const void* k, const void* v,
     }
     else
         hipLaunchKernelGGL(attn_fwd_kernel<true>, dim3((unsigned)n_splits, (unsigned)H, (unsigned)B), dim3(256), 0, s, a);
-    if (n_splits < 32)
-        hipLaunchKernelGGL(attn_decode_combine_kernel<true>, dim3((unsigned)H, (unsigned)B), dim3(512), 0, s, part_o, part_ml, (uint16_t*)o, (int)H, (int)n_splits);
-    else
-        hipLaunchKernelGGL(attn_decode_combine_kernel<false>, dim3((unsigned)H, (unsigned)B), dim3(512), 0, s, part_o, part_ml, (uint16_t*)o, (int)H, (int)n_splits);
+#define ATTN_COMBINE(ROWS) hipLaunchKernelGGL(attn_decode_combine_kernel<ROWS>, dim3((unsigned)H, (unsigned)B), dim3(512), 0, s, part_o, part_ml, (uint16_t*)o, (int)H, (int)n_splits)
+    if (n_splits <= 4) ATTN_COMBINE(1);
+    else if (n_splits <= 8) ATTN_COMBINE(2);
+    else if (n_splits <= 16) ATTN_COMBINE(4);
+    else if (n_splits < 32) ATTN_COMBINE(8);
+    else ATTN_COMBINE(0);
+#undef ATTN_COMBINE
     return evo_launch_status();
 }

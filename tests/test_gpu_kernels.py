@@ -503,6 +503,13 @@ def test_attention_decode_matches_oracle(ops, B, H, Tk, splits):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("splits", [1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 30, 31, 32, 33, 36])
+def test_attention_decode_merge_of_any_parts(ops, splits):
+    """Parts around the numbers that the merge asks for at once (4, 8, 16 and 31), with parts that have no key among them (700 keys are eleven blocks)."""
+    test_attention_decode_matches_oracle(ops, 2, 3, 700, splits)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("positions,scaling", [([5], 1.0), ([100, 60000, 131071], 16.0), ([100, 8191, 70000], 1.0),
                                                ([(37 * b + 5) % 300 for b in range(9)], 16.0)])
 def test_rope_append_decode_is_bitwise_table_rope_and_indexed_copy(positions, scaling):
